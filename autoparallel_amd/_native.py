@@ -87,6 +87,12 @@ EXPORTS = (
     "apc_redistribute_tables_static",
     "apc_strategy_inputs",
     "apc_validate_packed_tiles_host",
+    "apc_pack_tiles_host",
+    "apc_edge_classes_host",
+    "apc_count_tiles_host",
+    "apc_fill_tiles_host",
+    "apc_tile_records_host",
+    "apc_validate_tiling_host",
     "apc_build_tables_packed",
     "apc_calibrate_launch",
     "apc_calibrate_fill",
@@ -167,6 +173,32 @@ def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = lib().apc_last_error().decode("utf-8", "replace")
         raise RuntimeError(f"{what} failed ({rc}): {msg}")
+
+
+def _argument(a):
+    """A host entry point's argument: a contiguous numpy array as its address, ``None`` as NULL, an
+    integer as int64, a ctypes structure by reference."""
+    if a is None:
+        return ctypes.c_void_p(None)
+    if isinstance(a, int):
+        return ctypes.c_int64(a)
+    if isinstance(a, ctypes.Structure):
+        return ctypes.byref(a)
+    if not a.flags.c_contiguous:
+        raise ValueError("host entry points take contiguous arrays")
+    return ctypes.c_void_p(a.ctypes.data)
+
+
+def host_call(name: str, *args) -> None:
+    """Calls a host entry point of the library; raises RuntimeError with its message on an error."""
+    check(getattr(lib(), name)(*[_argument(a) for a in args]), name)
+
+
+def host_counts(name: str, *args) -> tuple:
+    """A host entry point whose last two arguments are ``int64_t *`` results: returns them."""
+    first, second = ctypes.c_int64(), ctypes.c_int64()
+    check(getattr(lib(), name)(*[_argument(a) for a in args], ctypes.byref(first), ctypes.byref(second)), name)
+    return first.value, second.value
 
 
 def vp(ptr) -> ctypes.c_void_p:

@@ -22,18 +22,22 @@
 #include <type_traits>
 
 #include "apcost.h"
+#include "apcost_error.h"
 
-namespace {
+static thread_local char g_err[512] = "";
 
-thread_local char g_err[512] = "";
-
-int fail(int code, const char *fmt, ...) {
+int apc_internal::fail(int code, const char *fmt, ...) {
   va_list ap;
   va_start(ap, fmt);
   vsnprintf(g_err, sizeof(g_err), fmt, ap);
   va_end(ap);
   return code;
 }
+
+using apc_internal::check_params;
+using apc_internal::fail;
+
+namespace {
 
 int check_launch(const char *what) {
   hipError_t e = hipGetLastError();
@@ -2568,7 +2572,9 @@ int check_width(int width) {
   return 0;
 }
 
-int check_params(const apc_params *p) {
+}  // namespace
+
+int apc_internal::check_params(const apc_params *p) {
   if (!p) return fail(-1, "params is NULL");
   if (p->mesh_ndim < 1 || p->mesh_ndim > APC_MAX_MESH)
     return fail(-1, "mesh_ndim %d outside [1, %d]", p->mesh_ndim, APC_MAX_MESH);
@@ -2586,114 +2592,11 @@ int check_params(const apc_params *p) {
   return 0;
 }
 
-}  // namespace
-
 extern "C" {
 
 int apc_version(void) { return APC_ABI_VERSION; }
 
 const char *apc_last_error(void) { return g_err; }
-
-int apc_validate_tables_host(const apc_params *params, int64_t n_tensors, const int32_t *tensor_rank,
-                             int64_t n_specs, const uint32_t *spec_codes, const int32_t *spec_tensor,
-                             int64_t n_edges, const int32_t *edge_src_begin, const int32_t *edge_n_src,
-                             const int32_t *edge_tgt_begin, const int32_t *edge_n_tgt,
-                             const int32_t *edge_flags, const int64_t *edge_pt_begin,
-                             const int64_t *edge_entry_begin, const int32_t *edge_strat_begin, int64_t n_pt,
-                             int64_t n_strategies, int64_t n_tiles, const apc_tile *tiles, int64_t n_dups,
-                             const int64_t *dup_entry_begin) {
-  if (int rc = check_params(params)) return rc;
-  const int M = params->mesh_ndim;
-  for (int64_t t = 0; t < n_tensors; ++t)
-    if (tensor_rank[t] < 0 || tensor_rank[t] > APC_MAX_RANK)
-      return fail(-2, "tensor %lld: rank %d outside [0, %d]", (long long)t, tensor_rank[t], APC_MAX_RANK);
-  for (int64_t s = 0; s < n_specs; ++s) {
-    const int t = spec_tensor[s];
-    if (t < -1 || t >= n_tensors)
-      return fail(-2, "spec %lld: tensor row %d out of range [-1, %lld)", (long long)s, t, (long long)n_tensors);
-    if (M < 4 && (spec_codes[s] >> (8 * M)) != 0)
-      return fail(-2, "spec %lld: placement bytes beyond mesh ndim %d are set (0x%08x)", (long long)s, M,
-                  spec_codes[s]);
-    for (int i = 0; i < M; ++i) {
-      const uint32_t c = (spec_codes[s] >> (8 * i)) & 0xFF;
-      if ((c >> 6) == 3) return fail(-2, "spec %lld: placement code 0x%02x has no meaning", (long long)s, c);
-      if ((c >> 6) == 0 && c != 0) return fail(-2, "spec %lld: placement code 0x%02x has no meaning", (long long)s, c);
-      if ((c >> 6) == 2 && t >= 0 && (int)(c & 0x0F) >= tensor_rank[t])
-        return fail(-2, "spec %lld: Shard(%d) on a rank-%d tensor", (long long)s, (int)(c & 0x0F), tensor_rank[t]);
-    }
-  }
-  int64_t expect = 0;
-  for (int64_t e = 0; e < n_edges; ++e) {
-    if (edge_entry_begin[e] != expect)
-      return fail(-2, "edge %lld: entry_begin %lld, expected %lld (offsets must be the running sum of n_tgt*n_src)",
-                  (long long)e, (long long)edge_entry_begin[e], (long long)expect);
-    const int64_t ns = edge_n_src[e], nt = edge_n_tgt[e];
-    if (ns < 0 || nt < 0) return fail(-2, "edge %lld: negative strategy count", (long long)e);
-    if (ns > APC_MAX_STRATEGIES || nt > APC_MAX_STRATEGIES)
-      return fail(-2, "edge %lld: %lld x %lld strategies, at most %d a side", (long long)e, (long long)nt,
-                  (long long)ns, APC_MAX_STRATEGIES);
-    if (edge_src_begin[e] < 0 || edge_src_begin[e] + ns > n_specs)
-      return fail(-2, "edge %lld: producer spec range [%d, +%lld) outside the spec table", (long long)e,
-                  edge_src_begin[e], (long long)ns);
-    if (edge_tgt_begin[e] < 0 || edge_tgt_begin[e] + nt > n_specs)
-      return fail(-2, "edge %lld: consumer spec range [%d, +%lld) outside the spec table", (long long)e,
-                  edge_tgt_begin[e], (long long)nt);
-    if (edge_strat_begin[e] < 0 || edge_strat_begin[e] + nt > n_strategies)
-      return fail(-2, "edge %lld: strategy rows [%d, +%lld) outside the strategy table", (long long)e,
-                  edge_strat_begin[e], (long long)nt);
-    bool needs_pt = (edge_flags[e] & APC_EDGE_NO_PRODUCER) != 0;
-    if (!needs_pt) {
-      for (int64_t j = 0; j < ns && !needs_pt; ++j) needs_pt = spec_tensor[edge_src_begin[e] + j] < 0;
-      for (int64_t j = 0; j < nt && !needs_pt; ++j) needs_pt = spec_tensor[edge_tgt_begin[e] + j] < 0;
-    }
-    if (needs_pt && (edge_pt_begin[e] < 0 || edge_pt_begin[e] + ns * nt > n_pt))
-      return fail(-2, "edge %lld: pass-through values [%lld, +%lld) outside pt_values", (long long)e,
-                  (long long)edge_pt_begin[e], (long long)(ns * nt));
-    expect += ns * nt;
-  }
-  if (edge_entry_begin[n_edges] != expect)
-    return fail(-2, "entry_begin[n_edges] = %lld, expected %lld", (long long)edge_entry_begin[n_edges],
-                (long long)expect);
-  for (int64_t t = 0; t < n_tiles; ++t) {
-    const apc_tile &tl = tiles[t];
-    const int e = tl.edge;
-    const int row_count = tl.counts & 0xFFFF, col_count = tl.counts >> 16;
-    if (e < 0 || e >= n_edges) return fail(-2, "tile %lld: edge %d out of range", (long long)t, e);
-    if (row_count < 1 || row_count > APC_TILE_MAX_ROWS || tl.row_begin < 0 ||
-        tl.row_begin + row_count > edge_n_tgt[e])
-      return fail(-2, "tile %lld: rows [%d, +%d) outside edge %d (n_tgt %d, max %d per tile)", (long long)t,
-                  tl.row_begin, row_count, e, edge_n_tgt[e], APC_TILE_MAX_ROWS);
-    if (col_count < 1 || col_count > APC_TILE_MAX_COLS || tl.col_begin < 0 ||
-        tl.col_begin + col_count > edge_n_src[e])
-      return fail(-2, "tile %lld: cols [%d, +%d) outside edge %d (n_src %d, max %d per tile)", (long long)t,
-                  tl.col_begin, col_count, e, edge_n_src[e], APC_TILE_MAX_COLS);
-    if (tl.src_begin != edge_src_begin[e] || tl.n_src != edge_n_src[e] || tl.tgt_begin != edge_tgt_begin[e] ||
-        tl.flags != edge_flags[e] || tl.strat_begin != edge_strat_begin[e] ||
-        tl.entry_begin != edge_entry_begin[e] || tl.pt_begin != edge_pt_begin[e])
-      return fail(-2, "tile %lld: record does not repeat the fields of edge %d", (long long)t, e);
-    if (tl.tensor != spec_tensor[edge_src_begin[e] + tl.col_begin])
-      return fail(-2, "tile %lld: tensor %d is not the tensor of its first producer spec", (long long)t, tl.tensor);
-    if (tl.dup_count < 0 || tl.dup_count > APC_TILE_MAX_DUPS || tl.dup_begin < 0 ||
-        (int64_t)tl.dup_begin + tl.dup_count > n_dups)
-      return fail(-2, "tile %lld: duplicate list [%d, +%d) outside dup_entry_begin", (long long)t, tl.dup_begin,
-                  tl.dup_count);
-    for (int d = 0; d < tl.dup_count; ++d) {
-      // the offset must be the start of another edge with the same matrix shape
-      const int64_t off = dup_entry_begin[tl.dup_begin + d];
-      int64_t lo = 0, hi = n_edges;  // first edge whose entry_begin >= off, then skip empty edges
-      while (lo < hi) {
-        const int64_t mid = (lo + hi) / 2;
-        if (edge_entry_begin[mid] < off) lo = mid + 1; else hi = mid;
-      }
-      while (lo < n_edges && (int64_t)edge_n_src[lo] * edge_n_tgt[lo] == 0) ++lo;
-      if (lo >= n_edges || edge_entry_begin[lo] != off || lo == e || edge_n_src[lo] != edge_n_src[e] ||
-          edge_n_tgt[lo] != edge_n_tgt[e])
-        return fail(-2, "tile %lld: duplicate offset %lld is not the start of an edge shaped like edge %d",
-                    (long long)t, (long long)off, e);
-    }
-  }
-  return 0;
-}
 
 int apc_tensor_tables(int64_t n, const int32_t *rank, const int32_t *itemsize, const int64_t *shape,
                       const int64_t *stride, int64_t *bytes, uint8_t *cont, void *stream) {
@@ -3076,25 +2979,6 @@ int apc_cost_objective(int64_t n_vars, int64_t n_groups, const int64_t *group_va
   return check_launch("apc_cost_objective");
 }
 
-int apc_validate_row_minima_host(int64_t n_edges, const int32_t *edge_n_src, const int32_t *edge_n_tgt, int64_t n_tiles,
-                                 const apc_tile *tiles) {
-  if (n_edges < 0 || n_tiles < 0) return fail(-1, "apc_validate_row_minima_host: negative count");
-  if ((n_edges > 0 && (!edge_n_src || !edge_n_tgt)) || (n_tiles > 0 && !tiles))
-    return fail(-1, "apc_validate_row_minima_host: NULL array");
-  for (int64_t e = 0; e < n_edges; ++e)
-    if (edge_n_tgt[e] > 0 && (edge_n_src[e] < 1 || edge_n_src[e] > APC_TILE_MAX_COLS))
-      return fail(-2, "edge %lld: %d producer strategies; row minima inside the table launch need 1 .. %d", (long long)e,
-                  edge_n_src[e], APC_TILE_MAX_COLS);
-  for (int64_t t = 0; t < n_tiles; ++t) {
-    const apc_tile &tl = tiles[t];
-    if (tl.edge < 0 || tl.edge >= n_edges) return fail(-2, "tile %lld: edge %d out of range", (long long)t, tl.edge);
-    if (tl.col_begin != 0 || (tl.counts >> 16) != edge_n_src[tl.edge])
-      return fail(-2, "tile %lld: columns [%d, +%d) are not the whole rows of edge %d (%d columns)", (long long)t,
-                  tl.col_begin, tl.counts >> 16, tl.edge, edge_n_src[tl.edge]);
-  }
-  return 0;
-}
-
 int apc_diffusion_sweeps(int32_t n_sweeps, int32_t n_colors, const int64_t *color_begin_host, const int32_t *color_nodes,
                          int64_t n_classes, const int64_t *label_begin, const int64_t *inc_begin, const int32_t *inc_edge,
                          const uint8_t *inc_side, const int64_t *edge_begin, const int32_t *edge_i, const int32_t *edge_j,
@@ -3194,82 +3078,13 @@ int apc_redistribute_tables_static(const apc_params *params, int64_t n_tensors, 
 }  // extern "C"
 
 // ------------------------------------------------------------------------------------------
-// Packed tiles: host-side check and launch.
+// Packed tiles: launch.
 // ------------------------------------------------------------------------------------------
 static_assert(sizeof(apc_packed_tile) == 2752 && sizeof(apc_packed_tile) % 64 == 0, "apc_packed_tile layout");
 static_assert(offsetof(apc_packed_tile, entry_begin) == 32 && offsetof(apc_packed_tile, tensor_shape) == 64,
               "the header is the record's first 64 bytes");
 
 extern "C" {
-
-int apc_validate_packed_tiles_host(int64_t n_tensors, const int32_t *tensor_rank, const int32_t *tensor_itemsize,
-                                   const int64_t *tensor_shape, const int64_t *tensor_stride, int64_t n_specs,
-                                   const uint32_t *spec_codes, const int32_t *spec_tensor, int64_t n_strategies,
-                                   const int64_t *flops, const int64_t *rw_bytes, const int8_t *dtype_code,
-                                   const uint8_t *zero_cost, const int32_t *num_args, int64_t n_edges,
-                                   const int64_t *edge_row_begin, int64_t n_tiles, const apc_tile *tiles, int64_t n_dups,
-                                   const int64_t *dup_entry_begin, const int64_t *dup_row_begin,
-                                   const apc_packed_tile *packed) {
-  if (n_tiles < 0 || n_tensors < 0 || n_specs < 0 || n_strategies < 0 || n_edges < 0 || n_dups < 0)
-    return fail(-1, "apc_validate_packed_tiles_host: negative count");
-  if (n_tiles == 0) return 0;
-  if (!tiles || !packed || !spec_codes || !spec_tensor || !edge_row_begin || !flops || !rw_bytes || !dtype_code || !zero_cost ||
-      !num_args || (n_dups > 0 && (!dup_entry_begin || !dup_row_begin)) ||
-      (n_tensors > 0 && (!tensor_rank || !tensor_itemsize || !tensor_shape || !tensor_stride)))
-    return fail(-1, "apc_validate_packed_tiles_host: NULL array");
-  for (int64_t t = 0; t < n_tiles; ++t) {
-    const apc_tile &tl = tiles[t];
-    const apc_packed_tile &pk = packed[t];
-    const int rows = tl.counts & 0xFFFF, cols = tl.counts >> 16;
-    if (tl.edge < 0 || tl.edge >= n_edges) return fail(-2, "tile %lld: edge %d out of range", (long long)t, tl.edge);
-    if (tl.col_begin != 0 || cols != tl.n_src || cols < 1 || cols > APC_TILE_MAX_COLS || rows < 1 || rows > APC_TILE_MAX_ROWS)
-      return fail(-2, "tile %lld: a packed tile holds 1 .. %d whole rows of at most %d columns (%d rows, columns [%d, +%d) of %d)",
-                  (long long)t, APC_TILE_MAX_ROWS, APC_TILE_MAX_COLS, rows, tl.col_begin, cols, tl.n_src);
-    if (tl.dup_count < 0 || tl.dup_count > APC_PACKED_MAX_DUPS || tl.dup_begin < 0 || (int64_t)tl.dup_begin + tl.dup_count > n_dups)
-      return fail(-2, "tile %lld: %d identical edges, a packed tile serves at most %d", (long long)t, tl.dup_count,
-                  APC_PACKED_MAX_DUPS);
-    if (tl.src_begin < 0 || (int64_t)tl.src_begin + cols > n_specs || tl.tgt_begin < 0 ||
-        (int64_t)tl.tgt_begin + tl.row_begin + rows > n_specs || tl.strat_begin < 0 ||
-        (int64_t)tl.strat_begin + tl.row_begin + rows > n_strategies)
-      return fail(-2, "tile %lld: spec or strategy rows outside their tables", (long long)t);
-    const int64_t first = (int64_t)tl.row_begin * cols;
-    bool mixed = false;
-    for (int j = 0; j < cols; ++j) {
-      const int64_t sp = (int64_t)tl.src_begin + j;
-      if (pk.col_codes[j] != spec_codes[sp] || pk.col_tensor[j] != spec_tensor[sp])
-        return fail(-2, "packed tile %lld: producer spec %d differs from the spec table", (long long)t, j);
-      mixed |= spec_tensor[sp] < 0 || spec_tensor[sp] != tl.tensor;
-    }
-    for (int j = 0; j < rows; ++j) {
-      const int64_t ts = (int64_t)tl.tgt_begin + tl.row_begin + j, sr = (int64_t)tl.strat_begin + tl.row_begin + j;
-      if (pk.row_codes[j] != spec_codes[ts] || pk.row_tensor[j] != spec_tensor[ts])
-        return fail(-2, "packed tile %lld: consumer spec %d differs from the spec table", (long long)t, j);
-      mixed |= spec_tensor[ts] < 0;
-      if (num_args[sr] < 1 || num_args[sr] > 0x7FFF)
-        return fail(-2, "packed tile %lld: num_args %d of consumer strategy %d does not fit its 15 bits", (long long)t,
-                    num_args[sr], j);
-      const int32_t meta = (int32_t)(uint8_t)dtype_code[sr] | ((int32_t)(zero_cost[sr] != 0) << 8) | (num_args[sr] << 16);
-      if (pk.row_flops[j] != flops[sr] || pk.row_rw_bytes[j] != rw_bytes[sr] || pk.row_meta[j] != meta)
-        return fail(-2, "packed tile %lld: consumer strategy %d differs from the strategy table", (long long)t, j);
-    }
-    if (pk.rows != rows || pk.cols != cols || pk.dup_count != tl.dup_count || pk.tensor != tl.tensor || pk.edge != tl.edge ||
-        pk.flags != (tl.flags | (mixed ? APC_PACKED_MIXED : 0)) || pk.entry_begin != tl.entry_begin + first ||
-        pk.row_begin != edge_row_begin[tl.edge] + tl.row_begin || pk.pt_begin != (tl.pt_begin < 0 ? -1 : tl.pt_begin + first))
-      return fail(-2, "packed tile %lld: header does not repeat the fields of tile record %lld", (long long)t, (long long)t);
-    if (tl.tensor >= 0) {
-      if (tl.tensor >= n_tensors) return fail(-2, "tile %lld: tensor %d out of range", (long long)t, tl.tensor);
-      if (pk.tensor_rank != tensor_rank[tl.tensor] || pk.tensor_itemsize != tensor_itemsize[tl.tensor] ||
-          memcmp(pk.tensor_shape, tensor_shape + (int64_t)tl.tensor * APC_MAX_RANK, sizeof(pk.tensor_shape)) != 0 ||
-          memcmp(pk.tensor_stride, tensor_stride + (int64_t)tl.tensor * APC_MAX_RANK, sizeof(pk.tensor_stride)) != 0)
-        return fail(-2, "packed tile %lld: tensor row differs from the tensor table", (long long)t);
-    }
-    for (int d = 0; d < tl.dup_count; ++d)
-      if (pk.dup_entry_begin[d] != dup_entry_begin[tl.dup_begin + d] + first ||
-          pk.dup_row_begin[d] != dup_row_begin[tl.dup_begin + d] + tl.row_begin)
-        return fail(-2, "packed tile %lld: identical edge %d differs from the duplicate lists", (long long)t, d);
-  }
-  return 0;
-}
 
 int apc_build_tables_packed(const apc_params *params, int64_t n_tensors, const int32_t *rank, const int32_t *itemsize,
                             const int64_t *shape, const int64_t *stride, int64_t *tensor_bytes, uint8_t *tensor_contiguous,

@@ -1,0 +1,14 @@
+// The library's error text (apc_last_error) and argument checks, shared by its translation units.
+#ifndef APCOST_ERROR_H
+#define APCOST_ERROR_H
+
+#include "apcost.h"
+
+namespace apc_internal {
+// Stores the formatted message for this thread and returns `code`.
+__attribute__((visibility("hidden"), format(printf, 2, 3))) int fail(int code, const char *fmt, ...);
+// The parameters' ranges and reciprocals.
+__attribute__((visibility("hidden"))) int check_params(const apc_params *p);
+}  // namespace apc_internal
+
+#endif

@@ -29,7 +29,6 @@ with v a variant id (0 = plain ``Shard``).
 
 from __future__ import annotations
 
-import ctypes
 from dataclasses import dataclass, fields
 from typing import Optional
 
@@ -266,43 +265,24 @@ class CostTables:
     def validate_row_minima(self) -> None:
         """Raises unless every matrix row lies inside one tile (the precondition of the
         ``apc_*_row_min`` entry points), through the library's host-side check."""
-        def p(a):
-            return a.ctypes.data_as(ctypes.c_void_p)
-
-        rc = _native.lib().apc_validate_row_minima_host(ctypes.c_int64(self.n_edges), p(self.edge_n_src), p(self.edge_n_tgt),
-                                                        ctypes.c_int64(self.n_tiles), p(self.tile_records))
-        _native.check(rc, "apc_validate_row_minima_host")
+        _native.host_call("apc_validate_row_minima_host", self.n_edges, self.edge_n_src, self.edge_n_tgt, self.n_tiles,
+                          self.tile_records)
 
     # ---- tiles -------------------------------------------------------------------------
-    def edge_signatures(self) -> list:
-        """One digest per edge over everything its matrix depends on: both spec lists
-        (codes and tensor rows), flags, the consumer strategies' compute-cost inputs and
-        the pass-through values.  Equal digests = bit-identical comm / transition / cost."""
-        import hashlib
-
-        sb, ns = self.edge_src_begin.astype(np.int64), self.edge_n_src.astype(np.int64)
-        tb, nt = self.edge_tgt_begin.astype(np.int64), self.edge_n_tgt.astype(np.int64)
-        st = self.edge_strat_begin.astype(np.int64)
-        codes, tensor = self.spec_codes, self.spec_tensor
-        strat = np.rec.fromarrays([self.strat_flops, self.strat_rw_bytes, self.strat_dtype, self.strat_zero_cost,
-                                   self.strat_num_args])
-        out = []
-        for e in range(self.n_edges):
-            h = hashlib.blake2b(digest_size=16)
-            h.update(np.array([ns[e], nt[e], self.edge_flags[e]], np.int64).tobytes())
-            h.update(codes[sb[e]:sb[e] + ns[e]].tobytes())
-            h.update(tensor[sb[e]:sb[e] + ns[e]].tobytes())
-            h.update(codes[tb[e]:tb[e] + nt[e]].tobytes())
-            h.update(tensor[tb[e]:tb[e] + nt[e]].tobytes())
-            h.update(strat[st[e]:st[e] + nt[e]].tobytes())
-            if self.edge_pt_begin[e] >= 0:
-                b = int(self.edge_pt_begin[e])
-                h.update(self.pt_values[b:b + int(ns[e] * nt[e])].tobytes())
-            out.append(h.digest())
-        return out
+    def edge_classes(self) -> np.ndarray:
+        """For every edge the first edge whose matrix depends on the same bytes: both spec lists
+        (codes and tensor rows), flags, the consumer strategies' compute-cost inputs and the
+        pass-through values.  Equal edges have bit-identical comm / transition / cost."""
+        first_same = np.empty(self.n_edges, np.int64)
+        _native.host_call(
+            "apc_edge_classes_host", self.n_specs, self.spec_codes, self.spec_tensor, self.n_strategies, self.strat_flops,
+            self.strat_rw_bytes, self.strat_dtype, self.strat_zero_cost, self.strat_num_args, self.n_edges, self.edge_src_begin,
+            self.edge_n_src, self.edge_tgt_begin, self.edge_n_tgt, self.edge_flags, self.edge_pt_begin, self.edge_strat_begin,
+            len(self.pt_values), self.pt_values, first_same)
+        return first_same
 
     def build_tiles(self, tile_entries: Optional[int] = None, dedupe: bool = False, max_copies: int = 16,
-                    signatures=None, rows_per_wavefront_pass: Optional[int] = None) -> None:
+                    rows_per_wavefront_pass: Optional[int] = None) -> None:
         """Cuts every edge matrix into rectangles of about ``tile_entries`` entries:
         whole rows when a row fits the LDS column budget, column chunks otherwise.  With
         ``dedupe`` only the first of every group of identical edges is tiled; its tiles
@@ -315,15 +295,20 @@ class CostTables:
         each walk ``64 // columns`` whole rows at a time cover in one pass (the packed-tile launch
         of a small table, whose slowest workgroup decides the launch; the automatic choice sets it
         to 4 for such a table)."""
+        classes = self.edge_classes() if dedupe and self.n_edges else None
+        canonical = np.empty(self.n_edges, np.int64)
+
+        def count(te, mc, rows):
+            return _native.host_counts("apc_count_tiles_host", self.n_edges, self.edge_n_src, self.edge_n_tgt, classes, te, mc, rows,
+                                       canonical)
+
         if tile_entries is None:
-            sigs = self.edge_signatures() if dedupe and self.n_edges else None
             te, mc = APC_TILE_MAX_ROWS * APC_TILE_MAX_COLS, int(max_copies)
             small = self.n_entries <= AUTO_SMALL_TABLE_ENTRIES
+            rows_per_wavefront_pass = 4 if small else None
             while True:
-                self.build_tiles(te, dedupe, mc, signatures=sigs, rows_per_wavefront_pass=4 if small else None)
-                n = self.n_tiles
-                if n == 0 or n >= AUTO_MIN_TILES or self.n_entries / n <= AUTO_MIN_STORED_PER_TILE \
-                        or self.n_entries <= AUTO_SMALL_TABLE_ENTRIES:
+                n, n_dups = count(te, mc, rows_per_wavefront_pass or 0)
+                if n == 0 or n >= AUTO_MIN_TILES or self.n_entries / n <= AUTO_MIN_STORED_PER_TILE or small:
                     break
                 if dedupe and mc > 4:
                     mc //= 2
@@ -335,88 +320,38 @@ class CostTables:
                     te //= 2
                 else:
                     break
-            return
-        self.tiling = {"tile_entries": int(tile_entries), "max_copies": int(max_copies) if dedupe else 1}
+        else:
+            te, mc = int(tile_entries), int(max_copies)
+            n, n_dups = count(te, mc, int(rows_per_wavefront_pass or 0))
+        self.tiling = {"tile_entries": te, "max_copies": mc if dedupe else 1}
         if rows_per_wavefront_pass:
             self.tiling["rows_per_wavefront_pass"] = int(rows_per_wavefront_pass)
-        ns = self.edge_n_src.astype(np.int64)
-        nt = self.edge_n_tgt.astype(np.int64)
-        canonical = np.arange(self.n_edges, dtype=np.int64)
-        if dedupe and self.n_edges:
-            first: dict = {}  # signature -> [canonical edge, copies it already serves]
-            for e, sig in enumerate(signatures if signatures is not None else self.edge_signatures()):
-                slot = first.get(sig)
-                if slot is None or slot[1] >= min(APC_TILE_MAX_DUPS, max(int(max_copies) - 1, 0)):
-                    first[sig] = [e, 0]  # a new canonical edge (also when the previous one is full)
-                else:
-                    canonical[e] = slot[0]
-                    slot[1] += 1
         self.edge_canonical = canonical
-        is_dup = canonical != np.arange(self.n_edges)
-        # duplicates grouped by canonical edge (stable: in edge order)
-        dup_edges = np.nonzero(is_dup)[0]
-        order = np.argsort(canonical[dup_edges], kind="stable")
-        dup_edges = dup_edges[order]
-        self.dup_entry_begin = _i64(self.edge_entry_begin[:-1][dup_edges]) if self.n_edges else _i64([])
-        self.dup_row_begin = _i64(self.edge_row_begin()[dup_edges]) if self.n_edges else _i64([])
-        self.edge_dup_count = np.bincount(canonical[dup_edges], minlength=self.n_edges).astype(np.int64)
-        self.edge_dup_begin = np.cumsum(self.edge_dup_count) - self.edge_dup_count
-        live = (ns > 0) & (nt > 0) & ~is_dup
-        ns1 = np.maximum(ns, 1)
-        nt1 = np.maximum(nt, 1)
-        ncc = -(-ns1 // APC_TILE_MAX_COLS)  # column chunks per edge
-        cw = -(-ns1 // ncc)  # chunk width
-        rpt = np.clip(tile_entries // cw, 1, APC_TILE_MAX_ROWS)
-        if rows_per_wavefront_pass:
-            rpt = np.where(ncc == 1, np.minimum(rpt, int(rows_per_wavefront_pass) * np.maximum(64 // cw, 1)), rpt)
-        nrt = -(-nt1 // rpt)  # row tiles per edge
-        rpt = -(-nt1 // nrt)  # balanced rows per tile
-        per_edge = np.where(live, ncc * nrt, 0)
-        total = int(per_edge.sum())
-        te = np.repeat(np.arange(self.n_edges, dtype=np.int64), per_edge)
-        first_tile = np.cumsum(per_edge) - per_edge
-        k = np.arange(total, dtype=np.int64) - np.repeat(first_tile, per_edge)
-        ci = k % ncc[te]
-        ri = k // ncc[te]
-        col_begin = ci * cw[te]
-        row_begin = ri * rpt[te]
-        self.tile_edge = _i32(te)
-        self.tile_col_begin = _i32(col_begin)
-        self.tile_col_count = _i32(np.minimum(cw[te], ns[te] - col_begin))
-        self.tile_row_begin = _i32(row_begin)
-        self.tile_row_count = _i32(np.minimum(rpt[te], nt[te] - row_begin))
+        self.edge_dup_begin, self.edge_dup_count = np.empty(self.n_edges, np.int64), np.empty(self.n_edges, np.int64)
+        self.dup_entry_begin, self.dup_row_begin = np.empty(n_dups, np.int64), np.empty(n_dups, np.int64)
+        self.tile_edge, self.tile_row_begin, self.tile_row_count, self.tile_col_begin, self.tile_col_count = (
+            np.empty(n, np.int32) for _ in range(5))
+        _native.host_call(
+            "apc_fill_tiles_host", self.n_edges, self.edge_n_src, self.edge_n_tgt, self.edge_entry_begin, canonical, te,
+            int(rows_per_wavefront_pass or 0), n, n_dups, self.edge_dup_begin, self.edge_dup_count, self.dup_entry_begin,
+            self.dup_row_begin, self.tile_edge, self.tile_row_begin, self.tile_row_count, self.tile_col_begin, self.tile_col_count)
         self.pack_tile_records()
 
     def pack_tile_records(self) -> None:
         """The tile rectangles plus the fields of their edge, as the packed records the
         table kernel reads (C struct ``apc_tile``)."""
-        te = self.tile_edge.astype(np.int64)
         if self.edge_canonical is None or len(self.edge_canonical) != self.n_edges:
             self.edge_canonical = np.arange(self.n_edges, dtype=np.int64)
             self.dup_entry_begin = _i64([])
             self.dup_row_begin = _i64([])
             self.edge_dup_count = np.zeros(self.n_edges, np.int64)
             self.edge_dup_begin = np.zeros(self.n_edges, np.int64)
-        rec = np.zeros(len(te), TILE_DTYPE)
-        inside = (te >= 0) & (te < self.n_edges)
-        tc = np.where(inside, te, 0)  # (out-of-range tiles are reported by validate())
-        rec["edge"] = self.tile_edge
-        rec["row_begin"], rec["col_begin"] = self.tile_row_begin, self.tile_col_begin
-        rec["counts"] = (self.tile_row_count.astype(np.int64) & 0xFFFF) | ((self.tile_col_count.astype(np.int64) & 0x7FFF) << 16)
-        if len(te) and self.n_edges:
-            rec["src_begin"] = self.edge_src_begin[tc]
-            rec["n_src"] = self.edge_n_src[tc]
-            rec["tgt_begin"] = self.edge_tgt_begin[tc]
-            rec["flags"] = self.edge_flags[tc]
-            rec["strat_begin"] = self.edge_strat_begin[tc]
-            rec["entry_begin"] = self.edge_entry_begin[:-1][tc]
-            rec["pt_begin"] = self.edge_pt_begin[tc]
-            rec["dup_begin"] = self.edge_dup_begin[tc]
-            rec["dup_count"] = self.edge_dup_count[tc]
-        if len(te) and self.n_specs and self.n_edges:
-            # (indices are clipped here; validate() reports ranges that fall outside the table)
-            first = np.clip(self.edge_src_begin[tc].astype(np.int64) + self.tile_col_begin, 0, self.n_specs - 1)
-            rec["tensor"] = self.spec_tensor[first]
+        rec = np.empty(self.n_tiles, TILE_DTYPE)
+        _native.host_call(
+            "apc_tile_records_host", self.n_specs, self.spec_tensor, self.n_edges, self.edge_src_begin, self.edge_n_src,
+            self.edge_tgt_begin, self.edge_flags, self.edge_pt_begin, self.edge_entry_begin, self.edge_strat_begin,
+            self.edge_dup_begin, self.edge_dup_count, self.n_tiles, self.tile_edge, self.tile_row_begin, self.tile_row_count,
+            self.tile_col_begin, self.tile_col_count, rec)
         self.tile_records = rec
 
     # ---- packed tiles ------------------------------------------------------------------
@@ -438,72 +373,21 @@ class CostTables:
         if not self.packable():
             raise RuntimeError("packed tiles need whole rows in every tile and at most "
                                f"{APC_PACKED_MAX_DUPS} identical edges per tile")
-        rec = self.tile_records
-        n = len(rec)
-        pk = np.zeros(n, PACKED_TILE_DTYPE)
-        rows = (rec["counts"] & 0xFFFF).astype(np.int64)
-        cols = (rec["counts"] >> 16).astype(np.int64)
-        rb = rec["row_begin"].astype(np.int64)
-        edge = rec["edge"].astype(np.int64)
-        first = rb * cols
-        pk["rows"], pk["cols"], pk["dup_count"], pk["tensor"], pk["edge"] = rows, cols, rec["dup_count"], rec["tensor"], rec["edge"]
-        pk["entry_begin"] = rec["entry_begin"] + first
-        pk["row_begin"] = self.edge_row_begin()[edge] + rb
-        pk["pt_begin"] = np.where(rec["pt_begin"] < 0, -1, rec["pt_begin"] + first)
-        t = rec["tensor"].astype(np.int64)
-        has = t >= 0
-        tc = np.where(has, t, 0)
-        if self.n_tensors:
-            pk["tensor_rank"] = np.where(has, self.tensor_rank[tc], 0)
-            pk["tensor_itemsize"] = np.where(has, self.tensor_itemsize[tc], 0)
-            pk["tensor_shape"] = np.where(has[:, None], self.tensor_shape[tc], 0)
-            pk["tensor_stride"] = np.where(has[:, None], self.tensor_stride[tc], 0)
-        j = np.arange(APC_TILE_MAX_COLS, dtype=np.int64)[None, :]
-        # producer specs
-        live = j < cols[:, None]
-        sp = np.where(live, rec["src_begin"].astype(np.int64)[:, None] + j, 0)
-        pk["col_codes"] = np.where(live, self.spec_codes[sp], 0)
-        col_tensor = np.where(live, self.spec_tensor[sp], 0)
-        pk["col_tensor"] = col_tensor
-        mixed = (live & ((col_tensor < 0) | (col_tensor != rec["tensor"][:, None]))).any(axis=1)
-        # consumer specs and their strategies
-        live = j < rows[:, None]
-        ts = np.where(live, (rec["tgt_begin"].astype(np.int64) + rb)[:, None] + j, 0)
-        pk["row_codes"] = np.where(live, self.spec_codes[ts], 0)
-        row_tensor = np.where(live, self.spec_tensor[ts], 0)
-        pk["row_tensor"] = row_tensor
-        mixed |= (live & (row_tensor < 0)).any(axis=1)
-        sr = np.where(live, (rec["strat_begin"].astype(np.int64) + rb)[:, None] + j, 0)
-        pk["row_flops"] = np.where(live, self.strat_flops[sr], 0)
-        pk["row_rw_bytes"] = np.where(live, self.strat_rw_bytes[sr], 0)
-        meta = (self.strat_dtype[sr].astype(np.int64) & 0xFF) | ((self.strat_zero_cost[sr] != 0).astype(np.int64) << 8) \
-            | (self.strat_num_args[sr].astype(np.int64) << 16)
-        pk["row_meta"] = np.where(live, meta, 0).astype(np.int32)
-        pk["flags"] = rec["flags"] | np.where(mixed, PACKED_MIXED, 0)
-        # identical edges
-        d = np.arange(APC_PACKED_MAX_DUPS, dtype=np.int64)[None, :]
-        live = d < rec["dup_count"].astype(np.int64)[:, None]
-        if len(self.dup_entry_begin):
-            at = np.where(live, rec["dup_begin"].astype(np.int64)[:, None] + d, 0)
-            pk["dup_entry_begin"] = np.where(live, self.dup_entry_begin[at] + first[:, None], 0)
-            pk["dup_row_begin"] = np.where(live, self.dup_row_begin[at] + rb[:, None], 0)
+        pk = np.empty(self.n_tiles, PACKED_TILE_DTYPE)
+        _native.host_call(
+            "apc_pack_tiles_host", self.n_tensors, self.tensor_rank, self.tensor_itemsize, self.tensor_shape, self.tensor_stride,
+            self.n_specs, self.spec_codes, self.spec_tensor, self.n_strategies, self.strat_flops, self.strat_rw_bytes,
+            self.strat_dtype, self.strat_zero_cost, self.strat_num_args, self.n_edges, self.edge_row_begin(), self.n_tiles,
+            self.tile_records, len(self.dup_entry_begin), self.dup_entry_begin, self.dup_row_begin, pk)
         return pk
 
     def validate_packed(self, packed: np.ndarray) -> None:
         """The packed records against the tables, through the library's host-side check."""
-        def p(a):
-            return np.ascontiguousarray(a).ctypes.data_as(ctypes.c_void_p)
-
-        keep = [np.ascontiguousarray(a) for a in (
-            self.tensor_rank, self.tensor_itemsize, self.tensor_shape, self.tensor_stride, self.spec_codes, self.spec_tensor,
-            self.strat_flops, self.strat_rw_bytes, self.strat_dtype, self.strat_zero_cost, self.strat_num_args,
-            self.edge_row_begin(), self.tile_records, self.dup_entry_begin, self.dup_row_begin, packed)]
-        (rank, item, shape, stride, codes, owner, flops, rw, dt, zero, nargs, erb, tiles, dups, dup_rows, pk) = keep
-        rc = _native.lib().apc_validate_packed_tiles_host(
-            ctypes.c_int64(self.n_tensors), p(rank), p(item), p(shape), p(stride), ctypes.c_int64(self.n_specs), p(codes), p(owner),
-            ctypes.c_int64(self.n_strategies), p(flops), p(rw), p(dt), p(zero), p(nargs), ctypes.c_int64(self.n_edges), p(erb),
-            ctypes.c_int64(self.n_tiles), p(tiles), ctypes.c_int64(len(dups)), p(dups), p(dup_rows), p(pk))
-        _native.check(rc, "apc_validate_packed_tiles_host")
+        _native.host_call(
+            "apc_validate_packed_tiles_host", self.n_tensors, self.tensor_rank, self.tensor_itemsize, self.tensor_shape,
+            self.tensor_stride, self.n_specs, self.spec_codes, self.spec_tensor, self.n_strategies, self.strat_flops,
+            self.strat_rw_bytes, self.strat_dtype, self.strat_zero_cost, self.strat_num_args, self.n_edges, self.edge_row_begin(),
+            self.n_tiles, self.tile_records, len(self.dup_entry_begin), self.dup_entry_begin, self.dup_row_begin, packed)
 
     # ---- checks ------------------------------------------------------------------------
     def validate(self, params) -> None:
@@ -522,44 +406,20 @@ class CostTables:
         for name in ("strat_rw_bytes", "strat_dtype", "strat_zero_cost", "strat_num_args"):
             if len(getattr(self, name)) != self.n_strategies:
                 raise RuntimeError(f"{name} must have n_strategies rows")
-        if self.n_strategies and int(self.strat_num_args.min()) < 1:
-            raise RuntimeError("strat_num_args must be >= 1")
-        if (self.strat_flops >= 2**53).any() or (self.strat_rw_bytes >= 2**53).any():
-            raise RuntimeError("flop / byte counts must stay below 2**53 to convert to fp64 exactly")
-        cp = params.to_c()
         if self.tile_records is None or len(self.tile_records) != self.n_tiles:
             raise RuntimeError("tile_records must have one record per tile (call pack_tile_records())")
-
-        def p(a):
-            return a.ctypes.data_as(ctypes.c_void_p)
-
-        rc = _native.lib().apc_validate_tables_host(
-            ctypes.byref(cp), ctypes.c_int64(self.n_tensors), p(self.tensor_rank),
-            ctypes.c_int64(self.n_specs), p(self.spec_codes), p(self.spec_tensor),
-            ctypes.c_int64(self.n_edges), p(self.edge_src_begin), p(self.edge_n_src), p(self.edge_tgt_begin),
-            p(self.edge_n_tgt), p(self.edge_flags), p(self.edge_pt_begin), p(self.edge_entry_begin),
-            p(self.edge_strat_begin), ctypes.c_int64(len(self.pt_values)), ctypes.c_int64(self.n_strategies),
-            ctypes.c_int64(self.n_tiles), p(self.tile_records), ctypes.c_int64(len(self.dup_entry_begin)),
-            p(self.dup_entry_begin))
-        _native.check(rc, "apc_validate_tables_host")
-        # every edge is either tiled completely or a duplicate of an edge that is
-        area = np.zeros(self.n_edges, np.int64)
-        np.add.at(area, self.tile_edge.astype(np.int64),
-                  self.tile_row_count.astype(np.int64) * self.tile_col_count.astype(np.int64))
-        want = self.edge_n_src.astype(np.int64) * self.edge_n_tgt.astype(np.int64)
-        tiled = self.edge_canonical == np.arange(self.n_edges)
-        if not np.array_equal(area[tiled], want[tiled]) or area[~tiled].any():
-            raise RuntimeError("tiles do not cover every (non-duplicate) edge matrix exactly once")
-        if int(self.edge_dup_count.sum()) != int((~tiled).sum()) or len(self.dup_entry_begin) != int((~tiled).sum()):
-            raise RuntimeError("duplicate-edge lists do not account for every de-duplicated edge")
-        # byte counts must convert to fp64 exactly (the kernels divide them as doubles)
-        if self.n_tensors:
-            r = np.arange(APC_MAX_RANK)[None, :] < self.tensor_rank[:, None]
-            if (np.where(r, self.tensor_shape, 0) < 0).any():
-                raise RuntimeError("tensor sizes must not be negative")
-            numel = np.where(r, self.tensor_shape, 1).astype(object).prod(axis=1)
-            if (numel * self.tensor_itemsize.astype(object) >= 2**53).any():
-                raise RuntimeError("tensor byte counts must stay below 2**53")
+        _native.host_call(
+            "apc_validate_tables_host", params.to_c(), self.n_tensors, self.tensor_rank, self.n_specs, self.spec_codes,
+            self.spec_tensor, self.n_edges, self.edge_src_begin, self.edge_n_src, self.edge_tgt_begin, self.edge_n_tgt,
+            self.edge_flags, self.edge_pt_begin, self.edge_entry_begin, self.edge_strat_begin, len(self.pt_values),
+            self.n_strategies, self.n_tiles, self.tile_records, len(self.dup_entry_begin), self.dup_entry_begin)
+        # what the device cannot check: every edge is tiled completely or a duplicate of an edge that is; flop and
+        # byte counts convert to fp64 exactly (the kernels divide them as doubles)
+        _native.host_call(
+            "apc_validate_tiling_host", self.n_tensors, self.tensor_rank, self.tensor_itemsize, self.tensor_shape,
+            self.n_strategies, self.strat_flops, self.strat_rw_bytes, self.strat_num_args, self.n_edges, self.edge_n_src,
+            self.edge_n_tgt, self.edge_canonical, self.edge_dup_count, len(self.dup_entry_begin), self.n_tiles, self.tile_edge,
+            self.tile_row_count, self.tile_col_count)
 
     def as_dict(self) -> dict:
         """Plain-data view (numpy arrays) of every table."""

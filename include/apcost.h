@@ -138,6 +138,51 @@ int apc_validate_tables_host(const apc_params *params, int64_t n_tensors, const 
                              int64_t n_pt, int64_t n_strategies, int64_t n_tiles, const apc_tile *tiles_host,
                              int64_t n_dups, const int64_t *dup_entry_begin_host);
 
+/* Which edges have the same matrix (HOST pointers): first_same[e] = the first edge whose spec lists
+ * (codes and tensor rows), flags, consumer strategies' rows of the strategy table and pass-through
+ * values equal those of edge e byte for byte, e itself when there is none before it.  Equal edges
+ * have bit-identical comm / transition / cost.  An edge whose ranges leave the tables stands for
+ * itself (apc_validate_tables_host reports it).  No counterpart in the reference. */
+int apc_edge_classes_host(int64_t n_specs, const uint32_t *spec_codes_host, const int32_t *spec_tensor_host, int64_t n_strategies,
+                          const int64_t *flops_host, const int64_t *rw_bytes_host, const int8_t *dtype_code_host,
+                          const uint8_t *zero_cost_host, const int32_t *num_args_host, int64_t n_edges,
+                          const int32_t *edge_src_begin_host, const int32_t *edge_n_src_host, const int32_t *edge_tgt_begin_host,
+                          const int32_t *edge_n_tgt_host, const int32_t *edge_flags_host, const int64_t *edge_pt_begin_host,
+                          const int32_t *edge_strat_begin_host, int64_t n_pt, const double *pt_values_host, int64_t *first_same_host);
+
+/* The tiling of a table (HOST pointers).  apc_count_tiles_host decides which edges are tiled
+ * (edge_canonical[e] = e) and which are duplicates of an earlier tiled edge (first_same: the classes
+ * of apc_edge_classes_host, NULL: every edge is tiled; one tiled edge serves at most max_copies - 1
+ * and at most APC_TILE_MAX_DUPS others) and counts the tiles: about tile_entries entries each, whole
+ * rows while a row fits APC_TILE_MAX_COLS, column chunks of equal width otherwise, rows balanced over
+ * the tiles of an edge; with rows_per_wavefront_pass = w > 0 a tile of whole rows holds at most
+ * w * (64 / columns) of them.  apc_fill_tiles_host writes the tiles and the duplicate lists for the
+ * same arguments, apc_tile_records_host the records the kernels read.  apc_validate_tiling_host
+ * checks what apc_validate_tables_host does not: every edge covered once or a duplicate, num_args >= 1,
+ * and flop, byte and tensor byte counts below 2^53.  No counterpart in the reference. */
+int apc_count_tiles_host(int64_t n_edges, const int32_t *edge_n_src_host, const int32_t *edge_n_tgt_host,
+                         const int64_t *first_same_host, int64_t tile_entries, int64_t max_copies, int64_t rows_per_wavefront_pass,
+                         int64_t *edge_canonical_host, int64_t *n_tiles, int64_t *n_duplicates);
+int apc_fill_tiles_host(int64_t n_edges, const int32_t *edge_n_src_host, const int32_t *edge_n_tgt_host,
+                        const int64_t *edge_entry_begin_host, const int64_t *edge_canonical_host, int64_t tile_entries,
+                        int64_t rows_per_wavefront_pass, int64_t n_tiles, int64_t n_duplicates, int64_t *edge_dup_begin_host,
+                        int64_t *edge_dup_count_host, int64_t *dup_entry_begin_host, int64_t *dup_row_begin_host,
+                        int32_t *tile_edge_host, int32_t *tile_row_begin_host, int32_t *tile_row_count_host,
+                        int32_t *tile_col_begin_host, int32_t *tile_col_count_host);
+int apc_tile_records_host(int64_t n_specs, const int32_t *spec_tensor_host, int64_t n_edges, const int32_t *edge_src_begin_host,
+                          const int32_t *edge_n_src_host, const int32_t *edge_tgt_begin_host, const int32_t *edge_flags_host,
+                          const int64_t *edge_pt_begin_host, const int64_t *edge_entry_begin_host,
+                          const int32_t *edge_strat_begin_host, const int64_t *edge_dup_begin_host,
+                          const int64_t *edge_dup_count_host, int64_t n_tiles, const int32_t *tile_edge_host,
+                          const int32_t *tile_row_begin_host, const int32_t *tile_row_count_host,
+                          const int32_t *tile_col_begin_host, const int32_t *tile_col_count_host, apc_tile *records_host);
+int apc_validate_tiling_host(int64_t n_tensors, const int32_t *tensor_rank_host, const int32_t *tensor_itemsize_host,
+                             const int64_t *tensor_shape_host, int64_t n_strategies, const int64_t *flops_host,
+                             const int64_t *rw_bytes_host, const int32_t *num_args_host, int64_t n_edges,
+                             const int32_t *edge_n_src_host, const int32_t *edge_n_tgt_host, const int64_t *edge_canonical_host,
+                             const int64_t *edge_dup_count_host, int64_t n_duplicates, int64_t n_tiles, const int32_t *tile_edge_host,
+                             const int32_t *tile_row_count_host, const int32_t *tile_col_count_host);
+
 /* Bytes and contiguity of every tensor row.
  * Replaces torch spec_to_bytes (distributed/tensor/_collective_utils.py:230-232) and
  * check_contiguous_sizes_strides (_prims_common/__init__.py:252-292) as called from
@@ -437,6 +482,16 @@ int apc_validate_packed_tiles_host(int64_t n_tensors, const int32_t *tensor_rank
                                    const int64_t *edge_row_begin_host, int64_t n_tiles, const apc_tile *tiles_host,
                                    int64_t n_dups, const int64_t *dup_entry_begin_host, const int64_t *dup_row_begin_host,
                                    const apc_packed_tile *packed_host);
+
+/* Writes the packed records of the tiles (HOST pointers; packed_host [n_tiles]): what
+ * apc_validate_packed_tiles_host checks.  A tile that names rows outside the tables is an error. */
+int apc_pack_tiles_host(int64_t n_tensors, const int32_t *tensor_rank_host, const int32_t *tensor_itemsize_host,
+                        const int64_t *tensor_shape_host, const int64_t *tensor_stride_host, int64_t n_specs,
+                        const uint32_t *spec_codes_host, const int32_t *spec_tensor_host, int64_t n_strategies,
+                        const int64_t *flops_host, const int64_t *rw_bytes_host, const int8_t *dtype_code_host,
+                        const uint8_t *zero_cost_host, const int32_t *num_args_host, int64_t n_edges,
+                        const int64_t *edge_row_begin_host, int64_t n_tiles, const apc_tile *tiles_host, int64_t n_dups,
+                        const int64_t *dup_entry_begin_host, const int64_t *dup_row_begin_host, apc_packed_tile *packed_host);
 
 /* The table pass of a planner over packed tiles, ONE launch: the tensor table, the compute costs,
  * the assembled cost of every entry and the row minima (what apc_build_tables_row_min writes with

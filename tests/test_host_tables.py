@@ -1,0 +1,105 @@
+"""The library's host-side table passes (identical edges, tilings, packed records, transfers)
+against plain restatements of what they are: CPU except where marked."""
+
+import numpy as np
+import pytest
+
+from autoparallel_amd import CostModelParams
+from autoparallel_amd._native import APC_TILE_MAX_COLS, APC_TILE_MAX_DUPS, APC_TILE_MAX_ROWS
+from autoparallel_amd.synthetic import stress_dag
+from test_abi_and_encoding import twin_graph
+
+
+def _content(tb, e):
+    """Everything edge e's matrix depends on, as bytes."""
+    ns, nt, sb, tg, st = (int(a[e]) for a in (tb.edge_n_src, tb.edge_n_tgt, tb.edge_src_begin, tb.edge_tgt_begin, tb.edge_strat_begin))
+    parts = [np.int64([ns, nt, tb.edge_flags[e], tb.edge_pt_begin[e] >= 0])]
+    parts += [a[sb:sb + ns] for a in (tb.spec_codes, tb.spec_tensor)] + [a[tg:tg + nt] for a in (tb.spec_codes, tb.spec_tensor)]
+    parts += [a[st:st + nt] for a in (tb.strat_flops, tb.strat_rw_bytes, tb.strat_dtype, tb.strat_zero_cost, tb.strat_num_args)]
+    if tb.edge_pt_begin[e] >= 0:
+        b = int(tb.edge_pt_begin[e])
+        parts.append(tb.pt_values[b:b + ns * nt])
+    return b"|".join(p.tobytes() for p in parts)
+
+
+@pytest.mark.parametrize("seed,nodes,hi", [(0, 1, 2), (1, 40, 3), (2, 300, 24), (3, 60, 100)])
+def test_edge_classes_are_the_edges_of_equal_content(seed, nodes, hi):
+    tb = twin_graph(stress_dag(seed=seed, n_nodes=nodes, mesh_sizes=(4, 2), min_strategies=1, max_strategies=hi))
+    rng = np.random.default_rng(seed)
+    for e in rng.integers(0, tb.n_edges, tb.n_edges // 4):  # some twins differ in one value each, in any part
+        which = rng.integers(0, 4)
+        if which == 0:
+            tb.spec_tensor[tb.edge_tgt_begin[e]] = -1
+        elif which == 1:
+            tb.strat_rw_bytes[tb.edge_strat_begin[e] + tb.edge_n_tgt[e] - 1] += 1
+        elif which == 2:
+            tb.edge_flags[e] ^= 1
+        elif tb.edge_pt_begin[e] >= 0:
+            tb.pt_values[tb.edge_pt_begin[e]] = np.inf
+    first, want = {}, []
+    for e in range(tb.n_edges):
+        want.append(first.setdefault(_content(tb, e), e))
+    assert np.array_equal(tb.edge_classes(), want)
+
+
+@pytest.mark.parametrize("te,copies,rows", [(1, 2, None), (64, 1, None), (300, 5, 3), (4096, 16, 4), (4096, 100, None)])
+@pytest.mark.parametrize("hi", [3, 64, 65, 130])
+def test_tilings_follow_their_definition(te, copies, rows, hi):
+    tb = twin_graph(twin_graph(stress_dag(seed=hi, n_nodes=30, mesh_sizes=(4, 2), min_strategies=1, max_strategies=hi)))
+    tb.build_tiles(te, dedupe=True, max_copies=copies, rows_per_wavefront_pass=rows)
+    tb.validate(CostModelParams.from_mesh((4, 2)))
+    # duplicates: each class of equal edges in runs of one tiled edge and at most copies - 1 others
+    room = min(APC_TILE_MAX_DUPS, max(copies - 1, 0))
+    open_edge, want = {}, []
+    for e, f in enumerate(tb.edge_classes().tolist()):
+        c, n = open_edge.get(f, (e, room))
+        c, n = (e, 0) if n >= room else (c, n + 1)
+        open_edge[f] = (c, n)
+        want.append(c)
+    assert np.array_equal(tb.edge_canonical, want)
+    row_begin = tb.edge_row_begin()
+    tiles = []
+    for e in range(tb.n_edges):
+        ns, nt = int(tb.edge_n_src[e]), int(tb.edge_n_tgt[e])
+        dups = [d for d in range(tb.n_edges) if want[d] == e and d != e]
+        at = slice(int(tb.edge_dup_begin[e]), int(tb.edge_dup_begin[e] + tb.edge_dup_count[e]))
+        assert np.array_equal(tb.dup_entry_begin[at], tb.edge_entry_begin[dups]) and np.array_equal(tb.dup_row_begin[at], row_begin[dups])
+        if want[e] != e or ns == 0 or nt == 0:
+            continue
+        chunks = -(-ns // APC_TILE_MAX_COLS)
+        width = -(-ns // chunks)
+        most = min(max(te // width, 1), APC_TILE_MAX_ROWS)
+        if rows and chunks == 1:
+            most = min(most, rows * max(64 // width, 1))
+        n = -(-nt // most)
+        per = -(-nt // n)
+        tiles += [(e, r * per, min(per, nt - r * per), c * width, min(width, ns - c * width)) for r in range(n) for c in range(chunks)]
+    got = np.stack([tb.tile_edge, tb.tile_row_begin, tb.tile_row_count, tb.tile_col_begin, tb.tile_col_count], 1)
+    assert np.array_equal(got, np.asarray(tiles).reshape(-1, 5))
+
+
+def test_packed_records_repeat_the_tables():
+    tb = twin_graph(stress_dag(seed=4, n_nodes=200, mesh_sizes=(4, 2), min_strategies=1, max_strategies=40, frac_nonspec_nodes=0.1))
+    tb.build_tiles(None, dedupe=True)
+    tb.validate_packed(tb.pack_tiles())  # (the validator compares field by field)
+    tb.tile_records["strat_begin"][3] = tb.n_strategies
+    with pytest.raises(RuntimeError, match="tile 3: rows outside the tables"):
+        tb.pack_tiles()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [[0], [1, 0, 3], [4 << 20], [(4 << 20) + 1, 255, 0, 257], [1, 40 << 20, 7, 9 << 20]])
+def test_transfers_bring_back_the_bytes(gpu_device, sizes):
+    """Sizes around the pinned chunk (4 MiB) and beyond the chunks in flight."""
+    import torch
+
+    from autoparallel_amd import _native
+
+    ops = _native.torch_ops()
+    host = [torch.randint(0, 256, (n,), dtype=torch.uint8) for n in sizes] + [torch.arange(5, dtype=torch.float64).reshape(5, 1)]
+    dev = ops.upload(host, gpu_device)
+    back = ops.download(dev)
+    for h, d, b in zip(host, dev, back):
+        assert d.is_cuda and d.shape == h.shape and d.dtype == h.dtype and torch.equal(b, h)
+        assert d.numel() == 0 or d.data_ptr() % 256 == 0
+    assert ops.upload([], gpu_device) == [] and ops.download([]) == []
