@@ -10,39 +10,82 @@ per-thread state) is carried over, so "the current stream" keeps meaning the cal
 
 Calls are serialised (one worker), nested calls run in place, exceptions come back to the
 caller unchanged.
+
+A call costs its two hand-overs between the threads: a queue of the interpreter's own (no Python
+code between put and get) one way, a lock the caller waits on the other.  (With an executor's
+futures, and the stream context entered for every call, 40 us a call; so 15.)
 """
 
 from __future__ import annotations
 
+import _thread
 import functools
 import os
+import queue
 import threading
-from concurrent.futures import ThreadPoolExecutor
+from concurrent.futures import Future
 
 _lock = threading.Lock()
-_pool: ThreadPoolExecutor | None = None
+_tasks: queue.SimpleQueue | None = None
 _worker_ident: int | None = None
 
 
-def _remember_ident():
+class _Call:
+    """One call: what to run, the caller's stream, and the outcome."""
+
+    __slots__ = ("fn", "args", "kwargs", "stream", "done", "result", "error")
+
+    def __init__(self, fn, args, kwargs, stream):
+        self.fn, self.args, self.kwargs, self.stream = fn, args, kwargs, stream
+        self.result = self.error = None
+        self.done = _thread.allocate_lock()
+        self.done.acquire()
+
+    def run(self):
+        try:
+            self.result = self.fn(*self.args, **self.kwargs)
+        except BaseException as e:  # noqa: BLE001 (raised again in the caller)
+            self.error = e
+        self.done.release()
+
+
+def _work(tasks):
     global _worker_ident
     _worker_ident = threading.get_ident()
+    current = None  # the stream this thread stands on; None: its own default
+    while True:
+        task = tasks.get()
+        if task.stream is not None and (current is None or task.stream != current):
+            import torch
+
+            torch.cuda.set_stream(task.stream)  # (sets the stream's device as well)
+            current = task.stream
+        elif task.stream is None and current is not None:
+            import torch
+
+            torch.cuda.set_stream(torch.cuda.default_stream(current.device))
+            current = None
+        task.run()
+        del task  # (nothing of a call outlives it here)
 
 
-def _executor() -> ThreadPoolExecutor:
-    global _pool
-    with _lock:
-        if _pool is None:
-            _pool = ThreadPoolExecutor(max_workers=1, thread_name_prefix="apcost-device",
-                                       initializer=_remember_ident)
-        return _pool
+def _queue() -> queue.SimpleQueue:
+    global _tasks
+    if _tasks is None:
+        with _lock:
+            if _tasks is None:
+                tasks = queue.SimpleQueue()
+                threading.Thread(target=_work, args=(tasks,), name="apcost-device_0", daemon=True).start()
+                _tasks = tasks
+    return _tasks
 
 
 def _forget_thread():
-    # a forked child has the parent's pool object but none of its threads
-    global _pool, _worker_ident
-    _pool = None
+    # a forked child has the parent's queue but not its thread
+    global _tasks, _worker_ident, _lock
+    _tasks = None
     _worker_ident = None
+    _lock = threading.Lock()
 
 
 os.register_at_fork(after_in_child=_forget_thread)
@@ -72,23 +115,30 @@ def call(fn, *args, **kwargs):
     work there needs a parent that had not initialised the GPU before the fork."""
     if threading.get_ident() == _worker_ident:
         return fn(*args, **kwargs)
-    import torch
-
-    stream = _callers_stream()
-
-    def task():
-        if stream is None:
-            return fn(*args, **kwargs)
-        with torch.cuda.stream(stream):  # (sets the stream's device as well)
-            return fn(*args, **kwargs)
-
-    return _executor().submit(task).result()
+    task = _Call(fn, args, kwargs, _callers_stream())
+    _queue().put(task)
+    task.done.acquire()
+    if task.error is not None:
+        try:
+            raise task.error
+        finally:
+            task.error = None  # (the traceback holds this frame: no cycle)
+    return task.result
 
 
 def submit(fn, *args, **kwargs):
     """Queues ``fn(*args, **kwargs)`` on the device thread and returns its future without
     waiting (work that may overlap the caller's: the device's first-use costs)."""
-    return _executor().submit(fn, *args, **kwargs)
+    future = Future()
+
+    def run():
+        try:
+            future.set_result(fn(*args, **kwargs))
+        except BaseException as e:  # noqa: BLE001 (the future's holder sees it)
+            future.set_exception(e)
+
+    _queue().put(_Call(run, (), {}, None))
+    return future
 
 
 def on_device_thread(fn):

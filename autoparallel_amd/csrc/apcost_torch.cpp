@@ -23,9 +23,11 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime.h>
 #include <torch/custom_class.h>
 #include <torch/library.h>
 
+#include <algorithm>
 #include <cstring>
 #include <functional>
 #include <optional>
@@ -34,6 +36,7 @@
 #include <vector>
 
 #include "apcost.h"
+#include "apcost_parallel.h"
 
 namespace {
 
@@ -125,6 +128,142 @@ StrategyTable strategy_table(const Tensor &flops, const Tensor &rw_bytes, const 
   TORCH_CHECK(rw_bytes.numel() == s.n && dtype.numel() == s.n && zero_cost.numel() == s.n && num_args.numel() == s.n,
               "apcost: the strategy arrays must have one row per strategy (", s.n, ")");
   return s;
+}
+
+// ---- host <-> device, several arrays at once -----------------------------------------------------
+// A copy between pageable memory and the device goes through the runtime's own small staging buffers and
+// waits for itself: 15 - 25 us each, whatever its size, and 5 GB/s for a large one.  A planner moves
+// dozens of arrays at a time, so they travel together: one device buffer, pinned staging in chunks
+// (from torch's caching host allocator, given back when the call returns), one wait.
+constexpr int64_t kStagingChunk = 4 << 20;  // bytes per pinned chunk
+constexpr int kStagingSlots = 4;            // chunks in flight
+
+void check_hip(hipError_t e, const char *what) { TORCH_CHECK(e == hipSuccess, "apcost: ", what, ": ", hipGetErrorString(e)); }
+
+// memcpy on a thread per megabyte (at most four: what one memory stream of this size gains from).
+void copy_bytes(void *to, const void *from, int64_t n) {
+  const int threads = (int)std::min<int64_t>(4, n >> 20);
+  apc_internal::in_parallel(n, threads, [&](int64_t b, int64_t e) {
+    std::memcpy(static_cast<char *>(to) + b, static_cast<const char *>(from) + b, e - b);
+  });
+}
+
+// The pinned chunks of one transfer and the events that say when each is free again.
+struct Staging {
+  explicit Staging(int64_t total) {
+    const int64_t n = std::min<int64_t>(kStagingSlots, std::max<int64_t>(1, (total + kStagingChunk - 1) / kStagingChunk));
+    for (int64_t i = 0; i < n; ++i) {
+      slots.push_back(at::empty({std::min(total, kStagingChunk)}, at::TensorOptions().dtype(at::kByte).pinned_memory(true)));
+      hipEvent_t e = nullptr;
+      if (n > 1) check_hip(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+      events.push_back(e);
+    }
+  }
+  ~Staging() {
+    for (hipEvent_t e : events)
+      if (e) (void)hipEventDestroy(e);
+  }
+  char *slot(int64_t i) { return static_cast<char *>(slots[i].data_ptr()); }
+  std::vector<Tensor> slots;
+  std::vector<hipEvent_t> events;
+};
+
+int64_t padded(int64_t n) { return (n + 255) / 256 * 256; }
+
+// CPU tensors -> device tensors of the same dtypes and shapes, views of one device buffer (each at a
+// 256-byte boundary), complete when the call returns.
+std::vector<Tensor> upload(const std::vector<Tensor> &arrays, at::Device device) {
+  TORCH_CHECK(device.is_cuda(), "apcost: upload needs a HIP device (got ", device, ")");
+  int64_t total = 0;
+  std::vector<int64_t> at_byte;
+  for (const Tensor &t : arrays) {
+    TORCH_CHECK(t.device().is_cpu() && t.is_contiguous(), "apcost: upload takes contiguous CPU tensors");
+    at_byte.push_back(total);
+    total += padded(t.nbytes());
+  }
+  c10::hip::HIPGuard guard(device.index());
+  const auto bytes_on_device = at::TensorOptions().dtype(at::kByte).device(device);
+  Tensor buffer = at::empty({total}, bytes_on_device);
+  if (total > 0) {
+    hipStream_t stream = c10::hip::getCurrentHIPStream(device.index()).stream();
+    char *base = static_cast<char *>(buffer.data_ptr());
+    Staging staging(total);
+    const int64_t n_slots = (int64_t)staging.slots.size();
+    size_t k = 0;  // the first array that reaches into the chunk
+    int64_t chunk = 0;
+    for (int64_t begin = 0; begin < total; begin += kStagingChunk, ++chunk) {
+      const int64_t end = std::min(total, begin + kStagingChunk), slot = chunk % n_slots;
+      if (chunk >= n_slots) check_hip(hipEventSynchronize(staging.events[slot]), "hipEventSynchronize");
+      char *to = staging.slot(slot);
+      while (k < arrays.size() && at_byte[k] + (int64_t)arrays[k].nbytes() <= begin) ++k;
+      for (size_t i = k; i < arrays.size() && at_byte[i] < end; ++i) {
+        const int64_t b = std::max(begin, at_byte[i]), e = std::min<int64_t>(end, at_byte[i] + (int64_t)arrays[i].nbytes());
+        if (e > b) copy_bytes(to + (b - begin), static_cast<const char *>(arrays[i].data_ptr()) + (b - at_byte[i]), e - b);
+      }
+      check_hip(hipMemcpyAsync(base + begin, to, end - begin, hipMemcpyHostToDevice, stream), "hipMemcpyAsync");
+      if (n_slots > 1) check_hip(hipEventRecord(staging.events[slot], stream), "hipEventRecord");
+    }
+    check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
+  }
+  std::vector<Tensor> out;
+  for (size_t i = 0; i < arrays.size(); ++i) {
+    const Tensor &t = arrays[i];
+    if (t.numel() == 0) out.push_back(at::empty(t.sizes(), bytes_on_device.dtype(t.scalar_type())));
+    else out.push_back(buffer.narrow(0, at_byte[i], t.nbytes()).view(t.scalar_type()).view(t.sizes()));
+  }
+  return out;
+}
+
+// Device tensors (all on one device) -> new CPU tensors, after everything enqueued before on the current stream.
+std::vector<Tensor> download(const std::vector<Tensor> &arrays) {
+  std::vector<Tensor> out;
+  if (arrays.empty()) return out;
+  const at::Device device = arrays[0].device();
+  int64_t total = 0;
+  for (const Tensor &t : arrays) {
+    TORCH_CHECK(t.is_cuda() && t.is_contiguous(), "apcost: download takes contiguous device tensors");
+    same_device(arrays[0], t, "an array");
+    total += padded(t.nbytes());
+    out.push_back(at::empty(t.sizes(), t.options().device(at::kCPU)));
+  }
+  if (total == 0) return out;
+  c10::hip::HIPGuard guard(device.index());
+  hipStream_t stream = c10::hip::getCurrentHIPStream(device.index()).stream();
+  Staging staging(total);
+  const int64_t n_slots = (int64_t)staging.slots.size();
+  struct Piece {  // part of array k, staged in `slot` at `at`
+    size_t k;
+    int64_t from, n, slot, at;
+  };
+  // pieces in order; a chunk holds consecutive pieces, arrays may be cut at its end
+  std::vector<std::vector<Piece>> chunks(1);
+  int64_t fill = 0;
+  for (size_t k = 0; k < arrays.size(); ++k)
+    for (int64_t from = 0, n = (int64_t)arrays[k].nbytes(); from < n;) {
+      if (fill >= kStagingChunk) {
+        chunks.emplace_back();
+        fill = 0;
+      }
+      const int64_t take = std::min(n - from, kStagingChunk - fill);
+      chunks.back().push_back(Piece{k, from, take, (int64_t)(chunks.size() - 1) % n_slots, fill});
+      fill += padded(take);
+      from += take;
+    }
+  auto enqueue = [&](size_t c) {
+    for (const Piece &p : chunks[c])
+      check_hip(hipMemcpyAsync(staging.slot(p.slot) + p.at, static_cast<const char *>(arrays[p.k].data_ptr()) + p.from, p.n,
+                               hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
+    if (n_slots > 1) check_hip(hipEventRecord(staging.events[c % n_slots], stream), "hipEventRecord");
+  };
+  const size_t n_chunks = chunks.size();
+  for (size_t c = 0; c < n_chunks && c < (size_t)n_slots; ++c) enqueue(c);
+  for (size_t c = 0; c < n_chunks; ++c) {
+    if (n_slots > 1) check_hip(hipEventSynchronize(staging.events[c % n_slots]), "hipEventSynchronize");
+    else check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    for (const Piece &p : chunks[c]) copy_bytes(static_cast<char *>(out[p.k].data_ptr()) + p.from, staging.slot(p.slot) + p.at, p.n);
+    if (c + n_slots < n_chunks) enqueue(c + n_slots);
+  }
+  return out;
 }
 
 // ---- functional operators --------------------------------------------------------------------
@@ -737,6 +876,8 @@ TORCH_LIBRARY(apcost, m) {
         "Tensor edge_n_src, Tensor edge_tgt_begin, Tensor edge_n_tgt, Tensor edge_flags, Tensor edge_pt_begin, "
         "Tensor edge_entry_begin, Tensor edge_strat_begin, int n_pt, int n_strategies, Tensor tiles, Tensor dup_entry_begin) -> ()",
         &validate_tables);
+  m.def("upload(Tensor[] arrays, Device device) -> Tensor[]", &upload);
+  m.def("download(Tensor[] arrays) -> Tensor[]", &download);
   m.def("tensor_tables(" APCOST_TENSOR_TABLE ") -> (Tensor tensor_bytes, Tensor tensor_contiguous)", &tensor_tables);
   m.def("shard_shapes_bytes(Tensor params, Tensor spec_codes, Tensor spec_tensor, " APCOST_TENSOR_TABLE
         ", int shape_width) -> (Tensor num_shards, Tensor local_shape, Tensor local_stride, Tensor local_numel, Tensor local_bytes)",

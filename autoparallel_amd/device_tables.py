@@ -31,14 +31,26 @@ _UPLOAD = (
 )
 
 
-def _to_device(a: np.ndarray, device) -> torch.Tensor:
+def _as_tensor(a: np.ndarray) -> torch.Tensor:
+    """The array as a CPU tensor over the same memory."""
     if a.dtype == np.uint32:  # same bits; torch's uint32 support is partial
         a = a.view(np.int32)
     if a.dtype.names is not None:  # packed records travel as raw int32 words
         a = np.ascontiguousarray(a).view(np.int32).reshape(len(a), a.dtype.itemsize // 4)
+    if not a.flags.c_contiguous:
+        a = np.ascontiguousarray(a)
     if a.size == 0:
-        return torch.empty(a.shape, dtype=torch.from_numpy(np.zeros(1, a.dtype)).dtype, device=device)
-    return torch.from_numpy(a).to(device, non_blocking=False)
+        return torch.empty(a.shape, dtype=_TORCH_DTYPE[a.dtype.type])
+    return torch.from_numpy(a)
+
+
+def _to_device(a: np.ndarray, device) -> torch.Tensor:
+    """One array on ``device`` (or the CPU): a copy of its own."""
+    t = _as_tensor(a)
+    device = torch.device(device)
+    if device.type != "cuda":
+        return t.clone()
+    return _native.torch_ops().upload([t], device)[0]
 
 
 _TORCH_DTYPE = {np.int32: torch.int32, np.int64: torch.int64, np.uint8: torch.uint8, np.float64: torch.float64,
@@ -58,8 +70,7 @@ class DeviceCostTables:
             tables.validate(params)
         self.c_params = params.to_c()
         self.p = _native.params_tensor(self.c_params)  # struct apc_params as the operators take it
-        with torch.cuda.device(self.device):
-            self.d = {k: _to_device(getattr(tables, k), self.device) for k in _UPLOAD}
+        self.d = dict(zip(_UPLOAD, self._upload(*(getattr(tables, k) for k in _UPLOAD))))
         self.tensor_bytes = None
         self.tensor_contiguous = None
         self.compute_cost = None
@@ -74,11 +85,13 @@ class DeviceCostTables:
     def refresh(self, *names):
         """Re-uploads host tables that changed after construction (strategy inputs filled in
         from the shard-shape table, tiles rebuilt with de-duplication)."""
-        with torch.cuda.device(self.device):
-            for k in names:
-                self.d[k] = _to_device(getattr(self.tables, k), self.device)
+        self.d.update(zip(names, self._upload(*(getattr(self.tables, k) for k in names))))
 
     # ---- helpers -------------------------------------------------------------------------
+    def _upload(self, *arrays):
+        """Host arrays as device tensors, in one transfer."""
+        return self.ops.upload([_as_tensor(a) for a in arrays], self.device)
+
     def _empty(self, shape, dtype):
         return torch.empty(shape, dtype=dtype, device=self.device)
 
@@ -143,13 +156,10 @@ class DeviceCostTables:
             need = 4 if (recipes.node_kind >= 4).any() else 3 if (recipes.node_kind == 3).any() else 2
             if spec["local_shape"].shape[1] < need:
                 raise ValueError("the spec table's shape rows are narrower than a flop formula's tensors")
-        strat_node = _to_device(np.repeat(np.arange(n_nodes, dtype=np.int32), n_strat), self.device)
-        up = {k: _to_device(np.ascontiguousarray(getattr(recipes, k)), self.device) for k in (
-            "node_kind", "node_dtype", "node_const_bytes", "node_row_begin", "byte_rows", "node_flop_rows")}
-        node_strat_begin = _to_device(np.ascontiguousarray(tb.node_strat_begin, np.int64), self.device)
-        out = self.ops.strategy_inputs(strat_node, node_strat_begin, up["node_kind"], up["node_dtype"], up["node_const_bytes"],
-                                       up["node_row_begin"], up["byte_rows"], up["node_flop_rows"].reshape(-1),
-                                       spec["local_shape"], spec["local_bytes"])
+        out = self.ops.strategy_inputs(*self._upload(
+            np.repeat(np.arange(n_nodes, dtype=np.int32), n_strat), np.ascontiguousarray(tb.node_strat_begin, np.int64),
+            recipes.node_kind, recipes.node_dtype, recipes.node_const_bytes, recipes.node_row_begin, recipes.byte_rows,
+            recipes.node_flop_rows.reshape(-1)), spec["local_shape"], spec["local_bytes"])
         for key, t in zip(("strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost"), out):
             self.d[key] = t
         return out
@@ -158,9 +168,7 @@ class DeviceCostTables:
     @_guarded
     def run_compute_costs(self):
         self.compute_cost, self.compute_cost_per_arg, err = self.ops.compute_cost(self.p, *self._strategy_table())
-        if int(err.item()) != 0:
-            # compute_estimation.py:198-201
-            raise ValueError(f"a strategy with non-zero flops uses a dtype not supported on {self.params.device_name}")
+        self._check_flag(int(err.item()))
         return self.compute_cost, self.compute_cost_per_arg
 
     # ---- redistribution-cost matrices ------------------------------------------------------
@@ -283,15 +291,11 @@ class DeviceCostTables:
         return tb.n_entries <= self.PACKED_MAX_ENTRIES and tb.packable()
 
     def _packed_tiles(self):
-        """The device copy of ``CostTables.pack_tiles()`` (checked against the tables by the
-        library's host-side validator), made once per tiling."""
+        """The device copy of ``CostTables.pack_tiles()``, made once per tiling."""
         cached = getattr(self, "_packed_cache", None)
         if cached is not None and cached[0] is self.tables.tile_records:
             return cached[1]
-        packed = self.tables.pack_tiles()
-        self.tables.validate_packed(packed)
-        with torch.cuda.device(self.device):
-            dev = _to_device(packed, self.device)
+        dev = _to_device(self.tables.pack_tiles(), self.device)
         self._packed_cache = (self.tables.tile_records, dev)
         return dev
 
@@ -364,7 +368,7 @@ class DeviceCostTables:
         if row_min:
             self.row_min = self._empty((tb.n_rows,), torch.float64)
             self.row_argmin = self._empty((tb.n_rows,), torch.int32)
-        if row_min_in_tiles:
+        if row_min_in_tiles and not packed:  # (packed tiles hold their rows' numbers themselves)
             rows = (_to_device(tb.edge_row_begin(), self.device), self.row_min, self.row_argmin)
         erb, rmin, rarg = rows if rows is not None else (None, None, None)
         dup_rows = d["dup_row_begin"] if rows is not None else None
@@ -391,7 +395,7 @@ class DeviceCostTables:
         if not one_launch and not packed:
             step["redistribute_tables"] = bind(self._bind_redistribute_tables(self.comm, self.transition, self.cost, rows))
         if row_min and not row_min_in_tiles:
-            row_ptr = torch.from_numpy(tb.row_ptr()).to(self.device)
+            row_ptr = _to_device(tb.row_ptr(), self.device)
             assert row_ptr.numel() - 1 == self.row_min.numel()
             copies = self._row_copies()
             if copies is not None:  # identical edges: every distinct row is read once, its minimum stored to all
@@ -424,7 +428,11 @@ class DeviceCostTables:
     def check_error_flag(self):
         """After a synchronisation: raises if a strategy with flops had an unsupported dtype."""
         err = getattr(self, "_step_error_flag", None)
-        if err is not None and int(err.item()) != 0:
+        if err is not None:
+            self._check_flag(int(err.item()))
+
+    def _check_flag(self, flag: int):
+        if flag != 0:
             # compute_estimation.py:198-201
             raise ValueError(f"a strategy with non-zero flops uses a dtype not supported on {self.params.device_name}")
 
@@ -450,9 +458,6 @@ class DeviceCostTables:
     def cost_objective(self, n_vars: int, group_var_begin, group_member_begin, member_entry_begin):
         """-> (objective f64[n_vars], forced_zero u8[n_vars]) on the device: the ILP objective
         summed from ``cost`` (``apc_cost_objective``).  The index arrays are host arrays."""
-        gv = _to_device(np.ascontiguousarray(group_var_begin, np.int64), self.device)
-        gm = _to_device(np.ascontiguousarray(group_member_begin, np.int64), self.device)
-        me = _to_device(np.ascontiguousarray(member_entry_begin, np.int64), self.device)
         n_groups = len(group_var_begin) - 1
         if n_groups < 0 or len(group_member_begin) != n_groups + 1:
             raise ValueError("group_var_begin and group_member_begin must have n_groups + 1 rows")
@@ -461,7 +466,8 @@ class DeviceCostTables:
             raise ValueError("group pointers do not span the variables / members")
         if n_groups and not bool((np.diff(np.asarray(group_var_begin, np.int64)) > 0).all()):
             raise ValueError("every variable group needs at least one variable (the kernel takes one workgroup per group)")
-        return self.ops.cost_objective(int(n_vars), gv, gm, me, self.fetch("cost"), float(self.params.inf_replacement_cost))
+        index = self._upload(*(np.ascontiguousarray(a, np.int64) for a in (group_var_begin, group_member_begin, member_entry_begin)))
+        return self.ops.cost_objective(int(n_vars), *index, self.fetch("cost"), float(self.params.inf_replacement_cost))
 
     @_guarded
     def capture_step_graph(self, step):
@@ -510,8 +516,7 @@ class DeviceCostTables:
         selected, copy_ptr, copy_rows, n_read = tb.row_copies()
         out = None
         if n_read <= 0.75 * tb.n_entries:
-            out = (_to_device(selected, self.device), _to_device(copy_ptr, self.device),
-                   _to_device(copy_rows, self.device), n_read)
+            out = (*self._upload(selected, copy_ptr, copy_rows), n_read)
         self._row_copies_cache = (tb.tile_records, out)
         return out
 
@@ -603,8 +608,8 @@ class DeviceCostTables:
         if row_min.numel() != t.n_rows:
             raise ValueError("row_min must hold one value per matrix row")
         if getattr(self, "_bound_index", None) is None:
-            self._bound_index = {k: _to_device(v, self.device) for k, v in t.strategy_bound_index().items()}
-            self._bound_index["node_strat_begin"] = _to_device(np.ascontiguousarray(t.node_strat_begin, np.int64), self.device)
+            index = dict(t.strategy_bound_index(), node_strat_begin=np.ascontiguousarray(t.node_strat_begin, np.int64))
+            self._bound_index = dict(zip(index, self._upload(*index.values())))
         ix = self._bound_index
         return self.ops.strategy_bounds(ix["strat_node"], ix["node_strat_begin"], ix["node_edge_begin"], ix["edges_by_node"],
                                         ix["edge_row_begin"], row_min)

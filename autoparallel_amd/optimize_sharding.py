@@ -93,7 +93,7 @@ class DeviceBackend:
     @on_device_thread
     def local_shapes(self):
         out = self.dev.run_spec_tables()
-        return out["local_shape"].cpu().numpy(), out["local_stride"].cpu().numpy()
+        return tuple(t.numpy() for t in self.dev.ops.download([out["local_shape"], out["local_stride"]]))
 
     @on_device_thread
     def strategy_inputs(self, recipes):
@@ -101,12 +101,10 @@ class DeviceBackend:
         ``apc_strategy_inputs`` over the per-node recipes); the host's strategy table receives
         copies (identical edges are found on the host, and flop / byte counts are part of an
         edge's identity)."""
-        flops, rw_bytes, dtype, zero = self.dev.run_strategy_inputs(recipes)
         tb = self.dev.tables
-        tb.strat_flops[:] = flops.cpu().numpy()
-        tb.strat_rw_bytes[:] = rw_bytes.cpu().numpy()
-        tb.strat_dtype[:] = dtype.cpu().numpy()
-        tb.strat_zero_cost[:] = zero.cpu().numpy()
+        counts = self.dev.ops.download(list(self.dev.run_strategy_inputs(recipes)))
+        for a, t in zip((tb.strat_flops, tb.strat_rw_bytes, tb.strat_dtype, tb.strat_zero_cost), counts):
+            a[:] = t.numpy()
         self._strategy_inputs_on_device = True
 
     def upload_strategy_inputs(self, tables, tile_entries=None, dedupe=True, max_copies=16):
@@ -138,17 +136,13 @@ class DeviceBackend:
         d = self.dev
         with torch.cuda.device(d.device):
             obj, forced = d.cost_objective(n_vars, group_var_begin, group_member_begin, member_entry_begin)
-            torch.cuda.synchronize(d.device)
-        d.check_error_flag()
+            t0 = time.perf_counter()
+            obj, forced, compute, per_arg, flag = (
+                t.numpy() for t in d.ops.download([obj, forced, d.compute_cost, d.compute_cost_per_arg, d._step_error_flag]))
+        self.timings["copy_back_s"] = time.perf_counter() - t0  # (the wait for the kernels included)
+        d._check_flag(int(flag[0]))
         self.timings["kernels_s"] = self._events[0].elapsed_time(self._events[1]) * 1e-3
-        t0 = time.perf_counter()
-        out = {
-            "objective": obj.cpu().numpy(),
-            "forced_zero": forced.cpu().numpy().astype(bool),
-            "compute": d.compute_cost.cpu().numpy(),
-            "compute_per_arg": d.compute_cost_per_arg.cpu().numpy(),
-        }
-        self.timings["copy_back_s"] = time.perf_counter() - t0
+        out = {"objective": obj, "forced_zero": forced.view(bool), "compute": compute, "compute_per_arg": per_arg}
         for k in ("kernels_s", "copy_back_s"):
             logger.info("%s %.6f s", k, self.timings[k])
         return out
@@ -157,7 +151,7 @@ class DeviceBackend:
     def host_array(self, name):
         """``comm`` / ``transition`` / ``cost`` of every entry, copied (computed first, if the
         table pass did not write it) now."""
-        return self.dev.fetch(name).cpu().numpy()
+        return self.dev.ops.download([self.dev.fetch(name)])[0].numpy()
 
     @on_device_thread
     def gather(self, name, entries):
@@ -175,7 +169,7 @@ class DeviceBackend:
             mins, args = self.dev.row_minima()
         else:
             mins, args = self.dev.segmented_min(self.dev.fetch("cost"), row_ptr)
-        return mins.cpu().numpy(), args.cpu().numpy()
+        return tuple(t.numpy() for t in self.dev.ops.download([mins, args]))
 
     def _are_matrix_rows(self, row_ptr) -> bool:
         tb = self.dev.tables
@@ -188,7 +182,7 @@ class DeviceBackend:
             mins, _ = self.dev.row_minima()
         else:
             mins, _ = self.dev.segmented_min(self.dev.fetch("cost"), row_ptr)
-        return tuple(x.cpu().numpy() for x in self.dev.greedy_strategies(mins))
+        return tuple(t.numpy() for t in self.dev.ops.download(list(self.dev.greedy_strategies(mins))))
 
 
 class CostRecords(Mapping):
