@@ -9,6 +9,8 @@ from __future__ import annotations
 import ctypes
 import os
 
+import numpy as np
+
 from ._build import LIB_PATH, TORCH_EXT_PATH
 
 APC_ABI_VERSION = 3  # include/apcost.h: the interface this binding's structs and limits mirror
@@ -93,6 +95,11 @@ EXPORTS = (
     "apc_fill_tiles_host",
     "apc_tile_records_host",
     "apc_validate_tiling_host",
+    "apc_label_incidence_host",
+    "apc_label_minima_host",
+    "apc_round_labels_host",
+    "apc_refine_labels_host",
+    "apc_prune_masks_host",
     "apc_build_tables_packed",
     "apc_calibrate_launch",
     "apc_calibrate_fill",
@@ -175,29 +182,35 @@ def check(rc: int, what: str) -> None:
         raise RuntimeError(f"{what} failed ({rc}): {msg}")
 
 
-def _argument(a):
-    """A host entry point's argument: a contiguous numpy array as its address, ``None`` as NULL, an
-    integer as int64, a ctypes structure by reference."""
+def argument(a):
+    """A host entry point's argument: what is one already, a contiguous numpy array as its address, ``None`` as NULL, an
+    integer as int64, a float as double, a ctypes structure by reference."""
+    if type(a) is np.ndarray:
+        if not a.flags.c_contiguous:
+            raise ValueError("host entry points take contiguous arrays")
+        return ctypes.c_void_p(a.ctypes.data)
     if a is None:
         return ctypes.c_void_p(None)
+    if isinstance(a, ctypes.c_void_p):
+        return a
     if isinstance(a, int):
         return ctypes.c_int64(a)
+    if isinstance(a, float):
+        return ctypes.c_double(a)
     if isinstance(a, ctypes.Structure):
         return ctypes.byref(a)
-    if not a.flags.c_contiguous:
-        raise ValueError("host entry points take contiguous arrays")
-    return ctypes.c_void_p(a.ctypes.data)
+    raise TypeError(f"host entry points take contiguous arrays and plain numbers: {type(a).__name__}")
 
 
 def host_call(name: str, *args) -> None:
     """Calls a host entry point of the library; raises RuntimeError with its message on an error."""
-    check(getattr(lib(), name)(*[_argument(a) for a in args]), name)
+    check(getattr(lib(), name)(*[argument(a) for a in args]), name)
 
 
 def host_counts(name: str, *args) -> tuple:
     """A host entry point whose last two arguments are ``int64_t *`` results: returns them."""
     first, second = ctypes.c_int64(), ctypes.c_int64()
-    check(getattr(lib(), name)(*[_argument(a) for a in args], ctypes.byref(first), ctypes.byref(second)), name)
+    check(getattr(lib(), name)(*[argument(a) for a in args], ctypes.byref(first), ctypes.byref(second)), name)
     return first.value, second.value
 
 

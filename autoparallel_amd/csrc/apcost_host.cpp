@@ -711,3 +711,225 @@ int apc_validate_packed_tiles_host(int64_t n_tensors, const int32_t *tensor_rank
 }
 
 }  // extern "C"
+
+// ------------------------------------------------------------------------------------------
+// Rounding and pruning of a labelling problem (apc_diffusion_sweeps states its arrays): the host's
+// part between two calls of the sweeps.  Sums in incidence order, one rounding per addition.
+// ------------------------------------------------------------------------------------------
+namespace {
+
+// The smallest of n values, +inf of none (eight running minima: the order of the comparisons is free).
+double least(const double *v, int64_t n) {
+  double d[8];
+  for (double &x : d) x = __builtin_inf();
+  int64_t i = 0;
+  for (; i + 8 <= n; i += 8)
+    for (int j = 0; j < 8; ++j) d[j] = v[i + j] < d[j] ? v[i + j] : d[j];
+  for (; i < n; ++i) d[0] = v[i] < d[0] ? v[i] : d[0];
+  for (int j = 1; j < 8; ++j) d[0] = d[j] < d[0] ? d[j] : d[0];
+  return d[0];
+}
+
+struct LabelProblem {
+  int64_t n_classes, n_edges;
+  const int64_t *label_begin, *inc_begin;
+  const int32_t *inc_edge;
+  const uint8_t *inc_side;
+  const int64_t *edge_begin;
+  const int32_t *edge_i, *edge_j;
+  const double *theta, *unary;
+
+  int64_t labels(int64_t c) const { return label_begin[c + 1] - label_begin[c]; }
+  int64_t other(int64_t k, int side) const { return side == 0 ? edge_j[k] : edge_i[k]; }
+  // every index the walks below use lies inside its array, and every matrix has its classes' shape
+  bool holds() const {
+    if (n_classes < 0 || n_edges < 0 || !label_begin || !inc_begin || !edge_begin || label_begin[0] != 0 || inc_begin[0] != 0 || edge_begin[0] != 0)
+      return false;
+    for (int64_t c = 0; c < n_classes; ++c)
+      if (label_begin[c + 1] < label_begin[c] || inc_begin[c + 1] < inc_begin[c]) return false;
+    for (int64_t k = 0; k < n_edges; ++k) {
+      if (edge_i[k] < 0 || edge_i[k] >= n_classes || edge_j[k] < 0 || edge_j[k] >= n_classes) return false;
+      if (edge_begin[k + 1] - edge_begin[k] != labels(edge_i[k]) * labels(edge_j[k])) return false;
+    }
+    for (int64_t c = 0; c < n_classes; ++c)
+      for (int64_t t = inc_begin[c]; t < inc_begin[c + 1]; ++t) {
+        const int64_t k = inc_edge[t];
+        if (k < 0 || k >= n_edges || inc_side[t] > 1 || (inc_side[t] == 0 ? edge_i[k] : edge_j[k]) != c) return false;
+      }
+    return true;
+  }
+  // out[x] = min over the other end's labels of the matrix of edge k, x a label of the class on side `side`
+  void minima(int64_t k, int side, double *out) const {
+    const double *m = theta + edge_begin[k];
+    const int64_t ni = labels(edge_i[k]), nj = labels(edge_j[k]);
+    if (side == 0) {
+      for (int64_t x = 0; x < ni; ++x) out[x] = least(m + x * nj, nj);
+    } else {
+      for (int64_t y = 0; y < nj; ++y) out[y] = __builtin_inf();
+      for (int64_t x = 0; x < ni; ++x)
+        for (int64_t y = 0; y < nj; ++y) out[y] = m[x * nj + y] < out[y] ? m[x * nj + y] : out[y];
+    }
+  }
+  // score[x] += the matrix of edge k at (x, label of the other end)
+  void add_fixed(int64_t k, int side, int64_t label, double *score) const {
+    const double *m = theta + edge_begin[k];
+    const int64_t ni = labels(edge_i[k]), nj = labels(edge_j[k]);
+    if (side == 0)
+      for (int64_t x = 0; x < ni; ++x) score[x] += m[x * nj + label];
+    else
+      for (int64_t y = 0; y < nj; ++y) score[y] += m[label * nj + y];
+  }
+};
+
+int64_t first_minimum(const double *v, int64_t n) {
+  int64_t at = 0;
+  for (int64_t i = 1; i < n; ++i)
+    if (v[i] < v[at]) at = i;
+  return at;
+}
+
+}  // namespace
+
+extern "C" {
+
+int apc_label_incidence_host(int64_t n_classes, int64_t n_edges, const int32_t *edge_i, const int32_t *edge_j, int64_t *inc_begin,
+                             int32_t *inc_edge, uint8_t *inc_side, int64_t *color) {
+  if (n_classes < 0 || n_edges < 0 || !inc_begin || (n_classes > 0 && !color) || (n_edges > 0 && (!edge_i || !edge_j || !inc_edge || !inc_side)))
+    return fail(-1, "apc_label_incidence_host: NULL array or negative count");
+  for (int64_t k = 0; k < n_edges; ++k)
+    if (edge_i[k] < 0 || edge_i[k] >= n_classes || edge_j[k] < 0 || edge_j[k] >= n_classes)
+      return fail(-2, "edge %lld: classes %d, %d outside [0, %lld)", (long long)k, edge_i[k], edge_j[k], (long long)n_classes);
+  std::fill(inc_begin, inc_begin + n_classes + 1, 0);
+  for (int64_t k = 0; k < n_edges; ++k) ++inc_begin[edge_i[k] + 1], ++inc_begin[edge_j[k] + 1];
+  for (int64_t c = 0; c < n_classes; ++c) inc_begin[c + 1] += inc_begin[c];
+  std::vector<int64_t> next(inc_begin, inc_begin + n_classes);
+  for (int64_t k = 0; k < n_edges; ++k)
+    for (int side = 0; side < 2; ++side) {
+      const int64_t at = next[side == 0 ? edge_i[k] : edge_j[k]]++;
+      inc_edge[at] = (int32_t)k;
+      inc_side[at] = (uint8_t)side;
+    }
+  std::vector<int64_t> used_by;  // colour -> the last class that saw it on a neighbour
+  for (int64_t c = 0; c < n_classes; ++c) color[c] = -1;
+  for (int64_t c = 0; c < n_classes; ++c) {
+    for (int64_t t = inc_begin[c]; t < inc_begin[c + 1]; ++t) {
+      const int64_t k = inc_edge[t], col = color[inc_side[t] == 0 ? edge_j[k] : edge_i[k]];
+      if (col >= 0) used_by[col] = c;
+    }
+    int64_t col = 0;
+    while (col < (int64_t)used_by.size() && used_by[col] == c) ++col;
+    if (col == (int64_t)used_by.size()) used_by.push_back(-1);
+    color[c] = col;
+  }
+  return 0;
+}
+
+#define APC_LABEL_PROBLEM                                                                                                     \
+  int64_t n_classes, const int64_t *label_begin, const int64_t *inc_begin, const int32_t *inc_edge, const uint8_t *inc_side,  \
+      int64_t n_edges, const int64_t *edge_begin, const int32_t *edge_i, const int32_t *edge_j, const double *theta,          \
+      const double *unary
+#define APC_LABEL_PROBLEM_OF(who)                                                                                             \
+  const LabelProblem g{n_classes, n_edges, label_begin, inc_begin, inc_edge, inc_side, edge_begin, edge_i, edge_j, theta, unary}; \
+  if (!g.holds()) return fail(-2, who ": the index arrays do not describe a labelling problem")
+
+int apc_label_minima_host(APC_LABEL_PROBLEM, double *class_min, double *edge_min) {
+  APC_LABEL_PROBLEM_OF("apc_label_minima_host");
+  for (int64_t c = 0; c < n_classes; ++c) {
+    const int64_t b = label_begin[c], e = label_begin[c + 1];
+    class_min[c] = e > b ? unary[b + first_minimum(unary + b, e - b)] : 0.0;
+  }
+  in_parallel(n_edges, threads_for(4 * edge_begin[n_edges]), [&](int64_t b, int64_t e) {
+    for (int64_t k = b; k < e; ++k) edge_min[k] = least(theta + edge_begin[k], edge_begin[k + 1] - edge_begin[k]);
+  });
+  return 0;
+}
+
+int apc_round_labels_host(APC_LABEL_PROBLEM, int64_t *labels) {
+  APC_LABEL_PROBLEM_OF("apc_round_labels_host");
+  std::vector<double> score, d;
+  for (int64_t c = 0; c < n_classes; ++c) labels[c] = -1;
+  for (int64_t c = 0; c < n_classes; ++c) {
+    const int64_t n = g.labels(c);
+    score.assign(unary + label_begin[c], unary + label_begin[c + 1]);
+    d.resize(n);
+    for (int64_t t = inc_begin[c]; t < inc_begin[c + 1]; ++t) {
+      const int64_t k = inc_edge[t];
+      const int side = inc_side[t];
+      const int64_t fixed = labels[g.other(k, side)];
+      if (fixed >= 0) {
+        g.add_fixed(k, side, fixed, score.data());
+      } else {
+        g.minima(k, side, d.data());
+        for (int64_t x = 0; x < n; ++x) score[x] += d[x];
+      }
+    }
+    if (n > 0) labels[c] = first_minimum(score.data(), n);
+  }
+  return 0;
+}
+
+int apc_refine_labels_host(APC_LABEL_PROBLEM, int64_t max_rounds, int64_t *labels) {
+  APC_LABEL_PROBLEM_OF("apc_refine_labels_host");
+  for (int64_t c = 0; c < n_classes; ++c)
+    if (labels[c] < -1 || labels[c] >= g.labels(c)) return fail(-2, "apc_refine_labels_host: label %lld of class %lld", (long long)labels[c], (long long)c);
+  std::vector<uint8_t> todo(n_classes, 1), again(n_classes);
+  std::vector<double> score;
+  for (int64_t round = 0; round < max_rounds; ++round) {
+    std::fill(again.begin(), again.end(), 0);
+    bool any = false;
+    for (int64_t c = 0; c < n_classes; ++c) {
+      if (!todo[c] || labels[c] < 0) continue;
+      score.assign(unary + label_begin[c], unary + label_begin[c + 1]);
+      for (int64_t t = inc_begin[c]; t < inc_begin[c + 1]; ++t) {
+        const int64_t k = inc_edge[t], o = g.other(k, inc_side[t]);
+        // (a neighbour without labels has nothing to fix)
+        if (labels[o] >= 0) g.add_fixed(k, inc_side[t], labels[o], score.data());
+      }
+      const int64_t best = first_minimum(score.data(), g.labels(c));
+      if (score[best] < score[labels[c]]) {
+        labels[c] = best;
+        for (int64_t t = inc_begin[c]; t < inc_begin[c + 1]; ++t) again[g.other(inc_edge[t], inc_side[t])] = 1, any = true;
+      }
+    }
+    if (!any) break;
+    todo.swap(again);
+  }
+  return 0;
+}
+
+int apc_prune_masks_host(APC_LABEL_PROBLEM, const double *class_min, const double *edge_min, double bound, double limit,
+                         uint8_t *dead_label, uint8_t *dead_pair) {
+  APC_LABEL_PROBLEM_OF("apc_prune_masks_host");
+  const int threads = threads_for(8 * edge_begin[n_edges]);
+  in_parallel(n_classes, threads, [&](int64_t begin, int64_t end) {
+    std::vector<double> b, d;
+    for (int64_t c = begin; c < end; ++c) {
+      const int64_t n = g.labels(c), l0 = label_begin[c];
+      b.resize(n);
+      d.resize(n);
+      for (int64_t x = 0; x < n; ++x) b[x] = (bound - class_min[c]) + unary[l0 + x];
+      for (int64_t t = inc_begin[c]; t < inc_begin[c + 1]; ++t) {
+        const int64_t k = inc_edge[t];
+        g.minima(k, inc_side[t], d.data());
+        for (int64_t x = 0; x < n; ++x) b[x] = (b[x] - edge_min[k]) + d[x];
+      }
+      for (int64_t x = 0; x < n; ++x) dead_label[l0 + x] = !(b[x] <= limit);  // (NaN: dead)
+    }
+  });
+  in_parallel(n_edges, threads, [&](int64_t begin, int64_t end) {
+    for (int64_t k = begin; k < end; ++k) {
+      const int64_t ni = g.labels(edge_i[k]), nj = g.labels(edge_j[k]);
+      const uint8_t *di = dead_label + label_begin[edge_i[k]], *dj = dead_label + label_begin[edge_j[k]];
+      const double *m = theta + edge_begin[k], rest = bound - edge_min[k];
+      uint8_t *out = dead_pair + edge_begin[k];
+      for (int64_t x = 0; x < ni; ++x)
+        for (int64_t y = 0; y < nj; ++y) out[x * nj + y] = (uint8_t)(!(rest + m[x * nj + y] <= limit)) | di[x] | dj[y];
+    }
+  });
+  return 0;
+}
+
+#undef APC_LABEL_PROBLEM
+#undef APC_LABEL_PROBLEM_OF
+
+}  // extern "C"

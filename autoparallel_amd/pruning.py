@@ -37,6 +37,8 @@ from dataclasses import dataclass, field
 
 import numpy as np
 
+from . import _native
+
 # a variable is fixed only if its bound exceeds the incumbent by more than this relative margin:
 # far above the rounding of a few hundred fp64 updates, far below one transition cost unit
 RELATIVE_MARGIN = 1e-7
@@ -71,6 +73,13 @@ class LabelGraph:
     color_nodes: np.ndarray  # int32: classes grouped by colour (no two of a colour share an edge)
     blocks: list = field(default_factory=list)
     class_of_choice_base: dict = field(default_factory=dict)
+    _addresses: tuple = field(default=None, repr=False, compare=False)  # of the index arrays, for the library
+
+    def __post_init__(self):
+        for name, dtype in (("label_begin", np.int64), ("unary", np.float64), ("edge_i", np.int32), ("edge_j", np.int32),
+                            ("edge_begin", np.int64), ("theta", np.float64), ("inc_begin", np.int64), ("inc_edge", np.int32),
+                            ("inc_side", np.uint8), ("color_begin", np.int64), ("color_nodes", np.int32)):
+            setattr(self, name, np.ascontiguousarray(getattr(self, name), dtype))
 
     @property
     def n_classes(self) -> int:
@@ -95,7 +104,9 @@ def build_label_graph(blocks: list, class_sizes: list, block_costs, masks: dict,
     n = len(class_sizes)
     label_begin = np.zeros(n + 1, np.int64)
     np.cumsum(class_sizes, out=label_begin[1:])
-    unary = [np.zeros(s) for s in class_sizes]
+    all_unary = np.zeros(int(label_begin[-1]))
+    at = label_begin.tolist()
+    unary = [all_unary[at[c]:at[c + 1]] for c in range(n)]
     merged: dict = {}
     order: list = []
 
@@ -110,7 +121,7 @@ def build_label_graph(blocks: list, class_sizes: list, block_costs, masks: dict,
             merged[(j, i)] = merged[(j, i)] + m.T
             key, tr = (j, i), True
         else:
-            merged[(i, j)] = m.copy()
+            merged[(i, j)] = m  # (read only: a second matrix of the pair makes a new one)
             order.append((i, j))
             key, tr = (i, j), False
         if block is not None:
@@ -125,7 +136,7 @@ def build_label_graph(blocks: list, class_sizes: list, block_costs, masks: dict,
     for i, j, m in ties:
         add_pair(i, j, m)
     for c, allowed in masks.items():
-        unary[c] = np.where(allowed, unary[c], np.inf)
+        unary[c][~np.asarray(allowed, bool)] = np.inf
     index = {key: k for k, key in enumerate(order)}
     for b in blocks:
         if isinstance(b.edge, tuple):
@@ -135,58 +146,45 @@ def build_label_graph(blocks: list, class_sizes: list, block_costs, masks: dict,
     sizes = np.asarray([class_sizes[i] * class_sizes[j] for i, j in order], np.int64)
     edge_begin = np.zeros(len(order) + 1, np.int64)
     np.cumsum(sizes, out=edge_begin[1:])
-    theta = np.concatenate([merged[key].ravel() for key in order]) if order else np.zeros(0)
-    # incidence, in edge order
-    inc: list = [[] for _ in range(n)]
-    for k, (i, j) in enumerate(order):
-        inc[i].append((k, 0))
-        inc[j].append((k, 1))
-    inc_begin = np.zeros(n + 1, np.int64)
-    np.cumsum([len(x) for x in inc], out=inc_begin[1:])
-    inc_edge = np.asarray([k for x in inc for k, _ in x], np.int32)
-    inc_side = np.asarray([s for x in inc for _, s in x], np.uint8)
-    # greedy colouring in class order: classes of one colour share no edge and update together
-    color = np.full(n, -1, np.int64)
-    for c in range(n):
-        used = {int(color[int(edge_j[k]) if s == 0 else int(edge_i[k])]) for k, s in inc[c]}
-        col = 0
-        while col in used:
-            col += 1
-        color[c] = col
+    theta = np.concatenate([merged[key].reshape(-1) for key in order]) if order else np.zeros(0)
+    # incidence in edge order; greedy colouring in class order: classes of one colour share no edge and update together
+    inc_begin, color = np.empty(n + 1, np.int64), np.empty(n, np.int64)
+    inc_edge, inc_side = np.empty(2 * len(order), np.int32), np.empty(2 * len(order), np.uint8)
+    _native.host_call("apc_label_incidence_host", n, len(order), edge_i, edge_j, inc_begin, inc_edge, inc_side, color)
     n_colors = int(color.max()) + 1 if n else 0
     color_nodes = np.argsort(color, kind="stable").astype(np.int32)
     color_begin = np.zeros(n_colors + 1, np.int64)
     np.cumsum(np.bincount(color, minlength=n_colors), out=color_begin[1:])
-    return LabelGraph(label_begin=label_begin, unary=np.concatenate(unary) if n else np.zeros(0), edge_i=edge_i,
+    return LabelGraph(label_begin=label_begin, unary=all_unary, edge_i=edge_i,
                       edge_j=edge_j, edge_begin=edge_begin, theta=np.ascontiguousarray(theta, np.float64),
                       inc_begin=inc_begin, inc_edge=inc_edge, inc_side=inc_side, color_begin=color_begin,
                       color_nodes=color_nodes, blocks=blocks)
 
 
+def _problem(g: LabelGraph, theta: np.ndarray, unary: np.ndarray) -> tuple:
+    """The arguments that the library's host entry points take for the problem."""
+    theta, unary = np.ascontiguousarray(theta, np.float64), np.ascontiguousarray(unary, np.float64)
+    if len(theta) != g.edge_begin[-1] or len(unary) != g.label_begin[-1]:
+        raise ValueError("theta / unary do not have the problem's size")
+    index = (g.label_begin, g.inc_begin, g.inc_edge, g.inc_side, g.edge_begin, g.edge_i, g.edge_j)
+    if g._addresses is None or any(x is not y for x, y in zip(g._addresses[0], index)):
+        g._addresses = (index, [_native.argument(a) for a in index])  # (the address of an array costs as much as the call)
+    a = g._addresses[1]
+    return (g.n_classes, *a[:4], g.n_edges, *a[4:], theta, unary)
+
+
 def lower_bound(g: LabelGraph, theta: np.ndarray, unary: np.ndarray):
     """-> (LB, per-class minimum of the unary vector, per-edge minimum of the matrix)"""
-    lb = g.label_begin
-    umin = np.asarray([unary[lb[c]:lb[c + 1]].min() if lb[c + 1] > lb[c] else 0.0 for c in range(g.n_classes)])
-    emin = np.asarray([theta[g.edge_begin[k]:g.edge_begin[k + 1]].min() for k in range(g.n_edges)])
-    return math.fsum(umin) + math.fsum(emin), umin, emin
+    umin, emin = np.empty(g.n_classes), np.empty(g.n_edges)
+    _native.host_call("apc_label_minima_host", *_problem(g, theta, unary), umin, emin)
+    return math.fsum(umin.tolist()) + math.fsum(emin.tolist()), umin, emin
 
 
 def decode(g: LabelGraph, theta: np.ndarray, unary: np.ndarray) -> np.ndarray:
     """A labelling from the reparametrised costs: classes in order, each takes the label that is
     cheapest given the labels already taken by its neighbours and the best case for the rest."""
-    n = g.n_classes
-    lab = np.full(n, -1, np.int64)
-    lb = g.label_begin
-    for c in range(n):
-        score = unary[lb[c]:lb[c + 1]].copy()
-        for t in range(int(g.inc_begin[c]), int(g.inc_begin[c + 1])):
-            k, side = int(g.inc_edge[t]), int(g.inc_side[t])
-            m = g.matrix(theta, k)
-            if side == 1:
-                m = m.T
-            other = int(g.edge_j[k]) if side == 0 else int(g.edge_i[k])
-            score = score + (m[:, lab[other]] if lab[other] >= 0 else m.min(axis=1))
-        lab[c] = int(np.argmin(score)) if len(score) else -1
+    lab = np.empty(g.n_classes, np.int64)
+    _native.host_call("apc_round_labels_host", *_problem(g, theta, unary), lab)
     return lab
 
 
@@ -194,29 +192,8 @@ def refine(g: LabelGraph, theta: np.ndarray, unary: np.ndarray, labels: np.ndarr
     """Local search from a labelling: class by class, the label that is cheapest given the labels
     of all its neighbours, until a round changes nothing (after the first round only classes with
     a changed neighbour are looked at again).  Never raises the labelling's cost."""
-    lab = labels.copy()
-    lb = g.label_begin
-    todo = np.ones(g.n_classes, bool)
-    for _ in range(max_rounds):
-        again = np.zeros(g.n_classes, bool)
-        for c in np.nonzero(todo)[0]:
-            if lab[c] < 0:
-                continue
-            score = unary[lb[c]:lb[c + 1]].copy()
-            others = []
-            for t in range(int(g.inc_begin[c]), int(g.inc_begin[c + 1])):
-                k, side = int(g.inc_edge[t]), int(g.inc_side[t])
-                m = g.matrix(theta, k)
-                other = int(g.edge_j[k]) if side == 0 else int(g.edge_i[k])
-                others.append(other)
-                score = score + (m[:, lab[other]] if side == 0 else m[lab[other], :])
-            best = int(np.argmin(score))
-            if score[best] < score[lab[c]]:
-                lab[c] = best
-                again[others] = True
-        if not again.any():
-            break
-        todo = again
+    lab = np.array(labels, np.int64)
+    _native.host_call("apc_refine_labels_host", *_problem(g, theta, unary), int(max_rounds), lab)
     return lab
 
 
@@ -226,21 +203,6 @@ def prune_masks(g: LabelGraph, theta: np.ndarray, unary: np.ndarray, ub: float):
     end is dead."""
     bound, umin, emin = lower_bound(g, theta, unary)
     limit = ub + RELATIVE_MARGIN * max(abs(ub), 1.0)
-    lb = g.label_begin
-    label_bound = np.empty(len(unary))
-    for c in range(g.n_classes):
-        b = (bound - umin[c]) + unary[lb[c]:lb[c + 1]]
-        for t in range(int(g.inc_begin[c]), int(g.inc_begin[c + 1])):
-            k, side = int(g.inc_edge[t]), int(g.inc_side[t])
-            m = g.matrix(theta, k)
-            b = (b - emin[k]) + (m.min(axis=1) if side == 0 else m.min(axis=0))
-        label_bound[lb[c]:lb[c + 1]] = b
-    dead_label = ~(label_bound <= limit)
-    dead_pair = np.zeros(len(theta), bool)
-    for k in range(g.n_edges):
-        i, j = int(g.edge_i[k]), int(g.edge_j[k])
-        m = g.matrix(theta, k)
-        d = ~((bound - emin[k]) + m <= limit)
-        d |= dead_label[lb[i]:lb[i + 1]][:, None] | dead_label[lb[j]:lb[j + 1]][None, :]
-        dead_pair[int(g.edge_begin[k]):int(g.edge_begin[k + 1])] = d.ravel()
+    dead_label, dead_pair = np.empty(len(unary), bool), np.empty(len(theta), bool)
+    _native.host_call("apc_prune_masks_host", *_problem(g, theta, unary), umin, emin, float(bound), float(limit), dead_label, dead_pair)
     return dead_label, dead_pair

@@ -412,6 +412,40 @@ int apc_diffusion_sweeps(int32_t n_sweeps, int32_t n_colors, const int64_t *colo
                          const int64_t *edge_begin, const int32_t *edge_i, const int32_t *edge_j, int32_t max_labels,
                          double *theta, double *unary, void *stream);
 
+/* The index arrays of a labelling problem from its edges (HOST pointers): incidence lists in edge order
+ * (inc_begin [n_classes + 1], inc_edge / inc_side [2 n_edges]) and a colour per class (greedy, in class
+ * order: the smallest colour no neighbour has yet).  No counterpart in the reference. */
+int apc_label_incidence_host(int64_t n_classes, int64_t n_edges, const int32_t *edge_i_host, const int32_t *edge_j_host,
+                             int64_t *inc_begin_host, int32_t *inc_edge_host, uint8_t *inc_side_host, int64_t *color_host);
+
+/* The host's part of the pruning, between calls of the sweeps (HOST pointers; the arrays as above; no
+ * counterpart in the reference).  Sums run in incidence order.
+ *   apc_label_minima_host   minimum of every class's unary vector (0 without labels) and of every matrix
+ *   apc_round_labels_host   a labelling: classes in order, each takes its first cheapest label given the
+ *                           labels already taken by its neighbours and the best case for the rest (-1: no labels)
+ *   apc_refine_labels_host  local search from `labels`, in place: class by class the cheapest label given all
+ *                           neighbours' labels, until a round changes nothing (from the second round on only
+ *                           classes with a changed neighbour); at most max_rounds
+ *   apc_prune_masks_host    labels whose min-marginal bound, pairs whose entry bound exceeds `limit` (1 = dead; a
+ *                           pair with a dead end is dead); class_min / edge_min as above, bound = their sum */
+int apc_label_minima_host(int64_t n_classes, const int64_t *label_begin_host, const int64_t *inc_begin_host,
+                          const int32_t *inc_edge_host, const uint8_t *inc_side_host, int64_t n_edges, const int64_t *edge_begin_host,
+                          const int32_t *edge_i_host, const int32_t *edge_j_host, const double *theta_host, const double *unary_host,
+                          double *class_min_host, double *edge_min_host);
+int apc_round_labels_host(int64_t n_classes, const int64_t *label_begin_host, const int64_t *inc_begin_host,
+                          const int32_t *inc_edge_host, const uint8_t *inc_side_host, int64_t n_edges, const int64_t *edge_begin_host,
+                          const int32_t *edge_i_host, const int32_t *edge_j_host, const double *theta_host, const double *unary_host,
+                          int64_t *labels_host);
+int apc_refine_labels_host(int64_t n_classes, const int64_t *label_begin_host, const int64_t *inc_begin_host,
+                          const int32_t *inc_edge_host, const uint8_t *inc_side_host, int64_t n_edges, const int64_t *edge_begin_host,
+                          const int32_t *edge_i_host, const int32_t *edge_j_host, const double *theta_host, const double *unary_host,
+                          int64_t max_rounds, int64_t *labels_host);
+int apc_prune_masks_host(int64_t n_classes, const int64_t *label_begin_host, const int64_t *inc_begin_host,
+                          const int32_t *inc_edge_host, const uint8_t *inc_side_host, int64_t n_edges, const int64_t *edge_begin_host,
+                          const int32_t *edge_i_host, const int32_t *edge_j_host, const double *theta_host, const double *unary_host,
+                          const double *class_min_host, const double *edge_min_host, double bound, double limit,
+                          uint8_t *dead_label_host, uint8_t *dead_pair_host);
+
 /* apc_redistribute_tables for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the
  * reference.  It takes the tensor and strategy tables themselves instead of the staging tables
