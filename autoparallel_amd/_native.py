@@ -21,6 +21,7 @@ APC_TILE_MAX_COLS = 64
 APC_TILE_MAX_ROWS = 64
 APC_TILE_MAX_DUPS = 32
 APC_PACKED_MAX_DUPS = 16
+APC_SWEEP_MAX_WORKGROUPS = 224
 
 EDGE_GRAD_RESCALE = 1
 EDGE_NO_PRODUCER = 2
@@ -86,6 +87,8 @@ EXPORTS = (
     "apc_cost_objective",
     "apc_validate_row_minima_host",
     "apc_diffusion_sweeps",
+    "apc_sweep_plan_host",
+    "apc_diffusion_sweeps_resident",
     "apc_redistribute_tables_static",
     "apc_strategy_inputs",
     "apc_validate_packed_tiles_host",

@@ -12,6 +12,7 @@
 //   torch/_prims_common/__init__.py:252-292
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstddef>
@@ -2553,6 +2554,280 @@ __global__ __launch_bounds__(kBlock) void diffusion_node_update_kernel(Diffusion
   }
 }
 
+// ------------------------------------------------------------------------------------------
+// The same sweeps with the matrices resident on the chip.  A sweep of a planning program touches a
+// few hundred matrices of a few hundred elements; as one launch per colour it is a chain of 480
+// launches for 160 sweeps, each of which waits for the one before, reads its matrices and writes them
+// back: 7.6 us a launch on a two-dimensional mesh (34 000 elements), 134 us on a three-dimensional one
+// (977 000 elements), where a class's matrices no longer fit the staging arrays.  Here every workgroup keeps a run of
+// consecutive matrices in its LDS over all sweeps, and what moves between workgroups is the minima of
+// classes whose matrices lie in several of them.
+//   A step (one colour of one sweep) of a workgroup: the minima of its rows (columns) of that colour, a
+//   row by 1 to 16 lanes -> barrier -> the same lanes take their class's total, in incidence order, and
+//   update the elements they still hold in registers -> barrier, in front of which the next step's rows
+//   are fetched.  Element by element the arithmetic and its order are those of the launches above.
+//   Exchange: a slot per (incidence, label) in memory holds a minimum as two 64-bit words, each half of
+//   the value under the sweep's number, written and read by relaxed device-scope atomics: a reader
+//   that sees the number it waits for in both words has the value, so no flag, fence or cache
+//   maintenance is needed.  Two sets of slots in turn: a workgroup is at most one update of a class
+//   ahead of the others that hold matrices of it, because it needs their minima for its next one.
+//   Progress: all workgroups have to be resident (one per compute unit, at most
+//   APC_SWEEP_MAX_WORKGROUPS of 256; a second such kernel may hold the rest).  A wait that lasts longer
+//   than `wait_ticks` ends the kernel: the status word is set, every workgroup leaves at its own next
+//   wait, and the caller, whose inputs are untouched, takes the launches above instead.
+// Bound by latency: 0.8 us a step of a workgroup alone (LDS round trips and two barriers in a chain; one
+// wavefront per SIMD, so every instruction is on it), 1.4 - 1.7 us with an exchange.  160 sweeps, against one
+// launch per colour: 36 509 elements, three colours, 84 workgroups 3.65 -> 0.85 ms; 1 016 497 elements, 212
+// workgroups of 1024 threads 64 -> 1.39 ms.
+// ------------------------------------------------------------------------------------------
+// The plan of one workgroup, int32 words, 16-byte aligned:
+//   [0] first element of theta, [1] elements, [2] rows, [3] incidences, [4] steps (the colours it has rows of)
+//   rows         8 words each, colour by colour: first element | count << 16, step | label within its class << 16,
+//                slot or -1, first incidence | degree << 16; then where the minima of its class's first four
+//                incidences at this label are: a row here, or 0x40000000 | a slot, or (none) the row behind the last,
+//                which holds 0.0
+//   per row      its label's position in `unary`; | 0x80000000 where this row stores it
+//   incidences   of classes with more than four: as above, of label 0
+//   steps        the first row of each; behind the last: the number of rows
+// A row and its class's total belong to G consecutive lanes, the same ones in every sweep.
+constexpr int kResidentInverses = 64;  // reciprocals of the degrees below this many are kept
+
+struct ResidentArgs {
+  const int32_t *plan;
+  const int64_t *plan_begin;
+  const double *theta, *unary;
+  double *theta_out, *unary_out;
+  uint64_t *slots;
+  int64_t n_slots;
+  uint64_t wait_ticks;
+  int32_t *status;
+  int n_sweeps;
+};
+
+__global__ __launch_bounds__(kBlock) void resident_sweeps_begin_kernel(uint64_t *slots, int64_t n_words, const double *unary,
+                                                                       double *unary_out, int64_t n_labels, int32_t *status) {
+  const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (i < n_words) slots[i] = 0;
+  if (i < n_labels) unary_out[i] = unary[i];
+  if (i == 0) *status = 0;
+}
+
+__device__ __forceinline__ void publish_minimum(uint64_t *slot, double d, uint32_t number) {
+  const uint64_t tag = (uint64_t)number << 32;
+  __hip_atomic_store(slot, tag | (uint32_t)__double2loint(d), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(slot + 1, tag | (uint32_t)__double2hiint(d), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The smaller of two numbers in one instruction (a comparison and two selects otherwise).
+__device__ __forceinline__ double min_of(double a, double b) {
+  double m;
+  __asm__("v_min_f64 %0, %1, %2" : "=v"(m) : "v"(a), "v"(b));
+  return m;
+}
+
+// The minimum over `lanes` (uniform; 1, 2, 4, 8 or 16) consecutive lanes, in every lane: within a row of 16,
+// vector ALU only.
+template <int CTRL>
+__device__ __forceinline__ double min_with_dpp(double d) {
+  const int lo = __double2loint(d), hi = __double2hiint(d);
+  return min_of(d, __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false),
+                                    __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false)));
+}
+__device__ __forceinline__ double min_over_lanes(double d, int lanes) {
+  if (lanes >= 2) d = min_with_dpp<0xB1>(d);    // quad_perm [1, 0, 3, 2]
+  if (lanes >= 4) d = min_with_dpp<0x4E>(d);    // quad_perm [2, 3, 0, 1]
+  if (lanes >= 8) d = min_with_dpp<0x141>(d);   // row_half_mirror
+  if (lanes >= 16) d = min_with_dpp<0x140>(d);  // row_mirror
+  return d;
+}
+
+struct ResidentLds {
+  int4 *row;
+  double *m, *d, *un, *inv;
+  int *inc, *steps, *abort;
+};
+
+// A lane's row of a step; nothing a step writes, so it is fetched while the step before runs.
+struct ResidentRow {
+  int4 r, ref;
+  int q;      // -1: no row
+  int lanes;  // lanes per row (uniform): as many as keep the workgroup busy, at most 16
+};
+
+template <int T>
+__device__ __forceinline__ ResidentRow resident_row(const ResidentLds &l, int begin, int end, int tid) {
+  const int rb = uniform_i32(begin), re = uniform_i32(end), rows = re - rb;
+  const int shift = rows * 16 <= T ? 4 : rows * 8 <= T ? 3 : rows * 4 <= T ? 2 : rows * 2 <= T ? 1 : 0;
+  ResidentRow x;
+  x.lanes = 1 << shift;
+  x.q = rb + (tid >> shift);
+  const int q = min(x.q, re - 1);  // (a step has rows)
+  x.r = l.row[2 * q];
+  x.ref = l.row[2 * q + 1];
+  if (x.q >= re) x.q = -1;
+  return x;
+}
+
+// The minimum of an incidence at a label: here, or (`slot`) waited for.
+struct PendingMinima {
+  double e[4];
+  int ref[4];
+};
+
+// Waits for the minima that other workgroups publish; false when the wait expired.
+__device__ __forceinline__ bool await_minima(const uint64_t *slots, uint32_t number, uint64_t wait_ticks, PendingMinima &p) {
+  int pending = 0;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) pending |= (p.ref[u] & 0x40000000) ? 1 << u : 0;
+  const uint64_t began = wall_clock64();
+  while (pending) {
+    uint64_t lo[4], hi[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (pending & (1 << u)) {
+        const uint64_t *slot = slots + 2 * (int64_t)(p.ref[u] & 0x3FFFFFFF);
+        lo[u] = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        hi[u] = __hip_atomic_load(slot + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if ((pending & (1 << u)) && (uint32_t)(lo[u] >> 32) == number && (uint32_t)(hi[u] >> 32) == number) {
+        p.e[u] = __hiloint2double((int)(uint32_t)hi[u], (int)(uint32_t)lo[u]);
+        pending &= ~(1 << u);
+      }
+    if (pending && wall_clock64() - began > wait_ticks) return false;
+  }
+  return true;
+}
+
+// One step of a workgroup, `x` its rows; on return those of the next step.  False: a wait expired in the
+// workgroup (every thread returns the same).
+template <int T>
+__device__ __forceinline__ bool resident_step(const ResidentLds &l, const ResidentArgs &a, uint64_t *slots, uint32_t number, int n_rows,
+                                              ResidentRow &x, int next_step, int tid) {
+  // Elements of a row that a lane holds between its minimum and its update.  A lane past the row's end
+  // holds its last element once more: the same value, stored again.
+  constexpr int kHeld = 4;
+  const double inf = __builtin_inf();
+  const int lanes = uniform_i32(x.lanes), sub = tid & (lanes - 1);
+  const int last = (int)((uint32_t)x.r.x >> 16) - 1, stride = x.r.y & 0xFFFF, label = (int)((uint32_t)x.r.y >> 16);
+  const int degree = (int)((uint32_t)x.r.w >> 16);
+  const bool live = x.q >= 0;
+  double *const m = l.m + (x.r.x & 0xFFFF);
+  int at[kHeld];
+  double v[kHeld];
+#pragma unroll
+  for (int u = 0; u < kHeld; ++u) {
+    at[u] = __mul24(min(sub + u * lanes, last), stride);
+    v[u] = m[at[u]];
+  }
+  const int expired_before = *l.abort;  // (written between the two barriers of a step, read outside of them)
+  const double unary = l.un[max(x.q, 0)], inv = l.inv[min(degree, kResidentInverses - 1)];
+  const int next_begin = l.steps[next_step], next_end = l.steps[next_step + 1];
+  double d = min_of(min_of(v[0], v[1]), min_of(v[2], v[3]));
+  for (int y = sub + kHeld * lanes; y <= last; y += lanes) d = min_of(m[__mul24(y, stride)], d);
+  if (uniform_i32(expired_before)) return false;
+  d = min_over_lanes(d, lanes);
+  if (sub == 0 && live) {
+    l.d[x.q] = d;
+    if (x.r.z >= 0) publish_minimum(slots + 2 * (int64_t)x.r.z, d, number);
+  }
+  const ResidentRow next = resident_row<T>(l, next_begin, next_end, tid);
+  __syncthreads();
+  if (live) {
+    PendingMinima p;
+    p.ref[0] = x.ref.x;
+    p.ref[1] = x.ref.y;
+    p.ref[2] = x.ref.z;
+    p.ref[3] = x.ref.w;
+    bool expired = false;
+    auto add = [&](double tot) {
+      int remote = 0;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        p.e[u] = l.d[(p.ref[u] & 0x40000000) ? n_rows : p.ref[u]];
+        remote |= p.ref[u];
+      }
+      if (remote & 0x40000000) expired = !await_minima(slots, number, a.wait_ticks, p);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) tot += p.e[u];  // (none: + 0.0)
+      return tot;
+    };
+    double tot = add(unary);
+    for (int t = 4; t < degree && !expired; t += 4) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) p.ref[u] = t + u < degree ? l.inc[(x.r.w & 0xFFFF) + t + u] + label : n_rows;
+      tot = add(tot);
+    }
+    if (expired) *l.abort = 1;
+    const bool finite = tot < inf;  // (then every minimum of the class is finite)
+    // (the quotient through the reciprocal is the division's: div_by)
+    double share = div_by(tot, (double)degree, inv);
+    if (degree >= kResidentInverses) share = tot / (double)degree;
+    if (sub == 0) l.un[x.q] = finite ? 0.0 : inf;
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) m[at[u]] = finite ? (v[u] - d) + share : inf;  // (a label that can never be taken: +inf)
+    for (int y = sub + kHeld * lanes; y <= last; y += lanes) {
+      double *const e = m + __mul24(y, stride);
+      *e = finite ? (*e - d) + share : inf;
+    }
+  }
+  x = next;
+  __syncthreads();
+  return true;
+}
+
+template <int T>
+__global__ __launch_bounds__(T) void diffusion_resident_kernel(ResidentArgs a) {
+  extern __shared__ __align__(16) unsigned char s_bytes[];
+  const int tid = threadIdx.x;
+  const int32_t *plan = a.plan + a.plan_begin[blockIdx.x];
+  const int64_t first = plan[0];
+  const int n_el = plan[1], n_rows = plan[2], n_inc = plan[3], n_steps = plan[4];
+  // the layout of LDS (apc_sweep_plan_host counts the same bytes)
+  ResidentLds l;
+  l.row = reinterpret_cast<int4 *>(s_bytes);
+  l.m = reinterpret_cast<double *>(l.row + 2 * n_rows);
+  l.d = l.m + n_el;  // (one more than rows: 0.0)
+  l.un = l.d + n_rows + 1;
+  l.inv = l.un + n_rows;
+  l.inc = reinterpret_cast<int *>(l.inv + kResidentInverses);
+  l.steps = l.inc + n_inc;
+  l.abort = l.steps + n_steps + 1;
+  const int4 *rows = reinterpret_cast<const int4 *>(plan + 8);
+  const int32_t *labels = reinterpret_cast<const int32_t *>(rows + 2 * n_rows);
+  const int32_t *incs = labels + n_rows;  // (the steps follow)
+  for (int i = tid; i < 2 * n_rows; i += T) l.row[i] = rows[i];
+  for (int i = tid; i < n_rows; i += T) l.un[i] = a.unary[labels[i] & 0x7FFFFFFF];
+  for (int i = tid; i < n_el; i += T) l.m[i] = a.theta[first + i];
+  for (int i = tid; i < n_inc + n_steps + 1; i += T) l.inc[i] = incs[i];
+  for (int i = tid; i < kResidentInverses; i += T) l.inv[i] = i > 0 ? 1.0 / (double)i : 0.0;
+  if (tid == 0) {
+    *l.abort = 0;
+    l.d[n_rows] = 0.0;
+  }
+  __syncthreads();
+  ResidentRow x = resident_row<T>(l, l.steps[0], l.steps[1], tid);
+  for (int sweep = 0; sweep < a.n_sweeps; ++sweep) {
+    const uint32_t number = (uint32_t)sweep + 1;
+    uint64_t *slots = a.slots + (sweep & 1) * 2 * a.n_slots;
+    for (int step = 0; step < n_steps; ++step)
+      if (!resident_step<T>(l, a, slots, number, n_rows, x, step + 1 < n_steps ? step + 1 : 0, tid)) {  // (uniform)
+        if (tid == 0) __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return;
+      }
+  }
+  if (*l.abort) {  // (set in the very last step, behind whose barrier this is)
+    if (tid == 0) __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
+  for (int i = tid; i < n_el; i += T) a.theta_out[first + i] = l.m[i];
+  for (int i = tid; i < n_rows; i += T) {
+    const int32_t label = labels[i];
+    if (label < 0) a.unary_out[label & 0x7FFFFFFF] = l.un[i];
+  }
+}
+
 inline unsigned blocks_for(int64_t n, int per_block) { return (unsigned)((n + per_block - 1) / per_block); }
 
 template <int G>
@@ -3003,6 +3278,35 @@ int apc_diffusion_sweeps(int32_t n_sweeps, int32_t n_colors, const int64_t *colo
     if (int rc = check_launch("apc_diffusion_sweeps")) return rc;
   }
   return 0;
+}
+
+int apc_diffusion_sweeps_resident(int32_t n_sweeps, int64_t n_workgroups, const int32_t *plan, const int64_t *plan_begin,
+                                  int64_t n_slots, int64_t lds_bytes, int32_t threads,
+                                  int64_t n_labels, const double *theta, const double *unary,
+                                  double *theta_out, double *unary_out, uint64_t *slots, uint64_t wait_ticks, int32_t *status,
+                                  void *stream) {
+  if (n_sweeps < 0 || n_slots < 0 || n_labels < 0) return fail(-1, "apc_diffusion_sweeps_resident: negative count");
+  if (n_workgroups < 1 || n_workgroups > APC_SWEEP_MAX_WORKGROUPS)
+    return fail(-1, "apc_diffusion_sweeps_resident: %lld workgroups, 1 .. %d can be resident", (long long)n_workgroups, APC_SWEEP_MAX_WORKGROUPS);
+  if (lds_bytes < 1 || lds_bytes > APC_SWEEP_LDS_BYTES)
+    return fail(-1, "apc_diffusion_sweeps_resident: %lld bytes of LDS, at most %d", (long long)lds_bytes, APC_SWEEP_LDS_BYTES);
+  if (threads != 256 && threads != 1024) return fail(-1, "apc_diffusion_sweeps_resident: workgroups of 256 or 1024 threads (%d)", threads);
+  if (!plan || !plan_begin || !theta || !unary || !theta_out || !unary_out || !status || (n_slots > 0 && !slots))
+    return fail(-1, "apc_diffusion_sweeps_resident: NULL array");
+  if (theta == theta_out || unary == unary_out) return fail(-1, "apc_diffusion_sweeps_resident: the outputs are arrays of their own");
+  hipStream_t s = (hipStream_t)stream;
+  const int64_t words = 4 * n_slots;  // two sets of two words
+  const int64_t n = std::max<int64_t>({words, n_labels, 1});
+  hipLaunchKernelGGL(resident_sweeps_begin_kernel, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s, slots, words, unary, unary_out, n_labels, status);
+  // at least half a compute unit's LDS plus a little: one workgroup per compute unit
+  const size_t lds = (size_t)std::max<int64_t>((lds_bytes + 15) / 16 * 16, 84 * 1024);
+  const void *kernel = threads == 256 ? reinterpret_cast<const void *>(diffusion_resident_kernel<256>) : reinterpret_cast<const void *>(diffusion_resident_kernel<1024>);
+  hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return fail(-3, "apc_diffusion_sweeps_resident: %s", hipGetErrorString(e));
+  const ResidentArgs a{plan, plan_begin, theta, unary, theta_out, unary_out, slots, n_slots, wait_ticks, status, n_sweeps};
+  if (threads == 256) hipLaunchKernelGGL(diffusion_resident_kernel<256>, dim3((unsigned)n_workgroups), dim3(256), lds, s, a);
+  else hipLaunchKernelGGL(diffusion_resident_kernel<1024>, dim3((unsigned)n_workgroups), dim3(1024), lds, s, a);
+  return check_launch("apc_diffusion_sweeps_resident");
 }
 
 }  // extern "C"

@@ -929,6 +929,170 @@ int apc_prune_masks_host(APC_LABEL_PROBLEM, const double *class_min, const doubl
   return 0;
 }
 
+// ------------------------------------------------------------------------------------------
+// Which workgroup of apc_diffusion_sweeps_resident holds which matrices, and what it needs to know
+// about them: the layout is stated at the kernel (ResidentPlan in apcost.hip).
+// ------------------------------------------------------------------------------------------
+int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin, const int64_t *inc_begin, const int32_t *inc_edge,
+                        const uint8_t *inc_side, int64_t n_edges, const int64_t *edge_begin, const int32_t *edge_i,
+                        const int32_t *edge_j, int64_t n_colors, const int64_t *color_begin, const int32_t *color_nodes,
+                        int64_t max_workgroups, int64_t capacity_words, int32_t *plan, int64_t *plan_begin, int64_t *sizes) {
+  const LabelProblem g{n_classes, n_edges, label_begin, inc_begin, inc_edge, inc_side, edge_begin, edge_i, edge_j, nullptr, nullptr};
+  if (!g.holds()) return fail(-2, "apc_sweep_plan_host: the index arrays do not describe a labelling problem");
+  if (!plan || !plan_begin || !sizes || !color_begin || max_workgroups < 1 || n_colors < 0) return fail(-1, "apc_sweep_plan_host: NULL array or no workgroup");
+  std::fill(sizes, sizes + 5, 0);
+  if (color_begin[0] != 0 || color_begin[n_colors] != n_classes) return fail(-2, "apc_sweep_plan_host: the colours must partition the classes");
+  std::vector<int32_t> color(n_classes, -1);
+  for (int64_t c = 0; c < n_colors; ++c)
+    for (int64_t k = color_begin[c]; k < color_begin[c + 1]; ++k) {
+      if (k < 0 || k >= n_classes || color_nodes[k] < 0 || color_nodes[k] >= n_classes) return fail(-2, "apc_sweep_plan_host: class out of range");
+      color[color_nodes[k]] = (int32_t)c;
+    }
+  for (int64_t k = 0; k < n_edges; ++k)
+    if (color[edge_i[k]] < 0 || color[edge_j[k]] < 0 || color[edge_i[k]] == color[edge_j[k]])
+      return fail(-2, "apc_sweep_plan_host: edge %lld joins two classes of one colour", (long long)k);
+  for (int64_t k = 0; k < n_edges; ++k)
+    if (edge_begin[k + 1] == edge_begin[k]) return 0;  // (an empty matrix: left to the launches)
+  if (n_edges == 0) return 0;  // (no plan: sizes[0] stays 0)
+  // Edges in order, workgroup by workgroup, until its share of the elements, its threads (one per row of a step)
+  // or its memory is full.  (Neighbouring edges of a planning program share classes: kept together, most
+  // exchanges stay inside a workgroup.)  256 threads, one wavefront per SIMD, unless that takes too many workgroups.
+  const int64_t total = edge_begin[n_edges];
+  int64_t share = std::max<int64_t>(APC_SWEEP_MIN_ELEMENTS, (total + APC_SWEEP_AIM_WORKGROUPS - 1) / APC_SWEEP_AIM_WORKGROUPS);
+  std::vector<int32_t> owner(n_edges);
+  auto bytes = [&](int64_t el, int64_t r, int64_t in) { return 8 * (el + 1) + (32 + 8 + 8) * r + 8 * 64 + 4 * in + 4 * (n_colors + 1) + 16; };
+  int64_t lds = 0, n_wg = 0;
+  auto assign = [&](int64_t threads) {
+    std::vector<int64_t> seen(n_classes, -1);  // the last workgroup that met the class
+    std::vector<int64_t> step_rows(n_colors, 0);
+    int64_t elements = 0, rows = 0, incs = 0;
+    n_wg = lds = 0;
+    for (int64_t k = 0; k < n_edges; ++k) {
+      const int64_t size = edge_begin[k + 1] - edge_begin[k], ni = g.labels(edge_i[k]), nj = g.labels(edge_j[k]);
+      for (int attempt = 0;; ++attempt) {
+        int64_t in = incs;
+        for (int64_t c : {edge_i[k], edge_j[k]})
+          if (seen[c] != n_wg) in += inc_begin[c + 1] - inc_begin[c];
+        int64_t &ri = step_rows[color[edge_i[k]]], &rj = step_rows[color[edge_j[k]]];
+        const bool fits = bytes(elements + size, rows + ni + nj, in) <= APC_SWEEP_LDS_BYTES && elements + size <= 0x10000 && in <= 0xFFFF &&
+                          ri + ni <= threads && rj + nj <= threads;
+        if (fits && (rows == 0 || elements + size <= share)) {
+          elements += size, rows += ni + nj, incs = in, ri += ni, rj += nj;
+          seen[edge_i[k]] = seen[edge_j[k]] = n_wg;
+          lds = std::max(lds, bytes(elements, rows, incs));
+          owner[k] = (int32_t)n_wg;
+          break;
+        }
+        if (attempt == 1 || rows == 0) return false;  // one matrix alone does not fit
+        ++n_wg;
+        elements = rows = incs = 0;
+        std::fill(step_rows.begin(), step_rows.end(), 0);
+      }
+    }
+    return ++n_wg <= max_workgroups;
+  };
+  // (the matrices do not fill the shares exactly: larger ones until the workgroups are few enough)
+  int64_t threads = 0;
+  for (int attempt = 0;; ++attempt, share += share / 4) {
+    threads = share > APC_SWEEP_WIDE_ELEMENTS ? 1024 : 256;
+    if (assign(threads) || assign(threads = 1024)) break;
+    if (attempt == 12) return 0;
+  }
+  // classes whose matrices lie in several workgroups exchange their minima through memory: a slot per (incidence, label)
+  std::vector<int64_t> slot(inc_begin[n_classes], -1);
+  int64_t n_slots = 0;
+  for (int64_t c = 0; c < n_classes; ++c) {
+    bool shared = false;
+    for (int64_t t = inc_begin[c]; t < inc_begin[c + 1]; ++t) shared |= owner[inc_edge[t]] != owner[inc_edge[inc_begin[c]]];
+    if (!shared) continue;
+    for (int64_t t = inc_begin[c]; t < inc_begin[c + 1]; ++t) {
+      slot[t] = n_slots;
+      n_slots += g.labels(c);
+    }
+  }
+  if (n_slots > 0x3FFFFFFF || total > INT32_MAX) return 0;
+  std::vector<int64_t> inc_of(2 * n_edges);  // (edge, side) -> incidence
+  for (int64_t t = 0; t < inc_begin[n_classes]; ++t) inc_of[2 * (int64_t)inc_edge[t] + inc_side[t]] = t;
+  int64_t at = 0;
+  std::vector<int64_t> row_of(2 * n_edges, 0), inc_at(n_classes, 0), met(n_classes, -1);
+  for (int64_t w = 0, first = 0; w < n_wg; ++w) {
+    int64_t last = first;
+    while (last < n_edges && owner[last] == w) ++last;
+    struct Side {  // one side of an edge: the rows of its class
+      int64_t k;
+      int side;
+      int64_t c;
+    };
+    std::vector<Side> sides;
+    for (int64_t k = first; k < last; ++k) sides.push_back({k, 0, edge_i[k]}), sides.push_back({k, 1, edge_j[k]});
+    std::stable_sort(sides.begin(), sides.end(), [&](const Side &x, const Side &y) { return color[x.c] < color[y.c]; });
+    int64_t n_rows = 0, n_inc = 0, n_el = 0;
+    std::vector<int64_t> classes;
+    std::vector<int64_t> steps;  // first rows of the colours that have any
+    int32_t last_color = -1;
+    for (const Side &x : sides) {
+      if (color[x.c] != last_color) {
+        steps.push_back(n_rows);
+        last_color = color[x.c];
+      }
+      row_of[2 * x.k + x.side] = n_rows;
+      n_rows += g.labels(x.c);
+      if (met[x.c] != w) {
+        met[x.c] = w;
+        classes.push_back(x.c);
+        inc_at[x.c] = n_inc;
+        n_inc += inc_begin[x.c + 1] - inc_begin[x.c];
+      }
+    }
+    steps.push_back(n_rows);
+    std::vector<int64_t> el_of(last - first);
+    for (int64_t k = first; k < last; ++k) {
+      el_of[k - first] = n_el;
+      n_el += edge_begin[k + 1] - edge_begin[k];
+    }
+    const int64_t words = (8 + 9 * n_rows + n_inc + (int64_t)steps.size() + 3) / 4 * 4;
+    if (at + words > capacity_words) return fail(-1, "apc_sweep_plan_host: the plan does not fit %lld words", (long long)capacity_words);
+    plan_begin[w] = at;
+    int32_t *p = plan + at;
+    std::fill(p, p + words, 0);
+    p[0] = (int32_t)edge_begin[first];  // (a workgroup's edges are consecutive: one run of theta)
+    p[1] = (int32_t)n_el;
+    p[2] = (int32_t)n_rows;
+    p[3] = (int32_t)n_inc;
+    p[4] = (int32_t)steps.size() - 1;
+    int32_t *q = p + 8, *label = p + 8 + 8 * n_rows;
+    // where the minima of incidence t at label 0 are: a row here, or a slot
+    auto place = [&](int64_t t) {
+      return owner[inc_edge[t]] == w ? row_of[2 * (int64_t)inc_edge[t] + inc_side[t]] : slot[t] | 0x40000000;
+    };
+    for (const Side &x : sides) {  // in the order of row_of
+      const int64_t nj = g.labels(edge_j[x.k]), ni = g.labels(edge_i[x.k]), n = g.labels(x.c), t = inc_of[2 * x.k + x.side];
+      const int64_t degree = inc_begin[x.c + 1] - inc_begin[x.c];
+      for (int64_t y = 0; y < n; ++y, q += 8) {
+        q[0] = (int32_t)(uint32_t)((el_of[x.k - first] + (x.side == 0 ? y * nj : y)) | ((x.side == 0 ? nj : ni) << 16));
+        q[1] = (int32_t)(uint32_t)((x.side == 0 ? 1 : nj) | (y << 16));
+        q[2] = slot[t] >= 0 ? (int32_t)(slot[t] + y) : -1;
+        q[3] = (int32_t)(uint32_t)(inc_at[x.c] | (degree << 16));
+        for (int64_t u = 0; u < 4; ++u) q[4 + u] = u < degree ? (int32_t)(place(inc_begin[x.c] + u) + y) : (int32_t)n_rows;
+        *label++ = (int32_t)((uint32_t)(label_begin[x.c] + y) | (t == inc_begin[x.c] ? 0x80000000u : 0u));  // (its first matrix stores a class)
+      }
+    }
+    q = label;
+    for (int64_t c : classes)
+      for (int64_t t = inc_begin[c]; t < inc_begin[c + 1]; ++t) *q++ = (int32_t)place(t);
+    for (int64_t r : steps) *q++ = (int32_t)r;
+    at += words;
+    first = last;
+  }
+  plan_begin[n_wg] = at;
+  sizes[0] = n_wg;
+  sizes[1] = at;
+  sizes[2] = n_slots;
+  sizes[3] = lds;
+  sizes[4] = threads;
+  return 0;
+}
+
 #undef APC_LABEL_PROBLEM
 #undef APC_LABEL_PROBLEM_OF
 

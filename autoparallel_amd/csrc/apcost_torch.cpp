@@ -778,6 +778,31 @@ void diffusion_sweeps_(int64_t n_sweeps, const Tensor &color_begin, const Tensor
   });
 }
 
+// The same sweeps with the matrices resident on the chip (apc_diffusion_sweeps_resident), out of place:
+// -> theta, unary, status (int32[1]; 1: a wait expired, the outputs are unusable).
+std::tuple<Tensor, Tensor, Tensor> diffusion_sweeps_resident(int64_t n_sweeps, const Tensor &plan, const Tensor &plan_begin, int64_t n_slots,
+                                                             int64_t lds_bytes, int64_t threads, int64_t n_labels_total, int64_t n_elements,
+                                                             const Tensor &theta, const Tensor &unary, int64_t wait_ticks) {
+  const int32_t *words = dev<int32_t>(plan, at::kInt, "plan");
+  const int64_t *begin = dev<int64_t>(plan_begin, at::kLong, "plan_begin");
+  const double *th = dev<double>(theta, at::kDouble, "theta"), *un = dev<double>(unary, at::kDouble, "unary");
+  TORCH_CHECK(plan_begin.numel() >= 2, "apcost: plan_begin needs n_workgroups + 1 rows");
+  TORCH_CHECK(unary.numel() == n_labels_total, "apcost: unary has ", unary.numel(), " values, the plan's problem ", n_labels_total, " labels");
+  TORCH_CHECK(theta.numel() == n_elements, "apcost: theta has ", theta.numel(), " values, the plan's problem ", n_elements, " elements");
+  TORCH_CHECK(wait_ticks >= 0, "apcost: wait_ticks must not be negative");
+  TORCH_CHECK(n_sweeps >= 0 && n_sweeps <= INT32_MAX, "apcost: n_sweeps ", n_sweeps, " out of range");
+  for (const Tensor *t : {&plan, &plan_begin, &unary}) same_device(theta, *t, "an array");
+  Tensor theta_out = at::empty_like(theta), unary_out = at::empty_like(unary), status = empty_like_device(theta, {1}, at::kInt),
+         slots = empty_like_device(theta, {4 * n_slots}, at::kLong);
+  on_current_stream(theta.device(), "apc_diffusion_sweeps_resident", [&](void *s) {
+    return apc_diffusion_sweeps_resident((int32_t)n_sweeps, plan_begin.numel() - 1, words, begin, n_slots, lds_bytes, (int32_t)threads, n_labels_total, th, un,
+                                         static_cast<double *>(theta_out.data_ptr()), static_cast<double *>(unary_out.data_ptr()),
+                                         reinterpret_cast<uint64_t *>(n_slots ? slots.data_ptr<int64_t>() : nullptr), (uint64_t)wait_ticks,
+                                         status.data_ptr<int32_t>(), s);
+  });
+  return {theta_out, unary_out, status};
+}
+
 // Flop and byte counts of every (node, strategy) from the spec table's local shapes and the
 // per-node recipes (compute_estimation.py:232-299, 334-349; apc_strategy_inputs).
 std::tuple<Tensor, Tensor, Tensor, Tensor> strategy_inputs(const Tensor &strat_node, const Tensor &node_strat_begin,
@@ -904,6 +929,9 @@ TORCH_LIBRARY(apcost, m) {
         "Tensor inc_edge, Tensor inc_side, Tensor edge_begin, Tensor edge_i, Tensor edge_j, int max_labels, int n_labels_total, int n_elements, Tensor(a!) theta, "
         "Tensor(b!) unary) -> ()",
         &diffusion_sweeps_);
+  m.def("diffusion_sweeps_resident(int n_sweeps, Tensor plan, Tensor plan_begin, int n_slots, int lds_bytes, int threads, "
+        "int n_labels_total, int n_elements, Tensor theta, Tensor unary, int wait_ticks) -> (Tensor theta, Tensor unary, Tensor status)",
+        &diffusion_sweeps_resident);
   m.def("bind_tensor_tables(" APCOST_TENSOR_TABLE ", Tensor tensor_bytes, Tensor tensor_contiguous) -> __torch__.torch.classes.apcost.BoundLaunch",
         &bind_tensor_tables);
   m.def("bind_spec_tables(Tensor params, Tensor spec_codes, Tensor spec_tensor, " APCOST_TENSOR_TABLE

@@ -557,45 +557,67 @@ class DeviceCostTables:
         return self.ops.segmented_min(values, seg_ptr)
 
     # ---- dual ascent over the planning program's labelling form ---------------------------------
+    # A wait of the resident sweeps for another workgroup's minima: microseconds when all workgroups are on the
+    # chip.  One that lasts this long (100 MHz ticks: 0.2 s) means that they are not, and ends the kernel.
+    SWEEP_WAIT_TICKS = 20_000_000
+
+    @staticmethod
+    def _sweep_plan(graph):
+        """-> (plan words, first word of every workgroup, slots, bytes of LDS, threads) of the resident sweeps
+        (``apc_sweep_plan_host``), None when the problem does not fit the chip's LDS."""
+        most = _native.APC_SWEEP_MAX_WORKGROUPS
+        labels, degree = np.diff(graph.label_begin), np.diff(graph.inc_begin)
+        ends = np.concatenate([graph.edge_i, graph.edge_j])
+        n_colors = len(graph.color_begin) - 1
+        capacity = (n_colors + 16) * most + int((9 * labels + degree)[ends].sum())
+        plan, begin, sizes = np.empty(capacity, np.int32), np.empty(most + 1, np.int64), np.empty(5, np.int64)
+        _native.host_call("apc_sweep_plan_host", graph.n_classes, graph.label_begin, graph.inc_begin, graph.inc_edge, graph.inc_side,
+                          graph.n_edges, graph.edge_begin, graph.edge_i, graph.edge_j, n_colors, graph.color_begin,
+                          graph.color_nodes, most, capacity, plan, begin, sizes)
+        n, words, *rest = sizes.tolist()
+        return (plan[:words], begin[:n + 1], *rest) if n else None
+
     @_guarded
     def diffusion_sweeps(self, graph, theta: np.ndarray, unary: np.ndarray, n_sweeps: int):
-        """``n_sweeps`` sweeps of min-sum diffusion (``apc_diffusion_sweeps``) over ``graph``
-        (``pruning.LabelGraph``) starting from the host arrays ``theta`` / ``unary``; returns the
-        updated pair as new host arrays (read-only: handed back to the next call unchanged, they
-        are not uploaded again).  The graph's index arrays are uploaded once, as one buffer."""
+        """``n_sweeps`` sweeps of min-sum diffusion over ``graph`` (``pruning.LabelGraph``) starting
+        from the host arrays ``theta`` / ``unary``; returns the updated pair as new host arrays
+        (read-only: handed back to the next call unchanged, they are not uploaded again).  A problem
+        that fits the chip's LDS takes one kernel for all sweeps (``apc_diffusion_sweeps_resident``), any
+        other one launch per colour (``apc_diffusion_sweeps``); the same bits.  What either needs of the
+        graph is worked out and uploaded once."""
         cached = getattr(self, "_diffusion_graph", None)
-        if cached is None or cached[0] is not graph:
-            names = ("color_nodes", "label_begin", "inc_begin", "inc_edge", "inc_side", "edge_begin", "edge_i", "edge_j")
-            # one host buffer, one copy: every array at a 16-byte boundary, viewed with its own dtype on the device
-            arrays = {k: np.ascontiguousarray(getattr(graph, k)) for k in names}
-            offsets, size = {}, 0
-            for k, a in arrays.items():
-                offsets[k] = size
-                size += -(-a.nbytes // 16) * 16
-            packed = np.zeros(max(size, 16), np.uint8)
-            for k, a in arrays.items():
-                packed[offsets[k]:offsets[k] + a.nbytes] = a.view(np.uint8).reshape(-1)
-            on_device = torch.from_numpy(packed).to(self.device)
-            views = {k: on_device[offsets[k]:offsets[k] + a.nbytes].view(_TORCH_DTYPE[a.dtype.type]) for k, a in arrays.items()}
-            cached = (graph, views, on_device)
-            self._diffusion_graph = cached
+        if cached is None or cached["graph"] is not graph:
+            cached = self._diffusion_graph = {"graph": graph, "plan": self._sweep_plan(graph)}
             self._diffusion_state = None
-        d = cached[1]
         state = getattr(self, "_diffusion_state", None)
         if state is not None and state[0] is theta and state[1] is unary:
             th, un = state[2], state[3]  # what the last call left on the device, returned as these very arrays
         else:
-            th = torch.from_numpy(np.ascontiguousarray(theta, np.float64)).to(self.device)
-            un = torch.from_numpy(np.ascontiguousarray(unary, np.float64)).to(self.device)
-        color_begin = torch.from_numpy(np.ascontiguousarray(graph.color_begin, np.int64))
-        max_labels = int(np.diff(graph.label_begin).max()) if graph.n_classes else 0
-        self.ops.diffusion_sweeps_(int(n_sweeps), color_begin, d["color_nodes"], d["label_begin"], d["inc_begin"],
-                                   d["inc_edge"], d["inc_side"], d["edge_begin"], d["edge_i"], d["edge_j"], max_labels,
-                                   int(graph.label_begin[-1]), int(graph.edge_begin[-1]), th, un)
-        theta_out, unary_out = th.cpu().numpy(), un.cpu().numpy()
+            th, un = self._upload(np.ascontiguousarray(theta, np.float64), np.ascontiguousarray(unary, np.float64))
+        plan = cached["plan"]
+        if plan is not None and "on_device" not in cached:
+            cached["on_device"] = self._upload(*plan[:2])
+        out = None
+        if plan is not None:
+            *pair, status = self.ops.diffusion_sweeps_resident(
+                int(n_sweeps), *cached["on_device"], *plan[2:], int(graph.label_begin[-1]), int(graph.edge_begin[-1]), th, un,
+                self.SWEEP_WAIT_TICKS)
+            theta_out, unary_out, flag = (t.numpy() for t in self.ops.download([*pair, status]))
+            if int(flag[0]) == 0:
+                out = pair
+        if out is None:
+            d = cached.get("index")
+            if d is None:
+                names = ("color_nodes", "label_begin", "inc_begin", "inc_edge", "inc_side", "edge_begin", "edge_i", "edge_j")
+                d = cached["index"] = self._upload(*(getattr(graph, k) for k in names))
+            out = (th, un)
+            max_labels = int(np.diff(graph.label_begin).max()) if graph.n_classes else 0
+            self.ops.diffusion_sweeps_(int(n_sweeps), torch.from_numpy(np.ascontiguousarray(graph.color_begin, np.int64)), *d, max_labels,
+                                       int(graph.label_begin[-1]), int(graph.edge_begin[-1]), *out)
+            theta_out, unary_out = (t.numpy() for t in self.ops.download(list(out)))
         theta_out.setflags(write=False)
         unary_out.setflags(write=False)
-        self._diffusion_state = (theta_out, unary_out, th, un)
+        self._diffusion_state = (theta_out, unary_out, *out)
         return theta_out, unary_out
 
     @_guarded

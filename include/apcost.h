@@ -412,6 +412,32 @@ int apc_diffusion_sweeps(int32_t n_sweeps, int32_t n_colors, const int64_t *colo
                          const int64_t *edge_begin, const int32_t *edge_i, const int32_t *edge_j, int32_t max_labels,
                          double *theta, double *unary, void *stream);
 
+/* The same sweeps, same bits, with the matrices resident in the compute units' LDS: one kernel for all
+ * sweeps instead of one launch per colour.  Out of place: theta / unary are read, theta_out / unary_out
+ * written.  apc_sweep_plan_host (HOST pointers) assigns the matrices to workgroups: plan_host holds at most
+ * capacity_words = 9 * (sum over edges of the label counts of both ends) + sum over edges of the degrees of both
+ * ends + max_workgroups * (n_colors + 16) words, plan_begin_host max_workgroups + 1 rows; sizes_host receives
+ * {workgroups, words, slots, bytes of LDS, threads per workgroup}, workgroups 0 when the problem does not fit (a matrix larger than a workgroup's share of LDS, too many workgroups or
+ * colours).  slots: 4 * n_slots words of device memory, cleared by the call.
+ * The workgroups wait for each other's minima, so all of them have to be resident: at most
+ * APC_SWEEP_MAX_WORKGROUPS, one per compute unit.  A wait longer than wait_ticks (100 MHz) ends the kernel
+ * with *status (device int32) = 1 and unusable outputs; the caller then runs apc_diffusion_sweeps on the
+ * inputs.  *status = 0: the outputs are complete. */
+#define APC_SWEEP_MAX_WORKGROUPS 224
+#define APC_SWEEP_LDS_BYTES (150 * 1024)
+#define APC_SWEEP_MIN_ELEMENTS 256    /* a workgroup's share of the matrix elements: at least this many, */
+#define APC_SWEEP_AIM_WORKGROUPS 200  /* or what spreads the problem over this many workgroups; */
+#define APC_SWEEP_WIDE_ELEMENTS 1536  /* above this many, workgroups of 1024 threads instead of 256 */
+int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin_host, const int64_t *inc_begin_host,
+                        const int32_t *inc_edge_host, const uint8_t *inc_side_host, int64_t n_edges, const int64_t *edge_begin_host,
+                        const int32_t *edge_i_host, const int32_t *edge_j_host, int64_t n_colors, const int64_t *color_begin_host,
+                        const int32_t *color_nodes_host, int64_t max_workgroups, int64_t capacity_words, int32_t *plan_host,
+                        int64_t *plan_begin_host, int64_t *sizes_host);
+int apc_diffusion_sweeps_resident(int32_t n_sweeps, int64_t n_workgroups, const int32_t *plan, const int64_t *plan_begin,
+                                  int64_t n_slots, int64_t lds_bytes, int32_t threads, int64_t n_labels, const double *theta, const double *unary,
+                                  double *theta_out, double *unary_out, uint64_t *slots, uint64_t wait_ticks, int32_t *status,
+                                  void *stream);
+
 /* The index arrays of a labelling problem from its edges (HOST pointers): incidence lists in edge order
  * (inc_begin [n_classes + 1], inc_edge / inc_side [2 n_edges]) and a colour per class (greedy, in class
  * order: the smallest colour no neighbour has yet).  No counterpart in the reference. */

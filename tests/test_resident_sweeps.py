@@ -1,0 +1,109 @@
+"""Sweeps of the dual ascent with the matrices resident on the chip (apc_diffusion_sweeps_resident)
+against the oracle's sweeps, bit for bit, at the sizes that choose workgroups, lanes per row and exchanges;
+the plan they run from; and the way out when a wait expires."""
+
+import numpy as np
+import pytest
+
+from autoparallel_amd import CostModelParams, pruning
+from autoparallel_amd.synthetic import stress_dag
+from test_pruning import _sweep
+
+
+def _problem(seed, sizes, pairs, p_inf=0.1):
+    rng = np.random.default_rng(seed)
+    blocks, costs, at = [], {}, 0
+    for i, j in pairs:
+        m = rng.uniform(0, 100, (sizes[i], sizes[j]))
+        m[rng.random(m.shape) < p_inf] = np.inf
+        blocks.append(pruning.Block(at, sizes[i], sizes[j], i, j))
+        costs[at] = m
+        at += m.size
+    masks = {0: np.arange(sizes[0]) % 3 != 1}
+    return pruning.build_label_graph(blocks, list(sizes), lambda b: costs[b.var_begin], masks, [])
+
+
+CASES = {
+    "one matrix of one element": ([1, 1], [(0, 1)], 0.0),
+    "rows of 1 to 70 elements, one workgroup's": ([1, 70, 2, 3], [(0, 1), (1, 2), (2, 3)], 0.1),
+    "a chain over many workgroups": ([5 + i % 20 for i in range(150)], [(i, i - 1) for i in range(1, 150)], 0.1),
+    "a class with 70 matrices (more than the kept reciprocals)": ([6] + [4] * 70, [(0, i) for i in range(1, 71)], 0.05),
+    "a class with five matrices in as many workgroups": ([60, 50, 50, 50, 50, 50], [(i, 0) for i in range(1, 6)], 0.1),
+    "as many rows in a step as threads": ([256, 1, 256], [(0, 1), (2, 1)], 0.0),
+    "more rows in a step than 256 threads": ([300, 3], [(0, 1)], 0.1),
+    "the largest matrix that fits": ([128, 134], [(0, 1)], 0.1),
+    "labels that can never be taken": ([4, 3, 2], [(0, 1), (1, 2)], 0.7),
+}
+
+
+def _device():
+    from autoparallel_amd.device_tables import DeviceCostTables
+
+    return DeviceCostTables(stress_dag(seed=1, n_nodes=10, mesh_sizes=(2, 2)), CostModelParams.from_mesh((2, 2)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", CASES)
+def test_resident_sweeps_equal_the_oracle(gpu_device, name):
+    sizes, pairs, p_inf = CASES[name]
+    g = _problem(len(name), sizes, pairs, p_inf)
+    dev = _device()
+    plan = dev._sweep_plan(g)
+    assert plan is not None, "the problem was meant to be resident"
+    theta, unary = g.theta, g.unary
+    want = (g.theta, g.unary)
+    for n in (1, 2, 7):
+        theta, unary = dev.diffusion_sweeps(g, theta, unary, n)
+        want = _sweep(g, *want, n)
+        assert np.array_equal(theta, want[0]) and np.array_equal(unary, want[1])
+    if "many workgroups" in name or "five" in name:
+        assert len(plan[1]) > 3 and plan[2] > 0  # (several workgroups, with something to exchange)
+
+
+@pytest.mark.gpu
+def test_an_expired_wait_leaves_the_sweeps_to_the_launches(gpu_device):
+    sizes, pairs, p_inf = CASES["a chain over many workgroups"]
+    g = _problem(3, sizes, pairs, p_inf)
+    dev = _device()
+    dev.SWEEP_WAIT_TICKS = 0  # no wait is long enough: every workgroup leaves at its first one
+    theta, unary = dev.diffusion_sweeps(g, g.theta, g.unary, 3)
+    want = _sweep(g, g.theta, g.unary, 3)
+    assert np.array_equal(theta, want[0]) and np.array_equal(unary, want[1])
+
+
+@pytest.mark.parametrize("sizes,pairs", [([140, 140], [(0, 1)]), ([1500, 2], [(0, 1)])])
+def test_problems_that_do_not_fit_have_no_plan(sizes, pairs):
+    from autoparallel_amd.device_tables import DeviceCostTables
+
+    assert DeviceCostTables._sweep_plan(_problem(0, sizes, pairs)) is None
+
+
+def test_a_plan_holds_every_matrix_once_and_places_every_minimum():
+    """Each workgroup's words against the problem: elements covered once, every class stored once, the
+    minima of an incidence read where its row, or its slot, is written."""
+    from autoparallel_amd.device_tables import DeviceCostTables
+
+    sizes, pairs, p_inf = CASES["a chain over many workgroups"]
+    g = _problem(5, sizes, pairs + [(149, 3), (80, 3), (20, 3), (120, 3), (60, 3)], p_inf)
+    words, begin, n_slots, lds, threads = DeviceCostTables._sweep_plan(g)
+    elements, stored, written, read = np.zeros(len(g.theta), int), np.zeros(len(g.unary), int), {}, {}
+    for b, e in zip(begin[:-1], begin[1:]):
+        p = words[b:e].astype(np.int64) & 0xFFFFFFFF
+        first, n_el, n_rows, n_inc, n_steps = p[:5].tolist()
+        rows = p[8:8 + 8 * n_rows].reshape(-1, 8)
+        labels = p[8 + 8 * n_rows:8 + 9 * n_rows]
+        elements[first:first + n_el] += 1
+        np.add.at(stored, (labels & 0x7FFFFFFF)[labels >> 31 == 1], 1)
+        assert ((rows[:, 0] & 0xFFFF) + ((rows[:, 0] >> 16) - 1) * (rows[:, 1] & 0xFFFF) < n_el).all()
+        for r, label in zip(rows.tolist(), (labels & 0x7FFFFFFF).tolist()):
+            if r[2] != 0xFFFFFFFF:
+                assert r[2] not in written
+                written[r[2]] = label
+            for ref in r[4:]:
+                if ref & 0x40000000:
+                    read.setdefault(ref & 0x3FFFFFFF, set()).add(label)
+                else:
+                    assert ref == n_rows or labels[ref] & 0x7FFFFFFF == label
+    degree = np.diff(g.inc_begin)
+    assert (elements == 1).all() and np.array_equal(stored, np.repeat(degree > 0, np.diff(g.label_begin)))
+    assert sorted(written) == list(range(n_slots)) and all(labels == {written[s]} for s, labels in read.items())
