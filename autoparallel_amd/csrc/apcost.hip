@@ -2984,6 +2984,29 @@ static int out_mode(int mesh_ndim, const double *comm_out, const uint8_t *trans_
   return kOutAny;
 }
 
+// Threads of a tile's workgroup.  More wavefronts stage and drain a tile sooner, fewer leave more tiles resident per
+// compute unit, so what counts is whether the tiles fill the chip and how many values one stores (n_entries
+// counts the copies written for identical edges too: work per tile either way).
+//   At most kTilesInOneRound tiles, all of them resident at once: four wavefronts (829 tiles of 387 values, (32, 8),
+//   one launch: 9.5 / 7.4 / 7.1 us with one / two / four; 968 tiles of 1 800 values 21.6 / 14.8 / 12.0).
+//   `many_states`: four (a tile stages the 496 states of a 4-D mesh: 9 852 tiles of 22 values 101 / 73 / 58 us).
+//   Else by the values per tile: two from `two`, four from `four`.  The launch over the tables' own copies (512, 2048):
+//   1 800 values, (8, 8, 8), 169 / 154 / 179 us; 3 236 values there - / 173 / 131; 2 390 values, (32, 8), - / 32.9 / 29.2.  The launch
+//   of all tables, whose tiles derive what the other reads (64, on 3-D meshes always; 3072): (32, 8), 398 values 18.5 /
+//   17.2 / 21.0, 2 638 values - / 21.4 / 23.8, 3 874 values - / 29.4 / 27.3, 22 values 13.9 / 15.7 / 24.5; (8, 8, 8), 22 values
+//   17.1 / 16.1 / 24.1 us.
+constexpr int64_t kTilesInOneRound = 1280;  // five workgroups of four wavefronts to a compute unit
+
+static int tile_threads(int64_t n_tiles, int64_t n_entries, bool many_states, int64_t two, int64_t four) {
+  int threads = 256;
+  if (n_tiles > kTilesInOneRound && !many_states) {
+    const int64_t per_tile = n_entries / n_tiles;
+    threads = per_tile >= four ? 256 : per_tile >= two ? 128 : 64;
+  }
+  if (const char *env = getenv("APC_TILE_THREADS")) threads = atoi(env);  // tuning override
+  return threads >= 256 ? 256 : threads >= 128 ? 128 : 64;
+}
+
 static int redistribute_tables_impl(const apc_params *params, const int64_t *tensor_bytes,
                                     const uint8_t *tensor_contiguous, const uint32_t *spec_codes,
                                     const int32_t *spec_tensor, const double *pt_values, const double *per_arg,
@@ -3005,15 +3028,8 @@ static int redistribute_tables_impl(const apc_params *params, const int64_t *ten
               rows ? rows->row_min : nullptr, rows ? rows->row_argmin : nullptr, term_layout(*params)};
   const int nt = (int)n_tiles, xs = xcd_shift();
   hipStream_t s = (hipStream_t)stream;
-  // Wavefronts per tile by the mean number of values a tile stores (n_entries counts the
-  // copies written for de-duplicated edges too: work per tile either way): one below 512,
-  // two up to 4096, four above.  Measured on tables of 290 .. 1800 values per tile: more
-  // wavefronts drain a long tile sooner, fewer leave more tiles resident per compute unit
-  // (1800 values per tile, Llama-3-70B: 169 / 154 / 179 us with one / two / four).
   const dim3 grid((unsigned)(((n_tiles + (1 << xs) - 1) >> xs) << xs));  // rounded up for xcd_chunked_unit
-  const int64_t per_tile = n_entries / n_tiles;
-  int threads = per_tile >= 4096 ? 256 : per_tile >= 512 ? 128 : 64;
-  if (const char *env = getenv("APC_TILE_THREADS")) threads = atoi(env);  // tuning override
+  const int threads = tile_threads(n_tiles, n_entries, params->mesh_ndim == 4 && a.lay.exponents == 0, 512, 2048);
   const int om = out_mode(params->mesh_ndim, comm_out, trans_out, cost_out);
 #define APC_LAUNCH_T(KERNEL_, M_, OUT_)                                                                               \
   const int wg = threads >= 256 ? 256 : threads >= 128 ? 128 : 64;                                                     \
@@ -3076,13 +3092,7 @@ static int build_tables_impl(const apc_params *params, int64_t n_tensors, const 
   // (a tile without a tensor still loads row 0 of the tensor table: unconditional loads)
   if (n_tiles > 0 && n_tensors == 0) return fail(-1, "apc_build_tables: tiles need a tensor table with at least one row");
   const int xs = xcd_shift();
-  int threads = 256;
-  if (n_tiles > 0) {
-    const int64_t per_tile = n_entries / n_tiles;
-    threads = per_tile >= 1536 ? 256 : per_tile >= 512 ? 128 : 64;
-  }
-  if (const char *env = getenv("APC_TILE_THREADS")) threads = atoi(env);  // tuning override
-  threads = threads >= 256 ? 256 : threads >= 128 ? 128 : 64;
+  const int threads = tile_threads(n_tiles, n_entries, params->mesh_ndim == 4, params->mesh_ndim == 3 ? 0 : 64, 3072);
   const int64_t tile_blocks = ((n_tiles + (1 << xs) - 1) >> xs) << xs;
   const int64_t sb = spec_table ? blocks_for(n_specs, threads) : 0, tb = blocks_for(n_tensors, threads),
                 cb = blocks_for(n_strategies, threads);

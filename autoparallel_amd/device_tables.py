@@ -247,8 +247,10 @@ class DeviceCostTables:
         tb = self.tables
         if tb.n_tiles == 0 or not tb.rows_fit_tiles():
             return False
-        computed = int((tb.tile_row_count.astype(np.int64) * tb.tile_col_count.astype(np.int64)).sum())
-        return 0.5e-3 * tb.n_tiles + 1.6e-6 * computed < 4.0 + 8.0 * tb.n_entries / 4.5e6
+        # (of the edges cut as little as they can be, where the tiling was chosen from the table: how it is cut further
+        # does not decide whether a planner finds the minima taken)
+        n_tiles, computed = (tb.tiling or {}).get("whole_edges") or (tb.n_tiles, tb.computed_entries())
+        return 0.5e-3 * n_tiles + 1.6e-6 * computed < 4.0 + 8.0 * tb.n_entries / 4.5e6
 
     def _alloc_input_tables(self, spec_table: bool):
         """Allocates (does not fill) the outputs of the tensor, compute-cost and, when wanted,
@@ -283,7 +285,7 @@ class DeviceCostTables:
     # A table up to this many entries is bound by the latency of one workgroup: its planner pass
     # runs over packed tiles (every wavefront on its own, one round of loads, no LDS staging).
     # Above, the per-entry arithmetic of that kernel (direct evaluation) costs more than the
-    # staging it saves.
+    # staging it saves; so it does below for the tables of which ``CostTables.staging_pays`` says so.
     PACKED_MAX_ENTRIES = 4_000_000
 
     def packed_pass_pays(self) -> bool:
@@ -316,7 +318,9 @@ class DeviceCostTables:
         the local shard shapes out (a planner has computed them before it could fill in the
         flop / byte counts this pass reads).  ``packed``: the one launch runs over packed tiles
         (``apc_build_tables_packed``: the assembled cost and the row minima, no spec table);
-        ``None`` takes them when the pass is of that kind and ``packed_pass_pays``."""
+        ``None`` takes them when the pass is of that kind, ``packed_pass_pays`` and staged tiles
+        (``CostTables.staging_pays``) are not faster still."""
+        tb = self.tables
         outputs = tuple(outputs)
         if not outputs or any(o not in ("comm", "transition", "cost") for o in outputs):
             raise ValueError(f"outputs must name some of comm, transition, cost: {outputs}")
@@ -335,14 +339,14 @@ class DeviceCostTables:
             one_launch = bool(fused_inputs) and total <= self.ONE_LAUNCH_MAX_BYTES
         packed_kind = bool(one_launch) and row_min_in_tiles and outputs == ("cost",) and not spec_table
         if packed is None:
-            packed = packed_kind and self.packed_pass_pays()
+            packed = packed_kind and self.packed_pass_pays() and not tb.staging_pays(tb.computed_entries(), tb.n_tiles)
         elif packed and not (packed_kind and self.tables.packable()):
             raise ValueError("a pass over packed tiles is one launch that writes the assembled cost and the row minima, "
                              "without the spec table, over tiles of whole rows")
         spec = self._alloc_input_tables(spec_table)
         self.alloc_outputs("comm" in outputs, "transition" in outputs, "cost" in outputs)
         self.row_min = self.row_argmin = None
-        ops, d, tb = self.ops, self.d, self.tables
+        ops, d = self.ops, self.d
         err = torch.zeros((1,), dtype=torch.int32, device=self.device)
         self._step_keepalive = [err, spec]
         spec_outputs = [spec[k] for k in ("num_shards", "local_shape", "local_stride", "local_numel", "local_bytes")] \

@@ -47,21 +47,37 @@ PARTIAL_OPS = ("sum", "avg", "min", "max", "product", "band", "bor", "bxor")
 EDGE_GRAD_RESCALE = _native.EDGE_GRAD_RESCALE
 EDGE_NO_PRODUCER = _native.EDGE_NO_PRODUCER
 
-# Tiling chosen when the caller names no tile size (measured on one MI355X): an edge matrix of
-# up to 64 x 64 entries is best served by one tile (its producer specs and cost terms are
-# staged once); a table that would then have too few tiles to fill the chip several times
-# over is cut finer (fewer copies per tiled edge first, then smaller tiles), as long as a
-# tile still stores a few thousand entries.  (Llama-3-70B on (8, 8, 8), 73 M entries: 126 us with
-# 11 732 tiles of 2048 entries and 4 copies; 134 us with 8 130 of 4096 / 4, 130 us with 16 192 of
-# 4096 / 2, 140 us with 23 376 of 2048 / 2, 155 us with 40 727 of 1024 / 2, 164 us with 2 085 of
-# 4096 / 16.)
-AUTO_MIN_TILES = 10000
-AUTO_MIN_STORED_PER_TILE = 2048
+# Tiling chosen when the caller names no tile size (measured on one MI355X).  Identical edges: as many copies
+# per tiled edge as leave at most AUTO_MAX_STORED_PER_TILE values for a tile to store, in small tiles: a
+# value computed once is stored to all copies, and a long workgroup is the launch's tail.  66 M entries on (8, 8, 8),
+# 80 layers, tile of about 512 entries and 8 copies (3 236 values) 131 us; 2048 / 4 137, 4096 / 4 145, 512 / 4 145, 512 / 16
+# (6 472 values) 161, 4096 / 16 195.  11 M on (32, 8), 40 layers: 512 / 8 (2 638 values) 26.6, 1024 / 8 27.3, 512 / 16 27.0, 512 / 4
+# 36.5, 2048 / 2 53.9; 6 M on (8, 8, 8), 10 layers: 512 / 16 (3 500) 18.2, 512 / 8 23.9, 2048 / 2 34.5 us.
+# Few or no copies: larger tiles, until one stores AUTO_MIN_STORED_PER_TILE (its specs and cost terms are staged once).
+# 5.5 M entries on (32, 8), no edge like another: 512 entries a tile 51.5, 1024 45.1, 2048 (869 values) 48.4, 4096 57.2 us;
+# 9.4 M on (16, 8, 4): 65.0, 57.5, 60.8, 68.6; 20 M there: 79.4, 65.3, 62.5, 63.3 us.
 AUTO_MIN_TILE_ENTRIES = 512
+AUTO_MIN_STORED_PER_TILE = 800
+AUTO_MAX_STORED_PER_TILE = 3600
 # A table this small is bound by the latency of one workgroup, not by work: it keeps the largest
 # tiles and up to 16 copies per tiled edge (Llama-3-8B on (32, 8), 1.8 M entries: 13.3 us with
 # 840 tiles of 16 copies against 14.6 us with 1 616 tiles of 8 and 17.7 us with 3 168 of 4).
 AUTO_SMALL_TABLE_ENTRIES = 4_000_000
+# ... unless there are many entries to compute, or rows too wide for a packed tile.  A packed tile costs a
+# record of 2.7 KB from memory and evaluates every entry directly; a staged tile evaluates the terms
+# once and looks them up, which wins when a table computes this many entries in tiles that hold this many each.
+# Whole pass, packed (tiles of four rows per wavefront) / staged: 900 989 entries on (32, 8) 23.2 / 15.5 us, on
+# (8, 8, 8) 28.4 / 14.7, on (3, 2, 2, 2) 40.6 / 24.0; 574 862 of at most 24 x 24 a matrix 18.4 / 15.5, 189 736
+# on (8, 8, 8) 9.1 / 7.1, on (32, 8) 7.8 / 7.6; the other way: 102 873 6.7 / 7.0, and 221 958 in matrices of 45
+# entries 18.3 / 21.1 (matrices of 139 entries on a 4-D mesh, whose terms cost most to stage, 31.6 / 34.1).
+STAGED_MIN_COMPUTED = 150_000
+STAGED_MIN_COMPUTED_PER_TILE = {1: 100, 2: 100, 3: 100, 4: 180}
+# Its tiles are cut until there are this many, (or they hold this few entries): enough workgroups for the chip, few
+# enough stagings.  (12, 6), rows up to 90 wide, 2.6 M entries: tiles of about 512 entries 19.9 us, 1024 (3 610 tiles)
+# 18.4, 2048 20.9, 4096 22.8, four rows per wavefront (7 369 tiles) 35.9.  On 4-D meshes a tile stages 496 states: 936 k
+# entries, 512 19.8, 1024 15.7, 2048 (927 tiles) 15.1, 4096 17.2, four rows per wavefront 54.6 us.
+STAGED_TILES = {1: 2800, 2: 2800, 3: 2800, 4: 900}
+STAGED_MIN_TILE_ENTRIES = {1: 512, 2: 512, 3: 512, 4: 1024}
 
 # numpy mirror of the C struct apc_tile (64 bytes)
 TILE_DTYPE = np.dtype([
@@ -294,7 +310,7 @@ class CostTables:
         tile of whole rows holds at most ``w * (64 // columns)`` of them, what ``w`` wavefronts that
         each walk ``64 // columns`` whole rows at a time cover in one pass (the packed-tile launch
         of a small table, whose slowest workgroup decides the launch; the automatic choice sets it
-        to 4 for such a table)."""
+        to 4 for such a table unless ``staging_pays`` or its rows are too wide to pack)."""
         classes = self.edge_classes() if dedupe and self.n_edges else None
         canonical = np.empty(self.n_edges, np.int64)
 
@@ -302,28 +318,45 @@ class CostTables:
             return _native.host_counts("apc_count_tiles_host", self.n_edges, self.edge_n_src, self.edge_n_tgt, classes, te, mc, rows,
                                        canonical)
 
-        if tile_entries is None:
+        def computed():  # (of the last count)
+            return int((self.edge_n_src.astype(np.int64) * self.edge_n_tgt)[canonical == np.arange(self.n_edges)].sum())
+
+        automatic = tile_entries is None
+        if automatic:
             te, mc = APC_TILE_MAX_ROWS * APC_TILE_MAX_COLS, int(max_copies)
             small = self.n_entries <= AUTO_SMALL_TABLE_ENTRIES
-            rows_per_wavefront_pass = 4 if small else None
-            while True:
-                n, n_dups = count(te, mc, rows_per_wavefront_pass or 0)
-                if n == 0 or n >= AUTO_MIN_TILES or self.n_entries / n <= AUTO_MIN_STORED_PER_TILE or small:
-                    break
-                if dedupe and mc > 4:
+            if small:
+                n, n_dups = packed_cut = count(te, mc, 4)
+                whole_edges = n, computed()
+                M = len(self.mesh_sizes)
+                fits = n == 0 or int(self.edge_n_src.max()) <= APC_TILE_MAX_COLS
+                rows_per_wavefront_pass = 4
+                if n and (not fits or whole_edges[1] >= STAGED_MIN_COMPUTED):
+                    n, n_dups = count(te, mc, 0)
+                    while n < STAGED_TILES[M] and te > STAGED_MIN_TILE_ENTRIES[M]:
+                        te //= 2
+                        n, n_dups = count(te, mc, 0)
+                    if not fits or self.staging_pays(whole_edges[1], n):
+                        rows_per_wavefront_pass = None
+                    else:
+                        te, (n, n_dups) = APC_TILE_MAX_ROWS * APC_TILE_MAX_COLS, packed_cut
+            else:
+                n, n_dups = count(te, mc, 0)
+                whole_edges = n, computed()
+                te = AUTO_MIN_TILE_ENTRIES
+                n, n_dups = count(te, mc, 0)
+                while self.n_entries > n * AUTO_MAX_STORED_PER_TILE and mc > 2 and n_dups:
                     mc //= 2
-                elif te > 2048:
-                    te //= 2
-                elif dedupe and mc > 2:
-                    mc //= 2
-                elif te > AUTO_MIN_TILE_ENTRIES:
-                    te //= 2
-                else:
-                    break
+                    n, n_dups = count(te, mc, 0)
+                while self.n_entries < n * AUTO_MIN_STORED_PER_TILE and te < APC_TILE_MAX_ROWS * APC_TILE_MAX_COLS:
+                    te *= 2
+                    n, n_dups = count(te, mc, 0)
         else:
             te, mc = int(tile_entries), int(max_copies)
             n, n_dups = count(te, mc, int(rows_per_wavefront_pass or 0))
         self.tiling = {"tile_entries": te, "max_copies": mc if dedupe else 1}
+        if automatic:
+            self.tiling["whole_edges"] = whole_edges
         if rows_per_wavefront_pass:
             self.tiling["rows_per_wavefront_pass"] = int(rows_per_wavefront_pass)
         self.edge_canonical = canonical
@@ -355,6 +388,14 @@ class CostTables:
         self.tile_records = rec
 
     # ---- packed tiles ------------------------------------------------------------------
+    def staging_pays(self, computed: int, n_tiles: int) -> bool:
+        """Whether tiles staged in LDS beat packed ones on a small table (above: STAGED_MIN_COMPUTED)."""
+        return computed >= STAGED_MIN_COMPUTED and computed >= n_tiles * STAGED_MIN_COMPUTED_PER_TILE[len(self.mesh_sizes)]
+
+    def computed_entries(self) -> int:
+        """Entries the tiles compute: those of identical edges once for all their copies."""
+        return int((self.tile_row_count.astype(np.int64) * self.tile_col_count.astype(np.int64)).sum())
+
     def packable(self) -> bool:
         """Every tile holds whole rows of at most APC_TILE_MAX_COLS columns and serves at most
         APC_PACKED_MAX_DUPS identical edges: the table can be built from packed tiles."""
