@@ -1704,19 +1704,43 @@ void redistribute_tiles_row_min_kernel(const apc_tile *tiles, int n_tiles, int x
 // table workgroups use (TableArgs), so the values are the same bits.  One launch instead of
 // two spares a table of a few tens of MB one ramp-up and one drain of the chip, which at that
 // size are a third of each kernel.
+// (On 3-D and 4-D meshes LDS is sized per launch for the layout in use: with the general layout's share held for every mesh, a
+// workgroup of a 4-D launch held 45 KB of which a power-of-two mesh uses 10.  6.4 M entries on (2, 4, 2, 2) 46.2 -> 32.9 us,
+// 9.4 M on (16, 8, 4) 64.6 -> 59.1, 901 k on (8, 8, 8) 14.9 -> 13.8.)
 // (Wavefronts per SIMD are capped at 5 on 1-D and 2-D meshes: with more resident, the launch's
 // many store streams hinder each other a little.  Llama-3-8B table, each pair on one box:
 // 18.5 us against 18.9 us uncapped, 18.7 us against 18.8 us on another box; capped at 6 as
 // uncapped; 20.3 us capped at 3 or when asked for 8.  The mixture-of-experts table: no change.)
+// (1-D and 2-D meshes hold the larger layout's share in a static array: sized per launch, what a 2-D launch does takes 2 %
+// longer, 18.3 -> 18.7 us for 2.6 M entries on (12, 6), also with the same bytes asked for.)
+template <int M, bool RM>
+static size_t build_tables_lds_bytes(const TermLayout &lay, int threads, bool spec_table) {
+  if (M <= 2) return 0;
+  const size_t stage = stage_lds_bytes<M, RM>(lay, threads);
+  const size_t rows = spec_table ? (size_t)threads * (APC_MAX_RANK + 1) * sizeof(int64_t) : 0;  // (spec_tables_block)
+  return stage > rows ? stage : rows;
+}
+
+// The LDS of build_tables_kernel.
+template <int M, int kThreads, bool RM>
+__device__ __forceinline__ unsigned char *build_tables_lds() {
+  if constexpr (M <= 2) {
+    constexpr size_t kRowBytes = (size_t)kThreads * (APC_MAX_RANK + 1) * sizeof(int64_t);
+    constexpr size_t kStage = sizeof(TileStage<M, RM>) + sizeof(StagingScratch) * (kThreads / 64);
+    __shared__ __align__(16) unsigned char s_fixed[kStage > kRowBytes ? kStage : kRowBytes];
+    return s_fixed;
+  } else {
+    extern __shared__ __align__(16) unsigned char s_stage_bytes[];  // build_tables_lds_bytes<M, RM>
+    return s_stage_bytes;
+  }
+}
+
 template <int M, int kThreads, bool RM, int OUT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(M <= 2 ? 5 : 1, M <= 2 ? 5 : 8)))
 void build_tables_kernel(const apc_tile *tiles, int n_tiles, int xcd_shift, int64_t tile_blocks, apc_params p, TableArgs a,
                          TensorTableArgs t, SpecTableArgs sp, ComputeCostArgs c, int64_t spec_blocks,
                          int64_t tensor_blocks) {
-  constexpr size_t kRowBytes = (size_t)kThreads * (APC_MAX_RANK + 1) * sizeof(int64_t);
-  constexpr size_t kStage = sizeof(TileStage<M, RM>) + sizeof(StagingScratch) * (kThreads / 64);
-  constexpr size_t kLds = kStage > kRowBytes ? kStage : kRowBytes;
-  __shared__ __align__(16) unsigned char s_raw[kLds];
+  unsigned char *const s_raw = build_tables_lds<M, kThreads, RM>();
   static_assert(kThreads == 64 || kThreads == 128 || kThreads == 256, "wavefronts per workgroup: 1, 2 or 4");
   const int64_t b = blockIdx.x;
   if (b < tile_blocks) {
@@ -2989,13 +3013,17 @@ static int out_mode(int mesh_ndim, const double *comm_out, const uint8_t *trans_
 // counts the copies written for identical edges too: work per tile either way).
 //   At most kTilesInOneRound tiles, all of them resident at once: four wavefronts (829 tiles of 387 values, (32, 8),
 //   one launch: 9.5 / 7.4 / 7.1 us with one / two / four; 968 tiles of 1 800 values 21.6 / 14.8 / 12.0).
-//   `many_states`: four (a tile stages the 496 states of a 4-D mesh: 9 852 tiles of 22 values 101 / 73 / 58 us).
+//   `many_states`: four (a tile stages the 496 states of a 4-D mesh: 9 852 tiles of 22 values 101 / 73 / 58 us; with
+//   power-of-two sizes the exponents' 14 arrays, one launch: 1 650 tiles of 546 values 35.6 / 23.1 / 20.0, 6 378 of 999
+//   35.1 / 32.9 / 38.7).
 //   Else by the values per tile: two from `two`, four from `four`.  The launch over the tables' own copies (512, 2048):
 //   1 800 values, (8, 8, 8), 169 / 154 / 179 us; 3 236 values there - / 173 / 131; 2 390 values, (32, 8), - / 32.9 / 29.2.  The launch
-//   of all tables, whose tiles derive what the other reads (64, on 3-D meshes always; 3072): (32, 8), 398 values 18.5 /
+//   of all tables, whose tiles derive what the other reads (64, on 3-D meshes always, with kTilesOfManyRounds 512; 3072): (32, 8), 398 values 18.5 /
 //   17.2 / 21.0, 2 638 values - / 21.4 / 23.8, 3 874 values - / 29.4 / 27.3, 22 values 13.9 / 15.7 / 24.5; (8, 8, 8), 22 values
-//   17.1 / 16.1 / 24.1 us.
+//   17.1 / 16.1 / 24.1 us; 36 157 tiles of 149 values 46.8 / 59.4 / 96.7 there, 46.7 / 56.5 / 94.9 on (16, 8, 4), 4 123 of 139
+//   on (8, 8, 8) 16.6 / 14.3 / 17.8.
 constexpr int64_t kTilesInOneRound = 1280;  // five workgroups of four wavefronts to a compute unit
+constexpr int64_t kTilesOfManyRounds = 16384;  // (of one wavefront: 32 workgroups to a compute unit, twice)
 
 static int tile_threads(int64_t n_tiles, int64_t n_entries, bool many_states, int64_t two, int64_t four) {
   int threads = 256;
@@ -3092,7 +3120,9 @@ static int build_tables_impl(const apc_params *params, int64_t n_tensors, const 
   // (a tile without a tensor still loads row 0 of the tensor table: unconditional loads)
   if (n_tiles > 0 && n_tensors == 0) return fail(-1, "apc_build_tables: tiles need a tensor table with at least one row");
   const int xs = xcd_shift();
-  const int threads = tile_threads(n_tiles, n_entries, params->mesh_ndim == 4, params->mesh_ndim == 3 ? 0 : 64, 3072);
+  const TermLayout lay = term_layout(*params);
+  const bool many_states = params->mesh_ndim == 4 && (lay.exponents == 0 || n_tiles <= 2 * kTilesInOneRound);
+  const int threads = tile_threads(n_tiles, n_entries, many_states, n_tiles > kTilesOfManyRounds ? 512 : params->mesh_ndim == 3 ? 0 : 64, 3072);
   const int64_t tile_blocks = ((n_tiles + (1 << xs) - 1) >> xs) << xs;
   const int64_t sb = spec_table ? blocks_for(n_specs, threads) : 0, tb = blocks_for(n_tensors, threads),
                 cb = blocks_for(n_strategies, threads);
@@ -3103,7 +3133,7 @@ static int build_tables_impl(const apc_params *params, int64_t n_tensors, const 
   TableArgs a{nullptr, nullptr, spec_codes, spec_tensor, pt_values, nullptr, tiles, dup_entry_begin,
               comm_out, trans_out, cost_out, rank, itemsize, shape, stride, flops, rw_bytes, dtype, zero_cost, num_args,
               rows ? rows->edge_row_begin : nullptr, rows ? rows->dup_row_begin : nullptr,
-              rows ? rows->row_min : nullptr, rows ? rows->row_argmin : nullptr, term_layout(*params)};
+              rows ? rows->row_min : nullptr, rows ? rows->row_argmin : nullptr, lay};
   const TensorTableArgs ta{n_tensors, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous};
   const SpecTableArgs sa{n_specs, spec_codes, spec_tensor, rank, itemsize, shape, stride, num_shards,
                          local_shape, local_stride, local_numel, local_bytes, shape_width};
@@ -3113,9 +3143,10 @@ static int build_tables_impl(const apc_params *params, int64_t n_tensors, const 
   const int nt = (int)n_tiles;
   const int om = out_mode(params->mesh_ndim, comm_out, trans_out, cost_out);
 #define APC_LAUNCH_ALL_T(M_, RM_, OUT_)                                                                                 \
-  if (threads == 256) hipLaunchKernelGGL((build_tables_kernel<M_, 256, RM_, OUT_>), grid, dim3(256), 0, s, a.tiles, nt, xs, tile_blocks, *params, a, ta, sa, ca, sb, tb); \
-  else if (threads == 128) hipLaunchKernelGGL((build_tables_kernel<M_, 128, RM_, OUT_>), grid, dim3(128), 0, s, a.tiles, nt, xs, tile_blocks, *params, a, ta, sa, ca, sb, tb); \
-  else hipLaunchKernelGGL((build_tables_kernel<M_, 64, RM_, OUT_>), grid, dim3(64), 0, s, a.tiles, nt, xs, tile_blocks, *params, a, ta, sa, ca, sb, tb)
+  const size_t lds = build_tables_lds_bytes<M_, RM_>(a.lay, threads, spec_table);                                      \
+  if (threads == 256) hipLaunchKernelGGL((build_tables_kernel<M_, 256, RM_, OUT_>), grid, dim3(256), lds, s, a.tiles, nt, xs, tile_blocks, *params, a, ta, sa, ca, sb, tb); \
+  else if (threads == 128) hipLaunchKernelGGL((build_tables_kernel<M_, 128, RM_, OUT_>), grid, dim3(128), lds, s, a.tiles, nt, xs, tile_blocks, *params, a, ta, sa, ca, sb, tb); \
+  else hipLaunchKernelGGL((build_tables_kernel<M_, 64, RM_, OUT_>), grid, dim3(64), lds, s, a.tiles, nt, xs, tile_blocks, *params, a, ta, sa, ca, sb, tb)
 #define APC_LAUNCH_ALL_RM(M_, RM_)                                   \
   if (om == kOutAll) { APC_LAUNCH_ALL_T(M_, RM_, kOutAll); }         \
   else if (om == kOutCost) { APC_LAUNCH_ALL_T(M_, RM_, kOutCost); }  \
