@@ -52,13 +52,13 @@ EDGE_NO_PRODUCER = _native.EDGE_NO_PRODUCER
 # value computed once is stored to all copies, and a long workgroup is the launch's tail.  66 M entries on (8, 8, 8),
 # 80 layers, tile of about 512 entries and 8 copies (3 236 values) 131 us; 2048 / 4 137, 4096 / 4 145, 512 / 4 145, 512 / 16
 # (6 472 values) 161, 4096 / 16 195.  11 M on (32, 8), 40 layers: 512 / 8 (2 638 values) 26.6, 1024 / 8 27.3, 512 / 16 27.0, 512 / 4
-# 36.5, 2048 / 2 53.9; 6 M on (8, 8, 8), 10 layers: 512 / 16 (3 500) 18.2, 512 / 8 23.9, 2048 / 2 34.5 us.
+# 36.5, 2048 / 2 53.9; Llama-3-70B on (8, 8, 8), 73 M entries: 512 / 8 (3 638 values) 124, 512 / 4 133, 2048 / 4 126; 6 M on (8, 8, 8), 10 layers: 512 / 16 (3 500) 18.2, 512 / 8 23.9, 2048 / 2 34.5 us.
 # Few or no copies: larger tiles, until one stores AUTO_MIN_STORED_PER_TILE (its specs and cost terms are staged once).
 # 5.5 M entries on (32, 8), no edge like another: 512 entries a tile 51.5, 1024 45.1, 2048 (869 values) 48.4, 4096 57.2 us;
 # 9.4 M on (16, 8, 4): 65.0, 57.5, 60.8, 68.6; 20 M there: 79.4, 65.3, 62.5, 63.3 us.
 AUTO_MIN_TILE_ENTRIES = 512
 AUTO_MIN_STORED_PER_TILE = 800
-AUTO_MAX_STORED_PER_TILE = 3600
+AUTO_MAX_STORED_PER_TILE = 4000
 # A table this small is bound by the latency of one workgroup, not by work: it keeps the largest
 # tiles and up to 16 copies per tiled edge (Llama-3-8B on (32, 8), 1.8 M entries: 13.3 us with
 # 840 tiles of 16 copies against 14.6 us with 1 616 tiles of 8 and 17.7 us with 3 168 of 4).
