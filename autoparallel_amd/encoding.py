@@ -195,7 +195,8 @@ class CostTables:
         "edge_flags": np.int32, "edge_pt_begin": np.int64, "edge_entry_begin": np.int64,
         "edge_strat_begin": np.int32, "pt_values": np.float64, "tile_edge": np.int32,
         "tile_row_begin": np.int32, "tile_row_count": np.int32, "tile_col_begin": np.int32,
-        "tile_col_count": np.int32,
+        "tile_col_count": np.int32, "edge_canonical": np.int64, "dup_entry_begin": np.int64,
+        "dup_row_begin": np.int64, "edge_dup_begin": np.int64, "edge_dup_count": np.int64,
     }
 
     def __post_init__(self):
@@ -212,6 +213,37 @@ class CostTables:
             self.build_tiles()
         elif self.tile_records is None:
             self.pack_tile_records()
+
+    def _rows(self, n: int, *names, exact: bool = False) -> list:
+        """The named arrays as the library's host entry points read them, which see an address and not where its
+        array ends: contiguous, of the table's dtype, with ``n`` rows at least (``exact``: just as many)."""
+        out = []
+        for name in names:
+            a = np.ascontiguousarray(getattr(self, name), self._DTYPES[name])
+            row = (APC_MAX_RANK,) if name in ("tensor_shape", "tensor_stride") else ()
+            if a.shape[1:] != row:
+                raise ValueError(f"{name} must have rows of shape {row}, it is {a.shape}")
+            if len(a) < n or (exact and len(a) != n):
+                raise ValueError(f"{name} must have {n} rows, it has {len(a)}")
+            out.append(a)
+        return out
+
+    def _tensor_rows(self) -> list:
+        return self._rows(self.n_tensors, "tensor_rank", "tensor_itemsize", "tensor_shape", "tensor_stride")
+
+    def _strategy_rows(self) -> list:
+        return self._rows(self.n_strategies, "strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost", "strat_num_args",
+                          exact=True)
+
+    def _matrix_sizes(self) -> list:
+        return self._rows(self.n_edges, "edge_n_src", "edge_n_tgt", exact=True)
+
+    @staticmethod
+    def _records(records, n: int, dtype) -> np.ndarray:
+        a = np.ascontiguousarray(records)
+        if a.nbytes < n * dtype.itemsize:
+            raise ValueError(f"{n} records of {dtype.itemsize} bytes are needed, there are {a.nbytes} bytes")
+        return a
 
     # ---- sizes -------------------------------------------------------------------------
     @property
@@ -281,8 +313,8 @@ class CostTables:
     def validate_row_minima(self) -> None:
         """Raises unless every matrix row lies inside one tile (the precondition of the
         ``apc_*_row_min`` entry points), through the library's host-side check."""
-        _native.host_call("apc_validate_row_minima_host", self.n_edges, self.edge_n_src, self.edge_n_tgt, self.n_tiles,
-                          self.tile_records)
+        _native.host_call("apc_validate_row_minima_host", self.n_edges, *self._matrix_sizes(), self.n_tiles,
+                          self._records(self.tile_records, self.n_tiles, TILE_DTYPE))
 
     # ---- tiles -------------------------------------------------------------------------
     def edge_classes(self) -> np.ndarray:
@@ -290,11 +322,13 @@ class CostTables:
         (codes and tensor rows), flags, the consumer strategies' compute-cost inputs and the
         pass-through values.  Equal edges have bit-identical comm / transition / cost."""
         first_same = np.empty(self.n_edges, np.int64)
+        n_src, n_tgt = self._matrix_sizes()
+        src_begin, tgt_begin, flags, pt_begin, strat_begin = self._rows(
+            self.n_edges, "edge_src_begin", "edge_tgt_begin", "edge_flags", "edge_pt_begin", "edge_strat_begin")
         _native.host_call(
-            "apc_edge_classes_host", self.n_specs, self.spec_codes, self.spec_tensor, self.n_strategies, self.strat_flops,
-            self.strat_rw_bytes, self.strat_dtype, self.strat_zero_cost, self.strat_num_args, self.n_edges, self.edge_src_begin,
-            self.edge_n_src, self.edge_tgt_begin, self.edge_n_tgt, self.edge_flags, self.edge_pt_begin, self.edge_strat_begin,
-            len(self.pt_values), self.pt_values, first_same)
+            "apc_edge_classes_host", self.n_specs, *self._rows(self.n_specs, "spec_codes", "spec_tensor"), self.n_strategies,
+            *self._strategy_rows(), self.n_edges, src_begin, n_src, tgt_begin, n_tgt, flags, pt_begin, strat_begin,
+            len(self.pt_values), *self._rows(0, "pt_values"), first_same)
         return first_same
 
     def build_tiles(self, tile_entries: Optional[int] = None, dedupe: bool = False, max_copies: int = 16,
@@ -313,13 +347,13 @@ class CostTables:
         to 4 for such a table unless ``staging_pays`` or its rows are too wide to pack)."""
         classes = self.edge_classes() if dedupe and self.n_edges else None
         canonical = np.empty(self.n_edges, np.int64)
+        n_src, n_tgt = self._matrix_sizes()
 
         def count(te, mc, rows):
-            return _native.host_counts("apc_count_tiles_host", self.n_edges, self.edge_n_src, self.edge_n_tgt, classes, te, mc, rows,
-                                       canonical)
+            return _native.host_counts("apc_count_tiles_host", self.n_edges, n_src, n_tgt, classes, te, mc, rows, canonical)
 
         def computed():  # (of the last count)
-            return int((self.edge_n_src.astype(np.int64) * self.edge_n_tgt)[canonical == np.arange(self.n_edges)].sum())
+            return int((n_src.astype(np.int64) * n_tgt)[canonical == np.arange(self.n_edges)].sum())
 
         automatic = tile_entries is None
         if automatic:
@@ -329,7 +363,7 @@ class CostTables:
                 n, n_dups = packed_cut = count(te, mc, 4)
                 whole_edges = n, computed()
                 M = len(self.mesh_sizes)
-                fits = n == 0 or int(self.edge_n_src.max()) <= APC_TILE_MAX_COLS
+                fits = n == 0 or int(n_src.max()) <= APC_TILE_MAX_COLS
                 rows_per_wavefront_pass = 4
                 if n and (not fits or whole_edges[1] >= STAGED_MIN_COMPUTED):
                     n, n_dups = count(te, mc, 0)
@@ -365,7 +399,7 @@ class CostTables:
         self.tile_edge, self.tile_row_begin, self.tile_row_count, self.tile_col_begin, self.tile_col_count = (
             np.empty(n, np.int32) for _ in range(5))
         _native.host_call(
-            "apc_fill_tiles_host", self.n_edges, self.edge_n_src, self.edge_n_tgt, self.edge_entry_begin, canonical, te,
+            "apc_fill_tiles_host", self.n_edges, n_src, n_tgt, *self._rows(self.n_edges + 1, "edge_entry_begin"), canonical, te,
             int(rows_per_wavefront_pass or 0), n, n_dups, self.edge_dup_begin, self.edge_dup_count, self.dup_entry_begin,
             self.dup_row_begin, self.tile_edge, self.tile_row_begin, self.tile_row_count, self.tile_col_begin, self.tile_col_count)
         self.pack_tile_records()
@@ -381,10 +415,12 @@ class CostTables:
             self.edge_dup_begin = np.zeros(self.n_edges, np.int64)
         rec = np.empty(self.n_tiles, TILE_DTYPE)
         _native.host_call(
-            "apc_tile_records_host", self.n_specs, self.spec_tensor, self.n_edges, self.edge_src_begin, self.edge_n_src,
-            self.edge_tgt_begin, self.edge_flags, self.edge_pt_begin, self.edge_entry_begin, self.edge_strat_begin,
-            self.edge_dup_begin, self.edge_dup_count, self.n_tiles, self.tile_edge, self.tile_row_begin, self.tile_row_count,
-            self.tile_col_begin, self.tile_col_count, rec)
+            "apc_tile_records_host", self.n_specs, *self._rows(self.n_specs, "spec_tensor"), self.n_edges,
+            *self._rows(self.n_edges, "edge_src_begin", "edge_n_src", "edge_tgt_begin", "edge_flags", "edge_pt_begin"),
+            *self._rows(self.n_edges + 1, "edge_entry_begin"),
+            *self._rows(self.n_edges, "edge_strat_begin", "edge_dup_begin", "edge_dup_count"),
+            self.n_tiles, *self._rows(self.n_tiles, "tile_edge", "tile_row_begin", "tile_row_count", "tile_col_begin",
+                                      "tile_col_count"), rec)
         self.tile_records = rec
 
     # ---- packed tiles ------------------------------------------------------------------
@@ -405,6 +441,14 @@ class CostTables:
             return False
         return bool(self.n_strategies == 0 or int(self.strat_num_args.max()) <= 0x7FFF)
 
+    def _packed_sources(self) -> list:
+        """What a packed tile is copied out of, as the library takes it."""
+        self._matrix_sizes()  # (the rows of all edges come from their sizes)
+        return [self.n_tensors, *self._tensor_rows(), self.n_specs, *self._rows(self.n_specs, "spec_codes", "spec_tensor"),
+                self.n_strategies, *self._strategy_rows(), self.n_edges, self.edge_row_begin(), self.n_tiles,
+                self._records(self.tile_records, self.n_tiles, TILE_DTYPE), len(self.dup_entry_begin),
+                *self._rows(len(self.dup_entry_begin), "dup_entry_begin", "dup_row_begin")]
+
     def pack_tiles(self) -> np.ndarray:
         """One ``apc_packed_tile`` record per tile: the tile's header, its tensor's row, the
         first entries / rows of its identical edges, its producer and consumer specs and its
@@ -415,20 +459,13 @@ class CostTables:
             raise RuntimeError("packed tiles need whole rows in every tile and at most "
                                f"{APC_PACKED_MAX_DUPS} identical edges per tile")
         pk = np.empty(self.n_tiles, PACKED_TILE_DTYPE)
-        _native.host_call(
-            "apc_pack_tiles_host", self.n_tensors, self.tensor_rank, self.tensor_itemsize, self.tensor_shape, self.tensor_stride,
-            self.n_specs, self.spec_codes, self.spec_tensor, self.n_strategies, self.strat_flops, self.strat_rw_bytes,
-            self.strat_dtype, self.strat_zero_cost, self.strat_num_args, self.n_edges, self.edge_row_begin(), self.n_tiles,
-            self.tile_records, len(self.dup_entry_begin), self.dup_entry_begin, self.dup_row_begin, pk)
+        _native.host_call("apc_pack_tiles_host", *self._packed_sources(), pk)
         return pk
 
     def validate_packed(self, packed: np.ndarray) -> None:
         """The packed records against the tables, through the library's host-side check."""
-        _native.host_call(
-            "apc_validate_packed_tiles_host", self.n_tensors, self.tensor_rank, self.tensor_itemsize, self.tensor_shape,
-            self.tensor_stride, self.n_specs, self.spec_codes, self.spec_tensor, self.n_strategies, self.strat_flops,
-            self.strat_rw_bytes, self.strat_dtype, self.strat_zero_cost, self.strat_num_args, self.n_edges, self.edge_row_begin(),
-            self.n_tiles, self.tile_records, len(self.dup_entry_begin), self.dup_entry_begin, self.dup_row_begin, packed)
+        _native.host_call("apc_validate_packed_tiles_host", *self._packed_sources(),
+                          self._records(packed, self.n_tiles, PACKED_TILE_DTYPE))
 
     # ---- checks ------------------------------------------------------------------------
     def validate(self, params) -> None:
@@ -449,18 +486,25 @@ class CostTables:
                 raise RuntimeError(f"{name} must have n_strategies rows")
         if self.tile_records is None or len(self.tile_records) != self.n_tiles:
             raise RuntimeError("tile_records must have one record per tile (call pack_tile_records())")
+        rank, itemsize, shape, _ = self._tensor_rows()
+        codes, spec_tensor = self._rows(self.n_specs, "spec_codes", "spec_tensor")
+        flops, rw_bytes, *_, num_args = self._strategy_rows()
+        n_src, n_tgt = self._matrix_sizes()
+        src_begin, tgt_begin, flags, pt_begin, strat_begin, canonical, dup_count = self._rows(
+            self.n_edges, "edge_src_begin", "edge_tgt_begin", "edge_flags", "edge_pt_begin", "edge_strat_begin", "edge_canonical",
+            "edge_dup_count")
+        (dup_entry_begin,) = self._rows(0, "dup_entry_begin")
         _native.host_call(
-            "apc_validate_tables_host", params.to_c(), self.n_tensors, self.tensor_rank, self.n_specs, self.spec_codes,
-            self.spec_tensor, self.n_edges, self.edge_src_begin, self.edge_n_src, self.edge_tgt_begin, self.edge_n_tgt,
-            self.edge_flags, self.edge_pt_begin, self.edge_entry_begin, self.edge_strat_begin, len(self.pt_values),
-            self.n_strategies, self.n_tiles, self.tile_records, len(self.dup_entry_begin), self.dup_entry_begin)
+            "apc_validate_tables_host", params.to_c(), self.n_tensors, rank, self.n_specs, codes, spec_tensor, self.n_edges,
+            src_begin, n_src, tgt_begin, n_tgt, flags, pt_begin, *self._rows(self.n_edges + 1, "edge_entry_begin"), strat_begin,
+            len(self.pt_values), self.n_strategies, self.n_tiles, self._records(self.tile_records, self.n_tiles, TILE_DTYPE),
+            len(dup_entry_begin), dup_entry_begin)
         # what the device cannot check: every edge is tiled completely or a duplicate of an edge that is; flop and
         # byte counts convert to fp64 exactly (the kernels divide them as doubles)
         _native.host_call(
-            "apc_validate_tiling_host", self.n_tensors, self.tensor_rank, self.tensor_itemsize, self.tensor_shape,
-            self.n_strategies, self.strat_flops, self.strat_rw_bytes, self.strat_num_args, self.n_edges, self.edge_n_src,
-            self.edge_n_tgt, self.edge_canonical, self.edge_dup_count, len(self.dup_entry_begin), self.n_tiles, self.tile_edge,
-            self.tile_row_count, self.tile_col_count)
+            "apc_validate_tiling_host", self.n_tensors, rank, itemsize, shape, self.n_strategies, flops, rw_bytes, num_args,
+            self.n_edges, n_src, n_tgt, canonical, dup_count, len(dup_entry_begin), self.n_tiles,
+            *self._rows(self.n_tiles, "tile_edge", "tile_row_count", "tile_col_count"))
 
     def as_dict(self) -> dict:
         """Plain-data view (numpy arrays) of every table."""

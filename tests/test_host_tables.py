@@ -87,6 +87,64 @@ def test_packed_records_repeat_the_tables():
         tb.pack_tiles()
 
 
+# what each host pass reads of the tables, besides the array whose length gives the number of rows
+READS = {
+    "edge_classes": ("spec_tensor", "strat_rw_bytes", "strat_dtype", "strat_zero_cost", "strat_num_args", "edge_src_begin",
+                     "edge_tgt_begin", "edge_n_tgt", "edge_flags", "edge_pt_begin", "edge_strat_begin"),
+    "build_tiles": ("edge_n_tgt", "edge_entry_begin", "spec_tensor", "edge_src_begin", "edge_tgt_begin", "edge_flags",
+                    "edge_pt_begin", "edge_strat_begin"),
+    "pack_tile_records": ("spec_tensor", "edge_src_begin", "edge_tgt_begin", "edge_flags", "edge_pt_begin", "edge_entry_begin",
+                          "edge_strat_begin", "edge_dup_begin", "edge_dup_count", "tile_row_begin", "tile_row_count",
+                          "tile_col_begin", "tile_col_count"),
+    "pack_tiles": ("tensor_itemsize", "tensor_shape", "tensor_stride", "spec_tensor", "strat_rw_bytes", "strat_dtype",
+                   "strat_zero_cost", "strat_num_args", "edge_n_tgt", "tile_records", "dup_row_begin"),
+    "validate_row_minima": ("edge_n_tgt", "tile_records"),
+    "validate": ("tensor_itemsize", "tensor_shape", "spec_tensor", "strat_rw_bytes", "strat_dtype", "strat_zero_cost",
+                 "strat_num_args", "edge_n_tgt", "edge_src_begin", "edge_tgt_begin", "edge_flags", "edge_pt_begin",
+                 "edge_entry_begin", "edge_strat_begin", "edge_canonical", "edge_dup_count", "tile_records", "tile_row_count",
+                 "tile_col_count"),
+}
+
+
+def _read(tb, method):
+    return getattr(tb, method)(*([CostModelParams.from_mesh((4, 2))] if method == "validate" else []))
+
+
+def _two_layers():
+    tb = twin_graph(stress_dag(seed=4, n_nodes=60, mesh_sizes=(4, 2), min_strategies=1, max_strategies=10))
+    tb.build_tiles(512, dedupe=True)
+    return tb
+
+
+@pytest.mark.parametrize("method,name", [(m, n) for m, names in READS.items() for n in names])
+def test_an_array_that_ends_early_is_refused_before_it_is_read(method, name):
+    """The library sees addresses: an array shorter than the table it belongs to must not reach it."""
+    for keep in (-1, 0):  # one row short; empty
+        tb = _two_layers()
+        setattr(tb, name, getattr(tb, name)[:keep])
+        with pytest.raises((ValueError, RuntimeError, IndexError)):
+            _read(tb, method)
+
+
+@pytest.mark.parametrize("method", READS)
+def test_arrays_of_other_types_and_strides_are_read_by_value(method):
+    want, tb = _two_layers(), _two_layers()
+    for name in READS[method] + ("strat_flops", "edge_n_src"):
+        a = getattr(tb, name)
+        if a.dtype.names is None and a.ndim == 1:
+            wider = np.zeros(2 * len(a), np.int32 if a.dtype == np.int64 else np.int64)
+            wider[::2] = a
+            setattr(tb, name, wider[::2])
+        else:
+            setattr(tb, name, np.repeat(a, 2, axis=0)[::2])
+    got = _read(tb, method)
+    assert (got is None) == (_read(want, method) is None)
+    if got is not None:
+        assert got.tobytes() == _read(want, method).tobytes()
+    elif method != "validate":
+        assert tb.tile_records.tobytes() == want.tile_records.tobytes()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("sizes", [[0], [1, 0, 3], [4 << 20], [(4 << 20) + 1, 255, 0, 257], [1, 40 << 20, 7, 9 << 20]])
 def test_transfers_bring_back_the_bytes(gpu_device, sizes):
