@@ -132,9 +132,10 @@ def test_arrays_of_other_types_and_strides_are_read_by_value(method):
     for name in READS[method] + ("strat_flops", "edge_n_src"):
         a = getattr(tb, name)
         if a.dtype.names is None and a.ndim == 1:
-            wider = np.zeros(2 * len(a), np.int32 if a.dtype == np.int64 else np.int64)
-            wider[::2] = a
-            setattr(tb, name, wider[::2])
+            other = np.int64 if a.dtype.itemsize < 8 or a.max(initial=0) > 2**31 - 1 else np.int32
+            spread = np.zeros(2 * len(a), other)
+            spread[::2] = a
+            setattr(tb, name, spread[::2])
         else:
             setattr(tb, name, np.repeat(a, 2, axis=0)[::2])
     got = _read(tb, method)
