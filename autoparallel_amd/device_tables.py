@@ -21,6 +21,7 @@ from . import _native
 from ._device_thread import on_device_thread as _guarded
 from .cost_model import CostModelParams
 from .encoding import CostTables
+from .pruning import index_arrays
 
 _UPLOAD = (
     "tensor_rank", "tensor_itemsize", "tensor_shape", "tensor_stride", "spec_codes", "spec_tensor",
@@ -575,9 +576,12 @@ class DeviceCostTables:
         n_colors = len(graph.color_begin) - 1
         capacity = (n_colors + 16) * most + int((9 * labels + degree)[ends].sum())
         plan, begin, sizes = np.empty(capacity, np.int32), np.empty(most + 1, np.int64), np.empty(5, np.int64)
-        _native.host_call("apc_sweep_plan_host", graph.n_classes, graph.label_begin, graph.inc_begin, graph.inc_edge, graph.inc_side,
-                          graph.n_edges, graph.edge_begin, graph.edge_i, graph.edge_j, n_colors, graph.color_begin,
-                          graph.color_nodes, most, capacity, plan, begin, sizes)
+        index = index_arrays(graph)
+        color_begin, color_nodes = np.ascontiguousarray(graph.color_begin, np.int64), np.ascontiguousarray(graph.color_nodes, np.int32)
+        if n_colors < 0 or len(color_nodes) < graph.n_classes:
+            raise ValueError("the colours must partition the classes")
+        _native.host_call("apc_sweep_plan_host", graph.n_classes, *index[:4], graph.n_edges, *index[4:], n_colors, color_begin,
+                          color_nodes, most, capacity, plan, begin, sizes)
         n, words, *rest = sizes.tolist()
         return (plan[:words], begin[:n + 1], *rest) if n else None
 

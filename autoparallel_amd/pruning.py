@@ -161,12 +161,30 @@ def build_label_graph(blocks: list, class_sizes: list, block_costs, masks: dict,
                       color_nodes=color_nodes, blocks=blocks)
 
 
+_INDEX = (("label_begin", np.int64), ("inc_begin", np.int64), ("inc_edge", np.int32), ("inc_side", np.uint8),
+          ("edge_begin", np.int64), ("edge_i", np.int32), ("edge_j", np.int32))
+
+
+def index_arrays(g: LabelGraph) -> tuple:
+    """The index arrays of the problem as the library's host entry points read them, which see an address and not
+    where its array ends: contiguous, of their types, none shorter than it is read."""
+    index = tuple(np.ascontiguousarray(getattr(g, name), dtype) for name, dtype in _INDEX)
+    n, ne = g.n_classes, g.n_edges
+    if len(index[1]) <= n:
+        raise ValueError(f"inc_begin must have {n + 1} rows")
+    n_inc = int(index[1][n])
+    for (name, _), a, rows in zip(_INDEX, index, (n + 1, n + 1, n_inc, n_inc, ne + 1, ne, ne)):
+        if a.ndim != 1 or len(a) < rows:
+            raise ValueError(f"{name} must have {rows} rows, it is {a.shape}")
+    return index
+
+
 def _problem(g: LabelGraph, theta: np.ndarray, unary: np.ndarray) -> tuple:
     """The arguments that the library's host entry points take for the problem."""
     theta, unary = np.ascontiguousarray(theta, np.float64), np.ascontiguousarray(unary, np.float64)
-    if len(theta) != g.edge_begin[-1] or len(unary) != g.label_begin[-1]:
+    index = index_arrays(g)
+    if theta.size != g.edge_begin[g.n_edges] or unary.size != g.label_begin[-1]:
         raise ValueError("theta / unary do not have the problem's size")
-    index = (g.label_begin, g.inc_begin, g.inc_edge, g.inc_side, g.edge_begin, g.edge_i, g.edge_j)
     if g._addresses is None or any(x is not y for x, y in zip(g._addresses[0], index)):
         g._addresses = (index, [_native.argument(a) for a in index])  # (the address of an array costs as much as the call)
     a = g._addresses[1]
@@ -193,6 +211,8 @@ def refine(g: LabelGraph, theta: np.ndarray, unary: np.ndarray, labels: np.ndarr
     of all its neighbours, until a round changes nothing (after the first round only classes with
     a changed neighbour are looked at again).  Never raises the labelling's cost."""
     lab = np.array(labels, np.int64)
+    if lab.ndim != 1 or len(lab) < g.n_classes:
+        raise ValueError("a labelling has one label per class")
     _native.host_call("apc_refine_labels_host", *_problem(g, theta, unary), int(max_rounds), lab)
     return lab
 

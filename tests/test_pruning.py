@@ -186,3 +186,33 @@ def test_refine_never_raises_the_cost_and_ends_where_no_single_change_helps(seed
     # the labelling decode proposes is only ever improved
     d = pruning.decode(g, theta, unary)
     assert _energy(g, theta, unary, pruning.refine(g, theta, unary, d)) <= _energy(g, theta, unary, d) + 1e-9
+
+
+@pytest.mark.parametrize("name", ["label_begin", "inc_begin", "inc_edge", "inc_side", "edge_begin", "edge_j", "color_nodes", "labels"])
+def test_index_arrays_that_end_early_are_refused_before_they_are_read(name):
+    """The library's host entry points see addresses."""
+    from autoparallel_amd.device_tables import DeviceCostTables
+
+    calls = {"lower_bound": lambda g: pruning.lower_bound(g, g.theta, g.unary), "decode": lambda g: pruning.decode(g, g.theta, g.unary),
+             "refine": lambda g: pruning.refine(g, g.theta, g.unary, np.zeros(6, np.int64)),
+             "prune_masks": lambda g: pruning.prune_masks(g, g.theta, g.unary, 1.0), "plan": DeviceCostTables._sweep_plan}
+    for call in calls.values():
+        g, _ = _random_problem(5)
+        call(g)  # (a good call before: nothing of it may stand for the next)
+        if name == "labels":
+            with pytest.raises(ValueError):
+                pruning.refine(g, g.theta, g.unary, np.zeros(g.n_classes - 1, np.int64))
+            continue
+        if name == "color_nodes" and call is not calls["plan"]:
+            continue
+        setattr(g, name, getattr(g, name)[:-1])
+        with pytest.raises((ValueError, RuntimeError)):
+            call(g)
+
+
+def test_index_arrays_of_other_types_and_strides_are_read_by_value():
+    g, _ = _random_problem(5)
+    want = pruning.lower_bound(g, g.theta, g.unary)[0], pruning.decode(g, g.theta, g.unary).tolist()
+    for name in ("label_begin", "inc_begin", "inc_edge", "inc_side", "edge_begin", "edge_i", "edge_j"):
+        setattr(g, name, np.repeat(getattr(g, name).astype(np.int32), 2)[::2])
+        assert (pruning.lower_bound(g, g.theta, g.unary)[0], pruning.decode(g, g.theta, g.unary).tolist()) == want, name
