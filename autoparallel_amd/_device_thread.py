@@ -43,28 +43,55 @@ class _Call:
 
     def run(self):
         try:
+            _stand_on(self.stream)
             self.result = self.fn(*self.args, **self.kwargs)
         except BaseException as e:  # noqa: BLE001 (raised again in the caller)
             self.error = e
         self.done.release()
 
 
+class _Submitted:
+    """Work that nobody waits for here: the outcome goes to a future."""
+
+    __slots__ = ("fn", "args", "kwargs", "future")
+
+    def __init__(self, fn, args, kwargs, future):
+        self.fn, self.args, self.kwargs, self.future = fn, args, kwargs, future
+
+    def run(self):
+        try:
+            _stand_on(None)
+            result = self.fn(*self.args, **self.kwargs)
+        except BaseException as e:  # noqa: BLE001 (the future's holder sees it)
+            self.future.set_exception(e)
+        else:
+            self.future.set_result(result)
+
+
+_moved = False  # a call with a stream has run on the worker
+
+
+def _stand_on(stream):
+    """Makes ``stream`` the worker's current one; None: the default stream of the device a thread starts on.  Part of the
+    call, so that a stream torch refuses is the caller's exception and not the end of the worker.  (Compared with what is
+    current, not with what the last call asked for: its function may have left another stream or device behind.)"""
+    global _moved
+    if stream is None and not _moved:
+        return
+    import torch
+
+    _moved = True
+    if stream is None:
+        stream = torch.cuda.default_stream(0)
+    if torch.cuda.current_stream() != stream:
+        torch.cuda.set_stream(stream)  # (sets the stream's device as well)
+
+
 def _work(tasks):
     global _worker_ident
     _worker_ident = threading.get_ident()
-    current = None  # the stream this thread stands on; None: its own default
     while True:
         task = tasks.get()
-        if task.stream is not None and (current is None or task.stream != current):
-            import torch
-
-            torch.cuda.set_stream(task.stream)  # (sets the stream's device as well)
-            current = task.stream
-        elif task.stream is None and current is not None:
-            import torch
-
-            torch.cuda.set_stream(torch.cuda.default_stream(current.device))
-            current = None
         task.run()
         del task  # (nothing of a call outlives it here)
 
@@ -82,9 +109,10 @@ def _queue() -> queue.SimpleQueue:
 
 def _forget_thread():
     # a forked child has the parent's queue but not its thread
-    global _tasks, _worker_ident, _lock
+    global _tasks, _worker_ident, _lock, _moved
     _tasks = None
     _worker_ident = None
+    _moved = False
     _lock = threading.Lock()
 
 
@@ -130,14 +158,7 @@ def submit(fn, *args, **kwargs):
     """Queues ``fn(*args, **kwargs)`` on the device thread and returns its future without
     waiting (work that may overlap the caller's: the device's first-use costs)."""
     future = Future()
-
-    def run():
-        try:
-            future.set_result(fn(*args, **kwargs))
-        except BaseException as e:  # noqa: BLE001 (the future's holder sees it)
-            future.set_exception(e)
-
-    _queue().put(_Call(run, (), {}, None))
+    _queue().put(_Submitted(fn, args, kwargs, future))
     return future
 
 

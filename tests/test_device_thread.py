@@ -160,3 +160,41 @@ def test_a_child_of_a_gpu_parent_is_told_so(monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_stream", lambda: (_ for _ in ()).throw(RuntimeError("something else")))
     with pytest.raises(RuntimeError, match="something else"):
         _device_thread._callers_stream()
+
+
+def test_a_stream_that_torch_refuses_is_the_callers_exception(monkeypatch):
+    """The switch to the caller's stream is part of the call: the caller gets its exception, and the calls after it run."""
+    def refuse(stream):
+        raise RuntimeError("no such stream")
+
+    monkeypatch.setattr(torch.cuda, "set_stream", refuse)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: "another stream")
+    monkeypatch.setattr(torch.cuda, "default_stream", lambda device: "another stream")
+    monkeypatch.setattr(_device_thread, "_callers_stream", lambda: "a stream")
+    seen = []
+
+    def caller():
+        try:
+            call(lambda: 1)
+        except RuntimeError as e:
+            seen.append(str(e))
+
+    waiting = threading.Thread(target=caller, daemon=True)  # (a caller that waits for ever must not hold up the test)
+    waiting.start()
+    waiting.join(30)
+    if waiting.is_alive():
+        _device_thread._forget_thread()
+    assert seen == ["no such stream"]
+    monkeypatch.setattr(_device_thread, "_callers_stream", lambda: "another stream")
+    assert call(lambda: 2) == 2 and _device_thread.submit(lambda: 3).result(timeout=30) == 3
+    _device_thread._forget_thread()  # (a worker that has stood on no stream, for the tests after this one)
+
+
+@pytest.mark.gpu
+def test_a_call_stands_on_its_callers_stream_whatever_the_last_one_left_behind(gpu_device):
+    mine, other = torch.cuda.Stream(), torch.cuda.Stream()  # default priority
+    with torch.cuda.stream(mine):
+        call(lambda: torch.cuda.set_stream(other))
+        assert call(torch.cuda.current_stream) == mine
+    call(lambda: torch.cuda.set_stream(other))
+    assert _device_thread.submit(torch.cuda.current_stream).result(timeout=60) == torch.cuda.default_stream()
