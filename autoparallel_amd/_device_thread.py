@@ -19,15 +19,18 @@ futures, and the stream context entered for every call, 40 us a call; so 15.)
 from __future__ import annotations
 
 import _thread
+import atexit
 import functools
 import os
 import queue
 import threading
 from concurrent.futures import Future
 
-_lock = threading.Lock()
+_lock = threading.RLock()
 _tasks: queue.SimpleQueue | None = None
+_worker: threading.Thread | None = None
 _worker_ident: int | None = None
+_closed = False
 
 
 class _Call:
@@ -92,28 +95,52 @@ def _work(tasks):
     _worker_ident = threading.get_ident()
     while True:
         task = tasks.get()
+        if task is None:
+            return
         task.run()
         del task  # (nothing of a call outlives it here)
 
 
-def _queue() -> queue.SimpleQueue:
-    global _tasks
-    if _tasks is None:
-        with _lock:
-            if _tasks is None:
-                tasks = queue.SimpleQueue()
-                threading.Thread(target=_work, args=(tasks,), name="apcost-device_0", daemon=True).start()
-                _tasks = tasks
-    return _tasks
+def _put(task):
+    """Queues ``task``; the worker starts with the first one."""
+    global _tasks, _worker
+    with _lock:  # (nothing may come behind the None that ends the worker: its caller would wait for ever)
+        if _closed:
+            raise RuntimeError("apcost: no device work can start any more, the interpreter is shutting down")
+        if _tasks is None:
+            tasks = queue.SimpleQueue()
+            worker = threading.Thread(target=_work, args=(tasks,), name="apcost-device_0", daemon=True)
+            worker.start()
+            _tasks, _worker = tasks, worker
+        _tasks.put(task)
+
+
+def _finish():
+    """What has been queued is finished before the interpreter ends (submitted work has nobody else who waits for it, and
+    an interpreter torn down under a thread inside a HIP call can crash)."""
+    global _closed
+    with _lock:
+        _closed = True
+        worker = _worker
+        if _tasks is not None:
+            _tasks.put(None)
+    if worker is not None:
+        worker.join()
+
+
+# (before the functions of ``atexit``, as the executors of concurrent.futures do, and in the children of
+# multiprocessing, which end without those)
+getattr(threading, "_register_atexit", atexit.register)(_finish)
 
 
 def _forget_thread():
     # a forked child has the parent's queue but not its thread
-    global _tasks, _worker_ident, _lock, _moved
+    global _tasks, _worker, _worker_ident, _lock, _moved
     _tasks = None
+    _worker = None
     _worker_ident = None
     _moved = False
-    _lock = threading.Lock()
+    _lock = threading.RLock()
 
 
 os.register_at_fork(after_in_child=_forget_thread)
@@ -144,7 +171,7 @@ def call(fn, *args, **kwargs):
     if threading.get_ident() == _worker_ident:
         return fn(*args, **kwargs)
     task = _Call(fn, args, kwargs, _callers_stream())
-    _queue().put(task)
+    _put(task)
     task.done.acquire()
     if task.error is not None:
         try:
@@ -158,7 +185,7 @@ def submit(fn, *args, **kwargs):
     """Queues ``fn(*args, **kwargs)`` on the device thread and returns its future without
     waiting (work that may overlap the caller's: the device's first-use costs)."""
     future = Future()
-    _queue().put(_Submitted(fn, args, kwargs, future))
+    _put(_Submitted(fn, args, kwargs, future))
     return future
 
 

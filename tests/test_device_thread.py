@@ -198,3 +198,41 @@ def test_a_call_stands_on_its_callers_stream_whatever_the_last_one_left_behind(g
         assert call(torch.cuda.current_stream) == mine
     call(lambda: torch.cuda.set_stream(other))
     assert _device_thread.submit(torch.cuda.current_stream).result(timeout=60) == torch.cuda.default_stream()
+
+
+_AT_EXIT = """
+import sys, time
+sys.path.insert(0, {root!r})
+{body}
+"""
+
+
+def _run(body):
+    import os
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    return subprocess.run([sys.executable, "-c", _AT_EXIT.format(root=root, body=body)], capture_output=True, text=True, timeout=120).stdout
+
+
+def test_submitted_work_is_finished_before_the_process_ends():
+    assert _run("from autoparallel_amd import _device_thread as d\n"
+                "d.submit(lambda: (time.sleep(1), print('finished', flush=True)))") == "finished\n"
+
+
+def test_submitted_work_is_finished_before_a_multiprocessing_child_ends():
+    assert _run("from autoparallel_amd import _device_thread as d\n"
+                "import multiprocessing\n"
+                "def child(): d.submit(lambda: (time.sleep(1), print('finished', flush=True)))\n"
+                "p = multiprocessing.get_context('fork').Process(target=child); p.start(); p.join()") == "finished\n"
+
+
+def test_work_after_the_end_is_refused_and_not_waited_for():
+    assert _run("import atexit\n"
+                "from autoparallel_amd import _device_thread as d\n"
+                "d.call(int)\n"
+                "def late():\n"
+                "    try: d.call(int)\n"
+                "    except RuntimeError as e: print(e)\n"
+                "atexit.register(late)") == "apcost: no device work can start any more, the interpreter is shutting down\n"
