@@ -62,6 +62,8 @@ class _Submitted:
         self.fn, self.args, self.kwargs, self.future = fn, args, kwargs, future
 
     def run(self):
+        if not self.future.set_running_or_notify_cancel():
+            return
         try:
             _stand_on(None)
             result = self.fn(*self.args, **self.kwargs)

@@ -200,6 +200,16 @@ def test_a_call_stands_on_its_callers_stream_whatever_the_last_one_left_behind(g
     assert _device_thread.submit(torch.cuda.current_stream).result(timeout=60) == torch.cuda.default_stream()
 
 
+def test_a_submitted_call_can_be_cancelled_until_it_runs():
+    hold, ran = threading.Event(), []
+    first = _device_thread.submit(hold.wait, 30)
+    second = _device_thread.submit(ran.append, 1)
+    assert second.cancel()
+    hold.set()
+    assert first.result(timeout=30) and call(lambda: list(ran)) == [] and second.cancelled()
+    assert not first.cancel()
+
+
 _AT_EXIT = """
 import sys, time
 sys.path.insert(0, {root!r})
