@@ -613,6 +613,9 @@ class DeviceCostTables:
             theta_out, unary_out, flag = (t.numpy() for t in self.ops.download([*pair, status]))
             if int(flag[0]) == 0:
                 out = pair
+            else:  # (the next chunk of sweeps would wait as long again)
+                cached["plan"] = None
+                del cached["on_device"]
         if out is None:
             d = cached.get("index")
             if d is None:

@@ -71,6 +71,40 @@ def test_an_expired_wait_leaves_the_sweeps_to_the_launches(gpu_device):
     assert np.array_equal(theta, want[0]) and np.array_equal(unary, want[1])
 
 
+def test_an_expired_wait_is_paid_once_per_problem():
+    """On the CPU, with operators that only keep count: after a wait that expired, the chunks that follow take the launches
+    at once; another problem has a plan again."""
+    import torch
+
+    from autoparallel_amd.device_tables import DeviceCostTables
+
+    class Ops:
+        resident = launches = 0
+
+        def upload(self, arrays, device):
+            return [t.clone() for t in arrays]
+
+        def download(self, arrays):
+            return [t.clone() for t in arrays]
+
+        def diffusion_sweeps_resident(self, n, plan, begin, slots, lds, threads, n_labels, n_elements, theta, unary, ticks):
+            Ops.resident += 1
+            return theta.clone(), unary.clone(), torch.ones(1, dtype=torch.int32)  # expired
+
+        def diffusion_sweeps_(self, *args):
+            Ops.launches += 1
+
+    dev = DeviceCostTables.__new__(DeviceCostTables)
+    dev.ops, dev.device = Ops(), torch.device("cpu")
+    sizes, pairs, p_inf = CASES["a chain over many workgroups"]
+    for i in (1, 2):
+        g = _problem(i, sizes, pairs, p_inf)
+        pair = g.theta, g.unary
+        for chunk in range(3):
+            pair = dev.diffusion_sweeps(g, *pair, 4)
+        assert (Ops.resident, Ops.launches) == (i, 3 * i)
+
+
 @pytest.mark.parametrize("sizes,pairs", [([140, 140], [(0, 1)]), ([1500, 2], [(0, 1)])])
 def test_problems_that_do_not_fit_have_no_plan(sizes, pairs):
     from autoparallel_amd.device_tables import DeviceCostTables
