@@ -107,9 +107,20 @@ def test_chain_bound_is_exact():
     assert math.isclose(_energy(g, g.theta, g.unary, pruning.decode(g, theta, unary)), best, rel_tol=1e-12)
 
 
+def _sweeps_take(way, monkeypatch):
+    """``launches``: as on a problem that does not fit the chip's LDS, one launch of the update kernel per colour.
+    ``resident``: the kernel that holds the matrices in LDS, which takes every problem here."""
+    from autoparallel_amd.device_tables import DeviceCostTables
+
+    if way == "launches":
+        monkeypatch.setattr(DeviceCostTables, "_sweep_plan", staticmethod(lambda graph: None))
+
+
 @pytest.mark.gpu
+@pytest.mark.parametrize("way", ["launches", "resident"])
 @pytest.mark.parametrize("seed,n,max_labels", [(0, 8, 5), (1, 40, 70), (2, 25, 130), (3, 150, 24)])
-def test_device_sweeps_equal_the_cpu_restatement(gpu_device, seed, n, max_labels):
+def test_device_sweeps_equal_the_cpu_restatement(gpu_device, seed, n, max_labels, way, monkeypatch):
+    _sweeps_take(way, monkeypatch)
     from autoparallel_amd import CostModelParams
     from autoparallel_amd.device_tables import DeviceCostTables
     from autoparallel_amd.synthetic import stress_dag
@@ -121,6 +132,7 @@ def test_device_sweeps_equal_the_cpu_restatement(gpu_device, seed, n, max_labels
     for chunk in (1, 3, 10):
         want_t, want_u = _sweep(g, theta, unary, chunk)
         theta, unary = dev.diffusion_sweeps(g, theta, unary, chunk)
+        assert (dev._diffusion_graph["plan"] is None) == (way == "launches")
         assert np.array_equal(theta, want_t) and np.array_equal(unary, want_u), chunk
 
 
@@ -140,6 +152,7 @@ def _star_problem(seed, centre_labels, leaf_labels, p_inf=0.1):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("way", ["launches", "resident"])
 @pytest.mark.parametrize("name,centre,leaves", [
     ("more labels than threads of a workgroup", 300, [5, 3, 6]),
     ("more incident matrices than are staged", 6, [3] * 70),
@@ -149,10 +162,12 @@ def _star_problem(seed, centre_labels, leaf_labels, p_inf=0.1):
     ("matrices larger than the staging array", 40, [60, 50, 70, 45]),
     ("a planning program's shape", 16, [16, 12, 9, 16, 15, 15, 8, 12, 16, 16, 22, 24, 16, 16, 16, 16]),
 ])
-def test_device_sweeps_on_the_shapes_that_choose_the_kernels_path(gpu_device, name, centre, leaves):
+def test_device_sweeps_on_the_shapes_that_choose_the_kernels_path(gpu_device, name, centre, leaves, way, monkeypatch):
     """The update kernel stages a class's incident matrices in LDS when their number, the pairs
     (matrix, label) and the elements fit, and works on them in memory otherwise: the bits of the
-    CPU restatement either way, at the limits and on both sides of them."""
+    CPU restatement either way, at the limits and on both sides of them.  (The same shapes through the
+    kernel that holds all matrices, which has limits of its own.)"""
+    _sweeps_take(way, monkeypatch)
     from autoparallel_amd import CostModelParams
     from autoparallel_amd.device_tables import DeviceCostTables
     from autoparallel_amd.synthetic import stress_dag
@@ -164,6 +179,7 @@ def test_device_sweeps_on_the_shapes_that_choose_the_kernels_path(gpu_device, na
     for chunk in (1, 4):
         want_t, want_u = _sweep(g, theta, unary, chunk)
         theta, unary = dev.diffusion_sweeps(g, theta, unary, chunk)
+        assert (dev._diffusion_graph["plan"] is None) == (way == "launches")
         assert np.array_equal(theta, want_t) and np.array_equal(unary, want_u), (name, chunk)
 
 
