@@ -331,8 +331,34 @@ class CostTables:
             len(self.pt_values), *self._rows(0, "pt_values"), first_same)
         return first_same
 
+    def edge_signatures(self) -> list:
+        """One digest per edge over what ``edge_classes`` compares, for comparing edges of several tables, or in a
+        program of one's own: equal digests = bit-identical comm / transition / cost."""
+        import hashlib
+
+        sb, ns = self.edge_src_begin.astype(np.int64), self.edge_n_src.astype(np.int64)
+        tb, nt = self.edge_tgt_begin.astype(np.int64), self.edge_n_tgt.astype(np.int64)
+        st = self.edge_strat_begin.astype(np.int64)
+        codes, tensor = self.spec_codes, self.spec_tensor
+        strat = np.rec.fromarrays([self.strat_flops, self.strat_rw_bytes, self.strat_dtype, self.strat_zero_cost,
+                                   self.strat_num_args])
+        out = []
+        for e in range(self.n_edges):
+            h = hashlib.blake2b(digest_size=16)
+            h.update(np.array([ns[e], nt[e], self.edge_flags[e]], np.int64).tobytes())
+            h.update(codes[sb[e]:sb[e] + ns[e]].tobytes())
+            h.update(tensor[sb[e]:sb[e] + ns[e]].tobytes())
+            h.update(codes[tb[e]:tb[e] + nt[e]].tobytes())
+            h.update(tensor[tb[e]:tb[e] + nt[e]].tobytes())
+            h.update(strat[st[e]:st[e] + nt[e]].tobytes())
+            if self.edge_pt_begin[e] >= 0:
+                b = int(self.edge_pt_begin[e])
+                h.update(self.pt_values[b:b + int(ns[e] * nt[e])].tobytes())
+            out.append(h.digest())
+        return out
+
     def build_tiles(self, tile_entries: Optional[int] = None, dedupe: bool = False, max_copies: int = 16,
-                    rows_per_wavefront_pass: Optional[int] = None) -> None:
+                    signatures=None, rows_per_wavefront_pass: Optional[int] = None) -> None:
         """Cuts every edge matrix into rectangles of about ``tile_entries`` entries:
         whole rows when a row fits the LDS column budget, column chunks otherwise.  With
         ``dedupe`` only the first of every group of identical edges is tiled; its tiles
@@ -344,8 +370,17 @@ class CostTables:
         tile of whole rows holds at most ``w * (64 // columns)`` of them, what ``w`` wavefronts that
         each walk ``64 // columns`` whole rows at a time cover in one pass (the packed-tile launch
         of a small table, whose slowest workgroup decides the launch; the automatic choice sets it
-        to 4 for such a table unless ``staging_pays`` or its rows are too wide to pack)."""
-        classes = self.edge_classes() if dedupe and self.n_edges else None
+        to 4 for such a table unless ``staging_pays`` or its rows are too wide to pack).
+        ``signatures``: with a tile size and ``dedupe``, one value per edge, equal where matrices are
+        (as of ``edge_signatures``); without, edges are compared by content."""
+        classes = None
+        if dedupe and self.n_edges and signatures is not None and tile_entries is not None:
+            first: dict = {}
+            classes = np.arange(self.n_edges, dtype=np.int64)
+            for e, signature in enumerate(signatures):
+                classes[e] = first.setdefault(signature, e)
+        elif dedupe and self.n_edges:
+            classes = self.edge_classes()
         canonical = np.empty(self.n_edges, np.int64)
         n_src, n_tgt = self._matrix_sizes()
 
@@ -386,9 +421,9 @@ class CostTables:
                     te *= 2
                     n, n_dups = count(te, mc, 0)
         else:
-            te, mc = int(tile_entries), int(max_copies)
+            te, mc = max(int(tile_entries), 1), int(max_copies)  # (below 1: one row a tile, as 1)
             n, n_dups = count(te, mc, int(rows_per_wavefront_pass or 0))
-        self.tiling = {"tile_entries": te, "max_copies": mc if dedupe else 1}
+        self.tiling = {"tile_entries": te if automatic else int(tile_entries), "max_copies": mc if dedupe else 1}
         if automatic:
             self.tiling["whole_edges"] = whole_edges
         if rows_per_wavefront_pass:

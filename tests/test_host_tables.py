@@ -87,6 +87,21 @@ def test_packed_records_repeat_the_tables():
         tb.pack_tiles()
 
 
+def test_tilings_from_signatures_and_of_less_than_one_entry():
+    want, tb = _two_layers(), _two_layers()
+    assert tb.edge_signatures() == want.edge_signatures() and len(tb.edge_signatures()) == tb.n_edges
+    tb.build_tiles(512, True, 16, tb.edge_signatures())
+    assert tb.tile_records.tobytes() == want.tile_records.tobytes()
+    tb.build_tiles(512, dedupe=True, signatures=range(tb.n_edges))  # no edge is like another
+    assert np.array_equal(tb.edge_canonical, np.arange(tb.n_edges))
+    tb.build_tiles(512, dedupe=True, signatures=["same"] * 3)  # (an edge without a signature stands for itself)
+    assert tb.edge_canonical.tolist() == [0, 0, 0, *range(3, tb.n_edges)]
+    want.build_tiles(1)
+    for te in (0, -7):
+        tb.build_tiles(te)
+        assert tb.tile_records.tobytes() == want.tile_records.tobytes() and tb.tiling["tile_entries"] == te
+
+
 # what each host pass reads of the tables, besides the array whose length gives the number of rows
 READS = {
     "edge_classes": ("spec_tensor", "strat_rw_bytes", "strat_dtype", "strat_zero_cost", "strat_num_args", "edge_src_begin",
