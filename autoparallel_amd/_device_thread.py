@@ -50,6 +50,7 @@ class _Call:
             self.result = self.fn(*self.args, **self.kwargs)
         except BaseException as e:  # noqa: BLE001 (raised again in the caller)
             self.error = e
+            _raised()
         self.done.release()
 
 
@@ -68,28 +69,37 @@ class _Submitted:
             _stand_on(None)
             result = self.fn(*self.args, **self.kwargs)
         except BaseException as e:  # noqa: BLE001 (the future's holder sees it)
+            _raised()
             self.future.set_exception(e)
         else:
             self.future.set_result(result)
 
 
-_moved = False  # a call with a stream has run on the worker
+_UNKNOWN = object()
+_stands_on = None  # the stream the worker stands on; None: its own default
 
 
 def _stand_on(stream):
     """Makes ``stream`` the worker's current one; None: the default stream of the device a thread starts on.  Part of the
-    call, so that a stream torch refuses is the caller's exception and not the end of the worker.  (Compared with what is
-    current, not with what the last call asked for: its function may have left another stream or device behind.)"""
-    global _moved
-    if stream is None and not _moved:
+    call, so that a stream torch refuses is the caller's exception and not the end of the worker.  (Compared with the stream
+    set last: what runs here puts a stream it changes back.  Asking torch for the current one costs 3 us a call on the
+    worker, on which the caller's wait can grow by 30.)"""
+    global _stands_on
+    if stream == _stands_on:
         return
     import torch
 
-    _moved = True
-    if stream is None:
-        stream = torch.cuda.default_stream(0)
-    if torch.cuda.current_stream() != stream:
-        torch.cuda.set_stream(stream)  # (sets the stream's device as well)
+    torch.cuda.set_stream(torch.cuda.default_stream(0) if stream is None else stream)  # (sets the stream's device as well)
+    _stands_on = stream
+
+
+def _raised():
+    # (a graph capture that fails, for one, leaves its stream behind)
+    global _stands_on
+    import torch
+
+    if torch.cuda.is_initialized():
+        _stands_on = _UNKNOWN
 
 
 def _work(tasks):
@@ -137,11 +147,11 @@ getattr(threading, "_register_atexit", atexit.register)(_finish)
 
 def _forget_thread():
     # a forked child has the parent's queue but not its thread
-    global _tasks, _worker, _worker_ident, _lock, _moved
+    global _tasks, _worker, _worker_ident, _lock, _stands_on
     _tasks = None
     _worker = None
     _worker_ident = None
-    _moved = False
+    _stands_on = None
     _lock = threading.RLock()
 
 

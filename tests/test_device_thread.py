@@ -168,8 +168,6 @@ def test_a_stream_that_torch_refuses_is_the_callers_exception(monkeypatch):
         raise RuntimeError("no such stream")
 
     monkeypatch.setattr(torch.cuda, "set_stream", refuse)
-    monkeypatch.setattr(torch.cuda, "current_stream", lambda: "another stream")
-    monkeypatch.setattr(torch.cuda, "default_stream", lambda device: "another stream")
     monkeypatch.setattr(_device_thread, "_callers_stream", lambda: "a stream")
     seen = []
 
@@ -185,18 +183,26 @@ def test_a_stream_that_torch_refuses_is_the_callers_exception(monkeypatch):
     if waiting.is_alive():
         _device_thread._forget_thread()
     assert seen == ["no such stream"]
-    monkeypatch.setattr(_device_thread, "_callers_stream", lambda: "another stream")
+    monkeypatch.setattr(torch.cuda, "set_stream", lambda stream: None)
+    monkeypatch.setattr(torch.cuda, "default_stream", lambda device: "the default stream")
     assert call(lambda: 2) == 2 and _device_thread.submit(lambda: 3).result(timeout=30) == 3
     _device_thread._forget_thread()  # (a worker that has stood on no stream, for the tests after this one)
 
 
 @pytest.mark.gpu
-def test_a_call_stands_on_its_callers_stream_whatever_the_last_one_left_behind(gpu_device):
+def test_a_call_stands_on_its_callers_stream_whatever_a_failed_one_left_behind(gpu_device):
     mine, other = torch.cuda.Stream(), torch.cuda.Stream()  # default priority
+
+    def leave_and_fail():
+        torch.cuda.set_stream(other)
+        raise KeyError
+
     with torch.cuda.stream(mine):
-        call(lambda: torch.cuda.set_stream(other))
+        with pytest.raises(KeyError):
+            call(leave_and_fail)
         assert call(torch.cuda.current_stream) == mine
-    call(lambda: torch.cuda.set_stream(other))
+    with pytest.raises(KeyError):
+        call(leave_and_fail)
     assert _device_thread.submit(torch.cuda.current_stream).result(timeout=60) == torch.cuda.default_stream()
 
 
