@@ -133,7 +133,7 @@ StrategyTable strategy_table(const Tensor &flops, const Tensor &rw_bytes, const 
 // ---- host <-> device, several arrays at once -----------------------------------------------------
 // A copy between pageable memory and the device goes through the runtime's own small staging buffers and
 // waits for itself: 15 - 25 us each, whatever its size, and 5 GB/s for a large one.  A planner moves
-// dozens of arrays at a time, so they travel together: one device buffer, pinned staging in chunks
+// dozens of arrays at a time, so they travel together: pinned staging in chunks
 // (from torch's caching host allocator, given back when the call returns), one wait.
 constexpr int64_t kStagingChunk = 4 << 20;  // bytes per pinned chunk
 constexpr int kStagingSlots = 4;            // chunks in flight
@@ -170,47 +170,75 @@ struct Staging {
 
 int64_t padded(int64_t n) { return (n + 255) / 256 * 256; }
 
-// CPU tensors -> device tensors of the same dtypes and shapes, views of one device buffer (each at a
-// 256-byte boundary), complete when the call returns.
+// Arrays up to this size share one device buffer. A shared buffer stays allocated for as long as any of its arrays
+// lives, so a larger array, which a later refresh of the tables may replace, has an allocation of its own: a copy more
+// to enqueue (10 us: 20 arrays of 70 KB in 81 us through one buffer, 277 us through 20), beside the 40 us and more that
+// the bytes of such an array take. What is held beyond an array's life is bounded by this size times the arrays of a call.
+constexpr int64_t kSharedArray = 1 << 20;
+
+// CPU tensors -> device tensors of the same dtypes and shapes (each at a 256-byte boundary), complete when the call
+// returns.
 std::vector<Tensor> upload(const std::vector<Tensor> &arrays, at::Device device) {
   TORCH_CHECK(device.is_cuda(), "apcost: upload needs a HIP device (got ", device, ")");
-  int64_t total = 0;
-  std::vector<int64_t> at_byte;
-  for (const Tensor &t : arrays) {
-    TORCH_CHECK(t.device().is_cpu() && t.is_contiguous(), "apcost: upload takes contiguous CPU tensors");
-    at_byte.push_back(total);
-    total += padded(t.nbytes());
-  }
   c10::hip::HIPGuard guard(device.index());
   const auto bytes_on_device = at::TensorOptions().dtype(at::kByte).device(device);
-  Tensor buffer = at::empty({total}, bytes_on_device);
-  if (total > 0) {
-    hipStream_t stream = c10::hip::getCurrentHIPStream(device.index()).stream();
-    char *base = static_cast<char *>(buffer.data_ptr());
-    Staging staging(total);
-    const int64_t n_slots = (int64_t)staging.slots.size();
-    size_t k = 0;  // the first array that reaches into the chunk
-    int64_t chunk = 0;
-    for (int64_t begin = 0; begin < total; begin += kStagingChunk, ++chunk) {
-      const int64_t end = std::min(total, begin + kStagingChunk), slot = chunk % n_slots;
-      if (chunk >= n_slots) check_hip(hipEventSynchronize(staging.events[slot]), "hipEventSynchronize");
-      char *to = staging.slot(slot);
-      while (k < arrays.size() && at_byte[k] + (int64_t)arrays[k].nbytes() <= begin) ++k;
-      for (size_t i = k; i < arrays.size() && at_byte[i] < end; ++i) {
-        const int64_t b = std::max(begin, at_byte[i]), e = std::min<int64_t>(end, at_byte[i] + (int64_t)arrays[i].nbytes());
-        if (e > b) copy_bytes(to + (b - begin), static_cast<const char *>(arrays[i].data_ptr()) + (b - at_byte[i]), e - b);
-      }
-      check_hip(hipMemcpyAsync(base + begin, to, end - begin, hipMemcpyHostToDevice, stream), "hipMemcpyAsync");
-      if (n_slots > 1) check_hip(hipEventRecord(staging.events[slot], stream), "hipEventRecord");
+  struct Part {  // array k is bytes [begin, end) of what is staged
+    size_t k;
+    int64_t begin, end;
+  };
+  std::vector<Part> parts;
+  int64_t shared = 0;
+  for (size_t k = 0; k < arrays.size(); ++k) {
+    const Tensor &t = arrays[k];
+    TORCH_CHECK(t.device().is_cpu() && t.is_contiguous(), "apcost: upload takes contiguous CPU tensors");
+    if ((int64_t)t.nbytes() > kSharedArray) continue;
+    parts.push_back(Part{k, shared, shared + (int64_t)t.nbytes()});
+    shared += padded(t.nbytes());
+  }
+  Tensor buffer = at::empty({shared}, bytes_on_device);
+  struct Run {  // bytes [begin, end) of what is staged go to one place on the device
+    int64_t begin, end;
+    char *to;
+  };
+  std::vector<Run> runs{{0, shared, static_cast<char *>(buffer.data_ptr())}};
+  std::vector<Tensor> out(arrays.size());
+  for (const Part &p : parts) {
+    const Tensor &t = arrays[p.k];
+    if (t.numel() == 0) out[p.k] = at::empty(t.sizes(), bytes_on_device.dtype(t.scalar_type()));
+    else out[p.k] = buffer.narrow(0, p.begin, p.end - p.begin).view(t.scalar_type()).view(t.sizes());
+  }
+  int64_t total = shared;
+  for (size_t k = 0; k < arrays.size(); ++k) {
+    const Tensor &t = arrays[k];
+    if ((int64_t)t.nbytes() <= kSharedArray) continue;
+    out[k] = at::empty(t.sizes(), bytes_on_device.dtype(t.scalar_type()));
+    parts.push_back(Part{k, total, total + (int64_t)t.nbytes()});
+    runs.push_back(Run{total, total + (int64_t)t.nbytes(), static_cast<char *>(out[k].data_ptr())});
+    total += padded(t.nbytes());
+  }
+  if (total == 0) return out;
+  hipStream_t stream = c10::hip::getCurrentHIPStream(device.index()).stream();
+  Staging staging(total);
+  const int64_t n_slots = (int64_t)staging.slots.size();
+  size_t p = 0, r = 0;  // the first part, the first run that reach into the chunk
+  int64_t chunk = 0;
+  for (int64_t begin = 0; begin < total; begin += kStagingChunk, ++chunk) {
+    const int64_t end = std::min(total, begin + kStagingChunk), slot = chunk % n_slots;
+    if (chunk >= n_slots) check_hip(hipEventSynchronize(staging.events[slot]), "hipEventSynchronize");
+    char *to = staging.slot(slot);
+    while (p < parts.size() && parts[p].end <= begin) ++p;
+    for (size_t i = p; i < parts.size() && parts[i].begin < end; ++i) {
+      const int64_t b = std::max(begin, parts[i].begin), e = std::min(end, parts[i].end);
+      if (e > b) copy_bytes(to + (b - begin), static_cast<const char *>(arrays[parts[i].k].data_ptr()) + (b - parts[i].begin), e - b);
     }
-    check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    while (r < runs.size() && runs[r].end <= begin) ++r;
+    for (size_t i = r; i < runs.size() && runs[i].begin < end; ++i) {
+      const int64_t b = std::max(begin, runs[i].begin), e = std::min(end, runs[i].end);
+      if (e > b) check_hip(hipMemcpyAsync(runs[i].to + (b - runs[i].begin), to + (b - begin), e - b, hipMemcpyHostToDevice, stream), "hipMemcpyAsync");
+    }
+    if (n_slots > 1) check_hip(hipEventRecord(staging.events[slot], stream), "hipEventRecord");
   }
-  std::vector<Tensor> out;
-  for (size_t i = 0; i < arrays.size(); ++i) {
-    const Tensor &t = arrays[i];
-    if (t.numel() == 0) out.push_back(at::empty(t.sizes(), bytes_on_device.dtype(t.scalar_type())));
-    else out.push_back(buffer.narrow(0, at_byte[i], t.nbytes()).view(t.scalar_type()).view(t.sizes()));
-  }
+  check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
   return out;
 }
 

@@ -162,9 +162,11 @@ def test_arrays_of_other_types_and_strides_are_read_by_value(method):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("sizes", [[0], [1, 0, 3], [4 << 20], [(4 << 20) + 1, 255, 0, 257], [1, 40 << 20, 7, 9 << 20]])
+@pytest.mark.parametrize("sizes", [[0], [1, 0, 3], [4 << 20], [(4 << 20) + 1, 255, 0, 257], [1, 40 << 20, 7, 9 << 20],
+                                   [1 << 20, (1 << 20) + 1, (1 << 20) - 1, 0] * 9, [5 << 20, (1 << 20) + 1, 100, 4 << 20]])
 def test_transfers_bring_back_the_bytes(gpu_device, sizes):
-    """Sizes around the pinned chunk (4 MiB) and beyond the chunks in flight."""
+    """Sizes around the pinned chunk (4 MiB) and beyond the chunks in flight, arrays that share a buffer (up to 1 MiB)
+    and arrays that do not."""
     import torch
 
     from autoparallel_amd import _native
@@ -177,3 +179,17 @@ def test_transfers_bring_back_the_bytes(gpu_device, sizes):
         assert d.is_cuda and d.shape == h.shape and d.dtype == h.dtype and torch.equal(b, h)
         assert d.numel() == 0 or d.data_ptr() % 256 == 0
     assert ops.upload([], gpu_device) == [] and ops.download([]) == []
+
+
+@pytest.mark.gpu
+def test_an_array_that_was_replaced_is_given_back(gpu_device):
+    """However long the arrays live that were uploaded with it."""
+    import torch
+
+    from autoparallel_amd import _native
+
+    big = torch.zeros(8 << 20, dtype=torch.uint8)
+    before = torch.cuda.memory_allocated(gpu_device)
+    a, small, b = _native.torch_ops().upload([big, torch.zeros(9), big], gpu_device)
+    del a, b
+    assert torch.cuda.memory_allocated(gpu_device) - before < 1 << 20 and not small.any()
