@@ -138,6 +138,9 @@ def unpack_codes(packed: int, ndim: int) -> tuple:
     return tuple((int(packed) >> (8 * i)) & 0xFF for i in range(ndim))
 
 
+_RANK_ROW = (APC_MAX_RANK,)
+
+
 def _i32(x):
     return np.ascontiguousarray(x, dtype=np.int32)
 
@@ -198,6 +201,7 @@ class CostTables:
         "tile_col_count": np.int32, "edge_canonical": np.int64, "dup_entry_begin": np.int64,
         "dup_row_begin": np.int64, "edge_dup_begin": np.int64, "edge_dup_count": np.int64,
     }
+    _DTYPES = {name: np.dtype(t) for name, t in _DTYPES.items()}
 
     def __post_init__(self):
         self.mesh_sizes = tuple(int(x) for x in self.mesh_sizes)
@@ -220,9 +224,8 @@ class CostTables:
         out = []
         for name in names:
             a = np.ascontiguousarray(getattr(self, name), self._DTYPES[name])
-            row = (APC_MAX_RANK,) if name in ("tensor_shape", "tensor_stride") else ()
-            if a.shape[1:] != row:
-                raise ValueError(f"{name} must have rows of shape {row}, it is {a.shape}")
+            if a.shape[1:] != (_RANK_ROW if name in ("tensor_shape", "tensor_stride") else ()):
+                raise ValueError(f"{name} has the shape {a.shape}")
             if len(a) < n or (exact and len(a) != n):
                 raise ValueError(f"{name} must have {n} rows, it has {len(a)}")
             out.append(a)

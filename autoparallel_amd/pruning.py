@@ -73,7 +73,6 @@ class LabelGraph:
     color_nodes: np.ndarray  # int32: classes grouped by colour (no two of a colour share an edge)
     blocks: list = field(default_factory=list)
     class_of_choice_base: dict = field(default_factory=dict)
-    _addresses: tuple = field(default=None, repr=False, compare=False)  # of the index arrays, for the library
 
     def __post_init__(self):
         for name, dtype in (("label_begin", np.int64), ("unary", np.float64), ("edge_i", np.int32), ("edge_j", np.int32),
@@ -185,10 +184,7 @@ def _problem(g: LabelGraph, theta: np.ndarray, unary: np.ndarray) -> tuple:
     index = index_arrays(g)
     if theta.size != g.edge_begin[g.n_edges] or unary.size != g.label_begin[-1]:
         raise ValueError("theta / unary do not have the problem's size")
-    if g._addresses is None or any(x is not y for x, y in zip(g._addresses[0], index)):
-        g._addresses = (index, [_native.argument(a) for a in index])  # (the address of an array costs as much as the call)
-    a = g._addresses[1]
-    return (g.n_classes, *a[:4], g.n_edges, *a[4:], theta, unary)
+    return (g.n_classes, *index[:4], g.n_edges, *index[4:], theta, unary)
 
 
 def lower_bound(g: LabelGraph, theta: np.ndarray, unary: np.ndarray):
