@@ -7,6 +7,9 @@
 namespace apc_internal {
 // Stores the formatted message for this thread and returns `code`.
 __attribute__((visibility("hidden"), format(printf, 2, 3))) int fail(int code, const char *fmt, ...);
+// The message of the exception in flight (a vector that no memory could be had for): called in a handler at an entry
+// point, which no exception may leave.
+__attribute__((visibility("hidden"))) int thrown(const char *who);
 // The parameters' ranges and reciprocals.
 __attribute__((visibility("hidden"))) int check_params(const apc_params *p);
 }  // namespace apc_internal

@@ -7,6 +7,7 @@
 #include <atomic>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <vector>
 
 #include "apcost.h"
@@ -17,6 +18,17 @@ using apc_internal::check_params;
 using apc_internal::fail;
 using apc_internal::in_parallel;
 using apc_internal::threads_for;
+using apc_internal::thrown;
+
+int apc_internal::thrown(const char *who) {
+  try {
+    throw;
+  } catch (const std::exception &e) {
+    return fail(-4, "%s: %s", who, e.what());
+  } catch (...) {
+    return fail(-4, "%s: an exception", who);
+  }
+}
 
 namespace {
 
@@ -112,7 +124,7 @@ int apc_edge_classes_host(int64_t n_specs, const uint32_t *spec_codes, const int
                           const int32_t *num_args, int64_t n_edges, const int32_t *edge_src_begin, const int32_t *edge_n_src,
                           const int32_t *edge_tgt_begin, const int32_t *edge_n_tgt, const int32_t *edge_flags,
                           const int64_t *edge_pt_begin, const int32_t *edge_strat_begin, int64_t n_pt, const double *pt_values,
-                          int64_t *first_same) {
+                          int64_t *first_same) try {
   if (n_specs < 0 || n_strategies < 0 || n_edges < 0 || n_pt < 0) return fail(-1, "apc_edge_classes_host: negative count");
   if (n_edges == 0) return 0;
   if (!edge_src_begin || !edge_n_src || !edge_tgt_begin || !edge_n_tgt || !edge_flags || !edge_pt_begin || !edge_strat_begin ||
@@ -165,6 +177,8 @@ int apc_edge_classes_host(int64_t n_specs, const uint32_t *spec_codes, const int
       if (first_same[e] != e && !c.equal(first_same[e], e)) first_same[e] = e;
   });
   return 0;
+} catch (...) {
+  return thrown("apc_edge_classes_host");
 }
 
 // ------------------------------------------------------------------------------------------
@@ -192,7 +206,7 @@ EdgeTiling cut(int64_t ns, int64_t nt, int64_t tile_entries, int64_t rows_per_wa
 
 int apc_count_tiles_host(int64_t n_edges, const int32_t *edge_n_src, const int32_t *edge_n_tgt, const int64_t *first_same,
                          int64_t tile_entries, int64_t max_copies, int64_t rows_per_wavefront_pass, int64_t *edge_canonical,
-                         int64_t *n_tiles, int64_t *n_duplicates) {
+                         int64_t *n_tiles, int64_t *n_duplicates) try {
   if (n_edges < 0 || tile_entries < 1) return fail(-1, "apc_count_tiles_host: n_edges >= 0 and tile_entries >= 1");
   if (!n_tiles || !n_duplicates || (n_edges > 0 && (!edge_n_src || !edge_n_tgt || !edge_canonical)))
     return fail(-1, "apc_count_tiles_host: NULL array");
@@ -225,13 +239,15 @@ int apc_count_tiles_host(int64_t n_edges, const int32_t *edge_n_src, const int32
     }
   }
   return 0;
+} catch (...) {
+  return thrown("apc_count_tiles_host");
 }
 
 int apc_fill_tiles_host(int64_t n_edges, const int32_t *edge_n_src, const int32_t *edge_n_tgt, const int64_t *edge_entry_begin,
                         const int64_t *edge_canonical, int64_t tile_entries, int64_t rows_per_wavefront_pass, int64_t n_tiles,
                         int64_t n_duplicates, int64_t *edge_dup_begin, int64_t *edge_dup_count, int64_t *dup_entry_begin,
                         int64_t *dup_row_begin, int32_t *tile_edge, int32_t *tile_row_begin, int32_t *tile_row_count,
-                        int32_t *tile_col_begin, int32_t *tile_col_count) {
+                        int32_t *tile_col_begin, int32_t *tile_col_count) try {
   if (n_edges < 0 || n_tiles < 0 || n_duplicates < 0 || tile_entries < 1) return fail(-1, "apc_fill_tiles_host: negative count");
   if (n_edges > 0 && (!edge_n_src || !edge_n_tgt || !edge_entry_begin || !edge_canonical || !edge_dup_begin || !edge_dup_count))
     return fail(-1, "apc_fill_tiles_host: NULL edge array");
@@ -279,6 +295,8 @@ int apc_fill_tiles_host(int64_t n_edges, const int32_t *edge_n_src, const int32_
   }
   if (t != n_tiles) return fail(-2, "%lld tiles, the arrays hold %lld", (long long)t, (long long)n_tiles);
   return 0;
+} catch (...) {
+  return thrown("apc_fill_tiles_host");
 }
 
 int apc_tile_records_host(int64_t n_specs, const int32_t *spec_tensor, int64_t n_edges, const int32_t *edge_src_begin,
@@ -325,7 +343,7 @@ int apc_validate_tiling_host(int64_t n_tensors, const int32_t *tensor_rank, cons
                              int64_t n_strategies, const int64_t *flops, const int64_t *rw_bytes, const int32_t *num_args,
                              int64_t n_edges, const int32_t *edge_n_src, const int32_t *edge_n_tgt, const int64_t *edge_canonical,
                              const int64_t *edge_dup_count, int64_t n_duplicates, int64_t n_tiles, const int32_t *tile_edge,
-                             const int32_t *tile_row_count, const int32_t *tile_col_count) {
+                             const int32_t *tile_row_count, const int32_t *tile_col_count) try {
   if (n_tensors < 0 || n_strategies < 0 || n_edges < 0 || n_tiles < 0) return fail(-1, "apc_validate_tiling_host: negative count");
   if ((n_tensors > 0 && (!tensor_rank || !tensor_itemsize || !tensor_shape)) || (n_strategies > 0 && (!flops || !rw_bytes || !num_args)) ||
       (n_edges > 0 && (!edge_n_src || !edge_n_tgt || !edge_canonical || !edge_dup_count)) ||
@@ -369,6 +387,8 @@ int apc_validate_tiling_host(int64_t n_tensors, const int32_t *tensor_rank, cons
     if (n >= (unsigned __int128)kExact) return fail(-2, "tensor byte counts must stay below 2**53");
   }
   return 0;
+} catch (...) {
+  return thrown("apc_validate_tiling_host");
 }
 
 int apc_pack_tiles_host(int64_t n_tensors, const int32_t *tensor_rank, const int32_t *tensor_itemsize, const int64_t *tensor_shape,
@@ -376,7 +396,7 @@ int apc_pack_tiles_host(int64_t n_tensors, const int32_t *tensor_rank, const int
                         int64_t n_strategies, const int64_t *flops, const int64_t *rw_bytes, const int8_t *dtype_code,
                         const uint8_t *zero_cost, const int32_t *num_args, int64_t n_edges, const int64_t *edge_row_begin,
                         int64_t n_tiles, const apc_tile *tiles, int64_t n_dups, const int64_t *dup_entry_begin,
-                        const int64_t *dup_row_begin, apc_packed_tile *packed) {
+                        const int64_t *dup_row_begin, apc_packed_tile *packed) try {
   if (n_tensors < 0 || n_specs < 0 || n_strategies < 0 || n_edges < 0 || n_tiles < 0 || n_dups < 0)
     return fail(-1, "apc_pack_tiles_host: negative count");
   if (n_tiles == 0) return 0;
@@ -436,6 +456,8 @@ int apc_pack_tiles_host(int64_t n_tensors, const int32_t *tensor_rank, const int
   });
   if (bad.load() < n_tiles) return fail(-2, "tile %lld: rows outside the tables", (long long)bad.load());
   return 0;
+} catch (...) {
+  return thrown("apc_pack_tiles_host");
 }
 
 }  // extern "C"
@@ -611,7 +633,7 @@ int apc_validate_tables_host(const apc_params *params, int64_t n_tensors, const 
                              const int32_t *edge_flags, const int64_t *edge_pt_begin,
                              const int64_t *edge_entry_begin, const int32_t *edge_strat_begin, int64_t n_pt,
                              int64_t n_strategies, int64_t n_tiles, const apc_tile *tiles, int64_t n_dups,
-                             const int64_t *dup_entry_begin) {
+                             const int64_t *dup_entry_begin) try {
   if (int rc = check_params(params)) return rc;
   if (!tables_hold(params, n_tensors, tensor_rank, n_specs, spec_codes, spec_tensor, n_edges, edge_src_begin, edge_n_src,
                    edge_tgt_begin, edge_n_tgt, edge_flags, edge_pt_begin, edge_entry_begin, edge_strat_begin, n_pt, n_strategies))
@@ -620,6 +642,8 @@ int apc_validate_tables_host(const apc_params *params, int64_t n_tensors, const 
       return rc;
   return check_tiles(spec_tensor, n_edges, edge_src_begin, edge_n_src, edge_tgt_begin, edge_n_tgt, edge_flags, edge_pt_begin,
                      edge_entry_begin, edge_strat_begin, n_tiles, tiles, n_dups, dup_entry_begin);
+} catch (...) {
+  return thrown("apc_validate_tables_host");
 }
 
 int apc_validate_row_minima_host(int64_t n_edges, const int32_t *edge_n_src, const int32_t *edge_n_tgt, int64_t n_tiles,
@@ -793,7 +817,7 @@ int64_t first_minimum(const double *v, int64_t n) {
 extern "C" {
 
 int apc_label_incidence_host(int64_t n_classes, int64_t n_edges, const int32_t *edge_i, const int32_t *edge_j, int64_t *inc_begin,
-                             int32_t *inc_edge, uint8_t *inc_side, int64_t *color) {
+                             int32_t *inc_edge, uint8_t *inc_side, int64_t *color) try {
   if (n_classes < 0 || n_edges < 0 || !inc_begin || (n_classes > 0 && !color) || (n_edges > 0 && (!edge_i || !edge_j || !inc_edge || !inc_side)))
     return fail(-1, "apc_label_incidence_host: NULL array or negative count");
   for (int64_t k = 0; k < n_edges; ++k)
@@ -822,6 +846,8 @@ int apc_label_incidence_host(int64_t n_classes, int64_t n_edges, const int32_t *
     color[c] = col;
   }
   return 0;
+} catch (...) {
+  return thrown("apc_label_incidence_host");
 }
 
 #define APC_LABEL_PROBLEM                                                                                                     \
@@ -832,7 +858,7 @@ int apc_label_incidence_host(int64_t n_classes, int64_t n_edges, const int32_t *
   const LabelProblem g{n_classes, n_edges, label_begin, inc_begin, inc_edge, inc_side, edge_begin, edge_i, edge_j, theta, unary}; \
   if (!g.holds()) return fail(-2, who ": the index arrays do not describe a labelling problem")
 
-int apc_label_minima_host(APC_LABEL_PROBLEM, double *class_min, double *edge_min) {
+int apc_label_minima_host(APC_LABEL_PROBLEM, double *class_min, double *edge_min) try {
   APC_LABEL_PROBLEM_OF("apc_label_minima_host");
   for (int64_t c = 0; c < n_classes; ++c) {
     const int64_t b = label_begin[c], e = label_begin[c + 1];
@@ -842,9 +868,11 @@ int apc_label_minima_host(APC_LABEL_PROBLEM, double *class_min, double *edge_min
     for (int64_t k = b; k < e; ++k) edge_min[k] = least(theta + edge_begin[k], edge_begin[k + 1] - edge_begin[k]);
   });
   return 0;
+} catch (...) {
+  return thrown("apc_label_minima_host");
 }
 
-int apc_round_labels_host(APC_LABEL_PROBLEM, int64_t *labels) {
+int apc_round_labels_host(APC_LABEL_PROBLEM, int64_t *labels) try {
   APC_LABEL_PROBLEM_OF("apc_round_labels_host");
   std::vector<double> score, d;
   for (int64_t c = 0; c < n_classes; ++c) labels[c] = -1;
@@ -866,9 +894,11 @@ int apc_round_labels_host(APC_LABEL_PROBLEM, int64_t *labels) {
     if (n > 0) labels[c] = first_minimum(score.data(), n);
   }
   return 0;
+} catch (...) {
+  return thrown("apc_round_labels_host");
 }
 
-int apc_refine_labels_host(APC_LABEL_PROBLEM, int64_t max_rounds, int64_t *labels) {
+int apc_refine_labels_host(APC_LABEL_PROBLEM, int64_t max_rounds, int64_t *labels) try {
   APC_LABEL_PROBLEM_OF("apc_refine_labels_host");
   for (int64_t c = 0; c < n_classes; ++c)
     if (labels[c] < -1 || labels[c] >= g.labels(c)) return fail(-2, "apc_refine_labels_host: label %lld of class %lld", (long long)labels[c], (long long)c);
@@ -895,10 +925,12 @@ int apc_refine_labels_host(APC_LABEL_PROBLEM, int64_t max_rounds, int64_t *label
     todo.swap(again);
   }
   return 0;
+} catch (...) {
+  return thrown("apc_refine_labels_host");
 }
 
 int apc_prune_masks_host(APC_LABEL_PROBLEM, const double *class_min, const double *edge_min, double bound, double limit,
-                         uint8_t *dead_label, uint8_t *dead_pair) {
+                         uint8_t *dead_label, uint8_t *dead_pair) try {
   APC_LABEL_PROBLEM_OF("apc_prune_masks_host");
   const int threads = threads_for(8 * edge_begin[n_edges]);
   in_parallel(n_classes, threads, [&](int64_t begin, int64_t end) {
@@ -927,6 +959,8 @@ int apc_prune_masks_host(APC_LABEL_PROBLEM, const double *class_min, const doubl
     }
   });
   return 0;
+} catch (...) {
+  return thrown("apc_prune_masks_host");
 }
 
 // ------------------------------------------------------------------------------------------
@@ -936,7 +970,7 @@ int apc_prune_masks_host(APC_LABEL_PROBLEM, const double *class_min, const doubl
 int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin, const int64_t *inc_begin, const int32_t *inc_edge,
                         const uint8_t *inc_side, int64_t n_edges, const int64_t *edge_begin, const int32_t *edge_i,
                         const int32_t *edge_j, int64_t n_colors, const int64_t *color_begin, const int32_t *color_nodes,
-                        int64_t max_workgroups, int64_t capacity_words, int32_t *plan, int64_t *plan_begin, int64_t *sizes) {
+                        int64_t max_workgroups, int64_t capacity_words, int32_t *plan, int64_t *plan_begin, int64_t *sizes) try {
   const LabelProblem g{n_classes, n_edges, label_begin, inc_begin, inc_edge, inc_side, edge_begin, edge_i, edge_j, nullptr, nullptr};
   if (!g.holds()) return fail(-2, "apc_sweep_plan_host: the index arrays do not describe a labelling problem");
   if (!plan || !plan_begin || !sizes || !color_begin || max_workgroups < 1 || n_colors < 0) return fail(-1, "apc_sweep_plan_host: NULL array or no workgroup");
@@ -1091,6 +1125,8 @@ int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin, const int
   sizes[3] = lds;
   sizes[4] = threads;
   return 0;
+} catch (...) {
+  return thrown("apc_sweep_plan_host");
 }
 
 #undef APC_LABEL_PROBLEM

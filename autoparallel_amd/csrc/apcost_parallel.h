@@ -5,6 +5,8 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdint>
+#include <exception>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -25,11 +27,19 @@ void in_parallel(int64_t n, int threads, F &&body) {
   }
   const int64_t chunk = std::max<int64_t>(1, n / (threads * 8));
   std::atomic<int64_t> next{0};
+  std::mutex first;
+  std::exception_ptr error;  // (of any thread: thrown again in the caller, once all have ended)
   auto work = [&] {
-    for (;;) {
-      const int64_t b = next.fetch_add(chunk, std::memory_order_relaxed);
-      if (b >= n) return;
-      body(b, std::min(n, b + chunk));
+    try {
+      for (;;) {
+        const int64_t b = next.fetch_add(chunk, std::memory_order_relaxed);
+        if (b >= n) return;
+        body(b, std::min(n, b + chunk));
+      }
+    } catch (...) {
+      next.store(n, std::memory_order_relaxed);
+      std::lock_guard<std::mutex> lock(first);
+      if (!error) error = std::current_exception();
     }
   };
   std::vector<std::thread> team;
@@ -39,6 +49,7 @@ void in_parallel(int64_t n, int threads, F &&body) {
   }
   work();
   for (auto &t : team) t.join();
+  if (error) std::rethrow_exception(error);
 }
 
 inline int threads_for(int64_t bytes) { return (int)std::min<int64_t>(kMaxThreads, 1 + (bytes >> 20)); }

@@ -161,6 +161,35 @@ def test_arrays_of_other_types_and_strides_are_read_by_value(method):
         assert tb.tile_records.tobytes() == want.tile_records.tobytes()
 
 
+_NO_MEMORY = """
+import sys
+sys.path.insert(0, {root!r})
+import numpy as np
+from autoparallel_amd import _native
+i64, i32 = (lambda *v: np.asarray(v, np.int64)), (lambda *v: np.asarray(v, np.int32))
+try:
+    if sys.argv[1] == "entry":  # (the vectors come before any array is read)
+        _native.host_counts("apc_count_tiles_host", 1 << 61, i32(1), i32(1), i64(0), 64, 2, 0, i64(0))
+    else:  # 1 M elements: several threads; one of them meets a class of 2**61 labels (and takes its memory first)
+        _native.host_call("apc_prune_masks_host", 3, i64(0, 1024, 2048, 2048 + (1 << 61)), i64(0, 1, 2, 2), i32(0, 0),
+                          np.asarray([0, 1], np.uint8), 1, i64(0, 1 << 20), i32(0), i32(1), np.zeros(1 << 20), np.zeros(2048),
+                          np.zeros(3), np.zeros(1), 0.0, 1.0, np.zeros(2048, bool), np.zeros(1 << 20, bool))
+except RuntimeError as e:
+    print(e, flush=True)
+"""
+
+
+@pytest.mark.parametrize("where", ["entry", "thread"])
+def test_memory_that_cannot_be_had_is_an_error_and_not_the_end_of_the_process(where):
+    import os
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", _NO_MEMORY.format(root=root), where], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0 and "failed (-4)" in out.stdout, (out.returncode, out.stderr[-500:])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("sizes", [[0], [1, 0, 3], [4 << 20], [(4 << 20) + 1, 255, 0, 257], [1, 40 << 20, 7, 9 << 20],
                                    [1 << 20, (1 << 20) + 1, (1 << 20) - 1, 0] * 9, [5 << 20, (1 << 20) + 1, 100, 4 << 20]])
