@@ -35,9 +35,8 @@ LINK_FLAGS = ["-shared", "-fPIC", "-pthread", "-Wl,-soname,libapcost.so"]
 OBJECT_DIR = os.path.join(_PKG, "build")
 
 
-def build_library(verbose: bool = False, sources=SOURCES) -> str:
-    """Compiles ``sources`` (all, unless the caller knows which of them changed), side by side, and
-    links the library."""
+def build_library(verbose: bool = False) -> str:
+    """Compiles the sources side by side and links the library."""
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     os.makedirs(OBJECT_DIR, exist_ok=True)
     objects = {src: os.path.join(OBJECT_DIR, os.path.basename(src) + ".o") for src in SOURCES}
@@ -57,7 +56,7 @@ def build_library(verbose: bool = False, sources=SOURCES) -> str:
                 print(err)
 
     run([[hipcc, *(HIPCC_FLAGS if src.endswith(".hip") else HOST_FLAGS), f"-I{INCLUDE}", "-c", "-o", objects[src], src]
-         for src in sources])
+         for src in SOURCES])
     run([[hipcc, *LINK_FLAGS, "-o", LIB_PATH, *objects.values()]])
     return LIB_PATH
 
