@@ -405,7 +405,7 @@ int apc_pack_tiles_host(int64_t n_tensors, const int32_t *tensor_rank, const int
       !num_args || (n_dups > 0 && (!dup_entry_begin || !dup_row_begin)) ||
       (n_tensors > 0 && (!tensor_rank || !tensor_itemsize || !tensor_shape || !tensor_stride)))
     return fail(-1, "apc_pack_tiles_host: NULL array");
-  std::atomic<int64_t> bad{n_tiles};  // the first tile that names rows outside the tables
+  std::atomic<int64_t> bad{n_tiles};  // the first tile that cannot be packed
   in_parallel(n_tiles, threads_for(n_tiles * (int64_t)sizeof(apc_packed_tile)), [&](int64_t begin, int64_t end) {
     for (int64_t t = begin; t < end; ++t) {
       const apc_tile &tl = tiles[t];
@@ -413,9 +413,12 @@ int apc_pack_tiles_host(int64_t n_tensors, const int32_t *tensor_rank, const int
       memset(&pk, 0, sizeof(pk));
       const int64_t rows = tl.counts & 0xFFFF, cols = tl.counts >> 16, rb = tl.row_begin, first = rb * cols;
       const int64_t sb = tl.src_begin, tb = (int64_t)tl.tgt_begin + rb, st = (int64_t)tl.strat_begin + rb;
-      if (tl.edge < 0 || tl.edge >= n_edges || rows < 1 || rows > APC_TILE_MAX_ROWS || cols < 1 || cols > APC_TILE_MAX_COLS || rb < 0 ||
-          sb < 0 || sb + cols > n_specs || tb < 0 || tb + rows > n_specs || st < 0 || st + rows > n_strategies || tl.tensor >= n_tensors ||
-          tl.dup_count < 0 || tl.dup_count > APC_PACKED_MAX_DUPS || tl.dup_begin < 0 || (int64_t)tl.dup_begin + tl.dup_count > n_dups) {
+      bool holds = tl.edge >= 0 && tl.edge < n_edges && rows >= 1 && rows <= APC_TILE_MAX_ROWS && cols >= 1 && cols <= APC_TILE_MAX_COLS &&
+                   tl.col_begin == 0 && cols == tl.n_src && rb >= 0 && sb >= 0 && sb + cols <= n_specs && tb >= 0 && tb + rows <= n_specs &&
+                   st >= 0 && st + rows <= n_strategies && tl.tensor < n_tensors && tl.dup_count >= 0 &&
+                   tl.dup_count <= APC_PACKED_MAX_DUPS && tl.dup_begin >= 0 && (int64_t)tl.dup_begin + tl.dup_count <= n_dups;
+      for (int64_t j = 0; holds && j < rows; ++j) holds = num_args[st + j] >= 1 && num_args[st + j] <= 0x7FFF;
+      if (!holds) {
         int64_t seen = bad.load();
         while (t < seen && !bad.compare_exchange_weak(seen, t)) {
         }
@@ -455,7 +458,8 @@ int apc_pack_tiles_host(int64_t n_tensors, const int32_t *tensor_rank, const int
       }
     }
   });
-  if (bad.load() < n_tiles) return fail(-2, "tile %lld: rows outside the tables", (long long)bad.load());
+  if (bad.load() < n_tiles)
+    return fail(-2, "tile %lld: rows outside the tables, not whole rows, or num_args outside 1 .. %d", (long long)bad.load(), 0x7FFF);
   return 0;
 } catch (...) {
   return thrown("apc_pack_tiles_host");

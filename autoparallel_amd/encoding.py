@@ -501,7 +501,8 @@ class CostTables:
         return pk
 
     def validate_packed(self, packed: np.ndarray) -> None:
-        """The packed records against the tables, through the library's host-side check."""
+        """Packed records against the tables, through the library's host-side check: for records that were kept or came
+        from elsewhere (``pack_tiles`` refuses the tables whose records this would refuse)."""
         _native.host_call("apc_validate_packed_tiles_host", *self._packed_sources(),
                           self._records(packed, self.n_tiles, PACKED_TILE_DTYPE))
 

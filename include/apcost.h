@@ -544,7 +544,8 @@ int apc_validate_packed_tiles_host(int64_t n_tensors, const int32_t *tensor_rank
                                    const apc_packed_tile *packed_host);
 
 /* Writes the packed records of the tiles (HOST pointers; packed_host [n_tiles]): what
- * apc_validate_packed_tiles_host checks.  A tile that names rows outside the tables is an error. */
+ * apc_validate_packed_tiles_host checks.  A tile that names rows outside the tables, does not hold whole rows, or
+ * serves a strategy whose num_args does not fit the record is an error. */
 int apc_pack_tiles_host(int64_t n_tensors, const int32_t *tensor_rank_host, const int32_t *tensor_itemsize_host,
                         const int64_t *tensor_shape_host, const int64_t *tensor_stride_host, int64_t n_specs,
                         const uint32_t *spec_codes_host, const int32_t *spec_tensor_host, int64_t n_strategies,

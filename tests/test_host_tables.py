@@ -87,6 +87,18 @@ def test_packed_records_repeat_the_tables():
         tb.pack_tiles()
 
 
+@pytest.mark.parametrize("field,value", [("num_args", 0), ("col_begin", 1), ("n_src", 63)])
+def test_tables_whose_packed_records_the_validator_refuses_are_not_packed(field, value):
+    """The planner's pass takes the packed records as they come from ``pack_tiles``."""
+    tb = stress_dag(seed=4, n_nodes=200, mesh_sizes=(4, 2), min_strategies=1, max_strategies=40)
+    if field == "num_args":
+        tb.strat_num_args[tb.edge_strat_begin[tb.tile_edge[3]]] = value
+    else:
+        tb.tile_records[field][3] += value
+    with pytest.raises(RuntimeError, match="tile [0-3]:"):
+        tb.pack_tiles()
+
+
 def test_tilings_from_signatures_and_of_less_than_one_entry():
     want, tb = _two_layers(), _two_layers()
     assert tb.edge_signatures() == want.edge_signatures() and len(tb.edge_signatures()) == tb.n_edges
