@@ -56,9 +56,13 @@ EDGE_NO_PRODUCER = _native.EDGE_NO_PRODUCER
 # Few or no copies: larger tiles, until one stores AUTO_MIN_STORED_PER_TILE (its specs and cost terms are staged once).
 # 5.5 M entries on (32, 8), no edge like another: 512 entries a tile 51.5, 1024 45.1, 2048 (869 values) 48.4, 4096 57.2 us;
 # 9.4 M on (16, 8, 4): 65.0, 57.5, 60.8, 68.6; 20 M there: 79.4, 65.3, 62.5, 63.3 us.
+# With more than AUTO_MANY_TILES of those tiles there are workgroups for the chip however large they are, and the largest
+# win: tiles of 2048 / 4096 entries, 59 M entries (70 662 / 61 636 tiles) on (32, 8) 202 / 205, on (16, 8, 4) 183 / 182 us;
+# 123 M (145 062 tiles of 2048) 404 / 402, 367 / 364; 228 M 722 / 713, 659 / 648; 464 M on (16, 8, 4) 1263 / 1228.
 AUTO_MIN_TILE_ENTRIES = 512
 AUTO_MIN_STORED_PER_TILE = 800
 AUTO_MAX_STORED_PER_TILE = 4000
+AUTO_MANY_TILES = 100_000
 # A table this small is bound by the latency of one workgroup, not by work: it keeps the largest
 # tiles and up to 16 copies per tiled edge (Llama-3-8B on (32, 8), 1.8 M entries: 13.3 us with
 # 840 tiles of 16 copies against 14.6 us with 1 616 tiles of 8 and 17.7 us with 3 168 of 4).
@@ -420,7 +424,8 @@ class CostTables:
                 while self.n_entries > n * AUTO_MAX_STORED_PER_TILE and mc > 2 and n_dups:
                     mc //= 2
                     n, n_dups = count(te, mc, 0)
-                while self.n_entries < n * AUTO_MIN_STORED_PER_TILE and te < APC_TILE_MAX_ROWS * APC_TILE_MAX_COLS:
+                while te < APC_TILE_MAX_ROWS * APC_TILE_MAX_COLS and (
+                        self.n_entries < n * AUTO_MIN_STORED_PER_TILE or (te > AUTO_MIN_TILE_ENTRIES and n > AUTO_MANY_TILES)):
                     te *= 2
                     n, n_dups = count(te, mc, 0)
         else:

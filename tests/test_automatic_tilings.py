@@ -54,6 +54,16 @@ def test_automatic_cut_follows_its_rules(mesh, nodes, hi, twins, large, monkeypa
     assert tb.tiling["whole_edges"] == (other.n_tiles, other.computed_entries())
 
 
+@pytest.mark.parametrize("many,te", [(100_000, 2048), (100, 4096)])
+def test_tiles_are_cut_larger_when_there_are_many_anyway(many, te, monkeypatch):
+    monkeypatch.setattr(encoding, "AUTO_SMALL_TABLE_ENTRIES", 0)
+    monkeypatch.setattr(encoding, "AUTO_MANY_TILES", many)
+    tb = stress_dag(seed=3, n_nodes=400, mesh_sizes=(16, 8, 4))  # (what the stress table is a larger one of)
+    tb.build_tiles(None, dedupe=True)
+    assert tb.tiling["tile_entries"] == te and tb.n_tiles > 100
+    tb.validate(CostModelParams.from_mesh((16, 8, 4)))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("large", [False, True])
 @pytest.mark.parametrize("mesh,nodes,hi,twins", TABLES)
