@@ -13,7 +13,7 @@ caller unchanged.
 
 A call costs its two hand-overs between the threads: a queue of the interpreter's own (no Python
 code between put and get) one way, a lock the caller waits on the other.  (With an executor's
-futures, and the stream context entered for every call, 40 us a call; so 15.)
+futures, and the stream context entered for every call, 40 us a call; so 14 - 20.)
 """
 
 from __future__ import annotations

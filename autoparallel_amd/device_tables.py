@@ -230,9 +230,12 @@ class DeviceCostTables:
 
     # ---- one full device-side pass with pre-bound arguments -------------------------------------
     # A pass over a table this small is bound by the ramp-up and drain of every launch, and
-    # one launch for all tables wins (Llama-3-8B on a (32, 8) mesh, 78 MB: 25 us against 30 us
-    # per pass); above it the tiles' own derivation of what they would otherwise read costs
-    # more than a launch (measured crossover between 90 MB and 170 MB of tables).
+    # one launch for all tables wins; above it the tiles' own derivation of what they would otherwise
+    # read costs more than a launch.  The cost alone, one launch / two: on (32, 8) 5.5 M entries (42 MB) 29.7 / 36.0 us, 11 M
+    # (87 MB) 47.6 / 51.1, 22 M in 8 384 tiles (170 MB) 37.5 / 40.2; on (16, 8, 4) 9.4 M (72 MB) 33.7 / 34.0, 20 M (156 MB)
+    # 65.1 / 58.1.  What the derivation costs goes by tiles and not by bytes, though: tables of many small tiles lose by
+    # this limit, 5.4 M entries in 36 157 tiles 54.8 / 43.7 on (32, 8), 47.1 / 43.9 on (16, 8, 4), 5.3 M in 162 354 tiles
+    # 179 / 107.
     ONE_LAUNCH_MAX_BYTES = 128 << 20
 
     def row_min_in_tiles_pays(self) -> bool:

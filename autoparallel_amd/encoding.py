@@ -51,11 +51,15 @@ EDGE_NO_PRODUCER = _native.EDGE_NO_PRODUCER
 # per tiled edge as leave at most AUTO_MAX_STORED_PER_TILE values for a tile to store, in small tiles: a
 # value computed once is stored to all copies, and a long workgroup is the launch's tail.  66 M entries on (8, 8, 8),
 # 80 layers, tile of about 512 entries and 8 copies (3 236 values) 131 us; 2048 / 4 137, 4096 / 4 145, 512 / 4 145, 512 / 16
-# (6 472 values) 161, 4096 / 16 195.  11 M on (32, 8), 40 layers: 512 / 8 (2 638 values) 26.6, 1024 / 8 27.3, 512 / 16 27.0, 512 / 4
-# 36.5, 2048 / 2 53.9; Llama-3-70B on (8, 8, 8), 73 M entries: 512 / 8 (3 638 values) 124, 512 / 4 133, 2048 / 4 126; 6 M on (8, 8, 8), 10 layers: 512 / 16 (3 500) 18.2, 512 / 8 23.9, 2048 / 2 34.5 us.
+# (6 472 values) 161, 4096 / 16 195.  11 M on (32, 8), 40 layers: 512 / 8 (2 638 values) 26.6, 1024 / 8 27.3, 512 / 16 27.0,
+# 512 / 4 36.5, 2048 / 2 53.9; Llama-3-70B on (8, 8, 8), 73 M entries: 512 / 8 (3 638 values) 124, 512 / 4 133, 2048 / 4 126;
+# 6 M on (8, 8, 8), 10 layers: 512 / 16 (3 500) 18.2, 512 / 8 23.9, 2048 / 2 34.5 us.  The line lies where large tables have
+# it; tables of up to 14 M entries would gain above it: 16 / 8 copies, 10 M, 48 strategies at most, 4 603 / 2 301 values 22.4 /
+# 24.1, 14 M 5 936 / 2 968 values 28.4 / 28.9 us.
 # Few or no copies: larger tiles, until one stores AUTO_MIN_STORED_PER_TILE (its specs and cost terms are staged once).
-# 5.5 M entries on (32, 8), no edge like another: 512 entries a tile 51.5, 1024 45.1, 2048 (869 values) 48.4, 4096 57.2 us;
-# 9.4 M on (16, 8, 4): 65.0, 57.5, 60.8, 68.6; 20 M there: 79.4, 65.3, 62.5, 63.3 us.
+# Tiles of 1024 / 2048 / 4096 entries, no edge like another, the matrices alone: 5.5 M entries on (32, 8) 29.4 / 29.7 (869
+# values) / 33.6 us, on (16, 8, 4) 25.5 / 24.0 / 27.1; 21 M 78 / 77 / 84, 64 / 60 / 62.  (Where the tiles take the row minima
+# too, as they do of the 5.5 M, 1024 are faster: 45.1 / 48.4 / 57.2.)
 # With more than AUTO_MANY_TILES of those tiles there are workgroups for the chip however large they are, and the largest
 # win: tiles of 2048 / 4096 entries, 59 M entries (70 662 / 61 636 tiles) on (32, 8) 202 / 205, on (16, 8, 4) 183 / 182 us;
 # 123 M (145 062 tiles of 2048) 404 / 402, 367 / 364; 228 M 722 / 713, 659 / 648; 464 M on (16, 8, 4) 1263 / 1228.
@@ -79,7 +83,10 @@ STAGED_MIN_COMPUTED_PER_TILE = {1: 100, 2: 100, 3: 100, 4: 180}
 # Its tiles are cut until there are this many, (or they hold this few entries): enough workgroups for the chip, few
 # enough stagings.  (12, 6), rows up to 90 wide, 2.6 M entries: tiles of about 512 entries 19.9 us, 1024 (3 610 tiles)
 # 18.4, 2048 20.9, 4096 22.8, four rows per wavefront (7 369 tiles) 35.9.  On 4-D meshes a tile stages 496 states: 936 k
-# entries, 512 19.8, 1024 15.7, 2048 (927 tiles) 15.1, 4096 17.2, four rows per wavefront 54.6 us.
+# entries, 512 19.8, 1024 15.7, 2048 (927 tiles) 15.1, 4096 17.2, four rows per wavefront 54.6 us.  On both sides of the 900,
+# with row minima in the tiles: (3, 2, 2, 2), 530 k entries, whole edges (979 tiles) 19.4, 1024 17.5; 1.8 M, 39.8, 41.7; 658 k,
+# (676 whole) 1024 18.3, 2048 16.6, 4096 20.2.  On (2, 4, 2, 2), whose term arrays are smaller, 1024 wins: 901 k 17.3 against
+# 20.3, 1.8 M 24.8 against 29.2.
 STAGED_TILES = {1: 2800, 2: 2800, 3: 2800, 4: 900}
 STAGED_MIN_TILE_ENTRIES = {1: 512, 2: 512, 3: 512, 4: 1024}
 
