@@ -592,11 +592,14 @@ def launch_shape(dev, tables, main):
     tile_blocks = (n_tiles + 7) // 8 * 8
     if main == "build_tables_packed":
         return tile_blocks + (tables.n_tensors + 255) // 256 + (tables.n_strategies + 255) // 256, 256
+    # (up to 3 mesh dims, as the workloads have)
     per_tile = tables.n_entries // max(n_tiles, 1)
+    two, four = 512, 2048
     if main == "build_tables":
-        threads = 256 if per_tile >= 1536 else 128 if per_tile >= 512 else 64
+        two, four = (512 if n_tiles > 16384 else 0 if len(tables.mesh_sizes) == 3 else 64), 3072
+    threads = 256 if n_tiles <= 1280 or per_tile >= four else 128 if per_tile >= two else 64
+    if main == "build_tables":
         return tile_blocks + (tables.n_tensors + threads - 1) // threads + (tables.n_strategies + threads - 1) // threads, threads
-    threads = 256 if per_tile >= 4096 else 128 if per_tile >= 512 else 64
     return tile_blocks, threads
 
 
@@ -741,7 +744,7 @@ def main():
         return
     if args.calibrate_launch:
         # the three workloads' launch shapes and bytes (bytes_per_launch of their roofline objects)
-        for name, nbytes, grid, threads in (("llama3_8b", 20_766_135, 1352, 256), ("llama3_70b", 596_653_014, 11736, 256),
+        for name, nbytes, grid, threads in (("llama3_8b", 20_766_135, 1329, 256), ("llama3_70b", 596_653_014, 20136, 256),
                                            ("stress", 3_825_705_690, 426920, 128)):
             floor_us, fill_us, per, through = calibrate_launch(nbytes, grid, threads)
             print(json.dumps({"workload": name, "bytes": nbytes, "grid": grid, "threads": threads, "launch_floor_us": floor_us,

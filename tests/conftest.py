@@ -9,7 +9,7 @@ if ROOT not in sys.path:
 
 
 def pytest_configure(config):
-    config.addinivalue_line("markers", "gpu: needs a real MI355X (run on the GPU box)")
+    config.addinivalue_line("markers", "gpu: needs a real MI355X")
     # load what is built; build only if nothing is
     from autoparallel_amd import _build
 

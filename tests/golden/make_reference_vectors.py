@@ -9,7 +9,7 @@ produces for the two steps of the path that no closed form pins:
     (autoparallel/compute_estimation.py:334-365), which runs each operator on fake tensors of the
     sharded argument shapes, so its result depends on every operator's meta kernel and flop formula.
 
-Runs only where /root/reference exists (never on a GPU box, never from a test).  What is imported:
+Runs only where /root/reference exists (never from a test).  What is imported:
 ``autoparallel.compute_estimation``, ``autoparallel.utils``, ``autoparallel.propagation_rules``
 (and through them ``autoparallel.dtensor_util``): torch-only modules.  Under the installed torch
 2.10 their import needs one name restored: ``register_op_strategy`` has moved from
