@@ -149,9 +149,6 @@ def unpack_codes(packed: int, ndim: int) -> tuple:
     return tuple((int(packed) >> (8 * i)) & 0xFF for i in range(ndim))
 
 
-_RANK_ROW = (APC_MAX_RANK,)
-
-
 def _i32(x):
     return np.ascontiguousarray(x, dtype=np.int32)
 
@@ -235,22 +232,24 @@ class CostTables:
         out = []
         for name in names:
             a = np.ascontiguousarray(getattr(self, name), self._DTYPES[name])
-            if a.shape[1:] != (_RANK_ROW if name in ("tensor_shape", "tensor_stride") else ()):
-                raise ValueError(f"{name} has the shape {a.shape}")
+            if name in ("tensor_shape", "tensor_stride"):
+                if a.shape[1:] != (APC_MAX_RANK,):
+                    raise ValueError(f"{name} must be [T, {APC_MAX_RANK}]")
+            elif a.ndim != 1:
+                if name not in ("spec_codes", "pt_values"):  # (whose rows are runs of values, whatever their shape)
+                    raise ValueError(f"{name} has the shape {a.shape}")
+                a = a.reshape(-1)
             if len(a) < n or (exact and len(a) != n):
                 raise ValueError(f"{name} must have {n} rows, it has {len(a)}")
             out.append(a)
         return out
 
-    def _tensor_rows(self) -> list:
-        return self._rows(self.n_tensors, "tensor_rank", "tensor_itemsize", "tensor_shape", "tensor_stride")
-
-    def _strategy_rows(self) -> list:
+    def _strategy_rows(self, exact: bool = False) -> list:
         return self._rows(self.n_strategies, "strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost", "strat_num_args",
-                          exact=True)
+                          exact=exact)
 
-    def _matrix_sizes(self) -> list:
-        return self._rows(self.n_edges, "edge_n_src", "edge_n_tgt", exact=True)
+    def _matrix_sizes(self, exact: bool = True) -> list:
+        return self._rows(self.n_edges, "edge_n_src", "edge_n_tgt", exact=exact)
 
     @staticmethod
     def _records(records, n: int, dtype) -> np.ndarray:
@@ -327,7 +326,7 @@ class CostTables:
     def validate_row_minima(self) -> None:
         """Raises unless every matrix row lies inside one tile (the precondition of the
         ``apc_*_row_min`` entry points), through the library's host-side check."""
-        _native.host_call("apc_validate_row_minima_host", self.n_edges, *self._matrix_sizes(), self.n_tiles,
+        _native.host_call("apc_validate_row_minima_host", self.n_edges, *self._matrix_sizes(exact=False), self.n_tiles,
                           self._records(self.tile_records, self.n_tiles, TILE_DTYPE))
 
     # ---- tiles -------------------------------------------------------------------------
@@ -341,7 +340,7 @@ class CostTables:
             self.n_edges, "edge_src_begin", "edge_tgt_begin", "edge_flags", "edge_pt_begin", "edge_strat_begin")
         _native.host_call(
             "apc_edge_classes_host", self.n_specs, *self._rows(self.n_specs, "spec_codes", "spec_tensor"), self.n_strategies,
-            *self._strategy_rows(), self.n_edges, src_begin, n_src, tgt_begin, n_tgt, flags, pt_begin, strat_begin,
+            *self._strategy_rows(exact=True), self.n_edges, src_begin, n_src, tgt_begin, n_tgt, flags, pt_begin, strat_begin,
             len(self.pt_values), *self._rows(0, "pt_values"), first_same)
         return first_same
 
@@ -494,7 +493,8 @@ class CostTables:
     def _packed_sources(self) -> list:
         """What a packed tile is copied out of, as the library takes it."""
         self._matrix_sizes()  # (the rows of all edges come from their sizes)
-        return [self.n_tensors, *self._tensor_rows(), self.n_specs, *self._rows(self.n_specs, "spec_codes", "spec_tensor"),
+        return [self.n_tensors, *self._rows(self.n_tensors, "tensor_rank", "tensor_itemsize", "tensor_shape", "tensor_stride"),
+                self.n_specs, *self._rows(self.n_specs, "spec_codes", "spec_tensor"),
                 self.n_strategies, *self._strategy_rows(), self.n_edges, self.edge_row_begin(), self.n_tiles,
                 self._records(self.tile_records, self.n_tiles, TILE_DTYPE), len(self.dup_entry_begin),
                 *self._rows(len(self.dup_entry_begin), "dup_entry_begin", "dup_row_begin")]
@@ -537,7 +537,7 @@ class CostTables:
                 raise RuntimeError(f"{name} must have n_strategies rows")
         if self.tile_records is None or len(self.tile_records) != self.n_tiles:
             raise RuntimeError("tile_records must have one record per tile (call pack_tile_records())")
-        rank, itemsize, shape, _ = self._tensor_rows()
+        rank, itemsize, shape = self._rows(self.n_tensors, "tensor_rank", "tensor_itemsize", "tensor_shape", exact=True)
         codes, spec_tensor = self._rows(self.n_specs, "spec_codes", "spec_tensor")
         flops, rw_bytes, *_, num_args = self._strategy_rows()
         n_src, n_tgt = self._matrix_sizes()
@@ -555,7 +555,7 @@ class CostTables:
         _native.host_call(
             "apc_validate_tiling_host", self.n_tensors, rank, itemsize, shape, self.n_strategies, flops, rw_bytes, num_args,
             self.n_edges, n_src, n_tgt, canonical, dup_count, len(dup_entry_begin), self.n_tiles,
-            *self._rows(self.n_tiles, "tile_edge", "tile_row_count", "tile_col_count"))
+            *self._rows(self.n_tiles, "tile_edge", "tile_row_count", "tile_col_count", exact=True))
 
     def as_dict(self) -> dict:
         """Plain-data view (numpy arrays) of every table."""

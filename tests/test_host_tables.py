@@ -153,6 +153,27 @@ def test_an_array_that_ends_early_is_refused_before_it_is_read(method, name):
             _read(tb, method)
 
 
+def test_tables_that_are_too_long_or_of_another_shape_are_refused_where_they_were():
+    """Where lengths have to agree, not only to suffice."""
+    for method, name in (("build_tiles", "edge_n_tgt"), ("edge_classes", "strat_flops"), ("edge_classes", "strat_num_args"),
+                         ("validate", "tensor_shape"), ("validate", "tile_row_count")):
+        tb = _two_layers()
+        a = getattr(tb, name)
+        setattr(tb, name, np.concatenate([a, a[-1:]]))
+        with pytest.raises(ValueError):
+            _read(tb, method)
+    for method, name in (("build_tiles", "edge_n_src"), ("pack_tiles", "spec_tensor"), ("edge_classes", "strat_dtype")):
+        tb = _two_layers()
+        setattr(tb, name, getattr(tb, name).reshape(-1, 1))
+        with pytest.raises(ValueError):
+            _read(tb, method)
+    want, tb = _two_layers(), _two_layers()
+    tb.pt_values, tb.spec_tensor = tb.pt_values.reshape(-1, 1), np.concatenate([tb.spec_tensor, [0]])
+    assert np.array_equal(tb.edge_classes(), want.edge_classes())
+    tb.build_tiles(512, dedupe=True)
+    assert tb.tile_records.tobytes() == want.tile_records.tobytes()
+
+
 @pytest.mark.parametrize("method", READS)
 def test_arrays_of_other_types_and_strides_are_read_by_value(method):
     want, tb = _two_layers(), _two_layers()
