@@ -232,3 +232,46 @@ def test_index_arrays_of_other_types_and_strides_are_read_by_value():
     for name in ("label_begin", "inc_begin", "inc_edge", "inc_side", "edge_begin", "edge_i", "edge_j"):
         setattr(g, name, np.repeat(getattr(g, name).astype(np.int32), 2)[::2])
         assert (pruning.lower_bound(g, g.theta, g.unary)[0], pruning.decode(g, g.theta, g.unary).tolist()) == want, name
+
+
+@pytest.mark.parametrize("what", [np.nan, -np.inf])
+@pytest.mark.parametrize("seed", range(6))
+def test_minima_over_nan_and_infinities_are_numpys(seed, what):
+    """A minimum over values with a NaN is a NaN, the first NaN is the smallest label's place, infinities of both signs are
+    values like others; sizes around the four rows and eight columns taken at a time."""
+    rng = np.random.default_rng(seed)
+    sizes = [9, 1 + seed, 8, 17, 4]
+    blocks, costs, at = [], {}, 0
+    for i, j in ((1, 0), (0, 2), (3, 2), (3, 4), (4, 1)):
+        m = rng.uniform(-5, 5, (sizes[i], sizes[j]))
+        m[rng.random(m.shape) < 0.1] = np.inf
+        m[rng.random(m.shape) < 0.04] = what
+        blocks.append(pruning.Block(at, sizes[i], sizes[j], i, j))
+        costs[at] = m
+        at += m.size
+    g = pruning.build_label_graph(blocks, sizes, lambda b: costs[b.var_begin], {}, [])
+    unary = rng.uniform(0, 5, len(g.unary))
+    unary[rng.random(len(unary)) < 0.05] = what
+    span = [slice(int(b), int(e)) for b, e in zip(g.label_begin[:-1], g.label_begin[1:])]
+    with np.errstate(invalid="ignore"):
+        _, umin, emin = pruning.lower_bound(g, g.theta, unary)
+        assert np.array_equal(umin, [unary[s].min() for s in span], equal_nan=True)
+        assert np.array_equal(emin, [g.matrix(g.theta, k).min() for k in range(g.n_edges)], equal_nan=True)
+        want = []
+        for c in range(g.n_classes):
+            score = unary[span[c]].copy()
+            for t in range(int(g.inc_begin[c]), int(g.inc_begin[c + 1])):
+                k, side = int(g.inc_edge[t]), int(g.inc_side[t])
+                m = g.matrix(g.theta, k) if side == 0 else g.matrix(g.theta, k).T
+                other = int(g.edge_j[k]) if side == 0 else int(g.edge_i[k])
+                score = score + (m[:, want[other]] if other < c else m.min(axis=1))
+            want.append(int(np.argmin(score)))
+        assert pruning.decode(g, g.theta, unary).tolist() == want
+
+
+def test_a_matrix_of_a_class_without_labels_is_refused():
+    g = pruning.build_label_graph([pruning.Block(0, 3, 0, 0, 1)], [3, 0], lambda b: np.zeros((3, 0)), {}, [])
+    for call in (lambda: pruning.lower_bound(g, g.theta, g.unary), lambda: pruning.decode(g, g.theta, g.unary),
+                 lambda: pruning.refine(g, g.theta, g.unary, np.array([0, -1])), lambda: pruning.prune_masks(g, g.theta, g.unary, 1.0)):
+        with pytest.raises(RuntimeError, match="without labels"):
+            call()
