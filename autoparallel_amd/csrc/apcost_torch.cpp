@@ -29,6 +29,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <optional>
 #include <string>
@@ -150,7 +151,7 @@ void copy_bytes(void *to, const void *from, int64_t n) {
 
 // The pinned chunks of one transfer and the events that say when each is free again.
 struct Staging {
-  explicit Staging(int64_t total) {
+  Staging(int64_t total, hipStream_t s) : stream(s) {
     const int64_t n = std::min<int64_t>(kStagingSlots, std::max<int64_t>(1, (total + kStagingChunk - 1) / kStagingChunk));
     for (int64_t i = 0; i < n; ++i) {
       slots.push_back(at::empty({std::min(total, kStagingChunk)}, at::TensorOptions().dtype(at::kByte).pinned_memory(true)));
@@ -160,10 +161,13 @@ struct Staging {
     }
   }
   ~Staging() {
+    // (an exception on the way: the chunks go back to the allocator, which knows nothing of the copies in flight)
+    if (std::uncaught_exceptions() > 0) (void)hipStreamSynchronize(stream);
     for (hipEvent_t e : events)
       if (e) (void)hipEventDestroy(e);
   }
   char *slot(int64_t i) { return static_cast<char *>(slots[i].data_ptr()); }
+  hipStream_t stream;
   std::vector<Tensor> slots;
   std::vector<hipEvent_t> events;
 };
@@ -218,7 +222,7 @@ std::vector<Tensor> upload(const std::vector<Tensor> &arrays, at::Device device)
   }
   if (total == 0) return out;
   hipStream_t stream = c10::hip::getCurrentHIPStream(device.index()).stream();
-  Staging staging(total);
+  Staging staging(total, stream);
   const int64_t n_slots = (int64_t)staging.slots.size();
   size_t p = 0, r = 0;  // the first part, the first run that reach into the chunk
   int64_t chunk = 0;
@@ -257,7 +261,7 @@ std::vector<Tensor> download(const std::vector<Tensor> &arrays) {
   if (total == 0) return out;
   c10::hip::HIPGuard guard(device.index());
   hipStream_t stream = c10::hip::getCurrentHIPStream(device.index()).stream();
-  Staging staging(total);
+  Staging staging(total, stream);
   const int64_t n_slots = (int64_t)staging.slots.size();
   struct Piece {  // part of array k, staged in `slot` at `at`
     size_t k;
