@@ -569,6 +569,9 @@ class DeviceCostTables:
     # chip.  One that lasts this long (100 MHz ticks: 0.2 s) means that they are not, and ends the kernel.
     SWEEP_WAIT_TICKS = 20_000_000
 
+    # what the plan, and the copies on the device, are made of (the last one stays on the host)
+    _SWEEP_INDEX = ("color_nodes", "label_begin", "inc_begin", "inc_edge", "inc_side", "edge_begin", "edge_i", "edge_j", "color_begin")
+
     @staticmethod
     def _sweep_plan(graph):
         """-> (plan words, first word of every workgroup, slots, bytes of LDS, threads) of the resident sweeps
@@ -595,10 +598,11 @@ class DeviceCostTables:
         (read-only: handed back to the next call unchanged, they are not uploaded again).  A problem
         that fits the chip's LDS takes one kernel for all sweeps (``apc_diffusion_sweeps_resident``), any
         other one launch per colour (``apc_diffusion_sweeps``); the same bits.  What either needs of the
-        graph is worked out and uploaded once."""
+        graph is worked out and uploaded once, and again when one of its index arrays was replaced."""
         cached = getattr(self, "_diffusion_graph", None)
-        if cached is None or cached["graph"] is not graph:
-            cached = self._diffusion_graph = {"graph": graph, "plan": self._sweep_plan(graph)}
+        arrays = [getattr(graph, k) for k in self._SWEEP_INDEX]
+        if cached is None or cached["graph"] is not graph or any(x is not y for x, y in zip(cached["arrays"], arrays)):
+            cached = self._diffusion_graph = {"graph": graph, "arrays": arrays, "plan": self._sweep_plan(graph)}
             self._diffusion_state = None
         state = getattr(self, "_diffusion_state", None)
         if state is not None and state[0] is theta and state[1] is unary:
@@ -622,8 +626,7 @@ class DeviceCostTables:
         if out is None:
             d = cached.get("index")
             if d is None:
-                names = ("color_nodes", "label_begin", "inc_begin", "inc_edge", "inc_side", "edge_begin", "edge_i", "edge_j")
-                d = cached["index"] = self._upload(*(getattr(graph, k) for k in names))
+                d = cached["index"] = self._upload(*arrays[:-1])
             out = (th, un)
             max_labels = int(np.diff(graph.label_begin).max()) if graph.n_classes else 0
             self.ops.diffusion_sweeps_(int(n_sweeps), torch.from_numpy(np.ascontiguousarray(graph.color_begin, np.int64)), *d, max_labels,

@@ -105,6 +105,36 @@ def test_an_expired_wait_is_paid_once_per_problem():
         assert (Ops.resident, Ops.launches) == (i, 3 * i)
 
 
+def test_a_graph_whose_arrays_were_replaced_has_a_new_plan():
+    """On the CPU: an old plan would index the new problem's arrays by the old one's sizes."""
+    import torch
+
+    from autoparallel_amd.device_tables import DeviceCostTables
+
+    seen = []
+
+    class Ops:
+        def upload(self, arrays, device):
+            return [t.clone() for t in arrays]
+
+        def download(self, arrays):
+            return [t.clone() for t in arrays]
+
+        def diffusion_sweeps_resident(self, n, plan, begin, slots, lds, threads, n_labels, n_elements, theta, unary, ticks):
+            seen.append((sum(int(plan[b + 1]) for b in begin[:-1]), n_elements))  # elements of the plan, of the problem
+            return theta.clone(), unary.clone(), torch.zeros(1, dtype=torch.int32)
+
+    dev = DeviceCostTables.__new__(DeviceCostTables)
+    dev.ops, dev.device = Ops(), torch.device("cpu")
+    g, small = (_problem(1, *CASES[name]) for name in ("a chain over many workgroups", "rows of 1 to 70 elements, one workgroup's"))
+    dev.diffusion_sweeps(g, g.theta, g.unary, 4)
+    for name in ("label_begin", "unary", "edge_i", "edge_j", "edge_begin", "theta", "inc_begin", "inc_edge", "inc_side", "color_begin",
+                 "color_nodes"):
+        setattr(g, name, getattr(small, name))
+    dev.diffusion_sweeps(g, g.theta, g.unary, 4)
+    assert all(a == b for a, b in seen) and seen[0][0] > seen[1][0] == len(small.theta)
+
+
 @pytest.mark.parametrize("sizes,pairs", [([140, 140], [(0, 1)]), ([1500, 2], [(0, 1)])])
 def test_problems_that_do_not_fit_have_no_plan(sizes, pairs):
     from autoparallel_amd.device_tables import DeviceCostTables
