@@ -749,30 +749,49 @@ namespace {
 
 // As numpy takes minima: of values with a NaN among them a NaN.  The running minima pass one over; whether there may be
 // one is read off the values' sum, a NaN for any (and where infinities cancel), at one addition a value.
-inline bool smaller(double v, double d) { return v < d || v != v; }
+inline double with_nan(const double *v, int64_t n, int64_t stride = 1) {
+  double d = __builtin_inf();
+  for (int64_t i = 0; i < n; ++i) {
+    const double x = v[i * stride];
+    d = x < d || x != x ? x : d;
+  }
+  return d;
+}
 
-// The smallest of n values, +inf of none (eight running minima: the order of the comparisons is free).
-double least(const double *v, int64_t n) {
-  double d[8], s[8] = {};
+// (a loop of its own: in one with the comparisons neither becomes vector instructions)
+inline void add_up(const double *v, int64_t n, double (&s)[8]) {
+  int64_t i = 0;
+  for (; i + 8 <= n; i += 8)
+    for (int j = 0; j < 8; ++j) s[j] += v[i + j];
+  for (; i < n; ++i) s[0] += v[i];
+}
+
+inline bool may_hold_nan(const double (&s)[8]) {
+  const double t = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+  return t != t;
+}
+
+// The smallest of n values, +inf of none (eight running minima: the order of the comparisons is free), NaN passed over.
+inline double least_number(const double *v, int64_t n) {
+  double d[8];
   for (double &x : d) x = __builtin_inf();
   int64_t i = 0;
   for (; i + 8 <= n; i += 8)
-    for (int j = 0; j < 8; ++j) {
-      d[j] = v[i + j] < d[j] ? v[i + j] : d[j];
-      s[j] += v[i + j];
-    }
-  for (; i < n; ++i) {
-    d[0] = v[i] < d[0] ? v[i] : d[0];
-    s[0] += v[i];
-  }
-  double sum = s[0];
-  for (int j = 1; j < 8; ++j) {
-    d[0] = d[j] < d[0] ? d[j] : d[0];
-    sum += s[j];
-  }
-  if (sum != sum)
-    for (i = 0; i < n; ++i) d[0] = smaller(v[i], d[0]) ? v[i] : d[0];
+    for (int j = 0; j < 8; ++j) d[j] = v[i + j] < d[j] ? v[i + j] : d[j];
+  for (; i < n; ++i) d[0] = v[i] < d[0] ? v[i] : d[0];
+  for (int j = 1; j < 8; ++j) d[0] = d[j] < d[0] ? d[j] : d[0];
   return d[0];
+}
+
+double least(const double *v, int64_t n) {
+  double d = __builtin_inf(), s[8] = {};
+  for (int64_t i = 0; i < n; i += 1024) {  // (runs that stay in the first cache between the two loops)
+    const int64_t run = std::min<int64_t>(1024, n - i);
+    const double x = least_number(v + i, run);
+    d = x < d ? x : d;
+    add_up(v + i, run, s);
+  }
+  return may_hold_nan(s) ? with_nan(v, n) : d;
 }
 
 struct LabelProblem {
@@ -783,7 +802,18 @@ struct LabelProblem {
   const int64_t *edge_begin;
   const int32_t *edge_i, *edge_j;
   const double *theta, *unary;
+  bool theta_may_hold_nan = false;  // (where minima() is used: look_for_nan() first)
 
+  void look_for_nan() {
+    std::atomic<bool> found{false};
+    const int64_t n = edge_begin[n_edges], runs = (n + 4095) / 4096;
+    in_parallel(runs, threads_for(4 * n), [&](int64_t b, int64_t e) {
+      double s[8] = {};
+      add_up(theta + b * 4096, std::min(n, e * 4096) - b * 4096, s);
+      if (may_hold_nan(s)) found.store(true, std::memory_order_relaxed);
+    });
+    theta_may_hold_nan = found.load();
+  }
   int64_t labels(int64_t c) const { return label_begin[c + 1] - label_begin[c]; }
   int64_t other(int64_t k, int side) const { return side == 0 ? edge_j[k] : edge_i[k]; }
   // every index the walks below use lies inside its array, and every matrix has its classes' shape
@@ -812,38 +842,14 @@ struct LabelProblem {
   void minima(int64_t k, int side, double *out) const {
     const double *m = theta + edge_begin[k];
     const int64_t ni = labels(edge_i[k]), nj = labels(edge_j[k]);
-    if (side == 0) {
-      for (int64_t x = 0; x < ni; ++x) out[x] = least(m + x * nj, nj);
+    if (theta_may_hold_nan) {
+      for (int64_t x = 0; x < (side == 0 ? ni : nj); ++x) out[x] = side == 0 ? with_nan(m + x * nj, nj) : with_nan(m + x, ni, nj);
+    } else if (side == 0) {
+      for (int64_t x = 0; x < ni; ++x) out[x] = least_number(m + x * nj, nj);
     } else {
       for (int64_t y = 0; y < nj; ++y) out[y] = __builtin_inf();
-      double s[8] = {};
-      int64_t x = 0;
-      for (; x + 4 <= ni; x += 4) {  // (four rows at a time: the running minima are loaded and stored once for them)
-        const double *const __restrict r = m + x * nj;
-        double *const __restrict o = out;
-        int64_t y = 0;
-        for (; y + 8 <= nj; y += 8)
-          for (int j = 0; j < 8; ++j) {
-            const double a = r[y + j], b = r[nj + y + j], c = r[2 * nj + y + j], d = r[3 * nj + y + j];
-            const double ab = b < a ? b : a, cd = d < c ? d : c, v = cd < ab ? cd : ab;
-            o[y + j] = v < o[y + j] ? v : o[y + j];
-            s[j] += (a + b) + (c + d);
-          }
-        for (; y < nj; ++y)
-          for (int i = 0; i < 4; ++i) {
-            o[y] = r[i * nj + y] < o[y] ? r[i * nj + y] : o[y];
-            s[0] += r[i * nj + y];
-          }
-      }
-      for (; x < ni; ++x)
-        for (int64_t y = 0; y < nj; ++y) {
-          out[y] = m[x * nj + y] < out[y] ? m[x * nj + y] : out[y];
-          s[0] += m[x * nj + y];
-        }
-      for (int j = 1; j < 8; ++j) s[0] += s[j];
-      if (s[0] != s[0])
-        for (int64_t x = 0; x < ni; ++x)
-          for (int64_t y = 0; y < nj; ++y) out[y] = smaller(m[x * nj + y], out[y]) ? m[x * nj + y] : out[y];
+      for (int64_t x = 0; x < ni; ++x)
+        for (int64_t y = 0; y < nj; ++y) out[y] = m[x * nj + y] < out[y] ? m[x * nj + y] : out[y];
     }
   }
   // score[x] += the matrix of edge k at (x, label of the other end)
@@ -913,7 +919,7 @@ int apc_label_incidence_host(int64_t n_classes, int64_t n_edges, const int32_t *
       int64_t n_edges, const int64_t *edge_begin, const int32_t *edge_i, const int32_t *edge_j, const double *theta,          \
       const double *unary
 #define APC_LABEL_PROBLEM_OF(who)                                                                                             \
-  const LabelProblem g{n_classes, n_edges, label_begin, inc_begin, inc_edge, inc_side, edge_begin, edge_i, edge_j, theta, unary}; \
+  LabelProblem g{n_classes, n_edges, label_begin, inc_begin, inc_edge, inc_side, edge_begin, edge_i, edge_j, theta, unary};      \
   if (!g.holds()) return fail(-2, who ": the index arrays do not describe a labelling problem");                               \
   if (g.has_empty_matrix()) return fail(-2, who ": a matrix of a class without labels has no minimum")
 
@@ -933,6 +939,7 @@ int apc_label_minima_host(APC_LABEL_PROBLEM, double *class_min, double *edge_min
 
 int apc_round_labels_host(APC_LABEL_PROBLEM, int64_t *labels) try {
   APC_LABEL_PROBLEM_OF("apc_round_labels_host");
+  g.look_for_nan();
   std::vector<double> score, d;
   for (int64_t c = 0; c < n_classes; ++c) labels[c] = -1;
   for (int64_t c = 0; c < n_classes; ++c) {
@@ -991,6 +998,7 @@ int apc_refine_labels_host(APC_LABEL_PROBLEM, int64_t max_rounds, int64_t *label
 int apc_prune_masks_host(APC_LABEL_PROBLEM, const double *class_min, const double *edge_min, double bound, double limit,
                          uint8_t *dead_label, uint8_t *dead_pair) try {
   APC_LABEL_PROBLEM_OF("apc_prune_masks_host");
+  g.look_for_nan();
   const int threads = threads_for(8 * edge_begin[n_edges]);
   in_parallel(n_classes, threads, [&](int64_t begin, int64_t end) {
     std::vector<double> b, d;
