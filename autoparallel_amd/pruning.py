@@ -160,21 +160,17 @@ def build_label_graph(blocks: list, class_sizes: list, block_costs, masks: dict,
                       color_nodes=color_nodes, blocks=blocks)
 
 
-_INDEX = (("label_begin", np.int64), ("inc_begin", np.int64), ("inc_edge", np.int32), ("inc_side", np.uint8),
-          ("edge_begin", np.int64), ("edge_i", np.int32), ("edge_j", np.int32))
-
-
 def index_arrays(g: LabelGraph) -> tuple:
     """The index arrays of the problem as the library's host entry points read them, which see an address and not
     where its array ends: contiguous, of their types, none shorter than it is read."""
-    index = tuple(np.ascontiguousarray(getattr(g, name), dtype) for name, dtype in _INDEX)
-    n, ne = g.n_classes, g.n_edges
-    if len(index[1]) <= n:
-        raise ValueError(f"inc_begin must have {n + 1} rows")
-    n_inc = int(index[1][n])
-    for (name, _), a, rows in zip(_INDEX, index, (n + 1, n + 1, n_inc, n_inc, ne + 1, ne, ne)):
-        if a.ndim != 1 or len(a) < rows:
-            raise ValueError(f"{name} must have {rows} rows, it is {a.shape}")
+    c = np.ascontiguousarray
+    index = (c(g.label_begin, np.int64), c(g.inc_begin, np.int64), c(g.inc_edge, np.int32), c(g.inc_side, np.uint8),
+             c(g.edge_begin, np.int64), c(g.edge_i, np.int32), c(g.edge_j, np.int32))
+    label_begin, inc_begin, inc_edge, inc_side, edge_begin, edge_i, edge_j = index
+    n, n_edges = label_begin.size - 1, edge_i.size
+    if n < 0 or inc_begin.size <= n or edge_begin.size <= n_edges or edge_j.size < n_edges \
+            or min(inc_edge.size, inc_side.size) < inc_begin[n]:
+        raise ValueError("the index arrays do not describe a labelling problem: one of them ends early")
     return index
 
 
