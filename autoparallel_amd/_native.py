@@ -104,6 +104,8 @@ EXPORTS = (
     "apc_refine_labels_host",
     "apc_prune_masks_host",
     "apc_build_tables_packed",
+    "apc_keep_next_launch",
+    "apc_run_kept",
     "apc_calibrate_launch",
     "apc_calibrate_fill",
 )

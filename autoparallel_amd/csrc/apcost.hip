@@ -73,6 +73,28 @@ template <typename T>
 __device__ __forceinline__ void store_through(T *p, T value) {
   __hip_atomic_store(p, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+// Where a launch's arguments lie.  The table kernels take more than a kilobyte of them, and what a launch passes by value
+// is read from a segment that the host has just written: every compute unit fetches it past the caches.  A launch that
+// is repeated keeps its arguments in a block of device memory, which the L2 holds, and passes the block's address; `kept`
+// is NULL where a launch is made once, and its arguments are then the by-value ones, which every kernel takes last, behind
+// kLaunchHeadBytes of others.  (Kernels that read 1 KB of arguments and store 2.3 MB, back to back: 5.6 us a launch by
+// value, 3.15 from a block, 2.45 without the arguments.  The planner's pass: 1.7 M entries on (32, 8) over packed tiles 8.9 ->
+// 8.15 us, 20 M on (16, 8, 4) in two launches 70.2 -> 68.7, 2.6 M on (12, 6) over staged tiles, whose wavefronts have other
+// loads to wait for at that time, 18.4 -> 18.7.)
+constexpr size_t kLaunchHeadBytes = 40;
+template <typename Block>
+__device__ __forceinline__ const Block &launch_block(const Block *kept) {
+  static_assert(alignof(Block) == 8, "the block follows the other arguments without padding");
+  // (chosen as a number: of two pointers, of which one comes from the global address space, the compiler makes a generic
+  // one, and of every load through it a flat one)
+  const uint64_t by_value = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr() + kLaunchHeadBytes;
+  const uint64_t at = kept ? (uint64_t)kept : by_value;
+  return *(const Block *)(const APC_CONSTANT Block *)at;
+}
+// (the arguments of every such kernel; `kept` arrives in registers with the wavefront, as do those in front of it)
+#define APC_LAUNCH_PARAMS(BLOCK_) \
+  const void *work, int n_tiles, int xcd_shift, int64_t tile_blocks, double *cost_out, const BLOCK_ *kept, BLOCK_ by_value
+
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 typedef int64_t i64x8 __attribute__((ext_vector_type(8)));
 
@@ -185,6 +207,21 @@ __device__ __forceinline__ void fetch_arguments_now(T0 v0, T1 v1, T2 v2, T3 v3, 
   __asm__ volatile("" ::"s"(v0), "s"(v1), "s"(v2), "s"(v3), "s"(v4), "s"(v5), "s"(v6), "s"(v7), "s"(v8), "s"(v9), "s"(v10), "s"(v11), "s"(v12), "s"(v13), "s"(v14), "s"(v15), "s"(v16), "s"(v17), "s"(v18), "s"(v19), "s"(v20), "s"(v21), "s"(v22), "s"(v23));
 }
 
+// Element `i` (a per-lane index below M) of one of the arrays of the kernel parameters, as a select chain over scalar registers.  (Indexing the array by a lane value
+// makes the compiler read the kernel arguments through vector memory, and a vector load
+// waits behind every store the compute unit has in flight.)
+template <int M, typename T, int N>
+__device__ __forceinline__ T pick(const T (&v)[N], int i) {
+  static_assert(M <= N, "array shorter than the mesh");
+  T e[M];  // every element is read (scalar loads) before the selects, so they stay selects
+#pragma unroll
+  for (int k = 0; k < M; ++k) e[k] = v[k];
+  T r = e[0];
+#pragma unroll
+  for (int k = 1; k < M; ++k) r = i == k ? e[k] : r;
+  return r;
+}
+
 // compute_estimation.py:302-314
 __device__ __forceinline__ double rw_time(double bytes, const apc_params &p) {
   double t = bytes / p.hbm_bw * 1e6;
@@ -192,10 +229,10 @@ __device__ __forceinline__ double rw_time(double bytes, const apc_params &p) {
   return t > p.launch_floor ? t : p.launch_floor;
 }
 
-// torch _collective_utils.py:281-313: latency + bandwidth term of a ring collective
-__device__ __forceinline__ double ring(double gb, const apc_params &p, int d, int hops) {
-  double latency = p.base_latency + (double)hops * p.lat[d];
-  double bw = (gb * (double)hops / (double)p.mesh_size[d]) / p.bw[d];
+// torch _collective_utils.py:281-313: latency + bandwidth term of a ring collective over a dim of `size` devices
+__device__ __forceinline__ double ring(double gb, const apc_params &p, int size, double lat, double bandwidth, int hops) {
+  double latency = p.base_latency + (double)hops * lat;
+  double bw = (gb * (double)hops / (double)size) / bandwidth;
   return latency + bw * 1e6;
 }
 
@@ -245,23 +282,24 @@ __device__ __forceinline__ double entry_cost(uint32_t srcp, uint32_t tgtp, doubl
     const int i = (M == 2 && flip) ? 1 - k : k;
     const uint32_t c = (srcp >> (8 * i)) & 0xFF, t = (tgtp >> (8 * i)) & 0xFF;
     if (c == t) continue;
-    const double n = (double)p.mesh_size[i];
+    const int size = pick<M>(p.mesh_size, i);
+    const double n = (double)size, lat = pick<M>(p.lat, i), bw = pick<M>(p.bw, i);
     if (!cont) cost += rw_time(gb * 2 * 1073741824.0, p);
     const int ck = kind_of(c), tk = kind_of(t);
     if (ck == 2 && tk == 0) {  // all-gather (:83-96)
       gb *= n;
-      cost += ring(gb, p, i, p.mesh_size[i] - 1);
+      cost += ring(gb, p, size, lat, bw, size - 1);
       if (dim_of(c) != 0) cost += rw_time(gb * 2 * 1073741824.0, p);
     } else if (ck == 2 && tk == 2) {  // all-to-all (:97-113)
-      double a2a = ring(gb, p, i, p.mesh_size[i] - 1);
+      double a2a = ring(gb, p, size, lat, bw, size - 1);
       a2a *= p.a2a_scale;
       cost += a2a;
       const int copies = (dim_of(c) != 0) + (dim_of(t) != 0);
       cost += (double)copies * rw_time(gb * 2 * 1073741824.0, p);
     } else if (ck == 1 && tk == 0) {  // all-reduce (:115-117)
-      cost += ring(gb, p, i, 2 * (p.mesh_size[i] - 1));
+      cost += ring(gb, p, size, lat, bw, 2 * (size - 1));
     } else if (ck == 1 && tk == 2) {  // reduce-scatter (:118-130)
-      cost += ring(gb, p, i, p.mesh_size[i] - 1);
+      cost += ring(gb, p, size, lat, bw, size - 1);
       if (dim_of(t) != 0) cost += rw_time(gb * 2 * 1073741824.0, p);
       gb /= n;
     } else if (tk == 1 && ck != 1) {  // Shard->Partial, Replicate->Partial banned (:131-138)
@@ -302,21 +340,6 @@ struct States {
 __device__ __forceinline__ int64_t xcd_chunked_unit(int shift) {
   const int64_t per = gridDim.x >> shift;
   return (int64_t)(blockIdx.x & ((1u << shift) - 1)) * per + (blockIdx.x >> shift);
-}
-
-// Element `i` (a per-lane index below M) of one of the arrays of the kernel parameters, as a select chain over scalar registers.  (Indexing the array by a lane value
-// makes the compiler read the kernel arguments through vector memory, and a vector load
-// waits behind every store the compute unit has in flight.)
-template <int M, typename T, int N>
-__device__ __forceinline__ T pick(const T (&v)[N], int i) {
-  static_assert(M <= N, "array shorter than the mesh");
-  T e[M];  // every element is read (scalar loads) before the selects, so they stay selects
-#pragma unroll
-  for (int k = 0; k < M; ++k) e[k] = v[k];
-  T r = e[0];
-#pragma unroll
-  for (int k = 1; k < M; ++k) r = i == k ? e[k] : r;
-  return r;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -650,14 +673,21 @@ __global__ __launch_bounds__(kBlock) void strategy_inputs_kernel(StrategyInputAr
 // The three tables above in one launch: workgroups [0, spec_blocks) take the spec table (the
 // largest), the next tensor_blocks the tensor table, the rest the compute costs.  None of the
 // three reads another's output.
-__global__ __launch_bounds__(kBlock) void input_tables_kernel(apc_params p, TensorTableArgs t, SpecTableArgs sp,
-                                                              ComputeCostArgs c, int64_t spec_blocks,
-                                                              int64_t tensor_blocks) {
+struct InputTablesBlock {
+  apc_params p;
+  TensorTableArgs t;
+  SpecTableArgs sp;
+  ComputeCostArgs c;
+  int64_t spec_blocks, tensor_blocks;
+};
+
+__global__ __launch_bounds__(kBlock) void input_tables_kernel(APC_LAUNCH_PARAMS(InputTablesBlock)) {
   __shared__ int64_t s_rows[kBlock * (APC_MAX_RANK + 1)];
+  const InputTablesBlock &k = launch_block(kept);
   const int64_t b = blockIdx.x;
-  if (b < spec_blocks) spec_tables_block<kBlock>(b, p, sp, s_rows);
-  else if (b < spec_blocks + tensor_blocks) tensor_tables_block<kBlock>(b - spec_blocks, t);
-  else compute_costs_block<kBlock>(b - spec_blocks - tensor_blocks, p, c);
+  if (b < k.spec_blocks) spec_tables_block<kBlock>(b, k.p, k.sp, s_rows);
+  else if (b < k.spec_blocks + k.tensor_blocks) tensor_tables_block<kBlock>(b - k.spec_blocks, k.t);
+  else compute_costs_block<kBlock>(b - k.spec_blocks - k.tensor_blocks, k.p, k.c);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1230,11 +1260,23 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
   if ((tid & 63) == 0) st.mixed[tid >> 6] = wave_mixed ? 1 : 0;
 }
 
+// The arguments an entry loop uses, in scalar registers before it begins.  (Left to the compiler, an argument is loaded
+// where it is used, in every pass, and a scalar load in flight makes the wait for an LDS read a wait for everything.)
+struct EntryConstants {
+  double rescale, inv_rescale;
+  int32_t transition_scale, state_stride;
+};
+__device__ __forceinline__ EntryConstants entry_constants(const apc_params &p, const TermLayout &lay) {
+  EntryConstants k{p.rescale, lay.inv_rescale, p.transition_scale, lay.state_stride};
+  __asm__ volatile("" : "+s"(k.rescale), "+s"(k.inv_rescale), "+s"(k.transition_scale), "+s"(k.state_stride));
+  return k;
+}
+
 // One entry of a tile whose producer specs all name one tensor (column c, row r of the tile).
 // Straight-line code: all lookups of an entry are independent of its fp additions, so they
 // are issued together; no vector memory loads.
 template <int M, bool CONT, bool RESCALE, bool RM>
-__device__ __forceinline__ void uniform_entry(const apc_params &p, const TermLayout &lay, const TileStage<M, RM> &st,
+__device__ __forceinline__ void uniform_entry(const apc_params &p, const EntryConstants &k, const TileStage<M, RM> &st,
                                               const char *terms, int r, int c, double &comm_o, double &total_o,
                                               int &trans_o) {
   const uint32_t src = st.col_codes[c];
@@ -1255,7 +1297,7 @@ __device__ __forceinline__ void uniform_entry(const apc_params &p, const TermLay
     term_at[i] = (w & 0xFFFFu) + at;
     rw_at[i] = term_at[i] + (uint32_t)(int32_t)(int8_t)(w >> 16);
     if (!CONT) nc_at[i] = *reinterpret_cast<const uint32_t *>(words + (kWordsPerDim * i + 5) * 4) + at;
-    at += (uint32_t)__mul24((int32_t)w >> 24, lay.state_stride);  // (24-bit multiplies issue at full rate)
+    at += (uint32_t)__mul24((int32_t)w >> 24, k.state_stride);  // (24-bit multiplies issue at full rate)
   }
   // ---- lookups ------------------------------------------------------------------------------
   double term[M], rw[M], nc[M];
@@ -1280,12 +1322,12 @@ __device__ __forceinline__ void uniform_entry(const apc_params &p, const TermLay
     cost += rw[i];  // 0, 1 or 2 read+writes: (double)copies * rw, picked from the staged multiples
   }
   double comm = cost;  // (a banned transition added the +inf term)
-  const int trans = x != 0u ? p.transition_scale : 0;  // optimize_sharding.py:345-351
+  const int trans = x != 0u ? k.transition_scale : 0;  // optimize_sharding.py:345-351
   if (M == 2 && src == 0x4040u && (row.slots & kRowAllShard)) {  // (Partial, Partial) -> all Shard walks dim 1 first
     comm = entry_cost<M>(src, tgt, st.gb_unsharded, CONT, p);
   }
   // :358-359; the quotient through the reciprocal is the division's (div_by), +inf stays +inf
-  if (RESCALE) comm = comm < __builtin_inf() ? div_by(comm, p.rescale, lay.inv_rescale) : comm;
+  if (RESCALE) comm = comm < __builtin_inf() ? div_by(comm, k.rescale, k.inv_rescale) : comm;
   comm_o = comm;
   total_o = comm + row.cpa + (double)trans;  // :368-372
   trans_o = trans;
@@ -1457,11 +1499,12 @@ __device__ __forceinline__ void uniform_tile_entries_row_min(const apc_params &p
   int r = first / v.cols, c = first - r * v.cols;
   const TileOut out{a.comm_out ? a.comm_out + tile_base : nullptr, a.trans_out ? a.trans_out + tile_base : nullptr,
                     a.cost_out ? a.cost_out + tile_base : nullptr, v.entry_begin};
+  const EntryConstants k = entry_constants(p, a.lay);
   for (int wave_first = tid - lane - shift; wave_first < n; wave_first += nthreads, idx += nthreads) {
     const bool active = idx >= 0 && idx < n;
     double comm = 0.0, total = 0.0;
     int trans = 0;
-    if (active) uniform_entry<M, CONT, RESCALE>(p, a.lay, st, term_base(st, nthreads), r, c, comm, total, trans);
+    if (active) uniform_entry<M, CONT, RESCALE>(p, k, st, term_base(st, nthreads), r, c, comm, total, trans);
     store_entry<OUT>(out, v.dup_count, copies, active, __umul24((uint32_t)r, (uint32_t)v.n_src) + (uint32_t)c, comm, total,
                      trans);
     row_min_chunk(st.rmin, st.rarg, active, total, r, c, v.cols, lane);
@@ -1497,11 +1540,12 @@ __device__ __forceinline__ void uniform_tile_entries(const apc_params &p, const 
   int r = first / v.cols, c = first - r * v.cols;
   const TileOut out{a.comm_out ? a.comm_out + tile_base : nullptr, a.trans_out ? a.trans_out + tile_base : nullptr,
                     a.cost_out ? a.cost_out + tile_base : nullptr, v.entry_begin};
+  const EntryConstants k = entry_constants(p, a.lay);
   for (int wave_first = tid - lane - shift; wave_first < n; wave_first += nthreads, idx += nthreads) {
     const bool active = idx >= 0 && idx < n;
     double comm = 0.0, total = 0.0;
     int trans = 0;
-    if (active) uniform_entry<M, CONT, RESCALE>(p, a.lay, st, term_base(st, nthreads), r, c, comm, total, trans);
+    if (active) uniform_entry<M, CONT, RESCALE>(p, k, st, term_base(st, nthreads), r, c, comm, total, trans);
     store_entry<OUT>(out, v.dup_count, copies, active, __umul24((uint32_t)r, (uint32_t)v.n_src) + (uint32_t)c, comm, total,
                      trans);
     if (active) {
@@ -1678,11 +1722,17 @@ constexpr int tile_waves_per_simd(int mesh_ndim, int threads, bool row_min) {
   return threads == 128 && !row_min ? 8 : 7;
 }
 
+struct TilesBlock {
+  apc_params p;
+  TableArgs a;
+};
+
 template <int M, int kTileThreads, int OUT>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(tile_waves_per_simd(M, kTileThreads, false), 8)))
-void redistribute_tiles_kernel(const apc_tile *tiles, int n_tiles, int xcd_shift, apc_params p, TableArgs a) {
+void redistribute_tiles_kernel(APC_LAUNCH_PARAMS(TilesBlock)) {
   extern __shared__ __align__(16) unsigned char s_stage_bytes[];  // stage_lds_bytes<M, false>
-  redistribute_tile<M, kTileThreads, false, OUT>(p, a, tiles, n_tiles, xcd_shift,
+  const TilesBlock &k = launch_block(kept);
+  redistribute_tile<M, kTileThreads, false, OUT>(k.p, k.a, static_cast<const apc_tile *>(work), n_tiles, xcd_shift,
                                                  *reinterpret_cast<TileStage<M, false> *>(s_stage_bytes));
 }
 
@@ -1690,9 +1740,10 @@ void redistribute_tiles_kernel(const apc_tile *tiles, int n_tiles, int xcd_shift
 template <int M, int kTileThreads, int OUT>
 __global__ __launch_bounds__(kTileThreads)
 __attribute__((amdgpu_waves_per_eu(tile_waves_per_simd(M, kTileThreads, true), 8)))
-void redistribute_tiles_row_min_kernel(const apc_tile *tiles, int n_tiles, int xcd_shift, apc_params p, TableArgs a) {
+void redistribute_tiles_row_min_kernel(APC_LAUNCH_PARAMS(TilesBlock)) {
   extern __shared__ __align__(16) unsigned char s_stage_bytes[];  // stage_lds_bytes<M, true>
-  redistribute_tile<M, kTileThreads, true, OUT>(p, a, tiles, n_tiles, xcd_shift,
+  const TilesBlock &k = launch_block(kept);
+  redistribute_tile<M, kTileThreads, true, OUT>(k.p, k.a, static_cast<const apc_tile *>(work), n_tiles, xcd_shift,
                                                 *reinterpret_cast<TileStage<M, true> *>(s_stage_bytes));
 }
 
@@ -1735,11 +1786,22 @@ __device__ __forceinline__ unsigned char *build_tables_lds() {
   }
 }
 
+struct BuildTablesBlock {
+  apc_params p;
+  TableArgs a;
+  TensorTableArgs t;
+  SpecTableArgs sp;
+  ComputeCostArgs c;
+  int64_t spec_blocks, tensor_blocks;
+};
+
 template <int M, int kThreads, bool RM, int OUT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(M <= 2 ? 5 : 1, M <= 2 ? 5 : 8)))
-void build_tables_kernel(const apc_tile *tiles, int n_tiles, int xcd_shift, int64_t tile_blocks, apc_params p, TableArgs a,
-                         TensorTableArgs t, SpecTableArgs sp, ComputeCostArgs c, int64_t spec_blocks,
-                         int64_t tensor_blocks) {
+void build_tables_kernel(APC_LAUNCH_PARAMS(BuildTablesBlock)) {
+  const BuildTablesBlock &k = launch_block(kept);
+  const apc_params &p = k.p;
+  const TableArgs &a = k.a;
+  const apc_tile *const tiles = static_cast<const apc_tile *>(work);
   unsigned char *const s_raw = build_tables_lds<M, kThreads, RM>();
   static_assert(kThreads == 64 || kThreads == 128 || kThreads == 256, "wavefronts per workgroup: 1, 2 or 4");
   const int64_t b = blockIdx.x;
@@ -1758,9 +1820,9 @@ void build_tables_kernel(const apc_tile *tiles, int n_tiles, int xcd_shift, int6
     return;
   }
   const int64_t tb = b - tile_blocks;
-  if (tb < spec_blocks) spec_tables_block<kThreads>(tb, p, sp, reinterpret_cast<int64_t *>(s_raw));
-  else if (tb < spec_blocks + tensor_blocks) tensor_tables_block<kThreads>(tb - spec_blocks, t);
-  else compute_costs_block<kThreads>(tb - spec_blocks - tensor_blocks, p, c);
+  if (tb < k.spec_blocks) spec_tables_block<kThreads>(tb, p, k.sp, reinterpret_cast<int64_t *>(s_raw));
+  else if (tb < k.spec_blocks + k.tensor_blocks) tensor_tables_block<kThreads>(tb - k.spec_blocks, k.t);
+  else compute_costs_block<kThreads>(tb - k.spec_blocks - k.tensor_blocks, p, k.c);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2099,22 +2161,28 @@ __device__ __forceinline__ void packed_tile(const apc_packed_tile *T, double *co
   }
 }
 
+struct PackedBlock {
+  PackedArgs a;
+  apc_params p;
+  TensorTableArgs t;
+  ComputeCostArgs c;
+  int64_t tensor_blocks;
+};
+
 template <int M, bool POW2>
-__global__ __launch_bounds__(kBlock) void build_tables_packed_kernel(const apc_packed_tile *tiles, int n_tiles, int xcd_shift,
-                                                                     int64_t tile_blocks, double *cost_out, PackedArgs a,
-                                                                     apc_params p, TensorTableArgs t, ComputeCostArgs c,
-                                                                     int64_t tensor_blocks) {
+__global__ __launch_bounds__(kBlock) void build_tables_packed_kernel(APC_LAUNCH_PARAMS(PackedBlock)) {
+  const PackedBlock &k = launch_block(kept);
   const int64_t b = blockIdx.x;
   if (b < tile_blocks) {
     const int64_t per = tile_blocks >> xcd_shift;
     const int64_t tile_id = (b & ((1 << xcd_shift) - 1)) * per + (b >> xcd_shift);
     if (tile_id >= n_tiles) return;
-    packed_tile<M, POW2>(tiles + tile_id, cost_out, a);
+    packed_tile<M, POW2>(static_cast<const apc_packed_tile *>(work) + tile_id, cost_out, k.a);
     return;
   }
   const int64_t tb = b - tile_blocks;
-  if (tb < tensor_blocks) tensor_tables_block<kBlock, true>(tb, t);
-  else compute_costs_block<kBlock, true>(tb - tensor_blocks, p, c);
+  if (tb < k.tensor_blocks) tensor_tables_block<kBlock, true>(tb, k.t);
+  else compute_costs_block<kBlock, true>(tb - k.tensor_blocks, k.p, k.c);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2955,41 +3023,55 @@ int apc_strategy_inputs(int64_t n_strategies, const int32_t *strat_node, int64_t
   return check_launch("apc_strategy_inputs");
 }
 
-int apc_input_tables(const apc_params *params, int64_t n_tensors, const int32_t *rank, const int32_t *itemsize,
-                     const int64_t *shape, const int64_t *stride, int64_t *tensor_bytes, uint8_t *tensor_contiguous,
-                     int64_t n_specs, const uint32_t *spec_codes, const int32_t *spec_tensor, int64_t *num_shards,
-                     int64_t *local_shape, int64_t *local_stride, int32_t shape_width, int64_t *local_numel,
-                     int64_t *local_bytes, int64_t n_strategies, const int64_t *flops, const int64_t *rw_bytes,
-                     const int8_t *dtype, const uint8_t *zero_cost, const int32_t *num_args, double *compute,
-                     double *per_arg, int32_t *error_flag, void *stream) {
-  if (int rc = check_params(params)) return rc;
-  if (n_tensors < 0 || n_specs < 0 || n_strategies < 0) return fail(-1, "apc_input_tables: negative count");
-  if (n_tensors > 0 && (!rank || !itemsize || !shape || !stride || !tensor_bytes || !tensor_contiguous))
-    return fail(-1, "apc_input_tables: NULL tensor array");
-  // the five spec-table outputs may all be NULL: the spec table is then skipped
-  const bool spec_table = num_shards || local_shape || local_stride || local_numel || local_bytes;
-  if (spec_table)
-    if (int rc = check_width(shape_width)) return rc;
-  if (spec_table && n_specs > 0 && (!spec_codes || !spec_tensor || !rank || !itemsize || !shape || !stride ||
-                                    !num_shards || !local_shape || !local_stride || !local_numel || !local_bytes))
-    return fail(-1, "apc_input_tables: the spec table needs all five of its outputs");
-  if (n_strategies > 0 && (!flops || !rw_bytes || !dtype || !zero_cost || !num_args))
-    return fail(-1, "apc_input_tables: NULL strategy array");
-  const int64_t sb = spec_table ? blocks_for(n_specs, kBlock) : 0, tb = blocks_for(n_tensors, kBlock),
-                cb = blocks_for(n_strategies, kBlock);
-  if (sb + tb + cb == 0) return 0;
-  if (sb + tb + cb > INT32_MAX) return fail(-1, "apc_input_tables: too many rows for one launch");
-  hipLaunchKernelGGL(input_tables_kernel, dim3((unsigned)(sb + tb + cb)), dim3(kBlock), 0, (hipStream_t)stream, *params,
-                     TensorTableArgs{n_tensors, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous},
-                     SpecTableArgs{n_specs, spec_codes, spec_tensor, rank, itemsize, shape, stride, num_shards,
-                                   local_shape, local_stride, local_numel, local_bytes, shape_width},
-                     ComputeCostArgs{n_strategies, flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg,
-                                     error_flag},
-                     sb, tb);
-  return check_launch("apc_input_tables");
+}  // extern "C"
+
+// Enqueues a table kernel, or (`to.keep`) records the launch for apc_run_kept.
+struct LaunchTo {
+  void *stream;
+  apc_kept_launch *keep;
+};
+
+// The launch that apc_keep_next_launch asked this thread to record (taken by the next table launch, whatever becomes of it).
+static thread_local apc_kept_launch *g_keep_next = nullptr;
+static LaunchTo launch_to(void *stream) {
+  const LaunchTo to{stream, g_keep_next};
+  g_keep_next = nullptr;
+  return to;
 }
 
-}  // extern "C"
+static int enqueue_kept(const apc_kept_launch &k, const void *block, void *stream) {
+  void *args[] = {const_cast<void **>(&k.work), const_cast<int32_t *>(&k.n_tiles), const_cast<int32_t *>(&k.xcd_shift),
+                  const_cast<int64_t *>(&k.tile_blocks), const_cast<double **>(&k.cost_out), &block, const_cast<int64_t *>(k.block)};
+  (void)hipLaunchKernel(k.kernel, dim3(k.grid), dim3(k.threads), args, k.lds_bytes, (hipStream_t)stream);
+  return check_launch(k.what);
+}
+
+template <typename Block>
+static int launch_table_kernel(const char *what, const LaunchTo &to, void (*kernel)(APC_LAUNCH_PARAMS(Block)), unsigned grid, int threads,
+                               size_t lds, const void *work, int n_tiles, int xcd_shift, int64_t tile_blocks, double *cost_out,
+                               const Block &block) {
+  static_assert(sizeof(Block) <= APC_KEPT_BLOCK_BYTES, "the arguments fit a kept launch");
+  static_assert(std::is_trivially_copyable<Block>::value, "the arguments travel as bytes");
+  if (!to.keep) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, (hipStream_t)to.stream, work, n_tiles, xcd_shift, tile_blocks, cost_out,
+                       (const Block *)nullptr, block);
+    return check_launch(what);
+  }
+  apc_kept_launch &k = *to.keep;
+  k.kernel = reinterpret_cast<const void *>(kernel);
+  k.what = what;
+  k.grid = grid;
+  k.threads = (uint32_t)threads;
+  k.lds_bytes = (uint32_t)lds;
+  k.block_bytes = (uint32_t)sizeof(Block);
+  k.work = const_cast<void *>(work);
+  k.n_tiles = n_tiles;
+  k.xcd_shift = xcd_shift;
+  k.tile_blocks = tile_blocks;
+  k.cost_out = cost_out;
+  std::memcpy(k.block, &block, sizeof(Block));
+  return 0;
+}
 
 // Row minima need their index arrays and, when some tile serves identical edges, those edges' rows.
 static int check_row_minima(const apc_row_minima *rows, const int64_t *dup_entry_begin, const char *who) {
@@ -3035,12 +3117,46 @@ static int tile_threads(int64_t n_tiles, int64_t n_entries, bool many_states, in
   return threads >= 256 ? 256 : threads >= 128 ? 128 : 64;
 }
 
+static int input_tables_impl(const apc_params *params, int64_t n_tensors, const int32_t *rank, const int32_t *itemsize,
+                     const int64_t *shape, const int64_t *stride, int64_t *tensor_bytes, uint8_t *tensor_contiguous,
+                     int64_t n_specs, const uint32_t *spec_codes, const int32_t *spec_tensor, int64_t *num_shards,
+                     int64_t *local_shape, int64_t *local_stride, int32_t shape_width, int64_t *local_numel,
+                     int64_t *local_bytes, int64_t n_strategies, const int64_t *flops, const int64_t *rw_bytes,
+                     const int8_t *dtype, const uint8_t *zero_cost, const int32_t *num_args, double *compute,
+                     double *per_arg, int32_t *error_flag, const LaunchTo &to) {
+  if (int rc = check_params(params)) return rc;
+  if (n_tensors < 0 || n_specs < 0 || n_strategies < 0) return fail(-1, "apc_input_tables: negative count");
+  if (n_tensors > 0 && (!rank || !itemsize || !shape || !stride || !tensor_bytes || !tensor_contiguous))
+    return fail(-1, "apc_input_tables: NULL tensor array");
+  // the five spec-table outputs may all be NULL: the spec table is then skipped
+  const bool spec_table = num_shards || local_shape || local_stride || local_numel || local_bytes;
+  if (spec_table)
+    if (int rc = check_width(shape_width)) return rc;
+  if (spec_table && n_specs > 0 && (!spec_codes || !spec_tensor || !rank || !itemsize || !shape || !stride ||
+                                    !num_shards || !local_shape || !local_stride || !local_numel || !local_bytes))
+    return fail(-1, "apc_input_tables: the spec table needs all five of its outputs");
+  if (n_strategies > 0 && (!flops || !rw_bytes || !dtype || !zero_cost || !num_args))
+    return fail(-1, "apc_input_tables: NULL strategy array");
+  const int64_t sb = spec_table ? blocks_for(n_specs, kBlock) : 0, tb = blocks_for(n_tensors, kBlock),
+                cb = blocks_for(n_strategies, kBlock);
+  if (sb + tb + cb == 0) return 0;
+  if (sb + tb + cb > INT32_MAX) return fail(-1, "apc_input_tables: too many rows for one launch");
+  const InputTablesBlock block{*params,
+                               {n_tensors, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous},
+                               {n_specs, spec_codes, spec_tensor, rank, itemsize, shape, stride, num_shards, local_shape, local_stride,
+                                local_numel, local_bytes, shape_width},
+                               {n_strategies, flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag},
+                               sb,
+                               tb};
+  return launch_table_kernel("apc_input_tables", to, input_tables_kernel, (unsigned)(sb + tb + cb), kBlock, 0, nullptr, 0, 0, 0, nullptr, block);
+}
+
 static int redistribute_tables_impl(const apc_params *params, const int64_t *tensor_bytes,
                                     const uint8_t *tensor_contiguous, const uint32_t *spec_codes,
                                     const int32_t *spec_tensor, const double *pt_values, const double *per_arg,
                                     int64_t n_tiles, const apc_tile *tiles, const int64_t *dup_entry_begin,
                                     int64_t n_entries, double *comm_out, uint8_t *trans_out, double *cost_out,
-                                    const apc_row_minima *rows, void *stream) {
+                                    const apc_row_minima *rows, const LaunchTo &to) {
   if (int rc = check_params(params)) return rc;
   if (n_tiles < 0 || n_tiles > (1 << 30)) return fail(-1, "n_tiles %lld out of range", (long long)n_tiles);
   if (n_tiles == 0) return 0;
@@ -3055,16 +3171,15 @@ static int redistribute_tables_impl(const apc_params *params, const int64_t *ten
               rows ? rows->edge_row_begin : nullptr, rows ? rows->dup_row_begin : nullptr,
               rows ? rows->row_min : nullptr, rows ? rows->row_argmin : nullptr, term_layout(*params)};
   const int nt = (int)n_tiles, xs = xcd_shift();
-  hipStream_t s = (hipStream_t)stream;
-  const dim3 grid((unsigned)(((n_tiles + (1 << xs) - 1) >> xs) << xs));  // rounded up for xcd_chunked_unit
+  const int64_t grid = ((n_tiles + (1 << xs) - 1) >> xs) << xs;  // rounded up for xcd_chunked_unit
+  const char *const what = rows ? "apc_redistribute_tables_row_min" : "apc_redistribute_tables";
   const int threads = tile_threads(n_tiles, n_entries, params->mesh_ndim == 4 && a.lay.exponents == 0, 512, 2048);
   const int om = out_mode(params->mesh_ndim, comm_out, trans_out, cost_out);
 #define APC_LAUNCH_T(KERNEL_, M_, OUT_)                                                                               \
   const int wg = threads >= 256 ? 256 : threads >= 128 ? 128 : 64;                                                     \
   const size_t lds = rows ? stage_lds_bytes<M_, true>(a.lay, wg) : stage_lds_bytes<M_, false>(a.lay, wg);              \
-  if (threads >= 256) hipLaunchKernelGGL((KERNEL_<M_, 256, OUT_>), grid, dim3(256), lds, s, a.tiles, nt, xs, *params, a);      \
-  else if (threads >= 128) hipLaunchKernelGGL((KERNEL_<M_, 128, OUT_>), grid, dim3(128), lds, s, a.tiles, nt, xs, *params, a); \
-  else hipLaunchKernelGGL((KERNEL_<M_, 64, OUT_>), grid, dim3(64), lds, s, a.tiles, nt, xs, *params, a)
+  const auto kernel = wg == 256 ? KERNEL_<M_, 256, OUT_> : wg == 128 ? KERNEL_<M_, 128, OUT_> : KERNEL_<M_, 64, OUT_>; \
+  return launch_table_kernel(what, to, kernel, (unsigned)grid, wg, lds, tiles, nt, xs, grid, cost_out, TilesBlock{*params, a})
 #define APC_LAUNCH_K(KERNEL_, M_)                                   \
   if (om == kOutAll) { APC_LAUNCH_T(KERNEL_, M_, kOutAll); }        \
   else if (om == kOutCost) { APC_LAUNCH_T(KERNEL_, M_, kOutCost); } \
@@ -3088,7 +3203,6 @@ static int redistribute_tables_impl(const apc_params *params, const int64_t *ten
 #undef APC_LAUNCH_T
 #undef APC_LAUNCH_K
 #undef APC_LAUNCH_ANY
-  return check_launch("apc_redistribute_tables");
 }
 
 static int build_tables_impl(const apc_params *params, int64_t n_tensors, const int32_t *rank, const int32_t *itemsize,
@@ -3099,7 +3213,7 @@ static int build_tables_impl(const apc_params *params, int64_t n_tensors, const 
                      const int8_t *dtype, const uint8_t *zero_cost, const int32_t *num_args, double *compute,
                      double *per_arg, int32_t *error_flag, const double *pt_values, int64_t n_tiles, const apc_tile *tiles,
                      const int64_t *dup_entry_begin, int64_t n_entries, double *comm_out, uint8_t *trans_out,
-                     double *cost_out, const apc_row_minima *rows, void *stream) {
+                     double *cost_out, const apc_row_minima *rows, const LaunchTo &to) {
   if (int rc = check_params(params)) return rc;
   if (n_tiles > 0)
     if (int rc = check_row_minima(rows, dup_entry_begin, "apc_build_tables_row_min")) return rc;
@@ -3138,15 +3252,15 @@ static int build_tables_impl(const apc_params *params, int64_t n_tensors, const 
   const SpecTableArgs sa{n_specs, spec_codes, spec_tensor, rank, itemsize, shape, stride, num_shards,
                          local_shape, local_stride, local_numel, local_bytes, shape_width};
   const ComputeCostArgs ca{n_strategies, flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag};
-  hipStream_t s = (hipStream_t)stream;
-  const dim3 grid((unsigned)blocks);
+  const char *const what = rows ? "apc_build_tables_row_min" : "apc_build_tables";
   const int nt = (int)n_tiles;
   const int om = out_mode(params->mesh_ndim, comm_out, trans_out, cost_out);
 #define APC_LAUNCH_ALL_T(M_, RM_, OUT_)                                                                                 \
   const size_t lds = build_tables_lds_bytes<M_, RM_>(a.lay, threads, spec_table);                                      \
-  if (threads == 256) hipLaunchKernelGGL((build_tables_kernel<M_, 256, RM_, OUT_>), grid, dim3(256), lds, s, a.tiles, nt, xs, tile_blocks, *params, a, ta, sa, ca, sb, tb); \
-  else if (threads == 128) hipLaunchKernelGGL((build_tables_kernel<M_, 128, RM_, OUT_>), grid, dim3(128), lds, s, a.tiles, nt, xs, tile_blocks, *params, a, ta, sa, ca, sb, tb); \
-  else hipLaunchKernelGGL((build_tables_kernel<M_, 64, RM_, OUT_>), grid, dim3(64), lds, s, a.tiles, nt, xs, tile_blocks, *params, a, ta, sa, ca, sb, tb)
+  const auto kernel = threads == 256 ? build_tables_kernel<M_, 256, RM_, OUT_>                                         \
+                      : threads == 128 ? build_tables_kernel<M_, 128, RM_, OUT_> : build_tables_kernel<M_, 64, RM_, OUT_>; \
+  return launch_table_kernel(what, to, kernel, (unsigned)blocks, threads, lds, tiles, nt, xs, tile_blocks, cost_out,  \
+                             BuildTablesBlock{*params, a, ta, sa, ca, sb, tb})
 #define APC_LAUNCH_ALL_RM(M_, RM_)                                   \
   if (om == kOutAll) { APC_LAUNCH_ALL_T(M_, RM_, kOutAll); }         \
   else if (om == kOutCost) { APC_LAUNCH_ALL_T(M_, RM_, kOutCost); }  \
@@ -3165,10 +3279,35 @@ static int build_tables_impl(const apc_params *params, int64_t n_tensors, const 
 #undef APC_LAUNCH_ALL_RM
 #undef APC_LAUNCH_ALL
 #undef APC_LAUNCH_ALL_ANY
-  return check_launch("apc_build_tables");
 }
 
 extern "C" {
+
+int apc_keep_next_launch(apc_kept_launch *out) {
+  if (!out) return fail(-1, "apc_keep_next_launch: NULL");
+  out->kernel = nullptr;
+  g_keep_next = out;
+  return 0;
+}
+
+int apc_run_kept(const apc_kept_launch *kept, const void *device_block, void *stream) {
+  if (!kept) return fail(-1, "apc_run_kept: NULL");
+  if (!kept->kernel) return 0;  // (nothing to launch)
+  if ((reinterpret_cast<uintptr_t>(device_block) & 63) != 0) return fail(-1, "apc_run_kept: the block must be 64-byte aligned");
+  return enqueue_kept(*kept, device_block, stream);
+}
+
+int apc_input_tables(const apc_params *params, int64_t n_tensors, const int32_t *rank, const int32_t *itemsize,
+                     const int64_t *shape, const int64_t *stride, int64_t *tensor_bytes, uint8_t *tensor_contiguous,
+                     int64_t n_specs, const uint32_t *spec_codes, const int32_t *spec_tensor, int64_t *num_shards,
+                     int64_t *local_shape, int64_t *local_stride, int32_t shape_width, int64_t *local_numel,
+                     int64_t *local_bytes, int64_t n_strategies, const int64_t *flops, const int64_t *rw_bytes,
+                     const int8_t *dtype, const uint8_t *zero_cost, const int32_t *num_args, double *compute,
+                     double *per_arg, int32_t *error_flag, void *stream) {
+  return input_tables_impl(params, n_tensors, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous, n_specs, spec_codes,
+                           spec_tensor, num_shards, local_shape, local_stride, shape_width, local_numel, local_bytes, n_strategies,
+                           flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag, launch_to(stream));
+}
 
 int apc_redistribute_tables(const apc_params *params, const int64_t *tensor_bytes, const uint8_t *tensor_contiguous,
                             const uint32_t *spec_codes, const int32_t *spec_tensor, const double *pt_values,
@@ -3177,7 +3316,7 @@ int apc_redistribute_tables(const apc_params *params, const int64_t *tensor_byte
                             double *cost_out, void *stream) {
   return redistribute_tables_impl(params, tensor_bytes, tensor_contiguous, spec_codes, spec_tensor, pt_values, per_arg,
                                   n_tiles, tiles, dup_entry_begin, n_entries, comm_out, trans_out, cost_out, nullptr,
-                                  stream);
+                                  launch_to(stream));
 }
 
 int apc_redistribute_tables_row_min(const apc_params *params, const int64_t *tensor_bytes,
@@ -3186,9 +3325,10 @@ int apc_redistribute_tables_row_min(const apc_params *params, const int64_t *ten
                                     int64_t n_tiles, const apc_tile *tiles, const int64_t *dup_entry_begin,
                                     int64_t n_entries, double *comm_out, uint8_t *trans_out, double *cost_out,
                                     const apc_row_minima *rows, void *stream) {
+  const LaunchTo to = launch_to(stream);
   if (!rows) return fail(-1, "apc_redistribute_tables_row_min: NULL rows");
   return redistribute_tables_impl(params, tensor_bytes, tensor_contiguous, spec_codes, spec_tensor, pt_values, per_arg,
-                                  n_tiles, tiles, dup_entry_begin, n_entries, comm_out, trans_out, cost_out, rows, stream);
+                                  n_tiles, tiles, dup_entry_begin, n_entries, comm_out, trans_out, cost_out, rows, to);
 }
 
 #define APC_BUILD_TABLES_PARAMS                                                                                         \
@@ -3207,12 +3347,13 @@ int apc_redistribute_tables_row_min(const apc_params *params, const int64_t *ten
       comm_out, trans_out, cost_out
 
 int apc_build_tables(APC_BUILD_TABLES_PARAMS, void *stream) {
-  return build_tables_impl(APC_BUILD_TABLES_ARGS, nullptr, stream);
+  return build_tables_impl(APC_BUILD_TABLES_ARGS, nullptr, launch_to(stream));
 }
 
 int apc_build_tables_row_min(APC_BUILD_TABLES_PARAMS, const apc_row_minima *rows, void *stream) {
+  const LaunchTo to = launch_to(stream);
   if (!rows) return fail(-1, "apc_build_tables_row_min: NULL rows");
-  return build_tables_impl(APC_BUILD_TABLES_ARGS, rows, stream);
+  return build_tables_impl(APC_BUILD_TABLES_ARGS, rows, to);
 }
 #undef APC_BUILD_TABLES_PARAMS
 #undef APC_BUILD_TABLES_ARGS
@@ -3412,12 +3553,13 @@ int apc_redistribute_tables_static(const apc_params *params, int64_t n_tensors, 
   // staging tables into the static array (no spec table, no per-strategy compute cost, no error
   // flag: a strategy with flops and an unsupported dtype shows as NaN costs), then the tiles;
   // both launches on the caller's stream, so the second sees what the first wrote
-  if (int rc = apc_input_tables(params, n_tensors, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous, 0, nullptr,
-                                nullptr, nullptr, nullptr, nullptr, 2, nullptr, nullptr, n_strategies, flops, rw_bytes, dtype,
-                                zero_cost, num_args, nullptr, per_arg, nullptr, stream))
+  const LaunchTo now{stream, nullptr};
+  if (int rc = input_tables_impl(params, n_tensors, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous, 0, nullptr,
+                                 nullptr, nullptr, nullptr, nullptr, 2, nullptr, nullptr, n_strategies, flops, rw_bytes, dtype,
+                                 zero_cost, num_args, nullptr, per_arg, nullptr, now))
     return rc;
   return redistribute_tables_impl(params, tensor_bytes, tensor_contiguous, spec_codes, spec_tensor, pt_values, per_arg, n_tiles,
-                                  tiles, dup_entry_begin, n_entries, comm_out, trans_out, cost_out, nullptr, stream);
+                                  tiles, dup_entry_begin, n_entries, comm_out, trans_out, cost_out, nullptr, now);
 }
 
 }  // extern "C"
@@ -3429,14 +3571,13 @@ static_assert(sizeof(apc_packed_tile) == 2752 && sizeof(apc_packed_tile) % 64 ==
 static_assert(offsetof(apc_packed_tile, entry_begin) == 32 && offsetof(apc_packed_tile, tensor_shape) == 64,
               "the header is the record's first 64 bytes");
 
-extern "C" {
-
-int apc_build_tables_packed(const apc_params *params, int64_t n_tensors, const int32_t *rank, const int32_t *itemsize,
+static int build_tables_packed_impl(const apc_params *params, int64_t n_tensors, const int32_t *rank, const int32_t *itemsize,
                             const int64_t *shape, const int64_t *stride, int64_t *tensor_bytes, uint8_t *tensor_contiguous,
                             int64_t n_strategies, const int64_t *flops, const int64_t *rw_bytes, const int8_t *dtype,
                             const uint8_t *zero_cost, const int32_t *num_args, double *compute, double *per_arg,
                             int32_t *error_flag, const double *pt_values, int64_t n_tiles, const apc_packed_tile *packed,
-                            int64_t n_entries, double *cost_out, double *row_min, int32_t *row_argmin, void *stream) {
+                            int64_t n_entries, double *cost_out, double *row_min, int32_t *row_argmin,
+                                    const LaunchTo &to) {
   if (int rc = check_params(params)) return rc;
   if (n_tensors < 0 || n_strategies < 0 || n_entries < 0) return fail(-1, "apc_build_tables_packed: negative count");
   if (n_tiles < 0 || n_tiles > (1 << 30)) return fail(-1, "n_tiles %lld out of range", (long long)n_tiles);
@@ -3459,24 +3600,31 @@ int apc_build_tables_packed(const apc_params *params, int64_t n_tensors, const i
   for (int i = 0; i < APC_MAX_MESH; ++i) a.lg[i] = lay.lg[i];
   const TensorTableArgs ta{n_tensors, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous};
   const ComputeCostArgs ca{n_strategies, flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag};
-  hipStream_t s = (hipStream_t)stream;
-  const dim3 grid((unsigned)blocks);
-  const int nt = (int)n_tiles;
-#define APC_LAUNCH_PACKED(M_)                                                                                                    \
-  if (lay.exponents)                                                                                                           \
-    hipLaunchKernelGGL((build_tables_packed_kernel<M_, true>), grid, dim3(kBlock), 0, s, packed, nt, xs, tile_blocks, cost_out, a, \
-                       *params, ta, ca, tb);                                                                                   \
-  else                                                                                                                         \
-    hipLaunchKernelGGL((build_tables_packed_kernel<M_, false>), grid, dim3(kBlock), 0, s, packed, nt, xs, tile_blocks, cost_out, a, \
-                       *params, ta, ca, tb)
+  const PackedBlock block{a, *params, ta, ca, tb};
+#define APC_LAUNCH_PACKED(M_)                                                                                             \
+  return launch_table_kernel("apc_build_tables_packed", to,                                                             \
+                             lay.exponents ? build_tables_packed_kernel<M_, true> : build_tables_packed_kernel<M_, false>, \
+                             (unsigned)blocks, kBlock, 0, packed, (int)n_tiles, xs, tile_blocks, cost_out, block)
   switch (params->mesh_ndim) {
-    case 1: APC_LAUNCH_PACKED(1); break;
-    case 2: APC_LAUNCH_PACKED(2); break;
-    case 3: APC_LAUNCH_PACKED(3); break;
-    default: APC_LAUNCH_PACKED(4); break;
+    case 1: APC_LAUNCH_PACKED(1);
+    case 2: APC_LAUNCH_PACKED(2);
+    case 3: APC_LAUNCH_PACKED(3);
+    default: APC_LAUNCH_PACKED(4);
   }
 #undef APC_LAUNCH_PACKED
-  return check_launch("apc_build_tables_packed");
+}
+
+extern "C" {
+
+int apc_build_tables_packed(const apc_params *params, int64_t n_tensors, const int32_t *rank, const int32_t *itemsize,
+                            const int64_t *shape, const int64_t *stride, int64_t *tensor_bytes, uint8_t *tensor_contiguous,
+                            int64_t n_strategies, const int64_t *flops, const int64_t *rw_bytes, const int8_t *dtype,
+                            const uint8_t *zero_cost, const int32_t *num_args, double *compute, double *per_arg,
+                            int32_t *error_flag, const double *pt_values, int64_t n_tiles, const apc_packed_tile *packed,
+                            int64_t n_entries, double *cost_out, double *row_min, int32_t *row_argmin, void *stream) {
+  return build_tables_packed_impl(params, n_tensors, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous, n_strategies,
+                                  flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag, pt_values, n_tiles, packed,
+                                  n_entries, cost_out, row_min, row_argmin, launch_to(stream));
 }
 
 }  // extern "C"

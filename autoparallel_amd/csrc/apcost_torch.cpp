@@ -31,6 +31,7 @@
 #include <cstring>
 #include <exception>
 #include <functional>
+#include <memory>
 #include <optional>
 #include <string>
 #include <tuple>
@@ -387,15 +388,32 @@ struct BoundLaunch : torch::CustomClassHolder {
   at::Device device{at::kCPU};
   std::function<int(void *)> launch;
   std::vector<Tensor> keep;  // every tensor whose memory the launch reads or writes
+  bool recordable = false;   // apc_keep_next_launch knows it
+  std::unique_ptr<apc_kept_launch> kept;
+  Tensor block;  // the kept launch's arguments on the device
 
+  // For a launch that will run again and again: its arguments go to device memory now (apc_kept_launch).
+  // Called by whoever bound the launch, before anyone runs it.
+  void keep_arguments() {
+    if (!recordable || kept) return;
+    auto k = std::make_unique<apc_kept_launch>();
+    check_rc(apc_keep_next_launch(k.get()), what.c_str());
+    check_rc(launch(nullptr), what.c_str());
+    if (k->kernel)
+      block = upload({at::from_blob(k->block, {(int64_t)k->block_bytes}, at::TensorOptions().dtype(at::kByte))}, device)[0];
+    kept = std::move(k);
+  }
+  void enqueue(void *stream) {
+    check_rc(kept ? apc_run_kept(kept.get(), block.defined() ? block.data_ptr() : nullptr, stream) : launch(stream), what.c_str());
+  }
   void run() {
     c10::hip::HIPGuard guard(device.index());
-    check_rc(launch(c10::hip::getCurrentHIPStream(device.index()).stream()), what.c_str());
+    enqueue(c10::hip::getCurrentHIPStream(device.index()).stream());
   }
   // The launch on a stream given by its handle (torch.cuda.Stream.cuda_stream).
   void run_on(int64_t stream) {
     c10::hip::HIPGuard guard(device.index());
-    check_rc(launch(reinterpret_cast<void *>(stream)), what.c_str());
+    enqueue(reinterpret_cast<void *>(stream));
   }
   std::string name() const { return what; }
 };
@@ -475,6 +493,7 @@ c10::intrusive_ptr<BoundLaunch> bind_redistribute_tables(
   const Outputs o = outputs_of(n_entries, comm, transition, cost, edge_row_begin, dup_row_begin, row_min, row_argmin, b->keep);
   TORCH_CHECK(comm.has_value() || transition.has_value() || cost.has_value(), "apcost: no per-entry output given");
   b->what = o.rows ? "apc_redistribute_tables_row_min" : "apc_redistribute_tables";
+  b->recordable = true;
   b->device = tensor_bytes.device();
   b->launch = [=](void *s) {
     if (o.rows)
@@ -561,6 +580,7 @@ c10::intrusive_ptr<BoundLaunch> bind_input_tables(APCOST_INPUT_TABLE_PARAMS) {
   auto b = c10::make_intrusive<BoundLaunch>();
   const InputTables in = input_tables_of(APCOST_INPUT_TABLE_ARGS, b->keep);
   b->what = "apc_input_tables";
+  b->recordable = true;
   b->device = rank.device();
   b->launch = [=](void *s) {
     return apc_input_tables(&in.p, in.t.n, in.t.rank, in.t.itemsize, in.t.shape, in.t.stride, in.tensor_bytes, in.tensor_contiguous,
@@ -589,6 +609,7 @@ c10::intrusive_ptr<BoundLaunch> bind_cost_tables(APCOST_INPUT_TABLE_PARAMS, cons
   }
   const Outputs o = outputs_of(n_entries, comm, transition, cost, edge_row_begin, dup_row_begin, row_min, row_argmin, b->keep);
   b->what = o.rows ? "apc_build_tables_row_min" : "apc_build_tables";
+  b->recordable = true;
   b->device = rank.device();
   b->launch = [=](void *s) {
 #define APCOST_BUILD_ARGS                                                                                                  \
@@ -640,6 +661,7 @@ c10::intrusive_ptr<BoundLaunch> bind_cost_tables_packed(const Tensor &params, co
     b->keep.push_back(*x);
   }
   b->what = "apc_build_tables_packed";
+  b->recordable = true;
   b->device = rank.device();
   b->launch = [=](void *s) {
     return apc_build_tables_packed(&p, t.n, t.rank, t.itemsize, t.shape, t.stride, bytes, contiguous, st.n, st.flops, st.rw_bytes,
@@ -917,7 +939,8 @@ int64_t library_abi_version() { return apc_version(); }
 }  // namespace
 
 TORCH_LIBRARY(apcost, m) {
-  m.class_<BoundLaunch>("BoundLaunch").def("run", &BoundLaunch::run).def("run_on", &BoundLaunch::run_on).def("name", &BoundLaunch::name);
+  m.class_<BoundLaunch>("BoundLaunch").def("run", &BoundLaunch::run).def("keep_arguments", &BoundLaunch::keep_arguments)
+      .def("run_on", &BoundLaunch::run_on).def("name", &BoundLaunch::name);
 #define APCOST_TENSOR_TABLE "Tensor tensor_rank, Tensor tensor_itemsize, Tensor tensor_shape, Tensor tensor_stride"
 #define APCOST_STRATEGY_TABLE "Tensor flops, Tensor rw_bytes, Tensor dtype_code, Tensor zero_cost, Tensor num_args"
 #define APCOST_INPUT_TABLES                                                                                          \

@@ -307,7 +307,7 @@ class DeviceCostTables:
 
     @_guarded
     def prepare_step(self, row_min=True, fused_inputs=False, one_launch=None, row_min_in_tiles=None,
-                     outputs=("comm", "transition", "cost"), spec_table=True, packed=None):
+                     outputs=("comm", "transition", "cost"), spec_table=True, packed=None, repeated=True):
         """Allocates every output once and returns ``{kernel name: zero-argument launcher}``
         in launch order.  A launcher only enqueues (no allocation, no synchronisation), so a
         timed loop measures the kernels and not Python argument marshalling.  With
@@ -323,7 +323,8 @@ class DeviceCostTables:
         flop / byte counts this pass reads).  ``packed``: the one launch runs over packed tiles
         (``apc_build_tables_packed``: the assembled cost and the row minima, no spec table);
         ``None`` takes them when the pass is of that kind, ``packed_pass_pays`` and staged tiles
-        (``CostTables.staging_pays``) are not faster still."""
+        (``CostTables.staging_pays``) are not faster still.  ``repeated=False``: the pass will run once, and the arguments
+        of its launches are not laid out in device memory first (``apc_kept_launch``: one copy, for 2 to 4 us less a launch)."""
         tb = self.tables
         outputs = tuple(outputs)
         if not outputs or any(o not in ("comm", "transition", "cost") for o in outputs):
@@ -362,6 +363,8 @@ class DeviceCostTables:
 
         def bind(bound):
             # a launcher only looks up the current stream (or takes the given one) and enqueues
+            if repeated:
+                bound.keep_arguments()
             run, run_on = bound.run, bound.run_on
 
             def launch(on_stream=None):
@@ -419,7 +422,7 @@ class DeviceCostTables:
     # ---- the planner's table build -------------------------------------------------------------
     PLANNER_OUTPUTS = ("cost",)
 
-    def planner_pass(self, packed=None):
+    def planner_pass(self, packed=None, repeated=True):
         """The launches ``ShardingOptimizer.build_ds`` issues once the flop / byte counts are in
         the strategy table (optimize_sharding.py:270-380 in one pass): the tensor and
         compute-cost tables and the assembled cost of every entry, the array the ILP objective
@@ -430,7 +433,7 @@ class DeviceCostTables:
         shapes before it could count flops); ``comm`` and ``transition`` are written only when a
         report asks (``fetch``)."""
         return self.prepare_step(row_min=self.row_min_in_tiles_pays(), fused_inputs=True,
-                                 outputs=self.PLANNER_OUTPUTS, spec_table=False, packed=packed)
+                                 outputs=self.PLANNER_OUTPUTS, spec_table=False, packed=packed, repeated=repeated)
 
     @_guarded
     def check_error_flag(self):

@@ -120,7 +120,7 @@ class DeviceBackend:
     def launch_tables(self):
         """Enqueues the planner's table pass (``DeviceCostTables.planner_pass``) and returns."""
         d = self.dev
-        step = d.planner_pass()
+        step = d.planner_pass(repeated=False)
         self.launches = tuple(step)
         self._events = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
         with torch.cuda.device(d.device):

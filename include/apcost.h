@@ -572,6 +572,31 @@ int apc_build_tables_packed(const apc_params *params, int64_t n_tensors, const i
                             int32_t *error_flag, const double *pt_values, int64_t n_tiles, const apc_packed_tile *packed,
                             int64_t n_entries, double *cost_out, double *row_min, int32_t *row_argmin, void *stream);
 
+/* A launch that is kept for repeating (a plan's pass).  A launch passes its arguments by value in a segment that the
+ * host has just written, which every compute unit reads past the caches; a kept launch has them in device memory.
+ *   apc_keep_next_launch(&k);              the next apc_input_tables, apc_redistribute_tables[_row_min],
+ *   apc_build_tables...(args, NULL);       apc_build_tables[_row_min] or apc_build_tables_packed of this thread checks
+ *                                          its arguments and is recorded in k instead of being enqueued; k.kernel stays
+ *                                          NULL when it fails or has nothing to launch
+ *   copy k.block (k.block_bytes) to device memory, 64-byte aligned
+ *   apc_run_kept(&k, device_block, stream) enqueues it, as often as wanted, from any thread (NULL device_block: by
+ *                                          value).  k, the block and every array the launch names stay as they are
+ *                                          while it runs.
+ * No counterpart in the reference. */
+#define APC_KEPT_BLOCK_BYTES 3072
+typedef struct apc_kept_launch {
+  const void *kernel;
+  const char *what; /* the entry point that recorded it */
+  uint32_t grid, threads, lds_bytes, block_bytes;
+  void *work;
+  int32_t n_tiles, xcd_shift;
+  int64_t tile_blocks;
+  double *cost_out;
+  int64_t block[APC_KEPT_BLOCK_BYTES / 8];
+} apc_kept_launch;
+int apc_keep_next_launch(apc_kept_launch *out);
+int apc_run_kept(const apc_kept_launch *kept, const void *device_block, void *stream);
+
 /* Measurement aids, no counterpart in the reference.  apc_calibrate_launch enqueues a kernel that
  * does nothing (n_workgroups workgroups of `threads` threads): launched back to back it shows what
  * a launch costs on the system before any work.  apc_calibrate_fill enqueues a kernel that only

@@ -1,0 +1,94 @@
+"""Launches whose arguments are kept in device memory (``apc_keep_next_launch`` / ``apc_run_kept``, ``BoundLaunch.keep_arguments``)
+against the same launches with their arguments passed by value."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from autoparallel_amd import CostModelParams, _native
+from autoparallel_amd.device_tables import DeviceCostTables
+from autoparallel_amd.synthetic import stress_dag
+
+
+class _Kept(ctypes.Structure):  # include/apcost.h: apc_kept_launch
+    _fields_ = [("kernel", ctypes.c_void_p), ("what", ctypes.c_char_p), ("grid", ctypes.c_uint32), ("threads", ctypes.c_uint32),
+                ("lds_bytes", ctypes.c_uint32), ("block_bytes", ctypes.c_uint32), ("work", ctypes.c_void_p),
+                ("n_tiles", ctypes.c_int32), ("xcd_shift", ctypes.c_int32), ("tile_blocks", ctypes.c_int64),
+                ("cost_out", ctypes.c_void_p), ("block", ctypes.c_int64 * 384)]
+
+
+def _redistribute(lib, params, n_tiles, per_arg):
+    one = ctypes.c_void_p(8)  # (a placeholder that is never read: a recorded call launches nothing)
+    return lib.apc_redistribute_tables(ctypes.byref(params), one, one, one, one, None, per_arg, ctypes.c_int64(n_tiles), one, None,
+                                       ctypes.c_int64(1), None, None, one, None)
+
+
+def test_recording_a_launch_checks_it_and_ends_with_it():
+    """The call after ``apc_keep_next_launch`` is checked as ever; a refused or an empty one leaves nothing to run, and the
+    recording ends with that call either way."""
+    lib = _native.lib()
+    params = CostModelParams.from_mesh((4, 2)).to_c()
+    assert lib.apc_keep_next_launch(None) != 0
+    kept = _Kept()
+    one = ctypes.c_void_p(8)
+    assert lib.apc_keep_next_launch(ctypes.byref(kept)) == 0
+    assert _redistribute(lib, params, 3, None) != 0 and b"compute_cost_per_arg" in lib.apc_last_error()  # refused
+    assert kept.kernel is None
+    assert lib.apc_run_kept(ctypes.byref(kept), None, None) == 0  # nothing to launch
+    assert _redistribute(lib, params, 0, one) == 0 and kept.kernel is None  # (not recorded: the recording has ended)
+    assert lib.apc_keep_next_launch(ctypes.byref(kept)) == 0
+    assert _redistribute(lib, params, 0, one) == 0 and kept.kernel is None  # no tiles
+    assert lib.apc_keep_next_launch(ctypes.byref(kept)) == 0
+    assert _redistribute(lib, params, 3, one) == 0
+    assert kept.kernel and kept.what == b"apc_redistribute_tables" and kept.n_tiles == 3 and kept.grid == 8
+    assert 0 < kept.block_bytes <= ctypes.sizeof(kept) - _Kept.block.offset
+    assert lib.apc_run_kept(ctypes.byref(kept), ctypes.c_void_p(8), None) != 0  # the block's alignment
+    assert b"64-byte" in lib.apc_last_error()
+
+
+def _outputs(d):
+    torch.cuda.synchronize()
+    arrays = (d.comm, d.transition, d.cost, d.tensor_bytes, d.tensor_contiguous, d.compute_cost, d.compute_cost_per_arg, d.row_min,
+              d.row_argmin)
+    return [None if t is None else t.cpu().numpy().copy() for t in arrays]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mesh", [(6,), (32, 8), (12, 6), (16, 8, 4), (2, 3, 2, 2)])
+def test_kept_launches_write_what_launches_by_value_write(gpu_device, mesh):
+    """Every form of the pass, from the current stream, from another one and from a captured graph (replayed with eager work
+    between the replays)."""
+    tb = stress_dag(seed=9, n_nodes=250, mesh_sizes=mesh, max_strategies=30, frac_nonspec_nodes=0.05, frac_noncontiguous=0.2)
+    p = CostModelParams.from_mesh(mesh, rescale=2.2)
+    all_three = ("comm", "transition", "cost")
+    forms = [dict(outputs=("cost",), spec_table=False, packed=True), dict(outputs=("cost",), spec_table=False, one_launch=True, packed=False),
+             dict(outputs=all_three, one_launch=True), dict(outputs=all_three, one_launch=False),
+             dict(outputs=("cost",), spec_table=False, one_launch=False, row_min_in_tiles=False)]
+    for form in forms:
+        want = None
+        for repeated in (False, True):
+            d = DeviceCostTables(tb, p, device=gpu_device)
+            step = d.prepare_step(**dict(dict(row_min=True, fused_inputs=True, row_min_in_tiles=True), **form), repeated=repeated)
+            for launch in step.values():
+                launch()
+            got = _outputs(d)
+            if want is None:
+                want = got
+                continue
+            assert all((g is None) == (w is None) and (g is None or np.array_equal(g, w)) for g, w in zip(got, want)), form
+            side = torch.cuda.Stream(device=d.device)
+            d.cost.zero_()
+            side.wait_stream(torch.cuda.current_stream())
+            for launch in step.values():
+                launch(side)
+            assert np.array_equal(_outputs(d)[2], want[2]), form
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                for launch in step.values():
+                    launch()
+            for _ in range(3):
+                d.cost.zero_()
+                graph.replay()
+                assert np.array_equal(_outputs(d)[2], want[2]), form
