@@ -834,7 +834,10 @@ constexpr int kMaxExponents = 32;
 constexpr int kGeneralStride = 8 * (8 + 1), kPow2Stride = 8 * (kMaxTermArrays + 1);  // bytes per state / exponent
 template <int M>
 struct TermTable {
-  static constexpr int kGeneral = kGeneralStride / 8 * States<M>::kCount;
+  // (a 2-D mesh has one state more, behind the others: the bytes of an unsharded producer after dim 1, before dim 0, for
+  // the order flip of TileStage::flip_words)
+  static constexpr int kStates = States<M>::kCount + (M == 2 ? 1 : 0);
+  static constexpr int kGeneral = kGeneralStride / 8 * kStates;
   static constexpr int kPow2 = kPow2Stride / 8 * kMaxExponents;
   static constexpr int kEntries = kGeneral > kPow2 ? kGeneral : kPow2;
 };
@@ -936,13 +939,14 @@ struct NoRowMinStage {};
 
 // A consumer spec of a tile: its placement codes; per mesh dim i, in byte i of `slots`, the
 // byte offset of its class's lookup word within a producer spec's words ((6 i + class) x 4;
-// byte 0 = 0xFF: not a DTensorSpec; on a 2-D mesh bit 24 = every dim is a Shard); the compute
+// byte 0 = 0xFF: not a DTensorSpec; on a 2-D mesh, when every dim is a Shard, bytes 2 and 3 are the
+// byte offsets of its two words in TileStage::flip_words, byte 3 never 0); the compute
 // cost / num_args of its strategy.  One 16-byte LDS read per entry.
 struct alignas(16) RowRecord {
   uint32_t codes, slots;
   double cpa;
 };
-constexpr uint32_t kRowNotASpec = 0xFFu, kRowAllShard = 1u << 24;
+constexpr uint32_t kRowNotASpec = 0xFFu;
 
 // The part of TermArrayConstants a value needs after its array's chain.
 struct alignas(16) TermValueConstants {
@@ -959,7 +963,12 @@ struct TileStage : std::conditional_t<RM, RowMinStage, NoRowMinStage> {
   // that the lanes of consecutive producer specs hit different banks
   uint32_t words[APC_TILE_MAX_COLS * (M * kWordsPerDim + 1)];
   alignas(16) uint32_t pair_base[M * 16];  // TermLayout::pair of the launch
-  double gb_unsharded;  // bytes / 1024^3 of the tile's tensor
+  // 2-D meshes: a (Partial, Partial) producer reaches an all-Shard consumer by two reduce-scatters, dim 1 first
+  // (collective_runtime_estimation.py:146-151).  The words of that walk, the same for every such producer: of dim 1, to
+  // Shard(0) and to another Shard, then of dim 0.  (Evaluated entry by entry, which a compiler partly does for all lanes,
+  // a pass of 64 entries took 102 vector instructions and the walk's own; by the words 45.  2.6 M entries on (12, 6):
+  // 18.7 -> 14.3 us.)
+  uint32_t flip_words[4];
   int mixed[4];         // per staging wavefront: some spec is not a DTensorSpec on the tile's tensor (generic loop)
   int cont;             // the tile's tensor is contiguous
   // Last: the tile kernels size their LDS per launch for the entries the layout in use needs
@@ -1043,7 +1052,7 @@ __device__ __forceinline__ double ring_at(double gb, const apc_params &p, int d,
 template <int M, bool DERIVE, bool RM>
 __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs &a, const apc_tile &tile,
                                            TileStage<M, RM> &st, int tid, int nthreads, TileCopies &copies) {
-  constexpr int NS = States<M>::kCount;
+  constexpr int NS = TermTable<M>::kStates;
   const int rows = tile.counts & 0xFFFF, cols = tile.counts >> 16;
   const int t0 = tile.tensor;  // spec_tensor of the tile's first producer spec (checked by the host)
   const bool no_producer = (tile.flags & APC_EDGE_NO_PRODUCER) != 0;
@@ -1150,15 +1159,15 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
       const int j = tid < E ? tid : tid - E;
       *reinterpret_cast<double *>(terms + j * kPow2Stride + (tid < E ? 0 : 8)) = tid < E ? 0.0 : __builtin_inf();
     }
-    if (tid == 0) st.gb_unsharded = fbytes / 1024 / 1024 / 1024;
   } else if (terms_wanted) {
     // every collective / read-write term the tile can need, once per running-bytes state, in
     // the reference's operation order (collective_runtime_estimation.py:66-68, :86, :128;
     // torch _collective_utils.py:281-313; compute_estimation.py:302-314)
     const double fbytes = (double)tensor_nbytes;
     for (int k = tid; k < NS; k += nthreads) {
-      const int level = 31 - __clz((k >> M) + 1);
-      const int rem = k - (((1 << level) - 1) << M);
+      const bool flip_state = M == 2 && k == States<M>::kCount;
+      const int level = flip_state ? 0 : 31 - __clz((k >> M) + 1);
+      const int rem = flip_state ? 0 : k - (((1 << level) - 1) << M);
       const int mask = rem >> level, hist = rem & ((1 << level) - 1);
       double shards = 1.0;  // exact: a product of mesh sizes (torch _dtensor_spec.py:555-561)
 #pragma unroll
@@ -1172,6 +1181,7 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
           gb = ((mask >> i) & 1) ? gb * m : div_by(gb, m, p.inv_mesh[i]);
         }
       }
+      if (flip_state) gb = div_by(gb, (double)p.mesh_size[1], p.inv_mesh[1]);
       double ag = 0.0, rs = 0.0, ar = 0.0;
       if (level >= 1) ag = ring_at<M>(gb, p, level - 1, 1);
       if (level < M) {
@@ -1191,13 +1201,17 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
       e[6] = ar;
       e[7] = a2a;
     }
-    if (tid == 0) st.gb_unsharded = fbytes / 1024 / 1024 / 1024;
-  } else if (tid == 0) {
-    st.gb_unsharded = 0.0;
   }
   // ---- what the loads brought, to LDS ---------------------------------------------------------
   if (tid == 0) st.cont = contiguous != 0;
   if (tid < 16 * M) st.pair_base[tid] = pair_word;
+  if (M == 2 && tid < 4) {  // (Partial -> Shard at dim 1, then at dim 0)
+    const int dim = tid < 2 ? 1 : 0;
+    const uint32_t base = st.pair_base[dim * 16 + 4 + 2 + (tid & 1)];
+    const uint32_t state = E != 0 ? (uint32_t)lay.lg_total : dim == 1 ? (uint32_t)States<M>::index(1, 0, 0) : (uint32_t)States<M>::kCount;
+    // (general layout: both states are named outright, no step between them)
+    st.flip_words[tid] = (E != 0 ? base : base & 0x00FFFFFFu) + __umul24(state, (uint32_t)lay.state_stride);
+  }
   if constexpr (RM) {
     if (tid < APC_TILE_MAX_ROWS) st.rmin[1][tid] = __builtin_inf();  // (slot 0 of every row is always written)
   }
@@ -1244,7 +1258,8 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
       slots |= (uint32_t)((kWordsPerDim * i + placement_class(t)) * 4) << (8 * i);
       all_shard &= kind_of(t) == 2;
     }
-    if (M == 2 && all_shard) slots |= kRowAllShard;
+    if (M == 2 && all_shard)
+      slots |= (dim_of((row_codes >> 8) & 0xFF) != 0 ? 4u : 0u) << 16 | (8u + (dim_of(row_codes & 0xFF) != 0 ? 4u : 0u)) << 24;
     if (row_tensor < 0) {  // a consumer spec that is not a DTensorSpec
       slots |= kRowNotASpec;
       mixed = true;
@@ -1276,7 +1291,7 @@ __device__ __forceinline__ EntryConstants entry_constants(const apc_params &p, c
 // Straight-line code: all lookups of an entry are independent of its fp additions, so they
 // are issued together; no vector memory loads.
 template <int M, bool CONT, bool RESCALE, bool RM>
-__device__ __forceinline__ void uniform_entry(const apc_params &p, const EntryConstants &k, const TileStage<M, RM> &st,
+__device__ __forceinline__ void uniform_entry(const EntryConstants &k, const TileStage<M, RM> &st,
                                               const char *terms, int r, int c, double &comm_o, double &total_o,
                                               int &trans_o) {
   const uint32_t src = st.col_codes[c];
@@ -1286,6 +1301,7 @@ __device__ __forceinline__ void uniform_entry(const apc_params &p, const EntryCo
   const char *words = reinterpret_cast<const char *>(st.words) + __umul24((uint32_t)c, (M * kWordsPerDim + 1) * 4);
   // ---- integer part: which term at which running index each mesh dim adds -------------------
   uint32_t at = 0;  // byte offset of the running index (history of the earlier dims / exponent steps), mod 2^32
+  const bool flip = M == 2 && src == 0x4040u && (row.slots >> 24) != 0u;  // dim 1 before dim 0 (flip_words)
   uint32_t term_at[M], rw_at[M], nc_at[M];
   bool neq[M];
 #pragma unroll
@@ -1293,7 +1309,9 @@ __device__ __forceinline__ void uniform_entry(const apc_params &p, const EntryCo
     neq[i] = ((x >> (8 * i)) & 0xFF) != 0;
     // (slot 4: same placement, nothing to add)
     const uint32_t slot = neq[i] ? (row.slots >> (8 * i)) & 0xFFu : (uint32_t)((kWordsPerDim * i + 4) * 4);
-    const uint32_t w = *reinterpret_cast<const uint32_t *>(words + slot);
+    const char *at_word = words + slot;
+    if (M == 2 && flip) at_word = reinterpret_cast<const char *>(st.flip_words) + ((row.slots >> (16 + 8 * i)) & 0xFFu);
+    const uint32_t w = *reinterpret_cast<const uint32_t *>(at_word);
     term_at[i] = (w & 0xFFFFu) + at;
     rw_at[i] = term_at[i] + (uint32_t)(int32_t)(int8_t)(w >> 16);
     if (!CONT) nc_at[i] = *reinterpret_cast<const uint32_t *>(words + (kWordsPerDim * i + 5) * 4) + at;
@@ -1323,9 +1341,6 @@ __device__ __forceinline__ void uniform_entry(const apc_params &p, const EntryCo
   }
   double comm = cost;  // (a banned transition added the +inf term)
   const int trans = x != 0u ? k.transition_scale : 0;  // optimize_sharding.py:345-351
-  if (M == 2 && src == 0x4040u && (row.slots & kRowAllShard)) {  // (Partial, Partial) -> all Shard walks dim 1 first
-    comm = entry_cost<M>(src, tgt, st.gb_unsharded, CONT, p);
-  }
   // :358-359; the quotient through the reciprocal is the division's (div_by), +inf stays +inf
   if (RESCALE) comm = comm < __builtin_inf() ? div_by(comm, k.rescale, k.inv_rescale) : comm;
   comm_o = comm;
@@ -1504,7 +1519,7 @@ __device__ __forceinline__ void uniform_tile_entries_row_min(const apc_params &p
     const bool active = idx >= 0 && idx < n;
     double comm = 0.0, total = 0.0;
     int trans = 0;
-    if (active) uniform_entry<M, CONT, RESCALE>(p, k, st, term_base(st, nthreads), r, c, comm, total, trans);
+    if (active) uniform_entry<M, CONT, RESCALE>(k, st, term_base(st, nthreads), r, c, comm, total, trans);
     store_entry<OUT>(out, v.dup_count, copies, active, __umul24((uint32_t)r, (uint32_t)v.n_src) + (uint32_t)c, comm, total,
                      trans);
     row_min_chunk(st.rmin, st.rarg, active, total, r, c, v.cols, lane);
@@ -1545,7 +1560,7 @@ __device__ __forceinline__ void uniform_tile_entries(const apc_params &p, const 
     const bool active = idx >= 0 && idx < n;
     double comm = 0.0, total = 0.0;
     int trans = 0;
-    if (active) uniform_entry<M, CONT, RESCALE>(p, k, st, term_base(st, nthreads), r, c, comm, total, trans);
+    if (active) uniform_entry<M, CONT, RESCALE>(k, st, term_base(st, nthreads), r, c, comm, total, trans);
     store_entry<OUT>(out, v.dup_count, copies, active, __umul24((uint32_t)r, (uint32_t)v.n_src) + (uint32_t)c, comm, total,
                      trans);
     if (active) {
