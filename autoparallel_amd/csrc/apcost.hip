@@ -925,18 +925,6 @@ static TermLayout term_layout(const apc_params &p) {
   return lay;
 }
 
-// Everything the entry loops need about one tile, in LDS.
-// What a tile that also takes its row minima keeps in LDS beside the rest (a launch that does
-// not want them is a different instantiation and does not pay for the space).
-struct RowMinStage {
-  // A row of at most 64 entries meets at most two of the 64-entry chunks the wavefronts
-  // walk.  Slot 0 takes the part that holds the row's first column, slot 1 the part that
-  // starts a chunk: one writer per slot, no atomics.
-  double rmin[2][APC_TILE_MAX_ROWS];
-  int rarg[2][APC_TILE_MAX_ROWS];
-};
-struct NoRowMinStage {};
-
 // A consumer spec of a tile: its placement codes; per mesh dim i, in byte i of `slots`, the
 // byte offset of its class's lookup word within a producer spec's words ((6 i + class) x 4;
 // byte 0 = 0xFF: not a DTensorSpec; on a 2-D mesh, when every dim is a Shard, bytes 2 and 3 are the
@@ -954,8 +942,9 @@ struct alignas(16) TermValueConstants {
   int32_t shift, pad_;
 };
 
+// Everything the entry loops need about one tile, in LDS.
 template <int M, bool RM>
-struct TileStage : std::conditional_t<RM, RowMinStage, NoRowMinStage> {
+struct TileStage {
   RowRecord row[APC_TILE_MAX_ROWS];  // consumer specs
   uint2 colh[APC_TILE_MAX_COLS];  // producer specs: x = codes, y = info
   uint32_t col_codes[APC_TILE_MAX_COLS];  // their codes again, packed (one LDS bank per lane)
@@ -973,7 +962,7 @@ struct TileStage : std::conditional_t<RM, RowMinStage, NoRowMinStage> {
   int cont;             // the tile's tensor is contiguous
   // Last: the tile kernels size their LDS per launch for the entries the layout in use needs
   // (stage_lds_bytes), so that the small power-of-two layout leaves room for more workgroups.
-  // In front of the entries, one StagingScratch per wavefront of the workgroup (a compile-time
+  // In front of the entries, one WaveScratch per wavefront of the workgroup (a compile-time
   // number in every kernel, so the entries still sit at a fixed offset): term_base.
   alignas(16) double terms[TermTable<M>::kEntries];
 };
@@ -983,17 +972,27 @@ struct alignas(16) StagingScratch {
   double chain[kMaxTermArrays];
   TermValueConstants value_of[kMaxTermArrays];
 };
+// What a wavefront has to itself: while it stages the term arrays, their chains; where the tile's row minima are
+// taken, in the same place afterwards, the values of the rows it is walking (tile_entries_row_min).
+constexpr int kRowMinValues = 512;
+template <bool RM>
+constexpr size_t kWaveScratchBytes = RM ? kRowMinValues * sizeof(double) : sizeof(StagingScratch);
+static_assert(kWaveScratchBytes<true> >= sizeof(StagingScratch), "the chains fit");
+template <int M, bool RM>
+__device__ __forceinline__ char *wave_scratch(const TileStage<M, RM> &st, int wave) {
+  return const_cast<char *>(reinterpret_cast<const char *>(st.terms)) + kWaveScratchBytes<RM> * (size_t)wave;
+}
 // Where the term arrays of a stage start, for a workgroup of `nthreads` threads.
-template <typename Stage>
-__device__ __forceinline__ char *term_base(Stage &st, int nthreads) {
-  return const_cast<char *>(reinterpret_cast<const char *>(st.terms)) + sizeof(StagingScratch) * (size_t)(nthreads >> 6);
+template <int M, bool RM>
+__device__ __forceinline__ char *term_base(const TileStage<M, RM> &st, int nthreads) {
+  return wave_scratch(st, nthreads >> 6);
 }
 
 // LDS bytes of a tile stage whose term arrays hold what the launch's layout needs.
 template <int M, bool RM>
 static size_t stage_lds_bytes(const TermLayout &lay, int threads) {
   const size_t entries = lay.exponents ? (size_t)(kPow2Stride / 8) * lay.exponents : (size_t)TermTable<M>::kGeneral;
-  return sizeof(TileStage<M, RM>) - sizeof(double) * TermTable<M>::kEntries + sizeof(StagingScratch) * (size_t)(threads / 64) +
+  return sizeof(TileStage<M, RM>) - sizeof(double) * TermTable<M>::kEntries + kWaveScratchBytes<RM> * (size_t)(threads / 64) +
          sizeof(double) * entries;
 }
 
@@ -1135,7 +1134,7 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
     // bytes (every wavefront its own copy: no barrier), then a lane per (array, exponent) the
     // value.
     const double fbytes = (double)tensor_nbytes;
-    StagingScratch &mine = reinterpret_cast<StagingScratch *>(st.terms)[wave];
+    StagingScratch &mine = *reinterpret_cast<StagingScratch *>(wave_scratch(st, wave));
     if (lane < kComputed) {
       mine.chain[lane] = div_by(div_by(fbytes * chain_of.hops, chain_of.div1, chain_of.inv_div1) * 1e6, chain_of.div2,
                                 chain_of.inv_div2);
@@ -1211,9 +1210,6 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
     const uint32_t state = E != 0 ? (uint32_t)lay.lg_total : dim == 1 ? (uint32_t)States<M>::index(1, 0, 0) : (uint32_t)States<M>::kCount;
     // (general layout: both states are named outright, no step between them)
     st.flip_words[tid] = (E != 0 ? base : base & 0x00FFFFFFu) + __umul24(state, (uint32_t)lay.state_stride);
-  }
-  if constexpr (RM) {
-    if (tid < APC_TILE_MAX_ROWS) st.rmin[1][tid] = __builtin_inf();  // (slot 0 of every row is always written)
   }
   if (has_col) {
     // info: bit0 valid spec, bit1 fully replicated, bits 4.. mask of sharded mesh dims
@@ -1404,15 +1400,14 @@ __device__ __forceinline__ double value_of_lane(double x, int lane) {  // lane: 
   return __hiloint2double(hi, lo);
 }
 
-// Row minima inside the tile kernel.  The 64 lanes of a wavefront hold 64 consecutive entries
+// Row minima of one pass, as the packed tiles take them.  The 64 lanes of a wavefront hold 64 consecutive entries
 // of the tile (inactive lanes: +inf), row after row.  `c` is the lane's column, `cols` the row
 // length.  First a segmented minimum by doubling inside every 16 lanes (data-parallel
 // primitives: vector ALU only, the LDS pipe stays free for the entry loop's lookups): a lane
 // then holds the minimum, and the first column that has it, of its row's entries from itself to
 // the end of its 16 lanes.  Lanes 16, 32 and 48 hold such a part for a row that came in from the
 // lanes before them: their values are read as scalars and joined, in lane order, by the lanes
-// whose row reaches them.  The first lane of every run of one row writes the row's slot.
-// row_min_in_wave: the reduction itself; on return a lane holds minimum and first argmin of its
+// whose row reaches them.  On return a lane holds minimum and first argmin of its
 // row's entries from itself to the row's end within the wavefront (the whole row for c == 0).
 __device__ __forceinline__ void row_min_in_wave(bool active, double value, int c, int cols, int lane, double &m, int &mc) {
   m = active ? value : __builtin_inf();
@@ -1450,89 +1445,107 @@ __device__ __forceinline__ void row_min_in_wave(bool active, double value, int c
 #undef APC_ROW_MIN_JOIN
 }
 
-__device__ __forceinline__ void row_min_chunk(double (&rmin)[2][APC_TILE_MAX_ROWS], int (&rarg)[2][APC_TILE_MAX_ROWS],
-                                              bool active, double value, int r, int c, int cols, int lane) {
-  double m;
-  int mc;
-  row_min_in_wave(active, value, c, cols, lane, m, mc);
-  if (active && (c == 0 || lane == 0)) {
-    const int slot = c == 0 ? 0 : 1;
-    rmin[slot][r] = m;
-    rarg[slot][r] = mc;
-  }
+__device__ __forceinline__ int from_lane(int v, int lane) { return __builtin_amdgcn_ds_bpermute(lane << 2, v); }
+__device__ __forceinline__ double from_lane(double v, int lane) {
+  return __hiloint2double(from_lane(__double2hiint(v), lane), from_lane(__double2loint(v), lane));
+}
+__device__ __forceinline__ int64_t from_lane_i64(int64_t v, int lane) {
+  const uint32_t lo = (uint32_t)from_lane((int)(uint32_t)v, lane), hi = (uint32_t)from_lane((int)(uint32_t)((uint64_t)v >> 32), lane);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
-// After every wavefront of the tile has written its slots: one thread per row joins the two
-// parts and stores minimum and first argmin to the row of the tile's edge and of every
-// identical edge.  (Called by every thread of the workgroup.)
-template <int M>
-__device__ __forceinline__ void row_min_finish(const TableArgs &a, TileStage<M, true> &st, const TileView &v,
-                                               const TileCopies &copies, int tid, int nthreads) {
-  __syncthreads();
-  // lane = row, wavefront w takes the copies w, w + waves, ...: copy 0 is the tile's own edge, copy
-  // d > 0 the d-th identical edge (a tile of many copies ends with a short store phase in every
-  // wavefront instead of a long one in the first)
-  const int row = tid & 63;
-  const bool live = row < v.rows;
-  double m = __builtin_inf();
-  int mc = 0;
-  if (live) {
-    m = st.rmin[0][row];
-    mc = st.rarg[0][row];
-    const double m1 = st.rmin[1][row];
-    if (m1 < m) {  // the later part wins only if strictly smaller
-      m = m1;
-      mc = st.rarg[1][row];
-    }
-  }
-  const int waves = nthreads >> 6;
-  for (int d = uniform_i32(tid >> 6); d <= v.dup_count; d += waves) {
-    const int64_t first = d == 0 ? uniform_i64(copies.row_out) : value_of_lane(copies.row0, d - 1);  // (uniform control flow)
-    if (live) {
-      const int64_t out = first + v.row_begin + row;
-      a.row_min_out[out] = m;
-      a.row_arg_out[out] = v.col_begin + mc;
-    }
-  }
+// The minimum, and the lowest column that has it, over neighbouring lanes of a row of 16: one step of a butterfly.
+template <int CTRL>
+__device__ __forceinline__ void lower_of_lanes(double &m, int &mc) {
+  const int lo = __double2loint(m), hi = __double2hiint(m);
+  const double om = __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false), __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false));
+  const int oc = __builtin_amdgcn_update_dpp(mc, mc, CTRL, 0xF, 0xF, false);
+  const bool take = om < m || (om == m && oc < mc);
+  m = take ? om : m;
+  mc = take ? oc : mc;
 }
 
-// The entry loop of a tile that holds whole rows, with the row minima: the walk of
-// uniform_tile_entries, except that every lane of a wavefront makes the same number of
-// passes (a lane in front of the tile's first entry idles in the first pass instead of
-// wrapping round), so that the lanes of one pass hold consecutive entries.
-template <int M, bool CONT, bool RESCALE, int OUT>
-__device__ __forceinline__ void uniform_tile_entries_row_min(const apc_params &p, const TableArgs &a, TileStage<M, true> &st,
-                                                             const TileView &v, const TileCopies &copies, int tid,
-                                                             int nthreads) {
-  const int n = v.rows * v.cols;
-  const int dr = nthreads / v.cols, dc = nthreads - dr * v.cols;
+// The entry loop of a tile that holds whole rows, with the row minima.  Every wavefront walks rows of its own, some at a
+// time: 64 consecutive entries a pass, evaluated (`entry`), stored, and kept in the wavefront's LDS; then 1 to 16 lanes a
+// row read it back, the lanes of a row the columns in turn, and join their minima.  The rows of a wavefront need no
+// barrier, and a value costs one write and one read of 8 bytes where a minimum taken across the lanes of every pass
+// (neighbours in doubling distances, value and column) was 70 vector instructions a pass, more than the entry's own 45.
+// kRowMinValues = 512, 384, 256: 38.7, 40.3, 41.5 us for 6.1 M entries on (64, 4), by passes 50.4, without the minima 27.4
+// (its rows' stores are 0.6 of that).
+template <int OUT, typename Entry>
+__device__ __forceinline__ void tile_entries_row_min(const TableArgs &a, double *values, const TileView &v, const TileCopies &copies,
+                                                     int tid, int nthreads, Entry entry) {
+  const int lane = tid & 63, wave = uniform_i32(tid >> 6), waves = nthreads >> 6;
+  const int cols = v.cols, stride = cols | 1;  // (odd: the lanes of consecutive rows read different banks)
+  const int at_once = min(kRowMinValues / stride, 64);
+  const int r0 = lane / cols, c0 = lane - r0 * cols, dr = 64 / cols, dc = 64 - dr * cols;
+  const int row_begin = v.rows * wave / waves, row_end = v.rows * (wave + 1) / waves;
   const int64_t tile_base = v.entry_begin + (int64_t)v.row_begin * v.n_src + v.col_begin;
-  const int shift = (int)(tile_base & 63);
-  const int lane = tid & 63;
-  int idx = tid - shift;
-  const int first = idx < 0 ? idx + nthreads : idx;
-  int r = first / v.cols, c = first - r * v.cols;
   const TileOut out{a.comm_out ? a.comm_out + tile_base : nullptr, a.trans_out ? a.trans_out + tile_base : nullptr,
                     a.cost_out ? a.cost_out + tile_base : nullptr, v.entry_begin};
-  const EntryConstants k = entry_constants(p, a.lay);
-  for (int wave_first = tid - lane - shift; wave_first < n; wave_first += nthreads, idx += nthreads) {
-    const bool active = idx >= 0 && idx < n;
-    double comm = 0.0, total = 0.0;
-    int trans = 0;
-    if (active) uniform_entry<M, CONT, RESCALE>(k, st, term_base(st, nthreads), r, c, comm, total, trans);
-    store_entry<OUT>(out, v.dup_count, copies, active, __umul24((uint32_t)r, (uint32_t)v.n_src) + (uint32_t)c, comm, total,
-                     trans);
-    row_min_chunk(st.rmin, st.rarg, active, total, r, c, v.cols, lane);
-    if (active) {
+  for (int first = row_begin; first < row_end; first += at_once) {
+    const int rows = min(at_once, row_end - first), n = rows * cols;
+    for (int at = 0, r = r0, c = c0; at < n; at += 64) {
+      const bool active = at + lane < n;
+      double comm = 0.0, total = 0.0;
+      int trans = 0;
+      if (active) entry(first + r, c, comm, total, trans);
+      store_entry<OUT>(out, v.dup_count, copies, active, __umul24((uint32_t)(first + r), (uint32_t)v.n_src) + (uint32_t)c, comm, total, trans);
+      if (active) values[__mul24(r, stride) + c] = total;
       c += dc;
       r += dr;
-      if (c >= v.cols) {
-        c -= v.cols;
+      if (c >= cols) {
+        c -= cols;
         r += 1;
       }
     }
+    __builtin_amdgcn_wave_barrier();  // (LDS operations of one wavefront complete in order)
+    const int shift = rows <= 4 ? 4 : rows <= 8 ? 3 : rows <= 16 ? 2 : rows <= 32 ? 1 : 0;  // 2^shift lanes a row
+    const int lanes = 1 << shift, row = lane >> shift, sub = lane & (lanes - 1);
+    const double *line = values + __mul24(min(row, rows - 1), stride);
+    const double head = line[0];
+    double m = __builtin_inf();
+    int mc = 0;
+    for (int y = sub; y < cols; y += 4 * lanes) {
+      int at[4];
+      double value[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        at[u] = min(y + u * lanes, cols - 1);  // (past the row's end: its last value once more)
+        value[u] = line[at[u]];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (value[u] < m) {  // strict: ties keep the lower column
+          m = value[u];
+          mc = at[u];
+        }
+    }
+    if (shift >= 1) lower_of_lanes<0xB1>(m, mc);   // quad_perm [1, 0, 3, 2]
+    if (shift >= 2) lower_of_lanes<0x4E>(m, mc);   // quad_perm [2, 3, 0, 1]
+    if (shift >= 3) lower_of_lanes<0x141>(m, mc);  // row_half_mirror
+    if (shift >= 4) lower_of_lanes<0x140>(m, mc);  // row_mirror
+    if (head != head) {  // (no value compares below a NaN in the first column)
+      m = head;
+      mc = 0;
+    }
+    __builtin_amdgcn_wave_barrier();
+    // all lanes of a row have the result: each stores it to a copy (copy 0 is the tile's own edge, copy d > 0 the d-th identical one)
+    const bool live = row < rows;
+    for (int copy0 = 0; copy0 <= v.dup_count; copy0 += lanes) {
+      const int copy = copy0 + sub;
+      int64_t first_row = copies.row_out;
+      if (v.dup_count > 0) {  // (uniform; every lane takes part)
+        const int64_t of_copy = from_lane_i64(copies.row0, max(copy - 1, 0));
+        first_row = copy == 0 ? first_row : of_copy;
+      }
+      if (live && copy <= v.dup_count) {
+        const int64_t o = first_row + v.row_begin + first + row;
+        a.row_min_out[o] = m;
+        a.row_arg_out[o] = v.col_begin + mc;
+      }
+    }
   }
-  row_min_finish<M>(a, st, v, copies, tid, nthreads);
 }
 
 // The per-entry loop of such a tile for `nthreads` threads (this one is `tid`): a flattened
@@ -1574,58 +1587,51 @@ __device__ __forceinline__ void uniform_tile_entries(const apc_params &p, const 
   }
 }
 
-// Generic loop: pass-through edges and edges whose producer specs name different tensors.
-// Every lane of a wavefront makes the same number of passes; ROW_MIN (tiles of whole rows only):
-// the row minima are taken on the way.
-template <int M, bool DERIVE, bool ROW_MIN, bool RM>
-__device__ __forceinline__ void generic_tile_entries(const apc_params &p, const TableArgs &a, TileStage<M, RM> &st,
-                                                     const TileView &v, const TileCopies &copies, int tid, int nthreads) {
+// The generic entry: pass-through edges and edges whose producer specs name different tensors (`local`: the entry's
+// place in its edge's matrix).
+template <int M, bool DERIVE, bool RM>
+__device__ __forceinline__ void generic_entry(const apc_params &p, const TableArgs &a, const TileStage<M, RM> &st, const TileView &v,
+                                              int r, int c, double &comm, double &total, int &trans) {
+  const int64_t local = (int64_t)(v.row_begin + r) * v.n_src + (v.col_begin + c);
+  const uint32_t src = st.colh[c].x, cinfo = st.colh[c].y;
+  const RowRecord row = st.row[r];
+  const uint32_t tgt = row.codes;
+  if ((v.flags & APC_EDGE_NO_PRODUCER) || !(cinfo & 1u) || (row.slots & 0xFFu) == kRowNotASpec) {
+    comm = a.pt_values[v.pt_begin + local];
+  } else {
+    trans = (src != tgt) ? p.transition_scale : 0;
+    const int sten = a.spec_tensor[v.src_begin + v.col_begin + c];
+    int64_t shards = 1;
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+      if (kind_of((src >> (8 * i)) & 0xFF) == 2) shards *= p.mesh_size[i];
+    int64_t sten_bytes;
+    bool sten_contiguous;
+    tensor_info<DERIVE>(a, sten, sten_bytes, sten_contiguous);
+    const double gb = (double)sten_bytes / (double)shards / 1024 / 1024 / 1024;
+    comm = entry_cost<M>(src, tgt, gb, sten_contiguous, p);
+  }
+  if (v.flags & APC_EDGE_GRAD_RESCALE) comm = comm / p.rescale;
+  total = comm + row.cpa + (double)trans;
+}
+
+// Their loop: every lane of a wavefront makes the same number of passes.
+template <int M, bool DERIVE, bool RM>
+__device__ __forceinline__ void generic_tile_entries(const apc_params &p, const TableArgs &a, const TileStage<M, RM> &st, const TileView &v,
+                                                     const TileCopies &copies, int tid, int nthreads) {
   const int n = v.rows * v.cols;
   const int lane = tid & 63;
   int r = tid / v.cols, c = tid - r * v.cols;
   const int dr = nthreads / v.cols, dc = nthreads - dr * v.cols;
-  const bool no_producer = (v.flags & APC_EDGE_NO_PRODUCER) != 0;
+  const int64_t tile_base = v.entry_begin + (int64_t)v.row_begin * v.n_src + v.col_begin;
+  const TileOut out{a.comm_out ? a.comm_out + tile_base : nullptr, a.trans_out ? a.trans_out + tile_base : nullptr,
+                    a.cost_out ? a.cost_out + tile_base : nullptr, v.entry_begin};
   for (int idx = tid; idx - lane < n; idx += nthreads) {
     const bool active = idx < n;
     double total = 0.0, comm = 0.0;
     int trans = 0;
-    int64_t o = 0;
-    if (active) {
-      const int64_t local = (int64_t)(v.row_begin + r) * v.n_src + (v.col_begin + c);
-      const uint32_t src = st.colh[c].x, cinfo = st.colh[c].y;
-      const RowRecord row = st.row[r];
-      const uint32_t tgt = row.codes;
-      if (no_producer || !(cinfo & 1u) || (row.slots & 0xFFu) == kRowNotASpec) {
-        comm = a.pt_values[v.pt_begin + local];
-      } else {
-        trans = (src != tgt) ? p.transition_scale : 0;
-        const int sten = a.spec_tensor[v.src_begin + v.col_begin + c];
-        int64_t shards = 1;
-#pragma unroll
-        for (int i = 0; i < M; ++i)
-          if (kind_of((src >> (8 * i)) & 0xFF) == 2) shards *= p.mesh_size[i];
-        int64_t sten_bytes;
-        bool sten_contiguous;
-        tensor_info<DERIVE>(a, sten, sten_bytes, sten_contiguous);
-        const double gb = (double)sten_bytes / (double)shards / 1024 / 1024 / 1024;
-        comm = entry_cost<M>(src, tgt, gb, sten_contiguous, p);
-      }
-      if (v.flags & APC_EDGE_GRAD_RESCALE) comm = comm / p.rescale;
-      o = v.entry_begin + local;
-      total = comm + row.cpa + (double)trans;
-      if (a.comm_out) a.comm_out[o] = comm;
-      if (a.trans_out) a.trans_out[o] = (uint8_t)trans;
-      if (a.cost_out) a.cost_out[o] = total;
-    }
-    for (int d = 0; d < v.dup_count; ++d) {
-      const int64_t delta = value_of_lane(copies.entry0, d) - v.entry_begin;  // (uniform control flow)
-      if (active) {
-        if (a.comm_out) a.comm_out[o + delta] = comm;
-        if (a.trans_out) a.trans_out[o + delta] = (uint8_t)trans;
-        if (a.cost_out) a.cost_out[o + delta] = total;
-      }
-    }
-    if constexpr (ROW_MIN && RM) row_min_chunk(st.rmin, st.rarg, active, total, r, c, v.cols, lane);
+    if (active) generic_entry<M, DERIVE>(p, a, st, v, r, c, comm, total, trans);
+    store_entry<kOutAny>(out, v.dup_count, copies, active, __umul24((uint32_t)r, (uint32_t)v.n_src) + (uint32_t)c, comm, total, trans);
     if (active) {
       c += dc;
       r += dr;
@@ -1635,7 +1641,6 @@ __device__ __forceinline__ void generic_tile_entries(const apc_params &p, const 
       }
     }
   }
-  if constexpr (ROW_MIN && RM) row_min_finish<M>(a, st, v, copies, tid, nthreads);
 }
 
 // All entries of a staged tile.  Row minima are taken when the caller wants them and the tile
@@ -1646,26 +1651,33 @@ __device__ __forceinline__ void tile_entries(const apc_params &p, const TableArg
   int mixed = st.mixed[0];
   for (int w = 1; w < nthreads / 64; ++w) mixed |= st.mixed[w];
   const bool row_minima = RM && v.cols == v.n_src;
+  double *const values = reinterpret_cast<double *>(wave_scratch(st, uniform_i32(tid >> 6)));
   if (uniform_i32(mixed)) {
     if constexpr (RM) {
       if (row_minima) {
-        generic_tile_entries<M, DERIVE, true>(p, a, st, v, copies, tid, nthreads);
+        tile_entries_row_min<kOutAny>(a, values, v, copies, tid, nthreads, [&](int r, int c, double &comm, double &total, int &trans) {
+          generic_entry<M, DERIVE>(p, a, st, v, r, c, comm, total, trans);
+        });
         return;
       }
     }
-    generic_tile_entries<M, DERIVE, false>(p, a, st, v, copies, tid, nthreads);
+    generic_tile_entries<M, DERIVE>(p, a, st, v, copies, tid, nthreads);
     return;
   }
   const bool rescale = (v.flags & APC_EDGE_GRAD_RESCALE) != 0;
-#define APC_TILE_LOOP(CONT_, RESCALE_)                                                            \
-  do {                                                                                            \
-    if constexpr (RM) {                                                                           \
-      if (row_minima) {                                                                           \
-        uniform_tile_entries_row_min<M, CONT_, RESCALE_, OUT>(p, a, st, v, copies, tid, nthreads); \
-        break;                                                                                    \
-      }                                                                                           \
-    }                                                                                             \
-    uniform_tile_entries<M, CONT_, RESCALE_, OUT>(p, a, st, v, copies, tid, nthreads);            \
+#define APC_TILE_LOOP(CONT_, RESCALE_)                                                                                                    \
+  do {                                                                                                                                    \
+    if constexpr (RM) {                                                                                                                   \
+      if (row_minima) {                                                                                                                   \
+        const EntryConstants k = entry_constants(p, a.lay);                                                                               \
+        const char *const terms = term_base(st, nthreads);                                                                                \
+        tile_entries_row_min<OUT>(a, values, v, copies, tid, nthreads, [&](int r, int c, double &comm, double &total, int &trans) {       \
+          uniform_entry<M, CONT_, RESCALE_>(k, st, terms, r, c, comm, total, trans);                                                      \
+        });                                                                                                                               \
+        break;                                                                                                                            \
+      }                                                                                                                                   \
+    }                                                                                                                                     \
+    uniform_tile_entries<M, CONT_, RESCALE_, OUT>(p, a, st, v, copies, tid, nthreads);                                                    \
   } while (0)
   if (uniform_i32(st.cont)) {
     if (rescale) { APC_TILE_LOOP(true, true); } else { APC_TILE_LOOP(true, false); }
@@ -1792,7 +1804,7 @@ template <int M, int kThreads, bool RM>
 __device__ __forceinline__ unsigned char *build_tables_lds() {
   if constexpr (M <= 2) {
     constexpr size_t kRowBytes = (size_t)kThreads * (APC_MAX_RANK + 1) * sizeof(int64_t);
-    constexpr size_t kStage = sizeof(TileStage<M, RM>) + sizeof(StagingScratch) * (kThreads / 64);
+    constexpr size_t kStage = sizeof(TileStage<M, RM>) + kWaveScratchBytes<RM> * (kThreads / 64);
     __shared__ __align__(16) unsigned char s_fixed[kStage > kRowBytes ? kStage : kRowBytes];
     return s_fixed;
   } else {
@@ -1973,15 +1985,6 @@ __device__ __forceinline__ double entry_cost_pow2(uint32_t srcp, uint32_t tgtp, 
   }
   if (srcp == 0u) return tgt_partial ? __builtin_inf() : 0.0;
   return banned ? __builtin_inf() : cost;
-}
-
-__device__ __forceinline__ int from_lane(int v, int lane) { return __builtin_amdgcn_ds_bpermute(lane << 2, v); }
-__device__ __forceinline__ double from_lane(double v, int lane) {
-  return __hiloint2double(from_lane(__double2hiint(v), lane), from_lane(__double2loint(v), lane));
-}
-__device__ __forceinline__ int64_t from_lane_i64(int64_t v, int lane) {
-  const uint32_t lo = (uint32_t)from_lane((int)(uint32_t)v, lane), hi = (uint32_t)from_lane((int)(uint32_t)((uint64_t)v >> 32), lane);
-  return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
 // value -> *(double *)((char *)base + byte_offset) for a wave-uniform base: the address stays a
