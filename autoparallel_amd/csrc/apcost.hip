@@ -329,17 +329,21 @@ struct States {
 };
 // ------------------------------------------------------------------------------------------
 // XCD-aware work order.  The dispatcher deals workgroups to the chip's 8 XCDs round-robin by
-// workgroup id, and every XCD has its own L2.  With the plain order, neighbouring units of
-// work (which write neighbouring memory and share the cache lines at their boundaries) sit
-// in eight different L2s and those lines are written back in parts.  The launchers round the
-// grid up to a multiple of 2^shift and the kernel takes unit (id mod 2^shift) * per + id /
-// 2^shift, so each XCD walks one contiguous share of the units.  (Measured: helps the tile
-// kernel, whose units end at arbitrary byte offsets; the kernels whose workgroups write
-// whole aligned blocks are faster in the plain order.)
+// workgroup id, and every XCD has its own L2.  With the plain order, neighbouring tiles
+// (which write neighbouring memory and share the cache lines at their boundaries) sit
+// in eight different L2s and those lines are written back in parts.  Runs of kXcdRun consecutive tiles go to one XCD
+// each, in turn; what is left behind the last full round of runs, in shares of one length.
+// (An XCD used to take one contiguous share of all tiles: a table whose copies are tiled unevenly, 19 layers as an edge for 16
+// and another for 3, then gave some XCDs five times the stores of others.  us a pass, contiguous shares / runs of 8 / 32 / 128
+// tiles: 5.8 M entries in 19 layers on (64, 4) 22.6 / 18.1 / 17.7 / 20.4; 37 M in 40 layers on (8, 8, 8) 70 / 63 / 67 / 68,
+// 73 M in 80 layers 131 / 137 / 126 / 127; the packed tables of 1.1 and 1.7 M as before.)
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ int64_t xcd_chunked_unit(int shift) {
-  const int64_t per = gridDim.x >> shift;
-  return (int64_t)(blockIdx.x & ((1u << shift) - 1)) * per + (blockIdx.x >> shift);
+constexpr int kXcdRun = APC_TILE_RUN;
+__device__ __forceinline__ int tile_of_block(int b, int n_tiles, int shift) {
+  const int round = kXcdRun << shift, full = n_tiles & ~(round - 1);  // (a power of two)
+  const int per = b < full ? kXcdRun : (n_tiles - full + (1 << shift) - 1) >> shift;
+  const int within = b < full ? b & (round - 1) : b - full;
+  return b - within + (within & ((1 << shift) - 1)) * per + (within >> shift);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1720,7 +1724,7 @@ __device__ __forceinline__ apc_tile fetch_tile(const apc_tile *tiles, int64_t ti
 template <int M, int kTileThreads, bool RM, int OUT>
 __device__ __forceinline__ void redistribute_tile(const apc_params &p, const TableArgs &a, const apc_tile *tiles, int n_tiles,
                                                   int xcd_shift, TileStage<M, RM> &stage) {
-  const int64_t tile_id = xcd_chunked_unit(xcd_shift);
+  const int tile_id = tile_of_block((int)blockIdx.x, n_tiles, xcd_shift);
   if (tile_id >= n_tiles) return;
   static_assert(kTileThreads == 64 || kTileThreads == 128 || kTileThreads == 256, "wavefronts per tile: 1, 2 or 4");
   static_assert(kTileThreads >= APC_TILE_MAX_COLS && kTileThreads >= APC_TILE_MAX_ROWS &&
@@ -1775,7 +1779,7 @@ void redistribute_tiles_row_min_kernel(APC_LAUNCH_PARAMS(TilesBlock)) {
 }
 
 // Every table of a pass in one launch: workgroups [0, tile_blocks) take the tiles of the
-// redistribution-cost matrices (tile_blocks = n_tiles rounded up to the XCD chunking), the
+// redistribution-cost matrices (tile_blocks = n_tiles rounded up to the number of XCDs), the
 // next spec_blocks the spec table, then the tensor table, then the compute costs, kThreads rows
 // per workgroup.  No workgroup reads what another writes: a tile derives its tensor's byte
 // count and contiguity and its consumer strategies' compute costs with the functions the
@@ -1833,8 +1837,7 @@ void build_tables_kernel(APC_LAUNCH_PARAMS(BuildTablesBlock)) {
   static_assert(kThreads == 64 || kThreads == 128 || kThreads == 256, "wavefronts per workgroup: 1, 2 or 4");
   const int64_t b = blockIdx.x;
   if (b < tile_blocks) {
-    const int64_t per = tile_blocks >> xcd_shift;
-    const int64_t tile_id = (b & ((1 << xcd_shift) - 1)) * per + (b >> xcd_shift);
+    const int tile_id = tile_of_block((int)b, n_tiles, xcd_shift);
     if (tile_id >= n_tiles) return;
     TileStage<M, RM> &stage = *reinterpret_cast<TileStage<M, RM> *>(s_raw);
     const apc_tile tile = fetch_tile<true, RM, OUT>(tiles, tile_id, a);
@@ -2192,8 +2195,7 @@ __global__ __launch_bounds__(kBlock) void build_tables_packed_kernel(APC_LAUNCH_
   const PackedBlock &k = launch_block(kept);
   const int64_t b = blockIdx.x;
   if (b < tile_blocks) {
-    const int64_t per = tile_blocks >> xcd_shift;
-    const int64_t tile_id = (b & ((1 << xcd_shift) - 1)) * per + (b >> xcd_shift);
+    const int tile_id = tile_of_block((int)b, n_tiles, xcd_shift);
     if (tile_id >= n_tiles) return;
     packed_tile<M, POW2>(static_cast<const apc_packed_tile *>(work) + tile_id, cost_out, k.a);
     return;
@@ -3189,7 +3191,7 @@ static int redistribute_tables_impl(const apc_params *params, const int64_t *ten
               rows ? rows->edge_row_begin : nullptr, rows ? rows->dup_row_begin : nullptr,
               rows ? rows->row_min : nullptr, rows ? rows->row_argmin : nullptr, term_layout(*params)};
   const int nt = (int)n_tiles, xs = xcd_shift();
-  const int64_t grid = ((n_tiles + (1 << xs) - 1) >> xs) << xs;  // rounded up for xcd_chunked_unit
+  const int64_t grid = ((n_tiles + (1 << xs) - 1) >> xs) << xs;  // rounded up for tile_of_block
   const char *const what = rows ? "apc_redistribute_tables_row_min" : "apc_redistribute_tables";
   const int threads = tile_threads(n_tiles, n_entries, params->mesh_ndim == 4 && a.lay.exponents == 0, 512, 2048);
   const int om = out_mode(params->mesh_ndim, comm_out, trans_out, cost_out);

@@ -62,6 +62,7 @@ extern "C" {
 #define APC_MAX_DTYPES 8
 #define APC_TILE_MAX_COLS 64 /* producer specs staged in LDS per tile */
 #define APC_TILE_MAX_ROWS 64 /* consumer specs staged in LDS per tile */
+#define APC_TILE_RUN 32 /* consecutive tiles that one of the chip's dies takes, in turn with the others (a power of two) */
 #define APC_TILE_MAX_DUPS 32 /* identical edges served by one tile (offsets staged in LDS); a larger group of
                               identical edges is served by several tiled edges.  apc_validate_tables_host
                               rejects a tile with more; the kernels leave such a tile unwritten */
