@@ -63,6 +63,25 @@ template <typename T>
 __device__ __forceinline__ T uniform_load(const T *p) {
   return *(const APC_CONSTANT T *)p;
 }
+// A place in LDS as its address: what a lane looks up lies at addresses it adds up, and an offset known when the code is
+// compiled becomes part of the load.
+#define APC_LDS __attribute__((address_space(3)))
+typedef uint32_t lds_address;
+__device__ __forceinline__ lds_address address_in_lds(const void *p) { return (lds_address)(uintptr_t)(const APC_LDS char *)p; }
+template <typename T>
+__device__ __forceinline__ T lds_read(lds_address at) {
+  return *(const APC_LDS T *)(uintptr_t)at;
+}
+template <typename T>
+__device__ __forceinline__ void lds_write(lds_address at, T value) {
+  *(APC_LDS T *)(uintptr_t)at = value;
+}
+// A lane's element of an array that starts at a wave-uniform address: the address stays a pair of scalar registers and
+// a 32-bit offset per lane.  (As one 64-bit index per lane a tile's eleven loads took 40 vector instructions for their addresses.)
+template <typename T>
+__device__ __forceinline__ T load_of_lane(const T *base, uint32_t lane) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + lane * (uint32_t)sizeof(T));
+}
 // A plain store that is written through to memory (system scope, no ordering).  What a launch of
 // a few tens of MB leaves in the L2 is written back when the kernel ends, after its last
 // wavefront, and the launch lasts until that is done; written through, the lines leave while the
@@ -97,6 +116,7 @@ __device__ __forceinline__ const Block &launch_block(const Block *kept) {
 
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 typedef int64_t i64x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // The value lane `lane` (wave-uniform) holds.
 __device__ __forceinline__ int64_t value_of_lane(int64_t x, int lane) {
@@ -799,9 +819,10 @@ __host__ __device__ constexpr uint32_t pair_action(int c, int t) {
   if (c == 1) return t == 0 ? AR : (RS | (tn << 3) | UPD);
   return t == 0 ? (AG | (cn << 3) | UPD) : (A2A | ((cn + tn) << 3));
 }
-__device__ __forceinline__ int placement_class(uint32_t code) {
-  const int k = kind_of(code);
-  return k == 2 ? 2 + (dim_of(code) != 0 ? 1 : 0) : k;
+// (of the placement at mesh dim i of packed codes; a Shard's code is 0x80 | .. | its dim)
+__device__ __forceinline__ uint32_t placement_class(uint32_t codes, int i) {
+  const uint32_t kind = (codes >> (8 * i + 6)) & 3u;
+  return kind + ((codes & (0x8Fu << (8 * i))) > (0x80u << (8 * i)) ? 1u : 0u);
 }
 
 // Term arrays staged per tile, interleaved: the entry of (state s, array a) sits at byte
@@ -839,7 +860,7 @@ constexpr int kGeneralStride = 8 * (8 + 1), kPow2Stride = 8 * (kMaxTermArrays + 
 template <int M>
 struct TermTable {
   // (a 2-D mesh has one state more, behind the others: the bytes of an unsharded producer after dim 1, before dim 0, for
-  // the order flip of TileStage::flip_words)
+  // the order flip's words)
   static constexpr int kStates = States<M>::kCount + (M == 2 ? 1 : 0);
   static constexpr int kGeneral = kGeneralStride / 8 * kStates;
   static constexpr int kPow2 = kPow2Stride / 8 * kMaxExponents;
@@ -863,6 +884,20 @@ static_assert(4 + 3 * APC_MAX_MESH <= kMaxTermArrays, "arrays of the power-of-tw
 // Slot 4 of a (spec, dim) is the word of "same placement": zeros, no step; slot 5 is the byte
 // offset of one read+write at the state BEFORE the dim, charged once to a non-contiguous tensor.
 constexpr int kWordsPerDim = 6;
+// The words of a producer spec: the dims', on a 2-D mesh the four of its order flip (below), its codes.  An odd number,
+// so that the lanes of consecutive producer specs hit different banks.
+// A (Partial, Partial) producer on a 2-D mesh reaches an all-Shard consumer by two reduce-scatters, dim 1 first
+// (collective_runtime_estimation.py:146-151): words kFlipWord.. hold that walk, of dim 1 to Shard(0) and to another Shard,
+// then of dim 0, and byte 3 of the producer's codes holds the shift (kFlipShift, 0 for any other producer) that takes a
+// consumer's flip slots in place of its plain ones (RowRecord).
+constexpr uint32_t kFlipShift = 16;
+template <int M>
+constexpr int kFlipWord = M * kWordsPerDim;
+template <int M>
+constexpr int kCodesWord = M * kWordsPerDim + (M == 2 ? 4 : 0);
+template <int M>
+constexpr int kColWords = kCodesWord<M> + 1;
+static_assert(kColWords<1> % 2 == 1 && kColWords<2> % 2 == 1 && kColWords<3> % 2 == 1 && kColWords<4> % 2 == 1, "an odd number of words");
 constexpr uint32_t kZerosArray = 0, kInfArray = 1, kRw1Array = 2;
 static_assert(TermTable<APC_MAX_MESH>::kEntries * 8 <= 0xFFFF + 1, "term offsets fit their 16 bits");
 
@@ -931,8 +966,8 @@ static TermLayout term_layout(const apc_params &p) {
 
 // A consumer spec of a tile: its placement codes; per mesh dim i, in byte i of `slots`, the
 // byte offset of its class's lookup word within a producer spec's words ((6 i + class) x 4;
-// byte 0 = 0xFF: not a DTensorSpec; on a 2-D mesh, when every dim is a Shard, bytes 2 and 3 are the
-// byte offsets of its two words in TileStage::flip_words, byte 3 never 0); the compute
+// byte 0 = 0xFF: not a DTensorSpec; on a 2-D mesh bytes 2 and 3 are what a (Partial, Partial) producer takes
+// instead: the same, or, when every dim is a Shard, the offsets of its two flip words); the compute
 // cost / num_args of its strategy.  One 16-byte LDS read per entry.
 struct alignas(16) RowRecord {
   uint32_t codes, slots;
@@ -951,17 +986,8 @@ template <int M, bool RM>
 struct TileStage {
   RowRecord row[APC_TILE_MAX_ROWS];  // consumer specs
   uint2 colh[APC_TILE_MAX_COLS];  // producer specs: x = codes, y = info
-  uint32_t col_codes[APC_TILE_MAX_COLS];  // their codes again, packed (one LDS bank per lane)
-  // lookup words per (producer spec, dim, consumer class); an odd number of words per spec, so
-  // that the lanes of consecutive producer specs hit different banks
-  uint32_t words[APC_TILE_MAX_COLS * (M * kWordsPerDim + 1)];
+  uint32_t words[APC_TILE_MAX_COLS * kColWords<M>];  // lookup words per (producer spec, dim, consumer class), and its codes
   alignas(16) uint32_t pair_base[M * 16];  // TermLayout::pair of the launch
-  // 2-D meshes: a (Partial, Partial) producer reaches an all-Shard consumer by two reduce-scatters, dim 1 first
-  // (collective_runtime_estimation.py:146-151).  The words of that walk, the same for every such producer: of dim 1, to
-  // Shard(0) and to another Shard, then of dim 0.  (Evaluated entry by entry, which a compiler partly does for all lanes,
-  // a pass of 64 entries took 102 vector instructions and the walk's own; by the words 45.  2.6 M entries on (12, 6):
-  // 18.7 -> 14.3 us.)
-  uint32_t flip_words[4];
   int mixed[4];         // per staging wavefront: some spec is not a DTensorSpec on the tile's tensor (generic loop)
   int cont;             // the tile's tensor is contiguous
   // Last: the tile kernels size their LDS per launch for the entries the layout in use needs
@@ -970,6 +996,23 @@ struct TileStage {
   // number in every kernel, so the entries still sit at a fixed offset): term_base.
   alignas(16) double terms[TermTable<M>::kEntries];
 };
+
+// Where its parts begin, in bytes.
+template <int M, bool RM>
+__host__ __device__ constexpr uint32_t rows_at() {
+  using Stage = TileStage<M, RM>;
+  return (uint32_t)offsetof(Stage, row);
+}
+template <int M, bool RM>
+__host__ __device__ constexpr uint32_t words_at() {
+  using Stage = TileStage<M, RM>;
+  return (uint32_t)offsetof(Stage, words);
+}
+template <int M, bool RM>
+__host__ __device__ constexpr uint32_t terms_at() {
+  using Stage = TileStage<M, RM>;
+  return (uint32_t)offsetof(Stage, terms);
+}
 
 // What one wavefront keeps while it stages the term arrays of the power-of-two layout.
 struct alignas(16) StagingScratch {
@@ -1071,8 +1114,8 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
   // power-of-two layout: the constants of array 2 + lane (whose chain this lane computes) and of
   // the array of the first value this thread computes, also read by lane
   constexpr int kComputed = 3 * M + 2;
-  TermArrayConstants chain_of{};
-  if (E != 0 && lane < kComputed) chain_of = lay.arrays[lane];
+  TermArrayConstants chain_of;
+  if (E != 0) chain_of = load_of_lane(lay.arrays, (uint32_t)min(lane, kComputed - 1));
   // ---- the round of vector loads ------------------------------------------------------------
   // producer spec tid, consumer spec nthreads - 1 - tid (taken from the far end: with two
   // wavefronts one loads the producer specs while the other loads the consumer specs).
@@ -1080,31 +1123,31 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
   // values are first touched after the state terms.
   const int jc = tid, jr = nthreads - 1 - tid;
   const bool has_col = jc < cols, has_row = jr < rows;
-  const int sp = tile.src_begin + tile.col_begin + (has_col ? jc : 0);
-  const int ts = tile.tgt_begin + tile.row_begin + (has_row ? jr : 0);
-  const int col_tensor = a.spec_tensor[sp];
-  const uint32_t col_codes = a.spec_codes[sp];
-  const uint32_t row_codes = a.spec_codes[ts];
-  const int row_tensor = a.spec_tensor[ts];
-  const int sr = tile.strat_begin + tile.row_begin + (has_row ? jr : 0);
+  const uint32_t at_col = has_col ? (uint32_t)jc : 0u, at_row = has_row ? (uint32_t)jr : 0u;
+  const int64_t sp = (int64_t)tile.src_begin + tile.col_begin, ts = (int64_t)tile.tgt_begin + tile.row_begin;
+  const int64_t sr = (int64_t)tile.strat_begin + tile.row_begin;
+  const int col_tensor = load_of_lane(a.spec_tensor + sp, at_col);
+  const uint32_t col_codes = load_of_lane(a.spec_codes + sp, at_col);
+  const uint32_t row_codes = load_of_lane(a.spec_codes + ts, at_row);
+  const int row_tensor = load_of_lane(a.spec_tensor + ts, at_row);
   double row_cpa = 0.0;
   int64_t row_flops = 0, row_rw = 0;
   int row_dtype = 0, row_zero = 1, row_args = 1;
   if (!DERIVE) {
-    if (a.per_arg) row_cpa = a.per_arg[sr];
+    if (a.per_arg) row_cpa = load_of_lane(a.per_arg + sr, at_row);
   } else {
-    row_flops = a.flops[sr];
-    row_rw = a.rw_bytes[sr];
-    row_dtype = a.dtype[sr];
-    row_zero = a.zero_cost[sr];
-    row_args = a.num_args[sr];
+    row_flops = load_of_lane(a.flops + sr, at_row);
+    row_rw = load_of_lane(a.rw_bytes + sr, at_row);
+    row_dtype = load_of_lane(a.dtype + sr, at_row);
+    row_zero = load_of_lane(a.zero_cost + sr, at_row);
+    row_args = load_of_lane(a.num_args + sr, at_row);
   }
   // (every wavefront its own copy of the identical edges' offsets, in lanes 0 .. dup_count - 1)
   const bool has_dup0 = lane < tile.dup_count;
   copies.entry0 = copies.row0 = copies.row_out = 0;
-  if (has_dup0) copies.entry0 = a.dup_entry_begin[tile.dup_begin + lane];
+  if (has_dup0) copies.entry0 = load_of_lane(a.dup_entry_begin + tile.dup_begin, (uint32_t)lane);
   if constexpr (RM) {
-    if (has_dup0) copies.row0 = a.dup_row_begin[tile.dup_begin + lane];
+    if (has_dup0) copies.row0 = load_of_lane(a.dup_row_begin + tile.dup_begin, (uint32_t)lane);
     // (wave-uniform, but needed last: with the vector loads of the round, so that the scalar
     // loads the term arrays wait for are one round and not two)
     copies.row_out = a.edge_row_begin[tile.edge];
@@ -1150,17 +1193,18 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
     // instantiations by hipcc 7.2: the placement-pair tests on 4-D power-of-two meshes show it.)
     char *terms = term_base(st, nthreads);
     for (int t = tid; t < kComputed * E; t += nthreads) {
-      const int arr = (int)(((uint32_t)t * lay.exponent_magic) >> 16);  // t / E
-      const int j = t - arr * E;  // the running bytes are bytes x 2^(j - L - 30)
+      // (24-bit multiplies: an integer multiply of 32 bits takes four times as long)
+      const int arr = (int)((uint32_t)__umul24((uint32_t)t, lay.exponent_magic) >> 16);  // t / E
+      const int j = t - __mul24(arr, E);  // the running bytes are bytes x 2^(j - L - 30)
       const TermValueConstants k = mine.value_of[arr];
       double v = k.lat + __builtin_ldexp(mine.chain[arr], j + k.shift);
       v = v > k.floor ? v : k.floor;
       v = v * k.scale;
-      *reinterpret_cast<double *>(terms + j * kPow2Stride + (arr + 2) * 8) = v;
+      *reinterpret_cast<double *>(terms + __mul24(j, kPow2Stride) + (arr + 2) * 8) = v;
     }
     if (tid < 2 * E) {
       const int j = tid < E ? tid : tid - E;
-      *reinterpret_cast<double *>(terms + j * kPow2Stride + (tid < E ? 0 : 8)) = tid < E ? 0.0 : __builtin_inf();
+      *reinterpret_cast<double *>(terms + __mul24(j, kPow2Stride) + (tid < E ? 0 : 8)) = tid < E ? 0.0 : __builtin_inf();
     }
   } else if (terms_wanted) {
     // every collective / read-write term the tile can need, once per running-bytes state, in
@@ -1208,13 +1252,6 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
   // ---- what the loads brought, to LDS ---------------------------------------------------------
   if (tid == 0) st.cont = contiguous != 0;
   if (tid < 16 * M) st.pair_base[tid] = pair_word;
-  if (M == 2 && tid < 4) {  // (Partial -> Shard at dim 1, then at dim 0)
-    const int dim = tid < 2 ? 1 : 0;
-    const uint32_t base = st.pair_base[dim * 16 + 4 + 2 + (tid & 1)];
-    const uint32_t state = E != 0 ? (uint32_t)lay.lg_total : dim == 1 ? (uint32_t)States<M>::index(1, 0, 0) : (uint32_t)States<M>::kCount;
-    // (general layout: both states are named outright, no step between them)
-    st.flip_words[tid] = (E != 0 ? base : base & 0x00FFFFFFu) + __umul24(state, (uint32_t)lay.state_stride);
-  }
   if (has_col) {
     // info: bit0 valid spec, bit1 fully replicated, bits 4.. mask of sharded mesh dims
     uint32_t info = (col_tensor >= 0 ? 1u : 0u) | (col_codes == 0u ? 2u : 0u);
@@ -1223,29 +1260,48 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
     for (int i = 0; i < M; ++i) mask |= (kind_of((col_codes >> (8 * i)) & 0xFF) == 2 ? 1u : 0u) << i;
     info |= mask << 4;
     st.colh[jc] = make_uint2(col_codes, info);
-    st.col_codes[jc] = col_codes;
-    // power-of-two mesh: the producer spec's exponent index, L - log2(its shards)
-    uint32_t j0 = (uint32_t)lay.lg_total;
+    uint32_t *const w_of_col = st.words + __umul24((uint32_t)jc, (uint32_t)kColWords<M>);
+    w_of_col[kCodesWord<M>] = col_codes;
+    const auto words_of_dims = [&](auto pow2) {
+      constexpr bool POW2 = decltype(pow2)::value;
+      // power-of-two mesh: the producer spec's exponent index, L - log2(its shards)
+      uint32_t j0 = (uint32_t)lay.lg_total;
+      if constexpr (POW2) {
 #pragma unroll
-    for (int i = 0; i < M; ++i) j0 -= ((mask >> i) & 1u) ? (uint32_t)lay.lg[i] : 0u;
+        for (int i = 0; i < M; ++i) j0 -= ((mask >> i) & 1u) ? (uint32_t)lay.lg[i] : 0u;
+      }
 #pragma unroll
-    for (int i = 0; i < M; ++i) {
-      const int cls = placement_class((col_codes >> (8 * i)) & 0xFF);
-      const uint4 base = reinterpret_cast<const uint4 *>(st.pair_base)[i * 4 + cls];
-      // general layout: states of this dim for history 0, before the dim and after an update at
-      // it; the all-gather (a sharding producer, a replicating consumer: class 0) is charged on
-      // the gathered bytes.  (Power-of-two layout: that shift is part of the word's base.)
-      const uint32_t k = (uint32_t)States<M>::index(i, 0, 0) + (mask << i);
-      const uint32_t k2 = (uint32_t)States<M>::index(i + 1, 0, 0) + (mask << (i + 1)) + (1u << i);
-      const uint32_t at = __umul24(E != 0 ? j0 : k, (uint32_t)lay.state_stride);
-      const uint32_t at0 = __umul24(E != 0 ? j0 : cls >= 2 ? k2 : k, (uint32_t)lay.state_stride);
-      uint32_t *w = st.words + jc * (M * kWordsPerDim + 1) + i * kWordsPerDim;
-      w[0] = base.x + at0;
-      w[1] = base.y + at;
-      w[2] = base.z + at;
-      w[3] = base.w + at;
-      w[4] = at;  // the zeros array, no read+write, no step
-      w[5] = at + kRw1Array * 8u;
+      for (int i = 0; i < M; ++i) {
+        const uint32_t cls = placement_class(col_codes, i);
+        const uint4 base = reinterpret_cast<const uint4 *>(st.pair_base)[i * 4 + cls];
+        // general layout: states of this dim for history 0, before the dim and after an update at
+        // it; the all-gather (a sharding producer, a replicating consumer: class 0) is charged on
+        // the gathered bytes.  (Power-of-two layout: that shift is part of the word's base.)
+        const uint32_t k = (uint32_t)States<M>::index(i, 0, 0) + (mask << i);
+        const uint32_t k2 = (uint32_t)States<M>::index(i + 1, 0, 0) + (mask << (i + 1)) + (1u << i);
+        const uint32_t at = (uint32_t)__umul24(POW2 ? j0 : k, POW2 ? (uint32_t)kPow2Stride : (uint32_t)kGeneralStride);
+        const uint32_t at0 = POW2 ? at : (uint32_t)__umul24(cls >= 2 ? k2 : k, (uint32_t)kGeneralStride);
+        uint32_t *w = w_of_col + i * kWordsPerDim;
+        w[0] = base.x + at0;
+        w[1] = base.y + at;
+        w[2] = base.z + at;
+        w[3] = base.w + at;
+        w[4] = at;  // the zeros array, no read+write, no step
+        w[5] = at + kRw1Array * 8u;
+      }
+    };
+    if (E != 0) words_of_dims(std::true_type{});
+    else words_of_dims(std::false_type{});
+    if (M == 2 && col_codes == 0x4040u) {
+      w_of_col[kCodesWord<M>] = col_codes | (kFlipShift << 24);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {  // (Partial -> Shard at dim 1, then at dim 0)
+        const int dim = k < 2 ? 1 : 0;
+        const uint32_t base = st.pair_base[dim * 16 + 4 + 2 + (k & 1)];
+        const uint32_t state = E != 0 ? (uint32_t)lay.lg_total : dim == 1 ? (uint32_t)States<M>::index(1, 0, 0) : (uint32_t)States<M>::kCount;
+        // (general layout: both states are named outright, no step between them)
+        w_of_col[kFlipWord<M> + k] = (E != 0 ? base : base & 0x00FFFFFFu) + __umul24(state, (uint32_t)lay.state_stride);
+      }
     }
     if (col_tensor != t0 || col_tensor < 0) mixed = true;
   }
@@ -1255,11 +1311,14 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
 #pragma unroll
     for (int i = 0; i < M; ++i) {
       const uint32_t t = (row_codes >> (8 * i)) & 0xFF;
-      slots |= (uint32_t)((kWordsPerDim * i + placement_class(t)) * 4) << (8 * i);
+      slots += ((uint32_t)(kWordsPerDim * i) + placement_class(row_codes, i)) << (8 * i + 2);
       all_shard &= kind_of(t) == 2;
     }
-    if (M == 2 && all_shard)
-      slots |= (dim_of((row_codes >> 8) & 0xFF) != 0 ? 4u : 0u) << 16 | (8u + (dim_of(row_codes & 0xFF) != 0 ? 4u : 0u)) << 24;
+    if (M == 2) {
+      const uint32_t flip = ((kFlipWord<M> * 4u + (dim_of((row_codes >> 8) & 0xFF) != 0 ? 4u : 0u)) << 16) |
+                            ((kFlipWord<M> * 4u + 8u + (dim_of(row_codes & 0xFF) != 0 ? 4u : 0u)) << 24);
+      slots |= all_shard ? flip : slots << 16;
+    }
     if (row_tensor < 0) {  // a consumer spec that is not a DTensorSpec
       slots |= kRowNotASpec;
       mixed = true;
@@ -1278,52 +1337,122 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
 // The arguments an entry loop uses, in scalar registers before it begins.  (Left to the compiler, an argument is loaded
 // where it is used, in every pass, and a scalar load in flight makes the wait for an LDS read a wait for everything.)
 struct EntryConstants {
-  double rescale, inv_rescale;
+  double rescale, inv_rescale, transition;
   int32_t transition_scale, state_stride;
 };
 __device__ __forceinline__ EntryConstants entry_constants(const apc_params &p, const TermLayout &lay) {
-  EntryConstants k{p.rescale, lay.inv_rescale, p.transition_scale, lay.state_stride};
-  __asm__ volatile("" : "+s"(k.rescale), "+s"(k.inv_rescale), "+s"(k.transition_scale), "+s"(k.state_stride));
+  EntryConstants k{p.rescale, lay.inv_rescale, (double)p.transition_scale, p.transition_scale, lay.state_stride};
+  __asm__ volatile("" : "+s"(k.rescale), "+s"(k.inv_rescale), "+v"(k.transition), "+s"(k.transition_scale), "+s"(k.state_stride));
   return k;
 }
 
-// One entry of a tile whose producer specs all name one tensor (column c, row r of the tile).
+// Where a lane is in a tile: the addresses of its producer spec's words and of its consumer spec's record, and the bytes to its
+// entry from the tile's first one.  (Kept as what the loads and the store need: of a column and a row, every pass would shift
+// and multiply again.)
+struct TileWalk {
+  lds_address col, row;
+  uint32_t out;
+};
+struct TileSteps {  // of one pass; `wrap`: when the column passes the row's end
+  uint32_t dcol, end, cols, drow, drow_wrap, dout, dout_wrap;
+};
+template <int M, bool RM>
+__device__ __forceinline__ TileWalk tile_walk(lds_address stage, int r, int c, int n_src) {
+  return TileWalk{stage + words_at<M, RM>() + (uint32_t)__mul24(c, kColWords<M> * 4),
+                  stage + rows_at<M, RM>() + (uint32_t)r * 16u,
+                  (uint32_t)(__mul24(r, n_src) + c) * 8u};
+}
+// (dr, dc: rows and columns of a pass; uniform, as everything here)
+template <int M, bool RM>
+__device__ __forceinline__ TileSteps tile_steps(lds_address stage, uint32_t dr, uint32_t dc, uint32_t cols, uint32_t n_src) {
+  constexpr uint32_t kCol = (uint32_t)kColWords<M> * 4u;
+  const uint32_t dout = (dr * n_src + dc) * 8u;
+  return TileSteps{dc * kCol, stage + words_at<M, RM>() + cols * kCol, cols * kCol, dr * 16u, dr * 16u + 16u, dout, dout + (n_src - cols) * 8u};
+}
+template <bool WHOLE>  // whole rows: the entries of a tile are consecutive
+__device__ __forceinline__ void advance(TileWalk &w, const TileSteps &s) {
+  const uint32_t col = w.col + s.dcol;
+  const bool wrap = col >= s.end;
+  w.col = wrap ? col - s.cols : col;
+  w.row += wrap ? s.drow_wrap : s.drow;
+  w.out += WHOLE ? s.dout : wrap ? s.dout_wrap : s.dout;
+}
+
+// x / d for a wave-uniform 0 < d <= 64 and 0 <= x <= 8192: (x + 1/2) / d is at least 1/128 away from a whole number,
+// its rounding and that of 1 / d in 24 bits are 2^-9 at most.  (An integer division is 20 instructions.)
+__device__ __forceinline__ uint32_t small_quotient(uint32_t x, float inv_d) { return (uint32_t)(((float)x + 0.5f) * inv_d); }
+// The same where x is uniform too, as a scalar.  (The conversion would be moved behind the read of the first lane, into a
+// vector register again.)
+__device__ __forceinline__ uint32_t uniform_quotient(uint32_t x, float inv_d) {
+  uint32_t q = small_quotient(x, inv_d);
+  __asm__("" : "+v"(q));
+  return (uint32_t)uniform_i32((int)q);
+}
+
+// The byte offset of the lookup word of mesh dim I: of the consumer's class (byte I of `slots`), or `same` where the
+// placements (byte I of the codes) are equal.  Two instructions that select bytes, where a compiler masks, compares,
+// shifts and selects.  (s_nop 1: two cycles from a comparison's result to the select that reads it; the compiler does not look
+// inside an asm statement.)
+template <int I>
+__device__ __forceinline__ uint32_t word_slot(uint32_t src, uint32_t tgt, uint32_t slots, uint32_t same) {
+  uint32_t slot;
+#define APC_WORD_SLOT(BYTE_)                                                                                            \
+  __asm__("v_cmp_ne_u32_sdwa vcc, %1, %2 src0_sel:" BYTE_ " src1_sel:" BYTE_ "\n\ts_nop 1\n\t"                         \
+          "v_cndmask_b32_sdwa %0, %3, %4, vcc dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:" BYTE_       \
+          : "=v"(slot)                                                                                                  \
+          : "v"(src), "v"(tgt), "v"(same), "v"(slots)                                                                   \
+          : "vcc")
+  if constexpr (I == 0) APC_WORD_SLOT("BYTE_0");
+  else if constexpr (I == 1) APC_WORD_SLOT("BYTE_1");
+  else if constexpr (I == 2) APC_WORD_SLOT("BYTE_2");
+  else APC_WORD_SLOT("BYTE_3");
+#undef APC_WORD_SLOT
+  return slot;
+}
+template <int I, int M>
+__device__ __forceinline__ void word_slots(uint32_t src, uint32_t tgt, uint32_t slots, uint32_t (&out)[M]) {
+  out[I] = word_slot<I>(src, tgt, slots, (uint32_t)((kWordsPerDim * I + 4) * 4));  // (slot 4: same placement, nothing to add)
+  if constexpr (I + 1 < M) word_slots<I + 1>(src, tgt, slots, out);
+}
+
+// One entry of a tile whose producer specs all name one tensor.
+// What bounds a table of large tiles is the vector instructions of a SIMD, all of its cycles (20 M entries on (16, 8, 4): 27.9 M
+// instructions, 108 thousand of a SIMD's cycles in a launch of 101 thousand; LDS 73 % busy), so a pass of 64 entries counts them:
+// 40 on a 3-D mesh with the walk and the store (54 when columns, rows and loop were kept as numbers of a lane and the codes
+// compared by mask), and a tile's staging, which two wavefronts share, about 330 (430).  us a pass: 20 M on (16, 8, 4) 57.0 ->
+// 50.8, 5.3 M on (2, 4, 2, 2) 41.8 -> 39.4, 5.1 M on (3, 2, 2, 2) 53.2 -> 50.7, 2.6 M on (12, 6) 14.4 -> 13.4, 587 k on
+// (6, 4, 2) 16.0 -> 15.4.  (Every copy's address in scalar registers, one instruction less a store, is 1 % slower.)
 // Straight-line code: all lookups of an entry are independent of its fp additions, so they
 // are issued together; no vector memory loads.
-template <int M, bool CONT, bool RESCALE, bool RM>
-__device__ __forceinline__ void uniform_entry(const EntryConstants &k, const TileStage<M, RM> &st,
-                                              const char *terms, int r, int c, double &comm_o, double &total_o,
+template <int M, bool CONT, bool RESCALE>
+__device__ __forceinline__ void uniform_entry(const EntryConstants &k, lds_address terms, const TileWalk &where, double &comm_o, double &total_o,
                                               int &trans_o) {
-  const uint32_t src = st.col_codes[c];
-  const RowRecord row = st.row[r];
-  const uint32_t tgt = row.codes;
-  const uint32_t x = src ^ tgt;
-  const char *words = reinterpret_cast<const char *>(st.words) + __umul24((uint32_t)c, (M * kWordsPerDim + 1) * 4);
+  const uint32_t src = lds_read<uint32_t>(where.col + kCodesWord<M> * 4);
+  const u32x4 raw = lds_read<u32x4>(where.row);
+  const RowRecord row{raw.x, raw.y, __hiloint2double((int)raw.w, (int)raw.z)};
+  const uint32_t x = src ^ row.codes;
+  const bool differs = M == 2 ? (x & 0xFFFFu) != 0 : x != 0;
+  // (2-D: a (Partial, Partial) producer's shift takes the slots of its order flip)
+  const uint32_t slots = M == 2 ? row.slots >> (src >> 24) : row.slots;
   // ---- integer part: which term at which running index each mesh dim adds -------------------
   uint32_t at = 0;  // byte offset of the running index (history of the earlier dims / exponent steps), mod 2^32
-  const bool flip = M == 2 && src == 0x4040u && (row.slots >> 24) != 0u;  // dim 1 before dim 0 (flip_words)
-  uint32_t term_at[M], rw_at[M], nc_at[M];
-  bool neq[M];
+  uint32_t slot[M], term_at[M], rw_at[M], nc_at[M];
+  word_slots<0>(src, row.codes, slots, slot);
 #pragma unroll
   for (int i = 0; i < M; ++i) {
-    neq[i] = ((x >> (8 * i)) & 0xFF) != 0;
-    // (slot 4: same placement, nothing to add)
-    const uint32_t slot = neq[i] ? (row.slots >> (8 * i)) & 0xFFu : (uint32_t)((kWordsPerDim * i + 4) * 4);
-    const char *at_word = words + slot;
-    if (M == 2 && flip) at_word = reinterpret_cast<const char *>(st.flip_words) + ((row.slots >> (16 + 8 * i)) & 0xFFu);
-    const uint32_t w = *reinterpret_cast<const uint32_t *>(at_word);
+    const uint32_t w = lds_read<uint32_t>(where.col + slot[i]);
     term_at[i] = (w & 0xFFFFu) + at;
     rw_at[i] = term_at[i] + (uint32_t)(int32_t)(int8_t)(w >> 16);
-    if (!CONT) nc_at[i] = *reinterpret_cast<const uint32_t *>(words + (kWordsPerDim * i + 5) * 4) + at;
+    if (!CONT) nc_at[i] = lds_read<uint32_t>(where.col + (kWordsPerDim * i + 5) * 4) + at;
     at += (uint32_t)__mul24((int32_t)w >> 24, k.state_stride);  // (24-bit multiplies issue at full rate)
   }
   // ---- lookups ------------------------------------------------------------------------------
   double term[M], rw[M], nc[M];
 #pragma unroll
   for (int i = 0; i < M; ++i) {
-    term[i] = *reinterpret_cast<const double *>(terms + term_at[i]);
-    rw[i] = *reinterpret_cast<const double *>(terms + rw_at[i]);
-    if (!CONT) nc[i] = *reinterpret_cast<const double *>(terms + nc_at[i]);
+    term[i] = lds_read<double>(terms + term_at[i]);
+    rw[i] = lds_read<double>(terms + rw_at[i]);
+    if (!CONT) nc[i] = lds_read<double>(terms + nc_at[i]);
   }
   // ---- additions in the reference's order (0.0 + t == t for these non-negative terms) ------------
   double cost = 0.0;
@@ -1332,20 +1461,21 @@ __device__ __forceinline__ void uniform_entry(const EntryConstants &k, const Til
 #pragma unroll
   for (int i = 0; i < M; ++i) {
     if (!CONT) {
-      cost += (neq[i] && !cont) ? nc[i] : 0.0;
-      cont = cont || neq[i];
+      const bool neq = ((x >> (8 * i)) & 0xFF) != 0;
+      cost += (neq && !cont) ? nc[i] : 0.0;
+      cont = cont || neq;
     }
     if (CONT && i == 0) cost = term[0];
     else cost += term[i];
     cost += rw[i];  // 0, 1 or 2 read+writes: (double)copies * rw, picked from the staged multiples
   }
   double comm = cost;  // (a banned transition added the +inf term)
-  const int trans = x != 0u ? k.transition_scale : 0;  // optimize_sharding.py:345-351
   // :358-359; the quotient through the reciprocal is the division's (div_by), +inf stays +inf
   if (RESCALE) comm = comm < __builtin_inf() ? div_by(comm, k.rescale, k.inv_rescale) : comm;
   comm_o = comm;
-  total_o = comm + row.cpa + (double)trans;  // :368-372
-  trans_o = trans;
+  // :345-351, :368-372
+  total_o = comm + row.cpa + (differs ? k.transition : 0.0);
+  trans_o = differs ? k.transition_scale : 0;
 }
 
 // The three output streams of one tile: wave-uniform bases, so an entry's addresses are a
@@ -1365,27 +1495,30 @@ struct TileOut {
 // is checked per store.
 enum : int { kOutAny = 0, kOutAll = 1, kOutCost = 2 };
 
-// Stores one entry's values to its edge and to every identical edge.  Called by every lane of
+// Evaluates one entry and stores its values to its edge and to every identical edge; -> its assembled cost.  Called by every lane of
 // the wavefront (`active`: this lane holds an entry), so that the copies' offsets are read from
 // their lanes under uniform control flow.
 template <int OUT>
-__device__ __forceinline__ void store_entry(const TileOut &o, int dup_count, const TileCopies &copies, bool active,
-                                            uint32_t local, double comm, double total, int trans) {
+__device__ __forceinline__ void store_values(const TileOut &o, int64_t delta, uint32_t off8, double comm, double total, int trans) {
   constexpr bool ALL = OUT == kOutAll, COST = OUT == kOutCost;
-  const uint32_t off8 = local * 8u;
+  if (ALL || (!COST && o.comm)) *reinterpret_cast<double *>(reinterpret_cast<char *>(o.comm + delta) + off8) = comm;
+  if (ALL || (!COST && o.trans)) (o.trans + delta)[off8 / 8u] = (uint8_t)trans;
+  if (ALL || COST || o.cost) *reinterpret_cast<double *>(reinterpret_cast<char *>(o.cost + delta) + off8) = total;
+}
+template <int OUT, typename Entry>
+__device__ __forceinline__ double store_entry(const TileOut &o, int dup_count, const TileCopies &copies, bool active, const TileWalk &where,
+                                              Entry entry) {
+  double comm, total;
+  int trans;
   if (active) {
-    if (ALL || (!COST && o.comm)) *reinterpret_cast<double *>(reinterpret_cast<char *>(o.comm) + off8) = comm;
-    if (ALL || (!COST && o.trans)) o.trans[local] = (uint8_t)trans;
-    if (ALL || COST || o.cost) *reinterpret_cast<double *>(reinterpret_cast<char *>(o.cost) + off8) = total;
+    entry(where, comm, total, trans);
+    store_values<OUT>(o, 0, where.out, comm, total, trans);
   }
   for (int d = 0; d < dup_count; ++d) {
     const int64_t delta = value_of_lane(copies.entry0, d) - o.entry_begin;
-    if (active) {
-      if (ALL || (!COST && o.comm)) *reinterpret_cast<double *>(reinterpret_cast<char *>(o.comm + delta) + off8) = comm;
-      if (ALL || (!COST && o.trans)) (o.trans + delta)[local] = (uint8_t)trans;
-      if (ALL || COST || o.cost) *reinterpret_cast<double *>(reinterpret_cast<char *>(o.cost + delta) + off8) = total;
-    }
+    if (active) store_values<OUT>(o, delta, where.out, comm, total, trans);
   }
+  return total;
 }
 
 // A 32-bit value from the lane `N` further on within the lane's row of 16 (DPP row_shl:N); a
@@ -1464,7 +1597,7 @@ __device__ __forceinline__ void lower_of_lanes(double &m, int &mc) {
   const int lo = __double2loint(m), hi = __double2hiint(m);
   const double om = __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false), __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false));
   const int oc = __builtin_amdgcn_update_dpp(mc, mc, CTRL, 0xF, 0xF, false);
-  const bool take = om < m || (om == m && oc < mc);
+  const bool take = (om < m) | ((om == m) & (oc < mc));
   m = take ? om : m;
   mc = take ? oc : mc;
 }
@@ -1473,41 +1606,44 @@ __device__ __forceinline__ void lower_of_lanes(double &m, int &mc) {
 // time: 64 consecutive entries a pass, evaluated (`entry`), stored, and kept in the wavefront's LDS; then 1 to 16 lanes a
 // row read it back, the lanes of a row the columns in turn, and join their minima.  The rows of a wavefront need no
 // barrier, and a value costs one write and one read of 8 bytes where a minimum taken across the lanes of every pass
-// (neighbours in doubling distances, value and column) was 70 vector instructions a pass, more than the entry's own 45.
+// (neighbours in doubling distances, value and column) was 70 vector instructions a pass, more than the entry's own.
 // kRowMinValues = 512, 384, 256: 38.7, 40.3, 41.5 us for 6.1 M entries on (64, 4), by passes 50.4, without the minima 27.4
 // (its rows' stores are 0.6 of that).
-template <int OUT, typename Entry>
-__device__ __forceinline__ void tile_entries_row_min(const TableArgs &a, double *values, const TileView &v, const TileCopies &copies,
+template <int M, int OUT, typename Entry>
+__device__ __forceinline__ void tile_entries_row_min(const TableArgs &a, lds_address stage, const TileView &v, const TileCopies &copies,
                                                      int tid, int nthreads, Entry entry) {
   const int lane = tid & 63, wave = uniform_i32(tid >> 6), waves = nthreads >> 6;
-  const int cols = v.cols, stride = cols | 1;  // (odd: the lanes of consecutive rows read different banks)
-  const int at_once = min(kRowMinValues / stride, 64);
-  const int r0 = lane / cols, c0 = lane - r0 * cols, dr = 64 / cols, dc = 64 - dr * cols;
-  const int row_begin = v.rows * wave / waves, row_end = v.rows * (wave + 1) / waves;
+  constexpr bool RM = true;
+  const lds_address values = stage + terms_at<M, RM>() + (uint32_t)kWaveScratchBytes<RM> * (uint32_t)wave;  // (wave_scratch)
+  const int cols = v.cols;
+  // bytes from row to row: an odd number of doubles, so that the lanes of consecutive rows read different banks
+  const uint32_t row_bytes = (uint32_t)(cols | 1) * 8u;
+  const float inv_cols = __builtin_amdgcn_rcpf((float)cols);
+  const int at_once = min((int)uniform_quotient(kRowMinValues, __builtin_amdgcn_rcpf((float)(cols | 1))), 64);
+  const int r0 = (int)small_quotient((uint32_t)lane, inv_cols), c0 = lane - __mul24(r0, cols);
+  const uint32_t dr = uniform_quotient(64, inv_cols), dc = 64u - dr * (uint32_t)cols;
+  const TileSteps steps = tile_steps<M, RM>(stage, dr, dc, (uint32_t)cols, (uint32_t)cols);
+  const int row_begin = (int)((uint32_t)(v.rows * wave) / (uint32_t)waves), row_end = (int)((uint32_t)(v.rows * (wave + 1)) / (uint32_t)waves);
   const int64_t tile_base = v.entry_begin + (int64_t)v.row_begin * v.n_src + v.col_begin;
   const TileOut out{a.comm_out ? a.comm_out + tile_base : nullptr, a.trans_out ? a.trans_out + tile_base : nullptr,
                     a.cost_out ? a.cost_out + tile_base : nullptr, v.entry_begin};
+  // a value's place in `values`: its place in the output and, where the rows are padded, 8 bytes a row
+  const uint32_t pad = (cols & 1) ? 31u : 1u;  // (a record of 16 bytes a row)
   for (int first = row_begin; first < row_end; first += at_once) {
     const int rows = min(at_once, row_end - first), n = rows * cols;
-    for (int at = 0, r = r0, c = c0; at < n; at += 64) {
+    TileWalk w = tile_walk<M, RM>(stage, first + r0, c0, cols);
+    const uint32_t to_values = values - (uint32_t)(first * cols) * 8u - ((stage + rows_at<M, RM>() + (uint32_t)first * 16u) >> pad);
+    for (int at = 0; at < n; at += 64) {
       const bool active = at + lane < n;
-      double comm = 0.0, total = 0.0;
-      int trans = 0;
-      if (active) entry(first + r, c, comm, total, trans);
-      store_entry<OUT>(out, v.dup_count, copies, active, __umul24((uint32_t)(first + r), (uint32_t)v.n_src) + (uint32_t)c, comm, total, trans);
-      if (active) values[__mul24(r, stride) + c] = total;
-      c += dc;
-      r += dr;
-      if (c >= cols) {
-        c -= cols;
-        r += 1;
-      }
+      const double total = store_entry<OUT>(out, v.dup_count, copies, active, w, entry);
+      if (active) lds_write(w.out + (w.row >> pad) + to_values, total);
+      advance<true>(w, steps);
     }
     __builtin_amdgcn_wave_barrier();  // (LDS operations of one wavefront complete in order)
     const int shift = rows <= 4 ? 4 : rows <= 8 ? 3 : rows <= 16 ? 2 : rows <= 32 ? 1 : 0;  // 2^shift lanes a row
     const int lanes = 1 << shift, row = lane >> shift, sub = lane & (lanes - 1);
-    const double *line = values + __mul24(min(row, rows - 1), stride);
-    const double head = line[0];
+    const lds_address line = values + (uint32_t)__umul24((uint32_t)min(row, rows - 1), row_bytes);
+    const double head = lds_read<double>(line);
     double m = __builtin_inf();
     int mc = 0;
     for (int y = sub; y < cols; y += 4 * lanes) {
@@ -1516,7 +1652,7 @@ __device__ __forceinline__ void tile_entries_row_min(const TableArgs &a, double 
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         at[u] = min(y + u * lanes, cols - 1);  // (past the row's end: its last value once more)
-        value[u] = line[at[u]];
+        value[u] = lds_read<double>(line + (uint32_t)at[u] * 8u);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u)
@@ -1552,54 +1688,45 @@ __device__ __forceinline__ void tile_entries_row_min(const TableArgs &a, double 
   }
 }
 
-// The per-entry loop of such a tile for `nthreads` threads (this one is `tid`): a flattened
+// The per-entry loop of a tile for `nthreads` threads (this one is `tid`): a flattened
 // (row, column) walk, so a wavefront writes 64 consecutive entries.
-template <int M, bool CONT, bool RESCALE, int OUT, bool RM>
-__device__ __forceinline__ void uniform_tile_entries(const apc_params &p, const TableArgs &a, const TileStage<M, RM> &st,
-                                                     const TileView &v, const TileCopies &copies, int tid, int nthreads) {
+// A full-width tile (WHOLE) is one contiguous run of entries: lanes are shifted so that every
+// wavefront store starts on a 64-entry boundary of the output arrays (whole 128-byte lines
+// of the fp64 streams) instead of straddling one more line than it fills.  Every lane of a
+// wavefront makes the same number of passes (a lane in front of the tile's first entry idles
+// in the first one), so the copies' offsets are read under uniform control flow.
+template <int M, int OUT, bool WHOLE, bool RM, typename Entry>
+__device__ __forceinline__ void tile_entries_walk(const TableArgs &a, lds_address stage, const TileView &v, const TileCopies &copies,
+                                                  int tid, int nthreads, Entry entry) {
   const int n = v.rows * v.cols;
-  const int dr = nthreads / v.cols, dc = nthreads - dr * v.cols;
+  const float inv_cols = __builtin_amdgcn_rcpf((float)v.cols);
+  const uint32_t dr = uniform_quotient((uint32_t)nthreads, inv_cols), dc = (uint32_t)nthreads - dr * (uint32_t)v.cols;
+  const int n_src = WHOLE ? v.cols : v.n_src;
+  const TileSteps steps = tile_steps<M, RM>(stage, dr, dc, (uint32_t)v.cols, (uint32_t)n_src);
   const int64_t tile_base = v.entry_begin + (int64_t)v.row_begin * v.n_src + v.col_begin;
-  // A full-width tile is one contiguous run of entries: lanes are shifted so that every
-  // wavefront store starts on a 64-entry boundary of the output arrays (whole 128-byte lines
-  // of the fp64 streams) instead of straddling one more line than it fills.  Every lane of a
-  // wavefront makes the same number of passes (a lane in front of the tile's first entry idles
-  // in the first one), so the copies' offsets are read under uniform control flow.
-  const int shift = v.cols == v.n_src ? (int)(tile_base & 63) : 0;
+  const int shift = WHOLE ? (int)(tile_base & 63) : 0;
   const int lane = tid & 63;
-  int idx = tid - shift;
-  const int first = idx < 0 ? idx + nthreads : idx;
-  int r = first / v.cols, c = first - r * v.cols;
+  // (in front of the tile's first entry rows count backwards: 64 rows are more than the shift)
+  const int r = (int)small_quotient((uint32_t)(tid - shift + 64 * v.cols), inv_cols) - 64;
+  TileWalk w = tile_walk<M, RM>(stage, r, tid - shift - __mul24(r, v.cols), n_src);
   const TileOut out{a.comm_out ? a.comm_out + tile_base : nullptr, a.trans_out ? a.trans_out + tile_base : nullptr,
                     a.cost_out ? a.cost_out + tile_base : nullptr, v.entry_begin};
-  const EntryConstants k = entry_constants(p, a.lay);
-  for (int wave_first = tid - lane - shift; wave_first < n; wave_first += nthreads, idx += nthreads) {
-    const bool active = idx >= 0 && idx < n;
-    double comm = 0.0, total = 0.0;
-    int trans = 0;
-    if (active) uniform_entry<M, CONT, RESCALE>(k, st, term_base(st, nthreads), r, c, comm, total, trans);
-    store_entry<OUT>(out, v.dup_count, copies, active, __umul24((uint32_t)r, (uint32_t)v.n_src) + (uint32_t)c, comm, total,
-                     trans);
-    if (active) {
-      c += dc;
-      r += dr;
-      if (c >= v.cols) {
-        c -= v.cols;
-        r += 1;
-      }
-    }
+  for (int at = uniform_i32(tid - lane) - shift; at < n; at += nthreads) {
+    store_entry<OUT>(out, v.dup_count, copies, (uint32_t)(at + lane) < (uint32_t)n, w, entry);
+    advance<WHOLE>(w, steps);
   }
 }
 
-// The generic entry: pass-through edges and edges whose producer specs name different tensors (`local`: the entry's
-// place in its edge's matrix).
+// The generic entry: pass-through edges and edges whose producer specs name different tensors.
 template <int M, bool DERIVE, bool RM>
-__device__ __forceinline__ void generic_entry(const apc_params &p, const TableArgs &a, const TileStage<M, RM> &st, const TileView &v,
-                                              int r, int c, double &comm, double &total, int &trans) {
+__device__ __forceinline__ void generic_entry(const apc_params &p, const TableArgs &a, const TileStage<M, RM> &st, lds_address stage, const TileView &v,
+                                              const TileWalk &where, double &comm, double &total, int &trans) {
+  const int r = (int)((where.row - stage - rows_at<M, RM>()) / 16u), c = (int)((where.col - stage - words_at<M, RM>()) / (uint32_t)(kColWords<M> * 4));
   const int64_t local = (int64_t)(v.row_begin + r) * v.n_src + (v.col_begin + c);
   const uint32_t src = st.colh[c].x, cinfo = st.colh[c].y;
   const RowRecord row = st.row[r];
   const uint32_t tgt = row.codes;
+  trans = 0;
   if ((v.flags & APC_EDGE_NO_PRODUCER) || !(cinfo & 1u) || (row.slots & 0xFFu) == kRowNotASpec) {
     comm = a.pt_values[v.pt_begin + local];
   } else {
@@ -1619,70 +1746,38 @@ __device__ __forceinline__ void generic_entry(const apc_params &p, const TableAr
   total = comm + row.cpa + (double)trans;
 }
 
-// Their loop: every lane of a wavefront makes the same number of passes.
-template <int M, bool DERIVE, bool RM>
-__device__ __forceinline__ void generic_tile_entries(const apc_params &p, const TableArgs &a, const TileStage<M, RM> &st, const TileView &v,
-                                                     const TileCopies &copies, int tid, int nthreads) {
-  const int n = v.rows * v.cols;
-  const int lane = tid & 63;
-  int r = tid / v.cols, c = tid - r * v.cols;
-  const int dr = nthreads / v.cols, dc = nthreads - dr * v.cols;
-  const int64_t tile_base = v.entry_begin + (int64_t)v.row_begin * v.n_src + v.col_begin;
-  const TileOut out{a.comm_out ? a.comm_out + tile_base : nullptr, a.trans_out ? a.trans_out + tile_base : nullptr,
-                    a.cost_out ? a.cost_out + tile_base : nullptr, v.entry_begin};
-  for (int idx = tid; idx - lane < n; idx += nthreads) {
-    const bool active = idx < n;
-    double total = 0.0, comm = 0.0;
-    int trans = 0;
-    if (active) generic_entry<M, DERIVE>(p, a, st, v, r, c, comm, total, trans);
-    store_entry<kOutAny>(out, v.dup_count, copies, active, __umul24((uint32_t)r, (uint32_t)v.n_src) + (uint32_t)c, comm, total, trans);
-    if (active) {
-      c += dc;
-      r += dr;
-      if (c >= v.cols) {
-        c -= v.cols;
-        r += 1;
-      }
-    }
-  }
-}
-
 // All entries of a staged tile.  Row minima are taken when the caller wants them and the tile
 // holds whole rows (which the host arranges for every tile of a table before asking).
 template <int M, bool DERIVE, bool RM, int OUT>
-__device__ __forceinline__ void tile_entries(const apc_params &p, const TableArgs &a, TileStage<M, RM> &st,
+__device__ __forceinline__ void tile_entries(const apc_params &p, const TableArgs &a, const TileStage<M, RM> &st, lds_address stage,
                                              const TileView &v, const TileCopies &copies, int tid, int nthreads) {
   int mixed = st.mixed[0];
   for (int w = 1; w < nthreads / 64; ++w) mixed |= st.mixed[w];
-  const bool row_minima = RM && v.cols == v.n_src;
-  double *const values = reinterpret_cast<double *>(wave_scratch(st, uniform_i32(tid >> 6)));
-  if (uniform_i32(mixed)) {
+  const bool whole = v.cols == v.n_src, row_minima = RM && whole;
+  const auto entries = [&](auto out, auto entry) {
+    constexpr int kOut = decltype(out)::value;
     if constexpr (RM) {
       if (row_minima) {
-        tile_entries_row_min<kOutAny>(a, values, v, copies, tid, nthreads, [&](int r, int c, double &comm, double &total, int &trans) {
-          generic_entry<M, DERIVE>(p, a, st, v, r, c, comm, total, trans);
-        });
+        tile_entries_row_min<M, kOut>(a, stage, v, copies, tid, nthreads, entry);
         return;
       }
     }
-    generic_tile_entries<M, DERIVE>(p, a, st, v, copies, tid, nthreads);
+    if (whole) tile_entries_walk<M, kOut, true, RM>(a, stage, v, copies, tid, nthreads, entry);
+    else tile_entries_walk<M, kOut, false, RM>(a, stage, v, copies, tid, nthreads, entry);
+  };
+  if (uniform_i32(mixed)) {
+    entries(std::integral_constant<int, kOutAny>{}, [&](const TileWalk &where, double &comm, double &total, int &trans) {
+      generic_entry<M, DERIVE>(p, a, st, stage, v, where, comm, total, trans);
+    });
     return;
   }
   const bool rescale = (v.flags & APC_EDGE_GRAD_RESCALE) != 0;
-#define APC_TILE_LOOP(CONT_, RESCALE_)                                                                                                    \
-  do {                                                                                                                                    \
-    if constexpr (RM) {                                                                                                                   \
-      if (row_minima) {                                                                                                                   \
-        const EntryConstants k = entry_constants(p, a.lay);                                                                               \
-        const char *const terms = term_base(st, nthreads);                                                                                \
-        tile_entries_row_min<OUT>(a, values, v, copies, tid, nthreads, [&](int r, int c, double &comm, double &total, int &trans) {       \
-          uniform_entry<M, CONT_, RESCALE_>(k, st, terms, r, c, comm, total, trans);                                                      \
-        });                                                                                                                               \
-        break;                                                                                                                            \
-      }                                                                                                                                   \
-    }                                                                                                                                     \
-    uniform_tile_entries<M, CONT_, RESCALE_, OUT>(p, a, st, v, copies, tid, nthreads);                                                    \
-  } while (0)
+  const EntryConstants k = entry_constants(p, a.lay);
+  const lds_address terms = stage + terms_at<M, RM>() + (uint32_t)kWaveScratchBytes<RM> * (uint32_t)(nthreads >> 6);  // (term_base)
+#define APC_TILE_LOOP(CONT_, RESCALE_)                                                                                       \
+  entries(std::integral_constant<int, OUT>{}, [&](const TileWalk &where, double &comm, double &total, int &trans) {          \
+    uniform_entry<M, CONT_, RESCALE_>(k, terms, where, comm, total, trans);                                                  \
+  })
   if (uniform_i32(st.cont)) {
     if (rescale) { APC_TILE_LOOP(true, true); } else { APC_TILE_LOOP(true, false); }
   } else {
@@ -1723,7 +1818,7 @@ __device__ __forceinline__ apc_tile fetch_tile(const apc_tile *tiles, int64_t ti
 
 template <int M, int kTileThreads, bool RM, int OUT>
 __device__ __forceinline__ void redistribute_tile(const apc_params &p, const TableArgs &a, const apc_tile *tiles, int n_tiles,
-                                                  int xcd_shift, TileStage<M, RM> &stage) {
+                                                  int xcd_shift, TileStage<M, RM> &stage, lds_address at) {
   const int tile_id = tile_of_block((int)blockIdx.x, n_tiles, xcd_shift);
   if (tile_id >= n_tiles) return;
   static_assert(kTileThreads == 64 || kTileThreads == 128 || kTileThreads == 256, "wavefronts per tile: 1, 2 or 4");
@@ -1736,7 +1831,7 @@ __device__ __forceinline__ void redistribute_tile(const apc_params &p, const Tab
   stage_tile<M, false, RM>(p, a, tile, stage, threadIdx.x, kTileThreads, copies);
   settle(copies);
   __syncthreads();
-  tile_entries<M, false, RM, OUT>(p, a, stage, view_of(tile), copies, threadIdx.x, kTileThreads);
+  tile_entries<M, false, RM, OUT>(p, a, stage, at, view_of(tile), copies, threadIdx.x, kTileThreads);
 }
 
 // Wavefronts per SIMD the tile kernels ask for: what the LDS of their larger, row-minimum
@@ -1748,9 +1843,9 @@ __device__ __forceinline__ void redistribute_tile(const apc_params &p, const Tab
 constexpr int tile_waves_per_simd(int mesh_ndim, int threads, bool row_min) {
   if (mesh_ndim >= 4) return threads >= 256 ? 4 : threads >= 128 ? 3 : 2;
   if (threads < 128) return mesh_ndim <= 1 ? 7 : mesh_ndim == 2 ? 6 : 4;
-  // two-wavefront tiles without the minima fit sixteen to a compute unit (under 10 KB of LDS
-  // each on a power-of-two mesh): all eight wavefront slots of a SIMD, 64 registers
-  return threads == 128 && !row_min ? 8 : 7;
+  // (Asked for eight, the compiler allows itself 78 scalar registers instead of 94, and spills; with the 53 vector
+  // registers that it takes, eight fit all the same.)
+  return 7;
 }
 
 struct TilesBlock {
@@ -1764,7 +1859,7 @@ void redistribute_tiles_kernel(APC_LAUNCH_PARAMS(TilesBlock)) {
   extern __shared__ __align__(16) unsigned char s_stage_bytes[];  // stage_lds_bytes<M, false>
   const TilesBlock &k = launch_block(kept);
   redistribute_tile<M, kTileThreads, false, OUT>(k.p, k.a, static_cast<const apc_tile *>(work), n_tiles, xcd_shift,
-                                                 *reinterpret_cast<TileStage<M, false> *>(s_stage_bytes));
+                                                 *reinterpret_cast<TileStage<M, false> *>(s_stage_bytes), address_in_lds(s_stage_bytes));
 }
 
 // The same with the row minima.
@@ -1775,7 +1870,7 @@ void redistribute_tiles_row_min_kernel(APC_LAUNCH_PARAMS(TilesBlock)) {
   extern __shared__ __align__(16) unsigned char s_stage_bytes[];  // stage_lds_bytes<M, true>
   const TilesBlock &k = launch_block(kept);
   redistribute_tile<M, kTileThreads, true, OUT>(k.p, k.a, static_cast<const apc_tile *>(work), n_tiles, xcd_shift,
-                                                *reinterpret_cast<TileStage<M, true> *>(s_stage_bytes));
+                                                *reinterpret_cast<TileStage<M, true> *>(s_stage_bytes), address_in_lds(s_stage_bytes));
 }
 
 // Every table of a pass in one launch: workgroups [0, tile_blocks) take the tiles of the
@@ -1789,10 +1884,8 @@ void redistribute_tiles_row_min_kernel(APC_LAUNCH_PARAMS(TilesBlock)) {
 // (On 3-D and 4-D meshes LDS is sized per launch for the layout in use: with the general layout's share held for every mesh, a
 // workgroup of a 4-D launch held 45 KB of which a power-of-two mesh uses 10.  6.4 M entries on (2, 4, 2, 2) 46.2 -> 32.9 us,
 // 9.4 M on (16, 8, 4) 64.6 -> 59.1, 901 k on (8, 8, 8) 14.9 -> 13.8.)
-// (Wavefronts per SIMD are capped at 5 on 1-D and 2-D meshes: with more resident, the launch's
-// many store streams hinder each other a little.  Llama-3-8B table, each pair on one box:
-// 18.5 us against 18.9 us uncapped, 18.7 us against 18.8 us on another box; capped at 6 as
-// uncapped; 20.3 us capped at 3 or when asked for 8.  The mixture-of-experts table: no change.)
+// (On 1-D and 2-D meshes seven wavefronts per SIMD are asked for, what 72 vector registers leave room for: 7.6 M entries on (32, 8),
+// 59 layers, 17.0 us with 5, 16.4 with 7, 2.6 M on (12, 6) 13.4 / 13.2, 6.1 M on (64, 4) with the minima the same.)
 // (1-D and 2-D meshes hold the larger layout's share in a static array: sized per launch, what a 2-D launch does takes 2 %
 // longer, 18.3 -> 18.7 us for 2.6 M entries on (12, 6), also with the same bytes asked for.)
 template <int M, bool RM>
@@ -1827,7 +1920,7 @@ struct BuildTablesBlock {
 };
 
 template <int M, int kThreads, bool RM, int OUT>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(M <= 2 ? 5 : 1, M <= 2 ? 5 : 8)))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(M <= 2 ? 7 : 1, 8)))
 void build_tables_kernel(APC_LAUNCH_PARAMS(BuildTablesBlock)) {
   const BuildTablesBlock &k = launch_block(kept);
   const apc_params &p = k.p;
@@ -1846,7 +1939,7 @@ void build_tables_kernel(APC_LAUNCH_PARAMS(BuildTablesBlock)) {
     stage_tile<M, true, RM>(p, a, tile, stage, threadIdx.x, kThreads, copies);
     settle(copies);
     __syncthreads();
-    tile_entries<M, true, RM, OUT>(p, a, stage, view_of(tile), copies, threadIdx.x, kThreads);
+    tile_entries<M, true, RM, OUT>(p, a, stage, address_in_lds(s_raw), view_of(tile), copies, threadIdx.x, kThreads);
     return;
   }
   const int64_t tb = b - tile_blocks;
