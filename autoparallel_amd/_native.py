@@ -96,6 +96,7 @@ EXPORTS = (
     "apc_edge_classes_host",
     "apc_count_tiles_host",
     "apc_fill_tiles_host",
+    "apc_order_tiles_host",
     "apc_tile_records_host",
     "apc_validate_tiling_host",
     "apc_label_incidence_host",

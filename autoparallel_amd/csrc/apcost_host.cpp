@@ -300,6 +300,37 @@ int apc_fill_tiles_host(int64_t n_edges, const int32_t *edge_n_src, const int32_
   return thrown("apc_fill_tiles_host");
 }
 
+int apc_order_tiles_host(int64_t n_tiles, const apc_tile *records, apc_tile *ordered) try {
+  if (n_tiles < 0) return fail(-1, "apc_order_tiles_host: negative count");
+  if (n_tiles > 0 && (!records || !ordered)) return fail(-1, "apc_order_tiles_host: NULL array");
+  // by counting: first the rank of the first tile of every size (a record that the validator would refuse counts as the largest)
+  constexpr int kMost = APC_TILE_MAX_ROWS * APC_TILE_MAX_COLS;
+  const auto size = [](const apc_tile &t) {
+    const uint32_t n = (uint32_t)(t.counts & 0xFFFF) * (uint32_t)(t.counts >> 16);
+    return n <= (uint32_t)kMost ? (int)n : kMost;
+  };
+  std::vector<uint64_t> next(kMost + 2, 0);
+  for (int64_t t = 0; t < n_tiles; ++t) ++next[kMost - size(records[t]) + 1];
+  for (int s = 0; s <= kMost; ++s) next[s + 1] += next[s];
+  // rank k is tile k / 8 of die k mod 8: where that one is in the launch's order (tile_of_block in apcost.hip)
+  constexpr uint64_t kDies = 8, kRound = kDies * APC_TILE_RUN;
+  const uint64_t full = (uint64_t)n_tiles / kRound * kRound, rest = (uint64_t)n_tiles - full, per = (rest + kDies - 1) / kDies;
+  // (the last, incomplete round: `whole` dies take `per` tiles each, one the `left` others)
+  const uint64_t whole = per > 0 ? rest / per : 0, left = rest - whole * per, dies = whole + (left > 0 ? 1 : 0);
+  for (int64_t t = 0; t < n_tiles; ++t) {
+    const uint64_t k = next[kMost - size(records[t])]++;
+    const uint64_t within = k < full ? k % kRound : k - full;
+    uint64_t at;
+    if (k < full) at = k - within + within % kDies * APC_TILE_RUN + within / kDies;
+    else if (within < left * dies) at = full + within % dies * per + within / dies;
+    else at = full + (within - left * dies) % whole * per + left + (within - left * dies) / whole;
+    ordered[at] = records[t];
+  }
+  return 0;
+} catch (...) {
+  return thrown("apc_order_tiles_host");
+}
+
 int apc_tile_records_host(int64_t n_specs, const int32_t *spec_tensor, int64_t n_edges, const int32_t *edge_src_begin,
                           const int32_t *edge_n_src, const int32_t *edge_tgt_begin, const int32_t *edge_flags,
                           const int64_t *edge_pt_begin, const int64_t *edge_entry_begin, const int32_t *edge_strat_begin,

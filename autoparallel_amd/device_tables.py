@@ -180,7 +180,7 @@ class DeviceCostTables:
         self.transition = self._empty((n,), torch.uint8) if transition else None
         self.cost = self._empty((n,), torch.float64) if cost else None
 
-    def _bind_redistribute_tables(self, comm, transition, cost, rows=None):
+    def _bind_redistribute_tables(self, comm, transition, cost, rows=None, repeated=False):
         """A bound launch of the table kernel over the tables already built, writing the given
         per-entry arrays (None: not written) and, with ``rows = (edge_row_begin, row_min,
         row_argmin)``, the row minima."""
@@ -188,7 +188,7 @@ class DeviceCostTables:
         erb, rmin, rarg = rows if rows is not None else (None, None, None)
         return self.ops.bind_redistribute_tables(
             self.p, self.tensor_bytes, self.tensor_contiguous, d["spec_codes"], d["spec_tensor"], d["pt_values"],
-            self.compute_cost_per_arg, d["tile_records"], d["dup_entry_begin"], self.tables.n_entries, comm, transition, cost,
+            self.compute_cost_per_arg, self._tile_records(repeated), d["dup_entry_begin"], self.tables.n_entries, comm, transition, cost,
             erb, d["dup_row_begin"] if rows is not None else None, rmin, rarg)
 
     @_guarded
@@ -296,14 +296,29 @@ class DeviceCostTables:
         tb = self.tables
         return tb.n_entries <= self.PACKED_MAX_ENTRIES and tb.packable()
 
-    def _packed_tiles(self):
-        """The device copy of ``CostTables.pack_tiles()``, made once per tiling."""
+    def _packed_tiles(self, repeated):
+        """The device copy of ``CostTables.pack_tiles()``, made once per tiling; in launch order for a pass that is repeated
+        (the order costs the host more than it saves one launch)."""
         cached = getattr(self, "_packed_cache", None)
-        if cached is not None and cached[0] is self.tables.tile_records:
-            return cached[1]
-        dev = _to_device(self.tables.pack_tiles(), self.device)
-        self._packed_cache = (self.tables.tile_records, dev)
+        if cached is not None and cached[0] is self.tables.tile_records and cached[1] == repeated:
+            return cached[2]
+        dev = _to_device(self.tables.pack_tiles(self.tables.launch_records() if repeated else None), self.device)
+        self._packed_cache = (self.tables.tile_records, repeated, dev)
         return dev
+
+    def _tile_records(self, repeated):
+        """The device copy of the tile records, in launch order for a pass that is repeated."""
+        tb = self.tables
+        if not repeated:
+            return self.d["tile_records"]
+        cached = getattr(self, "_ordered_cache", None)
+        if cached is None or cached[0] is not tb.tile_records or cached[1] is not self.d["tile_records"]:
+            records = tb.launch_records()
+            on_device = self.d["tile_records"]
+            if records is not tb.tile_records:
+                on_device = _to_device(records, self.device)
+            cached = self._ordered_cache = (tb.tile_records, self.d["tile_records"], on_device)
+        return cached[2]
 
     @_guarded
     def prepare_step(self, row_min=True, fused_inputs=False, one_launch=None, row_min_in_tiles=None,
@@ -324,7 +339,8 @@ class DeviceCostTables:
         (``apc_build_tables_packed``: the assembled cost and the row minima, no spec table);
         ``None`` takes them when the pass is of that kind, ``packed_pass_pays`` and staged tiles
         (``CostTables.staging_pays``) are not faster still.  ``repeated=False``: the pass will run once, and the arguments
-        of its launches are not laid out in device memory first (``apc_kept_launch``: one copy, for 2 to 4 us less a launch)."""
+        of its launches are not laid out in device memory first (``apc_kept_launch``: one copy, for 2 to 4 us less a launch),
+        nor its tiles put into launch order (``CostTables.launch_records``: 10 ns a tile on the host)."""
         tb = self.tables
         outputs = tuple(outputs)
         if not outputs or any(o not in ("comm", "transition", "cost") for o in outputs):
@@ -386,11 +402,11 @@ class DeviceCostTables:
         if packed:
             step = {"build_tables_packed": bind(ops.bind_cost_tables_packed(
                 self.p, *self._tensor_table(), self.tensor_bytes, self.tensor_contiguous, *self._strategy_table(),
-                self.compute_cost, self.compute_cost_per_arg, err, d["pt_values"], self._packed_tiles(), tb.n_entries, tb.n_rows,
+                self.compute_cost, self.compute_cost_per_arg, err, d["pt_values"], self._packed_tiles(bool(repeated)), tb.n_entries, tb.n_rows,
                 self.cost, self.row_min, self.row_argmin))}
         elif one_launch:
             step = {"build_tables": bind(ops.bind_cost_tables(
-                *input_tables, d["pt_values"], d["tile_records"], d["dup_entry_begin"], tb.n_entries, self.comm,
+                *input_tables, d["pt_values"], self._tile_records(repeated), d["dup_entry_begin"], tb.n_entries, self.comm,
                 self.transition, self.cost, erb, dup_rows, rmin, rarg))}
         elif fused_inputs:
             step = {"input_tables": bind(ops.bind_input_tables(*input_tables))}
@@ -404,7 +420,7 @@ class DeviceCostTables:
                                                              self.compute_cost_per_arg, err)),
             }
         if not one_launch and not packed:
-            step["redistribute_tables"] = bind(self._bind_redistribute_tables(self.comm, self.transition, self.cost, rows))
+            step["redistribute_tables"] = bind(self._bind_redistribute_tables(self.comm, self.transition, self.cost, rows, repeated))
         if row_min and not row_min_in_tiles:
             row_ptr = _to_device(tb.row_ptr(), self.device)
             assert row_ptr.numel() - 1 == self.row_min.numel()

@@ -67,6 +67,17 @@ AUTO_MIN_TILE_ENTRIES = 512
 AUTO_MIN_STORED_PER_TILE = 800
 AUTO_MAX_STORED_PER_TILE = 4000
 AUTO_MANY_TILES = 100_000
+# Tiles in the order of their size, the largest first: the launch ends with short workgroups instead of whichever edge is
+# last.  Neighbouring tiles then meet a line of the output between them from different dies at different times, and beyond
+# the caches every such line is written twice in part: what that costs goes by stored bytes, so not for tables with
+# many copies or many entries, and not where a tile is less than a pass of a wavefront anyway.  us a pass, edge by edge / by size: 6.1 M
+# entries on (64, 4) 36.5 / 30.0, 5.2 M on (12, 6) 36.2 / 28.1, 5.3 M on (2, 4, 2, 2) 39.4 / 31.6, 2.6 M on (12, 6) 13.5 / 12.7,
+# 488 k, packed, 17.6 / 16.5, 587 k on (6, 4, 2) 15.2 / 14.3, 20 M on (16, 8, 4) 69.8 / 64.2, 27 M 88 / 83; two layers 23.7 /
+# 21.7, four layers 19.0 / 18.6; the other way: 39 M entries 111 / 122, six layers 14.6 / 15.1, nineteen 18.5 / 19.2, 73 M in
+# eighty 127 / 204; 30 entries a tile 14.8 / 15.9.
+ORDERED_MAX_ENTRIES = 32_000_000
+ORDERED_MAX_COPIES = 4
+ORDERED_MIN_PER_TILE = 64
 # A table this small is bound by the latency of one workgroup, not by work: it keeps the largest
 # tiles and up to 16 copies per tiled edge (Llama-3-8B on (32, 8), 1.8 M entries: 13.3 us with
 # 840 tiles of 16 copies against 14.6 us with 1 616 tiles of 8 and 17.7 us with 3 168 of 4).
@@ -477,6 +488,22 @@ class CostTables:
         """Whether tiles staged in LDS beat packed ones on a small table (above: STAGED_MIN_COMPUTED)."""
         return computed >= STAGED_MIN_COMPUTED and computed >= n_tiles * STAGED_MIN_COMPUTED_PER_TILE[len(self.mesh_sizes)]
 
+    def largest_tiles_first_pays(self) -> bool:
+        """Whether a launch takes the tiles by size instead of edge by edge (above: ORDERED_MAX_ENTRIES)."""
+        if self.n_entries > ORDERED_MAX_ENTRIES or self.n_tiles == 0:
+            return False
+        computed = self.computed_entries()
+        return computed >= ORDERED_MIN_PER_TILE * self.n_tiles and self.n_entries <= ORDERED_MAX_COPIES * computed
+
+    def launch_records(self) -> np.ndarray:
+        """``tile_records`` in the order in which a launch takes them."""
+        if not self.largest_tiles_first_pays():
+            return self.tile_records
+        records = self._records(self.tile_records, self.n_tiles, TILE_DTYPE)
+        ordered = np.empty(self.n_tiles, TILE_DTYPE)
+        _native.host_call("apc_order_tiles_host", self.n_tiles, records, ordered)
+        return ordered
+
     def computed_entries(self) -> int:
         """Entries the tiles compute: those of identical edges once for all their copies."""
         return int((self.tile_row_count.astype(np.int64) * self.tile_col_count.astype(np.int64)).sum())
@@ -490,17 +517,17 @@ class CostTables:
             return False
         return bool(self.n_strategies == 0 or int(self.strat_num_args.max()) <= 0x7FFF)
 
-    def _packed_sources(self) -> list:
+    def _packed_sources(self, records=None) -> list:
         """What a packed tile is copied out of, as the library takes it."""
         self._matrix_sizes()  # (the rows of all edges come from their sizes)
         return [self.n_tensors, *self._rows(self.n_tensors, "tensor_rank", "tensor_itemsize", "tensor_shape", "tensor_stride"),
                 self.n_specs, *self._rows(self.n_specs, "spec_codes", "spec_tensor"),
                 self.n_strategies, *self._strategy_rows(), self.n_edges, self.edge_row_begin(), self.n_tiles,
-                self._records(self.tile_records, self.n_tiles, TILE_DTYPE), len(self.dup_entry_begin),
+                self._records(self.tile_records if records is None else records, self.n_tiles, TILE_DTYPE), len(self.dup_entry_begin),
                 *self._rows(len(self.dup_entry_begin), "dup_entry_begin", "dup_row_begin")]
 
-    def pack_tiles(self) -> np.ndarray:
-        """One ``apc_packed_tile`` record per tile: the tile's header, its tensor's row, the
+    def pack_tiles(self, records=None) -> np.ndarray:
+        """One ``apc_packed_tile`` record per tile (of ``records``, the table's own by default): the tile's header, its tensor's row, the
         first entries / rows of its identical edges, its producer and consumer specs and its
         consumer strategies' rows of the strategy table, copied out of the tables (after the
         strategy table is final).  A workgroup then loads nothing whose address depends on
@@ -509,7 +536,7 @@ class CostTables:
             raise RuntimeError("packed tiles need whole rows in every tile and at most "
                                f"{APC_PACKED_MAX_DUPS} identical edges per tile")
         pk = np.empty(self.n_tiles, PACKED_TILE_DTYPE)
-        _native.host_call("apc_pack_tiles_host", *self._packed_sources(), pk)
+        _native.host_call("apc_pack_tiles_host", *self._packed_sources(records), pk)
         return pk
 
     def validate_packed(self, packed: np.ndarray) -> None:

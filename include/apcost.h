@@ -170,6 +170,9 @@ int apc_fill_tiles_host(int64_t n_edges, const int32_t *edge_n_src_host, const i
                         int64_t *edge_dup_count_host, int64_t *dup_entry_begin_host, int64_t *dup_row_begin_host,
                         int32_t *tile_edge_host, int32_t *tile_row_begin_host, int32_t *tile_row_count_host,
                         int32_t *tile_col_begin_host, int32_t *tile_col_count_host);
+/* The records in the order of their tiles' entries, the most first (ties as they were), so that the last workgroups of a
+ * launch are short ones; dealt to the chip's dies one by one, in the runs of APC_TILE_RUN that the launches give to each. */
+int apc_order_tiles_host(int64_t n_tiles, const apc_tile *records_host, apc_tile *ordered_host);
 int apc_tile_records_host(int64_t n_specs, const int32_t *spec_tensor_host, int64_t n_edges, const int32_t *edge_src_begin_host,
                           const int32_t *edge_n_src_host, const int32_t *edge_tgt_begin_host, const int32_t *edge_flags_host,
                           const int64_t *edge_pt_begin_host, const int64_t *edge_entry_begin_host,
