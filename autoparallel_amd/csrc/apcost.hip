@@ -3208,22 +3208,26 @@ static int out_mode(int mesh_ndim, const double *comm_out, const uint8_t *trans_
 // counts the copies written for identical edges too: work per tile either way).
 //   At most kTilesInOneRound tiles, all of them resident at once: four wavefronts (829 tiles of 387 values, (32, 8),
 //   one launch: 9.5 / 7.4 / 7.1 us with one / two / four; 968 tiles of 1 800 values 21.6 / 14.8 / 12.0).
-//   `many_states`: four (a tile stages the 496 states of a 4-D mesh: 9 852 tiles of 22 values 101 / 73 / 58 us; with
-//   power-of-two sizes the exponents' 14 arrays, one launch: 1 650 tiles of 546 values 35.6 / 23.1 / 20.0, 6 378 of 999
-//   35.1 / 32.9 / 38.7).
+//   `many_states`: four (a tile stages the 496 states of a 4-D mesh: 9 852 tiles of 22 values 101 / 73 / 58 us).  With
+//   power-of-two sizes it stages the exponents' 14 arrays, as on other meshes: 2 218 tiles of 390 values - / 9.0 / 11.8, 1 540 of 560
+//   15.2 / 10.0 / 9.9, 8 747 of 609 - / 31.3 / 37.3.
 //   Else by the values per tile: two from `two`, four from `four`.  The launch over the tables' own copies (512, 2048):
 //   1 800 values, (8, 8, 8), 169 / 154 / 179 us; 3 236 values there - / 173 / 131; 2 390 values, (32, 8), - / 32.9 / 29.2.  The launch
 //   of all tables, whose tiles derive what the other reads (64, on 3-D meshes always, with kTilesOfManyRounds 512; 3072): (32, 8), 398 values 18.5 /
 //   17.2 / 21.0, 2 638 values - / 21.4 / 23.8, 3 874 values - / 29.4 / 27.3, 22 values 13.9 / 15.7 / 24.5; (8, 8, 8), 22 values
 //   17.1 / 16.1 / 24.1 us; 36 157 tiles of 149 values 46.8 / 59.4 / 96.7 there, 46.7 / 56.5 / 94.9 on (16, 8, 4), 4 123 of 139
 //   on (8, 8, 8) 16.6 / 14.3 / 17.8.
+//   Small tiles fill the chip sooner: from kSmallTilesInOneRound on, two for those of less than kSmallTile values (1 181 tiles of
+//   338 values, (8, 8, 8), 6.6 with two / 7.5 with four, 1 265 of 330, (12, 6), 7.0 / 8.0; the other way 880 of 480 7.9 / 7.1, 812 of
+//   490 7.5 / 6.7, 1 270 of 710 11.7 / 8.7).
 constexpr int64_t kTilesInOneRound = 1280;  // five workgroups of four wavefronts to a compute unit
+constexpr int64_t kSmallTilesInOneRound = 1024, kSmallTile = 448;
 constexpr int64_t kTilesOfManyRounds = 16384;  // (of one wavefront: 32 workgroups to a compute unit, twice)
 
 static int tile_threads(int64_t n_tiles, int64_t n_entries, bool many_states, int64_t two, int64_t four) {
   int threads = 256;
-  if (n_tiles > kTilesInOneRound && !many_states) {
-    const int64_t per_tile = n_entries / n_tiles;
+  const int64_t per_tile = n_tiles > 0 ? n_entries / n_tiles : 0;
+  if ((n_tiles > kTilesInOneRound || (n_tiles > kSmallTilesInOneRound && per_tile < kSmallTile)) && !many_states) {
     threads = per_tile >= four ? 256 : per_tile >= two ? 128 : 64;
   }
   if (const char *env = getenv("APC_TILE_THREADS")) threads = atoi(env);  // tuning override
@@ -3348,7 +3352,7 @@ static int build_tables_impl(const apc_params *params, int64_t n_tensors, const 
   if (n_tiles > 0 && n_tensors == 0) return fail(-1, "apc_build_tables: tiles need a tensor table with at least one row");
   const int xs = xcd_shift();
   const TermLayout lay = term_layout(*params);
-  const bool many_states = params->mesh_ndim == 4 && (lay.exponents == 0 || n_tiles <= 2 * kTilesInOneRound);
+  const bool many_states = params->mesh_ndim == 4 && lay.exponents == 0;
   const int threads = tile_threads(n_tiles, n_entries, many_states, n_tiles > kTilesOfManyRounds ? 512 : params->mesh_ndim == 3 ? 0 : 64, 3072);
   const int64_t tile_blocks = ((n_tiles + (1 << xs) - 1) >> xs) << xs;
   const int64_t sb = spec_table ? blocks_for(n_specs, threads) : 0, tb = blocks_for(n_tensors, threads),

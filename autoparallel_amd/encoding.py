@@ -78,6 +78,10 @@ AUTO_MANY_TILES = 100_000
 ORDERED_MAX_ENTRIES = 32_000_000
 ORDERED_MAX_COPIES = 4
 ORDERED_MIN_PER_TILE = 64
+# Their largest tiles are no tail, and may be larger than AUTO_MIN_STORED_PER_TILE would have them: 2048 / 4096 entries, 20 M on
+# (16, 8, 4) 63.5 (924 values) / 62.1 us, 27 M 83.4 (910) / 78.0, 5.1 M on (3, 2, 2, 2) 48.3 (868) / 44.5; 1024 / 2048 / 4096,
+# 5.3 M in two layers on (64, 4) 21.7 (960) / 20.9 (1 240) / 24.1.  (While there are tiles for more than a round or two.)
+ORDERED_MIN_STORED_PER_TILE, ORDERED_SOME_ROUNDS = 1000, 4000
 # A table this small is bound by the latency of one workgroup, not by work: it keeps the largest
 # tiles and up to 16 copies per tiled edge (Llama-3-8B on (32, 8), 1.8 M entries: 13.3 us with
 # 840 tiles of 16 copies against 14.6 us with 1 616 tiles of 8 and 17.7 us with 3 168 of 4).
@@ -91,15 +95,17 @@ AUTO_SMALL_TABLE_ENTRIES = 4_000_000
 # entries 18.3 / 21.1 (matrices of 139 entries on a 4-D mesh, whose terms cost most to stage, 31.6 / 34.1).
 STAGED_MIN_COMPUTED = 150_000
 STAGED_MIN_COMPUTED_PER_TILE = {1: 100, 2: 100, 3: 100, 4: 180}
-# Its tiles are cut until there are this many, (or they hold this few entries): enough workgroups for the chip, few
-# enough stagings.  (12, 6), rows up to 90 wide, 2.6 M entries: tiles of about 512 entries 19.9 us, 1024 (3 610 tiles)
-# 18.4, 2048 20.9, 4096 22.8, four rows per wavefront (7 369 tiles) 35.9.  On 4-D meshes a tile stages 496 states: 936 k
-# entries, 512 19.8, 1024 15.7, 2048 (927 tiles) 15.1, 4096 17.2, four rows per wavefront 54.6 us.  On both sides of the 900,
-# with row minima in the tiles: (3, 2, 2, 2), 530 k entries, whole edges (979 tiles) 19.4, 1024 17.5; 1.8 M, 39.8, 41.7; 658 k,
-# (676 whole) 1024 18.3, 2048 16.6, 4096 20.2.  On (2, 4, 2, 2), whose term arrays are smaller, 1024 wins: 901 k 17.3 against
-# 20.3, 1.8 M 24.8 against 29.2.
-STAGED_TILES = {1: 2800, 2: 2800, 3: 2800, 4: 900}
-STAGED_MIN_TILE_ENTRIES = {1: 512, 2: 512, 3: 512, 4: 1024}
+# Its tiles are cut until there are this many: enough workgroups for the chip, few enough stagings.  But no smaller than what
+# a STAGED_SMALLEST_SHARE-th of the entries to compute is (its power of two), at least 512: a launch is as long as its largest tile, and larger
+# tables last longer.  Tiles of about 512 / 1024 / 2048 / 4096 entries, by size:
+# 399 k entries on (8, 8, 8) 6.6 (1 181 tiles) / 6.7 / 7.7 / 8.4 us, 850 k 9.4 / 8.6 / 8.7 (1 270 tiles) / 9.3; 420 k on
+# (12, 6) 7.0 (1 265) / 7.1 / 7.9 / 8.3, 2.6 M 15.2 / 12.5 / 11.6 (2 431) / 11.9; 1.6 M on (32, 8) 16.2 / 13.6 / 13.5 (2 718) /
+# 13.3, on (6, 4, 2), without the minima, 2048 (2 930) 13.7, 4096 14.4; 587 k in 3 353 edges on (6, 4, 2) 14.8 (3 500) / 14.3.
+STAGED_TILES, STAGED_SMALLEST_SHARE, STAGED_MIN_TILE_ENTRIES = 2800, 750, 512
+# On a 4-D mesh with a size that is no power of two a tile stages 496 states: fewer, larger tiles.  On both sides of the
+# 900, with row minima in the tiles: (3, 2, 2, 2), 530 k entries, whole edges (979 tiles) 19.4, 1024 17.5; 1.8 M, 39.8, 41.7; 658 k
+# (676 whole) 1024 18.3, 2048 16.6, 4096 20.2; 900 k 512 27.5, 1024 20.4, 4096 (1 230) 18.8.
+STAGED_TILES_OF_MANY_STATES, STAGED_MIN_TILE_ENTRIES_OF_MANY_STATES = 900, 1024
 
 # numpy mirror of the C struct apc_tile (64 bytes)
 TILE_DTYPE = np.dtype([
@@ -426,7 +432,10 @@ class CostTables:
                 rows_per_wavefront_pass = 4
                 if n and (not fits or whole_edges[1] >= STAGED_MIN_COMPUTED):
                     n, n_dups = count(te, mc, 0)
-                    while n < STAGED_TILES[M] and te > STAGED_MIN_TILE_ENTRIES[M]:
+                    wanted, least = STAGED_TILES, max(STAGED_MIN_TILE_ENTRIES, whole_edges[1] // STAGED_SMALLEST_SHARE)
+                    if M == 4 and any(m & (m - 1) for m in self.mesh_sizes):
+                        wanted, least = STAGED_TILES_OF_MANY_STATES, STAGED_MIN_TILE_ENTRIES_OF_MANY_STATES
+                    while n < wanted and te // 2 >= 1 << (least.bit_length() - 1):
                         te //= 2
                         n, n_dups = count(te, mc, 0)
                     if not fits or self.staging_pays(whole_edges[1], n):
@@ -441,8 +450,11 @@ class CostTables:
                 while self.n_entries > n * AUTO_MAX_STORED_PER_TILE and mc > 2 and n_dups:
                     mc //= 2
                     n, n_dups = count(te, mc, 0)
-                while te < APC_TILE_MAX_ROWS * APC_TILE_MAX_COLS and (
-                        self.n_entries < n * AUTO_MIN_STORED_PER_TILE or (te > AUTO_MIN_TILE_ENTRIES and n > AUTO_MANY_TILES)):
+                ordered = self._orders(computed(), n)
+                while te < APC_TILE_MAX_ROWS * APC_TILE_MAX_COLS:
+                    stored = ORDERED_MIN_STORED_PER_TILE if ordered and n > ORDERED_SOME_ROUNDS else AUTO_MIN_STORED_PER_TILE
+                    if self.n_entries >= n * stored and not (te > AUTO_MIN_TILE_ENTRIES and n > AUTO_MANY_TILES):
+                        break
                     te *= 2
                     n, n_dups = count(te, mc, 0)
         else:
@@ -490,10 +502,11 @@ class CostTables:
 
     def largest_tiles_first_pays(self) -> bool:
         """Whether a launch takes the tiles by size instead of edge by edge (above: ORDERED_MAX_ENTRIES)."""
-        if self.n_entries > ORDERED_MAX_ENTRIES or self.n_tiles == 0:
-            return False
-        computed = self.computed_entries()
-        return computed >= ORDERED_MIN_PER_TILE * self.n_tiles and self.n_entries <= ORDERED_MAX_COPIES * computed
+        return self.n_entries <= ORDERED_MAX_ENTRIES and self.n_tiles > 0 and self._orders(self.computed_entries(), self.n_tiles)
+
+    def _orders(self, computed: int, n_tiles: int) -> bool:
+        return self.n_entries <= ORDERED_MAX_ENTRIES and ORDERED_MIN_PER_TILE * n_tiles <= computed \
+            and self.n_entries <= ORDERED_MAX_COPIES * computed
 
     def launch_records(self) -> np.ndarray:
         """``tile_records`` in the order in which a launch takes them."""
