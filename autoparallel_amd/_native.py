@@ -149,6 +149,7 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_runners = None
 _ops = None
 
 
@@ -173,6 +174,25 @@ def torch_ops():
                                f"sees a library of version {int(_ops.library_abi_version())}; this binding mirrors "
                                f"version {APC_ABI_VERSION}: rebuild both")
     return _ops
+
+
+def bound_runners():
+    """(run, run_on): ``BoundLaunch.run`` / ``run_on`` as functions of the object's ``handle()``, 0 when the launch is enqueued
+    (else ``bound_error()``).  The caller keeps the object."""
+    global _runners
+    if _runners is None:
+        torch_ops()
+        ext = ctypes.CDLL(TORCH_EXT_PATH)  # (the library that is loaded already)
+        run, run_on = ext.apcost_run_bound, ext.apcost_run_bound_on
+        run.argtypes, run_on.argtypes = (ctypes.c_void_p,), (ctypes.c_void_p, ctypes.c_int64)
+        ext.apcost_run_error.restype = ctypes.c_char_p
+        _runners = run, run_on, ext.apcost_run_error
+    return _runners[:2]
+
+
+def bound_error() -> RuntimeError:
+    """Why the last launch of this thread through ``bound_runners`` failed."""
+    return RuntimeError(_runners[2]().decode(errors="replace"))
 
 
 def params_tensor(c_params: "ApcParams"):

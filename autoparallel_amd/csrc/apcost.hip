@@ -100,19 +100,29 @@ __device__ __forceinline__ void store_through(T *p, T value) {
 // value, 3.15 from a block, 2.45 without the arguments.  The planner's pass: 1.7 M entries on (32, 8) over packed tiles 8.9 ->
 // 8.15 us, 20 M on (16, 8, 4) in two launches 70.2 -> 68.7, 2.6 M on (12, 6) over staged tiles, whose wavefronts have other
 // loads to wait for at that time, 18.4 -> 18.7.)
+// The host fills the by-value arguments in, and waits for room for them, for every launch, read or not.  The kernels of small passes,
+// which last no longer than that, have a form without them (KEPT); the others choose where they run.  (Together with a call that
+// does not go through boxed values: one block on (64,) 4.95 -> 3.3 us a pass, 399 k entries on (8, 8, 8) 7.0 -> 6.55, 420 k on (12, 6)
+// 7.1 -> 6.6.)
 constexpr size_t kLaunchHeadBytes = 40;
+template <typename Block, bool KEPT>
+struct BlockByValue {
+  Block block;
+};
 template <typename Block>
+struct BlockByValue<Block, true> {};
+template <bool KEPT, typename Block>
 __device__ __forceinline__ const Block &launch_block(const Block *kept) {
   static_assert(alignof(Block) == 8, "the block follows the other arguments without padding");
   // (chosen as a number: of two pointers, of which one comes from the global address space, the compiler makes a generic
   // one, and of every load through it a flat one)
   const uint64_t by_value = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr() + kLaunchHeadBytes;
-  const uint64_t at = kept ? (uint64_t)kept : by_value;
+  const uint64_t at = KEPT || kept ? (uint64_t)kept : by_value;
   return *(const Block *)(const APC_CONSTANT Block *)at;
 }
 // (the arguments of every such kernel; `kept` arrives in registers with the wavefront, as do those in front of it)
-#define APC_LAUNCH_PARAMS(BLOCK_) \
-  const void *work, int n_tiles, int xcd_shift, int64_t tile_blocks, double *cost_out, const BLOCK_ *kept, BLOCK_ by_value
+#define APC_LAUNCH_PARAMS(BLOCK_, KEPT_) \
+  const void *work, int n_tiles, int xcd_shift, int64_t tile_blocks, double *cost_out, const BLOCK_ *kept, BlockByValue<BLOCK_, KEPT_> by_value
 
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 typedef int64_t i64x8 __attribute__((ext_vector_type(8)));
@@ -705,9 +715,10 @@ struct InputTablesBlock {
   int64_t spec_blocks, tensor_blocks;
 };
 
-__global__ __launch_bounds__(kBlock) void input_tables_kernel(APC_LAUNCH_PARAMS(InputTablesBlock)) {
+template <bool KEPT>
+__global__ __launch_bounds__(kBlock) void input_tables_kernel(APC_LAUNCH_PARAMS(InputTablesBlock, KEPT)) {
   __shared__ int64_t s_rows[kBlock * (APC_MAX_RANK + 1)];
-  const InputTablesBlock &k = launch_block(kept);
+  const InputTablesBlock &k = launch_block<KEPT>(kept);
   const int64_t b = blockIdx.x;
   if (b < k.spec_blocks) spec_tables_block<kBlock>(b, k.p, k.sp, s_rows);
   else if (b < k.spec_blocks + k.tensor_blocks) tensor_tables_block<kBlock>(b - k.spec_blocks, k.t);
@@ -1855,9 +1866,9 @@ struct TilesBlock {
 
 template <int M, int kTileThreads, int OUT>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(tile_waves_per_simd(M, kTileThreads, false), 8)))
-void redistribute_tiles_kernel(APC_LAUNCH_PARAMS(TilesBlock)) {
+void redistribute_tiles_kernel(APC_LAUNCH_PARAMS(TilesBlock, false)) {
   extern __shared__ __align__(16) unsigned char s_stage_bytes[];  // stage_lds_bytes<M, false>
-  const TilesBlock &k = launch_block(kept);
+  const TilesBlock &k = launch_block<false>(kept);
   redistribute_tile<M, kTileThreads, false, OUT>(k.p, k.a, static_cast<const apc_tile *>(work), n_tiles, xcd_shift,
                                                  *reinterpret_cast<TileStage<M, false> *>(s_stage_bytes), address_in_lds(s_stage_bytes));
 }
@@ -1866,9 +1877,9 @@ void redistribute_tiles_kernel(APC_LAUNCH_PARAMS(TilesBlock)) {
 template <int M, int kTileThreads, int OUT>
 __global__ __launch_bounds__(kTileThreads)
 __attribute__((amdgpu_waves_per_eu(tile_waves_per_simd(M, kTileThreads, true), 8)))
-void redistribute_tiles_row_min_kernel(APC_LAUNCH_PARAMS(TilesBlock)) {
+void redistribute_tiles_row_min_kernel(APC_LAUNCH_PARAMS(TilesBlock, false)) {
   extern __shared__ __align__(16) unsigned char s_stage_bytes[];  // stage_lds_bytes<M, true>
-  const TilesBlock &k = launch_block(kept);
+  const TilesBlock &k = launch_block<false>(kept);
   redistribute_tile<M, kTileThreads, true, OUT>(k.p, k.a, static_cast<const apc_tile *>(work), n_tiles, xcd_shift,
                                                 *reinterpret_cast<TileStage<M, true> *>(s_stage_bytes), address_in_lds(s_stage_bytes));
 }
@@ -1919,10 +1930,10 @@ struct BuildTablesBlock {
   int64_t spec_blocks, tensor_blocks;
 };
 
-template <int M, int kThreads, bool RM, int OUT>
+template <int M, int kThreads, bool RM, int OUT, bool KEPT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(M <= 2 ? 7 : 1, 8)))
-void build_tables_kernel(APC_LAUNCH_PARAMS(BuildTablesBlock)) {
-  const BuildTablesBlock &k = launch_block(kept);
+void build_tables_kernel(APC_LAUNCH_PARAMS(BuildTablesBlock, KEPT)) {
+  const BuildTablesBlock &k = launch_block<KEPT>(kept);
   const apc_params &p = k.p;
   const TableArgs &a = k.a;
   const apc_tile *const tiles = static_cast<const apc_tile *>(work);
@@ -2283,9 +2294,9 @@ struct PackedBlock {
   int64_t tensor_blocks;
 };
 
-template <int M, bool POW2>
-__global__ __launch_bounds__(kBlock) void build_tables_packed_kernel(APC_LAUNCH_PARAMS(PackedBlock)) {
-  const PackedBlock &k = launch_block(kept);
+template <int M, bool POW2, bool KEPT>
+__global__ __launch_bounds__(kBlock) void build_tables_packed_kernel(APC_LAUNCH_PARAMS(PackedBlock, KEPT)) {
+  const PackedBlock &k = launch_block<KEPT>(kept);
   const int64_t b = blockIdx.x;
   if (b < tile_blocks) {
     const int tile_id = tile_of_block((int)b, n_tiles, xcd_shift);
@@ -3155,23 +3166,31 @@ static LaunchTo launch_to(void *stream) {
 static int enqueue_kept(const apc_kept_launch &k, const void *block, void *stream) {
   void *args[] = {const_cast<void **>(&k.work), const_cast<int32_t *>(&k.n_tiles), const_cast<int32_t *>(&k.xcd_shift),
                   const_cast<int64_t *>(&k.tile_blocks), const_cast<double **>(&k.cost_out), &block, const_cast<int64_t *>(k.block)};
-  (void)hipLaunchKernel(k.kernel, dim3(k.grid), dim3(k.threads), args, k.lds_bytes, (hipStream_t)stream);
+  (void)hipLaunchKernel(block ? k.kernel : k.kernel_by_value, dim3(k.grid), dim3(k.threads), args, k.lds_bytes, (hipStream_t)stream);
   return check_launch(k.what);
 }
 
+// A table kernel, and its form without arguments by value where it has one.
 template <typename Block>
-static int launch_table_kernel(const char *what, const LaunchTo &to, void (*kernel)(APC_LAUNCH_PARAMS(Block)), unsigned grid, int threads,
+struct TableKernel {
+  void (*by_value)(APC_LAUNCH_PARAMS(Block, false));
+  void (*kept)(APC_LAUNCH_PARAMS(Block, true)) = nullptr;
+};
+
+template <typename Block>
+static int launch_table_kernel(const char *what, const LaunchTo &to, const TableKernel<Block> &kernel, unsigned grid, int threads,
                                size_t lds, const void *work, int n_tiles, int xcd_shift, int64_t tile_blocks, double *cost_out,
                                const Block &block) {
   static_assert(sizeof(Block) <= APC_KEPT_BLOCK_BYTES, "the arguments fit a kept launch");
   static_assert(std::is_trivially_copyable<Block>::value, "the arguments travel as bytes");
   if (!to.keep) {
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(threads), lds, (hipStream_t)to.stream, work, n_tiles, xcd_shift, tile_blocks, cost_out,
-                       (const Block *)nullptr, block);
+    hipLaunchKernelGGL(kernel.by_value, dim3(grid), dim3(threads), lds, (hipStream_t)to.stream, work, n_tiles, xcd_shift, tile_blocks, cost_out,
+                       (const Block *)nullptr, BlockByValue<Block, false>{block});
     return check_launch(what);
   }
   apc_kept_launch &k = *to.keep;
-  k.kernel = reinterpret_cast<const void *>(kernel);
+  k.kernel = kernel.kept ? reinterpret_cast<const void *>(kernel.kept) : reinterpret_cast<const void *>(kernel.by_value);
+  k.kernel_by_value = reinterpret_cast<const void *>(kernel.by_value);
   k.what = what;
   k.grid = grid;
   k.threads = (uint32_t)threads;
@@ -3265,7 +3284,7 @@ static int input_tables_impl(const apc_params *params, int64_t n_tensors, const 
                                {n_strategies, flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag},
                                sb,
                                tb};
-  return launch_table_kernel("apc_input_tables", to, input_tables_kernel, (unsigned)(sb + tb + cb), kBlock, 0, nullptr, 0, 0, 0, nullptr, block);
+  return launch_table_kernel("apc_input_tables", to, TableKernel<InputTablesBlock>{input_tables_kernel<false>, input_tables_kernel<true>}, (unsigned)(sb + tb + cb), kBlock, 0, nullptr, 0, 0, 0, nullptr, block);
 }
 
 static int redistribute_tables_impl(const apc_params *params, const int64_t *tensor_bytes,
@@ -3295,7 +3314,7 @@ static int redistribute_tables_impl(const apc_params *params, const int64_t *ten
 #define APC_LAUNCH_T(KERNEL_, M_, OUT_)                                                                               \
   const int wg = threads >= 256 ? 256 : threads >= 128 ? 128 : 64;                                                     \
   const size_t lds = rows ? stage_lds_bytes<M_, true>(a.lay, wg) : stage_lds_bytes<M_, false>(a.lay, wg);              \
-  const auto kernel = wg == 256 ? KERNEL_<M_, 256, OUT_> : wg == 128 ? KERNEL_<M_, 128, OUT_> : KERNEL_<M_, 64, OUT_>; \
+  const TableKernel<TilesBlock> kernel{wg == 256 ? KERNEL_<M_, 256, OUT_> : wg == 128 ? KERNEL_<M_, 128, OUT_> : KERNEL_<M_, 64, OUT_>}; \
   return launch_table_kernel(what, to, kernel, (unsigned)grid, wg, lds, tiles, nt, xs, grid, cost_out, TilesBlock{*params, a})
 #define APC_LAUNCH_K(KERNEL_, M_)                                   \
   if (om == kOutAll) { APC_LAUNCH_T(KERNEL_, M_, kOutAll); }        \
@@ -3320,6 +3339,15 @@ static int redistribute_tables_impl(const apc_params *params, const int64_t *ten
 #undef APC_LAUNCH_T
 #undef APC_LAUNCH_K
 #undef APC_LAUNCH_ANY
+}
+
+// (kept: of the outputs a planner's pass has)
+template <int M, int kThreads, bool RM, int OUT>
+static TableKernel<BuildTablesBlock> build_tables_forms() {
+  if constexpr (OUT == kOutCost || M == 1 || M == 4)
+    return {build_tables_kernel<M, kThreads, RM, OUT, false>, build_tables_kernel<M, kThreads, RM, OUT, true>};
+  else
+    return {build_tables_kernel<M, kThreads, RM, OUT, false>};
 }
 
 static int build_tables_impl(const apc_params *params, int64_t n_tensors, const int32_t *rank, const int32_t *itemsize,
@@ -3374,8 +3402,8 @@ static int build_tables_impl(const apc_params *params, int64_t n_tensors, const 
   const int om = out_mode(params->mesh_ndim, comm_out, trans_out, cost_out);
 #define APC_LAUNCH_ALL_T(M_, RM_, OUT_)                                                                                 \
   const size_t lds = build_tables_lds_bytes<M_, RM_>(a.lay, threads, spec_table);                                      \
-  const auto kernel = threads == 256 ? build_tables_kernel<M_, 256, RM_, OUT_>                                         \
-                      : threads == 128 ? build_tables_kernel<M_, 128, RM_, OUT_> : build_tables_kernel<M_, 64, RM_, OUT_>; \
+  const auto kernel = threads == 256   ? build_tables_forms<M_, 256, RM_, OUT_>()                                       \
+                      : threads == 128 ? build_tables_forms<M_, 128, RM_, OUT_>() : build_tables_forms<M_, 64, RM_, OUT_>(); \
   return launch_table_kernel(what, to, kernel, (unsigned)blocks, threads, lds, tiles, nt, xs, tile_blocks, cost_out,  \
                              BuildTablesBlock{*params, a, ta, sa, ca, sb, tb})
 #define APC_LAUNCH_ALL_RM(M_, RM_)                                   \
@@ -3718,9 +3746,11 @@ static int build_tables_packed_impl(const apc_params *params, int64_t n_tensors,
   const TensorTableArgs ta{n_tensors, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous};
   const ComputeCostArgs ca{n_strategies, flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag};
   const PackedBlock block{a, *params, ta, ca, tb};
+  using K = TableKernel<PackedBlock>;
 #define APC_LAUNCH_PACKED(M_)                                                                                             \
   return launch_table_kernel("apc_build_tables_packed", to,                                                             \
-                             lay.exponents ? build_tables_packed_kernel<M_, true> : build_tables_packed_kernel<M_, false>, \
+                             lay.exponents ? K{build_tables_packed_kernel<M_, true, false>, build_tables_packed_kernel<M_, true, true>}     \
+                                           : K{build_tables_packed_kernel<M_, false, false>, build_tables_packed_kernel<M_, false, true>}, \
                              (unsigned)blocks, kBlock, 0, packed, (int)n_tiles, xs, tile_blocks, cost_out, block)
   switch (params->mesh_ndim) {
     case 1: APC_LAUNCH_PACKED(1);

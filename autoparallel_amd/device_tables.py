@@ -381,14 +381,12 @@ class DeviceCostTables:
             # a launcher only looks up the current stream (or takes the given one) and enqueues
             if repeated:
                 bound.keep_arguments()
-            run, run_on = bound.run, bound.run_on
+            (run, run_on), handle = _native.bound_runners(), bound.handle()
 
             def launch(on_stream=None):
-                if on_stream is None:
-                    run()
-                else:
-                    run_on(int(on_stream.cuda_stream))
-            launch.bound = bound
+                if run(handle) if on_stream is None else run_on(handle, int(on_stream.cuda_stream)):
+                    raise _native.bound_error()
+            launch.bound = bound  # (what the handle names lives as long as its launcher)
             return launch
 
         rows = None

@@ -587,7 +587,7 @@ int apc_build_tables_packed(const apc_params *params, int64_t n_tensors, const i
  *                                          value).  k, the block and every array the launch names stay as they are
  *                                          while it runs.
  * No counterpart in the reference. */
-#define APC_KEPT_BLOCK_BYTES 3072
+#define APC_KEPT_BLOCK_BYTES 3064
 typedef struct apc_kept_launch {
   const void *kernel;
   const char *what; /* the entry point that recorded it */
@@ -597,6 +597,7 @@ typedef struct apc_kept_launch {
   int64_t tile_blocks;
   double *cost_out;
   int64_t block[APC_KEPT_BLOCK_BYTES / 8];
+  const void *kernel_by_value; /* what runs without a device block */
 } apc_kept_launch;
 int apc_keep_next_launch(apc_kept_launch *out);
 int apc_run_kept(const apc_kept_launch *kept, const void *device_block, void *stream);
