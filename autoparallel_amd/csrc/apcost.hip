@@ -347,12 +347,21 @@ __device__ __forceinline__ double entry_cost(uint32_t srcp, uint32_t tgtp, doubl
 // values: it starts from bytes / num_shards (decided by WHICH mesh dims the producer
 // shards: a mask of M bits) and every earlier dim either left it alone or applied its
 // single possible update (x n after an all-gather when the producer shards that dim, / n
-// after a reduce-scatter when it does not).  State (level L, mask, history) indexes every
-// value that can occur; level L in [0, M] has 2^M masks x 2^L histories.
+// after a reduce-scatter).  State (level L, mask, history) indexes every
+// value that can occur; level L in [0, M) has 2^M masks x 2^L histories.  Behind the last dim
+// (level M) only an all-gather there is charged, of a producer that shards it: mask and history
+// hold the last dim, a quarter of the pairs, and are counted without it.  (4-D meshes: 304 states
+// where all pairs are 496, in 22 KB of LDS instead of 36: four workgroups to a compute unit, not three.  5.1 M entries on
+// (3, 2, 2, 2) 45.1 -> 33.7 us, 900 k 18.8 -> 13.7; 72 of 120 on 3-D meshes, 587 k on (6, 4, 2) 14.1 -> 12.0, 1.6 M 14.0 -> 12.2.)
 // ------------------------------------------------------------------------------------------
 template <int M>
 struct States {
-  static constexpr int kCount = (1 << M) * ((1 << (M + 1)) - 1);
+  static constexpr int kLast = ((1 << M) - 1) << M;  // the first of level M
+  static constexpr int kHalf = 1 << (M - 1);
+  static constexpr int kCount = kLast + kHalf * kHalf;
+  __device__ static __forceinline__ int last(int mask, int hist) {
+    return kLast + ((mask & (kHalf - 1)) << (M - 1)) + (hist & (kHalf - 1));
+  }
   __device__ static __forceinline__ int index(int level, int mask, int hist) {
     return (((1 << level) - 1) << M) + (mask << level) + hist;
   }
@@ -1090,14 +1099,15 @@ __device__ __forceinline__ TileView view_of(const apc_tile &tile) {
                   tile.flags,           tile.dup_count,    tile.src_begin, tile.entry_begin, tile.pt_begin};
 }
 
-// ring_r on a per-lane mesh dim d, with hops = hop_scale * (mesh_size[d] - 1).
+// ring_r on a per-lane mesh dim d, with mesh_size[d] - 1 hops and with twice as many: every step behind the first product
+// of twice the hops doubles exactly.
 template <int M>
-__device__ __forceinline__ double ring_at(double gb, const apc_params &p, int d, int hop_scale) {
+__device__ __forceinline__ void rings_at(double gb, const apc_params &p, int d, double &one, double &two) {
   const int n = pick<M>(p.mesh_size, d);
-  const double hops = (double)(hop_scale * (n - 1));
-  const double latency = p.base_latency + hops * pick<M>(p.lat, d);
-  const double bw = div_by(div_by(gb * hops, (double)n, pick<M>(p.inv_mesh, d)), pick<M>(p.bw, d), pick<M>(p.inv_bw, d));
-  return latency + bw * 1e6;
+  const double hops = (double)(n - 1), lat = pick<M>(p.lat, d);
+  const double bw = div_by(div_by(gb * hops, (double)n, pick<M>(p.inv_mesh, d)), pick<M>(p.bw, d), pick<M>(p.inv_bw, d)) * 1e6;
+  one = (p.base_latency + hops * lat) + bw;
+  two = (p.base_latency + (2.0 * hops) * lat) + 2.0 * bw;
 }
 
 // Stages tile `tile` with `nthreads` (>= 64) cooperating threads (this thread is `tid`).  The
@@ -1222,11 +1232,8 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
     // the reference's operation order (collective_runtime_estimation.py:66-68, :86, :128;
     // torch _collective_utils.py:281-313; compute_estimation.py:302-314)
     const double fbytes = (double)tensor_nbytes;
-    for (int k = tid; k < NS; k += nthreads) {
-      const bool flip_state = M == 2 && k == States<M>::kCount;
-      const int level = flip_state ? 0 : 31 - __clz((k >> M) + 1);
-      const int rem = flip_state ? 0 : k - (((1 << level) - 1) << M);
-      const int mask = rem >> level, hist = rem & ((1 << level) - 1);
+    double *const terms = reinterpret_cast<double *>(term_base(st, nthreads));
+    const auto bytes_at = [&](int level, int mask, int hist) {
       double shards = 1.0;  // exact: a product of mesh sizes (torch _dtensor_spec.py:555-561)
 #pragma unroll
       for (int i = 0; i < M; ++i)
@@ -1239,17 +1246,11 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
           gb = ((mask >> i) & 1) ? gb * m : div_by(gb, m, p.inv_mesh[i]);
         }
       }
-      if (flip_state) gb = div_by(gb, (double)p.mesh_size[1], p.inv_mesh[1]);
-      double ag = 0.0, rs = 0.0, ar = 0.0;
-      if (level >= 1) ag = ring_at<M>(gb, p, level - 1, 1);
-      if (level < M) {
-        rs = ring_at<M>(gb, p, level, 1);
-        ar = ring_at<M>(gb, p, level, 2);
-      }
-      double a2a = rs;
-      a2a *= p.a2a_scale;
+      return gb;
+    };
+    const auto store_state = [&](int k, double gb, double ag, double rs, double ar) {
       const double rw = rw_time_r(gb * 2 * 1073741824.0, p);
-      double *e = reinterpret_cast<double *>(term_base(st, nthreads)) + k * (kGeneralStride / 8);
+      double *e = terms + __mul24(k, kGeneralStride / 8);
       e[kZerosArray] = 0.0;
       e[kInfArray] = __builtin_inf();
       e[kRw1Array] = rw;
@@ -1257,7 +1258,32 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
       e[4] = ag;
       e[5] = rs;
       e[6] = ar;
-      e[7] = a2a;
+      e[7] = rs * p.a2a_scale;
+    };
+    // On 3-D and 4-D meshes the last level apart, which has an all-gather and a read+write alone.
+    constexpr bool kLastApart = M >= 3;
+    constexpr int kFirst = kLastApart ? States<M>::kLast : NS, kHalf = States<M>::kHalf;
+    for (int k = tid; k < kFirst; k += nthreads) {
+      const bool flip_state = M == 2 && k == States<M>::kCount, last = !kLastApart && k >= States<M>::kLast && !flip_state;
+      const int level = flip_state ? 0 : last ? M : 31 - __clz((k >> M) + 1);
+      const int rem = flip_state ? 0 : last ? k - States<M>::kLast : k - (((1 << level) - 1) << M);
+      const int mask = last ? kHalf | (rem >> (M - 1)) : rem >> level;
+      const int hist = last ? kHalf | (rem & (kHalf - 1)) : rem & ((1 << level) - 1);
+      double gb = bytes_at(level, mask, hist);
+      if (flip_state) gb = div_by(gb, (double)p.mesh_size[1], p.inv_mesh[1]);
+      double ag = 0.0, rs = 0.0, ar = 0.0, unused;
+      if (level >= 1) rings_at<M>(gb, p, level - 1, ag, unused);
+      if (level < M) rings_at<M>(gb, p, level, rs, ar);
+      store_state(k, gb, ag, rs, ar);
+    }
+    if constexpr (kLastApart) {
+      const int first = (tid + 8 * nthreads - 64 * ((kFirst + 63) / 64)) & (nthreads - 1);  // from the wavefronts that had fewer of the others
+      for (int u = first; u < kHalf * kHalf; u += nthreads) {
+        const double gb = bytes_at(M, kHalf | (u >> (M - 1)), kHalf | (u & (kHalf - 1)));
+        const double hops = (double)(p.mesh_size[M - 1] - 1);
+        const double bw = div_by(div_by(gb * hops, (double)p.mesh_size[M - 1], p.inv_mesh[M - 1]), p.bw[M - 1], p.inv_bw[M - 1]);
+        store_state(kFirst + u, gb, (p.base_latency + hops * p.lat[M - 1]) + bw * 1e6, 0.0, 0.0);
+      }
     }
   }
   // ---- what the loads brought, to LDS ---------------------------------------------------------
@@ -1289,7 +1315,8 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
         // it; the all-gather (a sharding producer, a replicating consumer: class 0) is charged on
         // the gathered bytes.  (Power-of-two layout: that shift is part of the word's base.)
         const uint32_t k = (uint32_t)States<M>::index(i, 0, 0) + (mask << i);
-        const uint32_t k2 = (uint32_t)States<M>::index(i + 1, 0, 0) + (mask << (i + 1)) + (1u << i);
+        const uint32_t k2 = i + 1 < M ? (uint32_t)States<M>::index(i + 1, 0, 0) + (mask << (i + 1)) + (1u << i)
+                                      : (uint32_t)States<M>::last((int)mask, 0);
         const uint32_t at = (uint32_t)__umul24(POW2 ? j0 : k, POW2 ? (uint32_t)kPow2Stride : (uint32_t)kGeneralStride);
         const uint32_t at0 = POW2 ? at : (uint32_t)__umul24(cls >= 2 ? k2 : k, (uint32_t)kGeneralStride);
         uint32_t *w = w_of_col + i * kWordsPerDim;
@@ -3227,7 +3254,7 @@ static int out_mode(int mesh_ndim, const double *comm_out, const uint8_t *trans_
 // counts the copies written for identical edges too: work per tile either way).
 //   At most kTilesInOneRound tiles, all of them resident at once: four wavefronts (829 tiles of 387 values, (32, 8),
 //   one launch: 9.5 / 7.4 / 7.1 us with one / two / four; 968 tiles of 1 800 values 21.6 / 14.8 / 12.0).
-//   `many_states`: four (a tile stages the 496 states of a 4-D mesh: 9 852 tiles of 22 values 101 / 73 / 58 us).  With
+//   `many_states`: four (a tile stages the 304 states of a 4-D mesh: 9 852 tiles of 22 values 101 / 73 / 58 us).  With
 //   power-of-two sizes it stages the exponents' 14 arrays, as on other meshes: 2 218 tiles of 390 values - / 9.0 / 11.8, 1 540 of 560
 //   15.2 / 10.0 / 9.9, 8 747 of 609 - / 31.3 / 37.3.
 //   Else by the values per tile: two from `two`, four from `four`.  The launch over the tables' own copies (512, 2048):

@@ -102,7 +102,7 @@ STAGED_MIN_COMPUTED_PER_TILE = {1: 100, 2: 100, 3: 100, 4: 180}
 # (12, 6) 7.0 (1 265) / 7.1 / 7.9 / 8.3, 2.6 M 15.2 / 12.5 / 11.6 (2 431) / 11.9; 1.6 M on (32, 8) 16.2 / 13.6 / 13.5 (2 718) /
 # 13.3, on (6, 4, 2), without the minima, 2048 (2 930) 13.7, 4096 14.4; 587 k in 3 353 edges on (6, 4, 2) 14.8 (3 500) / 14.3.
 STAGED_TILES, STAGED_SMALLEST_SHARE, STAGED_MIN_TILE_ENTRIES = 2800, 750, 512
-# On a 4-D mesh with a size that is no power of two a tile stages 496 states: fewer, larger tiles.  On both sides of the
+# On a 4-D mesh with a size that is no power of two a tile stages 304 states: fewer, larger tiles.  On both sides of the
 # 900, with row minima in the tiles: (3, 2, 2, 2), 530 k entries, whole edges (979 tiles) 19.4, 1024 17.5; 1.8 M, 39.8, 41.7; 658 k
 # (676 whole) 1024 18.3, 2048 16.6, 4096 20.2; 900 k 512 27.5, 1024 20.4, 4096 (1 230) 18.8.
 STAGED_TILES_OF_MANY_STATES, STAGED_MIN_TILE_ENTRIES_OF_MANY_STATES = 900, 1024
