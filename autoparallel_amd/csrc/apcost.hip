@@ -1041,7 +1041,7 @@ struct alignas(16) StagingScratch {
 };
 // What a wavefront has to itself: while it stages the term arrays, their chains; where the tile's row minima are
 // taken, in the same place afterwards, the values of the rows it is walking (tile_entries_row_min).
-constexpr int kRowMinValues = 512;
+constexpr int kRowMinValues = 320;
 template <bool RM>
 constexpr size_t kWaveScratchBytes = RM ? kRowMinValues * sizeof(double) : sizeof(StagingScratch);
 static_assert(kWaveScratchBytes<true> >= sizeof(StagingScratch), "the chains fit");
@@ -1645,8 +1645,10 @@ __device__ __forceinline__ void lower_of_lanes(double &m, int &mc) {
 // row read it back, the lanes of a row the columns in turn, and join their minima.  The rows of a wavefront need no
 // barrier, and a value costs one write and one read of 8 bytes where a minimum taken across the lanes of every pass
 // (neighbours in doubling distances, value and column) was 70 vector instructions a pass, more than the entry's own.
-// kRowMinValues = 512, 384, 256: 38.7, 40.3, 41.5 us for 6.1 M entries on (64, 4), by passes 50.4, without the minima 27.4
-// (its rows' stores are 0.6 of that).
+// (6.1 M entries on (64, 4) 50.4 -> 38.7 us, 27.4 without the minima.)  kRowMinValues: more rows are joined at once, fewer workgroups
+// fit a compute unit.  512 / 384 / 320 / 256, later: those entries 28.2 / 26.6 / 26.1 / 26.2 us, 5.2 M on (12, 6) 27.2 / 25.0 / 25.1 /
+// 24.7, 5.3 M in two layers on (64, 4) 21.2 / 20.0 / 20.1 / 19.3, 410 k on (32, 8) 11.0 / 10.3 / 10.2 / 9.0; 5.8 M in nineteen layers
+// 18.3 / 17.5 / 17.8 / 18.5, 850 k on (8, 8, 8), which fit once anyway, 8.5 / 8.6 / 8.7 / 9.1.
 template <int M, int OUT, typename Entry>
 __device__ __forceinline__ void tile_entries_row_min(const TableArgs &a, lds_address stage, const TileView &v, const TileCopies &copies,
                                                      int tid, int nthreads, Entry entry) {
@@ -1919,33 +1921,17 @@ void redistribute_tiles_row_min_kernel(APC_LAUNCH_PARAMS(TilesBlock, false)) {
 // table workgroups use (TableArgs), so the values are the same bits.  One launch instead of
 // two spares a table of a few tens of MB one ramp-up and one drain of the chip, which at that
 // size are a third of each kernel.
-// (On 3-D and 4-D meshes LDS is sized per launch for the layout in use: with the general layout's share held for every mesh, a
+// (LDS is sized per launch for the layout in use: with the general layout's share held for every mesh, a
 // workgroup of a 4-D launch held 45 KB of which a power-of-two mesh uses 10.  6.4 M entries on (2, 4, 2, 2) 46.2 -> 32.9 us,
-// 9.4 M on (16, 8, 4) 64.6 -> 59.1, 901 k on (8, 8, 8) 14.9 -> 13.8.)
+// 9.4 M on (16, 8, 4) 64.6 -> 59.1, 901 k on (8, 8, 8) 14.9 -> 13.8; on 1-D and 2-D meshes, where the larger layout was held, 6.1 M
+// on (64, 4) 29.5 -> 28.2, 41 k on (64,) 10.6 -> 9.6.)
 // (On 1-D and 2-D meshes seven wavefronts per SIMD are asked for, what 72 vector registers leave room for: 7.6 M entries on (32, 8),
 // 59 layers, 17.0 us with 5, 16.4 with 7, 2.6 M on (12, 6) 13.4 / 13.2, 6.1 M on (64, 4) with the minima the same.)
-// (1-D and 2-D meshes hold the larger layout's share in a static array: sized per launch, what a 2-D launch does takes 2 %
-// longer, 18.3 -> 18.7 us for 2.6 M entries on (12, 6), also with the same bytes asked for.)
 template <int M, bool RM>
 static size_t build_tables_lds_bytes(const TermLayout &lay, int threads, bool spec_table) {
-  if (M <= 2) return 0;
   const size_t stage = stage_lds_bytes<M, RM>(lay, threads);
   const size_t rows = spec_table ? (size_t)threads * (APC_MAX_RANK + 1) * sizeof(int64_t) : 0;  // (spec_tables_block)
   return stage > rows ? stage : rows;
-}
-
-// The LDS of build_tables_kernel.
-template <int M, int kThreads, bool RM>
-__device__ __forceinline__ unsigned char *build_tables_lds() {
-  if constexpr (M <= 2) {
-    constexpr size_t kRowBytes = (size_t)kThreads * (APC_MAX_RANK + 1) * sizeof(int64_t);
-    constexpr size_t kStage = sizeof(TileStage<M, RM>) + kWaveScratchBytes<RM> * (kThreads / 64);
-    __shared__ __align__(16) unsigned char s_fixed[kStage > kRowBytes ? kStage : kRowBytes];
-    return s_fixed;
-  } else {
-    extern __shared__ __align__(16) unsigned char s_stage_bytes[];  // build_tables_lds_bytes<M, RM>
-    return s_stage_bytes;
-  }
 }
 
 struct BuildTablesBlock {
@@ -1964,7 +1950,7 @@ void build_tables_kernel(APC_LAUNCH_PARAMS(BuildTablesBlock, KEPT)) {
   const apc_params &p = k.p;
   const TableArgs &a = k.a;
   const apc_tile *const tiles = static_cast<const apc_tile *>(work);
-  unsigned char *const s_raw = build_tables_lds<M, kThreads, RM>();
+  extern __shared__ __align__(16) unsigned char s_raw[];  // build_tables_lds_bytes<M, RM>
   static_assert(kThreads == 64 || kThreads == 128 || kThreads == 256, "wavefronts per workgroup: 1, 2 or 4");
   const int64_t b = blockIdx.x;
   if (b < tile_blocks) {
