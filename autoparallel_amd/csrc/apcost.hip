@@ -740,8 +740,8 @@ __global__ __launch_bounds__(kBlock) void input_tables_kernel(APC_LAUNCH_PARAMS(
 // are staged in LDS (TileStage); the per-entry loop walks the mesh dims, looks the terms of
 // the current state up and adds them in the reference's order, so results are bit-identical
 // to evaluating every entry directly (entry_cost).  The direct evaluation remains the path
-// for the rare cases the states do not cover: producer specs of one edge that point at
-// different tensors, and the 2-D (Partial, Partial) -> all-Shard order flip.
+// for the rare case the states do not cover: producer specs of one edge that point at
+// different tensors.
 //
 // One workgroup per tile.  (A variant in which a workgroup walked a run of tiles, one
 // wavefront staging tile t+1 into a second LDS stage while the others computed and stored
