@@ -1455,7 +1455,7 @@ __device__ __forceinline__ void word_slots(uint32_t src, uint32_t tgt, uint32_t 
 
 // One entry of a tile whose producer specs all name one tensor.
 // What bounds a table of large tiles is the vector instructions of a SIMD, all of its cycles (20 M entries on (16, 8, 4): 27.9 M
-// instructions, 108 thousand of a SIMD's cycles in a launch of 101 thousand; LDS 73 % busy), so a pass of 64 entries counts them:
+// instructions, 108 thousand of a SIMD's cycles in a launch of 101 thousand; now 20.4 M, 80 of 84 thousand, LDS 79 % busy), so a pass counts them:
 // 40 on a 3-D mesh with the walk and the store (54 when columns, rows and loop were kept as numbers of a lane and the codes
 // compared by mask), and a tile's staging, which two wavefronts share, about 330 (430).  us a pass: 20 M on (16, 8, 4) 57.0 ->
 // 50.8, 5.3 M on (2, 4, 2, 2) 41.8 -> 39.4, 5.1 M on (3, 2, 2, 2) 53.2 -> 50.7, 2.6 M on (12, 6) 14.4 -> 13.4, 587 k on
