@@ -431,6 +431,8 @@ class DeviceCostTables:
                 step["segmented_min"] = bind(ops.bind_segmented_min(self.cost, row_ptr, None, None, None, 0,
                                                                     self.row_min, self.row_argmin))
         self._step_error_flag = err
+        # (a program may drop ``step`` once it has enqueued or captured its launches, which read more than the arrays above)
+        self._step_keepalive.append([launch.bound for launch in step.values()])
         return step
 
     # ---- the planner's table build -------------------------------------------------------------
@@ -499,8 +501,8 @@ class DeviceCostTables:
         """Records one pass (the launchers of ``prepare_step``) into a HIP graph: one launch per
         pass, and the three kernels that only read the uploaded tables (tensor, spec and
         compute-cost tables) sit on parallel branches, so they overlap on the device instead
-        of queueing behind each other.  Returns the ``torch.cuda.CUDAGraph``; ``replay()``
-        enqueues the pass on the current stream.  For callers that want a single launch per
+        of queueing behind each other.  Returns the ``torch.cuda.CUDAGraph``, which holds every array
+        its launches read or write; ``replay()`` enqueues the pass on the current stream.  For callers that want a single launch per
         pass; it is not the fast way to loop over passes: on the Llama-3-8B table a replay was
         measured at 61 us against 39 us for the five plain launches in stream order (the
         runtime's per-node replay cost exceeds what the overlap saves), and equal on tables
@@ -525,7 +527,7 @@ class DeviceCostTables:
                 step["redistribute_tables"](main)
             if "segmented_min" in step:
                 step["segmented_min"](main)
-        self._step_keepalive.append(branches)
+        graph.apcost_launches = tuple(step.values()), branches
         return graph
 
     # ---- segmented min ---------------------------------------------------------------------

@@ -2,6 +2,8 @@
 against the same launches with their arguments passed by value."""
 
 import ctypes
+import gc
+import weakref
 
 import numpy as np
 import pytest
@@ -10,6 +12,8 @@ import torch
 from autoparallel_amd import CostModelParams, _native
 from autoparallel_amd.device_tables import DeviceCostTables
 from autoparallel_amd.synthetic import stress_dag
+from oracle import c_oracle
+from oracle import cost_oracle as po
 
 
 class _Kept(ctypes.Structure):  # include/apcost.h: apc_kept_launch
@@ -92,3 +96,45 @@ def test_kept_launches_write_what_launches_by_value_write(gpu_device, mesh):
                 d.cost.zero_()
                 graph.replay()
                 assert np.array_equal(_outputs(d)[2], want[2]), form
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("one_launch", [True, False])
+def test_a_graph_holds_what_its_launches_read(gpu_device, one_launch):
+    """``step`` and then the tables' device object are dropped: a graph of the pass still has the blocks of its launches."""
+    mesh = (16, 8, 4)
+    tb = stress_dag(seed=4, n_nodes=300, mesh_sizes=mesh, max_strategies=20)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
+    form = dict(row_min=False, fused_inputs=True, outputs=("cost",), spec_table=False, one_launch=one_launch, packed=False)
+    step = d.prepare_step(**form)
+    launches = [weakref.ref(launch) for launch in step.values()]
+    graph = d.capture_step_graph(step)
+    del step
+    gc.collect()
+    assert all(launch() is not None for launch in launches)
+    cost = d.cost
+    d.prepare_step(**form)  # (the device object holds the launches of its latest step only)
+    del d
+    gc.collect()
+    assert all(launch() is not None for launch in launches)
+    others = [torch.full((n,), 7, dtype=torch.int64, device=gpu_device) for n in (64, 128, 256, 383) for _ in range(8)]
+    want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh, rescale=2.2))["cost"]
+    for _ in range(3):
+        cost.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(cost.cpu().numpy(), want)
+    assert all(bool((t == 7).all()) for t in others)
+
+
+@pytest.mark.gpu
+def test_the_device_object_holds_the_launches_of_its_latest_step(gpu_device):
+    mesh = (32, 8)
+    tb = stress_dag(seed=4, n_nodes=300, mesh_sizes=mesh, max_strategies=20)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
+    for _ in range(2):
+        step = d.planner_pass()
+        bound = [weakref.ref(launch.bound) for launch in step.values()]
+        del step
+        gc.collect()
+        assert all(b() is not None for b in bound)
