@@ -177,14 +177,14 @@ def torch_ops():
 
 
 def bound_runners():
-    """(run, run_on): ``BoundLaunch.run`` / ``run_on`` as functions of the object's ``handle()``, 0 when the launch is enqueued
-    (else ``bound_error()``).  The caller keeps the object."""
+    """(run, run_on): ``BoundLaunch.run`` / ``run_on`` as functions of the object's ``handle()`` (``run_on``: and of a stream's
+    handle and torch's number of it, ``stream_id``), 0 when the launch is enqueued (else ``bound_error()``).  The caller keeps the object."""
     global _runners
     if _runners is None:
         torch_ops()
         ext = ctypes.CDLL(TORCH_EXT_PATH)  # (the library that is loaded already)
         run, run_on = ext.apcost_run_bound, ext.apcost_run_bound_on
-        run.argtypes, run_on.argtypes = (ctypes.c_void_p,), (ctypes.c_void_p, ctypes.c_int64)
+        run.argtypes, run_on.argtypes = (ctypes.c_void_p,), (ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64)
         ext.apcost_run_error.restype = ctypes.c_char_p
         _runners = run, run_on, ext.apcost_run_error
     return _runners[:2]

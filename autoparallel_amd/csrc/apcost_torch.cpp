@@ -21,6 +21,7 @@
 // Built against the installed torch: autoparallel_amd/_build.py (build_torch_extension).
 
 #include <ATen/ATen.h>
+#include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
@@ -28,10 +29,13 @@
 #include <torch/library.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <exception>
 #include <functional>
+#include <limits>
 #include <memory>
+#include <mutex>
 #include <optional>
 #include <string>
 #include <tuple>
@@ -408,13 +412,38 @@ struct BoundLaunch : torch::CustomClassHolder {
   }
   void run() {
     c10::hip::HIPGuard guard(device.index());
-    enqueue(c10::hip::getCurrentHIPStream(device.index()).stream());
+    const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(device.index());
+    used_on(stream.id(), stream.stream());
+    enqueue(stream.stream());
   }
-  // The launch on a stream given by its handle (torch.cuda.Stream.cuda_stream).
-  void run_on(int64_t stream) {
+  // The launch on a stream given by its handle (torch.cuda.Stream.cuda_stream) and, where the caller has it, torch's number
+  // of it (stream_id).
+  void run_on(int64_t handle, int64_t id) {
     c10::hip::HIPGuard guard(device.index());
-    enqueue(reinterpret_cast<void *>(stream));
+    used_on(id, reinterpret_cast<hipStream_t>(handle));
+    enqueue(reinterpret_cast<void *>(handle));
   }
+  void run_on_handle(int64_t handle) { run_on(handle, handle); }
+
+  // The tensors may go while the stream still works on them, and it need not be the one that they were made on: the
+  // allocator is told, once for each stream.  Not of a stream that torch does not own (its number is its handle): it may
+  // be gone when the tensors go.
+  void used_on(int64_t id, hipStream_t stream) {
+    if (id == last_stream.load(std::memory_order_relaxed)) return;
+    if (id != 0 && id == reinterpret_cast<int64_t>(stream)) return;
+    std::lock_guard<std::mutex> lock(streams_mutex);
+    if (std::find(streams.begin(), streams.end(), id) == streams.end()) {
+      const auto on = c10::hip::HIPStream::unpack3(id, device.index(), c10::DeviceType::HIP);
+      const auto allocator = c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get();
+      for (const Tensor &t : keep) allocator->recordStream(t.storage().data_ptr(), on);
+      if (block.defined()) allocator->recordStream(block.storage().data_ptr(), on);
+      streams.push_back(id);
+    }
+    last_stream.store(id, std::memory_order_relaxed);
+  }
+  std::atomic<int64_t> last_stream{std::numeric_limits<int64_t>::min()};
+  std::mutex streams_mutex;
+  std::vector<int64_t> streams;  // that the allocator knows of (torch has some dozens)
   std::string name() const { return what; }
   // What apcost_run_bound takes (valid while the object lives).
   int64_t handle() const { return reinterpret_cast<int64_t>(this); }
@@ -961,14 +990,14 @@ int run_caught(F f) noexcept {
 extern "C" __attribute__((visibility("default"))) int apcost_run_bound(void *bound) {
   return run_caught([&] { static_cast<BoundLaunch *>(bound)->run(); });
 }
-extern "C" __attribute__((visibility("default"))) int apcost_run_bound_on(void *bound, int64_t stream) {
-  return run_caught([&] { static_cast<BoundLaunch *>(bound)->run_on(stream); });
+extern "C" __attribute__((visibility("default"))) int apcost_run_bound_on(void *bound, int64_t handle, int64_t id) {
+  return run_caught([&] { static_cast<BoundLaunch *>(bound)->run_on(handle, id); });
 }
 extern "C" __attribute__((visibility("default"))) const char *apcost_run_error(void) { return g_run_error.c_str(); }
 
 TORCH_LIBRARY(apcost, m) {
   m.class_<BoundLaunch>("BoundLaunch").def("run", &BoundLaunch::run).def("keep_arguments", &BoundLaunch::keep_arguments)
-      .def("run_on", &BoundLaunch::run_on).def("name", &BoundLaunch::name).def("handle", &BoundLaunch::handle);
+      .def("run_on", &BoundLaunch::run_on_handle).def("name", &BoundLaunch::name).def("handle", &BoundLaunch::handle);
 #define APCOST_TENSOR_TABLE "Tensor tensor_rank, Tensor tensor_itemsize, Tensor tensor_shape, Tensor tensor_stride"
 #define APCOST_STRATEGY_TABLE "Tensor flops, Tensor rw_bytes, Tensor dtype_code, Tensor zero_cost, Tensor num_args"
 #define APCOST_INPUT_TABLES                                                                                          \

@@ -384,7 +384,8 @@ class DeviceCostTables:
             (run, run_on), handle = _native.bound_runners(), bound.handle()
 
             def launch(on_stream=None):
-                if run(handle) if on_stream is None else run_on(handle, int(on_stream.cuda_stream)):
+                if run(handle) if on_stream is None else run_on(
+                        handle, int(on_stream.cuda_stream), int(getattr(on_stream, "stream_id", on_stream.cuda_stream))):
                     raise _native.bound_error()
             launch.bound = bound  # (what the handle names lives as long as its launcher)
             return launch

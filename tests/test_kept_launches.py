@@ -138,3 +138,29 @@ def test_the_device_object_holds_the_launches_of_its_latest_step(gpu_device):
         del step
         gc.collect()
         assert all(b() is not None for b in bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("as_current", [True, False])
+def test_what_a_launch_on_another_stream_uses_is_not_given_out_before_it_ran(gpu_device, as_current):
+    """Launches behind other work of a second stream; everything is dropped, and arrays of the same sizes are allocated before
+    that stream gets to them."""
+    mesh = (16, 8, 4)
+    tb = stress_dag(seed=6, n_nodes=400, mesh_sizes=mesh, max_strategies=30)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
+    step = d.prepare_step(row_min=False, fused_inputs=True, outputs=("cost",), spec_table=False, packed=False)
+    arrays = (d.cost, d.compute_cost, d.compute_cost_per_arg, d.tensor_bytes)
+    used = {t.data_ptr() for t in arrays}
+    sizes = [t.numel() for t in arrays]
+    side = torch.cuda.Stream(device=d.device)
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(400_000_000)  # (0.2 s)
+        for launch in step.values():
+            launch() if as_current else launch(side)
+    del d, step, launch, arrays
+    others = [torch.full((n,), 7, dtype=torch.int64, device=gpu_device) for n in sizes for _ in range(3)]
+    assert not side.query()  # (it had not got to the launches)
+    assert used.isdisjoint(t.data_ptr() for t in others)
+    torch.cuda.synchronize()
+    assert all(bool((t == 7).all()) for t in others)
