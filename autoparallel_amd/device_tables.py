@@ -514,8 +514,9 @@ class DeviceCostTables:
             main = torch.cuda.current_stream()
             for b in branches:
                 b.wait_stream(main)
-            if "build_tables" in step:
-                step["build_tables"](main)
+            one_launch = step.get("build_tables") or step.get("build_tables_packed")
+            if one_launch is not None:
+                one_launch(main)
             elif "input_tables" in step:
                 step["input_tables"](main)
             else:

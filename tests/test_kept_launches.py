@@ -99,13 +99,14 @@ def test_kept_launches_write_what_launches_by_value_write(gpu_device, mesh):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("one_launch", [True, False])
-def test_a_graph_holds_what_its_launches_read(gpu_device, one_launch):
+@pytest.mark.parametrize("kind", [dict(one_launch=True, packed=False), dict(one_launch=False, packed=False),
+                                  dict(packed=True, row_min=True, row_min_in_tiles=True)])
+def test_a_graph_holds_what_its_launches_read(gpu_device, kind):
     """``step`` and then the tables' device object are dropped: a graph of the pass still has the blocks of its launches."""
     mesh = (16, 8, 4)
     tb = stress_dag(seed=4, n_nodes=300, mesh_sizes=mesh, max_strategies=20)
     d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
-    form = dict(row_min=False, fused_inputs=True, outputs=("cost",), spec_table=False, one_launch=one_launch, packed=False)
+    form = dict(dict(row_min=False, fused_inputs=True, outputs=("cost",), spec_table=False), **kind)
     step = d.prepare_step(**form)
     launches = [weakref.ref(launch) for launch in step.values()]
     graph = d.capture_step_graph(step)
