@@ -71,7 +71,8 @@ class DeviceCostTables:
             tables.validate(params)
         self.c_params = params.to_c()
         self.p = _native.params_tensor(self.c_params)  # struct apc_params as the operators take it
-        self.d = dict(zip(_UPLOAD, self._upload(*(getattr(tables, k) for k in _UPLOAD))))
+        self.d = {}
+        self._refresh(_UPLOAD)
         self.tensor_bytes = None
         self.tensor_contiguous = None
         self.compute_cost = None
@@ -86,7 +87,15 @@ class DeviceCostTables:
     def refresh(self, *names):
         """Re-uploads host tables that changed after construction (strategy inputs filled in
         from the shard-shape table, tiles rebuilt with de-duplication)."""
-        self.d.update(zip(names, self._upload(*(getattr(self.tables, k) for k in names))))
+        self._refresh(names)
+
+    def _refresh(self, names):
+        arrays = [getattr(self.tables, k) for k in names]
+        self.d.update(zip(names, self._upload(*arrays)))
+        if "tile_records" in names:
+            # (the host's table may be tiled anew before it is uploaded again: what is on the device stays one tiling)
+            self._tiles = self.d["tile_records"], arrays[names.index("tile_records")]
+            self._ordered_tiles = None
 
     # ---- helpers -------------------------------------------------------------------------
     def _upload(self, *arrays):
@@ -307,18 +316,15 @@ class DeviceCostTables:
         return dev
 
     def _tile_records(self, repeated):
-        """The device copy of the tile records, in launch order for a pass that is repeated."""
-        tb = self.tables
-        if not repeated:
+        """The device copy of the tile records, in launch order for a pass that is repeated: of the tiling that is on the
+        device with its copies' offsets."""
+        on_device, records = self._tiles
+        if not repeated or self.d["tile_records"] is not on_device:
             return self.d["tile_records"]
-        cached = getattr(self, "_ordered_cache", None)
-        if cached is None or cached[0] is not tb.tile_records or cached[1] is not self.d["tile_records"]:
-            records = tb.launch_records()
-            on_device = self.d["tile_records"]
-            if records is not tb.tile_records:
-                on_device = _to_device(records, self.device)
-            cached = self._ordered_cache = (tb.tile_records, self.d["tile_records"], on_device)
-        return cached[2]
+        if self._ordered_tiles is None:
+            ordered = self.tables.launch_records(records)
+            self._ordered_tiles = on_device if ordered is records else _to_device(ordered, self.device)
+        return self._ordered_tiles
 
     @_guarded
     def prepare_step(self, row_min=True, fused_inputs=False, one_launch=None, row_min_in_tiles=None,

@@ -508,13 +508,18 @@ class CostTables:
         return self.n_entries <= ORDERED_MAX_ENTRIES and ORDERED_MIN_PER_TILE * n_tiles <= computed \
             and self.n_entries <= ORDERED_MAX_COPIES * computed
 
-    def launch_records(self) -> np.ndarray:
-        """``tile_records`` in the order in which a launch takes them."""
-        if not self.largest_tiles_first_pays():
-            return self.tile_records
-        records = self._records(self.tile_records, self.n_tiles, TILE_DTYPE)
-        ordered = np.empty(self.n_tiles, TILE_DTYPE)
-        _native.host_call("apc_order_tiles_host", self.n_tiles, records, ordered)
+    def launch_records(self, records: Optional[np.ndarray] = None) -> np.ndarray:
+        """``tile_records``, or the ``records`` of an earlier tiling, in the order in which a launch takes them."""
+        if records is None:
+            records, n, pays = self.tile_records, self.n_tiles, self.largest_tiles_first_pays()
+        else:
+            n = len(records)
+            computed = int(((records["counts"] & 0xFFFF).astype(np.int64) * (records["counts"] >> 16)).sum())
+            pays = n > 0 and self._orders(computed, n)
+        if not pays:
+            return records
+        ordered = np.empty(n, TILE_DTYPE)
+        _native.host_call("apc_order_tiles_host", n, self._records(records, n, TILE_DTYPE), ordered)
         return ordered
 
     def computed_entries(self) -> int:
