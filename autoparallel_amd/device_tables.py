@@ -307,9 +307,9 @@ class DeviceCostTables:
 
     def _packed_tiles(self, repeated):
         """The device copy of ``CostTables.pack_tiles()``, made once per tiling; in launch order for a pass that is repeated
-        (the order costs the host more than it saves one launch)."""
+        (the order costs the host more than it saves one launch, which takes a copy that is there in either)."""
         cached = getattr(self, "_packed_cache", None)
-        if cached is not None and cached[0] is self.tables.tile_records and cached[1] == repeated:
+        if cached is not None and cached[0] is self.tables.tile_records and (cached[1] or not repeated):
             return cached[2]
         dev = _to_device(self.tables.pack_tiles(self.tables.launch_records() if repeated else None), self.device)
         self._packed_cache = (self.tables.tile_records, repeated, dev)
@@ -346,8 +346,11 @@ class DeviceCostTables:
         ``None`` takes them when the pass is of that kind, ``packed_pass_pays`` and staged tiles
         (``CostTables.staging_pays``) are not faster still.  ``repeated=False``: the pass will run once, and the arguments
         of its launches are not laid out in device memory first (``apc_kept_launch``: one copy, for 2 to 4 us less a launch),
-        nor its tiles put into launch order (``CostTables.launch_records``: 10 ns a tile on the host)."""
+        nor its tiles put into launch order (``CostTables.launch_records``: 10 ns a tile on the host).  Those copies, one a launch
+        and one of the tiles, are waited for.  So are the uploads of row indices and packed tiles (made once); a pass that needs
+        none of them can be prepared while the current stream captures, and is then prepared as with ``repeated=False``."""
         tb = self.tables
+        repeated = bool(repeated) and not torch.cuda.is_current_stream_capturing()
         outputs = tuple(outputs)
         if not outputs or any(o not in ("comm", "transition", "cost") for o in outputs):
             raise ValueError(f"outputs must name some of comm, transition, cost: {outputs}")
@@ -407,7 +410,7 @@ class DeviceCostTables:
         if packed:
             step = {"build_tables_packed": bind(ops.bind_cost_tables_packed(
                 self.p, *self._tensor_table(), self.tensor_bytes, self.tensor_contiguous, *self._strategy_table(),
-                self.compute_cost, self.compute_cost_per_arg, err, d["pt_values"], self._packed_tiles(bool(repeated)), tb.n_entries, tb.n_rows,
+                self.compute_cost, self.compute_cost_per_arg, err, d["pt_values"], self._packed_tiles(repeated), tb.n_entries, tb.n_rows,
                 self.cost, self.row_min, self.row_argmin))}
         elif one_launch:
             step = {"build_tables": bind(ops.bind_cost_tables(

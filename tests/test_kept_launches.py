@@ -165,3 +165,27 @@ def test_what_a_launch_on_another_stream_uses_is_not_given_out_before_it_ran(gpu
     assert used.isdisjoint(t.data_ptr() for t in others)
     torch.cuda.synchronize()
     assert all(bool((t == 7).all()) for t in others)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [dict(one_launch=True, packed=False), dict(one_launch=False, packed=False), dict(fused_inputs=False, spec_table=True),
+                                  dict(packed=True, row_min=True, row_min_in_tiles=True)])
+def test_a_pass_is_prepared_while_the_stream_captures(gpu_device, form):
+    """Without copies: of packed tiles, those of an earlier preparation are taken."""
+    mesh = (16, 8, 4)
+    tb = stress_dag(seed=12, n_nodes=250, mesh_sizes=mesh, max_strategies=20)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
+    form = dict(dict(row_min=False, fused_inputs=True, outputs=("cost",), spec_table=False), **form)
+    if form.get("packed"):
+        d.prepare_step(**form)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step = d.prepare_step(**form)
+        for launch in step.values():
+            launch()
+    want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh, rescale=2.2))["cost"]
+    for _ in range(3):
+        d.cost.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(d.cost.cpu().numpy(), want)
