@@ -79,8 +79,11 @@ ORDERED_MAX_ENTRIES = 32_000_000
 ORDERED_MAX_COPIES = 4
 ORDERED_MIN_PER_TILE = 64
 # Their largest tiles are no tail, and may be larger than AUTO_MIN_STORED_PER_TILE would have them: 2048 / 4096 entries, 20 M on
-# (16, 8, 4) 63.5 (924 values) / 62.1 us, 27 M 83.4 (910) / 78.0, 5.1 M on (3, 2, 2, 2) 48.3 (868) / 44.5; 1024 / 2048 / 4096,
-# 5.3 M in two layers on (64, 4) 21.7 (960) / 20.9 (1 240) / 24.1.  (While there are tiles for more than a round or two.)
+# (16, 8, 4) 66.5 (924 values) / 63.9 us, on (64, 4) 63.4 / 66.9, 30 M 92.1 (928) / 86.6 and 90.2 / 84.3, 14 M 59.6 (934) / 57.0 and
+# 57.0 / 53.8, 5.2 M 25.0 (952) / 23.6 and 22.5 / 23.8, on (2, 4, 2, 2) 27.5 / 26.8; 1024 / 2048 / 4096, 5.3 M in two layers on (64, 4)
+# 21.7 (960) / 20.9 (1 240) / 24.1.  (While there are tiles for more than a round or two.)  Only in that order: the same tables edge by
+# edge, which is how one that is launched once goes, 71.5 / 78.4 us, 70.0 / 76.2, 94.1 / 98.2, 93.1 / 96.6, 64.2 / 64.9, 62.1 / 63.7,
+# 29.8 / 33.9, 27.8 / 31.6, 34.0 / 39.9, with all three arrays written 95.9 / 103.7, 93.8 / 102.8 and so on.
 ORDERED_MIN_STORED_PER_TILE, ORDERED_SOME_ROUNDS = 1000, 4000
 # A table this small is bound by the latency of one workgroup, not by work: it keeps the largest
 # tiles and up to 16 copies per tiled edge (Llama-3-8B on (32, 8), 1.8 M entries: 13.3 us with
@@ -101,6 +104,8 @@ STAGED_MIN_COMPUTED_PER_TILE = {1: 100, 2: 100, 3: 100, 4: 180}
 # 399 k entries on (8, 8, 8) 6.6 (1 181 tiles) / 6.7 / 7.7 / 8.4 us, 850 k 9.4 / 8.6 / 8.7 (1 270 tiles) / 9.3; 420 k on
 # (12, 6) 7.0 (1 265) / 7.1 / 7.9 / 8.3, 2.6 M 15.2 / 12.5 / 11.6 (2 431) / 11.9; 1.6 M on (32, 8) 16.2 / 13.6 / 13.5 (2 718) /
 # 13.3, on (6, 4, 2), without the minima, 2048 (2 930) 13.7, 4096 14.4; 587 k in 3 353 edges on (6, 4, 2) 14.8 (3 500) / 14.3.
+# Edge by edge they lose little where they lose: 512 / 1024, 1.1 M on (12, 6) 11.2 / 11.3, on (32, 8) 10.7 / 11.2, on (6, 4, 2) 13.6 /
+# 12.3, 1.3 M 10.2 / 9.2, 9.6 / 9.1, 11.7 / 10.2; 1024 / 2048, 2.6 M on (12, 6) 12.7 / 13.8.
 STAGED_TILES, STAGED_SMALLEST_SHARE, STAGED_MIN_TILE_ENTRIES = 2800, 750, 512
 # On a 4-D mesh with a size that is no power of two a tile stages 304 states: fewer, larger tiles.  On both sides of the
 # 900, with row minima in the tiles: (3, 2, 2, 2), 530 k entries, whole edges (979 tiles) 19.4, 1024 17.5; 1.8 M, 39.8, 41.7; 658 k
@@ -388,7 +393,7 @@ class CostTables:
         return out
 
     def build_tiles(self, tile_entries: Optional[int] = None, dedupe: bool = False, max_copies: int = 16,
-                    signatures=None, rows_per_wavefront_pass: Optional[int] = None) -> None:
+                    signatures=None, rows_per_wavefront_pass: Optional[int] = None, repeated: bool = True) -> None:
         """Cuts every edge matrix into rectangles of about ``tile_entries`` entries:
         whole rows when a row fits the LDS column budget, column chunks otherwise.  With
         ``dedupe`` only the first of every group of identical edges is tiled; its tiles
@@ -402,7 +407,9 @@ class CostTables:
         of a small table, whose slowest workgroup decides the launch; the automatic choice sets it
         to 4 for such a table unless ``staging_pays`` or its rows are too wide to pack).
         ``signatures``: with a tile size and ``dedupe``, one value per edge, equal where matrices are
-        (as of ``edge_signatures``); without, edges are compared by content."""
+        (as of ``edge_signatures``); without, edges are compared by content.  ``repeated=False``: tile sizes for launches that
+        go edge by edge (a pass that runs once, a report); the default ones are for a repeated pass, which takes the tiles of
+        some tables by size (``largest_tiles_first_pays``)."""
         classes = None
         if dedupe and self.n_edges and signatures is not None and tile_entries is not None:
             first: dict = {}
@@ -450,7 +457,7 @@ class CostTables:
                 while self.n_entries > n * AUTO_MAX_STORED_PER_TILE and mc > 2 and n_dups:
                     mc //= 2
                     n, n_dups = count(te, mc, 0)
-                ordered = self._orders(computed(), n)
+                ordered = repeated and self._orders(computed(), n)
                 while te < APC_TILE_MAX_ROWS * APC_TILE_MAX_COLS:
                     stored = ORDERED_MIN_STORED_PER_TILE if ordered and n > ORDERED_SOME_ROUNDS else AUTO_MIN_STORED_PER_TILE
                     if self.n_entries >= n * stored and not (te > AUTO_MIN_TILE_ENTRIES and n > AUTO_MANY_TILES):

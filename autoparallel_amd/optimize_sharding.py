@@ -109,7 +109,7 @@ class DeviceBackend:
 
     def upload_strategy_inputs(self, tables, tile_entries=None, dedupe=True, max_copies=16):
         """The strategy table is final: tile the edges (identical edges once) and send both."""
-        tables.build_tiles(tile_entries, dedupe=dedupe, max_copies=max_copies)
+        tables.build_tiles(tile_entries, dedupe=dedupe, max_copies=max_copies, repeated=False)
         tables.validate(self.dev.params)
         names = ("tile_records", "dup_entry_begin", "dup_row_begin")
         if not getattr(self, "_strategy_inputs_on_device", False):

@@ -7,6 +7,7 @@ import torch
 
 from autoparallel_amd import CostModelParams, encoding
 from autoparallel_amd.device_tables import DeviceCostTables
+from autoparallel_amd.optimize_sharding import DeviceBackend
 from autoparallel_amd.synthetic import stress_dag
 from oracle import c_oracle
 from oracle import cost_oracle as po
@@ -62,6 +63,34 @@ def test_tiles_are_cut_larger_when_there_are_many_anyway(many, te, monkeypatch):
     tb.build_tiles(None, dedupe=True)
     assert tb.tiling["tile_entries"] == te and tb.n_tiles > 100
     tb.validate(CostModelParams.from_mesh((16, 8, 4)))
+
+
+def test_tile_sizes_for_launches_that_go_edge_by_edge(monkeypatch):
+    """The larger tiles of a table whose repeated pass takes them by size are not for a pass that runs once, which the
+    planner's is."""
+    monkeypatch.setattr(encoding, "AUTO_SMALL_TABLE_ENTRIES", 0)
+    monkeypatch.setattr(encoding, "ORDERED_SOME_ROUNDS", 100)
+    mesh = (16, 8, 4)
+    tb = stress_dag(seed=3, n_nodes=300, mesh_sizes=mesh, min_strategies=4, max_strategies=64, fanout_lambda=2.0)
+    tb.build_tiles(None, dedupe=True)
+    assert tb.largest_tiles_first_pays() and tb.tiling["tile_entries"] == 4096
+    whole = tb.tiling["whole_edges"]
+    tb.build_tiles(None, dedupe=True, repeated=False)
+    assert tb.tiling["tile_entries"] == 2048 and tb.tiling["whole_edges"] == whole
+    tb.validate(CostModelParams.from_mesh(mesh))
+    asked = tb.tile_records.copy()
+
+    class Device:
+        params = CostModelParams.from_mesh(mesh)
+
+        def refresh(self, *names):
+            pass
+
+    tb.build_tiles(None, dedupe=True)
+    backend = object.__new__(DeviceBackend)
+    backend.dev = Device()
+    backend.upload_strategy_inputs(tb)
+    assert np.array_equal(tb.tile_records, asked)
 
 
 @pytest.mark.gpu
