@@ -400,12 +400,15 @@ struct BoundLaunch : torch::CustomClassHolder {
   // Called by whoever bound the launch, before anyone runs it.
   void keep_arguments() {
     if (!recordable || kept) return;
+    c10::hip::HIPGuard guard(device.index());
+    const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(device.index());
     auto k = std::make_unique<apc_kept_launch>();
     check_rc(apc_keep_next_launch(k.get()), what.c_str());
     check_rc(launch(nullptr), what.c_str());
     if (k->kernel)
       block = upload({at::from_blob(k->block, {(int64_t)k->block_bytes}, at::TensorOptions().dtype(at::kByte))}, device)[0];
     kept = std::move(k);
+    used_on(stream.id(), stream.stream());  // (where it will most likely run: not the first pass's time)
   }
   void enqueue(void *stream) {
     check_rc(kept ? apc_run_kept(kept.get(), block.defined() ? block.data_ptr() : nullptr, stream) : launch(stream), what.c_str());
