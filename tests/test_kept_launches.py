@@ -3,6 +3,10 @@ against the same launches with their arguments passed by value."""
 
 import ctypes
 import gc
+import os
+import re
+import shutil
+import subprocess
 import weakref
 
 import numpy as np
@@ -16,11 +20,15 @@ from oracle import c_oracle
 from oracle import cost_oracle as po
 
 
+_HEADER = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include", "apcost.h")
+_BLOCK_BYTES = int(re.search(r"#define APC_KEPT_BLOCK_BYTES (\d+)", open(_HEADER).read()).group(1))
+
+
 class _Kept(ctypes.Structure):  # include/apcost.h: apc_kept_launch
     _fields_ = [("kernel", ctypes.c_void_p), ("what", ctypes.c_char_p), ("grid", ctypes.c_uint32), ("threads", ctypes.c_uint32),
                 ("lds_bytes", ctypes.c_uint32), ("block_bytes", ctypes.c_uint32), ("work", ctypes.c_void_p),
                 ("n_tiles", ctypes.c_int32), ("xcd_shift", ctypes.c_int32), ("tile_blocks", ctypes.c_int64),
-                ("cost_out", ctypes.c_void_p), ("block", ctypes.c_int64 * 384)]
+                ("cost_out", ctypes.c_void_p), ("block", ctypes.c_int64 * (_BLOCK_BYTES // 8)), ("kernel_by_value", ctypes.c_void_p)]
 
 
 def _redistribute(lib, params, n_tiles, per_arg):
@@ -47,9 +55,41 @@ def test_recording_a_launch_checks_it_and_ends_with_it():
     assert lib.apc_keep_next_launch(ctypes.byref(kept)) == 0
     assert _redistribute(lib, params, 3, one) == 0
     assert kept.kernel and kept.what == b"apc_redistribute_tables" and kept.n_tiles == 3 and kept.grid == 8
-    assert 0 < kept.block_bytes <= ctypes.sizeof(kept) - _Kept.block.offset
+    assert 0 < kept.block_bytes <= _BLOCK_BYTES and kept.kernel_by_value == kept.kernel  # (a kernel with one form)
     assert lib.apc_run_kept(ctypes.byref(kept), ctypes.c_void_p(8), None) != 0  # the block's alignment
     assert b"64-byte" in lib.apc_last_error()
+
+
+def test_the_kept_launch_mirrors_the_header(tmp_path):
+    fields = [name for name, _ in _Kept._fields_]
+    source = "#include <stdio.h>\n#include <stddef.h>\n#include \"apcost.h\"\nint main(void) {\n" + "".join(
+        f'printf("%zu ", offsetof(apc_kept_launch, {name}));\n' for name in fields) + 'printf("%zu", sizeof(apc_kept_launch));\nreturn 0; }\n'
+    (tmp_path / "layout.c").write_text(source)
+    subprocess.run([shutil.which("gcc") or "cc", f"-I{os.path.dirname(_HEADER)}", "-o", str(tmp_path / "layout"), str(tmp_path / "layout.c")],
+                   check=True)
+    got = [int(x) for x in subprocess.run([str(tmp_path / "layout")], check=True, capture_output=True, text=True).stdout.split()]
+    assert got == [getattr(_Kept, name).offset for name in fields] + [ctypes.sizeof(_Kept)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", [dict(packed=True, row_min=True, row_min_in_tiles=True), dict(one_launch=True, packed=False),
+                                  dict(one_launch=False, packed=False)])
+def test_kept_launches_without_a_block(gpu_device, form):
+    """``apc_run_kept`` with a NULL block: the recorded arguments by value, through the form of the kernel that takes them."""
+    mesh, lib = (16, 8, 4), _native.lib()
+    tb = stress_dag(seed=10, n_nodes=250, mesh_sizes=mesh, max_strategies=20)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
+    step = d.prepare_step(**dict(dict(row_min=False, fused_inputs=True, outputs=("cost",), spec_table=False), **form), repeated=False)
+    d.cost.zero_()
+    for launch in step.values():
+        kept = _Kept()
+        assert lib.apc_keep_next_launch(ctypes.byref(kept)) == 0
+        launch()  # (recorded and not enqueued)
+        assert kept.kernel and kept.kernel_by_value
+        for _ in range(2):
+            assert lib.apc_run_kept(ctypes.byref(kept), None, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    torch.cuda.synchronize()
+    assert np.array_equal(d.cost.cpu().numpy(), c_oracle.build_tables(tb.as_dict(), po.make_params(mesh, rescale=2.2))["cost"])
 
 
 def _outputs(d):
