@@ -249,14 +249,14 @@ class DeviceCostTables:
 
     def row_min_in_tiles_pays(self) -> bool:
         """Whether the launch that writes the cost matrices should take the row minima itself.
-        Inside the tiles the minima cost about 0.5 ns per tile (a barrier and the stores of the
-        row results) plus 1.6 ps per entry a tile computes (identical edges are computed, and
-        reduced, once for all their copies); a ``segmented_min`` launch costs about 4 us plus
-        reading every stored entry back at about 4.5 TB/s.  Measured, in tiles / separate:
-        Llama-3-8B on (32, 8), whose tiles compute an eighth of the entries they store, 18.8 /
-        23.9 us per pass with all three arrays written; the 464 M-entry stress table, where every
-        entry is computed, 2.42 ms for the launch that writes the cost alone with the minima
-        against 1.45 ms without them plus 0.87 ms for the separate launch."""
+        Priced inside the tiles: 0.5 ns per tile and 1.6 ps per entry a tile computes (identical edges are computed, and
+        reduced, once for all their copies); as a ``segmented_min`` launch: 4 us and every stored entry read back at 4.5 TB/s.
+        The first two are what minima across the lanes of a wavefront and a barrier a tile took.  With the rows of a wavefront
+        joined through its LDS the minima of tables that compute every entry cost 1.0 - 1.4 ps an entry, so the rule
+        is early to leave them to the separate launch.  Cost alone, us a pass without minima / in tiles / separate, by size:
+        5.2 M entries on (12, 6) 21.0 / 27.8 / 30.3, 9.4 M on (16, 8, 4) 29.0 / 42.3 / 50.7, on (2, 4, 2, 2) 35.4 / 46.2 / 52.7; where the
+        rule says separate: 20 M on (16, 8, 4) 65.1 / 85.0 / 96.6, 3.6 M on (64, 4) 17.3 / 22.3 / 25.5 (edge by edge 20.3 / 30.2 /
+        28.5).  It decides whether a planner finds the minima taken, and stays."""
         tb = self.tables
         if tb.n_tiles == 0 or not tb.rows_fit_tiles():
             return False
@@ -345,8 +345,9 @@ class DeviceCostTables:
         (``apc_build_tables_packed``: the assembled cost and the row minima, no spec table);
         ``None`` takes them when the pass is of that kind, ``packed_pass_pays`` and staged tiles
         (``CostTables.staging_pays``) are not faster still.  ``repeated=False``: the pass will run once, and the arguments
-        of its launches are not laid out in device memory first (``apc_kept_launch``: one copy, for 2 to 4 us less a launch),
-        nor its tiles put into launch order (``CostTables.launch_records``: 10 ns a tile on the host).  Those copies, one a launch
+        of its launches are not laid out in device memory first (``apc_kept_launch``: one copy, for 0.75 us less a launch over packed
+        tiles or a large table, nothing where staged tiles wait for other loads at that time), nor its tiles put
+        into launch order (``CostTables.launch_records``: 10 ns a tile on the host).  Those copies, one a launch
         and one of the tiles, are waited for.  So are the uploads of row indices and packed tiles (made once); a pass that needs
         none of them can be prepared while the current stream captures, and is then prepared as with ``repeated=False``."""
         tb = self.tables
