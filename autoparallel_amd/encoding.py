@@ -83,7 +83,9 @@ ORDERED_MIN_PER_TILE = 64
 # 57.0 / 53.8, 5.2 M 25.0 (952) / 23.6 and 22.5 / 23.8, on (2, 4, 2, 2) 27.5 / 26.8; 1024 / 2048 / 4096, 5.3 M in two layers on (64, 4)
 # 21.7 (960) / 20.9 (1 240) / 24.1.  (While there are tiles for more than a round or two.)  Only in that order: the same tables edge by
 # edge, which is how one that is launched once goes, 71.5 / 78.4 us, 70.0 / 76.2, 94.1 / 98.2, 93.1 / 96.6, 64.2 / 64.9, 62.1 / 63.7,
-# 29.8 / 33.9, 27.8 / 31.6, 34.0 / 39.9, with all three arrays written 95.9 / 103.7, 93.8 / 102.8 and so on.
+# 29.8 / 33.9, 27.8 / 31.6, 34.0 / 39.9, with all three arrays written 95.9 / 103.7, 93.8 / 102.8 and so on; the planner's one launch, on
+# what has just been uploaded, 5.2 M 42.2 / 46.1, 40.0 / 45.0 and on (8, 8, 8) 42.4 / 46.9, 20 M 67.7 / 74.7, 69.2 / 76.6, 74.2 / 78.6, 14 M
+# 75.7 / 77.9, 72.9 / 73.3, 75.7 / 77.4; the other way 9.4 M, 61.9 / 61.0, 59.3 / 58.1, 63.1 / 61.1.
 ORDERED_MIN_STORED_PER_TILE, ORDERED_SOME_ROUNDS = 1000, 4000
 # A table this small is bound by the latency of one workgroup, not by work: it keeps the largest
 # tiles and up to 16 copies per tiled edge (Llama-3-8B on (32, 8), 1.8 M entries: 13.3 us with
