@@ -196,13 +196,15 @@ def test_what_a_launch_on_another_stream_uses_is_not_given_out_before_it_ran(gpu
     side = torch.cuda.Stream(device=d.device)
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
-        torch.cuda._sleep(400_000_000)  # (0.2 s)
+        torch.cuda._sleep(1_000_000_000)  # (half a second)
         for launch in step.values():
             launch() if as_current else launch(side)
     del d, step, launch, arrays
-    others = [torch.full((n,), 7, dtype=torch.int64, device=gpu_device) for n in sizes for _ in range(3)]
+    others = [torch.empty(n, dtype=torch.int64, device=gpu_device) for n in sizes for _ in range(3)]
     assert not side.query()  # (it had not got to the launches)
     assert used.isdisjoint(t.data_ptr() for t in others)
+    for t in others:
+        t.fill_(7)
     torch.cuda.synchronize()
     assert all(bool((t == 7).all()) for t in others)
 
