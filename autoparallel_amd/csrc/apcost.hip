@@ -101,7 +101,8 @@ __device__ __forceinline__ void store_through(T *p, T value) {
 // 8.15 us, 20 M on (16, 8, 4) in two launches 70.2 -> 68.7, 2.6 M on (12, 6) over staged tiles, whose wavefronts have other
 // loads to wait for at that time, 18.4 -> 18.7.)
 // The host fills the by-value arguments in, and waits for room for them, for every launch, read or not.  The kernels of small passes,
-// which last no longer than that, have a form without them (KEPT); the others choose where they run.  (Together with a call that
+// which last no longer than that, have a form without them (KEPT); the others, the two-launch passes' among them, choose where
+// they run (every such form is one more kernel to compile: the library 4.7 -> 6.0 MB).  (Together with a call that
 // does not go through boxed values: one block on (64,) 4.95 -> 3.3 us a pass, 399 k entries on (8, 8, 8) 7.0 -> 6.55, 420 k on (12, 6)
 // 7.1 -> 6.6.)
 constexpr size_t kLaunchHeadBytes = 40;
