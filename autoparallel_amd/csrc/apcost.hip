@@ -354,17 +354,19 @@ __device__ __forceinline__ double entry_cost(uint32_t srcp, uint32_t tgtp, doubl
 // hold the last dim, a quarter of the pairs, and are counted without it.  (4-D meshes: 304 states
 // where all pairs are 496, in 22 KB of LDS instead of 36: four workgroups to a compute unit, not three.  5.1 M entries on
 // (3, 2, 2, 2) 45.1 -> 33.7 us, 900 k 18.8 -> 13.7; 72 of 120 on 3-D meshes, 587 k on (6, 4, 2) 14.1 -> 12.0, 1.6 M 14.0 -> 12.2.)
+// They are numbered mask by mask, and the states of a mask by level and history: a producer spec's first one and the
+// place within its mask add up, so what an entry looks up by its two classes is the same for every producer spec.
 // ------------------------------------------------------------------------------------------
 template <int M>
 struct States {
-  static constexpr int kLast = ((1 << M) - 1) << M;  // the first of level M
   static constexpr int kHalf = 1 << (M - 1);
+  static constexpr int kPerMask = (1 << M) - 1;       // levels 0 .. M - 1
+  static constexpr int kLast = kPerMask << M;         // of all masks; behind them, as they are counted below, level M
   static constexpr int kCount = kLast + kHalf * kHalf;
-  __device__ static __forceinline__ int last(int mask, int hist) {
-    return kLast + ((mask & (kHalf - 1)) << (M - 1)) + (hist & (kHalf - 1));
-  }
+  // the first state of a mask
+  __device__ static __forceinline__ int first(int mask) { return mask * kPerMask + (mask >= kHalf ? (mask & (kHalf - 1)) * kHalf : 0); }
   __device__ static __forceinline__ int index(int level, int mask, int hist) {
-    return (((1 << level) - 1) << M) + (mask << level) + hist;
+    return first(mask) + (level < M ? (1 << level) - 1 + hist : kPerMask + (hist & (kHalf - 1)));
   }
 };
 // ------------------------------------------------------------------------------------------
@@ -751,9 +753,8 @@ __global__ __launch_bounds__(kBlock) void input_tables_kernel(APC_LAUNCH_PARAMS(
 // ------------------------------------------------------------------------------------------
 
 // What is the same for every tile of a launch (see "Term arrays" and "Lookup words" below):
-// the layout of the term arrays, the part of the lookup words that does not depend on the
-// producer spec (by dim x 16 + producer class x 4 + consumer class; the producer spec's state
-// or exponent index is added when a tile is staged) and, for the power-of-two layout, the
+// the layout of the term arrays, the lookup words (by dim x 16 + producer class x 4 + consumer
+// class), how a producer spec's running index starts and, for the power-of-two layout, the
 // constants of every computed array.
 constexpr int kMaxTermArrays = 16;
 struct TermArrayConstants {  // value at exponent index j = max(lat + ldexp(B, j + shift), floor) x scale,
@@ -771,6 +772,10 @@ struct TermLayout {
   int32_t exponents;         // 0: general layout; else E, the number of exponents
   int32_t lg[APC_MAX_MESH];  // log2 of the mesh sizes (power-of-two layout)
   int32_t lg_total;          // L
+  // the running index of a producer spec: index0 + the weights of the dims it shards + (general layout, where it shards
+  // the last dim) last_weight x the mask of its other dims
+  int32_t index0, index_weight[APC_MAX_MESH], last_weight;
+  int32_t level_stride;      // bytes from one level's states to the next's (general layout; else 0), in units of 2^level - 1
   int32_t state_stride;      // bytes between the entries of two consecutive states / exponents
   uint32_t exponent_magic;   // ceil(65536 / E): t / E = (t * magic) >> 16 for t < 512
   double inv_rescale;        // 1.0 / params.rescale
@@ -889,12 +894,12 @@ struct TermTable {
 };
 static_assert(4 + 3 * APC_MAX_MESH <= kMaxTermArrays, "arrays of the power-of-two layout");
 
-// Lookup words.  What a mesh dim adds to an entry depends on the producer spec (its class at
-// that dim and which dims it shards), on the consumer's class at that dim and on the running
-// index left by the earlier dims; everything but the running index is known per (producer
-// spec, dim, consumer class) when the tile is staged.  One 32-bit word per such triple, in
-// fields an instruction can take as a half or a byte of a register:
-//   bits  0-15  byte offset of the collective's term for running index 0 (general: array of
+// Lookup words.  What a mesh dim adds to an entry depends on the producer's and the consumer's class at
+// that dim and on the running index, which starts at the producer spec's own (general: the first state of its mask;
+// power-of-two meshes: L - log2 of its shards) and goes on by the earlier dims.  One 32-bit word per (dim, producer
+// class, consumer class), the same for every tile of a launch (TermLayout::pair), in fields an instruction can take as a
+// half or a byte of a register:
+//   bits  0-15  byte offset of the collective's term from the running index' entry (general: array of
 //               pair_action's term, state of the bytes the collective moves: after the update
 //               for an all-gather, before it else; the +inf array for a banned transition)
 //   bits 16-23  signed: bytes from there to the read+write term of the same state (zeros / one
@@ -902,23 +907,22 @@ static_assert(4 + 3 * APC_MAX_MESH <= kMaxTermArrays, "arrays of the power-of-tw
 //   bits 24-31  signed step of the running index after this dim (general: the dim's history
 //               bit; power-of-two meshes: + log2 n after an all-gather, - log2 n after a
 //               reduce-scatter)
-// Slot 4 of a (spec, dim) is the word of "same placement": zeros, no step; slot 5 is the byte
-// offset of one read+write at the state BEFORE the dim, charged once to a non-contiguous tensor.
-constexpr int kWordsPerDim = 6;
-// The words of a producer spec: the dims', on a 2-D mesh the four of its order flip (below), its codes.  An odd number,
-// so that the lanes of consecutive producer specs hit different banks.
+// Word 0 (dim 0, Replicate to Replicate) adds nothing and serves every dim of an entry whose placements are the same.
+// A producer spec's record and a consumer spec's hold a byte per dim, (16 class) and (64 dim + 4 class): their sum is
+// the offset of the dim's word, all dims in one addition.
+// (The words used to be made for every producer spec of a tile, with its own index added: 85 vector instructions of a tile's
+// first wavefront and 19 words of LDS a spec, 4.9 KB, read at a stride; now 20 instructions and two words, and lanes that
+// share a word read it together.  us a pass: 704 k entries on (6, 4, 2) 13.0 -> 11.5, 5.9 M on (2, 4, 2, 2) 33.0 -> 29.8, on (64, 4)
+// 28.5 -> 26.7, 584 k on (3, 2, 2, 2) 11.4 -> 10.8, 1.8 M on (16, 8, 4) 16.0 -> 15.6, 2.6 M on (12, 6) 11.8 -> 11.6; tables of which
+// the stores are what takes the time, 20 M on (16, 8, 4) and 66 M in 80 layers, as before, 62.7 and 127.)
 // A (Partial, Partial) producer on a 2-D mesh reaches an all-Shard consumer by two reduce-scatters, dim 1 first
 // (collective_runtime_estimation.py:146-151): words kFlipWord.. hold that walk, of dim 1 to Shard(0) and to another Shard,
 // then of dim 0, and byte 3 of the producer's codes holds the shift (kFlipShift, 0 for any other producer) that takes a
 // consumer's flip slots in place of its plain ones (RowRecord).
 constexpr uint32_t kFlipShift = 16;
+constexpr int kFlipWord = 2 * 16;
 template <int M>
-constexpr int kFlipWord = M * kWordsPerDim;
-template <int M>
-constexpr int kCodesWord = M * kWordsPerDim + (M == 2 ? 4 : 0);
-template <int M>
-constexpr int kColWords = kCodesWord<M> + 1;
-static_assert(kColWords<1> % 2 == 1 && kColWords<2> % 2 == 1 && kColWords<3> % 2 == 1 && kColWords<4> % 2 == 1, "an odd number of words");
+constexpr int kPairWords = M * 16 + (M == 2 ? 4 : 0);
 constexpr uint32_t kZerosArray = 0, kInfArray = 1, kRw1Array = 2;
 static_assert(TermTable<APC_MAX_MESH>::kEntries * 8 <= 0xFFFF + 1, "term offsets fit their 16 bits");
 
@@ -955,7 +959,10 @@ static TermLayout term_layout(const apc_params &p) {
         uint32_t term_array, state = 0;
         int step;
         if (!pow2) {
+          // the first state of the level within its mask; an all-gather (a sharding producer, a replicating consumer) is charged
+          // on the gathered bytes, those of the next level, behind the last dim without its history bit (States)
           term_array = ban ? kInfArray : sel == 0u ? kZerosArray : 3u + sel;
+          state = sel != 1u ? (1u << i) - 1u : (2u << i) - 1u + (i + 1 < M ? 1u << i : 0u);
           step = upd ? (1 << i) : 0;
         } else {
           if (sel == 1u) state = (uint32_t)lay.lg[i];  // an all-gather is charged on the gathered bytes
@@ -966,6 +973,18 @@ static TermLayout term_layout(const apc_params &p) {
         lay.pair[i * 16 + c * 4 + t] = (state * (uint32_t)lay.state_stride + term_array * 8u) | ((uint32_t)(to_rw & 0xFF) << 16) |
                                        ((uint32_t)(step & 0xFF) << 24);
       }
+  if (M == 2)
+    for (int k = 0; k < 4; ++k) {  // the order flip: (Partial -> Shard at dim 1, then at dim 0), of an unsharded producer
+      const int dim = k < 2 ? 1 : 0;
+      const uint32_t word = lay.pair[dim * 16 + 4 + 2 + (k & 1)];
+      // (general layout: both states are named outright, no step between them)
+      const uint32_t own = (1u << dim) - 1u, state = dim == 1 ? 1u : (uint32_t)States<2>::kCount;
+      lay.pair[kFlipWord + k] = pow2 ? word : (word & 0x00FFFFFFu) + (state - own) * (uint32_t)lay.state_stride;
+    }
+  lay.index0 = lay.lg_total;
+  for (int i = 0; i < M; ++i) lay.index_weight[i] = pow2 ? -lay.lg[i] : ((1 << M) - 1) << i;
+  lay.last_weight = pow2 ? 0 : 1 << (M - 1);
+  lay.level_stride = pow2 ? 0 : kGeneralStride;
   if (pow2) {
     const double ninf = -INFINITY;
     // one read+write, two (compute_estimation.py:302-314 on bytes x 2^(e + 31))
@@ -985,16 +1004,26 @@ static TermLayout term_layout(const apc_params &p) {
   return lay;
 }
 
-// A consumer spec of a tile: its placement codes; per mesh dim i, in byte i of `slots`, the
-// byte offset of its class's lookup word within a producer spec's words ((6 i + class) x 4;
-// byte 0 = 0xFF: not a DTensorSpec; on a 2-D mesh bytes 2 and 3 are what a (Partial, Partial) producer takes
-// instead: the same, or, when every dim is a Shard, the offsets of its two flip words); the compute
+// A consumer spec of a tile: its placement codes; per mesh dim i, in byte i of `slots`, its part of the byte offset of
+// the dim's lookup word, 64 i + 4 class (byte 0 = 0xFF: not a DTensorSpec; on a 2-D mesh bytes 2 and 3 are what a (Partial,
+// Partial) producer takes instead: the same, or, when every dim is a Shard, what leads to its two flip words); the compute
 // cost / num_args of its strategy.  One 16-byte LDS read per entry.
 struct alignas(16) RowRecord {
   uint32_t codes, slots;
   double cpa;
 };
-constexpr uint32_t kRowNotASpec = 0xFFu;
+// A producer spec: its placement codes (2-D: the flip's shift in byte 3); its part of the words' offsets, 16 class (byte 0 =
+// 0xFF as above); its running index, in the byte of `slots` behind the dims', on a 4-D mesh in a word of its own.
+template <int M>
+struct alignas(8) ColRecord {
+  uint32_t codes, slots;
+};
+template <>
+struct alignas(16) ColRecord<4> {
+  uint32_t codes, slots, index, pad_;
+};
+static_assert(States<3>::kCount <= 256 && kMaxExponents <= 256 && APC_MAX_MESH == 4, "a running index fits its byte");
+constexpr uint32_t kNotASpec = 0xFFu;
 
 // The part of TermArrayConstants a value needs after its array's chain.
 struct alignas(16) TermValueConstants {
@@ -1006,9 +1035,8 @@ struct alignas(16) TermValueConstants {
 template <int M, bool RM>
 struct TileStage {
   RowRecord row[APC_TILE_MAX_ROWS];  // consumer specs
-  uint2 colh[APC_TILE_MAX_COLS];  // producer specs: x = codes, y = info
-  uint32_t words[APC_TILE_MAX_COLS * kColWords<M>];  // lookup words per (producer spec, dim, consumer class), and its codes
-  alignas(16) uint32_t pair_base[M * 16];  // TermLayout::pair of the launch
+  ColRecord<M> col[APC_TILE_MAX_COLS];  // producer specs
+  uint32_t words[kPairWords<M>];        // TermLayout::pair of the launch
   int mixed[4];         // per staging wavefront: some spec is not a DTensorSpec on the tile's tensor (generic loop)
   int cont;             // the tile's tensor is contiguous
   // Last: the tile kernels size their LDS per launch for the entries the layout in use needs
@@ -1023,6 +1051,11 @@ template <int M, bool RM>
 __host__ __device__ constexpr uint32_t rows_at() {
   using Stage = TileStage<M, RM>;
   return (uint32_t)offsetof(Stage, row);
+}
+template <int M, bool RM>
+__host__ __device__ constexpr uint32_t cols_at() {
+  using Stage = TileStage<M, RM>;
+  return (uint32_t)offsetof(Stage, col);
 }
 template <int M, bool RM>
 __host__ __device__ constexpr uint32_t words_at() {
@@ -1129,10 +1162,10 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
   const TermLayout &lay = a.lay;
   const int E = lay.exponents;  // wave-uniform; 0: general layout
   const int lane = tid & 63, wave = tid >> 6;
-  // (written and read by the first wavefront only, which stages the producer specs: in order.
-  // A kernel argument indexed by the lane: one vector load, part of the round below.)
+  // (A kernel argument indexed by the lane: one vector load, part of the round below.)
+  static_assert(kPairWords<M> <= 64, "one word a lane of the smallest workgroup");
   uint32_t pair_word = 0;
-  if (tid < 16 * M) pair_word = lay.pair[tid];
+  if (tid < kPairWords<M>) pair_word = lay.pair[tid];
   // power-of-two layout: the constants of array 2 + lane (whose chain this lane computes) and of
   // the array of the first value this thread computes, also read by lane
   constexpr int kComputed = 3 * M + 2;
@@ -1249,9 +1282,9 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
       }
       return gb;
     };
-    const auto store_state = [&](int k, double gb, double ag, double rs, double ar) {
+    const auto store_state = [&](int state, double gb, double ag, double rs, double ar) {
       const double rw = rw_time_r(gb * 2 * 1073741824.0, p);
-      double *e = terms + __mul24(k, kGeneralStride / 8);
+      double *e = terms + __mul24(state, kGeneralStride / 8);
       e[kZerosArray] = 0.0;
       e[kInfArray] = __builtin_inf();
       e[kRw1Array] = rw;
@@ -1275,73 +1308,38 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
       double ag = 0.0, rs = 0.0, ar = 0.0, unused;
       if (level >= 1) rings_at<M>(gb, p, level - 1, ag, unused);
       if (level < M) rings_at<M>(gb, p, level, rs, ar);
-      store_state(k, gb, ag, rs, ar);
+      store_state(flip_state ? States<M>::kCount : States<M>::index(level, mask, hist), gb, ag, rs, ar);
     }
     if constexpr (kLastApart) {
       const int first = (tid + 8 * nthreads - 64 * ((kFirst + 63) / 64)) & (nthreads - 1);  // from the wavefronts that had fewer of the others
       for (int u = first; u < kHalf * kHalf; u += nthreads) {
-        const double gb = bytes_at(M, kHalf | (u >> (M - 1)), kHalf | (u & (kHalf - 1)));
+        const int mask = kHalf | (u >> (M - 1)), hist = kHalf | (u & (kHalf - 1));
+        const double gb = bytes_at(M, mask, hist);
         const double hops = (double)(p.mesh_size[M - 1] - 1);
         const double bw = div_by(div_by(gb * hops, (double)p.mesh_size[M - 1], p.inv_mesh[M - 1]), p.bw[M - 1], p.inv_bw[M - 1]);
-        store_state(kFirst + u, gb, (p.base_latency + hops * p.lat[M - 1]) + bw * 1e6, 0.0, 0.0);
+        store_state(States<M>::index(M, mask, hist), gb, (p.base_latency + hops * p.lat[M - 1]) + bw * 1e6, 0.0, 0.0);
       }
     }
   }
   // ---- what the loads brought, to LDS ---------------------------------------------------------
   if (tid == 0) st.cont = contiguous != 0;
-  if (tid < 16 * M) st.pair_base[tid] = pair_word;
+  if (tid < kPairWords<M>) st.words[tid] = pair_word;
   if (has_col) {
-    // info: bit0 valid spec, bit1 fully replicated, bits 4.. mask of sharded mesh dims
-    uint32_t info = (col_tensor >= 0 ? 1u : 0u) | (col_codes == 0u ? 2u : 0u);
-    uint32_t mask = 0;
+    uint32_t slots = 0, codes = col_codes, others = 0;
+    int index = lay.index0;
 #pragma unroll
-    for (int i = 0; i < M; ++i) mask |= (kind_of((col_codes >> (8 * i)) & 0xFF) == 2 ? 1u : 0u) << i;
-    info |= mask << 4;
-    st.colh[jc] = make_uint2(col_codes, info);
-    uint32_t *const w_of_col = st.words + __umul24((uint32_t)jc, (uint32_t)kColWords<M>);
-    w_of_col[kCodesWord<M>] = col_codes;
-    const auto words_of_dims = [&](auto pow2) {
-      constexpr bool POW2 = decltype(pow2)::value;
-      // power-of-two mesh: the producer spec's exponent index, L - log2(its shards)
-      uint32_t j0 = (uint32_t)lay.lg_total;
-      if constexpr (POW2) {
-#pragma unroll
-        for (int i = 0; i < M; ++i) j0 -= ((mask >> i) & 1u) ? (uint32_t)lay.lg[i] : 0u;
-      }
-#pragma unroll
-      for (int i = 0; i < M; ++i) {
-        const uint32_t cls = placement_class(col_codes, i);
-        const uint4 base = reinterpret_cast<const uint4 *>(st.pair_base)[i * 4 + cls];
-        // general layout: states of this dim for history 0, before the dim and after an update at
-        // it; the all-gather (a sharding producer, a replicating consumer: class 0) is charged on
-        // the gathered bytes.  (Power-of-two layout: that shift is part of the word's base.)
-        const uint32_t k = (uint32_t)States<M>::index(i, 0, 0) + (mask << i);
-        const uint32_t k2 = i + 1 < M ? (uint32_t)States<M>::index(i + 1, 0, 0) + (mask << (i + 1)) + (1u << i)
-                                      : (uint32_t)States<M>::last((int)mask, 0);
-        const uint32_t at = (uint32_t)__umul24(POW2 ? j0 : k, POW2 ? (uint32_t)kPow2Stride : (uint32_t)kGeneralStride);
-        const uint32_t at0 = POW2 ? at : (uint32_t)__umul24(cls >= 2 ? k2 : k, (uint32_t)kGeneralStride);
-        uint32_t *w = w_of_col + i * kWordsPerDim;
-        w[0] = base.x + at0;
-        w[1] = base.y + at;
-        w[2] = base.z + at;
-        w[3] = base.w + at;
-        w[4] = at;  // the zeros array, no read+write, no step
-        w[5] = at + kRw1Array * 8u;
-      }
-    };
-    if (E != 0) words_of_dims(std::true_type{});
-    else words_of_dims(std::false_type{});
-    if (M == 2 && col_codes == 0x4040u) {
-      w_of_col[kCodesWord<M>] = col_codes | (kFlipShift << 24);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {  // (Partial -> Shard at dim 1, then at dim 0)
-        const int dim = k < 2 ? 1 : 0;
-        const uint32_t base = st.pair_base[dim * 16 + 4 + 2 + (k & 1)];
-        const uint32_t state = E != 0 ? (uint32_t)lay.lg_total : dim == 1 ? (uint32_t)States<M>::index(1, 0, 0) : (uint32_t)States<M>::kCount;
-        // (general layout: both states are named outright, no step between them)
-        w_of_col[kFlipWord<M> + k] = (E != 0 ? base : base & 0x00FFFFFFu) + __umul24(state, (uint32_t)lay.state_stride);
-      }
+    for (int i = 0; i < M; ++i) {
+      const uint32_t cls = placement_class(col_codes, i), sharded = cls >> 1;
+      slots += cls << (8 * i + 4);
+      index += __mul24((int)sharded, lay.index_weight[i]);
+      if (i + 1 < M) others += sharded << i;
+      else index += __mul24((int)(sharded * others), lay.last_weight);
     }
+    if (M == 2 && col_codes == 0x4040u) codes |= kFlipShift << 24;
+    if (M < 4) slots |= (uint32_t)index << 24;
+    if (col_tensor < 0) slots |= kNotASpec;
+    if constexpr (M < 4) st.col[jc] = ColRecord<M>{codes, slots};
+    else st.col[jc] = ColRecord<M>{codes, slots, (uint32_t)index, 0u};
     if (col_tensor != t0 || col_tensor < 0) mixed = true;
   }
   if (has_row) {
@@ -1350,16 +1348,17 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
 #pragma unroll
     for (int i = 0; i < M; ++i) {
       const uint32_t t = (row_codes >> (8 * i)) & 0xFF;
-      slots += ((uint32_t)(kWordsPerDim * i) + placement_class(row_codes, i)) << (8 * i + 2);
+      slots += (16u * i + placement_class(row_codes, i)) << (8 * i + 2);
       all_shard &= kind_of(t) == 2;
     }
     if (M == 2) {
-      const uint32_t flip = ((kFlipWord<M> * 4u + (dim_of((row_codes >> 8) & 0xFF) != 0 ? 4u : 0u)) << 16) |
-                            ((kFlipWord<M> * 4u + 8u + (dim_of(row_codes & 0xFF) != 0 ? 4u : 0u)) << 24);
+      // (the producer adds the 16 of its class, Partial)
+      const uint32_t flip = ((kFlipWord * 4u - 16u + (dim_of((row_codes >> 8) & 0xFF) != 0 ? 4u : 0u)) << 16) |
+                            ((kFlipWord * 4u - 16u + 8u + (dim_of(row_codes & 0xFF) != 0 ? 4u : 0u)) << 24);
       slots |= all_shard ? flip : slots << 16;
     }
     if (row_tensor < 0) {  // a consumer spec that is not a DTensorSpec
-      slots |= kRowNotASpec;
+      slots |= kNotASpec;
       mixed = true;
     }
     if (DERIVE) {  // the value compute_costs_block writes for this strategy
@@ -1377,15 +1376,16 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
 // where it is used, in every pass, and a scalar load in flight makes the wait for an LDS read a wait for everything.)
 struct EntryConstants {
   double rescale, inv_rescale, transition;
-  int32_t transition_scale, state_stride;
+  int32_t transition_scale, state_stride, level_stride;
 };
 __device__ __forceinline__ EntryConstants entry_constants(const apc_params &p, const TermLayout &lay) {
-  EntryConstants k{p.rescale, lay.inv_rescale, (double)p.transition_scale, p.transition_scale, lay.state_stride};
-  __asm__ volatile("" : "+s"(k.rescale), "+s"(k.inv_rescale), "+v"(k.transition), "+s"(k.transition_scale), "+s"(k.state_stride));
+  EntryConstants k{p.rescale, lay.inv_rescale, (double)p.transition_scale, p.transition_scale, lay.state_stride, lay.level_stride};
+  __asm__ volatile("" : "+s"(k.rescale), "+s"(k.inv_rescale), "+v"(k.transition), "+s"(k.transition_scale), "+s"(k.state_stride),
+                   "+s"(k.level_stride));
   return k;
 }
 
-// Where a lane is in a tile: the addresses of its producer spec's words and of its consumer spec's record, and the bytes to its
+// Where a lane is in a tile: the addresses of its producer spec's record and of its consumer spec's, and the bytes to its
 // entry from the tile's first one.  (Kept as what the loads and the store need: of a column and a row, every pass would shift
 // and multiply again.)
 struct TileWalk {
@@ -1397,16 +1397,16 @@ struct TileSteps {  // of one pass; `wrap`: when the column passes the row's end
 };
 template <int M, bool RM>
 __device__ __forceinline__ TileWalk tile_walk(lds_address stage, int r, int c, int n_src) {
-  return TileWalk{stage + words_at<M, RM>() + (uint32_t)__mul24(c, kColWords<M> * 4),
+  return TileWalk{stage + cols_at<M, RM>() + (uint32_t)c * (uint32_t)sizeof(ColRecord<M>),
                   stage + rows_at<M, RM>() + (uint32_t)r * 16u,
                   (uint32_t)(__mul24(r, n_src) + c) * 8u};
 }
 // (dr, dc: rows and columns of a pass; uniform, as everything here)
 template <int M, bool RM>
 __device__ __forceinline__ TileSteps tile_steps(lds_address stage, uint32_t dr, uint32_t dc, uint32_t cols, uint32_t n_src) {
-  constexpr uint32_t kCol = (uint32_t)kColWords<M> * 4u;
+  constexpr uint32_t kCol = (uint32_t)sizeof(ColRecord<M>);
   const uint32_t dout = (dr * n_src + dc) * 8u;
-  return TileSteps{dc * kCol, stage + words_at<M, RM>() + cols * kCol, cols * kCol, dr * 16u, dr * 16u + 16u, dout, dout + (n_src - cols) * 8u};
+  return TileSteps{dc * kCol, stage + cols_at<M, RM>() + cols * kCol, cols * kCol, dr * 16u, dr * 16u + 16u, dout, dout + (n_src - cols) * 8u};
 }
 template <bool WHOLE>  // whole rows: the entries of a tile are consecutive
 __device__ __forceinline__ void advance(TileWalk &w, const TileSteps &s) {
@@ -1428,7 +1428,7 @@ __device__ __forceinline__ uint32_t uniform_quotient(uint32_t x, float inv_d) {
   return (uint32_t)uniform_i32((int)q);
 }
 
-// The byte offset of the lookup word of mesh dim I: of the consumer's class (byte I of `slots`), or `same` where the
+// The byte offset of the lookup word of mesh dim I: byte I of `slots`, or `same` where the
 // placements (byte I of the codes) are equal.  Two instructions that select bytes, where a compiler masks, compares,
 // shifts and selects.  (s_nop 1: two cycles from a comparison's result to the select that reads it; the compiler does not look
 // inside an asm statement.)
@@ -1450,7 +1450,7 @@ __device__ __forceinline__ uint32_t word_slot(uint32_t src, uint32_t tgt, uint32
 }
 template <int I, int M>
 __device__ __forceinline__ void word_slots(uint32_t src, uint32_t tgt, uint32_t slots, uint32_t (&out)[M]) {
-  out[I] = word_slot<I>(src, tgt, slots, (uint32_t)((kWordsPerDim * I + 4) * 4));  // (slot 4: same placement, nothing to add)
+  out[I] = word_slot<I>(src, tgt, slots, 0u);  // (word 0: nothing to add)
   if constexpr (I + 1 < M) word_slots<I + 1>(src, tgt, slots, out);
 }
 
@@ -1458,40 +1458,45 @@ __device__ __forceinline__ void word_slots(uint32_t src, uint32_t tgt, uint32_t 
 // What bounds a table of large tiles is the vector instructions of a SIMD, all of its cycles (20 M entries on (16, 8, 4): 27.9 M
 // instructions, 108 thousand of a SIMD's cycles in a launch of 101 thousand; now 20.4 M, 80 of 84 thousand, LDS 79 % busy), so a pass counts them:
 // 40 on a 3-D mesh with the walk and the store (54 when columns, rows and loop were kept as numbers of a lane and the codes
-// compared by mask), and a tile's staging, which two wavefronts share, about 330 (430).  us a pass: 20 M on (16, 8, 4) 57.0 ->
+// compared by mask), and a tile's staging, which two wavefronts share, about 330 (430; 250 since the words are the launch's).  us a pass: 20 M on (16, 8, 4) 57.0 ->
 // 50.8, 5.3 M on (2, 4, 2, 2) 41.8 -> 39.4, 5.1 M on (3, 2, 2, 2) 53.2 -> 50.7, 2.6 M on (12, 6) 14.4 -> 13.4, 587 k on
 // (6, 4, 2) 16.0 -> 15.4.  (Every copy's address in scalar registers, one instruction less a store, is 1 % slower.)
 // Straight-line code: all lookups of an entry are independent of its fp additions, so they
 // are issued together; no vector memory loads.
-template <int M, bool CONT, bool RESCALE>
-__device__ __forceinline__ void uniform_entry(const EntryConstants &k, lds_address terms, const TileWalk &where, double &comm_o, double &total_o,
-                                              int &trans_o) {
-  const uint32_t src = lds_read<uint32_t>(where.col + kCodesWord<M> * 4);
+template <int M, bool RM, bool CONT, bool RESCALE>
+__device__ __forceinline__ void uniform_entry(const EntryConstants &k, lds_address stage, lds_address terms, const TileWalk &where, double &comm_o,
+                                              double &total_o, int &trans_o) {
+  typedef uint32_t col_words __attribute__((ext_vector_type(sizeof(ColRecord<M>) / 4)));
+  const col_words col = lds_read<col_words>(where.col);
   const u32x4 raw = lds_read<u32x4>(where.row);
+  const uint32_t src = col.x;
   const RowRecord row{raw.x, raw.y, __hiloint2double((int)raw.w, (int)raw.z)};
   const uint32_t x = src ^ row.codes;
   const bool differs = M == 2 ? (x & 0xFFFFu) != 0 : x != 0;
   // (2-D: a (Partial, Partial) producer's shift takes the slots of its order flip)
-  const uint32_t slots = M == 2 ? row.slots >> (src >> 24) : row.slots;
+  const uint32_t slots = (M == 2 ? row.slots >> (src >> 24) : row.slots) + col.y;
+  uint32_t index;
+  if constexpr (M < 4) index = col.y >> 24;
+  else index = col.z;
   // ---- integer part: which term at which running index each mesh dim adds -------------------
-  uint32_t at = 0;  // byte offset of the running index (history of the earlier dims / exponent steps), mod 2^32
+  uint32_t at = terms + __umul24(index, (uint32_t)k.state_stride);  // the running index' entry
   uint32_t slot[M], term_at[M], rw_at[M], nc_at[M];
   word_slots<0>(src, row.codes, slots, slot);
 #pragma unroll
   for (int i = 0; i < M; ++i) {
-    const uint32_t w = lds_read<uint32_t>(where.col + slot[i]);
+    const uint32_t w = lds_read<uint32_t>(stage + words_at<M, RM>() + slot[i]);
     term_at[i] = (w & 0xFFFFu) + at;
     rw_at[i] = term_at[i] + (uint32_t)(int32_t)(int8_t)(w >> 16);
-    if (!CONT) nc_at[i] = lds_read<uint32_t>(where.col + (kWordsPerDim * i + 5) * 4) + at;
+    if (!CONT) nc_at[i] = at + (uint32_t)(kRw1Array * 8u + ((1u << i) - 1u) * (uint32_t)k.level_stride);  // (the state before the dim)
     at += (uint32_t)__mul24((int32_t)w >> 24, k.state_stride);  // (24-bit multiplies issue at full rate)
   }
   // ---- lookups ------------------------------------------------------------------------------
   double term[M], rw[M], nc[M];
 #pragma unroll
   for (int i = 0; i < M; ++i) {
-    term[i] = lds_read<double>(terms + term_at[i]);
-    rw[i] = lds_read<double>(terms + rw_at[i]);
-    if (!CONT) nc[i] = lds_read<double>(terms + nc_at[i]);
+    term[i] = lds_read<double>(term_at[i]);
+    rw[i] = lds_read<double>(rw_at[i]);
+    if (!CONT) nc[i] = lds_read<double>(nc_at[i]);
   }
   // ---- additions in the reference's order (0.0 + t == t for these non-negative terms) ------------
   double cost = 0.0;
@@ -1762,13 +1767,14 @@ __device__ __forceinline__ void tile_entries_walk(const TableArgs &a, lds_addres
 template <int M, bool DERIVE, bool RM>
 __device__ __forceinline__ void generic_entry(const apc_params &p, const TableArgs &a, const TileStage<M, RM> &st, lds_address stage, const TileView &v,
                                               const TileWalk &where, double &comm, double &total, int &trans) {
-  const int r = (int)((where.row - stage - rows_at<M, RM>()) / 16u), c = (int)((where.col - stage - words_at<M, RM>()) / (uint32_t)(kColWords<M> * 4));
+  const int r = (int)((where.row - stage - rows_at<M, RM>()) / 16u), c = (int)((where.col - stage - cols_at<M, RM>()) / (uint32_t)sizeof(ColRecord<M>));
   const int64_t local = (int64_t)(v.row_begin + r) * v.n_src + (v.col_begin + c);
-  const uint32_t src = st.colh[c].x, cinfo = st.colh[c].y;
+  const ColRecord<M> col = st.col[c];
+  const uint32_t src = M == 2 ? col.codes & 0xFFFFu : col.codes;  // (without the flip's shift)
   const RowRecord row = st.row[r];
   const uint32_t tgt = row.codes;
   trans = 0;
-  if ((v.flags & APC_EDGE_NO_PRODUCER) || !(cinfo & 1u) || (row.slots & 0xFFu) == kRowNotASpec) {
+  if ((v.flags & APC_EDGE_NO_PRODUCER) || (col.slots & 0xFFu) == kNotASpec || (row.slots & 0xFFu) == kNotASpec) {
     comm = a.pt_values[v.pt_begin + local];
   } else {
     trans = (src != tgt) ? p.transition_scale : 0;
@@ -1817,7 +1823,7 @@ __device__ __forceinline__ void tile_entries(const apc_params &p, const TableArg
   const lds_address terms = stage + terms_at<M, RM>() + (uint32_t)kWaveScratchBytes<RM> * (uint32_t)(nthreads >> 6);  // (term_base)
 #define APC_TILE_LOOP(CONT_, RESCALE_)                                                                                       \
   entries(std::integral_constant<int, OUT>{}, [&](const TileWalk &where, double &comm, double &total, int &trans) {          \
-    uniform_entry<M, CONT_, RESCALE_>(k, terms, where, comm, total, trans);                                                  \
+    uniform_entry<M, RM, CONT_, RESCALE_>(k, stage, terms, where, comm, total, trans);                                                  \
   })
   if (uniform_i32(st.cont)) {
     if (rescale) { APC_TILE_LOOP(true, true); } else { APC_TILE_LOOP(true, false); }
