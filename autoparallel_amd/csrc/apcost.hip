@@ -590,26 +590,9 @@ struct ComputeCostArgs {
   int32_t *error_flag;
 };
 
-// Compute cost of one strategy (compute_estimation.py:334-365); `unsupported` is set when the
-// strategy has flops and its dtype has no throughput on the device row (the result is NaN).
-__device__ __forceinline__ double compute_cost_of(const apc_params &p, bool zero_cost, int64_t rw_bytes, int64_t flops,
-                                                  int dt, bool &unsupported) {
-  unsupported = false;
-  if (zero_cost) return 0.0;
-  const double rw = rw_time((double)rw_bytes, p);
-  if (flops == 0) return rw;
-  const double gf = (dt >= 0 && dt < APC_MAX_DTYPES) ? pick<APC_MAX_DTYPES>(p.gpu_flops, dt) : 0.0;
-  if (gf == 0.0) {
-    unsupported = true;  // compute_estimation.py:198-201 raises ValueError
-    return NAN;
-  }
-  double t = (double)flops / gf * 1e6;
-  t = t / p.compute_eff;
-  return t > rw ? t : rw;
-}
-
-// The same value with the divisions taken through the checked reciprocals (div_by): gf / inv_gf =
-// the device row's throughput for the strategy's dtype and its reciprocal, 0 when unsupported.
+// Compute cost of one strategy (compute_estimation.py:334-365), the divisions taken through the checked reciprocals
+// (div_by): gf / inv_gf = the device row's throughput for the strategy's dtype and its reciprocal, 0 when unsupported (then,
+// with flops, the result is NaN).
 __device__ __forceinline__ double compute_cost_through_reciprocals(const apc_params &p, bool zero_cost, int64_t rw_bytes,
                                                                    int64_t flops, double gf, double inv_gf) {
   if (zero_cost) return 0.0;
@@ -625,8 +608,8 @@ template <int BS, bool THROUGH = false>
 __device__ __forceinline__ void compute_costs_block(int64_t block, const apc_params &p, const ComputeCostArgs &a) {
   const int64_t s = block * BS + threadIdx.x;
   if (s >= a.n) return;
-  // (the divisions through the checked reciprocals: the same bits as compute_cost_of, a third of
-  // its instructions; these workgroups share the chip with the ones that write the matrices)
+  // (the divisions through the checked reciprocals: a third of the instructions; these workgroups share the chip with the
+  // ones that write the matrices)
   const int dt = a.dtype[s];
   const bool zero = a.zero_cost[s] != 0;
   const int64_t flops = a.flops[s];
@@ -1144,6 +1127,60 @@ __device__ __forceinline__ void rings_at(double gb, const apc_params &p, int d, 
   two = (p.base_latency + (2.0 * hops) * lat) + 2.0 * bw;
 }
 
+__device__ __forceinline__ int from_lane(int v, int lane) { return __builtin_amdgcn_ds_bpermute(lane << 2, v); }
+__device__ __forceinline__ double from_lane(double v, int lane) {
+  return __hiloint2double(from_lane(__double2hiint(v), lane), from_lane(__double2loint(v), lane));
+}
+__device__ __forceinline__ int64_t from_lane_i64(int64_t v, int lane) {
+  const uint32_t lo = (uint32_t)from_lane((int)(uint32_t)v, lane), hi = (uint32_t)from_lane((int)(uint32_t)((uint64_t)v >> 32), lane);
+  return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// The value of the lane `N` further on within the lane's row of 16 (DPP row_shl:N), `beyond` behind the row's end.
+template <int N>
+__device__ __forceinline__ double from_lane_behind(double x, double beyond) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(beyond), __double2loint(x), 0x100 + N, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(beyond), __double2hiint(x), 0x100 + N, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+
+// Bytes (as a double) and contiguity of the tensor whose dim lane & 7 this lane holds (size x, stride y): what
+// tensor_bytes_and_contiguity_of returns, in every lane, from the whole wavefront.  A dim's expected stride is the product
+// of the sizes behind it: three steps of a scan over the lanes in doubles, exact while the product of all is below 2^53.
+// Any other tensor (and one with an empty dim, where the two expected strides differ) goes dim by dim in integers.
+// (As scalar integers the eight dims are 190 instructions one behind the other, on the one scalar unit of a compute unit,
+// in every wavefront; 35 vector instructions now.  With a tile's compute costs through the checked reciprocals, us a pass: 1.8 M entries on
+// (16, 8, 4) 15.6 -> 14.6, 5.9 M on (64, 4) 27.2 -> 26.2, 704 k on (6, 4, 2) 11.6 -> 11.2, 1.7 M on (32, 8) over packed tiles 8.42 -> 8.32.)
+__device__ __forceinline__ void tensor_info_of_lanes(int rank, int itemsize, int64_t x, int64_t y, int lane, double &bytes, bool &contiguous) {
+  const int dim = lane & 15;
+  const bool live = dim < min(rank, APC_MAX_RANK);  // (lanes 8 .. 15 of a row hold no dim)
+  const double size = live ? (double)x : 1.0;
+  double product = size;
+  product *= from_lane_behind<1>(product, 1.0);
+  product *= from_lane_behind<2>(product, 1.0);
+  product *= from_lane_behind<4>(product, 1.0);
+  const double expected = from_lane_behind<1>(product, 1.0);
+  const bool differs = size != 1.0 && (double)y != expected;
+  contiguous = __ballot(differs) == 0;
+  const double total = __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(product)),
+                                        __builtin_amdgcn_readfirstlane(__double2loint(product))) * (double)itemsize;
+  bytes = total;
+  if (__ballot(!(size >= 1.0) || !(product < 0x1p53) || !(total < 0x1p53)) != 0) {  // (uniform)
+    int64_t nbytes = itemsize, one = 1, most = 1;
+    contiguous = true;
+#pragma unroll 1
+    for (int i = min(rank, APC_MAX_RANK) - 1; i >= 0; --i) {
+      const int64_t xi = value_of_lane(x, i), yi = value_of_lane(y, i);
+      nbytes *= xi;
+      if (xi == 1) continue;
+      if (yi != one && yi != most) contiguous = false;
+      most *= xi > 1 ? xi : 1;
+      one *= xi;
+    }
+    bytes = (double)nbytes;
+  }
+}
+
 // Stages tile `tile` with `nthreads` (>= 64) cooperating threads (this thread is `tid`).  The
 // caller synchronises before the stage is read.  Only global loads and LDS writes: no stores.
 // Every vector load of the tile is issued first, in one round, and the state terms are
@@ -1188,9 +1225,17 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
   double row_cpa = 0.0;
   int64_t row_flops = 0, row_rw = 0;
   int row_dtype = 0, row_zero = 1, row_args = 1;
+  const int t0c = t0 >= 0 ? t0 : 0;  // (row 0 when the tile has no tensor: unconditional loads, the values are not used then)
+  int64_t dim_size = 0, dim_stride = 0;
+  double gf_of_lane = 0.0, inv_gf_of_lane = 0.0;
   if (!DERIVE) {
     if (a.per_arg) row_cpa = load_of_lane(a.per_arg + sr, at_row);
   } else {
+    dim_size = load_of_lane(a.shape + (int64_t)t0c * APC_MAX_RANK, (uint32_t)lane & (APC_MAX_RANK - 1));
+    dim_stride = load_of_lane(a.stride + (int64_t)t0c * APC_MAX_RANK, (uint32_t)lane & (APC_MAX_RANK - 1));
+    // (lane j holds the throughput of dtype code j & 7: fetched by the lanes that need it, below)
+    gf_of_lane = load_of_lane(p.gpu_flops, (uint32_t)lane & (APC_MAX_DTYPES - 1));
+    inv_gf_of_lane = load_of_lane(p.inv_gpu_flops, (uint32_t)lane & (APC_MAX_DTYPES - 1));
     row_flops = load_of_lane(a.flops + sr, at_row);
     row_rw = load_of_lane(a.rw_bytes + sr, at_row);
     row_dtype = load_of_lane(a.dtype + sr, at_row);
@@ -1208,34 +1253,27 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
     copies.row_out = a.edge_row_begin[tile.edge];
   }
   // ---- the scalar loads of the round (wave-uniform addresses), issued together ---------------------
-  // The tile's tensor (row 0 when the tile has none: unconditional loads, the values are not
-  // used then) and the first matrix row of its edge.  The contiguity byte is read as the aligned
-  // word around it (which lies in the byte's own page).
-  const int t0c = t0 >= 0 ? t0 : 0;
-  uint32_t contiguous = 1;
-  int64_t tensor_nbytes = 0;
+  // The contiguity byte is read as the aligned word around it (which lies in the byte's own page).
+  bool contiguous;
+  double fbytes;
   if constexpr (!DERIVE) {
     const uint8_t *flag = a.tensor_contiguous + t0c;
     const uint32_t byte = (uint32_t)(reinterpret_cast<uintptr_t>(flag) & 3);
     const uint32_t word = uniform_load(reinterpret_cast<const uint32_t *>(flag - byte));
-    tensor_nbytes = uniform_load(a.tensor_bytes + t0c);
+    const int64_t tensor_nbytes = uniform_load(a.tensor_bytes + t0c);
     fetch_arguments_now(word, tensor_nbytes);
-    contiguous = (word >> (8 * byte)) & 0xFFu;
+    contiguous = ((word >> (8 * byte)) & 0xFFu) != 0;
+    fbytes = (double)tensor_nbytes;
   } else {
     const int t_rank = uniform_load(a.rank + t0c), t_item = uniform_load(a.itemsize + t0c);
-    const i64x8 t_shape = uniform_load(reinterpret_cast<const i64x8 *>(a.shape + (int64_t)t0c * APC_MAX_RANK));
-    const i64x8 t_stride = uniform_load(reinterpret_cast<const i64x8 *>(a.stride + (int64_t)t0c * APC_MAX_RANK));
-    fetch_arguments_now(t_rank, t_item, t_shape[0], t_stride[0]);
-    bool ok;
-    tensor_bytes_and_contiguity_of(t_rank, t_item, t_shape, t_stride, tensor_nbytes, ok);
-    contiguous = ok ? 1u : 0u;
+    fetch_arguments_now(t_rank, t_item);
+    tensor_info_of_lanes(t_rank, t_item, dim_size, dim_stride, lane, fbytes, contiguous);
   }
-  // ---- term arrays (scalar operands only) ---------------------------------------------------
+  // ---- term arrays --------------------------------------------------------------------------
   if (terms_wanted && E != 0) {
     // power-of-two mesh.  A lane per computed array takes the array's chain on the tensor's
     // bytes (every wavefront its own copy: no barrier), then a lane per (array, exponent) the
     // value.
-    const double fbytes = (double)tensor_nbytes;
     StagingScratch &mine = *reinterpret_cast<StagingScratch *>(wave_scratch(st, wave));
     if (lane < kComputed) {
       mine.chain[lane] = div_by(div_by(fbytes * chain_of.hops, chain_of.div1, chain_of.inv_div1) * 1e6, chain_of.div2,
@@ -1265,7 +1303,6 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
     // every collective / read-write term the tile can need, once per running-bytes state, in
     // the reference's operation order (collective_runtime_estimation.py:66-68, :86, :128;
     // torch _collective_utils.py:281-313; compute_estimation.py:302-314)
-    const double fbytes = (double)tensor_nbytes;
     double *const terms = reinterpret_cast<double *>(term_base(st, nthreads));
     const auto bytes_at = [&](int level, int mask, int hist) {
       double shards = 1.0;  // exact: a product of mesh sizes (torch _dtensor_spec.py:555-561)
@@ -1322,7 +1359,7 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
     }
   }
   // ---- what the loads brought, to LDS ---------------------------------------------------------
-  if (tid == 0) st.cont = contiguous != 0;
+  if (tid == 0) st.cont = contiguous;
   if (tid < kPairWords<M>) st.words[tid] = pair_word;
   if (has_col) {
     uint32_t slots = 0, codes = col_codes, others = 0;
@@ -1341,6 +1378,14 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
     if constexpr (M < 4) st.col[jc] = ColRecord<M>{codes, slots};
     else st.col[jc] = ColRecord<M>{codes, slots, (uint32_t)index, 0u};
     if (col_tensor != t0 || col_tensor < 0) mixed = true;
+  }
+  double row_cost = 0.0;
+  if constexpr (DERIVE) {  // (every lane takes part in the exchange; by the wavefronts that hold rows)
+    if (uniform_i32(nthreads - 64 - (tid - lane)) < rows) {
+      const bool known = row_dtype >= 0 && row_dtype < APC_MAX_DTYPES;
+      const double gf = from_lane(gf_of_lane, row_dtype & (APC_MAX_DTYPES - 1)), inv_gf = from_lane(inv_gf_of_lane, row_dtype & (APC_MAX_DTYPES - 1));
+      row_cost = compute_cost_through_reciprocals(p, row_zero != 0, row_rw, row_flops, known ? gf : 0.0, known ? inv_gf : 0.0);
+    }
   }
   if (has_row) {
     uint32_t slots = 0;
@@ -1361,10 +1406,7 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
       slots |= kNotASpec;
       mixed = true;
     }
-    if (DERIVE) {  // the value compute_costs_block writes for this strategy
-      bool unsupported;
-      row_cpa = compute_cost_of(p, row_zero != 0, row_rw, row_flops, row_dtype, unsupported) / (double)row_args;
-    }
+    if (DERIVE) row_cpa = row_cost / (double)row_args;  // the value compute_costs_block writes for this strategy
     st.row[jr] = RowRecord{row_codes, slots, row_cpa};
   }
   // one flag per wavefront, written unconditionally: nothing to clear beforehand
@@ -1624,15 +1666,6 @@ __device__ __forceinline__ void row_min_in_wave(bool active, double value, int c
     APC_ROW_MIN_JOIN(48)
   }
 #undef APC_ROW_MIN_JOIN
-}
-
-__device__ __forceinline__ int from_lane(int v, int lane) { return __builtin_amdgcn_ds_bpermute(lane << 2, v); }
-__device__ __forceinline__ double from_lane(double v, int lane) {
-  return __hiloint2double(from_lane(__double2hiint(v), lane), from_lane(__double2loint(v), lane));
-}
-__device__ __forceinline__ int64_t from_lane_i64(int64_t v, int lane) {
-  const uint32_t lo = (uint32_t)from_lane((int)(uint32_t)v, lane), hi = (uint32_t)from_lane((int)(uint32_t)((uint64_t)v >> 32), lane);
-  return (int64_t)(((uint64_t)hi << 32) | lo);
 }
 
 // The minimum, and the lowest column that has it, over neighbouring lanes of a row of 16: one step of a butterfly.
@@ -2150,8 +2183,7 @@ __device__ __forceinline__ void packed_tile(const apc_packed_tile *T, double *co
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
   // ---- the one round of loads: nothing here depends on another load ---------------------------
   const i32x16 h = uniform_load(reinterpret_cast<const i32x16 *>(T));
-  const i64x8 t_shape = uniform_load(reinterpret_cast<const i64x8 *>(T->tensor_shape));
-  const i64x8 t_stride = uniform_load(reinterpret_cast<const i64x8 *>(T->tensor_stride));
+  const int64_t dim_size = T->tensor_shape[lane & (APC_MAX_RANK - 1)], dim_stride = T->tensor_stride[lane & (APC_MAX_RANK - 1)];
   TileCopies copies;
   copies.entry0 = T->dup_entry_begin[lane & (APC_PACKED_MAX_DUPS - 1)];
   copies.row0 = T->dup_row_begin[lane & (APC_PACKED_MAX_DUPS - 1)];
@@ -2163,7 +2195,7 @@ __device__ __forceinline__ void packed_tile(const apc_packed_tile *T, double *co
   // (lane j holds the throughput of dtype code j & 7: fetched by the lanes that need it, below)
   const double gf_of_lane = a.p.gpu_flops[lane & (APC_MAX_DTYPES - 1)], inv_gf_of_lane = a.p.inv_gpu_flops[lane & (APC_MAX_DTYPES - 1)];
   // (kernel arguments the wavefront needs first or in its store loops, under the same wait)
-  fetch_arguments_now(h[0], t_shape[0], t_stride[0], a.row_min_out, a.row_arg_out, p.hbm_bw, p.inv_hbm_bw, p.rw_eff, p.inv_rw_eff,
+  fetch_arguments_now(h[0], a.row_min_out, a.row_arg_out, p.hbm_bw, p.inv_hbm_bw, p.rw_eff, p.inv_rw_eff,
                       p.launch_floor, p.compute_eff, p.inv_compute_eff, a.inv_rescale, p.rescale, p.a2a_scale, p.base_latency);
   const int rows = h[0], cols = h[1], flags = h[2], dup_count = h[3], t0 = h[4];
   if ((unsigned)rows > (unsigned)APC_TILE_MAX_ROWS || (unsigned)(cols - 1) >= (unsigned)APC_TILE_MAX_COLS ||
@@ -2175,10 +2207,9 @@ __device__ __forceinline__ void packed_tile(const apc_packed_tile *T, double *co
   const int rows_per_pass = (int)((64u * magic) >> 16);
   if (wave * rows_per_pass >= rows) return;  // a wavefront without rows (a tile of fewer rows than the workgroup walks at once)
   // ---- per wavefront: the tensor's bytes, the rows' compute costs -------------------------------
-  int64_t nbytes;
+  double fbytes;
   bool contiguous;
-  tensor_bytes_and_contiguity_of(h[5], h[6], t_shape, t_stride, nbytes, contiguous);
-  const double fbytes = (double)nbytes;
+  tensor_info_of_lanes(h[5], h[6], dim_size, dim_stride, lane, fbytes, contiguous);
   const int dt = (int)(int8_t)(row_meta & 0xFF);
   const bool known_dtype = dt >= 0 && dt < APC_MAX_DTYPES;
   const double gf = from_lane(gf_of_lane, dt & (APC_MAX_DTYPES - 1)), inv_gf = from_lane(inv_gf_of_lane, dt & (APC_MAX_DTYPES - 1));
