@@ -751,7 +751,9 @@ struct TermArrayConstants {  // value at exponent index j = max(lat + ldexp(B, j
   int32_t pad_;
 };
 struct TermLayout {
-  uint32_t pair[APC_MAX_MESH * 16];
+  // What a tile's first wavefront copies into LDS, 16 bytes a lane (TileStage::image): the lookup words, then the constants
+  // of arrays 2 .. of the power-of-two layout (TermArrayConstants)
+  uint32_t image[APC_MAX_MESH * 16 + (kMaxTermArrays - 2) * (int)sizeof(TermArrayConstants) / 4];
   int32_t exponents;         // 0: general layout; else E, the number of exponents
   int32_t lg[APC_MAX_MESH];  // log2 of the mesh sizes (power-of-two layout)
   int32_t lg_total;          // L
@@ -762,7 +764,6 @@ struct TermLayout {
   int32_t state_stride;      // bytes between the entries of two consecutive states / exponents
   uint32_t exponent_magic;   // ceil(65536 / E): t / E = (t * magic) >> 16 for t < 512
   double inv_rescale;        // 1.0 / params.rescale
-  TermArrayConstants arrays[kMaxTermArrays - 2];  // of arrays 2 .. (power-of-two layout)
 };
 
 struct TableArgs {
@@ -880,7 +881,7 @@ static_assert(4 + 3 * APC_MAX_MESH <= kMaxTermArrays, "arrays of the power-of-tw
 // Lookup words.  What a mesh dim adds to an entry depends on the producer's and the consumer's class at
 // that dim and on the running index, which starts at the producer spec's own (general: the first state of its mask;
 // power-of-two meshes: L - log2 of its shards) and goes on by the earlier dims.  One 32-bit word per (dim, producer
-// class, consumer class), the same for every tile of a launch (TermLayout::pair), in fields an instruction can take as a
+// class, consumer class), the same for every tile of a launch (TermLayout::image), in fields an instruction can take as a
 // half or a byte of a register:
 //   bits  0-15  byte offset of the collective's term from the running index' entry (general: array of
 //               pair_action's term, state of the bytes the collective moves: after the update
@@ -912,6 +913,8 @@ static_assert(TermTable<APC_MAX_MESH>::kEntries * 8 <= 0xFFFF + 1, "term offsets
 static TermLayout term_layout(const apc_params &p) {
   TermLayout lay{};
   const int M = p.mesh_ndim;
+  uint32_t pair[APC_MAX_MESH * 16] = {};
+  TermArrayConstants arrays[kMaxTermArrays - 2] = {};
   bool pow2 = getenv("APC_GENERAL_TERMS") == nullptr;  // (testing override: the general layout on any mesh)
   int total = 0;
   for (int i = 0; i < M; ++i) {
@@ -953,16 +956,16 @@ static TermLayout term_layout(const apc_params &p) {
           step = !upd ? 0 : sel == 1u ? lay.lg[i] : -lay.lg[i];
         }
         const int to_rw = ((int)rw_array - (int)term_array) * 8;
-        lay.pair[i * 16 + c * 4 + t] = (state * (uint32_t)lay.state_stride + term_array * 8u) | ((uint32_t)(to_rw & 0xFF) << 16) |
+        pair[i * 16 + c * 4 + t] = (state * (uint32_t)lay.state_stride + term_array * 8u) | ((uint32_t)(to_rw & 0xFF) << 16) |
                                        ((uint32_t)(step & 0xFF) << 24);
       }
   if (M == 2)
     for (int k = 0; k < 4; ++k) {  // the order flip: (Partial -> Shard at dim 1, then at dim 0), of an unsharded producer
       const int dim = k < 2 ? 1 : 0;
-      const uint32_t word = lay.pair[dim * 16 + 4 + 2 + (k & 1)];
+      const uint32_t word = pair[dim * 16 + 4 + 2 + (k & 1)];
       // (general layout: both states are named outright, no step between them)
       const uint32_t own = (1u << dim) - 1u, state = dim == 1 ? 1u : (uint32_t)States<2>::kCount;
-      lay.pair[kFlipWord + k] = pow2 ? word : (word & 0x00FFFFFFu) + (state - own) * (uint32_t)lay.state_stride;
+      pair[kFlipWord + k] = pow2 ? word : (word & 0x00FFFFFFu) + (state - own) * (uint32_t)lay.state_stride;
     }
   lay.index0 = lay.lg_total;
   for (int i = 0; i < M; ++i) lay.index_weight[i] = pow2 ? -lay.lg[i] : ((1 << M) - 1) << i;
@@ -971,19 +974,22 @@ static TermLayout term_layout(const apc_params &p) {
   if (pow2) {
     const double ninf = -INFINITY;
     // one read+write, two (compute_estimation.py:302-314 on bytes x 2^(e + 31))
-    lay.arrays[0] = {1.0, p.hbm_bw, p.inv_hbm_bw, p.rw_eff, p.inv_rw_eff, 0.0, p.launch_floor, 1.0, -total - 30 + 31, 0};
-    lay.arrays[1] = lay.arrays[0];
-    lay.arrays[1].scale = 2.0;
+    arrays[0] = {1.0, p.hbm_bw, p.inv_hbm_bw, p.rw_eff, p.inv_rw_eff, 0.0, p.launch_floor, 1.0, -total - 30 + 31, 0};
+    arrays[1] = arrays[0];
+    arrays[1].scale = 2.0;
     for (int d = 0; d < M; ++d) {  // torch _collective_utils.py:281-313 on bytes x 2^e
       const double h = (double)(p.mesh_size[d] - 1);
       const double lat1 = p.base_latency + h * p.lat[d];
       const double lat2 = p.base_latency + (2.0 * h) * p.lat[d];
       const int shift = -total - 30 - lay.lg[d];
-      lay.arrays[2 + 3 * d] = {h, p.bw[d], p.inv_bw[d], 1.0, 1.0, lat1, ninf, 1.0, shift, 0};
-      lay.arrays[3 + 3 * d] = {h, p.bw[d], p.inv_bw[d], 1.0, 1.0, lat2, ninf, 1.0, shift + 1, 0};
-      lay.arrays[4 + 3 * d] = {h, p.bw[d], p.inv_bw[d], 1.0, 1.0, lat1, ninf, p.a2a_scale, shift, 0};
+      arrays[2 + 3 * d] = {h, p.bw[d], p.inv_bw[d], 1.0, 1.0, lat1, ninf, 1.0, shift, 0};
+      arrays[3 + 3 * d] = {h, p.bw[d], p.inv_bw[d], 1.0, 1.0, lat2, ninf, 1.0, shift + 1, 0};
+      arrays[4 + 3 * d] = {h, p.bw[d], p.inv_bw[d], 1.0, 1.0, lat1, ninf, p.a2a_scale, shift, 0};
     }
   }
+  const size_t words = sizeof(uint32_t) * (size_t)(M * 16 + (M == 2 ? 4 : 0));  // (kPairWords)
+  std::memcpy(lay.image, pair, words);
+  std::memcpy(reinterpret_cast<char *>(lay.image) + words, arrays, sizeof(TermArrayConstants) * (size_t)(3 * M + 2));
   return lay;
 }
 
@@ -1008,76 +1014,64 @@ struct alignas(16) ColRecord<4> {
 static_assert(States<3>::kCount <= 256 && kMaxExponents <= 256 && APC_MAX_MESH == 4, "a running index fits its byte");
 constexpr uint32_t kNotASpec = 0xFFu;
 
-// The part of TermArrayConstants a value needs after its array's chain.
-struct alignas(16) TermValueConstants {
-  double lat, floor, scale;
-  int32_t shift, pad_;
-};
+template <int M>
+constexpr int kComputedArrays = 3 * M + 2;  // arrays 2 .. of the power-of-two layout
+template <int M>
+constexpr int kImagePieces = (kPairWords<M> * 4 + kComputedArrays<M> * (int)sizeof(TermArrayConstants) + 15) / 16;
+static_assert(kPairWords<1> % 4 == 0 && kPairWords<2> % 4 == 0 && kPairWords<3> % 4 == 0 && kPairWords<4> % 4 == 0 && kImagePieces<APC_MAX_MESH> <= 128 &&
+                  kImagePieces<APC_MAX_MESH> * 16 <= (int)sizeof(TermLayout::image), "an image in pieces of 16 bytes, two a lane at most");
 
 // Everything the entry loops need about one tile, in LDS.
-template <int M, bool RM>
+template <int M>
 struct TileStage {
-  RowRecord row[APC_TILE_MAX_ROWS];  // consumer specs
-  ColRecord<M> col[APC_TILE_MAX_COLS];  // producer specs
-  uint32_t words[kPairWords<M>];        // TermLayout::pair of the launch
-  int mixed[4];         // per staging wavefront: some spec is not a DTensorSpec on the tile's tensor (generic loop)
-  int cont;             // the tile's tensor is contiguous
-  // Last: the tile kernels size their LDS per launch for the entries the layout in use needs
-  // (stage_lds_bytes), so that the small power-of-two layout leaves room for more workgroups.
-  // In front of the entries, one WaveScratch per wavefront of the workgroup (a compile-time
-  // number in every kernel, so the entries still sit at a fixed offset): term_base.
+  RowRecord row[APC_TILE_MAX_ROWS];              // consumer specs
+  ColRecord<M> col[APC_TILE_MAX_COLS];           // producer specs
+  alignas(16) uint32_t image[kImagePieces<M> * 4];  // TermLayout::image: the lookup words, the constants of the term arrays
+  double chain[kMaxTermArrays];                  // of the computed arrays, on the tensor's bytes
+  int mixed[4];  // per wavefront: some spec is not a DTensorSpec on the tile's tensor (generic loop)
+  int cont;      // the tile's tensor is contiguous
+  // Last: the tile kernels size their LDS per launch for the entries the layout in use needs (stage_lds_bytes), so that the
+  // small power-of-two layout leaves room for more workgroups.  Behind the entries, where the tile's row minima are taken,
+  // the values of the rows each wavefront is walking (tile_entries_row_min).
   alignas(16) double terms[TermTable<M>::kEntries];
 };
 
 // Where its parts begin, in bytes.
-template <int M, bool RM>
+template <int M>
 __host__ __device__ constexpr uint32_t rows_at() {
-  using Stage = TileStage<M, RM>;
+  using Stage = TileStage<M>;
   return (uint32_t)offsetof(Stage, row);
 }
-template <int M, bool RM>
+template <int M>
 __host__ __device__ constexpr uint32_t cols_at() {
-  using Stage = TileStage<M, RM>;
+  using Stage = TileStage<M>;
   return (uint32_t)offsetof(Stage, col);
 }
-template <int M, bool RM>
+template <int M>
 __host__ __device__ constexpr uint32_t words_at() {
-  using Stage = TileStage<M, RM>;
-  return (uint32_t)offsetof(Stage, words);
+  using Stage = TileStage<M>;
+  return (uint32_t)offsetof(Stage, image);
 }
-template <int M, bool RM>
+template <int M>
 __host__ __device__ constexpr uint32_t terms_at() {
-  using Stage = TileStage<M, RM>;
+  using Stage = TileStage<M>;
   return (uint32_t)offsetof(Stage, terms);
 }
 
-// What one wavefront keeps while it stages the term arrays of the power-of-two layout.
-struct alignas(16) StagingScratch {
-  double chain[kMaxTermArrays];
-  TermValueConstants value_of[kMaxTermArrays];
-};
-// What a wavefront has to itself: while it stages the term arrays, their chains; where the tile's row minima are
-// taken, in the same place afterwards, the values of the rows it is walking (tile_entries_row_min).
+// LDS a wavefront has to itself where the tile's row minima are taken: the values of the rows it is walking.
 constexpr int kRowMinValues = 320;
 template <bool RM>
-constexpr size_t kWaveScratchBytes = RM ? kRowMinValues * sizeof(double) : sizeof(StagingScratch);
-static_assert(kWaveScratchBytes<true> >= sizeof(StagingScratch), "the chains fit");
-template <int M, bool RM>
-__device__ __forceinline__ char *wave_scratch(const TileStage<M, RM> &st, int wave) {
-  return const_cast<char *>(reinterpret_cast<const char *>(st.terms)) + kWaveScratchBytes<RM> * (size_t)wave;
-}
-// Where the term arrays of a stage start, for a workgroup of `nthreads` threads.
-template <int M, bool RM>
-__device__ __forceinline__ char *term_base(const TileStage<M, RM> &st, int nthreads) {
-  return wave_scratch(st, nthreads >> 6);
+constexpr size_t kWaveScratchBytes = RM ? kRowMinValues * sizeof(double) : 0;
+// Bytes of the term arrays in the launch's layout.
+template <int M>
+__host__ __device__ __forceinline__ uint32_t term_bytes(const TermLayout &lay) {
+  return lay.exponents ? (uint32_t)kPow2Stride * (uint32_t)lay.exponents : (uint32_t)TermTable<M>::kGeneral * 8u;
 }
 
 // LDS bytes of a tile stage whose term arrays hold what the launch's layout needs.
 template <int M, bool RM>
 static size_t stage_lds_bytes(const TermLayout &lay, int threads) {
-  const size_t entries = lay.exponents ? (size_t)(kPow2Stride / 8) * lay.exponents : (size_t)TermTable<M>::kGeneral;
-  return sizeof(TileStage<M, RM>) - sizeof(double) * TermTable<M>::kEntries + kWaveScratchBytes<RM> * (size_t)(threads / 64) +
-         sizeof(double) * entries;
+  return terms_at<M>() + term_bytes<M>(lay) + kWaveScratchBytes<RM> * (size_t)(threads / 64);
 }
 
 // Where the copies of a tile's values go: lane k of EVERY wavefront holds the first entry and the
@@ -1183,14 +1177,17 @@ __device__ __forceinline__ void tensor_info_of_lanes(int rank, int itemsize, int
 
 // Stages tile `tile` with `nthreads` (>= 64) cooperating threads (this thread is `tid`).  The
 // caller synchronises before the stage is read.  Only global loads and LDS writes: no stores.
-// Every vector load of the tile is issued first, in one round, and the state terms are
-// computed from scalar operands while the loads are in flight: under a store-bound kernel
-// each dependent round of vector loads queues behind the stores of the other workgroups of
-// the compute unit, so the number of rounds, not of loads, is what staging costs.
+// A vector load waits behind every store the compute unit has in flight, so what staging costs under a store-bound
+// kernel is the vector loads it issues: all of them at once, in one round, and each by one wavefront of the tile only.  The
+// first takes the producer specs, the image and (DERIVE) the tensor, the last the consumer specs; what is the same for all lanes comes
+// through the scalar cache.  (When every wavefront loaded everything, twelve loads each, four more cost the one launch over 66 M
+// entries in 80 layers 11 of 142 us.  us a pass, twelve loads a wavefront / five a tile: 20 M entries on (16, 8, 4) 62.6 / 61.4, 47 M in eight
+// layers on (64, 4) 129.7 / 123.8, 5.9 M there 26.4 / 25.2, 1.8 M on (16, 8, 4) 14.5 / 13.4, 2.6 M on (12, 6) 11.5 / 11.4, 66 M in 80 layers
+// 127.1 / 126.4; the other way 704 k on (6, 4, 2) 11.3 / 11.6.)
 template <int M, bool DERIVE, bool RM>
 __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs &a, const apc_tile &tile,
-                                           TileStage<M, RM> &st, int tid, int nthreads, TileCopies &copies) {
-  constexpr int NS = TermTable<M>::kStates;
+                                           TileStage<M> &st, int tid, int nthreads, TileCopies &copies) {
+  constexpr int NS = TermTable<M>::kStates, kComputed = kComputedArrays<M>, kPieces = kImagePieces<M>;
   const int rows = tile.counts & 0xFFFF, cols = tile.counts >> 16;
   const int t0 = tile.tensor;  // spec_tensor of the tile's first producer spec (checked by the host)
   const bool no_producer = (tile.flags & APC_EDGE_NO_PRODUCER) != 0;
@@ -1198,64 +1195,65 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
   bool mixed = !terms_wanted;
   const TermLayout &lay = a.lay;
   const int E = lay.exponents;  // wave-uniform; 0: general layout
-  const int lane = tid & 63, wave = tid >> 6;
-  // (A kernel argument indexed by the lane: one vector load, part of the round below.)
-  static_assert(kPairWords<M> <= 64, "one word a lane of the smallest workgroup");
-  uint32_t pair_word = 0;
-  if (tid < kPairWords<M>) pair_word = lay.pair[tid];
-  // power-of-two layout: the constants of array 2 + lane (whose chain this lane computes) and of
-  // the array of the first value this thread computes, also read by lane
-  constexpr int kComputed = 3 * M + 2;
-  TermArrayConstants chain_of;
-  if (E != 0) chain_of = load_of_lane(lay.arrays, (uint32_t)min(lane, kComputed - 1));
-  // ---- the round of vector loads ------------------------------------------------------------
-  // producer spec tid, consumer spec nthreads - 1 - tid (taken from the far end: with two
-  // wavefronts one loads the producer specs while the other loads the consumer specs).
-  // Threads past the tile's specs load its first spec again: unconditional loads, whose
-  // values are first touched after the state terms.
-  const int jc = tid, jr = nthreads - 1 - tid;
-  const bool has_col = jc < cols, has_row = jr < rows;
-  const uint32_t at_col = has_col ? (uint32_t)jc : 0u, at_row = has_row ? (uint32_t)jr : 0u;
-  const int64_t sp = (int64_t)tile.src_begin + tile.col_begin, ts = (int64_t)tile.tgt_begin + tile.row_begin;
-  const int64_t sr = (int64_t)tile.strat_begin + tile.row_begin;
-  const int col_tensor = load_of_lane(a.spec_tensor + sp, at_col);
-  const uint32_t col_codes = load_of_lane(a.spec_codes + sp, at_col);
-  const uint32_t row_codes = load_of_lane(a.spec_codes + ts, at_row);
-  const int row_tensor = load_of_lane(a.spec_tensor + ts, at_row);
-  double row_cpa = 0.0;
-  int64_t row_flops = 0, row_rw = 0;
-  int row_dtype = 0, row_zero = 1, row_args = 1;
+  const int lane = tid & 63, wave = uniform_i32(tid >> 6);
+  static_assert(APC_TILE_MAX_COLS <= 64 && APC_TILE_MAX_ROWS <= 64, "a wavefront for the specs of either side");
+  const bool first_wave = wave == 0, last_wave = wave == (nthreads >> 6) - 1;
   const int t0c = t0 >= 0 ? t0 : 0;  // (row 0 when the tile has no tensor: unconditional loads, the values are not used then)
+  // ---- the round of vector loads ------------------------------------------------------------
+  // Lanes past the tile's specs load its first spec again.
+  const bool has_col = first_wave && lane < cols, has_row = last_wave && lane < rows;
+  const uint32_t at_col = has_col ? (uint32_t)lane : 0u, at_row = has_row ? (uint32_t)lane : 0u;
+  u32x4 piece{}, piece2{};
+  int col_tensor = 0, row_tensor = 0;
+  uint32_t col_codes = 0, row_codes = 0;
   int64_t dim_size = 0, dim_stride = 0;
-  double gf_of_lane = 0.0, inv_gf_of_lane = 0.0;
-  if (!DERIVE) {
-    if (a.per_arg) row_cpa = load_of_lane(a.per_arg + sr, at_row);
-  } else {
+  if (first_wave) {
+    struct __attribute__((packed, aligned(8))) Piece {
+      u32x4 v;
+    };
+    const Piece *image = reinterpret_cast<const Piece *>(lay.image);
+    piece = load_of_lane(image, (uint32_t)min(lane, kPieces - 1)).v;
+    if (kPieces > 64) piece2 = load_of_lane(image, (uint32_t)min(lane + 64, kPieces - 1)).v;
+    const int64_t sp = (int64_t)tile.src_begin + tile.col_begin;
+    col_codes = load_of_lane(a.spec_codes + sp, at_col);
+    col_tensor = load_of_lane(a.spec_tensor + sp, at_col);
+  }
+  if (DERIVE && (first_wave || E == 0)) {  // (general layout: every wavefront takes part in the states)
     dim_size = load_of_lane(a.shape + (int64_t)t0c * APC_MAX_RANK, (uint32_t)lane & (APC_MAX_RANK - 1));
     dim_stride = load_of_lane(a.stride + (int64_t)t0c * APC_MAX_RANK, (uint32_t)lane & (APC_MAX_RANK - 1));
-    // (lane j holds the throughput of dtype code j & 7: fetched by the lanes that need it, below)
-    gf_of_lane = load_of_lane(p.gpu_flops, (uint32_t)lane & (APC_MAX_DTYPES - 1));
-    inv_gf_of_lane = load_of_lane(p.inv_gpu_flops, (uint32_t)lane & (APC_MAX_DTYPES - 1));
-    row_flops = load_of_lane(a.flops + sr, at_row);
-    row_rw = load_of_lane(a.rw_bytes + sr, at_row);
-    row_dtype = load_of_lane(a.dtype + sr, at_row);
-    row_zero = load_of_lane(a.zero_cost + sr, at_row);
-    row_args = load_of_lane(a.num_args + sr, at_row);
+  }
+  double row_cpa = 0.0, gf_of_lane = 0.0, inv_gf_of_lane = 0.0;
+  int64_t row_flops = 0, row_rw = 0;
+  int row_dtype = 0, row_zero = 1, row_args = 1;
+  if (last_wave) {
+    const int64_t ts = (int64_t)tile.tgt_begin + tile.row_begin, sr = (int64_t)tile.strat_begin + tile.row_begin;
+    row_codes = load_of_lane(a.spec_codes + ts, at_row);
+    row_tensor = load_of_lane(a.spec_tensor + ts, at_row);
+    if (!DERIVE) {
+      if (a.per_arg) row_cpa = load_of_lane(a.per_arg + sr, at_row);
+    } else {
+      // (lane j holds the throughput of dtype code j & 7: fetched by the lanes that need it, below)
+      gf_of_lane = load_of_lane(p.gpu_flops, (uint32_t)lane & (APC_MAX_DTYPES - 1));
+      inv_gf_of_lane = load_of_lane(p.inv_gpu_flops, (uint32_t)lane & (APC_MAX_DTYPES - 1));
+      row_flops = load_of_lane(a.flops + sr, at_row);
+      row_rw = load_of_lane(a.rw_bytes + sr, at_row);
+      row_dtype = load_of_lane(a.dtype + sr, at_row);
+      row_zero = load_of_lane(a.zero_cost + sr, at_row);
+      row_args = load_of_lane(a.num_args + sr, at_row);
+    }
   }
   // (every wavefront its own copy of the identical edges' offsets, in lanes 0 .. dup_count - 1)
-  const bool has_dup0 = lane < tile.dup_count;
   copies.entry0 = copies.row0 = copies.row_out = 0;
-  if (has_dup0) copies.entry0 = load_of_lane(a.dup_entry_begin + tile.dup_begin, (uint32_t)lane);
-  if constexpr (RM) {
-    if (has_dup0) copies.row0 = load_of_lane(a.dup_row_begin + tile.dup_begin, (uint32_t)lane);
-    // (wave-uniform, but needed last: with the vector loads of the round, so that the scalar
-    // loads the term arrays wait for are one round and not two)
-    copies.row_out = a.edge_row_begin[tile.edge];
+  if (tile.dup_count > 0 && lane < tile.dup_count) {
+    copies.entry0 = load_of_lane(a.dup_entry_begin + tile.dup_begin, (uint32_t)lane);
+    if constexpr (RM) copies.row0 = load_of_lane(a.dup_row_begin + tile.dup_begin, (uint32_t)lane);
   }
   // ---- the scalar loads of the round (wave-uniform addresses), issued together ---------------------
-  // The contiguity byte is read as the aligned word around it (which lies in the byte's own page).
-  bool contiguous;
-  double fbytes;
+  // The tile's tensor and the first matrix row of its edge.  The contiguity byte is read as the aligned word around it (which
+  // lies in the byte's own page).
+  if constexpr (RM) copies.row_out = uniform_load(a.edge_row_begin + tile.edge);
+  bool contiguous = true;
+  double fbytes = 0.0;
   if constexpr (!DERIVE) {
     const uint8_t *flag = a.tensor_contiguous + t0c;
     const uint32_t byte = (uint32_t)(reinterpret_cast<uintptr_t>(flag) & 3);
@@ -1267,43 +1265,29 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
   } else {
     const int t_rank = uniform_load(a.rank + t0c), t_item = uniform_load(a.itemsize + t0c);
     fetch_arguments_now(t_rank, t_item);
-    tensor_info_of_lanes(t_rank, t_item, dim_size, dim_stride, lane, fbytes, contiguous);
+    if (first_wave || E == 0) tensor_info_of_lanes(t_rank, t_item, dim_size, dim_stride, lane, fbytes, contiguous);
   }
+  char *const image = reinterpret_cast<char *>(st.image);
+  if (first_wave) {
+    if (lane < kPieces) *reinterpret_cast<u32x4 *>(image + lane * 16) = piece;
+    if (kPieces > 64 && lane < kPieces - 64) *reinterpret_cast<u32x4 *>(image + (lane + 64) * 16) = piece2;
+  }
+  const char *const arrays = image + kPairWords<M> * 4;  // (TermArrayConstants)
   // ---- term arrays --------------------------------------------------------------------------
-  if (terms_wanted && E != 0) {
-    // power-of-two mesh.  A lane per computed array takes the array's chain on the tensor's
-    // bytes (every wavefront its own copy: no barrier), then a lane per (array, exponent) the
-    // value.
-    StagingScratch &mine = *reinterpret_cast<StagingScratch *>(wave_scratch(st, wave));
-    if (lane < kComputed) {
-      mine.chain[lane] = div_by(div_by(fbytes * chain_of.hops, chain_of.div1, chain_of.inv_div1) * 1e6, chain_of.div2,
-                                chain_of.inv_div2);
-      mine.value_of[lane] = TermValueConstants{chain_of.lat, chain_of.floor, chain_of.scale, chain_of.shift, 0};
-    }
+  if (terms_wanted && E != 0 && first_wave) {
+    // power-of-two mesh.  A lane per computed array takes the array's chain on the tensor's bytes; below a lane per (array,
+    // exponent) the value.
     __builtin_amdgcn_wave_barrier();  // (LDS operations of one wavefront complete in order)
-    // (The value constants go through LDS as well.  Read from the kernel arguments by a per-lane
-    // index inside the loop below, `lat + ldexp(..)` was compiled to `x + x` in the 4-D
-    // instantiations by hipcc 7.2: the placement-pair tests on 4-D power-of-two meshes show it.)
-    char *terms = term_base(st, nthreads);
-    for (int t = tid; t < kComputed * E; t += nthreads) {
-      // (24-bit multiplies: an integer multiply of 32 bits takes four times as long)
-      const int arr = (int)((uint32_t)__umul24((uint32_t)t, lay.exponent_magic) >> 16);  // t / E
-      const int j = t - __mul24(arr, E);  // the running bytes are bytes x 2^(j - L - 30)
-      const TermValueConstants k = mine.value_of[arr];
-      double v = k.lat + __builtin_ldexp(mine.chain[arr], j + k.shift);
-      v = v > k.floor ? v : k.floor;
-      v = v * k.scale;
-      *reinterpret_cast<double *>(terms + __mul24(j, kPow2Stride) + (arr + 2) * 8) = v;
+    if (lane < kComputed) {
+      const TermArrayConstants &k = *reinterpret_cast<const TermArrayConstants *>(arrays + lane * sizeof(TermArrayConstants));
+      st.chain[lane] = div_by(div_by(fbytes * k.hops, k.div1, k.inv_div1) * 1e6, k.div2, k.inv_div2);
     }
-    if (tid < 2 * E) {
-      const int j = tid < E ? tid : tid - E;
-      *reinterpret_cast<double *>(terms + __mul24(j, kPow2Stride) + (tid < E ? 0 : 8)) = tid < E ? 0.0 : __builtin_inf();
-    }
-  } else if (terms_wanted) {
+  }
+  if (terms_wanted && E == 0) {
     // every collective / read-write term the tile can need, once per running-bytes state, in
     // the reference's operation order (collective_runtime_estimation.py:66-68, :86, :128;
     // torch _collective_utils.py:281-313; compute_estimation.py:302-314)
-    double *const terms = reinterpret_cast<double *>(term_base(st, nthreads));
+    double *const terms = st.terms;
     const auto bytes_at = [&](int level, int mask, int hist) {
       double shards = 1.0;  // exact: a product of mesh sizes (torch _dtensor_spec.py:555-561)
 #pragma unroll
@@ -1360,7 +1344,6 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
   }
   // ---- what the loads brought, to LDS ---------------------------------------------------------
   if (tid == 0) st.cont = contiguous;
-  if (tid < kPairWords<M>) st.words[tid] = pair_word;
   if (has_col) {
     uint32_t slots = 0, codes = col_codes, others = 0;
     int index = lay.index0;
@@ -1375,13 +1358,13 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
     if (M == 2 && col_codes == 0x4040u) codes |= kFlipShift << 24;
     if (M < 4) slots |= (uint32_t)index << 24;
     if (col_tensor < 0) slots |= kNotASpec;
-    if constexpr (M < 4) st.col[jc] = ColRecord<M>{codes, slots};
-    else st.col[jc] = ColRecord<M>{codes, slots, (uint32_t)index, 0u};
+    if constexpr (M < 4) st.col[lane] = ColRecord<M>{codes, slots};
+    else st.col[lane] = ColRecord<M>{codes, slots, (uint32_t)index, 0u};
     if (col_tensor != t0 || col_tensor < 0) mixed = true;
   }
   double row_cost = 0.0;
-  if constexpr (DERIVE) {  // (every lane takes part in the exchange; by the wavefronts that hold rows)
-    if (uniform_i32(nthreads - 64 - (tid - lane)) < rows) {
+  if constexpr (DERIVE) {  // (every lane takes part in the exchange)
+    if (last_wave) {
       const bool known = row_dtype >= 0 && row_dtype < APC_MAX_DTYPES;
       const double gf = from_lane(gf_of_lane, row_dtype & (APC_MAX_DTYPES - 1)), inv_gf = from_lane(inv_gf_of_lane, row_dtype & (APC_MAX_DTYPES - 1));
       row_cost = compute_cost_through_reciprocals(p, row_zero != 0, row_rw, row_flops, known ? gf : 0.0, known ? inv_gf : 0.0);
@@ -1407,12 +1390,35 @@ __device__ __forceinline__ void stage_tile(const apc_params &p, const TableArgs 
       mixed = true;
     }
     if (DERIVE) row_cpa = row_cost / (double)row_args;  // the value compute_costs_block writes for this strategy
-    st.row[jr] = RowRecord{row_codes, slots, row_cpa};
+    st.row[lane] = RowRecord{row_codes, slots, row_cpa};
   }
   // one flag per wavefront, written unconditionally: nothing to clear beforehand
   const bool wave_mixed = __ballot(mixed) != 0;
-  if ((tid & 63) == 0) st.mixed[tid >> 6] = wave_mixed ? 1 : 0;
+  if (lane == 0) st.mixed[wave] = wave_mixed ? 1 : 0;
+  // ---- the values of the power-of-two layout's arrays ------------------------------------------
+  if (terms_wanted && E != 0) {
+    if (nthreads > 64) __syncthreads();
+    else __builtin_amdgcn_wave_barrier();
+    char *const terms = reinterpret_cast<char *>(st.terms);
+    for (int t = tid; t < kComputed * E; t += nthreads) {
+      // (24-bit multiplies: an integer multiply of 32 bits takes four times as long)
+      const int arr = (int)((uint32_t)__umul24((uint32_t)t, lay.exponent_magic) >> 16);  // t / E
+      const int j = t - __mul24(arr, E);  // the running bytes are bytes x 2^(j - L - 30)
+      // (Constants out of LDS.  Read from the kernel arguments by a per-lane index inside this loop, `lat + ldexp(..)` was
+      // compiled to `x + x` in the 4-D instantiations by hipcc 7.2: the placement-pair tests on 4-D power-of-two meshes show it.)
+      const TermArrayConstants &k = *reinterpret_cast<const TermArrayConstants *>(arrays + __mul24(arr, (int)sizeof(TermArrayConstants)));
+      double v = k.lat + __builtin_ldexp(st.chain[arr], j + k.shift);
+      v = v > k.floor ? v : k.floor;
+      v = v * k.scale;
+      *reinterpret_cast<double *>(terms + __mul24(j, kPow2Stride) + (arr + 2) * 8) = v;
+    }
+    if (tid < 2 * E) {
+      const int j = tid < E ? tid : tid - E;
+      *reinterpret_cast<double *>(terms + __mul24(j, kPow2Stride) + (tid < E ? 0 : 8)) = tid < E ? 0.0 : __builtin_inf();
+    }
+  }
 }
+
 
 // The arguments an entry loop uses, in scalar registers before it begins.  (Left to the compiler, an argument is loaded
 // where it is used, in every pass, and a scalar load in flight makes the wait for an LDS read a wait for everything.)
@@ -1437,18 +1443,18 @@ struct TileWalk {
 struct TileSteps {  // of one pass; `wrap`: when the column passes the row's end
   uint32_t dcol, end, cols, drow, drow_wrap, dout, dout_wrap;
 };
-template <int M, bool RM>
+template <int M>
 __device__ __forceinline__ TileWalk tile_walk(lds_address stage, int r, int c, int n_src) {
-  return TileWalk{stage + cols_at<M, RM>() + (uint32_t)c * (uint32_t)sizeof(ColRecord<M>),
-                  stage + rows_at<M, RM>() + (uint32_t)r * 16u,
+  return TileWalk{stage + cols_at<M>() + (uint32_t)c * (uint32_t)sizeof(ColRecord<M>),
+                  stage + rows_at<M>() + (uint32_t)r * 16u,
                   (uint32_t)(__mul24(r, n_src) + c) * 8u};
 }
 // (dr, dc: rows and columns of a pass; uniform, as everything here)
-template <int M, bool RM>
+template <int M>
 __device__ __forceinline__ TileSteps tile_steps(lds_address stage, uint32_t dr, uint32_t dc, uint32_t cols, uint32_t n_src) {
   constexpr uint32_t kCol = (uint32_t)sizeof(ColRecord<M>);
   const uint32_t dout = (dr * n_src + dc) * 8u;
-  return TileSteps{dc * kCol, stage + cols_at<M, RM>() + cols * kCol, cols * kCol, dr * 16u, dr * 16u + 16u, dout, dout + (n_src - cols) * 8u};
+  return TileSteps{dc * kCol, stage + cols_at<M>() + cols * kCol, cols * kCol, dr * 16u, dr * 16u + 16u, dout, dout + (n_src - cols) * 8u};
 }
 template <bool WHOLE>  // whole rows: the entries of a tile are consecutive
 __device__ __forceinline__ void advance(TileWalk &w, const TileSteps &s) {
@@ -1505,7 +1511,7 @@ __device__ __forceinline__ void word_slots(uint32_t src, uint32_t tgt, uint32_t 
 // (6, 4, 2) 16.0 -> 15.4.  (Every copy's address in scalar registers, one instruction less a store, is 1 % slower.)
 // Straight-line code: all lookups of an entry are independent of its fp additions, so they
 // are issued together; no vector memory loads.
-template <int M, bool RM, bool CONT, bool RESCALE>
+template <int M, bool CONT, bool RESCALE>
 __device__ __forceinline__ void uniform_entry(const EntryConstants &k, lds_address stage, lds_address terms, const TileWalk &where, double &comm_o,
                                               double &total_o, int &trans_o) {
   typedef uint32_t col_words __attribute__((ext_vector_type(sizeof(ColRecord<M>) / 4)));
@@ -1526,7 +1532,7 @@ __device__ __forceinline__ void uniform_entry(const EntryConstants &k, lds_addre
   word_slots<0>(src, row.codes, slots, slot);
 #pragma unroll
   for (int i = 0; i < M; ++i) {
-    const uint32_t w = lds_read<uint32_t>(stage + words_at<M, RM>() + slot[i]);
+    const uint32_t w = lds_read<uint32_t>(stage + words_at<M>() + slot[i]);
     term_at[i] = (w & 0xFFFFu) + at;
     rw_at[i] = term_at[i] + (uint32_t)(int32_t)(int8_t)(w >> 16);
     if (!CONT) nc_at[i] = at + (uint32_t)(kRw1Array * 8u + ((1u << i) - 1u) * (uint32_t)k.level_stride);  // (the state before the dim)
@@ -1693,7 +1699,7 @@ __device__ __forceinline__ void tile_entries_row_min(const TableArgs &a, lds_add
                                                      int tid, int nthreads, Entry entry) {
   const int lane = tid & 63, wave = uniform_i32(tid >> 6), waves = nthreads >> 6;
   constexpr bool RM = true;
-  const lds_address values = stage + terms_at<M, RM>() + (uint32_t)kWaveScratchBytes<RM> * (uint32_t)wave;  // (wave_scratch)
+  const lds_address values = stage + terms_at<M>() + term_bytes<M>(a.lay) + (uint32_t)kWaveScratchBytes<RM> * (uint32_t)wave;
   const int cols = v.cols;
   // bytes from row to row: an odd number of doubles, so that the lanes of consecutive rows read different banks
   const uint32_t row_bytes = (uint32_t)(cols | 1) * 8u;
@@ -1701,7 +1707,7 @@ __device__ __forceinline__ void tile_entries_row_min(const TableArgs &a, lds_add
   const int at_once = min((int)uniform_quotient(kRowMinValues, __builtin_amdgcn_rcpf((float)(cols | 1))), 64);
   const int r0 = (int)small_quotient((uint32_t)lane, inv_cols), c0 = lane - __mul24(r0, cols);
   const uint32_t dr = uniform_quotient(64, inv_cols), dc = 64u - dr * (uint32_t)cols;
-  const TileSteps steps = tile_steps<M, RM>(stage, dr, dc, (uint32_t)cols, (uint32_t)cols);
+  const TileSteps steps = tile_steps<M>(stage, dr, dc, (uint32_t)cols, (uint32_t)cols);
   const int row_begin = (int)((uint32_t)(v.rows * wave) / (uint32_t)waves), row_end = (int)((uint32_t)(v.rows * (wave + 1)) / (uint32_t)waves);
   const int64_t tile_base = v.entry_begin + (int64_t)v.row_begin * v.n_src + v.col_begin;
   const TileOut out{a.comm_out ? a.comm_out + tile_base : nullptr, a.trans_out ? a.trans_out + tile_base : nullptr,
@@ -1710,8 +1716,8 @@ __device__ __forceinline__ void tile_entries_row_min(const TableArgs &a, lds_add
   const uint32_t pad = (cols & 1) ? 31u : 1u;  // (a record of 16 bytes a row)
   for (int first = row_begin; first < row_end; first += at_once) {
     const int rows = min(at_once, row_end - first), n = rows * cols;
-    TileWalk w = tile_walk<M, RM>(stage, first + r0, c0, cols);
-    const uint32_t to_values = values - (uint32_t)(first * cols) * 8u - ((stage + rows_at<M, RM>() + (uint32_t)first * 16u) >> pad);
+    TileWalk w = tile_walk<M>(stage, first + r0, c0, cols);
+    const uint32_t to_values = values - (uint32_t)(first * cols) * 8u - ((stage + rows_at<M>() + (uint32_t)first * 16u) >> pad);
     for (int at = 0; at < n; at += 64) {
       const bool active = at + lane < n;
       const double total = store_entry<OUT>(out, v.dup_count, copies, active, w, entry);
@@ -1774,20 +1780,20 @@ __device__ __forceinline__ void tile_entries_row_min(const TableArgs &a, lds_add
 // of the fp64 streams) instead of straddling one more line than it fills.  Every lane of a
 // wavefront makes the same number of passes (a lane in front of the tile's first entry idles
 // in the first one), so the copies' offsets are read under uniform control flow.
-template <int M, int OUT, bool WHOLE, bool RM, typename Entry>
+template <int M, int OUT, bool WHOLE, typename Entry>
 __device__ __forceinline__ void tile_entries_walk(const TableArgs &a, lds_address stage, const TileView &v, const TileCopies &copies,
                                                   int tid, int nthreads, Entry entry) {
   const int n = v.rows * v.cols;
   const float inv_cols = __builtin_amdgcn_rcpf((float)v.cols);
   const uint32_t dr = uniform_quotient((uint32_t)nthreads, inv_cols), dc = (uint32_t)nthreads - dr * (uint32_t)v.cols;
   const int n_src = WHOLE ? v.cols : v.n_src;
-  const TileSteps steps = tile_steps<M, RM>(stage, dr, dc, (uint32_t)v.cols, (uint32_t)n_src);
+  const TileSteps steps = tile_steps<M>(stage, dr, dc, (uint32_t)v.cols, (uint32_t)n_src);
   const int64_t tile_base = v.entry_begin + (int64_t)v.row_begin * v.n_src + v.col_begin;
   const int shift = WHOLE ? (int)(tile_base & 63) : 0;
   const int lane = tid & 63;
   // (in front of the tile's first entry rows count backwards: 64 rows are more than the shift)
   const int r = (int)small_quotient((uint32_t)(tid - shift + 64 * v.cols), inv_cols) - 64;
-  TileWalk w = tile_walk<M, RM>(stage, r, tid - shift - __mul24(r, v.cols), n_src);
+  TileWalk w = tile_walk<M>(stage, r, tid - shift - __mul24(r, v.cols), n_src);
   const TileOut out{a.comm_out ? a.comm_out + tile_base : nullptr, a.trans_out ? a.trans_out + tile_base : nullptr,
                     a.cost_out ? a.cost_out + tile_base : nullptr, v.entry_begin};
   for (int at = uniform_i32(tid - lane) - shift; at < n; at += nthreads) {
@@ -1797,10 +1803,10 @@ __device__ __forceinline__ void tile_entries_walk(const TableArgs &a, lds_addres
 }
 
 // The generic entry: pass-through edges and edges whose producer specs name different tensors.
-template <int M, bool DERIVE, bool RM>
-__device__ __forceinline__ void generic_entry(const apc_params &p, const TableArgs &a, const TileStage<M, RM> &st, lds_address stage, const TileView &v,
+template <int M, bool DERIVE>
+__device__ __forceinline__ void generic_entry(const apc_params &p, const TableArgs &a, const TileStage<M> &st, lds_address stage, const TileView &v,
                                               const TileWalk &where, double &comm, double &total, int &trans) {
-  const int r = (int)((where.row - stage - rows_at<M, RM>()) / 16u), c = (int)((where.col - stage - cols_at<M, RM>()) / (uint32_t)sizeof(ColRecord<M>));
+  const int r = (int)((where.row - stage - rows_at<M>()) / 16u), c = (int)((where.col - stage - cols_at<M>()) / (uint32_t)sizeof(ColRecord<M>));
   const int64_t local = (int64_t)(v.row_begin + r) * v.n_src + (v.col_begin + c);
   const ColRecord<M> col = st.col[c];
   const uint32_t src = M == 2 ? col.codes & 0xFFFFu : col.codes;  // (without the flip's shift)
@@ -1829,7 +1835,7 @@ __device__ __forceinline__ void generic_entry(const apc_params &p, const TableAr
 // All entries of a staged tile.  Row minima are taken when the caller wants them and the tile
 // holds whole rows (which the host arranges for every tile of a table before asking).
 template <int M, bool DERIVE, bool RM, int OUT>
-__device__ __forceinline__ void tile_entries(const apc_params &p, const TableArgs &a, const TileStage<M, RM> &st, lds_address stage,
+__device__ __forceinline__ void tile_entries(const apc_params &p, const TableArgs &a, const TileStage<M> &st, lds_address stage,
                                              const TileView &v, const TileCopies &copies, int tid, int nthreads) {
   int mixed = st.mixed[0];
   for (int w = 1; w < nthreads / 64; ++w) mixed |= st.mixed[w];
@@ -1842,8 +1848,8 @@ __device__ __forceinline__ void tile_entries(const apc_params &p, const TableArg
         return;
       }
     }
-    if (whole) tile_entries_walk<M, kOut, true, RM>(a, stage, v, copies, tid, nthreads, entry);
-    else tile_entries_walk<M, kOut, false, RM>(a, stage, v, copies, tid, nthreads, entry);
+    if (whole) tile_entries_walk<M, kOut, true>(a, stage, v, copies, tid, nthreads, entry);
+    else tile_entries_walk<M, kOut, false>(a, stage, v, copies, tid, nthreads, entry);
   };
   if (uniform_i32(mixed)) {
     entries(std::integral_constant<int, kOutAny>{}, [&](const TileWalk &where, double &comm, double &total, int &trans) {
@@ -1853,10 +1859,10 @@ __device__ __forceinline__ void tile_entries(const apc_params &p, const TableArg
   }
   const bool rescale = (v.flags & APC_EDGE_GRAD_RESCALE) != 0;
   const EntryConstants k = entry_constants(p, a.lay);
-  const lds_address terms = stage + terms_at<M, RM>() + (uint32_t)kWaveScratchBytes<RM> * (uint32_t)(nthreads >> 6);  // (term_base)
+  const lds_address terms = stage + terms_at<M>();
 #define APC_TILE_LOOP(CONT_, RESCALE_)                                                                                       \
   entries(std::integral_constant<int, OUT>{}, [&](const TileWalk &where, double &comm, double &total, int &trans) {          \
-    uniform_entry<M, RM, CONT_, RESCALE_>(k, stage, terms, where, comm, total, trans);                                                  \
+    uniform_entry<M, CONT_, RESCALE_>(k, stage, terms, where, comm, total, trans);                                                  \
   })
   if (uniform_i32(st.cont)) {
     if (rescale) { APC_TILE_LOOP(true, true); } else { APC_TILE_LOOP(true, false); }
@@ -1898,7 +1904,7 @@ __device__ __forceinline__ apc_tile fetch_tile(const apc_tile *tiles, int64_t ti
 
 template <int M, int kTileThreads, bool RM, int OUT>
 __device__ __forceinline__ void redistribute_tile(const apc_params &p, const TableArgs &a, const apc_tile *tiles, int n_tiles,
-                                                  int xcd_shift, TileStage<M, RM> &stage, lds_address at) {
+                                                  int xcd_shift, TileStage<M> &stage, lds_address at) {
   const int tile_id = tile_of_block((int)blockIdx.x, n_tiles, xcd_shift);
   if (tile_id >= n_tiles) return;
   static_assert(kTileThreads == 64 || kTileThreads == 128 || kTileThreads == 256, "wavefronts per tile: 1, 2 or 4");
@@ -1939,7 +1945,7 @@ void redistribute_tiles_kernel(APC_LAUNCH_PARAMS(TilesBlock, false)) {
   extern __shared__ __align__(16) unsigned char s_stage_bytes[];  // stage_lds_bytes<M, false>
   const TilesBlock &k = launch_block<false>(kept);
   redistribute_tile<M, kTileThreads, false, OUT>(k.p, k.a, static_cast<const apc_tile *>(work), n_tiles, xcd_shift,
-                                                 *reinterpret_cast<TileStage<M, false> *>(s_stage_bytes), address_in_lds(s_stage_bytes));
+                                                 *reinterpret_cast<TileStage<M> *>(s_stage_bytes), address_in_lds(s_stage_bytes));
 }
 
 // The same with the row minima.
@@ -1950,7 +1956,7 @@ void redistribute_tiles_row_min_kernel(APC_LAUNCH_PARAMS(TilesBlock, false)) {
   extern __shared__ __align__(16) unsigned char s_stage_bytes[];  // stage_lds_bytes<M, true>
   const TilesBlock &k = launch_block<false>(kept);
   redistribute_tile<M, kTileThreads, true, OUT>(k.p, k.a, static_cast<const apc_tile *>(work), n_tiles, xcd_shift,
-                                                *reinterpret_cast<TileStage<M, true> *>(s_stage_bytes), address_in_lds(s_stage_bytes));
+                                                *reinterpret_cast<TileStage<M> *>(s_stage_bytes), address_in_lds(s_stage_bytes));
 }
 
 // Every table of a pass in one launch: workgroups [0, tile_blocks) take the tiles of the
@@ -1996,7 +2002,7 @@ void build_tables_kernel(APC_LAUNCH_PARAMS(BuildTablesBlock, KEPT)) {
   if (b < tile_blocks) {
     const int tile_id = tile_of_block((int)b, n_tiles, xcd_shift);
     if (tile_id >= n_tiles) return;
-    TileStage<M, RM> &stage = *reinterpret_cast<TileStage<M, RM> *>(s_raw);
+    TileStage<M> &stage = *reinterpret_cast<TileStage<M> *>(s_raw);
     const apc_tile tile = fetch_tile<true, RM, OUT>(tiles, tile_id, a);
     if ((unsigned)tile.dup_count > (unsigned)APC_TILE_MAX_DUPS) return;  // (see redistribute_tile)
     TileCopies copies;
