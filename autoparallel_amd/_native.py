@@ -84,6 +84,8 @@ EXPORTS = (
     "apc_segmented_min",
     "apc_segmented_min_copies",
     "apc_strategy_bounds",
+    "apc_greedy_strategies",
+    "apc_edge_rows",
     "apc_cost_objective",
     "apc_validate_row_minima_host",
     "apc_diffusion_sweeps",

@@ -2493,6 +2493,83 @@ __global__ __launch_bounds__(kBlock) void strategy_bounds_kernel(int64_t n_strat
   bound[s] = sum;
 }
 
+// The bounds, the smallest of every node and the first strategy that has it: G consecutive lanes to a node, its
+// strategies and their order those of segmented_min_kernel, so that the result is its result, NaN included.  (One launch instead of two,
+// and a node's edges are looked up by a lane once for its strategies.)
+template <int G>
+__global__ __launch_bounds__(kBlock) void greedy_strategies_kernel(int64_t n_nodes, const int64_t *__restrict__ node_strat_begin,
+                                                                   const int64_t *__restrict__ node_edge_begin,
+                                                                   const int32_t *__restrict__ edges_by_node,
+                                                                   const int64_t *__restrict__ edge_row_begin,
+                                                                   const double *__restrict__ row_min, double *__restrict__ bound,
+                                                                   double *__restrict__ node_min, int32_t *__restrict__ node_argmin) {
+  const int sub = threadIdx.x & (G - 1);
+  const int64_t n = (int64_t)blockIdx.x * (kBlock / G) + (threadIdx.x / G);
+  const bool live = n < n_nodes;
+  const int64_t lo = live ? node_strat_begin[n] : 0, hi = live ? node_strat_begin[n + 1] : 0;
+  const int64_t e0 = live ? node_edge_begin[n] : 0, e1 = live ? node_edge_begin[n + 1] : 0;
+  double best = INFINITY;
+  int64_t arg = INT64_MAX;  // INT64_MAX = none seen
+  auto take = [&](double v, int64_t j) {
+    bound[j] = v;
+    if (arg == INT64_MAX || v < best) {
+      best = v;
+      arg = j;
+    }
+  };
+  for (int64_t j = lo + 2 * sub; j < hi; j += 2 * G) {
+    const bool second = j + 1 < hi;
+    double x = 0.0, y = 0.0;
+    for (int64_t e = e0; e < e1; ++e) {
+      const double *row = row_min + edge_row_begin[edges_by_node[e]] + (j - lo);
+      x += row[0];
+      if (second) y += row[1];
+    }
+    take(x, j);
+    if (second) take(y, j + 1);
+  }
+#pragma unroll
+  for (int off = G / 2; off > 0; off >>= 1) {
+    const double ob = __shfl_xor(best, off, 64);
+    const int64_t oa = __shfl_xor(arg, off, 64);
+    if (oa != INT64_MAX && (arg == INT64_MAX || ob < best || (ob == best && oa < arg))) {
+      best = ob;
+      arg = oa;
+    }
+  }
+  if (live && sub == 0) {
+    node_min[n] = best;
+    node_argmin[n] = arg == INT64_MAX ? -1 : (int32_t)(arg - lo);
+  }
+}
+
+// First matrix row of every edge: one workgroup, a run of edges a thread, the runs' sums scanned across it.  (8 300 edges: 5 us on the
+// device, where the host's sum, a transfer and its wait took 42.)
+constexpr int kScanThreads = 1024;
+__global__ __launch_bounds__(kScanThreads) void edge_rows_kernel(int64_t n_edges, const int32_t *__restrict__ n_tgt, int64_t *__restrict__ begin) {
+  __shared__ int64_t s_wave[kScanThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t run = (n_edges + kScanThreads - 1) / kScanThreads;
+  const int64_t first = run * tid < n_edges ? run * tid : n_edges, last = first + run < n_edges ? first + run : n_edges;
+  int64_t sum = 0;
+#pragma unroll 4
+  for (int64_t e = first; e < last; ++e) sum += n_tgt[e];
+  int64_t upto = sum;  // of this wavefront's runs, this one's included
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int64_t o = __shfl_up(upto, off, 64);
+    if (lane >= off) upto += o;
+  }
+  if (lane == 63) s_wave[wave] = upto;
+  __syncthreads();
+  int64_t at = upto - sum;
+  for (int w = 0; w < wave; ++w) at += s_wave[w];
+  for (int64_t e = first; e < last; ++e) {
+    begin[e] = at;
+    at += n_tgt[e];
+  }
+}
+
 // ------------------------------------------------------------------------------------------
 // The ILP objective, summed on the device.  Entries of linked nodes share an ILP variable
 // (optimize_sharding.py:211-231) and the objective coefficient of a variable is the sum of the
@@ -3562,6 +3639,17 @@ int apc_build_tables_row_min(APC_BUILD_TABLES_PARAMS, const apc_row_minima *rows
 
 }  // extern "C"
 
+// Lanes per segment: about a tenth of the mean length, so that a lane has several
+// independent loads in flight (measured best on both benchmark tables; APC_SEGMIN_GROUP
+// overrides, for tuning).
+static int segment_lanes(int64_t n_values, int64_t n_seg) {
+  const double mean = (double)n_values / (double)n_seg;
+  int g = 2;
+  while (g < 64 && g * 12 <= mean) g *= 2;
+  if (const char *env = getenv("APC_SEGMIN_GROUP")) g = atoi(env);
+  return g;
+}
+
 static int segmented_min_impl(const double *values, const int64_t *seg_ptr, int64_t n_seg, int64_t n_values, double *mins,
                               int32_t *args, const SegmentCopies *copies, const char *who, void *stream) {
   if (n_seg < 0 || n_values < 0) return fail(-1, "negative count");
@@ -3569,13 +3657,7 @@ static int segmented_min_impl(const double *values, const int64_t *seg_ptr, int6
   if (!seg_ptr || !mins || !args || (!values && n_values > 0)) return fail(-1, "%s: NULL array", who);
   if (n_seg > (int64_t)INT32_MAX * 4) return fail(-1, "n_segments %lld too large", (long long)n_seg);
   hipStream_t s = (hipStream_t)stream;
-  // lanes per segment: about a tenth of the mean length, so that a lane has several
-  // independent loads in flight (measured best on both benchmark tables; APC_SEGMIN_GROUP
-  // overrides, for tuning)
-  const double mean = (double)n_values / (double)n_seg;
-  int g = 2;
-  while (g < 64 && g * 12 <= mean) g *= 2;
-  if (const char *env = getenv("APC_SEGMIN_GROUP")) g = atoi(env);
+  const int g = segment_lanes(n_values, n_seg);
   switch (g) {
     case 1: launch_segmented_min<1>(values, seg_ptr, n_seg, mins, args, copies, s); break;
     case 2: launch_segmented_min<2>(values, seg_ptr, n_seg, mins, args, copies, s); break;
@@ -3617,6 +3699,44 @@ int apc_strategy_bounds(int64_t n_strategies, const int32_t *strat_node, const i
                      n_strategies, strat_node, node_strat_begin, node_edge_begin, edges_by_node, edge_row_begin, row_min,
                      bound);
   return check_launch("apc_strategy_bounds");
+}
+
+int apc_greedy_strategies(int64_t n_nodes, int64_t n_strategies, const int64_t *node_strat_begin, const int64_t *node_edge_begin,
+                          const int32_t *edges_by_node, const int64_t *edge_row_begin, const double *row_min, double *bound,
+                          double *node_min, int32_t *node_argmin, void *stream) {
+  if (n_nodes < 0 || n_strategies < 0) return fail(-1, "apc_greedy_strategies: negative count");
+  if (n_nodes == 0) return 0;
+  // (edges_by_node may be NULL when no node has an edge, the arrays of strategies when there is none)
+  if (!node_strat_begin || !node_edge_begin || !node_min || !node_argmin || (n_strategies > 0 && !bound))
+    return fail(-1, "apc_greedy_strategies: NULL array");
+  if (n_nodes > (int64_t)INT32_MAX * 4) return fail(-1, "n_nodes %lld too large", (long long)n_nodes);
+  const int g = segment_lanes(n_strategies, n_nodes);
+#define APC_GREEDY(G_)                                                                                                       \
+  case G_:                                                                                                                   \
+    hipLaunchKernelGGL((greedy_strategies_kernel<G_>), dim3(blocks_for(n_nodes, kBlock / G_)), dim3(kBlock), 0,               \
+                       (hipStream_t)stream, n_nodes, node_strat_begin, node_edge_begin, edges_by_node, edge_row_begin,        \
+                       row_min, bound, node_min, node_argmin);                                                               \
+    break
+  switch (g) {
+    APC_GREEDY(1);
+    APC_GREEDY(2);
+    APC_GREEDY(4);
+    APC_GREEDY(8);
+    APC_GREEDY(16);
+    APC_GREEDY(32);
+    APC_GREEDY(64);
+    default: return fail(-1, "segment group width %d is not a power of two up to 64", g);
+  }
+#undef APC_GREEDY
+  return check_launch("apc_greedy_strategies");
+}
+
+int apc_edge_rows(int64_t n_edges, const int32_t *edge_n_tgt, int64_t *edge_row_begin, void *stream) {
+  if (n_edges < 0) return fail(-1, "apc_edge_rows: n_edges < 0");
+  if (n_edges == 0) return 0;
+  if (!edge_n_tgt || !edge_row_begin) return fail(-1, "apc_edge_rows: NULL array");
+  hipLaunchKernelGGL(edge_rows_kernel, dim3(1), dim3(kScanThreads), 0, (hipStream_t)stream, n_edges, edge_n_tgt, edge_row_begin);
+  return check_launch("apc_edge_rows");
 }
 
 int apc_cost_objective(int64_t n_vars, int64_t n_groups, const int64_t *group_var_begin, const int64_t *group_member_begin,

@@ -667,6 +667,64 @@ InputTables input_tables_of(const Tensor &params, const Tensor &rank, const Tens
       shape_width, flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag
 
 // apc_input_tables: tensor table, compute costs and (with spec_outputs) the spec table in one launch.
+Tensor edge_rows(const Tensor &edge_n_tgt) {
+  const int32_t *nt = dev<int32_t>(edge_n_tgt, at::kInt, "edge_n_tgt");
+  Tensor begin = empty_like_device(edge_n_tgt, {edge_n_tgt.numel()}, at::kLong);
+  on_current_stream(edge_n_tgt.device(), "apc_edge_rows", [&](void *s) {
+    return apc_edge_rows(edge_n_tgt.numel(), nt, static_cast<int64_t *>(begin.data_ptr()), s);
+  });
+  return begin;
+}
+
+// The tables of a report: tensor and compute-cost tables in one launch, then every per-entry array and, where edge_n_tgt is given,
+// the row minima.  -> ([tensor_bytes, tensor_contiguous, compute, per_arg, comm, transition, cost, row_min, row_argmin], whether a
+// strategy with flops has an unsupported dtype).  Waits for the first launch's flag only, which a copy behind that launch brings
+// while the second one runs.
+std::tuple<std::vector<Tensor>, bool> report_tables(
+    const Tensor &params, const Tensor &rank, const Tensor &itemsize, const Tensor &shape, const Tensor &stride,
+    const Tensor &spec_codes, const Tensor &spec_tensor, const Tensor &flops, const Tensor &rw_bytes, const Tensor &dtype,
+    const Tensor &zero_cost, const Tensor &num_args, const Tensor &pt_values, const Tensor &tiles, const Tensor &dup_entry_begin,
+    int64_t n_entries, const OptTensor &edge_n_tgt, const OptTensor &dup_row_begin, int64_t n_rows) {
+  const apc_params p = params_of(params);
+  const TensorTable t = tensor_table(rank, itemsize, shape, stride);
+  const StrategyTable st = strategy_table(flops, rw_bytes, dtype, zero_cost, num_args);
+  TORCH_CHECK(n_entries >= 0 && n_rows >= 0, "apcost: negative count");
+  same_device(rank, flops, "flops");
+  c10::hip::HIPGuard guard(rank.device().index());
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(rank.device().index()).stream();
+  Tensor bytes = empty_like_device(rank, {t.n}, at::kLong), contiguous = empty_like_device(rank, {t.n}, at::kByte);
+  Tensor compute = empty_like_device(rank, {st.n}, at::kDouble), per_arg = empty_like_device(rank, {st.n}, at::kDouble);
+  Tensor error = at::zeros({1}, rank.options().dtype(at::kInt));
+  check_rc(apc_input_tables(&p, t.n, t.rank, t.itemsize, t.shape, t.stride, dev<int64_t>(bytes, at::kLong, "tensor_bytes"),
+                            dev<uint8_t>(contiguous, at::kByte, "tensor_contiguous"), 0, nullptr, nullptr, nullptr, nullptr, nullptr, 2,
+                            nullptr, nullptr, st.n, st.flops, st.rw_bytes, st.dtype, st.zero_cost, st.num_args,
+                            dev<double>(compute, at::kDouble, "compute"), dev<double>(per_arg, at::kDouble, "per_arg"),
+                            error.data_ptr<int32_t>(), stream),
+           "apc_input_tables");
+  Staging flag((int64_t)sizeof(int32_t), stream, 2);  // (with an event)
+  check_hip(hipMemcpyAsync(flag.slot(0), error.data_ptr(), sizeof(int32_t), hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
+  check_hip(hipEventRecord(flag.events[0], stream), "hipEventRecord");
+  Tensor comm = empty_like_device(rank, {n_entries}, at::kDouble), transition = empty_like_device(rank, {n_entries}, at::kByte),
+         cost = empty_like_device(rank, {n_entries}, at::kDouble);
+  std::vector<Tensor> out{bytes, contiguous, compute, per_arg, comm, transition, cost};
+  OptTensor row_begin, dup_rows, row_min, row_argmin;
+  if (edge_n_tgt.has_value()) {
+    row_begin = edge_rows(*edge_n_tgt);
+    dup_rows = dup_row_begin;
+    row_min = empty_like_device(rank, {n_rows}, at::kDouble);
+    row_argmin = empty_like_device(rank, {n_rows}, at::kInt);
+    out.push_back(*row_min);
+    out.push_back(*row_argmin);
+  }
+  bind_redistribute_tables(params, bytes, contiguous, spec_codes, spec_tensor, pt_values, per_arg, tiles, dup_entry_begin, n_entries, comm,
+                           transition, cost, row_begin, dup_rows, row_min, row_argmin)
+      ->run();
+  check_hip(hipEventSynchronize(flag.events[0]), "hipEventSynchronize");
+  int32_t unsupported;
+  std::memcpy(&unsupported, flag.slot(0), sizeof(unsupported));
+  return {out, unsupported != 0};
+}
+
 c10::intrusive_ptr<BoundLaunch> bind_input_tables(APCOST_INPUT_TABLE_PARAMS) {
   auto b = c10::make_intrusive<BoundLaunch>();
   const InputTables in = input_tables_of(APCOST_INPUT_TABLE_ARGS, b->keep);
@@ -874,6 +932,27 @@ c10::intrusive_ptr<BoundLaunch> bind_segmented_min(const Tensor &values, const T
     b->launch = [=](void *s) { return apc_segmented_min(v, ptr, n_seg, n_values, mins, args, s); };
   }
   return b;
+}
+
+std::tuple<Tensor, Tensor, Tensor> greedy_strategies(const Tensor &node_strat_begin, const Tensor &node_edge_begin, const Tensor &edges_by_node,
+                                                     const Tensor &edge_row_begin, const Tensor &row_min, int64_t n_strategies) {
+  const int64_t *nsb = dev<int64_t>(node_strat_begin, at::kLong, "node_strat_begin"), *neb = dev<int64_t>(node_edge_begin, at::kLong, "node_edge_begin");
+  const int32_t *ebn = dev<int32_t>(edges_by_node, at::kInt, "edges_by_node");
+  const int64_t *erb = dev<int64_t>(edge_row_begin, at::kLong, "edge_row_begin");
+  const double *rm = dev<double>(row_min, at::kDouble, "row_min");
+  TORCH_CHECK(node_strat_begin.numel() >= 1 && node_strat_begin.numel() == node_edge_begin.numel(),
+              "apcost: node_strat_begin and node_edge_begin need n_nodes + 1 rows each");
+  TORCH_CHECK(edges_by_node.numel() == edge_row_begin.numel(), "apcost: edges_by_node and edge_row_begin need one row per edge");
+  TORCH_CHECK(n_strategies >= 0, "apcost: negative count");
+  for (const Tensor *t : {&node_strat_begin, &node_edge_begin, &edges_by_node, &edge_row_begin}) same_device(row_min, *t, "an index array");
+  const int64_t n = node_strat_begin.numel() - 1;
+  Tensor bound = empty_like_device(row_min, {n_strategies}, at::kDouble), node_min = empty_like_device(row_min, {n}, at::kDouble),
+         node_argmin = empty_like_device(row_min, {n}, at::kInt);
+  on_current_stream(row_min.device(), "apc_greedy_strategies", [&](void *s) {
+    return apc_greedy_strategies(n, n_strategies, nsb, neb, ebn, erb, rm, dev<double>(bound, at::kDouble, "bound"),
+                                 static_cast<double *>(node_min.data_ptr()), static_cast<int32_t *>(node_argmin.data_ptr()), s);
+  });
+  return {bound, node_min, node_argmin};
 }
 
 Tensor strategy_bounds(const Tensor &strat_node, const Tensor &node_strat_begin, const Tensor &node_edge_begin,
@@ -1097,6 +1176,14 @@ TORCH_LIBRARY(apcost, m) {
   m.def("strategy_bounds(Tensor strat_node, Tensor node_strat_begin, Tensor node_edge_begin, Tensor edges_by_node, "
         "Tensor edge_row_begin, Tensor row_min) -> Tensor",
         &strategy_bounds);
+  m.def("greedy_strategies(Tensor node_strat_begin, Tensor node_edge_begin, Tensor edges_by_node, Tensor edge_row_begin, Tensor row_min, "
+        "int n_strategies) -> (Tensor bound, Tensor node_min, Tensor node_argmin)",
+        &greedy_strategies);
+  m.def("edge_rows(Tensor edge_n_tgt) -> Tensor edge_row_begin", &edge_rows);
+  m.def("report_tables(Tensor params, " APCOST_TENSOR_TABLE ", Tensor spec_codes, Tensor spec_tensor, " APCOST_STRATEGY_TABLE
+        ", Tensor pt_values, Tensor tiles, Tensor dup_entry_begin, int n_entries, Tensor? edge_n_tgt, Tensor? dup_row_begin, int n_rows) "
+        "-> (Tensor[] tables, bool unsupported)",
+        &report_tables);
   m.def("diffusion_sweeps_(int n_sweeps, Tensor color_begin, Tensor color_nodes, Tensor label_begin, Tensor inc_begin, "
         "Tensor inc_edge, Tensor inc_side, Tensor edge_begin, Tensor edge_i, Tensor edge_j, int max_labels, int n_labels_total, int n_elements, Tensor(a!) theta, "
         "Tensor(b!) unary) -> ()",

@@ -206,7 +206,7 @@ class DeviceCostTables:
         also writes ``row_min`` / ``row_argmin`` (allocated by ``run_redistribute_tables``)."""
         rows = None
         if row_min:
-            rows = (_to_device(self.tables.edge_row_begin(), self.device), self.row_min, self.row_argmin)
+            rows = (self.ops.edge_rows(self.d["edge_n_tgt"]), self.row_min, self.row_argmin)
         self._bind_redistribute_tables(self.comm, self.transition, self.cost, rows).run()
 
     @_guarded
@@ -232,10 +232,22 @@ class DeviceCostTables:
 
     @_guarded
     def build_all(self):
-        """tensor tables -> compute costs -> cost matrices, all on the current stream."""
-        self.run_tensor_tables()
-        self.run_compute_costs()
-        return self.run_redistribute_tables()
+        """tensor tables and compute costs -> cost matrices (with the row minima when ``row_min_in_tiles_pays``), all on
+        the current stream, in two launches.  A strategy with flops and an unsupported dtype raises, as in
+        ``run_compute_costs``; the matrices are not kept then."""
+        tb, d = self.tables, self.d
+        row_min = self.row_min_in_tiles_pays()
+        if row_min:
+            tb.validate_row_minima()  # raises when some matrix row is spread over tiles
+        out, unsupported = self.ops.report_tables(
+            self.p, *self._tensor_table(), d["spec_codes"], d["spec_tensor"], *self._strategy_table(), d["pt_values"], d["tile_records"],
+            d["dup_entry_begin"], tb.n_entries, d["edge_n_tgt"] if row_min else None, d["dup_row_begin"] if row_min else None,
+            tb.n_rows if row_min else 0)
+        self.tensor_bytes, self.tensor_contiguous, self.compute_cost, self.compute_cost_per_arg = out[:4]
+        self._check_flag(int(unsupported))
+        self.comm, self.transition, self.cost = out[4:7]
+        self.row_min, self.row_argmin = out[7:] if row_min else (None, None)
+        return self.comm, self.transition, self.cost
 
     # ---- one full device-side pass with pre-bound arguments -------------------------------------
     # A pass over a table this small is bound by the ramp-up and drain of every launch, and
@@ -668,10 +680,7 @@ class DeviceCostTables:
         self._diffusion_state = (theta_out, unary_out, *out)
         return theta_out, unary_out
 
-    @_guarded
-    def strategy_bounds(self, row_min: torch.Tensor) -> torch.Tensor:
-        """Per-(node, strategy) sum of the row minima of the node's edges (``row_min`` in the
-        order of ``CostTables.row_ptr()``)."""
+    def _index_of_bounds(self, row_min):
         t = self.tables
         if row_min.dtype != torch.float64 or not row_min.is_contiguous():
             raise TypeError("strategy_bounds takes a contiguous float64 array of row minima")
@@ -680,7 +689,13 @@ class DeviceCostTables:
         if getattr(self, "_bound_index", None) is None:
             index = dict(t.strategy_bound_index(), node_strat_begin=np.ascontiguousarray(t.node_strat_begin, np.int64))
             self._bound_index = dict(zip(index, self._upload(*index.values())))
-        ix = self._bound_index
+        return self._bound_index
+
+    @_guarded
+    def strategy_bounds(self, row_min: torch.Tensor) -> torch.Tensor:
+        """Per-(node, strategy) sum of the row minima of the node's edges (``row_min`` in the
+        order of ``CostTables.row_ptr()``)."""
+        ix = self._index_of_bounds(row_min)
         return self.ops.strategy_bounds(ix["strat_node"], ix["node_strat_begin"], ix["node_edge_begin"], ix["edges_by_node"],
                                         ix["edge_row_begin"], row_min)
 
@@ -688,6 +703,6 @@ class DeviceCostTables:
     def greedy_strategies(self, row_min: torch.Tensor):
         """-> (bound per strategy, min per node, argmin per node): the cheapest strategy of every
         node when each of its edges is charged its row minimum."""
-        bound = self.strategy_bounds(row_min)
-        node_min, node_arg = self.segmented_min(bound, self._bound_index["node_strat_begin"], check=False)
-        return bound, node_min, node_arg
+        ix = self._index_of_bounds(row_min)
+        return self.ops.greedy_strategies(ix["node_strat_begin"], ix["node_edge_begin"], ix["edges_by_node"], ix["edge_row_begin"], row_min,
+                                          ix["strat_node"].numel())

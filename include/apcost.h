@@ -376,6 +376,17 @@ int apc_strategy_bounds(int64_t n_strategies, const int32_t *strat_node, const i
                         const int64_t *node_edge_begin, const int32_t *edges_by_node, const int64_t *edge_row_begin,
                         const double *row_min, double *bound, void *stream);
 
+/* apc_strategy_bounds and the segmented minimum of its result over node_strat_begin in one launch: bound[s] of every
+ * strategy, the smallest of every node and the first strategy that has it (of a node without strategies +inf, -1).  The
+ * same bits as the two.  The caller checks the index arrays. */
+int apc_greedy_strategies(int64_t n_nodes, int64_t n_strategies, const int64_t *node_strat_begin, const int64_t *node_edge_begin,
+                          const int32_t *edges_by_node, const int64_t *edge_row_begin, const double *row_min, double *bound,
+                          double *node_min, int32_t *node_argmin, void *stream);
+
+/* The first matrix row of every edge, rows numbered edge by edge (apc_row_minima::edge_row_begin): edge_row_begin[e] = the
+ * sum of edge_n_tgt[0 .. e). */
+int apc_edge_rows(int64_t n_edges, const int32_t *edge_n_tgt, int64_t *edge_row_begin, void *stream);
+
 /* The ILP objective vector, summed on the device so that only one number per variable (not
  * three arrays per entry) has to leave it.
  * Replaces the accumulation at optimize_sharding.py:650-655 (opt_target[va] += cost over
