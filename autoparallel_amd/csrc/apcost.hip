@@ -3370,11 +3370,17 @@ static int out_mode(int mesh_ndim, const double *comm_out, const uint8_t *trans_
 //   17.2 / 21.0, 2 638 values - / 21.4 / 23.8, 3 874 values - / 29.4 / 27.3, 22 values 13.9 / 15.7 / 24.5; (8, 8, 8), 22 values
 //   17.1 / 16.1 / 24.1 us; 36 157 tiles of 149 values 46.8 / 59.4 / 96.7 there, 46.7 / 56.5 / 94.9 on (16, 8, 4), 4 123 of 139
 //   on (8, 8, 8) 16.6 / 14.3 / 17.8.
+//   ... and (256, 300) from the second round of its workgroups on one wavefront takes the tiles that store less than that: us with one / two,
+//   4 694 tiles of 129 values, (16, 8, 4), 9.4 / 10.8, 10 834 of 246, (8, 8, 8), 14.8 / 16.3, 8 566 of 207 12.6 / 13.3, 10 278 of 159, (32, 8),
+//   12.3 / 13.3, 9 426 of 200, (2, 4, 2, 2), 14.5 / 15.7, 10 278 of 266, (6,), 13.5 / 14.7, 2 906 of 5, (64,), 5.5 / 6.4; the other way 6 950 of 273,
+//   (32, 8), 13.9 / 11.3, 6 335 of 287, (16, 8, 4), 12.3 / 11.7, 9 425 of 420 18.0 / 17.1.  Not with the 72 states of a 3-D mesh to
+//   stage: 6 333 of 202, (6, 4, 2), 14.0 / 13.3, 9 425 of 255 18.6 / 18.1, 8 967 of 17 13.3 / 13.1.
 //   Small tiles fill the chip sooner: from kSmallTilesInOneRound on, two for those of less than kSmallTile values (1 181 tiles of
 //   338 values, (8, 8, 8), 6.6 with two / 7.5 with four, 1 265 of 330, (12, 6), 7.0 / 8.0; the other way 880 of 480 7.9 / 7.1, 812 of
 //   490 7.5 / 6.7, 1 270 of 710 11.7 / 8.7).
 constexpr int64_t kTilesInOneRound = 1280;  // five workgroups of four wavefronts to a compute unit
 constexpr int64_t kSmallTilesInOneRound = 1024, kSmallTile = 448;
+constexpr int64_t kTilesOfTwoRounds = 2048, kTilesOfSomeRounds = 8192;
 constexpr int64_t kTilesOfManyRounds = 16384;  // (of one wavefront: 32 workgroups to a compute unit, twice)
 
 static int tile_threads(int64_t n_tiles, int64_t n_entries, bool many_states, int64_t two, int64_t four) {
@@ -3515,7 +3521,13 @@ static int build_tables_impl(const apc_params *params, int64_t n_tensors, const 
   const int xs = xcd_shift();
   const TermLayout lay = term_layout(*params);
   const bool many_states = params->mesh_ndim == 4 && lay.exponents == 0;
-  const int threads = tile_threads(n_tiles, n_entries, many_states, n_tiles > kTilesOfManyRounds ? 512 : params->mesh_ndim == 3 ? 0 : 64, 3072);
+  const int64_t two = n_tiles > kTilesOfManyRounds                       ? 512
+                      : params->mesh_ndim == 3 && lay.exponents == 0 ? 0
+                      : n_tiles > kTilesOfSomeRounds                  ? 300
+                      : n_tiles > kTilesOfTwoRounds                   ? 256
+                      : params->mesh_ndim == 3                       ? 0
+                                                                     : 64;
+  const int threads = tile_threads(n_tiles, n_entries, many_states, two, 3072);
   const int64_t tile_blocks = ((n_tiles + (1 << xs) - 1) >> xs) << xs;
   const int64_t sb = spec_table ? blocks_for(n_specs, threads) : 0, tb = blocks_for(n_tensors, threads),
                 cb = blocks_for(n_strategies, threads);
