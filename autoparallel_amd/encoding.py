@@ -91,15 +91,21 @@ ORDERED_MIN_STORED_PER_TILE, ORDERED_SOME_ROUNDS = 1000, 4000
 # tiles and up to 16 copies per tiled edge (Llama-3-8B on (32, 8), 1.8 M entries: 13.3 us with
 # 840 tiles of 16 copies against 14.6 us with 1 616 tiles of 8 and 17.7 us with 3 168 of 4).
 AUTO_SMALL_TABLE_ENTRIES = 4_000_000
-# ... unless there are many entries to compute, or rows too wide for a packed tile.  A packed tile costs a
-# record of 2.7 KB from memory and evaluates every entry directly; a staged tile evaluates the terms
-# once and looks them up, which wins when a table computes this many entries in tiles that hold this many each.
-# Whole pass, packed (tiles of four rows per wavefront) / staged: 900 989 entries on (32, 8) 23.2 / 15.5 us, on
-# (8, 8, 8) 28.4 / 14.7, on (3, 2, 2, 2) 40.6 / 24.0; 574 862 of at most 24 x 24 a matrix 18.4 / 15.5, 189 736
-# on (8, 8, 8) 9.1 / 7.1, on (32, 8) 7.8 / 7.6; the other way: 102 873 6.7 / 7.0, and 221 958 in matrices of 45
-# entries 18.3 / 21.1 (matrices of 139 entries on a 4-D mesh, whose terms cost most to stage, 31.6 / 34.1).
-STAGED_MIN_COMPUTED = 150_000
-STAGED_MIN_COMPUTED_PER_TILE = {1: 100, 2: 100, 3: 100, 4: 180}
+# ... over packed tiles, where it is all copies or next to nothing to compute.  A packed tile costs a record of 2.7 KB from
+# memory and evaluates every entry directly; a staged tile evaluates the terms once and looks them up, and where there are no copies
+# to store wins from the second round of workgroups on.  Whole pass, packed (tiles of four rows per wavefront) / staged, us:
+#   computed entries, no copies, from STAGED_MIN_COMPUTED: 366 k in 7 884 tiles on (32, 8) 16.9 / 11.4, 149 k 6.8 / 5.6, 54 k 4.9 / 4.4,
+#   409 k on (8, 8, 8) 16.0 / 10.0, 53 k 6.3 / 5.5, 836 k on (2, 4, 2, 2) 34.2 / 14.8, 337 k on (6, 4, 2) 15.8 / 12.1; about equal at
+#   46 k 4.4 / 4.4, 4 copies of 54 k 5.2 / 5.1; the other way 26 k 4.9 / 5.2, 19 k 4.0 / 4.3, 13 k 3.9 / 4.3, 2 k 3.6 / 4.2;
+#   more than STAGED_MANY_EDGES tiled edges, whatever they hold: 15 k in 2 906 on (64,) 6.3 / 5.5, 16 copies of them 9.1 / 7.8, 12 copies of
+#   50 k in 3 060 on (32, 8) 8.9 / 8.2, 8 copies of 102 k in 3 059 on (8, 8, 8) 11.2 / 9.2; about equal at 2 324, 8 copies of 58 k, 8.2 / 8.3;
+#   more than STAGED_MAX_COPIES copies: 8 of 54 k in 474 5.6 / 6.1, 16 7.0 / 8.5, 16 of 109 k on (32, 8) 8.4 / 10.3, 10 of 119 k on
+#   (8, 8, 8) 7.6 / 8.7; then staged from this many computed entries on, in tiles that hold this many each, as (measured before the staging
+#   got cheaper) 901 k on (32, 8) 23.2 / 15.5, on (8, 8, 8) 28.4 / 14.7, 575 k 18.4 / 15.5, 190 k on (8, 8, 8) 9.1 / 7.1;
+#   a 4-D mesh with a size that is no power of two, whose states cost most to stage, by the last line alone: 430 k in tiles of 91 entries
+#   25.0 / 25.7, 149 k of 94 11.3 / 11.6, 81 k of 17 15.7 / 25.2.
+STAGED_MIN_COMPUTED, STAGED_MAX_COPIES, STAGED_MANY_EDGES = 40_000, 6, 2048
+STAGED_MIN_COMPUTED_OF_COPIES, STAGED_MIN_COMPUTED_PER_TILE = 150_000, {1: 100, 2: 100, 3: 100, 4: 180}
 # Its tiles are cut until there are this many: enough workgroups for the chip, few enough stagings.  But no smaller than what
 # a STAGED_SMALLEST_SHARE-th of the entries to compute is (its power of two), at least 512: a launch is as long as its largest tile, and larger
 # tables last longer.  Tiles of about 512 / 1024 / 2048 / 4096 entries, by size:
@@ -436,18 +442,18 @@ class CostTables:
             if small:
                 n, n_dups = packed_cut = count(te, mc, 4)
                 whole_edges = n, computed()
-                M = len(self.mesh_sizes)
+                tiled_edges = int(np.count_nonzero((canonical == np.arange(self.n_edges)) & (n_src > 0) & (n_tgt > 0)))
                 fits = n == 0 or int(n_src.max()) <= APC_TILE_MAX_COLS
                 rows_per_wavefront_pass = 4
-                if n and (not fits or whole_edges[1] >= STAGED_MIN_COMPUTED):
+                if n and (not fits or self._staging_may_pay(whole_edges[1], tiled_edges)):
                     n, n_dups = count(te, mc, 0)
                     wanted, least = STAGED_TILES, max(STAGED_MIN_TILE_ENTRIES, whole_edges[1] // STAGED_SMALLEST_SHARE)
-                    if M == 4 and any(m & (m - 1) for m in self.mesh_sizes):
+                    if self._many_states():
                         wanted, least = STAGED_TILES_OF_MANY_STATES, STAGED_MIN_TILE_ENTRIES_OF_MANY_STATES
                     while n < wanted and te // 2 >= 1 << (least.bit_length() - 1):
                         te //= 2
                         n, n_dups = count(te, mc, 0)
-                    if not fits or self.staging_pays(whole_edges[1], n):
+                    if not fits or self.staging_pays(whole_edges[1], n, tiled_edges):
                         rows_per_wavefront_pass = None
                     else:
                         te, (n, n_dups) = APC_TILE_MAX_ROWS * APC_TILE_MAX_COLS, packed_cut
@@ -472,6 +478,8 @@ class CostTables:
         self.tiling = {"tile_entries": te if automatic else int(tile_entries), "max_copies": mc if dedupe else 1}
         if automatic:
             self.tiling["whole_edges"] = whole_edges
+            if small:
+                self.tiling["tiled_edges"] = tiled_edges
         if rows_per_wavefront_pass:
             self.tiling["rows_per_wavefront_pass"] = int(rows_per_wavefront_pass)
         self.edge_canonical = canonical
@@ -505,9 +513,22 @@ class CostTables:
         self.tile_records = rec
 
     # ---- packed tiles ------------------------------------------------------------------
-    def staging_pays(self, computed: int, n_tiles: int) -> bool:
-        """Whether tiles staged in LDS beat packed ones on a small table (above: STAGED_MIN_COMPUTED)."""
-        return computed >= STAGED_MIN_COMPUTED and computed >= n_tiles * STAGED_MIN_COMPUTED_PER_TILE[len(self.mesh_sizes)]
+    def _many_states(self) -> bool:
+        return len(self.mesh_sizes) == 4 and any(m & (m - 1) for m in self.mesh_sizes)
+
+    def _staging_may_pay(self, computed: int, tiled_edges: int) -> bool:
+        """``staging_pays`` of some number of tiles."""
+        return computed >= STAGED_MIN_COMPUTED_OF_COPIES or self.staging_pays(computed, computed + 1, tiled_edges)
+
+    def staging_pays(self, computed: int, n_tiles: int, tiled_edges: Optional[int] = None) -> bool:
+        """Whether tiles staged in LDS beat packed ones on a small table (above: STAGED_MIN_COMPUTED).  ``tiled_edges``: the edges
+        that have tiles, by default those of the current tiling where it was chosen from the table."""
+        if tiled_edges is None:
+            tiled_edges = (self.tiling or {}).get("tiled_edges", 0)
+        if not self._many_states():
+            if tiled_edges > STAGED_MANY_EDGES or (computed >= STAGED_MIN_COMPUTED and self.n_entries <= STAGED_MAX_COPIES * computed):
+                return True
+        return computed >= STAGED_MIN_COMPUTED_OF_COPIES and computed >= n_tiles * STAGED_MIN_COMPUTED_PER_TILE[len(self.mesh_sizes)]
 
     def largest_tiles_first_pays(self) -> bool:
         """Whether a launch takes the tiles by size instead of edge by edge (above: ORDERED_MAX_ENTRIES)."""
