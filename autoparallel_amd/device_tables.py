@@ -252,12 +252,18 @@ class DeviceCostTables:
     # ---- one full device-side pass with pre-bound arguments -------------------------------------
     # A pass over a table this small is bound by the ramp-up and drain of every launch, and
     # one launch for all tables wins; above it the tiles' own derivation of what they would otherwise
-    # read costs more than a launch.  The cost alone, one launch / two: on (32, 8) 5.5 M entries (42 MB) 29.7 / 36.0 us, 11 M
-    # (87 MB) 47.6 / 51.1, 22 M in 8 384 tiles (170 MB) 37.5 / 40.2; on (16, 8, 4) 9.4 M (72 MB) 33.7 / 34.0, 20 M (156 MB)
-    # 65.1 / 58.1.  What the derivation costs goes by tiles and not by bytes, though: tables of many small tiles lose by
-    # this limit, 5.4 M entries in 36 157 tiles 54.8 / 43.7 on (32, 8), 47.1 / 43.9 on (16, 8, 4), 5.3 M in 162 354 tiles
-    # 179 / 107.
-    ONE_LAUNCH_MAX_BYTES = 128 << 20
+    # read costs more than a launch.  The cost alone, one launch / two: on (16, 8, 4) 10.6 M entries 36.5 / 39.6 us, 20 M (163 MB) 58.8 /
+    # 59.9, 28 M 78.6 / 74.3, 42 M 125 / 120; on meshes of one or two dims, where a tile derives as much and stages less, up to
+    # ONE_LAUNCH_MAX_BYTES_FLAT: on (64, 4) 20 M 56.0 / 62.8, 42 M (334 MB) 116.6 / 119.6, on (32, 8) 20 M 64.4 / 67.7, 26 M in 40 layers
+    # 57.3 / 59.0, on (12, 6) 20 M 65.7 / 68.9; the other way 47 M in eight layers on (64, 4) 129 / 124.  What the derivation costs goes by
+    # tiles and not by bytes, though: tables of many small tiles lose by these limits, 5.4 M entries in 36 157 tiles 54.8 / 43.7 on
+    # (32, 8), 47.1 / 43.9 on (16, 8, 4), 5.3 M in 162 354 tiles 179 / 107 (measured when both took longer).
+    ONE_LAUNCH_MAX_BYTES = 192 << 20
+    ONE_LAUNCH_MAX_BYTES_FLAT = 344 << 20
+
+    def one_launch_limit(self) -> int:
+        flat = len(self.tables.mesh_sizes) <= 2
+        return max(self.ONE_LAUNCH_MAX_BYTES, self.ONE_LAUNCH_MAX_BYTES_FLAT) if flat and self.ONE_LAUNCH_MAX_BYTES else self.ONE_LAUNCH_MAX_BYTES
 
     def row_min_in_tiles_pays(self) -> bool:
         """Whether the launch that writes the cost matrices should take the row minima itself.
@@ -379,7 +385,7 @@ class DeviceCostTables:
             raise ValueError("a segmented_min launch over the rows reads the cost array: ask for it")
         total = self.pass_bytes(outputs, spec_table, row_min_in_tiles)
         if one_launch is None:
-            one_launch = bool(fused_inputs) and total <= self.ONE_LAUNCH_MAX_BYTES
+            one_launch = bool(fused_inputs) and total <= self.one_launch_limit()
         packed_kind = bool(one_launch) and row_min_in_tiles and outputs == ("cost",) and not spec_table
         if packed is None:
             packed = packed_kind and self.packed_pass_pays() and not tb.staging_pays(tb.computed_entries(), tb.n_tiles)
