@@ -96,6 +96,8 @@ class DeviceCostTables:
             # (the host's table may be tiled anew before it is uploaded again: what is on the device stays one tiling)
             self._tiles = self.d["tile_records"], arrays[names.index("tile_records")]
             self._ordered_tiles = None
+        if "edge_n_tgt" in names:
+            self._edge_rows = None
 
     # ---- helpers -------------------------------------------------------------------------
     def _upload(self, *arrays):
@@ -366,10 +368,12 @@ class DeviceCostTables:
         of its launches are not laid out in device memory first (``apc_kept_launch``: one copy, for 0.75 us less a launch over packed
         tiles or a large table, nothing where staged tiles wait for other loads at that time), nor its tiles put
         into launch order (``CostTables.launch_records``: 10 ns a tile on the host).  Those copies, one a launch
-        and one of the tiles, are waited for.  So are the uploads of row indices and packed tiles (made once); a pass that needs
-        none of them can be prepared while the current stream captures, and is then prepared as with ``repeated=False``."""
+        and one of the tiles, are waited for.  So are the uploads of row indices and packed tiles; while the current stream
+        captures, a pass is prepared as with ``repeated=False`` and takes the edges' first rows, or the packed tiles, of an earlier preparation
+        (a table that staged tiles are faster for goes over packed ones where only those are there)."""
         tb = self.tables
-        repeated = bool(repeated) and not torch.cuda.is_current_stream_capturing()
+        capturing = torch.cuda.is_current_stream_capturing()
+        repeated = bool(repeated) and not capturing
         outputs = tuple(outputs)
         if not outputs or any(o not in ("comm", "transition", "cost") for o in outputs):
             raise ValueError(f"outputs must name some of comm, transition, cost: {outputs}")
@@ -388,7 +392,8 @@ class DeviceCostTables:
             one_launch = bool(fused_inputs) and total <= self.one_launch_limit()
         packed_kind = bool(one_launch) and row_min_in_tiles and outputs == ("cost",) and not spec_table
         if packed is None:
-            packed = packed_kind and self.packed_pass_pays() and not tb.staging_pays(tb.computed_entries(), tb.n_tiles)
+            packed = packed_kind and self.packed_pass_pays() and not (
+                tb.staging_pays(tb.computed_entries(), tb.n_tiles) and (self._edge_rows is not None or not capturing))
         elif packed and not (packed_kind and self.tables.packable()):
             raise ValueError("a pass over packed tiles is one launch that writes the assembled cost and the row minima, "
                              "without the spec table, over tiles of whole rows")
@@ -423,7 +428,9 @@ class DeviceCostTables:
             self.row_min = self._empty((tb.n_rows,), torch.float64)
             self.row_argmin = self._empty((tb.n_rows,), torch.int32)
         if row_min_in_tiles and not packed:  # (packed tiles hold their rows' numbers themselves)
-            rows = (_to_device(tb.edge_row_begin(), self.device), self.row_min, self.row_argmin)
+            if self._edge_rows is None or not capturing:
+                self._edge_rows = _to_device(tb.edge_row_begin(), self.device)
+            rows = (self._edge_rows, self.row_min, self.row_argmin)
         erb, rmin, rarg = rows if rows is not None else (None, None, None)
         dup_rows = d["dup_row_begin"] if rows is not None else None
         if packed:

@@ -231,3 +231,29 @@ def test_a_pass_is_prepared_while_the_stream_captures(gpu_device, form):
         graph.replay()
         torch.cuda.synchronize()
         assert np.array_equal(d.cost.cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("before", [None, True])
+def test_the_default_pass_is_prepared_while_the_stream_captures(gpu_device, before):
+    """A small table that staged tiles are faster for, with the row minima: over staged tiles after a preparation by default,
+    over packed ones where only those were prepared before."""
+    mesh = (16, 8, 4)
+    tb = stress_dag(seed=13, n_nodes=250, mesh_sizes=mesh, max_strategies=24)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
+    assert d.packed_pass_pays() and d.row_min_in_tiles_pays() and tb.staging_pays(tb.computed_entries(), tb.n_tiles)
+    d.planner_pass(packed=before)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step = d.planner_pass()
+        for launch in step.values():
+            launch()
+    assert list(step) == ["build_tables_packed" if before else "build_tables"]
+    want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh, rescale=2.2))["cost"]
+    lowest = np.minimum.reduceat(want, tb.row_ptr()[:-1])
+    for _ in range(3):
+        for t in (d.cost, d.row_min):
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(d.cost.cpu().numpy(), want) and np.array_equal(d.row_min.cpu().numpy(), lowest)
