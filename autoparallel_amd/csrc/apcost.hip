@@ -1972,7 +1972,9 @@ void redistribute_tiles_row_min_kernel(APC_LAUNCH_PARAMS(TilesBlock, false)) {
 // 9.4 M on (16, 8, 4) 64.6 -> 59.1, 901 k on (8, 8, 8) 14.9 -> 13.8; on 1-D and 2-D meshes, where the larger layout was held, 6.1 M
 // on (64, 4) 29.5 -> 28.2, 41 k on (64,) 10.6 -> 9.6.)
 // (On 1-D and 2-D meshes seven wavefronts per SIMD are asked for, what 72 vector registers leave room for: 7.6 M entries on (32, 8),
-// 59 layers, 17.0 us with 5, 16.4 with 7, 2.6 M on (12, 6) 13.4 / 13.2, 6.1 M on (64, 4) with the minima the same.)
+// 59 layers, 17.0 us with 5, 16.4 with 7, 2.6 M on (12, 6) 13.4 / 13.2, 6.1 M on (64, 4) with the minima the same.  On 3-D meshes without
+// the minima too: the compiler then takes 94 scalar registers instead of 106, and with its 62 vector registers eight wavefronts are
+// resident instead of seven, 20 M entries on (16, 8, 4) 60.1 -> 58.6 us; with the minima it takes 67, and spills for nothing.)
 template <int M, bool RM>
 static size_t build_tables_lds_bytes(const TermLayout &lay, int threads, bool spec_table) {
   const size_t stage = stage_lds_bytes<M, RM>(lay, threads);
@@ -1990,7 +1992,7 @@ struct BuildTablesBlock {
 };
 
 template <int M, int kThreads, bool RM, int OUT, bool KEPT>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(M <= 2 ? 7 : 1, 8)))
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(M <= 2 || (M == 3 && !RM) ? 7 : 1, 8)))
 void build_tables_kernel(APC_LAUNCH_PARAMS(BuildTablesBlock, KEPT)) {
   const BuildTablesBlock &k = launch_block<KEPT>(kept);
   const apc_params &p = k.p;
