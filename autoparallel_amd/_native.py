@@ -86,6 +86,7 @@ EXPORTS = (
     "apc_strategy_bounds",
     "apc_greedy_strategies",
     "apc_edge_rows",
+    "apc_check_tables",
     "apc_cost_objective",
     "apc_validate_row_minima_host",
     "apc_diffusion_sweeps",

@@ -2573,6 +2573,106 @@ __global__ __launch_bounds__(kScanThreads) void edge_rows_kernel(int64_t n_edges
 }
 
 // ------------------------------------------------------------------------------------------
+// Whether the tables are well formed, where they are about to be read: a lane a spec and a tensor, a wavefront an edge and a tile, every
+// index checked before it is used.  Bound by the launch and by the wait for its answer: 315 k specs, 15 104 edges and 4 000 tiles with 15 000
+// copies are 8 MB of reads.  (The host takes 0.35 ms for the specs and edges, on eight threads, and as long for every 5 000 copies'
+// offsets, one after the other.)
+// ------------------------------------------------------------------------------------------
+struct CheckTablesArgs {
+  int32_t mesh_ndim;
+  int64_t n_tensors, n_specs, n_edges, n_pt, n_strategies, n_tiles, n_dups;
+  const int32_t *tensor_rank;
+  const uint32_t *spec_codes;
+  const int32_t *spec_tensor;
+  const int32_t *src_begin, *n_src, *tgt_begin, *n_tgt, *flags, *strat_begin;
+  const int64_t *pt_begin, *entry_begin;
+  const apc_tile *tiles;
+  const int64_t *dup_entry_begin;
+  int64_t tensor_blocks, spec_blocks, edge_blocks;
+  int32_t *malformed;
+};
+constexpr int kEmptyEdgesPassed = 64;  // in a row, in front of a copy's edge
+
+__device__ bool spec_holds(const CheckTablesArgs &a, int64_t s) {
+  const int t = a.spec_tensor[s];
+  if (t < -1 || t >= a.n_tensors) return false;
+  const uint32_t codes = a.spec_codes[s];
+  if (a.mesh_ndim < 4 && (codes >> (8 * a.mesh_ndim)) != 0) return false;
+  const int rank = t >= 0 ? a.tensor_rank[t] : APC_MAX_RANK + 16;  // (no DTensorSpec: a Shard of any dim passes)
+  bool holds = true;
+#pragma unroll
+  for (int i = 0; i < APC_MAX_MESH; ++i) {
+    const uint32_t c = (codes >> (8 * i)) & 0xFF;
+    holds &= kind_of(c) != 3 && (kind_of(c) != 0 || c == 0) && (kind_of(c) != 2 || dim_of(c) < rank);
+  }
+  return holds;
+}
+
+// (uniform but for the lanes' share of the specs)
+__device__ bool edge_holds(const CheckTablesArgs &a, int64_t e, int lane) {
+  const int64_t ns = a.n_src[e], nt = a.n_tgt[e], sb = a.src_begin[e], tb = a.tgt_begin[e], st = a.strat_begin[e], pt = a.pt_begin[e];
+  if (!(ns >= 0 && nt >= 0 && ns <= APC_MAX_STRATEGIES && nt <= APC_MAX_STRATEGIES && sb >= 0 && sb + ns <= a.n_specs && tb >= 0 &&
+        tb + nt <= a.n_specs && st >= 0 && st + nt <= a.n_strategies && a.entry_begin[e + 1] - a.entry_begin[e] == ns * nt))
+    return false;
+  if (pt >= 0 && pt <= a.n_pt && ns * nt <= a.n_pt - pt) return true;
+  // without pass-through values: a producer and a tensor behind every spec
+  bool needs_pt = (a.flags[e] & APC_EDGE_NO_PRODUCER) != 0;
+  for (int64_t j = lane; j < ns; j += 64) needs_pt |= a.spec_tensor[sb + j] < 0;
+  for (int64_t j = lane; j < nt; j += 64) needs_pt |= a.spec_tensor[tb + j] < 0;
+  return !needs_pt;
+}
+
+// (uniform but for a copy's offset a lane)
+__device__ bool tile_holds(const CheckTablesArgs &a, int64_t t, int lane) {
+  const apc_tile &tl = a.tiles[t];
+  const int e = tl.edge, rows = tl.counts & 0xFFFF, cols = tl.counts >> 16;
+  if (e < 0 || e >= a.n_edges) return false;
+  const int ns = a.n_src[e], nt = a.n_tgt[e];
+  if (rows < 1 || rows > APC_TILE_MAX_ROWS || tl.row_begin < 0 || (int64_t)tl.row_begin + rows > nt) return false;
+  if (cols < 1 || cols > APC_TILE_MAX_COLS || tl.col_begin < 0 || (int64_t)tl.col_begin + cols > ns) return false;
+  const int64_t sp = (int64_t)tl.src_begin + tl.col_begin;
+  if (tl.src_begin != a.src_begin[e] || tl.n_src != ns || tl.tgt_begin != a.tgt_begin[e] || tl.flags != a.flags[e] ||
+      tl.strat_begin != a.strat_begin[e] || tl.entry_begin != a.entry_begin[e] || tl.pt_begin != a.pt_begin[e])
+    return false;
+  if (sp < 0 || sp >= a.n_specs || tl.tensor != a.spec_tensor[sp]) return false;
+  if (tl.dup_count < 0 || tl.dup_count > APC_TILE_MAX_DUPS || tl.dup_begin < 0 || (int64_t)tl.dup_begin + tl.dup_count > a.n_dups) return false;
+  if (lane >= tl.dup_count) return true;
+  // the start of another edge with a matrix of the same shape
+  const int64_t offset = a.dup_entry_begin[tl.dup_begin + lane];
+  int64_t lo = 0, hi = a.n_edges;  // the first edge that begins there, then past the edges without entries
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) / 2;
+    if (a.entry_begin[mid] < offset) lo = mid + 1;
+    else hi = mid;
+  }
+  for (int passed = 0; lo < a.n_edges && (a.n_src[lo] == 0 || a.n_tgt[lo] == 0); ++lo)
+    if (++passed > kEmptyEdgesPassed) return false;
+  return lo < a.n_edges && a.entry_begin[lo] == offset && lo != e && a.n_src[lo] == ns && a.n_tgt[lo] == nt;
+}
+
+__global__ __launch_bounds__(kBlock) void check_tables_kernel(CheckTablesArgs a) {
+  int64_t b = blockIdx.x;
+  const int64_t row = threadIdx.x, item = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  bool holds = true;
+  if (b < a.tensor_blocks) {
+    const int64_t t = b * kBlock + row;
+    if (t < a.n_tensors) holds = a.tensor_rank[t] >= 0 && a.tensor_rank[t] <= APC_MAX_RANK;
+    if (t == 0) holds &= a.entry_begin[0] == 0;
+  } else if ((b -= a.tensor_blocks) < a.spec_blocks) {
+    const int64_t s = b * kBlock + row;
+    if (s < a.n_specs) holds = spec_holds(a, s);
+  } else if ((b -= a.spec_blocks) < a.edge_blocks) {
+    const int64_t e = b * (kBlock / 64) + item;
+    if (e < a.n_edges) holds = edge_holds(a, e, lane);
+  } else {
+    const int64_t t = (b - a.edge_blocks) * (kBlock / 64) + item;
+    if (t < a.n_tiles) holds = tile_holds(a, t, lane);
+  }
+  if (__ballot(!holds) != 0 && lane == 0) *a.malformed = 1;
+}
+
+// ------------------------------------------------------------------------------------------
 // The ILP objective, summed on the device.  Entries of linked nodes share an ILP variable
 // (optimize_sharding.py:211-231) and the objective coefficient of a variable is the sum of the
 // costs of its entries, added one by one in entry order starting from 0
@@ -3751,6 +3851,40 @@ int apc_edge_rows(int64_t n_edges, const int32_t *edge_n_tgt, int64_t *edge_row_
   if (!edge_n_tgt || !edge_row_begin) return fail(-1, "apc_edge_rows: NULL array");
   hipLaunchKernelGGL(edge_rows_kernel, dim3(1), dim3(kScanThreads), 0, (hipStream_t)stream, n_edges, edge_n_tgt, edge_row_begin);
   return check_launch("apc_edge_rows");
+}
+
+int apc_check_tables(const apc_params *params, int32_t with_rows, int64_t n_tensors, const int32_t *tensor_rank, int64_t n_specs,
+                     const uint32_t *spec_codes, const int32_t *spec_tensor, int64_t n_edges, const int32_t *edge_src_begin,
+                     const int32_t *edge_n_src, const int32_t *edge_tgt_begin, const int32_t *edge_n_tgt, const int32_t *edge_flags,
+                     const int64_t *edge_pt_begin, const int64_t *edge_entry_begin, const int32_t *edge_strat_begin, int64_t n_pt,
+                     int64_t n_strategies, int64_t n_tiles, const apc_tile *tiles, int64_t n_dups, const int64_t *dup_entry_begin,
+                     int32_t *malformed, void *stream) {
+  if (int rc = check_params(params)) return rc;
+  if (n_tensors < 0 || n_specs < 0 || n_edges < 0 || n_pt < 0 || n_strategies < 0 || n_tiles < 0 || n_dups < 0)
+    return fail(-1, "apc_check_tables: negative count");
+  if (!malformed || !edge_entry_begin || (n_tensors > 0 && !tensor_rank) || (n_specs > 0 && (!spec_codes || !spec_tensor)) ||
+      (n_edges > 0 && (!edge_src_begin || !edge_n_src || !edge_tgt_begin || !edge_n_tgt || !edge_flags || !edge_pt_begin || !edge_strat_begin)) ||
+      (n_tiles > 0 && !tiles) || (n_dups > 0 && !dup_entry_begin))
+    return fail(-1, "apc_check_tables: NULL array");
+  CheckTablesArgs a{};
+  a.mesh_ndim = params->mesh_ndim;
+  a.n_tensors = n_tensors, a.n_specs = n_specs, a.n_edges = n_edges, a.n_pt = n_pt, a.n_strategies = n_strategies;
+  a.n_tiles = n_tiles, a.n_dups = n_dups;
+  a.tensor_rank = tensor_rank, a.spec_codes = spec_codes, a.spec_tensor = spec_tensor;
+  a.src_begin = edge_src_begin, a.n_src = edge_n_src, a.tgt_begin = edge_tgt_begin, a.n_tgt = edge_n_tgt, a.flags = edge_flags;
+  a.strat_begin = edge_strat_begin, a.pt_begin = edge_pt_begin, a.entry_begin = edge_entry_begin;
+  a.tiles = tiles, a.dup_entry_begin = dup_entry_begin, a.malformed = malformed;
+  constexpr int64_t kItems = kBlock / 64;
+  if (with_rows) {
+    a.tensor_blocks = std::max<int64_t>(1, (n_tensors + kBlock - 1) / kBlock);  // (one for the first entry at least)
+    a.spec_blocks = (n_specs + kBlock - 1) / kBlock;
+    a.edge_blocks = (n_edges + kItems - 1) / kItems;
+  }
+  const int64_t blocks = a.tensor_blocks + a.spec_blocks + a.edge_blocks + (n_tiles + kItems - 1) / kItems;
+  if (blocks == 0) return 0;
+  if (blocks > INT32_MAX) return fail(-1, "apc_check_tables: too many workgroups");
+  hipLaunchKernelGGL(check_tables_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, (hipStream_t)stream, a);
+  return check_launch("apc_check_tables");
 }
 
 int apc_cost_objective(int64_t n_vars, int64_t n_groups, const int64_t *group_var_begin, const int64_t *group_member_begin,

@@ -676,6 +676,46 @@ Tensor edge_rows(const Tensor &edge_n_tgt) {
   return begin;
 }
 
+// Whether the tables (with_rows) and the tile records, uploaded, are well formed, as far as the device checks them (apc_check_tables).  Waits
+// for the answer.
+bool tables_hold(const Tensor &params, bool with_rows, const Tensor &tensor_rank, const Tensor &spec_codes, const Tensor &spec_tensor,
+                 const Tensor &edge_src_begin, const Tensor &edge_n_src, const Tensor &edge_tgt_begin, const Tensor &edge_n_tgt,
+                 const Tensor &edge_flags, const Tensor &edge_pt_begin, const Tensor &edge_entry_begin, const Tensor &edge_strat_begin,
+                 int64_t n_pt, int64_t n_strategies, const Tensor &tiles, const Tensor &dup_entry_begin) {
+  const apc_params p = params_of(params);
+  const int64_t n_edges = edge_src_begin.numel();
+  for (const Tensor *t : {&edge_n_src, &edge_tgt_begin, &edge_n_tgt, &edge_flags, &edge_pt_begin, &edge_strat_begin})
+    TORCH_CHECK(t->numel() == n_edges, "apcost: the edge arrays must have one row per edge (", n_edges, ")");
+  TORCH_CHECK(edge_entry_begin.numel() == n_edges + 1, "apcost: edge_entry_begin needs n_edges + 1 rows");
+  TORCH_CHECK(spec_tensor.numel() == spec_codes.numel(), "apcost: spec_tensor and spec_codes differ in length");
+  constexpr int64_t kWords = sizeof(apc_tile) / 4;
+  TORCH_CHECK(tiles.numel() % kWords == 0, "apcost: tiles must be [n_tiles, ", kWords, "] int32 words (struct apc_tile)");
+  for (const Tensor *t : {&tensor_rank, &spec_codes, &spec_tensor, &edge_src_begin, &edge_n_src, &edge_tgt_begin, &edge_n_tgt, &edge_flags,
+                          &edge_pt_begin, &edge_strat_begin, &tiles, &dup_entry_begin})
+    same_device(edge_entry_begin, *t, "a table");
+  c10::hip::HIPGuard guard(edge_entry_begin.device().index());
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(edge_entry_begin.device().index()).stream();
+  Tensor malformed = at::zeros({1}, edge_entry_begin.options().dtype(at::kInt));
+  check_rc(apc_check_tables(
+               &p, with_rows ? 1 : 0, tensor_rank.numel(), dev<int32_t>(tensor_rank, at::kInt, "tensor_rank"), spec_codes.numel(),
+               reinterpret_cast<const uint32_t *>(dev<int32_t>(spec_codes, at::kInt, "spec_codes")),
+               dev<int32_t>(spec_tensor, at::kInt, "spec_tensor"), n_edges, dev<int32_t>(edge_src_begin, at::kInt, "edge_src_begin"),
+               dev<int32_t>(edge_n_src, at::kInt, "edge_n_src"), dev<int32_t>(edge_tgt_begin, at::kInt, "edge_tgt_begin"),
+               dev<int32_t>(edge_n_tgt, at::kInt, "edge_n_tgt"), dev<int32_t>(edge_flags, at::kInt, "edge_flags"),
+               dev<int64_t>(edge_pt_begin, at::kLong, "edge_pt_begin"), dev<int64_t>(edge_entry_begin, at::kLong, "edge_entry_begin"),
+               dev<int32_t>(edge_strat_begin, at::kInt, "edge_strat_begin"), n_pt, n_strategies, tiles.numel() / kWords,
+               reinterpret_cast<const apc_tile *>(dev<int32_t>(tiles, at::kInt, "tiles")), dup_entry_begin.numel(),
+               dev<int64_t>(dup_entry_begin, at::kLong, "dup_entry_begin"), malformed.data_ptr<int32_t>(), stream),
+           "apc_check_tables");
+  Staging answer((int64_t)sizeof(int32_t), stream, 2);  // (with an event)
+  check_hip(hipMemcpyAsync(answer.slot(0), malformed.data_ptr(), sizeof(int32_t), hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
+  check_hip(hipEventRecord(answer.events[0], stream), "hipEventRecord");
+  check_hip(hipEventSynchronize(answer.events[0]), "hipEventSynchronize");
+  int32_t word;
+  std::memcpy(&word, answer.slot(0), sizeof(word));
+  return word == 0;
+}
+
 // The tables of a report: tensor and compute-cost tables in one launch, then every per-entry array and, where edge_n_tgt is given,
 // the row minima.  -> ([tensor_bytes, tensor_contiguous, compute, per_arg, comm, transition, cost, row_min, row_argmin], whether a
 // strategy with flops has an unsupported dtype).  Waits for the first launch's flag only, which a copy behind that launch brings
@@ -1180,6 +1220,10 @@ TORCH_LIBRARY(apcost, m) {
         "int n_strategies) -> (Tensor bound, Tensor node_min, Tensor node_argmin)",
         &greedy_strategies);
   m.def("edge_rows(Tensor edge_n_tgt) -> Tensor edge_row_begin", &edge_rows);
+  m.def("tables_hold(Tensor params, bool with_rows, Tensor tensor_rank, Tensor spec_codes, Tensor spec_tensor, Tensor edge_src_begin, "
+        "Tensor edge_n_src, Tensor edge_tgt_begin, Tensor edge_n_tgt, Tensor edge_flags, Tensor edge_pt_begin, Tensor edge_entry_begin, "
+        "Tensor edge_strat_begin, int n_pt, int n_strategies, Tensor tiles, Tensor dup_entry_begin) -> bool",
+        &tables_hold);
   m.def("report_tables(Tensor params, " APCOST_TENSOR_TABLE ", Tensor spec_codes, Tensor spec_tensor, " APCOST_STRATEGY_TABLE
         ", Tensor pt_values, Tensor tiles, Tensor dup_entry_begin, int n_entries, Tensor? edge_n_tgt, Tensor? dup_row_begin, int n_rows) "
         "-> (Tensor[] tables, bool unsupported)",

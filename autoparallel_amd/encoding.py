@@ -597,6 +597,11 @@ class CostTables:
     def validate(self, params) -> None:
         """Structural check through the library's host-side validator; raises
         RuntimeError naming the first malformed row."""
+        self._validate(params, None)
+
+    def _validate(self, params, on_device) -> None:
+        """``on_device``: called where lengths and types are right; -> what needs no check of the host's any more, ``"tiles"``
+        (with the copies' offsets), ``"tables"`` (those and every row) or nothing."""
         if tuple(params.mesh_sizes) != self.mesh_sizes:
             raise RuntimeError(f"tables were encoded for mesh {self.mesh_sizes}, params describe {params.mesh_sizes}")
         if len(self.edge_entry_begin) != self.n_edges + 1:
@@ -620,12 +625,15 @@ class CostTables:
             self.n_edges, "edge_src_begin", "edge_tgt_begin", "edge_flags", "edge_pt_begin", "edge_strat_begin", "edge_canonical",
             "edge_dup_count")
         (dup_entry_begin,) = self._rows(0, "dup_entry_begin")
-        _native.host_call(
-            "apc_validate_tables_host", params.to_c(), self.n_tensors, rank, self.n_specs, codes, spec_tensor, self.n_edges,
-            src_begin, n_src, tgt_begin, n_tgt, flags, pt_begin, *self._rows(self.n_edges + 1, "edge_entry_begin"), strat_begin,
-            len(self.pt_values), self.n_strategies, self.n_tiles, self._records(self.tile_records, self.n_tiles, TILE_DTYPE),
-            len(dup_entry_begin), dup_entry_begin)
-        # what the device cannot check: every edge is tiled completely or a duplicate of an edge that is; flop and
+        (entry_begin,) = self._rows(self.n_edges + 1, "edge_entry_begin")
+        records = self._records(self.tile_records, self.n_tiles, TILE_DTYPE)
+        held = on_device() if on_device is not None else None
+        if held != "tables":
+            _native.host_call(
+                "apc_validate_tables_host", params.to_c(), self.n_tensors, rank, self.n_specs, codes, spec_tensor, self.n_edges,
+                src_begin, n_src, tgt_begin, n_tgt, flags, pt_begin, entry_begin, strat_begin,
+                len(self.pt_values), self.n_strategies, 0 if held == "tiles" else self.n_tiles, records, len(dup_entry_begin), dup_entry_begin)
+        # what the kernels cannot check: every edge is tiled completely or a duplicate of an edge that is; flop and
         # byte counts convert to fp64 exactly (the kernels divide them as doubles)
         _native.host_call(
             "apc_validate_tiling_host", self.n_tensors, rank, itemsize, shape, self.n_strategies, flops, rw_bytes, num_args,

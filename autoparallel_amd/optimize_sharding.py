@@ -110,11 +110,14 @@ class DeviceBackend:
     def upload_strategy_inputs(self, tables, tile_entries=None, dedupe=True, max_copies=16):
         """The strategy table is final: tile the edges (identical edges once) and send both."""
         tables.build_tiles(tile_entries, dedupe=dedupe, max_copies=max_copies, repeated=False)
-        tables.validate(self.dev.params)
         names = ("tile_records", "dup_entry_begin", "dup_row_begin")
         if not getattr(self, "_strategy_inputs_on_device", False):
             names = ("strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost") + names
-        self.dev.refresh(*names)
+        if tables is self.dev.tables:
+            self.dev.refresh_tiling(*names)
+        else:
+            tables.validate(self.dev.params)
+            self.dev.refresh(*names)
 
     @on_device_thread
     def launch_tables(self):

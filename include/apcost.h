@@ -383,6 +383,18 @@ int apc_greedy_strategies(int64_t n_nodes, int64_t n_strategies, const int64_t *
                           const int32_t *edges_by_node, const int64_t *edge_row_begin, const double *row_min, double *bound,
                           double *node_min, int32_t *node_argmin, void *stream);
 
+/* What apc_validate_tables_host checks, of tables that are on the device: *malformed (on the device, cleared by the caller) is
+ * set to 1 unless every row is well formed.  It may be set too for rows the host's check takes (a copy's offset behind a long run
+ * of edges without entries): which row it is, and whether it is one, that check says.  with_rows = 0: the tile records and the
+ * copies' offsets alone.  Every array has the length its count says, checked by the caller; beyond that nothing is
+ * assumed of the values. */
+int apc_check_tables(const apc_params *params, int32_t with_rows, int64_t n_tensors, const int32_t *tensor_rank, int64_t n_specs,
+                     const uint32_t *spec_codes, const int32_t *spec_tensor, int64_t n_edges, const int32_t *edge_src_begin,
+                     const int32_t *edge_n_src, const int32_t *edge_tgt_begin, const int32_t *edge_n_tgt, const int32_t *edge_flags,
+                     const int64_t *edge_pt_begin, const int64_t *edge_entry_begin, const int32_t *edge_strat_begin, int64_t n_pt,
+                     int64_t n_strategies, int64_t n_tiles, const apc_tile *tiles, int64_t n_dups, const int64_t *dup_entry_begin,
+                     int32_t *malformed, void *stream);
+
 /* The first matrix row of every edge, rows numbered edge by edge (apc_row_minima::edge_row_begin): edge_row_begin[e] = the
  * sum of edge_n_tgt[0 .. e). */
 int apc_edge_rows(int64_t n_edges, const int32_t *edge_n_tgt, int64_t *edge_row_begin, void *stream);

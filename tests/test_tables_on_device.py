@@ -1,0 +1,114 @@
+"""The structural check of tables that are on the device (``apc_check_tables``) against the host's (``apc_validate_tables_host``).
+Every index is checked before it is used, on either side."""
+import numpy as np
+import pytest
+
+from autoparallel_amd import CostModelParams
+from autoparallel_amd.device_tables import DeviceCostTables
+from autoparallel_amd.optimize_sharding import DeviceBackend
+from autoparallel_amd.synthetic import stress_dag
+
+from test_abi_and_encoding import twin_graph
+
+MESHES = [(8,), (12, 6), (4, 2, 2), (2, 2, 2, 2)]
+
+
+@pytest.fixture(autouse=True)
+def always_on_device(monkeypatch):
+    monkeypatch.setattr(DeviceCostTables, "CHECK_ON_DEVICE_MIN_ROWS", 0)
+
+
+def _tables(mesh, seed=8):
+    tb = twin_graph(stress_dag(seed=seed, n_nodes=60, mesh_sizes=mesh, max_strategies=10))
+    tb.build_tiles(256, dedupe=True)
+    return tb
+
+
+def _refused(f):
+    try:
+        f()
+    except RuntimeError as e:
+        return str(e)
+    return None
+
+
+def _set(name, row, value):
+    def mutate(t):
+        a = getattr(t, name)
+        a[row % len(a)] = value(t, a[row % len(a)]) if callable(value) else value
+    return mutate
+
+
+def _set_record(field, row, change):
+    def mutate(t):
+        t.tile_records[field][row % t.n_tiles] += change
+    return mutate
+
+
+MUTATIONS = (
+    [_set("tensor_rank", 0, 9), _set("tensor_rank", 1, -1), _set("spec_tensor", 3, 10**6), _set("spec_tensor", 5, -2), _set("spec_tensor", 7, -1),
+     _set("edge_entry_begin", 0, 1), _set("edge_entry_begin", 2, lambda t, v: v + 1), _set("edge_entry_begin", -1, 0)]
+    + [_set("spec_codes", k, c) for k, c in enumerate((0xC0, 0x01, 0x8F, 0x80, 0x82, 0x40, 0x8000, 0x800000, 0xC0000000, 0x80000000, 0))]
+    + [_set(n, e, lambda t, v, d=d: v + d) for n in ("edge_src_begin", "edge_tgt_begin", "edge_strat_begin", "edge_n_src", "edge_n_tgt")
+       for e, d in ((1, 1), (4, -1), (6, 10**6), (2, -10**6))]
+    + [_set("edge_pt_begin", e, v) for e in range(0, 60, 7) for v in (-1, 10**9, 0)]
+    + [_set("edge_flags", e, lambda t, v: v ^ 1) for e in (0, 5, 9)]
+    + [_set_record(f, t, d) for f in ("edge", "row_begin", "col_begin", "counts", "src_begin", "n_src", "tgt_begin", "flags", "strat_begin",
+                                      "tensor", "entry_begin", "pt_begin", "dup_begin", "dup_count") for t, d in ((0, 1), (5, -1), (-1, 10**6))]
+    + [_set("dup_entry_begin", k, lambda t, v, d=d: v + d) for k in (0, 3, -1) for d in (1, -10**7, 10**7)]
+    + [_set("dup_entry_begin", 0, lambda t, v: t.tile_records["entry_begin"][t.tile_records["dup_count"] > 0][0])]
+)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mesh", MESHES)
+def test_the_device_refuses_what_the_host_refuses(gpu_device, mesh):
+    params = CostModelParams.from_mesh(mesh)
+    sound = _tables(mesh)
+    d = DeviceCostTables(sound, params, device=gpu_device)
+    assert d._refresh_and_check(("tile_records",), "tables") == "tables" and d._refresh_and_check((), "tiles") == "tiles"
+    refused = 0
+    for k, mutate in enumerate(MUTATIONS):
+        tb = _tables(mesh)
+        mutate(tb)
+        want = _refused(lambda: tb.validate(params))
+        d.tables = tb
+        held = d._refresh_and_check([n for n in d.d if n not in ("strat_flops",)], "tables")
+        rows_hold = _refused(lambda: tb._validate(params, lambda: "tiles")) is None
+        # (what only the host checks, the tiling, is checked either way)
+        structure = _refused(lambda: tb._validate(params, lambda: "tables"))
+        assert (held == "tables") == (want is None or want == structure), (k, want)
+        if rows_hold:  # the records alone, of tables whose rows hold
+            assert (d._refresh_and_check((), "tiles") == "tiles") == (held == "tables"), (k, want)
+        got = _refused(lambda: DeviceCostTables(tb, params, device=gpu_device))
+        assert got == want, k
+        refused += want is not None
+    assert refused > len(MUTATIONS) // 2
+
+
+@pytest.mark.gpu
+def test_a_tiling_that_is_refused_leaves_the_old_one_on_the_device(gpu_device):
+    mesh = (4, 2, 2)
+    tb = _tables(mesh)
+    backend = DeviceBackend(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
+    before = dict(backend.dev.d)
+    tb.build_tiles = lambda *a, **k: tb.dup_entry_begin.__setitem__(0, 1)
+    with pytest.raises(RuntimeError, match="duplicate offset"):
+        backend.upload_strategy_inputs(tb)
+    assert all(backend.dev.d[k] is before[k] for k in before)
+
+
+@pytest.mark.gpu
+def test_long_runs_of_edges_without_entries_are_left_to_the_host(gpu_device):
+    """A copy whose edge lies behind more edges without entries than a lane passes over: the host finds it sound."""
+    mesh, n = (4, 2), 70
+    tb = _tables(mesh)
+    at = int(np.nonzero((tb.edge_entry_begin[:-1] == tb.dup_entry_begin[-1]) & (tb.edge_n_src > 0))[0][0])
+    for name in ("edge_node", "edge_arg", "edge_src_begin", "edge_n_src", "edge_tgt_begin", "edge_n_tgt", "edge_flags", "edge_pt_begin",
+                 "edge_entry_begin", "edge_strat_begin"):
+        a = getattr(tb, name)
+        setattr(tb, name, np.insert(a, at, np.full(n, 0 if name == "edge_n_src" else a[at], a.dtype)))
+    tb.build_tiles(256, dedupe=True)
+    assert tb.edge_entry_begin[at + n] in tb.dup_entry_begin
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
+    assert d._refresh_and_check((), "tiles") is None
