@@ -113,7 +113,7 @@ class DeviceBackend:
         names = ("tile_records", "dup_entry_begin", "dup_row_begin")
         if not getattr(self, "_strategy_inputs_on_device", False):
             names = ("strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost") + names
-        if tables is self.dev.tables:
+        if getattr(self.dev, "tables", None) is tables:
             self.dev.refresh_tiling(*names)
         else:
             tables.validate(self.dev.params)
