@@ -87,6 +87,7 @@ EXPORTS = (
     "apc_greedy_strategies",
     "apc_edge_rows",
     "apc_check_tables",
+    "apc_edge_classes",
     "apc_cost_objective",
     "apc_validate_row_minima_host",
     "apc_diffusion_sweeps",

@@ -2673,6 +2673,111 @@ __global__ __launch_bounds__(kBlock) void check_tables_kernel(CheckTablesArgs a)
 }
 
 // ------------------------------------------------------------------------------------------
+// Identical edges of tables on the device (apc_edge_classes): a wavefront an edge hashes what its matrix depends on and enters the hash
+// into a table, whose slot keeps the smallest edge; then it compares itself with that edge.  Two launches, bound by latency: 15 104 edges with
+// 326 k specs, 54 us with the workspaces cleared and the wait for the result.  (The host hashes, enters and compares in 0.7 ms on eight threads.)
+// ------------------------------------------------------------------------------------------
+struct EdgeClassArgs {
+  int64_t n_specs, n_strategies, n_edges, n_pt, n_slots;
+  const uint32_t *spec_codes;
+  const int32_t *spec_tensor;
+  const int64_t *flops, *rw_bytes;
+  const int8_t *dtype;
+  const uint8_t *zero_cost;
+  const int32_t *num_args;
+  const int32_t *src_begin, *n_src, *tgt_begin, *n_tgt, *flags, *strat_begin;
+  const int64_t *pt_begin;
+  const double *pt_values;
+  unsigned long long *keys;
+  int32_t *first, *slots;
+  int64_t *first_same;
+};
+
+// The multiply-and-fold step of the host's hash (Hash128), with its constants.
+__device__ __forceinline__ uint64_t fold(uint64_t x, uint64_t y) { return (x * y) ^ __umul64hi(x, y); }
+// One value of an edge at its place: a sum over all of them does not depend on the order they are added in.
+__device__ __forceinline__ uint64_t hash_of(uint64_t value, int64_t place, int array) {
+  return fold(value ^ 0x0CC4A61194F81761ull, ((uint64_t)place * 16 + (uint64_t)array) * 0x5815A7BE0543C11Dull + 0x261DC1F2B8A998C9ull);
+}
+
+struct EdgeRanges {
+  int64_t ns, nt, sb, tb, st, pt;
+  bool inside;
+};
+__device__ __forceinline__ EdgeRanges ranges_of(const EdgeClassArgs &a, int64_t e) {
+  EdgeRanges r{a.n_src[e], a.n_tgt[e], a.src_begin[e], a.tgt_begin[e], a.strat_begin[e], a.pt_begin[e], true};
+  r.inside = r.ns >= 0 && r.nt >= 0 && r.sb >= 0 && r.tb >= 0 && r.st >= 0 && r.sb + r.ns <= a.n_specs && r.tb + r.nt <= a.n_specs &&
+             r.st + r.nt <= a.n_strategies && (r.pt < 0 || (r.ns * r.nt <= a.n_pt && r.pt <= a.n_pt - r.ns * r.nt));
+  return r;
+}
+
+__global__ __launch_bounds__(kBlock) void edge_hashes_kernel(EdgeClassArgs a) {
+  const int64_t e = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (e >= a.n_edges) return;
+  const EdgeRanges r = ranges_of(a, e);
+  if (!r.inside) {  // (uniform)
+    if (lane == 0) a.slots[e] = -1;
+    return;
+  }
+  uint64_t sum = 0;
+  for (int64_t j = lane; j < r.ns; j += 64) {
+    sum += hash_of(a.spec_codes[r.sb + j], j, 0);
+    sum += hash_of((uint32_t)a.spec_tensor[r.sb + j], j, 1);
+  }
+  for (int64_t j = lane; j < r.nt; j += 64) {
+    sum += hash_of(((uint64_t)a.spec_codes[r.tb + j] << 32) | (uint32_t)a.spec_tensor[r.tb + j], j, 2);
+    sum += hash_of((uint64_t)a.flops[r.st + j], j, 3);
+    sum += hash_of((uint64_t)a.rw_bytes[r.st + j], j, 4);
+    sum += hash_of(((uint64_t)(uint32_t)a.num_args[r.st + j] << 16) | ((uint64_t)(uint8_t)a.dtype[r.st + j] << 8) | a.zero_cost[r.st + j], j, 5);
+  }
+  if (r.pt >= 0)
+    for (int64_t j = lane; j < r.ns * r.nt; j += 64) sum += hash_of((uint64_t)__double_as_longlong(a.pt_values[r.pt + j]), j, 6);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += (uint64_t)__shfl_xor((unsigned long long)sum, off, 64);
+  if (lane != 0) return;
+  sum += hash_of(((uint64_t)r.ns << 32) | (uint64_t)r.nt, (uint32_t)a.flags[e], r.pt >= 0 ? 7 : 8);
+  unsigned long long key = fold(sum, 0x70B7ED67FC9B5C43ull);
+  if (key == 0) key = 1;  // (0: an empty slot)
+  int64_t at = (int64_t)(key & (unsigned long long)(a.n_slots - 1)), slot = -1;
+  for (int64_t probe = 0; probe < a.n_slots; ++probe, at = (at + 1) & (a.n_slots - 1)) {  // (half of them stay empty)
+    const unsigned long long there = atomicCAS(a.keys + at, 0ull, key);
+    if (there != 0ull && there != key) continue;
+    atomicMin(a.first + at, (int)e);
+    slot = at;
+    break;
+  }
+  a.slots[e] = (int32_t)slot;
+}
+
+__global__ __launch_bounds__(kBlock) void edge_classes_kernel(EdgeClassArgs a) {
+  const int64_t e = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (e >= a.n_edges) return;
+  const int slot = a.slots[e];
+  const int64_t f = slot < 0 ? e : a.first[slot];
+  bool same = f >= 0 && f < e;
+  if (same) {  // (uniform)
+    const EdgeRanges x = ranges_of(a, f), y = ranges_of(a, e);
+    same = x.ns == y.ns && x.nt == y.nt && a.flags[f] == a.flags[e] && (x.pt >= 0) == (y.pt >= 0) && x.inside && y.inside;
+    if (same) {
+      for (int64_t j = lane; j < x.ns; j += 64)
+        same &= a.spec_codes[x.sb + j] == a.spec_codes[y.sb + j] && a.spec_tensor[x.sb + j] == a.spec_tensor[y.sb + j];
+      for (int64_t j = lane; j < x.nt; j += 64)
+        same &= a.spec_codes[x.tb + j] == a.spec_codes[y.tb + j] && a.spec_tensor[x.tb + j] == a.spec_tensor[y.tb + j] &&
+                a.flops[x.st + j] == a.flops[y.st + j] && a.rw_bytes[x.st + j] == a.rw_bytes[y.st + j] &&
+                a.num_args[x.st + j] == a.num_args[y.st + j] && a.dtype[x.st + j] == a.dtype[y.st + j] &&
+                a.zero_cost[x.st + j] == a.zero_cost[y.st + j];
+      if (x.pt >= 0)
+        for (int64_t j = lane; j < x.ns * x.nt; j += 64)
+          same &= __double_as_longlong(a.pt_values[x.pt + j]) == __double_as_longlong(a.pt_values[y.pt + j]);
+    }
+  }
+  same = __ballot(!same) == 0;
+  if (lane == 0) a.first_same[e] = same ? f : e;
+}
+
+// ------------------------------------------------------------------------------------------
 // The ILP objective, summed on the device.  Entries of linked nodes share an ILP variable
 // (optimize_sharding.py:211-231) and the objective coefficient of a variable is the sum of the
 // costs of its entries, added one by one in entry order starting from 0
@@ -3885,6 +3990,34 @@ int apc_check_tables(const apc_params *params, int32_t with_rows, int64_t n_tens
   if (blocks > INT32_MAX) return fail(-1, "apc_check_tables: too many workgroups");
   hipLaunchKernelGGL(check_tables_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, (hipStream_t)stream, a);
   return check_launch("apc_check_tables");
+}
+
+int apc_edge_classes(int64_t n_specs, const uint32_t *spec_codes, const int32_t *spec_tensor, int64_t n_strategies, const int64_t *flops,
+                     const int64_t *rw_bytes, const int8_t *dtype_code, const uint8_t *zero_cost, const int32_t *num_args, int64_t n_edges,
+                     const int32_t *edge_src_begin, const int32_t *edge_n_src, const int32_t *edge_tgt_begin, const int32_t *edge_n_tgt,
+                     const int32_t *edge_flags, const int64_t *edge_pt_begin, const int32_t *edge_strat_begin, int64_t n_pt,
+                     const double *pt_values, int64_t n_slots, uint64_t *keys, int32_t *first, int32_t *slots, int64_t *first_same,
+                     void *stream) {
+  if (n_specs < 0 || n_strategies < 0 || n_edges < 0 || n_pt < 0) return fail(-1, "apc_edge_classes: negative count");
+  if (n_edges == 0) return 0;
+  if (n_edges > INT32_MAX / 4 || n_slots < 2 * n_edges || n_slots > INT32_MAX || (n_slots & (n_slots - 1)) != 0)
+    return fail(-1, "apc_edge_classes: %lld slots for %lld edges: a power of two, at least twice as many", (long long)n_slots, (long long)n_edges);
+  if (!edge_src_begin || !edge_n_src || !edge_tgt_begin || !edge_n_tgt || !edge_flags || !edge_pt_begin || !edge_strat_begin || !keys ||
+      !first || !slots || !first_same || (n_specs > 0 && (!spec_codes || !spec_tensor)) || (n_pt > 0 && !pt_values) ||
+      (n_strategies > 0 && (!flops || !rw_bytes || !dtype_code || !zero_cost || !num_args)))
+    return fail(-1, "apc_edge_classes: NULL array");
+  EdgeClassArgs a{};
+  a.n_specs = n_specs, a.n_strategies = n_strategies, a.n_edges = n_edges, a.n_pt = n_pt, a.n_slots = n_slots;
+  a.spec_codes = spec_codes, a.spec_tensor = spec_tensor, a.flops = flops, a.rw_bytes = rw_bytes, a.dtype = dtype_code;
+  a.zero_cost = zero_cost, a.num_args = num_args;
+  a.src_begin = edge_src_begin, a.n_src = edge_n_src, a.tgt_begin = edge_tgt_begin, a.n_tgt = edge_n_tgt, a.flags = edge_flags;
+  a.strat_begin = edge_strat_begin, a.pt_begin = edge_pt_begin, a.pt_values = pt_values;
+  a.keys = reinterpret_cast<unsigned long long *>(keys), a.first = first, a.slots = slots, a.first_same = first_same;
+  const dim3 grid((unsigned)((n_edges + kBlock / 64 - 1) / (kBlock / 64)));
+  hipLaunchKernelGGL(edge_hashes_kernel, grid, dim3(kBlock), 0, (hipStream_t)stream, a);
+  if (int rc = check_launch("apc_edge_classes")) return rc;
+  hipLaunchKernelGGL(edge_classes_kernel, grid, dim3(kBlock), 0, (hipStream_t)stream, a);
+  return check_launch("apc_edge_classes");
 }
 
 int apc_cost_objective(int64_t n_vars, int64_t n_groups, const int64_t *group_var_begin, const int64_t *group_member_begin,

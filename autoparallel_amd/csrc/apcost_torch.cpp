@@ -716,6 +716,40 @@ bool tables_hold(const Tensor &params, bool with_rows, const Tensor &tensor_rank
   return word == 0;
 }
 
+// For every edge the first one whose matrix depends on the same bytes (apc_edge_classes).
+Tensor edge_classes(const Tensor &spec_codes, const Tensor &spec_tensor, const Tensor &flops, const Tensor &rw_bytes, const Tensor &dtype,
+                    const Tensor &zero_cost, const Tensor &num_args, const Tensor &edge_src_begin, const Tensor &edge_n_src,
+                    const Tensor &edge_tgt_begin, const Tensor &edge_n_tgt, const Tensor &edge_flags, const Tensor &edge_pt_begin,
+                    const Tensor &edge_strat_begin, const Tensor &pt_values) {
+  const StrategyTable st = strategy_table(flops, rw_bytes, dtype, zero_cost, num_args);
+  const int64_t n_edges = edge_src_begin.numel();
+  for (const Tensor *t : {&edge_n_src, &edge_tgt_begin, &edge_n_tgt, &edge_flags, &edge_pt_begin, &edge_strat_begin})
+    TORCH_CHECK(t->numel() == n_edges, "apcost: the edge arrays must have one row per edge (", n_edges, ")");
+  TORCH_CHECK(spec_tensor.numel() == spec_codes.numel(), "apcost: spec_tensor and spec_codes differ in length");
+  for (const Tensor *t : {&spec_codes, &spec_tensor, &flops, &edge_n_src, &edge_tgt_begin, &edge_n_tgt, &edge_flags, &edge_pt_begin, &edge_strat_begin,
+                          &pt_values})
+    same_device(edge_src_begin, *t, "a table");
+  TORCH_CHECK(n_edges <= INT32_MAX / 4, "apcost: too many edges (", n_edges, ")");
+  int64_t n_slots = 16;
+  while (n_slots < 2 * n_edges) n_slots *= 2;
+  c10::hip::HIPGuard guard(edge_src_begin.device().index());
+  Tensor keys = at::zeros({n_slots}, edge_src_begin.options().dtype(at::kLong));
+  Tensor first = at::full({n_slots}, 0x7F7F7F7F, edge_src_begin.options());
+  Tensor slots = empty_like_device(edge_src_begin, {n_edges}, at::kInt), out = empty_like_device(edge_src_begin, {n_edges}, at::kLong);
+  on_current_stream(edge_src_begin.device(), "apc_edge_classes", [&](void *s) {
+    return apc_edge_classes(
+        spec_codes.numel(), reinterpret_cast<const uint32_t *>(dev<int32_t>(spec_codes, at::kInt, "spec_codes")),
+        dev<int32_t>(spec_tensor, at::kInt, "spec_tensor"), st.n, st.flops, st.rw_bytes, st.dtype, st.zero_cost, st.num_args, n_edges,
+        dev<int32_t>(edge_src_begin, at::kInt, "edge_src_begin"), dev<int32_t>(edge_n_src, at::kInt, "edge_n_src"),
+        dev<int32_t>(edge_tgt_begin, at::kInt, "edge_tgt_begin"), dev<int32_t>(edge_n_tgt, at::kInt, "edge_n_tgt"),
+        dev<int32_t>(edge_flags, at::kInt, "edge_flags"), dev<int64_t>(edge_pt_begin, at::kLong, "edge_pt_begin"),
+        dev<int32_t>(edge_strat_begin, at::kInt, "edge_strat_begin"), pt_values.numel(), dev<double>(pt_values, at::kDouble, "pt_values"), n_slots,
+        reinterpret_cast<uint64_t *>(keys.data_ptr()), first.data_ptr<int32_t>(), n_edges ? slots.data_ptr<int32_t>() : nullptr,
+        n_edges ? static_cast<int64_t *>(out.data_ptr()) : nullptr, s);
+  });
+  return out;
+}
+
 // The tables of a report: tensor and compute-cost tables in one launch, then every per-entry array and, where edge_n_tgt is given,
 // the row minima.  -> ([tensor_bytes, tensor_contiguous, compute, per_arg, comm, transition, cost, row_min, row_argmin], whether a
 // strategy with flops has an unsupported dtype).  Waits for the first launch's flag only, which a copy behind that launch brings
@@ -1220,6 +1254,10 @@ TORCH_LIBRARY(apcost, m) {
         "int n_strategies) -> (Tensor bound, Tensor node_min, Tensor node_argmin)",
         &greedy_strategies);
   m.def("edge_rows(Tensor edge_n_tgt) -> Tensor edge_row_begin", &edge_rows);
+  m.def("edge_classes(Tensor spec_codes, Tensor spec_tensor, " APCOST_STRATEGY_TABLE ", Tensor edge_src_begin, Tensor edge_n_src, "
+        "Tensor edge_tgt_begin, Tensor edge_n_tgt, Tensor edge_flags, Tensor edge_pt_begin, Tensor edge_strat_begin, Tensor pt_values) "
+        "-> Tensor first_same",
+        &edge_classes);
   m.def("tables_hold(Tensor params, bool with_rows, Tensor tensor_rank, Tensor spec_codes, Tensor spec_tensor, Tensor edge_src_begin, "
         "Tensor edge_n_src, Tensor edge_tgt_begin, Tensor edge_n_tgt, Tensor edge_flags, Tensor edge_pt_begin, Tensor edge_entry_begin, "
         "Tensor edge_strat_begin, int n_pt, int n_strategies, Tensor tiles, Tensor dup_entry_begin) -> bool",

@@ -130,6 +130,14 @@ class DeviceCostTables:
         return what if hold else None
 
     @_guarded
+    def edge_classes(self):
+        """``CostTables.edge_classes`` of what is on the device (host array)."""
+        d = self.d
+        return self.ops.download([self.ops.edge_classes(
+            d["spec_codes"], d["spec_tensor"], *self._strategy_table(), d["edge_src_begin"], d["edge_n_src"], d["edge_tgt_begin"],
+            d["edge_n_tgt"], d["edge_flags"], d["edge_pt_begin"], d["edge_strat_begin"], d["pt_values"])])[0].numpy()
+
+    @_guarded
     def refresh_tiling(self, *names):
         """``CostTables.validate``, and a re-upload of ``names``, the tiling among them, of tables whose other rows are on the device
         as the constructor found them; where the check raises, the device keeps what it had."""

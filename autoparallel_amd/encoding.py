@@ -418,6 +418,11 @@ class CostTables:
         (as of ``edge_signatures``); without, edges are compared by content.  ``repeated=False``: tile sizes for launches that
         go edge by edge (a pass that runs once, a report); the default ones are for a repeated pass, which takes the tiles of
         some tables by size (``largest_tiles_first_pays``)."""
+        self._build_tiles(self.edge_classes, tile_entries, dedupe, max_copies, signatures, rows_per_wavefront_pass, repeated)
+
+    def _build_tiles(self, edge_classes, tile_entries, dedupe, max_copies=16, signatures=None, rows_per_wavefront_pass=None,
+                     repeated=True) -> None:
+        """``edge_classes``: what finds the identical edges."""
         classes = None
         if dedupe and self.n_edges and signatures is not None and tile_entries is not None:
             first: dict = {}
@@ -425,7 +430,7 @@ class CostTables:
             for e, signature in enumerate(signatures):
                 classes[e] = first.setdefault(signature, e)
         elif dedupe and self.n_edges:
-            classes = self.edge_classes()
+            classes = edge_classes()
         canonical = np.empty(self.n_edges, np.int64)
         n_src, n_tgt = self._matrix_sizes()
 

@@ -109,11 +109,15 @@ class DeviceBackend:
 
     def upload_strategy_inputs(self, tables, tile_entries=None, dedupe=True, max_copies=16):
         """The strategy table is final: tile the edges (identical edges once) and send both."""
-        tables.build_tiles(tile_entries, dedupe=dedupe, max_copies=max_copies, repeated=False)
         names = ("tile_records", "dup_entry_begin", "dup_row_begin")
-        if not getattr(self, "_strategy_inputs_on_device", False):
+        own, on_device = getattr(self.dev, "tables", None) is tables, getattr(self, "_strategy_inputs_on_device", False)
+        if own and on_device and self.dev._check_on_device_pays():  # (all that an edge's identity depends on is there)
+            tables._build_tiles(self.dev.edge_classes, tile_entries, dedupe, max_copies, repeated=False)
+        else:
+            tables.build_tiles(tile_entries, dedupe=dedupe, max_copies=max_copies, repeated=False)
+        if not on_device:
             names = ("strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost") + names
-        if getattr(self.dev, "tables", None) is tables:
+        if own:
             self.dev.refresh_tiling(*names)
         else:
             tables.validate(self.dev.params)

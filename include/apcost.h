@@ -395,6 +395,17 @@ int apc_check_tables(const apc_params *params, int32_t with_rows, int64_t n_tens
                      int64_t n_strategies, int64_t n_tiles, const apc_tile *tiles, int64_t n_dups, const int64_t *dup_entry_begin,
                      int32_t *malformed, void *stream);
 
+/* apc_edge_classes_host of tables that are on the device: first_same[e] = the first edge whose matrix depends on the same bytes
+ * as that of edge e.  Edges meet through a hash of what they depend on and are then compared; two that only share the hash stand
+ * for themselves.  Workspaces of the caller's: keys [n_slots], cleared, and first [n_slots], every byte 0x7F, n_slots a power of two >=
+ * 2 n_edges; slots [n_edges].  Every array has the length its count says; an edge whose ranges leave the tables stands for itself. */
+int apc_edge_classes(int64_t n_specs, const uint32_t *spec_codes, const int32_t *spec_tensor, int64_t n_strategies, const int64_t *flops,
+                     const int64_t *rw_bytes, const int8_t *dtype_code, const uint8_t *zero_cost, const int32_t *num_args, int64_t n_edges,
+                     const int32_t *edge_src_begin, const int32_t *edge_n_src, const int32_t *edge_tgt_begin, const int32_t *edge_n_tgt,
+                     const int32_t *edge_flags, const int64_t *edge_pt_begin, const int32_t *edge_strat_begin, int64_t n_pt,
+                     const double *pt_values, int64_t n_slots, uint64_t *keys, int32_t *first, int32_t *slots, int64_t *first_same,
+                     void *stream);
+
 /* The first matrix row of every edge, rows numbered edge by edge (apc_row_minima::edge_row_begin): edge_row_begin[e] = the
  * sum of edge_n_tgt[0 .. e). */
 int apc_edge_rows(int64_t n_edges, const int32_t *edge_n_tgt, int64_t *edge_row_begin, void *stream);

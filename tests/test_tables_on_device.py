@@ -3,8 +3,8 @@ Every index is checked before it is used, on either side."""
 import numpy as np
 import pytest
 
-from autoparallel_amd import CostModelParams
-from autoparallel_amd.device_tables import DeviceCostTables
+from autoparallel_amd import CostModelParams, _native
+from autoparallel_amd.device_tables import _UPLOAD, DeviceCostTables
 from autoparallel_amd.optimize_sharding import DeviceBackend
 from autoparallel_amd.synthetic import stress_dag
 
@@ -112,3 +112,40 @@ def test_long_runs_of_edges_without_entries_are_left_to_the_host(gpu_device):
     assert tb.edge_entry_begin[at + n] in tb.dup_entry_begin
     d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
     assert d._refresh_and_check((), "tiles") is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mesh", MESHES)
+@pytest.mark.parametrize("max_strategies", [1, 10, 90])  # (lists shorter and longer than a wavefront)
+def test_identical_edges_are_the_same_on_the_device(gpu_device, mesh, max_strategies):
+    """Twins of every edge, some of them then changed in one value each of what a matrix depends on."""
+    tb = twin_graph(stress_dag(seed=21, n_nodes=80, mesh_sizes=mesh, min_strategies=1, max_strategies=max_strategies))
+    rng = np.random.default_rng(max_strategies)
+    for name in ("strat_flops", "strat_rw_bytes", "strat_dtype", "strat_num_args", "spec_codes"):
+        a = getattr(tb, name)
+        a[rng.integers(len(a) // 2, len(a), 3)] += 1
+    zero = tb.strat_zero_cost[-1:]
+    zero[:] = 1 - zero
+    if len(tb.pt_values):
+        tb.pt_values[-1] = np.nan  # (compared by its bits, as -0.0)
+        tb.pt_values[0], tb.pt_values[len(tb.pt_values) // 2] = 0.0, -0.0
+    tb.edge_flags[-3] ^= 2
+    tb.edge_src_begin[-1] = tb.n_specs  # (outside the tables: stands for itself)
+    d = object.__new__(DeviceCostTables)
+    d.ops, d.tables, d.device, d.d = _native.torch_ops(), tb, gpu_device, {}
+    d._refresh(_UPLOAD)
+    got = d.edge_classes()
+    assert np.array_equal(got, tb.edge_classes())
+    assert 0 < np.count_nonzero(got != np.arange(tb.n_edges)) < tb.n_edges // 2
+
+
+@pytest.mark.gpu
+def test_the_planner_tiles_by_the_classes_of_the_device(gpu_device):
+    mesh = (4, 2, 2)
+    tb = _tables(mesh)
+    tb.build_tiles(None, dedupe=True, repeated=False)
+    want = tb.tile_records.copy()
+    backend = DeviceBackend(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
+    backend._strategy_inputs_on_device = True
+    backend.upload_strategy_inputs(tb)
+    assert np.array_equal(tb.tile_records, want) and np.array_equal(backend.dev.d["tile_records"].cpu().numpy().view(np.uint8).ravel(), want.view(np.uint8))
