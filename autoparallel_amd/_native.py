@@ -88,6 +88,7 @@ EXPORTS = (
     "apc_edge_rows",
     "apc_check_tables",
     "apc_edge_classes",
+    "apc_pack_tiles",
     "apc_cost_objective",
     "apc_validate_row_minima_host",
     "apc_diffusion_sweeps",

@@ -2675,7 +2675,8 @@ __global__ __launch_bounds__(kBlock) void check_tables_kernel(CheckTablesArgs a)
 // ------------------------------------------------------------------------------------------
 // Identical edges of tables on the device (apc_edge_classes): a wavefront an edge hashes what its matrix depends on and enters the hash
 // into a table, whose slot keeps the smallest edge; then it compares itself with that edge.  Two launches, bound by latency: 15 104 edges with
-// 326 k specs, 54 us with the workspaces cleared and the wait for the result.  (The host hashes, enters and compares in 0.7 ms on eight threads.)
+// 326 k specs, 54 us with the workspaces cleared and the wait for the result, 0.2 ms with the host's strategy table sent in front.  (The host
+// hashes, enters and compares in 0.7 ms on eight threads.)
 // ------------------------------------------------------------------------------------------
 struct EdgeClassArgs {
   int64_t n_specs, n_strategies, n_edges, n_pt, n_slots;
@@ -2775,6 +2776,94 @@ __global__ __launch_bounds__(kBlock) void edge_classes_kernel(EdgeClassArgs a) {
   }
   same = __ballot(!same) == 0;
   if (lane == 0) a.first_same[e] = same ? f : e;
+}
+
+// ------------------------------------------------------------------------------------------
+// Packed records out of tables on the device: a wavefront a tile, lane j producer spec j, consumer spec j and its strategy.  1 138 tiles
+// are 3.1 MB: 50 us with the rows of the edges in front and the wait for the answer, 0.2 ms with the host's strategy table sent.  (The host
+// copies them together in 0.28 ms and sends them in 0.3.)
+// ------------------------------------------------------------------------------------------
+struct PackArgs {
+  TensorTableArgs t;
+  int64_t n_specs, n_strategies, n_edges, n_tiles, n_dups;
+  const uint32_t *spec_codes;
+  const int32_t *spec_tensor;
+  const int64_t *flops, *rw_bytes;
+  const int8_t *dtype;
+  const uint8_t *zero_cost;
+  const int32_t *num_args;
+  const int64_t *edge_row_begin;
+  const apc_tile *tiles;
+  const int64_t *dup_entry_begin, *dup_row_begin;
+  apc_packed_tile *packed;
+  int32_t *refused;
+};
+
+__global__ __launch_bounds__(kBlock) void pack_tiles_kernel(PackArgs a) {
+  static_assert(APC_TILE_MAX_COLS == 64 && APC_TILE_MAX_ROWS == 64 && APC_PACKED_MAX_DUPS <= 64 && APC_MAX_RANK <= 64, "a lane each");
+  const int64_t id = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (id >= a.n_tiles) return;
+  const apc_tile tl = a.tiles[id];
+  const int rows = tl.counts & 0xFFFF, cols = tl.counts >> 16, rb = tl.row_begin, n_dups = tl.dup_count;
+  const int64_t first = (int64_t)rb * cols, sb = tl.src_begin, tb = (int64_t)tl.tgt_begin + rb, st = (int64_t)tl.strat_begin + rb;
+  bool holds = tl.edge >= 0 && tl.edge < a.n_edges && rows >= 1 && rows <= APC_TILE_MAX_ROWS && cols >= 1 && cols <= APC_TILE_MAX_COLS &&
+               tl.col_begin == 0 && cols == tl.n_src && rb >= 0 && sb >= 0 && sb + cols <= a.n_specs && tb >= 0 && tb + rows <= a.n_specs &&
+               st >= 0 && st + rows <= a.n_strategies && tl.tensor < a.t.n && n_dups >= 0 && n_dups <= APC_PACKED_MAX_DUPS &&
+               tl.dup_begin >= 0 && (int64_t)tl.dup_begin + n_dups <= a.n_dups;
+  const bool col = holds && lane < cols, row = holds && lane < rows;
+  uint32_t col_codes = 0, row_codes = 0;
+  int32_t col_tensor = 0, row_tensor = 0, meta = 0;
+  int64_t flops = 0, rw_bytes = 0;
+  if (col) {
+    col_codes = a.spec_codes[sb + lane];
+    col_tensor = a.spec_tensor[sb + lane];
+  }
+  if (row) {
+    row_codes = a.spec_codes[tb + lane];
+    row_tensor = a.spec_tensor[tb + lane];
+    flops = a.flops[st + lane];
+    rw_bytes = a.rw_bytes[st + lane];
+    const int num_args = a.num_args[st + lane];
+    holds = num_args >= 1 && num_args <= 0x7FFF;
+    meta = (int32_t)((uint32_t)(uint8_t)a.dtype[st + lane] | (a.zero_cost[st + lane] != 0 ? 1u << 8 : 0u) | ((uint32_t)num_args << 16));
+  }
+  if (__ballot(!holds) != 0) {
+    if (lane == 0) *a.refused = 1;
+    return;
+  }
+  const bool mixed = __ballot((col && (col_tensor < 0 || col_tensor != tl.tensor)) || (row && row_tensor < 0)) != 0;
+  apc_packed_tile &pk = a.packed[id];
+  pk.col_codes[lane] = col_codes;
+  pk.col_tensor[lane] = col_tensor;
+  pk.row_codes[lane] = row_codes;
+  pk.row_tensor[lane] = row_tensor;
+  pk.row_flops[lane] = flops;
+  pk.row_rw_bytes[lane] = rw_bytes;
+  pk.row_meta[lane] = meta;
+  if (lane < APC_MAX_RANK) {
+    const int64_t at = (int64_t)tl.tensor * APC_MAX_RANK + lane;
+    pk.tensor_shape[lane] = tl.tensor >= 0 ? a.t.shape[at] : 0;
+    pk.tensor_stride[lane] = tl.tensor >= 0 ? a.t.stride[at] : 0;
+  }
+  if (lane < APC_PACKED_MAX_DUPS) {
+    pk.dup_entry_begin[lane] = lane < n_dups ? a.dup_entry_begin[tl.dup_begin + lane] + first : 0;
+    pk.dup_row_begin[lane] = lane < n_dups ? a.dup_row_begin[tl.dup_begin + lane] + rb : 0;
+  }
+  if (lane == 0) {
+    pk.rows = rows;
+    pk.cols = cols;
+    pk.flags = tl.flags | (mixed ? APC_PACKED_MIXED : 0);
+    pk.dup_count = n_dups;
+    pk.tensor = tl.tensor;
+    pk.tensor_rank = tl.tensor >= 0 ? a.t.rank[tl.tensor] : 0;
+    pk.tensor_itemsize = tl.tensor >= 0 ? a.t.itemsize[tl.tensor] : 0;
+    pk.edge = tl.edge;
+    pk.entry_begin = tl.entry_begin + first;
+    pk.row_begin = a.edge_row_begin[tl.edge] + rb;
+    pk.pt_begin = tl.pt_begin < 0 ? -1 : tl.pt_begin + first;
+    pk.reserved = 0;
+  }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -4018,6 +4107,31 @@ int apc_edge_classes(int64_t n_specs, const uint32_t *spec_codes, const int32_t 
   if (int rc = check_launch("apc_edge_classes")) return rc;
   hipLaunchKernelGGL(edge_classes_kernel, grid, dim3(kBlock), 0, (hipStream_t)stream, a);
   return check_launch("apc_edge_classes");
+}
+
+int apc_pack_tiles(int64_t n_tensors, const int32_t *tensor_rank, const int32_t *tensor_itemsize, const int64_t *tensor_shape,
+                   const int64_t *tensor_stride, int64_t n_specs, const uint32_t *spec_codes, const int32_t *spec_tensor,
+                   int64_t n_strategies, const int64_t *flops, const int64_t *rw_bytes, const int8_t *dtype_code,
+                   const uint8_t *zero_cost, const int32_t *num_args, int64_t n_edges, const int64_t *edge_row_begin, int64_t n_tiles,
+                   const apc_tile *tiles, int64_t n_dups, const int64_t *dup_entry_begin, const int64_t *dup_row_begin,
+                   apc_packed_tile *packed, int32_t *refused, void *stream) {
+  if (n_tensors < 0 || n_specs < 0 || n_strategies < 0 || n_edges < 0 || n_tiles < 0 || n_dups < 0)
+    return fail(-1, "apc_pack_tiles: negative count");
+  if (n_tiles == 0) return 0;
+  if (!tiles || !packed || !refused || !spec_codes || !spec_tensor || !edge_row_begin || !flops || !rw_bytes || !dtype_code || !zero_cost ||
+      !num_args || (n_dups > 0 && (!dup_entry_begin || !dup_row_begin)) ||
+      (n_tensors > 0 && (!tensor_rank || !tensor_itemsize || !tensor_shape || !tensor_stride)))
+    return fail(-1, "apc_pack_tiles: NULL array");
+  const int64_t blocks = (n_tiles + kBlock / 64 - 1) / (kBlock / 64);
+  if (blocks > INT32_MAX) return fail(-1, "apc_pack_tiles: too many workgroups");
+  PackArgs a{};
+  a.t.n = n_tensors, a.t.rank = tensor_rank, a.t.itemsize = tensor_itemsize, a.t.shape = tensor_shape, a.t.stride = tensor_stride;
+  a.n_specs = n_specs, a.n_strategies = n_strategies, a.n_edges = n_edges, a.n_tiles = n_tiles, a.n_dups = n_dups;
+  a.spec_codes = spec_codes, a.spec_tensor = spec_tensor, a.flops = flops, a.rw_bytes = rw_bytes, a.dtype = dtype_code;
+  a.zero_cost = zero_cost, a.num_args = num_args, a.edge_row_begin = edge_row_begin, a.tiles = tiles;
+  a.dup_entry_begin = dup_entry_begin, a.dup_row_begin = dup_row_begin, a.packed = packed, a.refused = refused;
+  hipLaunchKernelGGL(pack_tiles_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, (hipStream_t)stream, a);
+  return check_launch("apc_pack_tiles");
 }
 
 int apc_cost_objective(int64_t n_vars, int64_t n_groups, const int64_t *group_var_begin, const int64_t *group_member_begin,

@@ -676,6 +676,17 @@ Tensor edge_rows(const Tensor &edge_n_tgt) {
   return begin;
 }
 
+// The value of a word on the device, once `stream` has got there.
+int32_t word_on_host(const Tensor &word, hipStream_t stream) {
+  Staging answer((int64_t)sizeof(int32_t), stream, 2);  // (with an event)
+  check_hip(hipMemcpyAsync(answer.slot(0), word.data_ptr(), sizeof(int32_t), hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
+  check_hip(hipEventRecord(answer.events[0], stream), "hipEventRecord");
+  check_hip(hipEventSynchronize(answer.events[0]), "hipEventSynchronize");
+  int32_t value;
+  std::memcpy(&value, answer.slot(0), sizeof(value));
+  return value;
+}
+
 // Whether the tables (with_rows) and the tile records, uploaded, are well formed, as far as the device checks them (apc_check_tables).  Waits
 // for the answer.
 bool tables_hold(const Tensor &params, bool with_rows, const Tensor &tensor_rank, const Tensor &spec_codes, const Tensor &spec_tensor,
@@ -707,13 +718,35 @@ bool tables_hold(const Tensor &params, bool with_rows, const Tensor &tensor_rank
                reinterpret_cast<const apc_tile *>(dev<int32_t>(tiles, at::kInt, "tiles")), dup_entry_begin.numel(),
                dev<int64_t>(dup_entry_begin, at::kLong, "dup_entry_begin"), malformed.data_ptr<int32_t>(), stream),
            "apc_check_tables");
-  Staging answer((int64_t)sizeof(int32_t), stream, 2);  // (with an event)
-  check_hip(hipMemcpyAsync(answer.slot(0), malformed.data_ptr(), sizeof(int32_t), hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
-  check_hip(hipEventRecord(answer.events[0], stream), "hipEventRecord");
-  check_hip(hipEventSynchronize(answer.events[0]), "hipEventSynchronize");
-  int32_t word;
-  std::memcpy(&word, answer.slot(0), sizeof(word));
-  return word == 0;
+  return !word_on_host(malformed, stream);
+}
+
+// One packed record per tile of the uploaded tables (apc_pack_tiles); -> (records, whether all tiles could be packed).  Waits for the answer.
+std::tuple<Tensor, bool> pack_tiles(const Tensor &rank, const Tensor &itemsize, const Tensor &shape, const Tensor &stride, const Tensor &spec_codes,
+                                    const Tensor &spec_tensor, const Tensor &flops, const Tensor &rw_bytes, const Tensor &dtype,
+                                    const Tensor &zero_cost, const Tensor &num_args, const Tensor &edge_n_tgt, const Tensor &tiles,
+                                    const Tensor &dup_entry_begin, const Tensor &dup_row_begin) {
+  const TensorTable t = tensor_table(rank, itemsize, shape, stride);
+  const StrategyTable st = strategy_table(flops, rw_bytes, dtype, zero_cost, num_args);
+  TORCH_CHECK(spec_tensor.numel() == spec_codes.numel(), "apcost: spec_tensor and spec_codes differ in length");
+  TORCH_CHECK(dup_row_begin.numel() == dup_entry_begin.numel(), "apcost: dup_row_begin and dup_entry_begin differ in length");
+  constexpr int64_t kWords = sizeof(apc_tile) / 4, kPackedWords = sizeof(apc_packed_tile) / 4;
+  TORCH_CHECK(tiles.numel() % kWords == 0, "apcost: tiles must be [n_tiles, ", kWords, "] int32 words (struct apc_tile)");
+  for (const Tensor *other : {&spec_codes, &spec_tensor, &flops, &edge_n_tgt, &tiles, &dup_entry_begin, &dup_row_begin}) same_device(rank, *other, "a table");
+  c10::hip::HIPGuard guard(rank.device().index());
+  const hipStream_t stream = c10::hip::getCurrentHIPStream(rank.device().index()).stream();
+  const int64_t n_tiles = tiles.numel() / kWords;
+  Tensor packed = empty_like_device(rank, {n_tiles, kPackedWords}, at::kInt), refused = at::zeros({1}, rank.options().dtype(at::kInt));
+  const Tensor row_begin = edge_rows(edge_n_tgt);
+  check_rc(apc_pack_tiles(t.n, t.rank, t.itemsize, t.shape, t.stride, spec_codes.numel(),
+                          reinterpret_cast<const uint32_t *>(dev<int32_t>(spec_codes, at::kInt, "spec_codes")),
+                          dev<int32_t>(spec_tensor, at::kInt, "spec_tensor"), st.n, st.flops, st.rw_bytes, st.dtype, st.zero_cost, st.num_args,
+                          edge_n_tgt.numel(), dev<int64_t>(row_begin, at::kLong, "edge_row_begin"), n_tiles,
+                          reinterpret_cast<const apc_tile *>(dev<int32_t>(tiles, at::kInt, "tiles")), dup_entry_begin.numel(),
+                          dev<int64_t>(dup_entry_begin, at::kLong, "dup_entry_begin"), dev<int64_t>(dup_row_begin, at::kLong, "dup_row_begin"),
+                          n_tiles ? reinterpret_cast<apc_packed_tile *>(packed.data_ptr()) : nullptr, refused.data_ptr<int32_t>(), stream),
+           "apc_pack_tiles");
+  return {packed, word_on_host(refused, stream) == 0};
 }
 
 // For every edge the first one whose matrix depends on the same bytes (apc_edge_classes).
@@ -1258,6 +1291,9 @@ TORCH_LIBRARY(apcost, m) {
         "Tensor edge_tgt_begin, Tensor edge_n_tgt, Tensor edge_flags, Tensor edge_pt_begin, Tensor edge_strat_begin, Tensor pt_values) "
         "-> Tensor first_same",
         &edge_classes);
+  m.def("pack_tiles(" APCOST_TENSOR_TABLE ", Tensor spec_codes, Tensor spec_tensor, " APCOST_STRATEGY_TABLE
+        ", Tensor edge_n_tgt, Tensor tiles, Tensor dup_entry_begin, Tensor dup_row_begin) -> (Tensor packed, bool all_packed)",
+        &pack_tiles);
   m.def("tables_hold(Tensor params, bool with_rows, Tensor tensor_rank, Tensor spec_codes, Tensor spec_tensor, Tensor edge_src_begin, "
         "Tensor edge_n_src, Tensor edge_tgt_begin, Tensor edge_n_tgt, Tensor edge_flags, Tensor edge_pt_begin, Tensor edge_entry_begin, "
         "Tensor edge_strat_begin, int n_pt, int n_strategies, Tensor tiles, Tensor dup_entry_begin) -> bool",

@@ -38,6 +38,10 @@ _CHECKED = (
 )
 
 
+_PACKED_FROM = {"spec_codes": torch.int32, "spec_tensor": torch.int32, "edge_n_tgt": torch.int32, "dup_entry_begin": torch.int64,
+                "dup_row_begin": torch.int64}
+
+
 def _as_tensor(a: np.ndarray) -> torch.Tensor:
     """The array as a CPU tensor over the same memory."""
     if a.dtype == np.uint32:  # same bits; torch's uint32 support is partial
@@ -131,10 +135,10 @@ class DeviceCostTables:
 
     @_guarded
     def edge_classes(self):
-        """``CostTables.edge_classes`` of what is on the device (host array)."""
+        """``CostTables.edge_classes`` (host array), of the spec and edge tables on the device and the host's strategy table."""
         d = self.d
         return self.ops.download([self.ops.edge_classes(
-            d["spec_codes"], d["spec_tensor"], *self._strategy_table(), d["edge_src_begin"], d["edge_n_src"], d["edge_tgt_begin"],
+            d["spec_codes"], d["spec_tensor"], *self._upload(*self.tables._strategy_rows(exact=True)), d["edge_src_begin"], d["edge_n_src"], d["edge_tgt_begin"],
             d["edge_n_tgt"], d["edge_flags"], d["edge_pt_begin"], d["edge_strat_begin"], d["pt_values"])])[0].numpy()
 
     @_guarded
@@ -379,12 +383,20 @@ class DeviceCostTables:
         return tb.n_entries <= self.PACKED_MAX_ENTRIES and tb.packable()
 
     def _packed_tiles(self, repeated):
-        """The device copy of ``CostTables.pack_tiles()``, made once per tiling; in launch order for a pass that is repeated
+        """``CostTables.pack_tiles()`` on the device, out of the tables there, made once per tiling; in launch order for a pass that is repeated
         (the order costs the host more than it saves one launch, which takes a copy that is there in either)."""
         cached = getattr(self, "_packed_cache", None)
         if cached is not None and cached[0] is self.tables.tile_records and (cached[1] or not repeated):
             return cached[2]
-        dev = _to_device(self.tables.pack_tiles(self.tables.launch_records() if repeated else None), self.device)
+        dev, packed = None, False
+        if self._tiles[1] is self.tables.tile_records and self.d["tile_records"] is self._tiles[0] and not any(
+                self.d[k].dtype != t for k, t in _PACKED_FROM.items()):  # (the tiling that is on the device)
+            d, tb = self.d, self.tables
+            dev, packed = self.ops.pack_tiles(  # (with the strategy table as the host has it)
+                *self._tensor_table(), d["spec_codes"], d["spec_tensor"], *self._upload(*(a[:tb.n_strategies] for a in tb._strategy_rows())),
+                d["edge_n_tgt"], self._tile_records(repeated), d["dup_entry_begin"], d["dup_row_begin"])
+        if not packed:  # (the host packs them, or says which it cannot)
+            dev = _to_device(self.tables.pack_tiles(self.tables.launch_records() if repeated else None), self.device)
         self._packed_cache = (self.tables.tile_records, repeated, dev)
         return dev
 

@@ -111,7 +111,7 @@ class DeviceBackend:
         """The strategy table is final: tile the edges (identical edges once) and send both."""
         names = ("tile_records", "dup_entry_begin", "dup_row_begin")
         own, on_device = getattr(self.dev, "tables", None) is tables, getattr(self, "_strategy_inputs_on_device", False)
-        if own and on_device and self.dev._check_on_device_pays():  # (all that an edge's identity depends on is there)
+        if own and dedupe and self.dev._check_on_device_pays():
             tables._build_tiles(self.dev.edge_classes, tile_entries, dedupe, max_copies, repeated=False)
         else:
             tables.build_tiles(tile_entries, dedupe=dedupe, max_copies=max_copies, repeated=False)

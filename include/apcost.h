@@ -569,6 +569,15 @@ typedef struct apc_packed_tile {
   int32_t row_meta[APC_TILE_MAX_ROWS];          /* dtype code (low byte, signed) | zero_cost << 8 | num_args << 16 */
 } apc_packed_tile;
 
+/* apc_pack_tiles_host of tables that are on the device: packed[t] = everything tile t reads.  *refused (on the device, cleared by the
+ * caller) is set to 1 where a tile cannot be packed, or names rows outside the tables; its record is not written then. */
+int apc_pack_tiles(int64_t n_tensors, const int32_t *tensor_rank, const int32_t *tensor_itemsize, const int64_t *tensor_shape,
+                   const int64_t *tensor_stride, int64_t n_specs, const uint32_t *spec_codes, const int32_t *spec_tensor,
+                   int64_t n_strategies, const int64_t *flops, const int64_t *rw_bytes, const int8_t *dtype_code,
+                   const uint8_t *zero_cost, const int32_t *num_args, int64_t n_edges, const int64_t *edge_row_begin, int64_t n_tiles,
+                   const apc_tile *tiles, int64_t n_dups, const int64_t *dup_entry_begin, const int64_t *dup_row_begin,
+                   apc_packed_tile *packed, int32_t *refused, void *stream);
+
 /* Host-side check (HOST pointers) that packed[t] repeats, field by field, what tiles[t] and the
  * tables say; tiles must hold whole rows (apc_validate_row_minima_host) and at most
  * APC_PACKED_MAX_DUPS identical edges each.  edge_row_begin[e] = first matrix row of edge e. */

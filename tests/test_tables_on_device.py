@@ -92,7 +92,7 @@ def test_a_tiling_that_is_refused_leaves_the_old_one_on_the_device(gpu_device):
     tb = _tables(mesh)
     backend = DeviceBackend(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
     before = dict(backend.dev.d)
-    tb.build_tiles = lambda *a, **k: tb.dup_entry_begin.__setitem__(0, 1)
+    tb._build_tiles = lambda *a, **k: tb.dup_entry_begin.__setitem__(0, 1)
     with pytest.raises(RuntimeError, match="duplicate offset"):
         backend.upload_strategy_inputs(tb)
     assert all(backend.dev.d[k] is before[k] for k in before)
@@ -146,6 +146,42 @@ def test_the_planner_tiles_by_the_classes_of_the_device(gpu_device):
     tb.build_tiles(None, dedupe=True, repeated=False)
     want = tb.tile_records.copy()
     backend = DeviceBackend(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
-    backend._strategy_inputs_on_device = True
     backend.upload_strategy_inputs(tb)
     assert np.array_equal(tb.tile_records, want) and np.array_equal(backend.dev.d["tile_records"].cpu().numpy().view(np.uint8).ravel(), want.view(np.uint8))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mesh", MESHES)
+@pytest.mark.parametrize("max_strategies", [1, 10, 64])
+def test_tiles_packed_on_the_device_are_the_hosts(gpu_device, mesh, max_strategies):
+    """Byte for byte, in the table's order and in launch order; with pass-through edges, twins and specs of no tensor."""
+    tb = twin_graph(stress_dag(seed=31, n_nodes=80, mesh_sizes=mesh, min_strategies=1, max_strategies=max_strategies))
+    tb.build_tiles(None, dedupe=True)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
+    assert tb.packable() and (tb.tile_records["dup_count"] > 0).any()
+    for repeated in (False, True):
+        want = tb.pack_tiles(tb.launch_records() if repeated else None)
+        dev, packed = d.ops.pack_tiles(*d._tensor_table(), d.d["spec_codes"], d.d["spec_tensor"], *d._strategy_table(), d.d["edge_n_tgt"],
+                                       d._tile_records(repeated), d.d["dup_entry_begin"], d.d["dup_row_begin"])
+        assert packed and dev.cpu().numpy().tobytes() == want.tobytes()
+    # a strategy with more arguments than a record holds, and a record that leaves the tables
+    many = d.d["strat_num_args"].clone()
+    many[int(tb.tile_records["strat_begin"][0] + tb.tile_records["row_begin"][0])] = 0x8000
+    records = d.d["tile_records"].clone()
+    records[0, 4] = tb.n_specs  # (src_begin)
+    for strategies, tiles in (((*d._strategy_table()[:4], many), d.d["tile_records"]), (d._strategy_table(), records)):
+        assert not d.ops.pack_tiles(*d._tensor_table(), d.d["spec_codes"], d.d["spec_tensor"], *strategies, d.d["edge_n_tgt"], tiles,
+                                    d.d["dup_entry_begin"], d.d["dup_row_begin"])[1]
+
+
+@pytest.mark.gpu
+def test_classes_and_packed_tiles_are_of_the_hosts_strategy_table(gpu_device):
+    """A strategy table changed on the host after the upload."""
+    mesh = (4, 2, 2)
+    tb = _tables(mesh)
+    tb.build_tiles(None, dedupe=True)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
+    tb.strat_flops[:] = tb.strat_rw_bytes
+    assert d._packed_tiles(False).cpu().numpy().tobytes() == tb.pack_tiles().tobytes()
+    tb.strat_num_args[::3] += 1
+    assert np.array_equal(d.edge_classes(), tb.edge_classes())
