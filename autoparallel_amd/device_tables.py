@@ -420,7 +420,7 @@ class DeviceCostTables:
         ``fused_inputs`` the tensor, spec and compute-cost tables are one launch
         (``input_tables``) instead of three; with ``one_launch`` they and the cost matrices
         are one (``build_tables``); ``one_launch=None`` takes one launch for tables up to
-        ``ONE_LAUNCH_MAX_BYTES`` when ``fused_inputs`` is set.  ``row_min_in_tiles``: the launch
+        ``one_launch_limit()`` when ``fused_inputs`` is set.  ``row_min_in_tiles``: the launch
         that writes the cost matrices takes the row minima too (no ``segmented_min`` launch, no
         second read of the matrices); it needs every row inside one tile
         (``CostTables.rows_fit_tiles``), and ``None`` takes it when ``row_min_in_tiles_pays``.
@@ -437,7 +437,7 @@ class DeviceCostTables:
         captures, a pass is prepared as with ``repeated=False`` and takes the edges' first rows, or the packed tiles, of an earlier preparation
         (a table that staged tiles are faster for goes over packed ones where only those are there)."""
         tb = self.tables
-        capturing = torch.cuda.is_current_stream_capturing()
+        capturing, runs_once = torch.cuda.is_current_stream_capturing(), not repeated
         repeated = bool(repeated) and not capturing
         outputs = tuple(outputs)
         if not outputs or any(o not in ("comm", "transition", "cost") for o in outputs):
@@ -458,7 +458,7 @@ class DeviceCostTables:
         packed_kind = bool(one_launch) and row_min_in_tiles and outputs == ("cost",) and not spec_table
         if packed is None:
             packed = packed_kind and self.packed_pass_pays() and not (
-                tb.staging_pays(tb.computed_entries(), tb.n_tiles) and (self._edge_rows is not None or not capturing))
+                tb.staging_pays(tb.computed_entries(), tb.n_tiles, repeated=not runs_once) and (self._edge_rows is not None or not capturing))
         elif packed and not (packed_kind and self.tables.packable()):
             raise ValueError("a pass over packed tiles is one launch that writes the assembled cost and the row minima, "
                              "without the spec table, over tiles of whole rows")
@@ -543,7 +543,7 @@ class DeviceCostTables:
         """The launches ``ShardingOptimizer.build_ds`` issues once the flop / byte counts are in
         the strategy table (optimize_sharding.py:270-380 in one pass): the tensor and
         compute-cost tables and the assembled cost of every entry, the array the ILP objective
-        is summed from, in one launch for tables up to ``ONE_LAUNCH_MAX_BYTES`` (else the input
+        is summed from, in one launch for tables up to ``one_launch_limit()`` (else the input
         tables, then the matrices); the launch also takes the row minima when that is cheaper
         than reading the matrices back (``row_min_in_tiles_pays``), otherwise they are taken
         when asked for.  The spec table is not part of it (the planner needed the local shard

@@ -450,7 +450,7 @@ class CostTables:
                 tiled_edges = int(np.count_nonzero((canonical == np.arange(self.n_edges)) & (n_src > 0) & (n_tgt > 0)))
                 fits = n == 0 or int(n_src.max()) <= APC_TILE_MAX_COLS
                 rows_per_wavefront_pass = 4
-                if n and (not fits or self._staging_may_pay(whole_edges[1], tiled_edges)):
+                if n and (not fits or self._staging_may_pay(whole_edges[1], tiled_edges, repeated)):
                     n, n_dups = count(te, mc, 0)
                     wanted, least = STAGED_TILES, max(STAGED_MIN_TILE_ENTRIES, whole_edges[1] // STAGED_SMALLEST_SHARE)
                     if self._many_states():
@@ -458,7 +458,7 @@ class CostTables:
                     while n < wanted and te // 2 >= 1 << (least.bit_length() - 1):
                         te //= 2
                         n, n_dups = count(te, mc, 0)
-                    if not fits or self.staging_pays(whole_edges[1], n, tiled_edges):
+                    if not fits or self.staging_pays(whole_edges[1], n, tiled_edges, repeated):
                         rows_per_wavefront_pass = None
                     else:
                         te, (n, n_dups) = APC_TILE_MAX_ROWS * APC_TILE_MAX_COLS, packed_cut
@@ -521,16 +521,18 @@ class CostTables:
     def _many_states(self) -> bool:
         return len(self.mesh_sizes) == 4 and any(m & (m - 1) for m in self.mesh_sizes)
 
-    def _staging_may_pay(self, computed: int, tiled_edges: int) -> bool:
+    def _staging_may_pay(self, computed: int, tiled_edges: int, repeated: bool) -> bool:
         """``staging_pays`` of some number of tiles."""
-        return computed >= STAGED_MIN_COMPUTED_OF_COPIES or self.staging_pays(computed, computed + 1, tiled_edges)
+        return computed >= STAGED_MIN_COMPUTED_OF_COPIES or self.staging_pays(computed, computed + 1, tiled_edges, repeated)
 
-    def staging_pays(self, computed: int, n_tiles: int, tiled_edges: Optional[int] = None) -> bool:
+    def staging_pays(self, computed: int, n_tiles: int, tiled_edges: Optional[int] = None, repeated: bool = True) -> bool:
         """Whether tiles staged in LDS beat packed ones on a small table (above: STAGED_MIN_COMPUTED).  ``tiled_edges``: the edges
-        that have tiles, by default those of the current tiling where it was chosen from the table."""
+        that have tiles, by default those of the current tiling where it was chosen from the table.  A pass that runs once
+        (``repeated=False``, a planner's) goes over packed tiles unless much is computed: their records hold the strategy table as the
+        host has it, which a planner may have written there, where staged tiles read the device's; a few us are nothing to it."""
         if tiled_edges is None:
             tiled_edges = (self.tiling or {}).get("tiled_edges", 0)
-        if not self._many_states():
+        if repeated and not self._many_states():
             if tiled_edges > STAGED_MANY_EDGES or (computed >= STAGED_MIN_COMPUTED and self.n_entries <= STAGED_MAX_COPIES * computed):
                 return True
         return computed >= STAGED_MIN_COMPUTED_OF_COPIES and computed >= n_tiles * STAGED_MIN_COMPUTED_PER_TILE[len(self.mesh_sizes)]

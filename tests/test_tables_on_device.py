@@ -8,6 +8,8 @@ from autoparallel_amd.device_tables import _UPLOAD, DeviceCostTables
 from autoparallel_amd.optimize_sharding import DeviceBackend
 from autoparallel_amd.synthetic import stress_dag
 
+from oracle import c_oracle
+from oracle import cost_oracle as po
 from test_abi_and_encoding import twin_graph
 
 MESHES = [(8,), (12, 6), (4, 2, 2), (2, 2, 2, 2)]
@@ -185,3 +187,19 @@ def test_classes_and_packed_tiles_are_of_the_hosts_strategy_table(gpu_device):
     assert d._packed_tiles(False).cpu().numpy().tobytes() == tb.pack_tiles().tobytes()
     tb.strat_num_args[::3] += 1
     assert np.array_equal(d.edge_classes(), tb.edge_classes())
+
+
+@pytest.mark.gpu
+def test_a_pass_that_runs_once_is_of_the_hosts_strategy_table(gpu_device):
+    """A small table that a repeated pass takes over staged tiles, built once by a planner that has changed the strategy table."""
+    mesh = (16, 8, 4)
+    tb = stress_dag(seed=13, n_nodes=250, mesh_sizes=mesh, max_strategies=24)
+    assert tb.staging_pays(tb.computed_entries(), tb.n_tiles) and not tb.staging_pays(tb.computed_entries(), tb.n_tiles, repeated=False)
+    backend = DeviceBackend(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
+    backend._strategy_inputs_on_device = True
+    tb.strat_flops[:] = tb.strat_rw_bytes
+    backend.upload_strategy_inputs(tb)
+    backend.launch_tables()
+    assert backend.launches == ("build_tables_packed",)
+    want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh))["cost"]
+    assert np.array_equal(backend.dev.cost.cpu().numpy(), want)
