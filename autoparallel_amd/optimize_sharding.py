@@ -99,8 +99,8 @@ class DeviceBackend:
     def strategy_inputs(self, recipes):
         """Flop and byte counts of every strategy on the device (spec table, then
         ``apc_strategy_inputs`` over the per-node recipes); the host's strategy table receives
-        copies (identical edges are found on the host, and flop / byte counts are part of an
-        edge's identity)."""
+        copies (flop / byte counts are part of an edge's identity, which is decided by the host's
+        tables)."""
         tb = self.dev.tables
         counts = self.dev.ops.download(list(self.dev.run_strategy_inputs(recipes)))
         for a, t in zip((tb.strat_flops, tb.strat_rw_bytes, tb.strat_dtype, tb.strat_zero_cost), counts):
@@ -111,14 +111,15 @@ class DeviceBackend:
         """The strategy table is final: tile the edges (identical edges once) and send both."""
         names = ("tile_records", "dup_entry_begin", "dup_row_begin")
         own, on_device = getattr(self.dev, "tables", None) is tables, getattr(self, "_strategy_inputs_on_device", False)
-        if own and dedupe and self.dev._check_on_device_pays():
-            tables._build_tiles(self.dev.edge_classes, tile_entries, dedupe, max_copies, repeated=False)
+        rows = self.dev.send_rows() if own and dedupe and self.dev._check_on_device_pays() else None
+        if rows is not None:
+            tables._build_tiles(lambda: self.dev.edge_classes(rows), tile_entries, dedupe, max_copies, repeated=False)
         else:
             tables.build_tiles(tile_entries, dedupe=dedupe, max_copies=max_copies, repeated=False)
         if not on_device:
             names = ("strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost") + names
         if own:
-            self.dev.refresh_tiling(*names)
+            self.dev.refresh_tiling(*names, rows=rows)
         else:
             tables.validate(self.dev.params)
             self.dev.refresh(*names)

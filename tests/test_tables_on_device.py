@@ -5,6 +5,7 @@ import pytest
 
 from autoparallel_amd import CostModelParams, _native
 from autoparallel_amd.device_tables import _UPLOAD, DeviceCostTables
+from autoparallel_amd.encoding import EDGE_GRAD_RESCALE
 from autoparallel_amd.optimize_sharding import DeviceBackend
 from autoparallel_amd.synthetic import stress_dag
 
@@ -202,4 +203,39 @@ def test_a_pass_that_runs_once_is_of_the_hosts_strategy_table(gpu_device):
     backend.launch_tables()
     assert backend.launches == ("build_tables_packed",)
     want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh))["cost"]
+    assert np.array_equal(backend.dev.cost.cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["edge_flags", "edge_src_begin", "edge_tgt_begin", "edge_strat_begin", "edge_pt_begin", "spec_codes",
+                                  "spec_tensor", "pt_values"])
+def test_classes_are_of_the_hosts_edges_and_specs(gpu_device, name):
+    """Twins that were changed on the host after the upload."""
+    mesh = (4, 2, 2)
+    tb = _tables(mesh)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
+    before = tb.edge_classes()
+    a = getattr(tb, name)
+    if name == "edge_flags":
+        a[len(a) // 2::2] ^= EDGE_GRAD_RESCALE
+    elif name == "pt_values":
+        a[len(a) // 2:] = np.arange(len(a) - len(a) // 2)
+    else:
+        a[len(a) // 2:] = a[len(a) // 2:][::-1]
+    want = tb.edge_classes()
+    assert not np.array_equal(want, before) and np.array_equal(d.edge_classes(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mesh", MESHES)
+def test_a_twin_that_was_changed_after_the_upload_gets_its_own_costs(gpu_device, mesh):
+    """Every other twin with the other gradient rescale, set on the host between the backend's construction and the tiling."""
+    tb = _tables(mesh)
+    backend = DeviceBackend(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
+    tb.edge_flags[tb.n_edges // 2::2] ^= EDGE_GRAD_RESCALE
+    backend.upload_strategy_inputs(tb)
+    want_classes = tb.edge_classes()
+    assert np.array_equal(want_classes[tb.edge_canonical], want_classes)  # (a copy is a copy of its like)
+    backend.launch_tables()
+    want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh, rescale=2.2))["cost"]
     assert np.array_equal(backend.dev.cost.cpu().numpy(), want)
