@@ -239,3 +239,25 @@ def test_a_twin_that_was_changed_after_the_upload_gets_its_own_costs(gpu_device,
     backend.launch_tables()
     want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh, rescale=2.2))["cost"]
     assert np.array_equal(backend.dev.cost.cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["spec_codes", "spec_tensor", "tensor_rank", "tensor_itemsize", "tensor_shape", "tensor_stride", "strat_rw_bytes",
+                                  "edge_n_tgt", "tile_records", "dup_entry_begin", "dup_row_begin"])
+def test_packed_tiles_are_of_the_hosts_tables(gpu_device, name):
+    """Tables that were changed on the host after the upload, and one of them to another integer type."""
+    mesh = (4, 2, 2)
+    tb = _tables(mesh)
+    tb.build_tiles(None, dedupe=True)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
+    before = tb.pack_tiles().tobytes()
+    a = getattr(tb, name)
+    a[:] = a[::-1].copy()
+    want = tb.pack_tiles().tobytes()
+    assert want != before or name == "tensor_itemsize"  # (of which there is one)
+    if a.dtype == np.int32:
+        setattr(tb, name, a.astype(np.int64))
+    for repeated in (False, True):
+        d._packed_cache = None
+        want = tb.pack_tiles(tb.launch_records() if repeated else None).tobytes()
+        assert d._packed_tiles(repeated).cpu().numpy().tobytes() == want
