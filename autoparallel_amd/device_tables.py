@@ -45,6 +45,13 @@ _CLASSED = (
 )
 
 
+# what packed tiles are made of (``_pack_on_device``)
+_PACKED = (
+    "tensor_rank", "tensor_itemsize", "tensor_shape", "tensor_stride", "spec_codes", "spec_tensor", "strat_flops", "strat_rw_bytes",
+    "strat_dtype", "strat_zero_cost", "strat_num_args", "edge_n_tgt", "tile_records", "dup_entry_begin", "dup_row_begin",
+)
+
+
 def _as_tensor(a: np.ndarray) -> torch.Tensor:
     """The array as a CPU tensor over the same memory."""
     if a.dtype == np.uint32:  # same bits; torch's uint32 support is partial
@@ -114,6 +121,8 @@ class DeviceCostTables:
             self._ordered_tiles = None
         if "edge_n_tgt" in names:
             self._edge_rows = None
+        if self._packed_cache is not None and not set(_PACKED).isdisjoint(names):
+            self._pack_again()
 
     # Tables of fewer rows are checked on the host: it takes 0.35 ms for 315 k specs and 15 104 edges, with their tiles 0.45 and with
     # 15 000 copies' offsets 0.9, where a launch and the wait for its answer are 45 us.
@@ -167,11 +176,11 @@ class DeviceCostTables:
             self.tables.validate(self.params)
             self._refresh(names)
             return
-        before = dict(self.d), self._tiles, self._ordered_tiles, self._edge_rows
+        before = dict(self.d), self._tiles, self._ordered_tiles, self._edge_rows, self._packed_cache, self._packed_current
         try:
             self.tables._validate(self.params, lambda: self._refresh_and_check(names, "tables", rows or self.send_rows()))
         except BaseException:
-            self.d, self._tiles, self._ordered_tiles, self._edge_rows = before
+            self.d, self._tiles, self._ordered_tiles, self._edge_rows, self._packed_cache, self._packed_current = before
             raise
 
     # ---- helpers -------------------------------------------------------------------------
@@ -249,6 +258,7 @@ class DeviceCostTables:
             recipes.node_flop_rows.reshape(-1)), spec["local_shape"], spec["local_bytes"])
         for key, t in zip(("strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost"), out):
             self.d[key] = t
+        self._packed_current = False  # (the host's strategy table is about to change)
         return out
 
     # ---- per-strategy compute cost ---------------------------------------------------------
@@ -400,26 +410,49 @@ class DeviceCostTables:
         tb = self.tables
         return tb.n_entries <= self.PACKED_MAX_ENTRIES and tb.packable()
 
+    # (tile records, whether in launch order, the packed ones on the device), and whether those are of the tables as they are now
+    _packed_cache, _packed_current = None, True
+
     def _packed_tiles(self, repeated):
-        """``CostTables.pack_tiles()`` on the device, made once per tiling; in launch order for a pass that is repeated
-        (the order costs the host more than it saves one launch, which takes a copy that is there in either).  Put together
-        there out of the host's tables, sent beside those that launches read (0.32 ms for the 314 k specs and 129 k strategies of 15 104
-        edges, 0.35 by the host; 0.38 / 1.47 for 10 022 tiles of 428 k and 136 k, 0.085 / 0.15 for 436 of 1 766 and 730)."""
-        cached = getattr(self, "_packed_cache", None)
-        if cached is not None and cached[0] is self.tables.tile_records and (cached[1] or not repeated):
+        """``CostTables.pack_tiles()`` on the device, made once per tiling and again when a table it is made of was uploaded anew; in launch
+        order for a pass that is repeated (the order costs the host more than it saves one launch, which takes a copy that is there in
+        either)."""
+        tb, cached = self.tables, self._packed_cache
+        if cached is not None and cached[0] is tb.tile_records and (cached[1] or not repeated) and (
+                self._packed_current or torch.cuda.is_current_stream_capturing()):
             return cached[2]
+        dev, packed = self._pack_on_device(repeated)
+        if not packed:  # (the host packs them, or says which it cannot)
+            dev = _to_device(tb.pack_tiles(tb.launch_records() if repeated else None), self.device)
+        self._packed_cache, self._packed_current = (tb.tile_records, repeated, dev), True
+        return dev
+
+    def _pack_on_device(self, repeated):
+        """-> (packed tiles of the host's tables, whether all could be packed): put together on the device, the tables sent beside those that
+        launches read (0.32 ms for the 314 k specs and 129 k strategies of 15 104 edges, 0.35 by the host; 0.38 / 1.47 for 10 022 tiles
+        of 428 k and 136 k, 0.085 / 0.15 for 436 of 1 766 and 730)."""
         tb = self.tables
         records = tb.launch_records() if repeated else tb.tile_records
         n_dups = len(tb.dup_entry_begin)
-        dev, packed = self.ops.pack_tiles(*self._upload(
+        return self.ops.pack_tiles(*self._upload(
             *(a[:tb.n_tensors] for a in tb._rows(tb.n_tensors, "tensor_rank", "tensor_itemsize", "tensor_shape", "tensor_stride")),
             *(a[:tb.n_specs] for a in tb._rows(tb.n_specs, "spec_codes", "spec_tensor")),
             *(a[:tb.n_strategies] for a in tb._strategy_rows()), tb._matrix_sizes()[1], tb._records(records, tb.n_tiles, TILE_DTYPE),
             *(a[:n_dups] for a in tb._rows(n_dups, "dup_entry_begin", "dup_row_begin"))))
-        if not packed:  # (the host packs them, or says which it cannot)
-            dev = _to_device(tb.pack_tiles(records), self.device)
-        self._packed_cache = (self.tables.tile_records, repeated, dev)
-        return dev
+
+    def _pack_again(self):
+        """The packed tiles anew where a table they are made of was uploaded: a pass that is prepared next, also while the stream
+        captures, finds them.  (Launches bound earlier keep theirs.)"""
+        records, repeated, _ = self._packed_cache
+        self._packed_cache = None
+        if records is not self.tables.tile_records:
+            return
+        try:
+            dev, packed = self._pack_on_device(repeated)
+        except ValueError:  # (host tables of different lengths: one of several that are being replaced)
+            return
+        if packed:
+            self._packed_cache, self._packed_current = (records, repeated, dev), True
 
     def _tile_records(self, repeated):
         """The device copy of the tile records, in launch order for a pass that is repeated: of the tiling that is on the

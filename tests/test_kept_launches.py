@@ -15,6 +15,7 @@ import torch
 
 from autoparallel_amd import CostModelParams, _native
 from autoparallel_amd.device_tables import DeviceCostTables
+from autoparallel_amd.graphs.cost_inputs import StrategyRecipes
 from autoparallel_amd.synthetic import stress_dag
 from oracle import c_oracle
 from oracle import cost_oracle as po
@@ -257,3 +258,65 @@ def test_the_default_pass_is_prepared_while_the_stream_captures(gpu_device, befo
         graph.replay()
         torch.cuda.synchronize()
         assert np.array_equal(d.cost.cpu().numpy(), want) and np.array_equal(d.row_min.cpu().numpy(), lowest)
+
+
+def _small_packed(gpu_device):
+    mesh = (32, 8)
+    tb = stress_dag(seed=5, n_nodes=120, mesh_sizes=mesh, max_strategies=12)
+    tb.build_tiles(None, dedupe=True)
+    return tb, DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device), po.make_params(mesh, rescale=2.2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change", ["refresh", "refresh, captured", "strategy inputs"])
+def test_packed_tiles_are_of_the_tables_uploaded_last(gpu_device, change):
+    """A packed pass, then another strategy table on the same tiling: the next pass has its costs, and the launches bound
+    before keep theirs."""
+    tb, d, op = _small_packed(gpu_device)
+    first = d.planner_pass(packed=True)
+    first_cost = d.cost
+    before = c_oracle.build_tables(tb.as_dict(), op)["cost"]
+    if change == "strategy inputs":  # (the device counts, and the host's table receives the result)
+        recipes = StrategyRecipes(tb.n_nodes)
+        recipes.node_kind[:] = 1  # (bytes of the specs from the first on)
+        recipes.node_row_begin[:] = np.arange(tb.n_nodes + 1)
+        recipes.byte_rows = np.zeros(tb.n_nodes, np.int32)
+        counts = [t.cpu().numpy() for t in d.run_strategy_inputs(recipes)]
+        for name, a in zip(("strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost"), counts):
+            getattr(tb, name)[:] = a
+    else:
+        tb.strat_rw_bytes[:] = tb.strat_rw_bytes * 3 + (1 << 30)
+        d.refresh("strat_rw_bytes")
+    want = c_oracle.build_tables(tb.as_dict(), op)["cost"]
+    assert not np.array_equal(want, before)
+    if change.endswith("captured"):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for launch in d.planner_pass(packed=True).values():
+                launch()
+        runs = [graph.replay] * 3
+    else:
+        runs = list(d.planner_pass(packed=True).values())
+    for run in runs:
+        d.cost.zero_()
+        run()
+        torch.cuda.synchronize()
+        assert np.array_equal(d.cost.cpu().numpy(), want)
+    for launch in first.values():
+        launch()
+    assert np.array_equal(first_cost.cpu().numpy(), before)
+
+
+@pytest.mark.gpu
+def test_host_tables_between_two_lengths_can_be_refreshed(gpu_device):
+    """Packed tiles are not made again of tables of which some have been replaced; a pass prepared then says so."""
+    tb, d, op = _small_packed(gpu_device)
+    d.planner_pass(packed=True)
+    kept = tb.strat_flops
+    tb.strat_flops = np.append(kept, 0)
+    d.refresh("strat_flops")
+    tb.strat_flops = kept
+    d.refresh("strat_flops")
+    for launch in d.planner_pass(packed=True).values():
+        launch()
+    assert np.array_equal(d.cost.cpu().numpy(), c_oracle.build_tables(tb.as_dict(), op)["cost"])
