@@ -783,8 +783,8 @@ Tensor edge_classes(const Tensor &spec_codes, const Tensor &spec_tensor, const T
   return out;
 }
 
-// The tables of a report: tensor and compute-cost tables in one launch, then every per-entry array and, where edge_n_tgt is given,
-// the row minima.  -> ([tensor_bytes, tensor_contiguous, compute, per_arg, comm, transition, cost, row_min, row_argmin], whether a
+// The tables of a report: tensor and compute-cost tables in one launch, then every per-entry array and, where edge_n_tgt is given
+// (on the host or on the device), the row minima.  -> ([tensor_bytes, tensor_contiguous, compute, per_arg, comm, transition, cost, row_min, row_argmin], whether a
 // strategy with flops has an unsupported dtype).  Waits for the first launch's flag only, which a copy behind that launch brings
 // while the second one runs.
 std::tuple<std::vector<Tensor>, bool> report_tables(
@@ -808,15 +808,32 @@ std::tuple<std::vector<Tensor>, bool> report_tables(
                             dev<double>(compute, at::kDouble, "compute"), dev<double>(per_arg, at::kDouble, "per_arg"),
                             error.data_ptr<int32_t>(), stream),
            "apc_input_tables");
+  OptTensor row_begin, dup_rows, row_min, row_argmin;
+  Tensor row_begin_on_host;  // (pinned; the flag's event stands behind its copy too, and the flag goes first)
   Staging flag((int64_t)sizeof(int32_t), stream, 2);  // (with an event)
+  if (edge_n_tgt.has_value() && edge_n_tgt->is_cpu()) {  // (its running sum, 8 300 edges in 8 us, behind the first launch)
+    TORCH_CHECK(edge_n_tgt->scalar_type() == at::kInt && edge_n_tgt->is_contiguous(), "apcost: edge_n_tgt must be a contiguous int32 tensor");
+    const int64_t n = edge_n_tgt->numel();
+    row_begin_on_host = at::empty({n}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+    row_begin = empty_like_device(rank, {n}, at::kLong);
+    const int32_t *n_tgt = edge_n_tgt->data_ptr<int32_t>();
+    int64_t *begin = row_begin_on_host.data_ptr<int64_t>(), sum = 0;
+    for (int64_t e = 0; e < n; ++e) {
+      begin[e] = sum;
+      sum += n_tgt[e];
+    }
+    TORCH_CHECK(sum == n_rows, "apcost: edge_n_tgt has ", sum, " rows, n_rows says ", n_rows);
+    if (n)
+      check_hip(hipMemcpyAsync(row_begin->data_ptr(), begin, sizeof(int64_t) * (size_t)n, hipMemcpyHostToDevice, stream), "hipMemcpyAsync");
+  } else if (edge_n_tgt.has_value()) {
+    row_begin = edge_rows(*edge_n_tgt);
+  }
   check_hip(hipMemcpyAsync(flag.slot(0), error.data_ptr(), sizeof(int32_t), hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
   check_hip(hipEventRecord(flag.events[0], stream), "hipEventRecord");
   Tensor comm = empty_like_device(rank, {n_entries}, at::kDouble), transition = empty_like_device(rank, {n_entries}, at::kByte),
          cost = empty_like_device(rank, {n_entries}, at::kDouble);
   std::vector<Tensor> out{bytes, contiguous, compute, per_arg, comm, transition, cost};
-  OptTensor row_begin, dup_rows, row_min, row_argmin;
   if (edge_n_tgt.has_value()) {
-    row_begin = edge_rows(*edge_n_tgt);
     dup_rows = dup_row_begin;
     row_min = empty_like_device(rank, {n_rows}, at::kDouble);
     row_argmin = empty_like_device(rank, {n_rows}, at::kInt);

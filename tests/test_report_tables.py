@@ -6,7 +6,11 @@ import torch
 
 from autoparallel_amd import CostModelParams, _native
 from autoparallel_amd.device_tables import DeviceCostTables
+from autoparallel_amd.optimize_sharding import DeviceBackend
 from autoparallel_amd.synthetic import stress_dag
+
+from oracle import c_oracle
+from oracle import cost_oracle as po
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +69,50 @@ def test_an_unsupported_dtype_is_refused(gpu_device):
     with pytest.raises(ValueError, match="dtype not supported"):
         d.build_all()
     assert d.cost is kept[2] and bool(torch.isnan(d.compute_cost).any())
+
+
+EDGE_ARRAYS = ("edge_src_begin", "edge_n_src", "edge_tgt_begin", "edge_n_tgt", "edge_flags", "edge_strat_begin")
+
+
+@pytest.mark.parametrize("how", ["build_all", "run_redistribute_tables", "upload_strategy_inputs"])
+def test_edge_arrays_of_another_integer_type(gpu_device, how, monkeypatch):
+    """Set after the construction: the host converts them where it reads them, and no kernel reads them."""
+    monkeypatch.setattr(DeviceCostTables, "CHECK_ON_DEVICE_MIN_ROWS", 0)
+    mesh = (4, 2)
+    tb = stress_dag(seed=5, n_nodes=200, mesh_sizes=mesh)
+    tb.build_tiles(None, dedupe=True)
+    backend = DeviceBackend(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
+    d = backend.dev
+    for name in EDGE_ARRAYS:
+        setattr(tb, name, getattr(tb, name).astype(np.int64))
+    d.refresh(*EDGE_ARRAYS)
+    if how == "build_all":
+        d.build_all()
+    elif how == "run_redistribute_tables":
+        d.run_redistribute_tables(row_min=True)
+    else:
+        backend.upload_strategy_inputs(tb)
+        backend.launch_tables()
+    want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh, rescale=2.2))["cost"]
+    assert np.array_equal(d.cost.cpu().numpy(), want)
+    want_min, want_arg = c_oracle.segmented_min(want, tb.row_ptr())
+    assert d.row_min is not None
+    assert np.array_equal(d.row_min.cpu().numpy(), want_min) and np.array_equal(d.row_argmin.cpu().numpy(), want_arg)
+
+
+def test_the_rows_of_a_report_from_the_host_and_the_device(gpu_device):
+    mesh = (4, 2)
+    tb = stress_dag(seed=5, n_nodes=200, mesh_sizes=mesh)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
+
+    def report(n_tgt, n_rows):
+        return d.ops.report_tables(
+            d.p, *d._tensor_table(), d.d["spec_codes"], d.d["spec_tensor"], *d._strategy_table(), d.d["pt_values"], d.d["tile_records"],
+            d.d["dup_entry_begin"], tb.n_entries, n_tgt, d.d["dup_row_begin"], n_rows)[0]
+
+    on_host = torch.from_numpy(tb.edge_n_tgt)
+    for a, b in zip(report(on_host, tb.n_rows), report(on_host.to(gpu_device), tb.n_rows)):
+        assert torch.equal(a, b)
+    for n_tgt, n_rows in ((on_host.long(), tb.n_rows), (on_host, tb.n_rows - 1), (on_host[:-1], tb.n_rows)):
+        with pytest.raises(RuntimeError, match="edge_n_tgt"):
+            report(n_tgt, n_rows)
