@@ -15,15 +15,17 @@ from oracle import cost_oracle as po
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [0, 1, 2, 1023, 1024, 1025, 70_001])
+@pytest.mark.parametrize("n", [0, 1, 2, 1023, 1024, 1025, 4095, 4096, 4097, 8195, 210_003])
 def test_first_rows_of_the_edges(gpu_device, n):
+    """Sums beyond 32 bits within a thread's edges, across a wavefront, across the wavefronts and from block to block."""
     n_tgt = np.random.default_rng(n).integers(0, 90, n).astype(np.int32)
-    if n > 2:
-        n_tgt[n // 2] = 1 << 22  # (sums beyond 32 bits)
-        n_tgt[-1] = 0
-    n_tgt = np.tile(n_tgt, 1 if n < 2000 else 3)
+    n_tgt[n // 3:n // 3 + 4] = 2**31 - 1
+    n_tgt[n // 2::37] = 1 << 30
+    n_tgt[-1:] = 0
+    want = np.cumsum(n_tgt.astype(np.int64)) - n_tgt
+    assert n < 1000 or (want > 2**33).sum() > n // 3
     got = _native.torch_ops().edge_rows(torch.from_numpy(n_tgt).to(gpu_device))
-    assert got.dtype == torch.int64 and np.array_equal(got.cpu().numpy(), np.cumsum(n_tgt.astype(np.int64)) - n_tgt)
+    assert got.dtype == torch.int64 and np.array_equal(got.cpu().numpy(), want)
 
 
 @pytest.mark.parametrize("group", [None, 1, 2, 4, 8, 16, 32, 64])
