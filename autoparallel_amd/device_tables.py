@@ -121,8 +121,10 @@ class DeviceCostTables:
             self._ordered_tiles = None
         if "edge_n_tgt" in names:
             self._edge_rows = None
-        if self._packed_cache is not None and not set(_PACKED).isdisjoint(names):
-            self._pack_again()
+        if not set(_PACKED).isdisjoint(names):
+            self._host_on_device = False
+            if self._packed_cache is not None:
+                self._pack_again()
 
     # Tables of fewer rows are checked on the host: it takes 0.35 ms for 315 k specs and 15 104 edges, with their tiles 0.45 and with
     # 15 000 copies' offsets 0.9, where a launch and the wait for its answer are 45 us.
@@ -258,7 +260,7 @@ class DeviceCostTables:
             recipes.node_flop_rows.reshape(-1)), spec["local_shape"], spec["local_bytes"])
         for key, t in zip(("strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost"), out):
             self.d[key] = t
-        self._packed_current = False  # (the host's strategy table is about to change)
+        self._packed_current = self._host_on_device = False  # (the host's strategy table is about to change)
         return out
 
     # ---- per-strategy compute cost ---------------------------------------------------------
@@ -431,14 +433,35 @@ class DeviceCostTables:
         """-> (packed tiles of the host's tables, whether all could be packed): put together on the device, the tables sent beside those that
         launches read (0.32 ms for the 314 k specs and 129 k strategies of 15 104 edges, 0.35 by the host; 0.38 / 1.47 for 10 022 tiles
         of 428 k and 136 k, 0.085 / 0.15 for 436 of 1 766 and 730)."""
+        return self.ops.pack_tiles(*self._upload(*self._packed_of(repeated)))
+
+    def _packed_of(self, repeated) -> list:
+        """The host's tables that packed tiles are made of (``_PACKED``)."""
         tb = self.tables
         records = tb.launch_records() if repeated else tb.tile_records
         n_dups = len(tb.dup_entry_begin)
-        return self.ops.pack_tiles(*self._upload(
+        return [
             *(a[:tb.n_tensors] for a in tb._rows(tb.n_tensors, "tensor_rank", "tensor_itemsize", "tensor_shape", "tensor_stride")),
             *(a[:tb.n_specs] for a in tb._rows(tb.n_specs, "spec_codes", "spec_tensor")),
             *(a[:tb.n_strategies] for a in tb._strategy_rows()), tb._matrix_sizes()[1], tb._records(records, tb.n_tiles, TILE_DTYPE),
-            *(a[:n_dups] for a in tb._rows(n_dups, "dup_entry_begin", "dup_row_begin"))))
+            *(a[:n_dups] for a in tb._rows(n_dups, "dup_entry_begin", "dup_row_begin"))]
+
+    _host_on_device = False  # whether a preparation found the host's tables on the device, and none was uploaded since
+
+    def _staged_is_as_packed(self, capturing) -> bool:
+        """Whether a pass over staged tiles, which read the tables on the device, has the results of one over packed ones, which are
+        the host's: whether no table was changed on the host and not uploaded (0.1 to 0.4 ms a preparation).  While the stream captures, as
+        an earlier preparation found it, or left it without packed tiles."""
+        if capturing:
+            return self._host_on_device or self._packed_cache is None or self._packed_cache[0] is not self.tables.tile_records
+        sent, there = self._upload(*self._packed_of(False)), [self.d[k] for k in _PACKED]
+
+        def joined(arrays):
+            return torch.cat([a.reshape(-1).view(torch.uint8) for a in arrays])
+
+        self._host_on_device = all(a.dtype == b.dtype and a.shape == b.shape for a, b in zip(sent, there)) and torch.equal(
+            joined(sent), joined(there))
+        return self._host_on_device
 
     def _pack_again(self):
         """The packed tiles anew where a table they are made of was uploaded: a pass that is prepared next, also while the stream
@@ -483,7 +506,9 @@ class DeviceCostTables:
         flop / byte counts this pass reads).  ``packed``: the one launch runs over packed tiles
         (``apc_build_tables_packed``: the assembled cost and the row minima, no spec table);
         ``None`` takes them when the pass is of that kind, ``packed_pass_pays`` and staged tiles
-        (``CostTables.staging_pays``) are not faster still.  ``repeated=False``: the pass will run once, and the arguments
+        (``CostTables.staging_pays``) are not faster still.  Packed tiles hold the host's tables as they are at the
+        preparation; where staged tiles are faster for the repeated pass of a small table, they are taken if the tables on the device, which
+        they read, are the same.  ``repeated=False``: the pass will run once, and the arguments
         of its launches are not laid out in device memory first (``apc_kept_launch``: one copy, for 0.75 us less a launch over packed
         tiles or a large table, nothing where staged tiles wait for other loads at that time), nor its tiles put
         into launch order (``CostTables.launch_records``: 10 ns a tile on the host).  Those copies, one a launch
@@ -511,8 +536,11 @@ class DeviceCostTables:
             one_launch = bool(fused_inputs) and total <= self.one_launch_limit()
         packed_kind = bool(one_launch) and row_min_in_tiles and outputs == ("cost",) and not spec_table
         if packed is None:
-            packed = packed_kind and self.packed_pass_pays() and not (
-                tb.staging_pays(tb.computed_entries(), tb.n_tiles, repeated=not runs_once) and (self._edge_rows is not None or not capturing))
+            packed = packed_kind and self.packed_pass_pays()
+            if packed and (self._edge_rows is not None or not capturing):
+                of_tiles = tb.computed_entries(), tb.n_tiles
+                packed = not (tb.staging_pays(*of_tiles, repeated=False) or (
+                    not runs_once and tb.staging_pays(*of_tiles) and self._staged_is_as_packed(capturing)))
         elif packed and not (packed_kind and self.tables.packable()):
             raise ValueError("a pass over packed tiles is one launch that writes the assembled cost and the row minima, "
                              "without the spec table, over tiles of whole rows")

@@ -528,8 +528,9 @@ class CostTables:
     def staging_pays(self, computed: int, n_tiles: int, tiled_edges: Optional[int] = None, repeated: bool = True) -> bool:
         """Whether tiles staged in LDS beat packed ones on a small table (above: STAGED_MIN_COMPUTED).  ``tiled_edges``: the edges
         that have tiles, by default those of the current tiling where it was chosen from the table.  A pass that runs once
-        (``repeated=False``, a planner's) goes over packed tiles unless much is computed: their records hold the strategy table as the
-        host has it, which a planner may have written there, where staged tiles read the device's; a few us are nothing to it."""
+        (``repeated=False``, a planner's) goes over packed tiles unless much is computed: their records hold the tables as the
+        host has them, which a planner may have written there, where staged tiles read the device's; a few us are nothing to it.  A
+        repeated one compares the two (``DeviceCostTables.prepare_step``)."""
         if tiled_edges is None:
             tiled_edges = (self.tiling or {}).get("tiled_edges", 0)
         if repeated and not self._many_states():

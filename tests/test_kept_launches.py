@@ -320,3 +320,47 @@ def test_host_tables_between_two_lengths_can_be_refreshed(gpu_device):
     for launch in d.planner_pass(packed=True).values():
         launch()
     assert np.array_equal(d.cost.cpu().numpy(), c_oracle.build_tables(tb.as_dict(), op)["cost"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["strat_rw_bytes", "spec_codes", "tensor_shape", None])
+def test_the_default_pass_is_of_the_hosts_tables(gpu_device, name):
+    """A small table that staged tiles are faster for, one of whose tables was changed on the host after the upload: over packed
+    tiles, as every small table; over staged ones, captured ones too, where it was uploaded again or nothing was changed."""
+    mesh = (16, 8, 4)
+    tb = stress_dag(seed=13, n_nodes=250, mesh_sizes=mesh, max_strategies=24)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
+    op = po.make_params(mesh, rescale=2.2)
+    assert d.packed_pass_pays() and tb.staging_pays(tb.computed_entries(), tb.n_tiles) and not tb.staging_pays(
+        tb.computed_entries(), tb.n_tiles, repeated=False)
+    if name is not None:
+        a, row = getattr(tb, name), int(tb.edge_tgt_begin[-1])
+        if name == "spec_codes":
+            a[row:row + tb.edge_n_tgt[-1]] = a[row:row + tb.edge_n_tgt[-1]][::-1].copy()
+        else:
+            a[:] *= 2
+    want = c_oracle.build_tables(tb.as_dict(), op)["cost"]
+    lowest = np.minimum.reduceat(want, tb.row_ptr()[:-1])
+
+    def check(runs, kind):
+        assert list(step) == [kind]
+        for run in runs:
+            for t in (d.cost, d.row_min):
+                t.zero_()
+            run()
+            torch.cuda.synchronize()
+            assert np.array_equal(d.cost.cpu().numpy(), want) and np.array_equal(d.row_min.cpu().numpy(), lowest)
+
+    step = d.planner_pass()
+    check(step.values(), "build_tables" if name is None else "build_tables_packed")
+    if name is not None:
+        d.refresh(name)
+        step = d.planner_pass()
+        check(step.values(), "build_tables")
+        d.refresh(name)  # (no preparation between this and the capture)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step = d.planner_pass()
+        for launch in step.values():
+            launch()
+    check([graph.replay] * 3, "build_tables" if name is None else "build_tables_packed")
