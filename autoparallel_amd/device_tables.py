@@ -52,6 +52,9 @@ _PACKED = (
 )
 
 
+_ONE_LAUNCH_MAX_BYTES = 192 << 20
+
+
 def _as_tensor(a: np.ndarray) -> torch.Tensor:
     """The array as a CPU tensor over the same memory."""
     if a.dtype == np.uint32:  # same bits; torch's uint32 support is partial
@@ -339,20 +342,32 @@ class DeviceCostTables:
         return self.comm, self.transition, self.cost
 
     # ---- one full device-side pass with pre-bound arguments -------------------------------------
-    # A pass over a table this small is bound by the ramp-up and drain of every launch, and
-    # one launch for all tables wins; above it the tiles' own derivation of what they would otherwise
-    # read costs more than a launch.  The cost alone, one launch / two: on (16, 8, 4) 10.6 M entries 36.5 / 39.6 us, 20 M (163 MB) 58.8 /
-    # 59.9, 28 M 78.6 / 74.3, 42 M 125 / 120; on meshes of one or two dims, where a tile derives as much and stages less, up to
-    # ONE_LAUNCH_MAX_BYTES_FLAT: on (64, 4) 20 M 56.0 / 62.8, 42 M (334 MB) 116.6 / 119.6, on (32, 8) 20 M 64.4 / 67.7, 26 M in 40 layers
-    # 57.3 / 59.0, on (12, 6) 20 M 65.7 / 68.9; the other way 47 M in eight layers on (64, 4) 129 / 124.  What the derivation costs goes by
-    # tiles and not by bytes, though: tables of many small tiles lose by these limits, 5.4 M entries in 36 157 tiles 54.8 / 43.7 on
-    # (32, 8), 47.1 / 43.9 on (16, 8, 4), 5.3 M in 162 354 tiles 179 / 107 (measured when both took longer).
-    ONE_LAUNCH_MAX_BYTES = 192 << 20
+    # One launch for all tables saves a ramp-up and drain, about 6 us; the tiles' own derivation of what they would otherwise read costs 0.1
+    # to 0.15 ns a tile beside the work that both have.  The cost alone, us in one launch / two:
+    #   up to ONE_LAUNCH_MAX_BYTES on 3-D and 4-D meshes, (16, 8, 4), 16 M entries (136 MiB) 33.3 / 34.5, 21.7 M (183 MiB) 44.1 / 44.6, on
+    #   (6, 4, 2) 49.3 / 49.7, on (2, 4, 2, 2) 53.7 / 54.4, with three states in turn 28 M 78.6 / 74.3, 42 M 125 / 120;
+    #   up to ONE_LAUNCH_MAX_BYTES_FLAT on meshes of one or two dims, where a tile stages less: on (64, 4) 32.7 M (274 MiB) 84.5 / 85.2, 40 M
+    #   (336 MiB) 109 / 114, 37.8 M in eight layers (331 MiB) 83.4 / 83.2, on (32, 8) 41.7 M (350 MiB) 112.5 / 118, 32.3 M in 40 layers 70.4 / 78.6,
+    #   on (12, 6) 41.7 M 116 / 121; with three states in turn 47 M in eight layers on (64, 4) (376 MiB) 129 / 124;
+    #   beyond ONE_LAUNCH_MAX_BYTES_OF_MANY_TILES not in more than ONE_LAUNCH_MANY_TILES, where the tiles cost what the launch saves: 44 850 tiles
+    #   (above) and 46 056 116 / 121, then 49 238 on (32, 8) 55.6 / 54.5, 70 738 63.5 / 60.9, 96 217 77.8 / 72.5, 427 120 on (64, 4) 263 / 238, on (16, 8, 4)
+    #   45 064 54.6 / 53.5, 70 737 61.4 / 59.4, on (6, 4, 2) 96.9 / 89.3; nor on a 4-D mesh with a size that is no power of two, whose states cost most
+    #   to stage, 20 016 tiles (184 MiB) 89.8 / 88.4, 42 860 (177 MiB) 152 / 141.  Smaller tables are one launch whatever their tiles: it decides
+    #   whether they can go over packed ones (5.3 M entries in 162 354 tiles lose by it, 179 / 107, measured when both took longer).
+    ONE_LAUNCH_MAX_BYTES = _ONE_LAUNCH_MAX_BYTES
     ONE_LAUNCH_MAX_BYTES_FLAT = 344 << 20
+    ONE_LAUNCH_MAX_BYTES_OF_MANY_TILES = 128 << 20
+    ONE_LAUNCH_MANY_TILES = 48 << 10
 
     def one_launch_limit(self) -> int:
-        flat = len(self.tables.mesh_sizes) <= 2
-        return max(self.ONE_LAUNCH_MAX_BYTES, self.ONE_LAUNCH_MAX_BYTES_FLAT) if flat and self.ONE_LAUNCH_MAX_BYTES else self.ONE_LAUNCH_MAX_BYTES
+        """Bytes of the largest pass that is one launch: ``ONE_LAUNCH_MAX_BYTES`` where a program has set it, else by the mesh and the
+        tiles."""
+        tb, limit = self.tables, self.ONE_LAUNCH_MAX_BYTES
+        if limit != _ONE_LAUNCH_MAX_BYTES:
+            return limit
+        if tb.n_tiles > self.ONE_LAUNCH_MANY_TILES or tb._many_states():
+            return self.ONE_LAUNCH_MAX_BYTES_OF_MANY_TILES
+        return self.ONE_LAUNCH_MAX_BYTES_FLAT if len(tb.mesh_sizes) <= 2 else limit
 
     def row_min_in_tiles_pays(self) -> bool:
         """Whether the launch that writes the cost matrices should take the row minima itself.

@@ -117,3 +117,18 @@ def test_pass_over_the_automatic_cut_matches_the_oracle(gpu_device, mesh, nodes,
         if d.row_min is not None:
             mins, args = c_oracle.segmented_min(want["cost"], tb.row_ptr())
             assert np.array_equal(d.row_min.cpu().numpy(), mins) and np.array_equal(d.row_argmin.cpu().numpy(), args)
+
+
+@pytest.mark.parametrize("mesh,limit,of_many", [((64,), 344, 128), ((32, 8), 344, 128), ((8, 8, 8), 192, 128), ((2, 4, 2, 2), 192, 128),
+                                                ((3, 2, 2, 2), 128, 128)])
+def test_bytes_of_the_largest_pass_in_one_launch(mesh, limit, of_many):
+    d = object.__new__(DeviceCostTables)
+    d.tables = _table(mesh, 40, 4, False)
+    assert d.one_launch_limit() == limit << 20
+    d.ONE_LAUNCH_MANY_TILES = d.tables.n_tiles
+    assert d.one_launch_limit() == limit << 20
+    d.ONE_LAUNCH_MANY_TILES -= 1
+    assert d.one_launch_limit() == of_many << 20
+    for asked in (0, 1 << 20, 1 << 40):  # (what a program sets is the limit on every mesh)
+        d.ONE_LAUNCH_MAX_BYTES = asked
+        assert d.one_launch_limit() == asked
