@@ -255,3 +255,19 @@ def test_an_array_that_was_replaced_is_given_back(gpu_device):
     a, small, b = _native.torch_ops().upload([big, torch.zeros(9), big], gpu_device)
     del a, b
     assert torch.cuda.memory_allocated(gpu_device) - before < 1 << 20 and not small.any()
+
+
+@pytest.mark.gpu
+def test_what_a_large_transfer_brings_is_an_ordinary_tensor(gpu_device):
+    """Arrays of 32 MiB and more, cut over the threads' parts: in memory that torch can resize, as every other."""
+    import torch
+
+    from autoparallel_amd import _native
+
+    sizes = [(32 << 20) - 1, 32 << 20, (40 << 20) + 3, 100]
+    dev = [torch.randint(0, 256, (n,), dtype=torch.uint8, device=gpu_device) for n in sizes]
+    for back, there in zip(_native.torch_ops().download(dev), dev):
+        want = there.cpu()
+        assert torch.equal(back, want) and back.untyped_storage().resizable()
+        grown = back.resize_(len(back) + 5)
+        assert torch.equal(grown[:-5], want)
