@@ -682,10 +682,9 @@ Tensor edge_rows(const Tensor &edge_n_tgt) {
 
 // The value of a word on the device, once `stream` has got there.
 int32_t word_on_host(const Tensor &word, hipStream_t stream) {
-  Staging answer((int64_t)sizeof(int32_t), stream, 2);  // (with an event)
+  Staging answer((int64_t)sizeof(int32_t), stream);
   check_hip(hipMemcpyAsync(answer.slot(0), word.data_ptr(), sizeof(int32_t), hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
-  check_hip(hipEventRecord(answer.events[0], stream), "hipEventRecord");
-  check_hip(hipEventSynchronize(answer.events[0]), "hipEventSynchronize");
+  check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
   int32_t value;
   std::memcpy(&value, answer.slot(0), sizeof(value));
   return value;
