@@ -427,6 +427,9 @@ class DeviceCostTables:
         tb = self.tables
         return tb.n_entries <= self.PACKED_MAX_ENTRIES and tb.packable()
 
+    # Fewer tiles are packed by the host: 93 take it 56 us with their transfer and the device 80, 437 128 / 80.
+    PACK_ON_DEVICE_MIN_TILES = 200
+
     # (tile records, whether in launch order, the packed ones on the device), and whether those are of the tables as they are now
     _packed_cache, _packed_current = None, True
 
@@ -438,7 +441,7 @@ class DeviceCostTables:
         if cached is not None and cached[0] is tb.tile_records and (cached[1] or not repeated) and (
                 self._packed_current or torch.cuda.is_current_stream_capturing()):
             return cached[2]
-        dev, packed = self._pack_on_device(repeated)
+        dev, packed = self._pack_on_device(repeated) if tb.n_tiles >= self.PACK_ON_DEVICE_MIN_TILES else (None, False)
         if not packed:  # (the host packs them, or says which it cannot)
             dev = _to_device(tb.pack_tiles(tb.launch_records() if repeated else None), self.device)
         self._packed_cache, self._packed_current = (tb.tile_records, repeated, dev), True

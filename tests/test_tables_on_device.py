@@ -19,6 +19,7 @@ MESHES = [(8,), (12, 6), (4, 2, 2), (2, 2, 2, 2)]
 @pytest.fixture(autouse=True)
 def always_on_device(monkeypatch):
     monkeypatch.setattr(DeviceCostTables, "CHECK_ON_DEVICE_MIN_ROWS", 0)
+    monkeypatch.setattr(DeviceCostTables, "PACK_ON_DEVICE_MIN_TILES", 0)
 
 
 def _tables(mesh, seed=8):
@@ -261,3 +262,19 @@ def test_packed_tiles_are_of_the_hosts_tables(gpu_device, name):
         d._packed_cache = None
         want = tb.pack_tiles(tb.launch_records() if repeated else None).tobytes()
         assert d._packed_tiles(repeated).cpu().numpy().tobytes() == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("least", [0, 1 << 30])
+def test_packed_by_the_host_or_on_the_device(gpu_device, least, monkeypatch):
+    monkeypatch.setattr(DeviceCostTables, "PACK_ON_DEVICE_MIN_TILES", least)
+    mesh = (4, 2, 2)
+    tb = _tables(mesh)
+    tb.build_tiles(None, dedupe=True)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh), device=gpu_device)
+    on_device = []
+    monkeypatch.setattr(d, "_pack_on_device", lambda repeated: on_device.append(1) or DeviceCostTables._pack_on_device(d, repeated))
+    for repeated in (False, True):
+        want = tb.pack_tiles(tb.launch_records() if repeated else None).tobytes()
+        assert d._packed_tiles(repeated).cpu().numpy().tobytes() == want
+    assert bool(on_device) == (least == 0)
