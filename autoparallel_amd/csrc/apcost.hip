@@ -2546,14 +2546,23 @@ __global__ __launch_bounds__(kBlock) void greedy_strategies_kernel(int64_t n_nod
 }
 
 // First matrix row of every edge: one workgroup walks the edges in blocks of four a thread, whose sums are scanned across it; the next
-// block's counts are on their way meanwhile.  Bound by the chain of blocks, 2.4 us each.  (us a call with its wait, a consecutive run of
-// edges a thread / blocks / the host's sum and its transfer: 8 300 edges 19 / 18 / 26, 100 000 135 / 71 / 97, 1 000 000 2 116 / 609 / 1 110.)
+// block's counts are on their way meanwhile.  Bound by the chain of blocks, 1.8 us each.  (us a call with its wait, a consecutive run of
+// edges a thread / blocks / the host's sum and its transfer: 8 300 edges 19 / 18 / 26, 100 000 135 / 54 / 97, 1 000 000 2 116 / 464 / 1 110.)
 constexpr int kScanThreads = 1024, kScanEdges = 4;
 __global__ __launch_bounds__(kScanThreads) void edge_rows_kernel(int64_t n_edges, const int32_t *__restrict__ n_tgt, int64_t *__restrict__ begin) {
   __shared__ int64_t s_wave[2][kScanThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int32_t ahead[kScanEdges];
+  struct __attribute__((packed, aligned(4))) Counts {
+    int32_t v[kScanEdges];
+  };
   const auto fetch = [&](int64_t first) {
+    if (first + kScanEdges <= n_edges) {  // (one load: the counts may be in host memory)
+      const Counts c = *reinterpret_cast<const Counts *>(n_tgt + first);
+#pragma unroll
+      for (int k = 0; k < kScanEdges; ++k) ahead[k] = c.v[k];
+      return;
+    }
 #pragma unroll
     for (int k = 0; k < kScanEdges; ++k) ahead[k] = first + k < n_edges ? n_tgt[first + k] : 0;
   };

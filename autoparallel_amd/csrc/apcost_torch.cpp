@@ -812,22 +812,19 @@ std::tuple<std::vector<Tensor>, bool> report_tables(
                             error.data_ptr<int32_t>(), stream),
            "apc_input_tables");
   OptTensor row_begin, dup_rows, row_min, row_argmin;
-  Tensor row_begin_on_host;  // (pinned; the flag's event stands behind its copy too, and the flag goes first)
+  Tensor counts;  // (pinned; the flag's event stands behind the launch that reads them too, and the flag goes first)
   Staging flag((int64_t)sizeof(int32_t), stream, 2);  // (with an event)
-  if (edge_n_tgt.has_value() && edge_n_tgt->is_cpu()) {  // (its running sum, 8 300 edges in 8 us, behind the first launch)
+  if (edge_n_tgt.has_value() && edge_n_tgt->is_cpu()) {  // (read where they are: a copy to the device first is 10 us more)
     TORCH_CHECK(edge_n_tgt->scalar_type() == at::kInt && edge_n_tgt->is_contiguous(), "apcost: edge_n_tgt must be a contiguous int32 tensor");
     const int64_t n = edge_n_tgt->numel();
-    row_begin_on_host = at::empty({n}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
+    counts = at::empty({n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
     row_begin = empty_like_device(rank, {n}, at::kLong);
     const int32_t *n_tgt = edge_n_tgt->data_ptr<int32_t>();
-    int64_t *begin = row_begin_on_host.data_ptr<int64_t>(), sum = 0;
-    for (int64_t e = 0; e < n; ++e) {
-      begin[e] = sum;
-      sum += n_tgt[e];
-    }
+    int64_t sum = 0;
+    for (int64_t e = 0; e < n; ++e) sum += n_tgt[e];
     TORCH_CHECK(sum == n_rows, "apcost: edge_n_tgt has ", sum, " rows, n_rows says ", n_rows);
-    if (n)
-      check_hip(hipMemcpyAsync(row_begin->data_ptr(), begin, sizeof(int64_t) * (size_t)n, hipMemcpyHostToDevice, stream), "hipMemcpyAsync");
+    if (n) std::memcpy(counts.data_ptr(), n_tgt, sizeof(int32_t) * (size_t)n);
+    check_rc(apc_edge_rows(n, counts.data_ptr<int32_t>(), static_cast<int64_t *>(row_begin->data_ptr()), stream), "apc_edge_rows");
   } else if (edge_n_tgt.has_value()) {
     row_begin = edge_rows(*edge_n_tgt);
   }
