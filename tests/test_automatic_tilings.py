@@ -132,3 +132,17 @@ def test_bytes_of_the_largest_pass_in_one_launch(mesh, limit, of_many):
     for asked in (0, 1 << 20, 1 << 40):  # (what a program sets is the limit on every mesh)
         d.ONE_LAUNCH_MAX_BYTES = asked
         assert d.one_launch_limit() == asked
+
+
+@pytest.mark.parametrize("mesh,at_30,below", [((6, 4, 2), True, False), ((8, 4, 2), True, True), ((12, 6), True, True), ((3, 2, 2, 2), False, False),
+                                              ((2, 4, 2, 2), True, True)])
+def test_staging_of_small_matrices(mesh, at_30, below):
+    """Many tiled edges of few entries each, with and without copies; a pass that runs once is over packed tiles either way."""
+    tb = _table(mesh, 40, 4, False)
+    edges = 3000
+    for copies in (1, 5):
+        tb.edge_entry_begin[-1] = 30 * edges * copies
+        for computed, want in ((30 * edges, at_30), (30 * edges - 1, below)):
+            assert tb.staging_pays(computed, edges, edges) == tb._staging_may_pay(computed, edges, True) == want
+            assert tb.staging_pays(computed, edges, 0) == (want if copies == 1 or computed * 6 >= tb.n_entries else False)
+            assert not tb.staging_pays(computed, edges, edges, repeated=False)
