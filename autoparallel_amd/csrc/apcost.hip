@@ -3695,11 +3695,14 @@ static int out_mode(int mesh_ndim, const double *comm_out, const uint8_t *trans_
 //   17.2 / 21.0, 2 638 values - / 21.4 / 23.8, 3 874 values - / 29.4 / 27.3, 22 values 13.9 / 15.7 / 24.5; (8, 8, 8), 22 values
 //   17.1 / 16.1 / 24.1 us; 36 157 tiles of 149 values 46.8 / 59.4 / 96.7 there, 46.7 / 56.5 / 94.9 on (16, 8, 4), 4 123 of 139
 //   on (8, 8, 8) 16.6 / 14.3 / 17.8.
-//   ... and (a 20th of the tiles, 256 at most; 300) from the second round of its workgroups on one wavefront takes the tiles that store less
-//   than that (few rounds end with the largest tiles, which one wavefront takes longest over): us with one / two,
+//   ... and (a 20th of the tiles, 256 at most, and 256 where matrices of fewer entries have copies, 512 where they have 64 at most; 300) from the
+//   second round of its workgroups on one wavefront takes the tiles that store less than that (few rounds end with the largest tiles, which
+//   one wavefront takes longest over; a second one has no part in 64 entries, however many copies they are stored to): us with one / two,
 //   2 081 tiles of 191 values, (16, 8, 4), 7.8 / 6.4, (2, 4, 2, 2) 8.9 / 6.8, 2 650 of 166, (8, 8, 8), 8.0 / 7.4, 3 093 of 222, (32, 8), 9.8 / 8.2, (12, 6)
 //   10.0 / 9.2; the other way 2 548 of 95, (12, 6), 7.0 / 7.8, 3 334 of 146, (8, 8, 8), 8.0 / 8.9, 4 017 of 99, (64, 4), 7.4 / 8.9, (2, 4, 2, 2) 8.3 / 9.6; about
-//   equal 3 900 of 171, (8, 8, 8) 10.3 / 9.6, (12, 6) 10.0 / 10.6, 4 872 of 217, (16, 8, 4) 11.8 / 11.7, (64, 4) 11.2 / 11.4, 6 533 of 161, (8, 8, 8), 9.9 / 9.9;
+//   equal 3 900 of 171, (8, 8, 8) 10.3 / 9.6, (12, 6) 10.0 / 10.6, 4 872 of 217, (16, 8, 4) 11.8 / 11.7, (64, 4) 11.2 / 11.4, 6 533 of 161, (8, 8, 8), 9.9 / 9.9; 16
+//   copies of 8 in 2 582, (64,), 7.3 / 8.9, 12 of 18 in 2 582, (12, 6), 8.1 / 9.4, 16 9.0 / 10.1, (32, 8) 8.4 / 9.3,
+//   (2, 4, 2, 2) 9.0 / 10.0, 16 of 17 in 4 478, (8, 8, 8), 10.8 / 13.2;
 //   4 694 tiles of 129 values, (16, 8, 4), 9.4 / 10.8, 10 834 of 246, (8, 8, 8), 14.8 / 16.3, 8 566 of 207 12.6 / 13.3, 10 278 of 159, (32, 8),
 //   12.3 / 13.3, 9 426 of 200, (2, 4, 2, 2), 14.5 / 15.7, 10 278 of 266, (6,), 13.5 / 14.7, 2 906 of 5, (64,), 5.5 / 6.4; the other way 6 950 of 273,
 //   (32, 8), 13.9 / 11.3, 6 335 of 287, (16, 8, 4), 12.3 / 11.7, 9 425 of 420 18.0 / 17.1.  Not with the 72 states of a 3-D mesh to
@@ -3709,7 +3712,7 @@ static int out_mode(int mesh_ndim, const double *comm_out, const uint8_t *trans_
 //   490 7.5 / 6.7, 1 270 of 710 11.7 / 8.7).
 constexpr int64_t kTilesInOneRound = 1280;  // five workgroups of four wavefronts to a compute unit
 constexpr int64_t kSmallTilesInOneRound = 1024, kSmallTile = 448;
-constexpr int64_t kTilesOfTwoRounds = 2048, kTilesOfSomeRounds = 8192, kTilesPerValueOfOne = 20;
+constexpr int64_t kTilesOfTwoRounds = 2048, kTilesOfSomeRounds = 8192, kTilesPerValueOfOne = 20, kSideOfOne = 4;
 constexpr int64_t kTilesOfManyRounds = 16384;  // (of one wavefront: 32 workgroups to a compute unit, twice)
 
 static int tile_threads(int64_t n_tiles, int64_t n_entries, bool many_states, int64_t two, int64_t four) {
@@ -3850,10 +3853,12 @@ static int build_tables_impl(const apc_params *params, int64_t n_tensors, const 
   const int xs = xcd_shift();
   const TermLayout lay = term_layout(*params);
   const bool many_states = params->mesh_ndim == 4 && lay.exponents == 0;
+  // (about the side of a matrix: a spec is a row of one and, where it is a node's, a column of its readers')
+  const int64_t side = n_specs > 0 ? 8 * n_entries / (5 * n_specs) : 0, a_20th = n_tiles / kTilesPerValueOfOne;
   const int64_t two = n_tiles > kTilesOfManyRounds                       ? 512
                       : params->mesh_ndim == 3 && lay.exponents == 0 ? 0
                       : n_tiles > kTilesOfSomeRounds                  ? 300
-                      : n_tiles > kTilesOfTwoRounds                   ? std::min<int64_t>(256, n_tiles / kTilesPerValueOfOne)
+                      : n_tiles > kTilesOfTwoRounds                   ? (side <= kSideOfOne ? 512 : side * side < a_20th ? 256 : std::min<int64_t>(256, a_20th))
                       : params->mesh_ndim == 3                       ? 0
                                                                      : 64;
   const int threads = tile_threads(n_tiles, n_entries, many_states, two, 3072);

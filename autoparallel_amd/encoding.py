@@ -97,10 +97,12 @@ AUTO_SMALL_TABLE_ENTRIES = 4_000_000
 #   computed entries, no copies, from STAGED_MIN_COMPUTED: 366 k in 7 884 tiles on (32, 8) 16.9 / 11.4, 149 k 6.8 / 5.6, 54 k 4.9 / 4.4,
 #   409 k on (8, 8, 8) 16.0 / 10.0, 53 k 6.3 / 5.5, 836 k on (2, 4, 2, 2) 34.2 / 14.8, 337 k on (6, 4, 2) 15.8 / 12.1; about equal at
 #   46 k 4.4 / 4.4, 4 copies of 54 k 5.2 / 5.1; the other way 26 k 4.9 / 5.2, 19 k 4.0 / 4.3, 13 k 3.9 / 4.3, 2 k 3.6 / 4.2;
-#   more than STAGED_MANY_EDGES tiled edges, whatever they hold (the round of packed workgroups behind the first costs more on meshes of more
+#   more than STAGED_MANY_EDGES tiled edges, on meshes of one or two dims of at most STAGED_MAX_STORED_PER_EDGE values with their copies (the round of packed workgroups behind the first costs more on meshes of more
 #   dims: the line lies where it does on those of one): on (6,) 11 k in 2 025 4.8 / 5.0, 4 copies 5.5 / 5.4, 16 7.3 / 7.5, 20 k in 3 353 6.6 / 6.1, 24 k in
 #   4 080 7.6 / 6.3, on (64,) 15 k in 2 906 6.3 / 5.5, 16 copies 9.1 / 7.8, on (32, 8) 16 k in 2 027 5.4 / 5.0, 16 copies 7.7 / 7.2, 28 k in 3 354 7.2 / 6.3, on
-#   (8, 8, 8) 16 k in 2 030 6.0 / 5.3, 8 copies 7.1 / 6.2, on (2, 4, 2, 2) 7.0 / 5.3; the other way 5 copies of 34 k in 2 244 on (6,) 5.6 / 6.1;
+#   (8, 8, 8) 16 k in 2 030 6.0 / 5.3, 8 copies 7.1 / 6.2, on (2, 4, 2, 2) 7.0 / 5.3; the other way 5 copies of 34 k in 2 244 on (6,) 5.6 / 6.1, 337
+#   values each in 2 582 on (32, 8) 8.4 / 8.9, on (12, 6) 9.1 / 9.8, 449 9.1 / 9.8 and 9.6 / 10.6, 310 in 4 478 12.0 / 12.6 and 12.8 / 13.7 (on (8, 8, 8) 337 in 2 582
+#   9.9 / 8.9, on (2, 4, 2, 2) 12.1 / 9.6);
 #   more than STAGED_MAX_COPIES copies: 8 of 54 k in 474 5.6 / 6.1, 16 7.0 / 8.5, 16 of 109 k on (32, 8) 8.4 / 10.3, 10 of 119 k on
 #   (8, 8, 8) 7.6 / 8.7; then staged from this many computed entries on, in tiles that hold this many each, as (measured before the staging
 #   got cheaper) 901 k on (32, 8) 23.2 / 15.5, on (8, 8, 8) 28.4 / 14.7, 575 k 18.4 / 15.5, 190 k on (8, 8, 8) 9.1 / 7.1;
@@ -110,6 +112,7 @@ AUTO_SMALL_TABLE_ENTRIES = 4_000_000
 #   a 4-D mesh with a size that is no power of two, whose states cost most to stage, by the last line alone: 430 k in tiles of 91 entries
 #   25.0 / 25.7, 149 k of 94 11.3 / 11.6, 81 k of 17 15.7 / 25.2.
 STAGED_MIN_COMPUTED, STAGED_MAX_COPIES, STAGED_MANY_EDGES, STAGED_MIN_PER_EDGE_OF_STATES = 40_000, 6, 2048, 30
+STAGED_MAX_STORED_PER_EDGE = 304
 STAGED_MIN_COMPUTED_OF_COPIES, STAGED_MIN_COMPUTED_PER_TILE = 150_000, {1: 100, 2: 100, 3: 100, 4: 180}
 # Its tiles are cut until there are this many: enough workgroups for the chip, few enough stagings.  But no smaller than what
 # a STAGED_SMALLEST_SHARE-th of the entries to compute is (its power of two), at least 512: a launch is as long as its largest tile, and larger
@@ -541,7 +544,8 @@ class CostTables:
         M = len(self.mesh_sizes)
         states = M >= 3 and any(m & (m - 1) for m in self.mesh_sizes)  # (staged one by one)
         if repeated and (not states or (M == 3 and computed >= STAGED_MIN_PER_EDGE_OF_STATES * (tiled_edges or n_tiles))):
-            if tiled_edges > STAGED_MANY_EDGES or (computed >= STAGED_MIN_COMPUTED and self.n_entries <= STAGED_MAX_COPIES * computed):
+            stored = M >= 3 or self.n_entries <= STAGED_MAX_STORED_PER_EDGE * tiled_edges
+            if (tiled_edges > STAGED_MANY_EDGES and stored) or (computed >= STAGED_MIN_COMPUTED and self.n_entries <= STAGED_MAX_COPIES * computed):
                 return True
         return computed >= STAGED_MIN_COMPUTED_OF_COPIES and computed >= n_tiles * STAGED_MIN_COMPUTED_PER_TILE[M]
 
