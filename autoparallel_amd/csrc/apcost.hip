@@ -1178,10 +1178,12 @@ __device__ __forceinline__ void tensor_info_of_lanes(int rank, int itemsize, int
 // Stages tile `tile` with `nthreads` (>= 64) cooperating threads (this thread is `tid`).  The
 // caller synchronises before the stage is read.  Only global loads and LDS writes: no stores.
 // A vector load waits behind every store the compute unit has in flight, so what staging costs under a store-bound
-// kernel is the vector loads it issues: all of them at once, in one round, and each by one wavefront of the tile only.  The
-// first takes the producer specs, the image and (DERIVE) the tensor, the last the consumer specs; what is the same for all lanes comes
-// through the scalar cache.  (When every wavefront loaded everything, twelve loads each, four more cost the one launch over 66 M
-// entries in 80 layers 11 of 142 us.  us a pass, twelve loads a wavefront / five a tile: 20 M entries on (16, 8, 4) 62.6 / 61.4, 47 M in eight
+// kernel is the vector loads it issues: all of them at once, in one round, and each by one wavefront of the tile where one needs it.
+// The first takes the producer specs and the image (three loads, four on 4-D meshes) and, DERIVE, the tensor (two), the last the consumer
+// specs and their costs (three; DERIVE: nine, with what those are worked out of).  Every wavefront takes the copies' offsets, where there
+// are some (one, RM two), and DERIVE in the general layout the tensor (two), whose states all of them work out; what is the same for
+// all lanes comes through the scalar cache.  (When every wavefront loaded everything, twelve loads each, four more cost the one launch over 66 M
+// entries in 80 layers 11 of 142 us.  us a pass, everything by every wavefront / by one: 20 M entries on (16, 8, 4) 62.6 / 61.4, 47 M in eight
 // layers on (64, 4) 129.7 / 123.8, 5.9 M there 26.4 / 25.2, 1.8 M on (16, 8, 4) 14.5 / 13.4, 2.6 M on (12, 6) 11.5 / 11.4, 66 M in 80 layers
 // 127.1 / 126.4; the other way 704 k on (6, 4, 2) 11.3 / 11.6.)
 template <int M, bool DERIVE, bool RM>
@@ -1503,9 +1505,9 @@ __device__ __forceinline__ void word_slots(uint32_t src, uint32_t tgt, uint32_t 
 }
 
 // One entry of a tile whose producer specs all name one tensor.
-// What bounds a table of large tiles is the vector instructions of a SIMD, all of its cycles (20 M entries on (16, 8, 4): 27.9 M
-// instructions, 108 thousand of a SIMD's cycles in a launch of 101 thousand; now 20.4 M, 80 of 84 thousand, LDS 79 % busy), so a pass counts them:
-// 40 on a 3-D mesh with the walk and the store (54 when columns, rows and loop were kept as numbers of a lane and the codes
+// What bounds a table of large tiles: its stores, and under them the vector instructions (20 M entries on (16, 8, 4): stores alone 42 us, 23.2 M
+// instructions, 91 thousand of a SIMD's cycles or 38 us, LDS 22 us, one launch 46.5 us where the output stays in the caches and 56.8 where it
+// does not), which only partly run beside each other, so a pass counts both: 40 vector instructions on a 3-D mesh with the walk and the store (54 when columns, rows and loop were kept as numbers of a lane and the codes
 // compared by mask), and a tile's staging, which two wavefronts share, about 330 (430; 250 since the words are the launch's).  us a pass: 20 M on (16, 8, 4) 57.0 ->
 // 50.8, 5.3 M on (2, 4, 2, 2) 41.8 -> 39.4, 5.1 M on (3, 2, 2, 2) 53.2 -> 50.7, 2.6 M on (12, 6) 14.4 -> 13.4, 587 k on
 // (6, 4, 2) 16.0 -> 15.4.  (Every copy's address in scalar registers, one instruction less a store, is 1 % slower.)
@@ -2026,7 +2028,7 @@ void build_tables_kernel(APC_LAUNCH_PARAMS(BuildTablesBlock, KEPT)) {
 // A table of a few million entries is bound by the latency of one workgroup: all workgroups are
 // resident at once, stage and then store in step, and the chain of dependent loads in front of
 // the first store decides the launch.  Here a workgroup's loads depend on nothing but its index
-// (one fixed-size record per tile, copied out of the tables by the host: apc_packed_tile), and
+// (one fixed-size record per tile, copied out of the tables beforehand: apc_packed_tile), and
 // nothing is staged in LDS: lane j of every wavefront holds producer spec j, consumer spec j and
 // the compute cost / num_args of consumer strategy j; a wavefront walks whole matrix rows,
 // fetches an entry's two specs from their lanes, evaluates the entry directly

@@ -670,7 +670,7 @@ InputTables input_tables_of(const Tensor &params, const Tensor &rank, const Tens
   params, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous, spec_codes, spec_tensor, spec_outputs,           \
       shape_width, flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag
 
-// apc_input_tables: tensor table, compute costs and (with spec_outputs) the spec table in one launch.
+// The first matrix row of every edge (apc_edge_rows).
 Tensor edge_rows(const Tensor &edge_n_tgt) {
   const int32_t *nt = dev<int32_t>(edge_n_tgt, at::kInt, "edge_n_tgt");
   Tensor begin = empty_like_device(edge_n_tgt, {edge_n_tgt.numel()}, at::kLong);
@@ -849,6 +849,7 @@ std::tuple<std::vector<Tensor>, bool> report_tables(
   return {out, unsupported != 0};
 }
 
+// apc_input_tables: tensor table, compute costs and (with spec_outputs) the spec table in one launch.
 c10::intrusive_ptr<BoundLaunch> bind_input_tables(APCOST_INPUT_TABLE_PARAMS) {
   auto b = c10::make_intrusive<BoundLaunch>();
   const InputTables in = input_tables_of(APCOST_INPUT_TABLE_ARGS, b->keep);

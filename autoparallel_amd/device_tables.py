@@ -129,8 +129,11 @@ class DeviceCostTables:
             if self._packed_cache is not None:
                 self._pack_again()
 
-    # Tables of fewer rows are checked on the host: it takes 0.35 ms for 315 k specs and 15 104 edges, with their tiles 0.45 and with
-    # 15 000 copies' offsets 0.9, where a launch and the wait for its answer are 45 us.
+    # Tables of fewer rows (specs + 4 edges) are checked, and tiled by classes found, on the host; a re-tiling sends the rows for both
+    # (``send_rows``).  us, by the host / on the device, with the rows sent once for classes and check: 3.5 k rows 60 / 140, 23 k 200 / 150, 47 k
+    # 370 / 180, 94 k 600 / 215, 187 k 840 / 290, 375 k (15 104 edges, 14 160 copies) 1 350 / 470; a new table's check alone 31 / 46, 67 / 51, 110 / 57,
+    # 280 / 68, 460 / 91, 850 / 140.  The two meet at some 15 k rows; the line leaves tables with a few tenths of a ms at stake to the host, which
+    # says which row is malformed without a second look.
     CHECK_ON_DEVICE_MIN_ROWS = 60_000
 
     def _check_on_device_pays(self) -> bool:
@@ -648,7 +651,8 @@ class DeviceCostTables:
         than reading the matrices back (``row_min_in_tiles_pays``), otherwise they are taken
         when asked for.  The spec table is not part of it (the planner needed the local shard
         shapes before it could count flops); ``comm`` and ``transition`` are written only when a
-        report asks (``fetch``)."""
+        report asks (``fetch``).  The cost of a small table is of the host's tables as they are now (``prepare_step``), of any
+        other table of those uploaded last."""
         return self.prepare_step(row_min=self.row_min_in_tiles_pays(), fused_inputs=True,
                                  outputs=self.PLANNER_OUTPUTS, spec_table=False, packed=packed, repeated=repeated)
 

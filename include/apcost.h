@@ -407,7 +407,7 @@ int apc_edge_classes(int64_t n_specs, const uint32_t *spec_codes, const int32_t 
                      void *stream);
 
 /* The first matrix row of every edge, rows numbered edge by edge (apc_row_minima::edge_row_begin): edge_row_begin[e] = the
- * sum of edge_n_tgt[0 .. e). */
+ * sum of edge_n_tgt[0 .. e).  The counts may be in pinned host memory. */
 int apc_edge_rows(int64_t n_edges, const int32_t *edge_n_tgt, int64_t *edge_row_begin, void *stream);
 
 /* The ILP objective vector, summed on the device so that only one number per variable (not
