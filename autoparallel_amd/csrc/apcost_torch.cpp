@@ -802,6 +802,23 @@ std::tuple<std::vector<Tensor>, bool> report_tables(
   same_device(rank, flops, "flops");
   c10::hip::HIPGuard guard(rank.device().index());
   const hipStream_t stream = c10::hip::getCurrentHIPStream(rank.device().index()).stream();
+  OptTensor row_begin, dup_rows, row_min, row_argmin;
+  Tensor counts;  // (pinned; the flag's event stands behind the launch that reads them too, and the flag goes first)
+  Staging flag((int64_t)sizeof(int32_t), stream, 2);  // (with an event)
+  if (edge_n_tgt.has_value() && edge_n_tgt->is_cpu()) {  // (read where they are, while the launch behind is prepared: a copy first is 10 us more)
+    TORCH_CHECK(edge_n_tgt->scalar_type() == at::kInt && edge_n_tgt->is_contiguous(), "apcost: edge_n_tgt must be a contiguous int32 tensor");
+    const int64_t n = edge_n_tgt->numel();
+    counts = at::empty({n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    row_begin = empty_like_device(rank, {n}, at::kLong);
+    const int32_t *n_tgt = edge_n_tgt->data_ptr<int32_t>();
+    int32_t *to = counts.data_ptr<int32_t>();
+    int64_t sum = 0;
+    for (int64_t e = 0; e < n; ++e) sum += to[e] = n_tgt[e];
+    TORCH_CHECK(sum == n_rows, "apcost: edge_n_tgt has ", sum, " rows, n_rows says ", n_rows);
+    check_rc(apc_edge_rows(n, to, static_cast<int64_t *>(row_begin->data_ptr()), stream), "apc_edge_rows");
+  } else if (edge_n_tgt.has_value()) {
+    row_begin = edge_rows(*edge_n_tgt);
+  }
   Tensor bytes = empty_like_device(rank, {t.n}, at::kLong), contiguous = empty_like_device(rank, {t.n}, at::kByte);
   Tensor compute = empty_like_device(rank, {st.n}, at::kDouble), per_arg = empty_like_device(rank, {st.n}, at::kDouble);
   Tensor error = at::zeros({1}, rank.options().dtype(at::kInt));
@@ -811,23 +828,6 @@ std::tuple<std::vector<Tensor>, bool> report_tables(
                             dev<double>(compute, at::kDouble, "compute"), dev<double>(per_arg, at::kDouble, "per_arg"),
                             error.data_ptr<int32_t>(), stream),
            "apc_input_tables");
-  OptTensor row_begin, dup_rows, row_min, row_argmin;
-  Tensor counts;  // (pinned; the flag's event stands behind the launch that reads them too, and the flag goes first)
-  Staging flag((int64_t)sizeof(int32_t), stream, 2);  // (with an event)
-  if (edge_n_tgt.has_value() && edge_n_tgt->is_cpu()) {  // (read where they are: a copy to the device first is 10 us more)
-    TORCH_CHECK(edge_n_tgt->scalar_type() == at::kInt && edge_n_tgt->is_contiguous(), "apcost: edge_n_tgt must be a contiguous int32 tensor");
-    const int64_t n = edge_n_tgt->numel();
-    counts = at::empty({n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-    row_begin = empty_like_device(rank, {n}, at::kLong);
-    const int32_t *n_tgt = edge_n_tgt->data_ptr<int32_t>();
-    int64_t sum = 0;
-    for (int64_t e = 0; e < n; ++e) sum += n_tgt[e];
-    TORCH_CHECK(sum == n_rows, "apcost: edge_n_tgt has ", sum, " rows, n_rows says ", n_rows);
-    if (n) std::memcpy(counts.data_ptr(), n_tgt, sizeof(int32_t) * (size_t)n);
-    check_rc(apc_edge_rows(n, counts.data_ptr<int32_t>(), static_cast<int64_t *>(row_begin->data_ptr()), stream), "apc_edge_rows");
-  } else if (edge_n_tgt.has_value()) {
-    row_begin = edge_rows(*edge_n_tgt);
-  }
   check_hip(hipMemcpyAsync(flag.slot(0), error.data_ptr(), sizeof(int32_t), hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
   check_hip(hipEventRecord(flag.events[0], stream), "hipEventRecord");
   Tensor comm = empty_like_device(rank, {n_entries}, at::kDouble), transition = empty_like_device(rank, {n_entries}, at::kByte),
