@@ -125,7 +125,7 @@ class DeviceCostTables:
         if "edge_n_tgt" in names:
             self._edge_rows = None
         if not set(_PACKED).isdisjoint(names):
-            self._host_on_device = False
+            self._host_on_device = None
             if self._packed_cache is not None:
                 self._pack_again()
 
@@ -266,7 +266,7 @@ class DeviceCostTables:
             recipes.node_flop_rows.reshape(-1)), spec["local_shape"], spec["local_bytes"])
         for key, t in zip(("strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost"), out):
             self.d[key] = t
-        self._packed_current = self._host_on_device = False  # (the host's strategy table is about to change)
+        self._packed_current, self._host_on_device = False, None  # (the host's strategy table is about to change)
         return out
 
     # ---- per-strategy compute cost ---------------------------------------------------------
@@ -467,22 +467,25 @@ class DeviceCostTables:
             *(a[:tb.n_strategies] for a in tb._strategy_rows()), tb._matrix_sizes()[1], tb._records(records, tb.n_tiles, TILE_DTYPE),
             *(a[:n_dups] for a in tb._rows(n_dups, "dup_entry_begin", "dup_row_begin"))]
 
-    _host_on_device = False  # whether a preparation found the host's tables on the device, and none was uploaded since
+    _host_on_device = None  # (tile records, whether a preparation over them found the host's tables on the device), since the last upload
 
     def _staged_is_as_packed(self, capturing) -> bool:
         """Whether a pass over staged tiles, which read the tables on the device, has the results of one over packed ones, which are
-        the host's: whether no table was changed on the host and not uploaded (0.1 to 0.4 ms a preparation).  While the stream captures, as
-        an earlier preparation found it, or left it without packed tiles."""
+        the host's: whether no table was changed on the host and not uploaded.  Found once per tiling, as those are made (0.1 to 0.4 ms); while
+        the stream captures, as an earlier preparation found it, or left it without packed tiles."""
+        tb, known = self.tables, self._host_on_device
+        if known is not None and known[0] is tb.tile_records:
+            return known[1]
         if capturing:
-            return self._host_on_device or self._packed_cache is None or self._packed_cache[0] is not self.tables.tile_records
+            return self._packed_cache is None or self._packed_cache[0] is not tb.tile_records
         sent, there = self._upload(*self._packed_of(False)), [self.d[k] for k in _PACKED]
 
         def joined(arrays):
             return torch.cat([a.reshape(-1).view(torch.uint8) for a in arrays])
 
-        self._host_on_device = all(a.dtype == b.dtype and a.shape == b.shape for a, b in zip(sent, there)) and torch.equal(
-            joined(sent), joined(there))
-        return self._host_on_device
+        same = all(a.dtype == b.dtype and a.shape == b.shape for a, b in zip(sent, there)) and torch.equal(joined(sent), joined(there))
+        self._host_on_device = tb.tile_records, same
+        return same
 
     def _pack_again(self):
         """The packed tiles anew where a table they are made of was uploaded: a pass that is prepared next, also while the stream
@@ -527,8 +530,8 @@ class DeviceCostTables:
         flop / byte counts this pass reads).  ``packed``: the one launch runs over packed tiles
         (``apc_build_tables_packed``: the assembled cost and the row minima, no spec table);
         ``None`` takes them when the pass is of that kind, ``packed_pass_pays`` and staged tiles
-        (``CostTables.staging_pays``) are not faster still.  Packed tiles hold the host's tables as they are at the
-        preparation; where staged tiles are faster for the repeated pass of a small table, they are taken if the tables on the device, which
+        (``CostTables.staging_pays``) are not faster still.  Packed tiles hold the host's tables as they are at the first
+        preparation after a tiling or an upload; where staged tiles are faster for the repeated pass of a small table, they are taken if the tables on the device, which
         they read, are the same.  ``repeated=False``: the pass will run once, and the arguments
         of its launches are not laid out in device memory first (``apc_kept_launch``: one copy, for 0.75 us less a launch over packed
         tiles or a large table, nothing where staged tiles wait for other loads at that time), nor its tiles put

@@ -353,6 +353,10 @@ def test_the_default_pass_is_of_the_hosts_tables(gpu_device, name):
 
     step = d.planner_pass()
     check(step.values(), "build_tables" if name is None else "build_tables_packed")
+    tb.strat_flops[:] += 1 << 40  # (what is prepared later on the same tiling, without an upload, is of the same tables)
+    step = d.planner_pass()
+    check(step.values(), "build_tables" if name is None else "build_tables_packed")
+    tb.strat_flops[:] -= 1 << 40
     if name is not None:
         d.refresh(name)
         step = d.planner_pass()
