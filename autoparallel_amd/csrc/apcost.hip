@@ -2547,58 +2547,65 @@ __global__ __launch_bounds__(kBlock) void greedy_strategies_kernel(int64_t n_nod
   }
 }
 
-// First matrix row of every edge: one workgroup walks the edges in blocks of four a thread, whose sums are scanned across it; the next
-// block's counts are on their way meanwhile.  Bound by the chain of blocks, 1.8 us each.  (us a call with its wait, a consecutive run of
-// edges a thread / blocks / the host's sum and its transfer: 8 300 edges 19 / 18 / 26, 100 000 135 / 54 / 97, 1 000 000 2 116 / 464 / 1 110.)
-constexpr int kScanThreads = 1024, kScanEdges = 4;
+// First matrix row of every edge: one workgroup walks the edges in blocks of four a thread, four blocks at a time, whose sums are scanned
+// across it behind one barrier.  Bound by the latency of the counts, which may be in host memory.  (us a call with its wait, a consecutive
+// run of edges a thread / these / the host's sum and its transfer: 8 300 edges 19 / 18 / 25, 100 000 135 / 54 / 97, 1 000 000 2 116 / 430 / 1 110.)
+constexpr int kScanThreads = 1024, kScanEdges = 4, kScanBlocks = 4;
 __global__ __launch_bounds__(kScanThreads) void edge_rows_kernel(int64_t n_edges, const int32_t *__restrict__ n_tgt, int64_t *__restrict__ begin) {
-  __shared__ int64_t s_wave[2][kScanThreads / 64];
+  constexpr int kWaves = kScanThreads / 64;
+  constexpr int64_t kBlockEdges = kScanThreads * kScanEdges;
+  __shared__ int64_t s_wave[2][kScanBlocks][kWaves];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int32_t ahead[kScanEdges];
   struct __attribute__((packed, aligned(4))) Counts {
     int32_t v[kScanEdges];
   };
-  const auto fetch = [&](int64_t first) {
-    if (first + kScanEdges <= n_edges) {  // (one load: the counts may be in host memory)
-      const Counts c = *reinterpret_cast<const Counts *>(n_tgt + first);
-#pragma unroll
-      for (int k = 0; k < kScanEdges; ++k) ahead[k] = c.v[k];
-      return;
-    }
-#pragma unroll
-    for (int k = 0; k < kScanEdges; ++k) ahead[k] = first + k < n_edges ? n_tgt[first + k] : 0;
-  };
-  fetch((int64_t)tid * kScanEdges);
   int64_t carry = 0;
   int buffer = 0;
-  for (int64_t block = 0; block < n_edges; block += kScanThreads * kScanEdges, buffer ^= 1) {
-    const int64_t first = block + (int64_t)tid * kScanEdges;
-    int64_t rows[kScanEdges], sum = 0;
+  for (int64_t blocks = 0; blocks < n_edges; blocks += kScanBlocks * kBlockEdges, buffer ^= 1) {
+    int32_t rows[kScanBlocks][kScanEdges];
 #pragma unroll
-    for (int k = 0; k < kScanEdges; ++k) {
-      rows[k] = ahead[k];
-      sum += rows[k];
-    }
-    fetch(first + kScanThreads * kScanEdges);
-    int64_t upto = sum;  // of this wavefront's edges, this thread's included
+    for (int b = 0; b < kScanBlocks; ++b) {
+      const int64_t first = blocks + b * kBlockEdges + (int64_t)tid * kScanEdges;
+      if (first + kScanEdges <= n_edges) {
+        const Counts c = *reinterpret_cast<const Counts *>(n_tgt + first);
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int64_t o = __shfl_up(upto, off, 64);
-      if (lane >= off) upto += o;
+        for (int k = 0; k < kScanEdges; ++k) rows[b][k] = c.v[k];
+      } else {
+#pragma unroll
+        for (int k = 0; k < kScanEdges; ++k) rows[b][k] = first + k < n_edges ? n_tgt[first + k] : 0;
+      }
     }
-    if (lane == 63) s_wave[buffer][wave] = upto;
+    int64_t in_front[kScanBlocks];  // of this thread's edges, within its wavefront
+#pragma unroll
+    for (int b = 0; b < kScanBlocks; ++b) {
+      int64_t sum = 0;
+#pragma unroll
+      for (int k = 0; k < kScanEdges; ++k) sum += rows[b][k];
+      int64_t upto = sum;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int64_t o = __shfl_up(upto, off, 64);
+        if (lane >= off) upto += o;
+      }
+      if (lane == 63) s_wave[buffer][b][wave] = upto;
+      in_front[b] = upto - sum;
+    }
     __syncthreads();  // (the other buffer is written again behind the next one)
-    int64_t at = carry + upto - sum;
 #pragma unroll
-    for (int w = 0; w < kScanThreads / 64; ++w) {
-      const int64_t of_wave = s_wave[buffer][w];
-      at += w < wave ? of_wave : 0;
-      carry += of_wave;
-    }
+    for (int b = 0; b < kScanBlocks; ++b) {
+      int64_t at = carry + in_front[b];
 #pragma unroll
-    for (int k = 0; k < kScanEdges; ++k) {
-      if (first + k < n_edges) begin[first + k] = at;
-      at += rows[k];
+      for (int w = 0; w < kWaves; ++w) {
+        const int64_t of_wave = s_wave[buffer][b][w];
+        at += w < wave ? of_wave : 0;
+        carry += of_wave;
+      }
+      const int64_t first = blocks + b * kBlockEdges + (int64_t)tid * kScanEdges;
+#pragma unroll
+      for (int k = 0; k < kScanEdges; ++k) {
+        if (first + k < n_edges) begin[first + k] = at;
+        at += rows[b][k];
+      }
     }
   }
 }

@@ -334,10 +334,11 @@ class DeviceCostTables:
         row_min = self.row_min_in_tiles_pays()
         if row_min:
             tb.validate_row_minima()  # raises when some matrix row is spread over tiles
+        n_tgt = tb._rows(tb.n_edges, "edge_n_tgt", exact=True)[0] if row_min else None
         out, unsupported = self.ops.report_tables(
             self.p, *self._tensor_table(), d["spec_codes"], d["spec_tensor"], *self._strategy_table(), d["pt_values"], d["tile_records"],
-            d["dup_entry_begin"], tb.n_entries, _as_tensor(tb._rows(tb.n_edges, "edge_n_tgt", exact=True)[0]) if row_min else None, d["dup_row_begin"] if row_min else None,
-            tb.n_rows if row_min else 0)
+            d["dup_entry_begin"], tb.n_entries, *((_as_tensor(n_tgt), d["dup_row_begin"], int(n_tgt.sum(dtype=np.int64))) if row_min else
+                                                  (None, None, 0)))
         self.tensor_bytes, self.tensor_contiguous, self.compute_cost, self.compute_cost_per_arg = out[:4]
         self._check_flag(int(unsupported))
         self.comm, self.transition, self.cost = out[4:7]

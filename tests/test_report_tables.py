@@ -15,7 +15,7 @@ from oracle import cost_oracle as po
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [0, 1, 2, 1023, 1024, 1025, 4095, 4096, 4097, 8195, 210_003])
+@pytest.mark.parametrize("n", [0, 1, 2, 1023, 1024, 1025, 4095, 4096, 4097, 8195, 16_383, 16_384, 16_385, 32_771, 210_003])
 def test_first_rows_of_the_edges(gpu_device, n):
     """Sums beyond 32 bits within a thread's edges, across a wavefront, across the wavefronts and from block to block."""
     n_tgt = np.random.default_rng(n).integers(0, 90, n).astype(np.int32)
