@@ -3700,8 +3700,9 @@ static int out_mode(int mesh_ndim, const double *comm_out, const uint8_t *trans_
 //   15.2 / 10.0 / 9.9, 8 747 of 609 - / 31.3 / 37.3.
 //   Else by the values per tile: two from `two`, four from `four`.  The launch over the tables' own copies (512, 2048):
 //   1 800 values, (8, 8, 8), 169 / 154 / 179 us; 3 236 values there - / 173 / 131; 2 390 values, (32, 8), - / 32.9 / 29.2.  The launch
-//   of all tables, whose tiles derive what the other reads (64, on 3-D meshes always, with kTilesOfManyRounds 512; 3072): (32, 8), 398 values 18.5 /
-//   17.2 / 21.0, 2 638 values - / 21.4 / 23.8, 3 874 values - / 29.4 / 27.3, 22 values 13.9 / 15.7 / 24.5; (8, 8, 8), 22 values
+//   of all tables, whose tiles derive what the other reads (64, on 3-D meshes always, with kTilesOfManyRounds 512; 2304): (32, 8), 398 values 18.5 /
+//   17.2 / 21.0, 2 166 in 6 850 tiles - / 46.5 / 44.9, 2 178 in 10 836 - / 70.3 / 70.7, (16, 8, 4) - / 68.5 / 72.4, then 2 435 in 5 890, (32, 8), - / 43.7 / 40.8,
+//   2 412 in 9 235 - / 65.5 / 63.3, 2 951 in 10 165 - / 82.2 / 75.2, (16, 8, 4), 2 348 in 2 840 - / 16.3 / 16.5, 2 923 in 5 098 - / 44.1 / 41.0, 22 values 13.9 / 15.7 / 24.5; (8, 8, 8), 22 values
 //   17.1 / 16.1 / 24.1 us; 36 157 tiles of 149 values 46.8 / 59.4 / 96.7 there, 46.7 / 56.5 / 94.9 on (16, 8, 4), 4 123 of 139
 //   on (8, 8, 8) 16.6 / 14.3 / 17.8.
 //   ... and (a 20th of the tiles, 256 at most, and 256 where matrices of fewer entries have copies, 512 where they have 64 at most; 300) from the
@@ -3870,7 +3871,7 @@ static int build_tables_impl(const apc_params *params, int64_t n_tensors, const 
                       : n_tiles > kTilesOfTwoRounds                   ? (side <= kSideOfOne ? 512 : side * side < a_20th ? 256 : std::min<int64_t>(256, a_20th))
                       : params->mesh_ndim == 3                       ? 0
                                                                      : 64;
-  const int threads = tile_threads(n_tiles, n_entries, many_states, two, 3072);
+  const int threads = tile_threads(n_tiles, n_entries, many_states, two, 2304);
   const int64_t tile_blocks = ((n_tiles + (1 << xs) - 1) >> xs) << xs;
   const int64_t sb = spec_table ? blocks_for(n_specs, threads) : 0, tb = blocks_for(n_tensors, threads),
                 cb = blocks_for(n_strategies, threads);

@@ -353,6 +353,9 @@ class DeviceCostTables:
     #   up to ONE_LAUNCH_MAX_BYTES_FLAT on meshes of one or two dims, where a tile stages less: on (64, 4) 32.7 M (274 MiB) 84.5 / 85.2, 40 M
     #   (336 MiB) 109 / 114, 37.8 M in eight layers (331 MiB) 83.4 / 83.2, on (32, 8) 41.7 M (350 MiB) 112.5 / 118, 32.3 M in 40 layers 70.4 / 78.6,
     #   on (12, 6) 41.7 M 116 / 121; with three states in turn 47 M in eight layers on (64, 4) (376 MiB) 129 / 124;
+    #   with the row minima in the tiles there up to ONE_LAUNCH_MAX_BYTES_FLAT_MINIMA, three states in turn, on (32, 8) 16.3 M in 300 layers (203 MiB)
+    #   62.6 / 64.8, 18.7 M in 40 (172 MiB) 49.9 / 50.7, 25.3 M (230 MiB) 64.3 / 63.8, then 30 M (272 MiB) 75.2 / 74.0, on (64, 4) 37 M in four (324 MiB) 92.8 / 89.6, 37.8 M
+    #   in eight (331 MiB) 87.8 / 84.4;
     #   beyond ONE_LAUNCH_MAX_BYTES_OF_MANY_TILES not in more than ONE_LAUNCH_MANY_TILES, where the tiles cost what the launch saves: 44 850 tiles
     #   (above) and 46 056 116 / 121, then 49 238 on (32, 8) 55.6 / 54.5, 70 738 63.5 / 60.9, 96 217 77.8 / 72.5, 427 120 on (64, 4) 263 / 238, on (16, 8, 4)
     #   45 064 54.6 / 53.5, 70 737 61.4 / 59.4, on (6, 4, 2) 96.9 / 89.3; nor on a 4-D mesh with a size that is no power of two, whose states cost most
@@ -360,18 +363,21 @@ class DeviceCostTables:
     #   whether they can go over packed ones (5.3 M entries in 162 354 tiles lose by it, 179 / 107, measured when both took longer).
     ONE_LAUNCH_MAX_BYTES = _ONE_LAUNCH_MAX_BYTES
     ONE_LAUNCH_MAX_BYTES_FLAT = 344 << 20
+    ONE_LAUNCH_MAX_BYTES_FLAT_MINIMA = 256 << 20
     ONE_LAUNCH_MAX_BYTES_OF_MANY_TILES = 128 << 20
     ONE_LAUNCH_MANY_TILES = 48 << 10
 
-    def one_launch_limit(self) -> int:
-        """Bytes of the largest pass that is one launch: ``ONE_LAUNCH_MAX_BYTES`` where a program has set it, else by the mesh and the
-        tiles."""
+    def one_launch_limit(self, row_min_in_tiles: bool = False) -> int:
+        """Bytes of the largest pass that is one launch: ``ONE_LAUNCH_MAX_BYTES`` where a program has set it, else by the mesh, the
+        tiles and whether they take the row minima."""
         tb, limit = self.tables, self.ONE_LAUNCH_MAX_BYTES
         if limit != _ONE_LAUNCH_MAX_BYTES:
             return limit
         if tb.n_tiles > self.ONE_LAUNCH_MANY_TILES or tb._many_states():
             return self.ONE_LAUNCH_MAX_BYTES_OF_MANY_TILES
-        return self.ONE_LAUNCH_MAX_BYTES_FLAT if len(tb.mesh_sizes) <= 2 else limit
+        if len(tb.mesh_sizes) <= 2:
+            return self.ONE_LAUNCH_MAX_BYTES_FLAT_MINIMA if row_min_in_tiles else self.ONE_LAUNCH_MAX_BYTES_FLAT
+        return limit
 
     def row_min_in_tiles_pays(self) -> bool:
         """Whether the launch that writes the cost matrices should take the row minima itself.
@@ -558,7 +564,7 @@ class DeviceCostTables:
             raise ValueError("a segmented_min launch over the rows reads the cost array: ask for it")
         total = self.pass_bytes(outputs, spec_table, row_min_in_tiles)
         if one_launch is None:
-            one_launch = bool(fused_inputs) and total <= self.one_launch_limit()
+            one_launch = bool(fused_inputs) and total <= self.one_launch_limit(row_min_in_tiles)
         packed_kind = bool(one_launch) and row_min_in_tiles and outputs == ("cost",) and not spec_table
         if packed is None:
             packed = packed_kind and self.packed_pass_pays()

@@ -125,13 +125,14 @@ def test_bytes_of_the_largest_pass_in_one_launch(mesh, limit, of_many):
     d = object.__new__(DeviceCostTables)
     d.tables = _table(mesh, 40, 4, False)
     assert d.one_launch_limit() == limit << 20
+    assert d.one_launch_limit(row_min_in_tiles=True) == min(limit, 256) << 20
     d.ONE_LAUNCH_MANY_TILES = d.tables.n_tiles
     assert d.one_launch_limit() == limit << 20
     d.ONE_LAUNCH_MANY_TILES -= 1
     assert d.one_launch_limit() == of_many << 20
     for asked in (0, 1 << 20, 1 << 40):  # (what a program sets is the limit on every mesh)
         d.ONE_LAUNCH_MAX_BYTES = asked
-        assert d.one_launch_limit() == asked
+        assert d.one_launch_limit() == d.one_launch_limit(row_min_in_tiles=True) == asked
 
 
 @pytest.mark.parametrize("mesh,at_30,below", [((6, 4, 2), True, False), ((8, 4, 2), True, True), ((12, 6), True, True), ((3, 2, 2, 2), False, False),
