@@ -3461,10 +3461,368 @@ __device__ __forceinline__ bool resident_step(const ResidentLds &l, const Reside
   return true;
 }
 
+// ------------------------------------------------------------------------------------------
+// The same sweeps by teams: a matrix belongs to a team of 1, 2, 4, 8 or 16 wavefronts of a workgroup, which updates its rows
+// and its columns in turn and waits for nothing but the classes at its two ends.  (Above, a workgroup holds a run of
+// matrices and steps through the colours behind barriers: every step of it is as long as its slowest exchange.)
+//   A minimum lies in a place of two 64-bit words, each half of the value under the sweep's number: in LDS for the
+//   workgroup's teams, and in memory too where a matrix of the class lies in another workgroup.  A reader that
+//   sees the number in both words has the value: no barrier, no fence.  Two sets of places in turn, as above.
+//   What a lane needs of the plan stays in its registers over all sweeps.  All labels of a class have an incidence's minima at the
+//   same kind of place, so how many places are read, and which of them in memory, is uniform: scalar branches.
+//   The wavefronts of a team share its matrix: each counts its finished updates, and waits for the others' counts before it
+//   reads.  (The LDS operations of one wavefront complete in order.)
+//   Classes with more than four matrices: the next four places are on their way while the first four are waited for.
+// Lanes beyond a wavefront's rows repeat its last row: the same values, to the same addresses.
+// Bound by latency: an update is three round trips through LDS and some 200 instructions in a chain, 0.4 - 0.5 us, and an exchange
+// through memory 0.4 - 0.65 us more; a sweep is as long as the longest cycle of classes, three updates and more around a class
+// with many.  us a sweep, before (runs) and now: 358 matrices of at most 24 labels 5.5 -> 3.5, of at most 124 8.5 -> 6.7, 794 of 40
+// in five colours 14.7 -> 9.4, 1 098 of 12 6.0 -> 3.9, 1 428 of 64 12.0 -> 7.8.  Runs stay where one workgroup holds them all, which
+// exchanges nothing (27 matrices of at most 3 labels 2.7 against 3.3, 38 of 6 2.3 against 2.6), and where the matrices are too many.
+// Tried: any wavefront waiting per lane instead of uniformly, with the plan's rows read from LDS for every step (16 % slower than the
+// barriers); waiting wavefronts at the priority of the others (13 % slower); sleeping between two looks (no difference).
+// ------------------------------------------------------------------------------------------
+// The plan of a workgroup: as above, with [3] incidences of classes with more than four, [4] 0, [5] APC_SWEEP_TEAMS; the rows
+// team by team, the side of the lower colour first; behind the incidences, instead of steps,
+//   wavefronts   APC_SWEEP_MAX_WAVES x 4 words: first row, rows of the first side | rows of the second << 16,
+//                team | wavefront of the team << 8 | wavefronts of the team << 16 (0: idle), 0
+struct TeamLds {
+  double *m;
+  uint64_t *places;  // [row][set][2]
+  uint32_t *finished;
+  int *inc, *abort;
+  uint32_t looks;  // the clock is read at every (looks + 1)th: it takes longer than the LDS
+};
+
+__device__ __forceinline__ void keep_order() { __asm__ volatile("" ::: "memory"); }
+
+// One side of a team's matrix, as a lane sees it.
+struct TeamSide {
+  uint32_t at[4], last;  // LDS addresses of the lane's first elements, and of the row's last one
+  lds_address own;       // its row's place
+  uint32_t slot;         // its place in memory, bytes
+  uint32_t ref[4];       // the places of its class's first four incidences: LDS addresses, or bytes in memory
+  double unary;
+  bool finite;
+  int label;
+  // uniform
+  uint32_t step;  // bytes from an element of the lane to its next
+  int rounds;     // of four elements, beyond the first
+  int lanes, degree, inc;
+  int far;     // which of the first four incidences lie in memory
+  int shared;  // the own row has a place there
+  int idle;
+  double inverse;
+};
+
+// (a uniform number that the compiler has to test where it is used: hoisted out of the sweeps, the outcomes of all tests
+// took more scalar registers than there are, and came back through vector registers)
+__device__ __forceinline__ int here(int v) {
+  v = uniform_i32(v);
+  __asm__ volatile("" : "+s"(v));
+  return v;
+}
+__device__ __forceinline__ uint64_t half_under(uint32_t number, int half) { return (uint64_t)number << 32 | (uint32_t)half; }
+
+// A wait that lasts too long is given up: the workgroup's results are then not used, and what follows goes on with whatever it finds,
+// without waiting.
+struct Patience {
+  uint64_t began;
+  uint32_t tries;
+};
+__device__ __forceinline__ bool give_up(Patience &w, const TeamLds &l, uint64_t wait_ticks) {
+  if ((++w.tries & l.looks) != 0) return false;
+  const uint64_t now = (uint64_t)wall_clock64();
+  if (w.tries == l.looks + 1) w.began = now;
+  if (uniform_i32(__hip_atomic_load(l.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) == 0 && now - w.began < wait_ticks) return false;
+  __hip_atomic_store(l.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  return true;
+}
+
+struct Halves {
+  uint64_t lo, hi;
+  __device__ __forceinline__ bool of(uint32_t number) const { return (uint32_t)(lo >> 32) == number && (uint32_t)(hi >> 32) == number; }
+  __device__ __forceinline__ double value() const { return __hiloint2double((int)(uint32_t)hi, (int)(uint32_t)lo); }
+};
+__device__ __forceinline__ Halves near_place(uint32_t ref) {
+  const APC_LDS uint64_t *p = (const APC_LDS uint64_t *)(uintptr_t)ref;
+  return Halves{__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP),
+                __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)};
+}
+__device__ __forceinline__ Halves far_place(const uint64_t *slots, uint32_t ref) {
+  const uint64_t *p = reinterpret_cast<const uint64_t *>(reinterpret_cast<const char *>(slots) + ref);
+  return Halves{__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)};
+}
+
+// The minima of N incidences that all lie in LDS, added to `tot` in order.  (Where there are fewer, the last places are the own
+// row's: read, and not added.)
+template <int N>
+__device__ __forceinline__ void add_near(const TeamLds &l, uint32_t number, uint64_t wait_ticks, const uint32_t (&ref)[4], int n, double &tot) {
+  Halves h[N];
+  Patience wait{0, 0};
+  for (;;) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) h[u] = near_place(ref[u]);
+    bool there = true;
+#pragma unroll
+    for (int u = 0; u < N; ++u) there = there & h[u].of(number);
+    if (__all(there) || give_up(wait, l, wait_ticks)) break;
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u)
+    if (u < N / 2 || u < here(n)) tot += h[u].value();
+}
+
+// Four incidences (or the last n) of a class, those of `far` in memory.
+struct Four {
+  uint32_t ref[4];
+  int n, far;
+  Halves f[4];
+  __device__ __forceinline__ void fetch_far(const uint64_t *slots) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if ((here(far) >> u) & 1) f[u] = far_place(slots, ref[u]);
+  }
+  // Their minima, added to `tot` in order; the far ones are on their way.
+  __device__ __forceinline__ void add(const TeamLds &l, const uint64_t *slots, uint32_t number, uint64_t wait_ticks, double &tot) {
+    Halves h[4];
+    if (const int near = here(((1 << n) - 1) & ~far)) {
+      Patience wait{0, 0};
+      for (;;) {
+        bool there = true;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if ((here(near) >> u) & 1) h[u] = near_place(ref[u]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if ((here(near) >> u) & 1) there = there & h[u].of(number);
+        if (__all(there) || give_up(wait, l, wait_ticks)) break;
+      }
+    }
+    if (here(far)) {
+      Patience wait{0, 0};
+      for (;;) {
+        bool there = true;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if ((here(far) >> u) & 1) there = there & f[u].of(number);
+        if (__all(there) || give_up(wait, l, wait_ticks)) break;
+        fetch_far(slots);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (u < here(n)) tot += (here(far) >> u) & 1 ? f[u].value() : h[u].value();
+  }
+};
+
+// The update of one side.
+__device__ __forceinline__ void team_update(const TeamLds &l, const ResidentArgs &a, TeamSide &x, uint32_t number, int waves, uint32_t *finished,
+                                            uint32_t updates, int lane) {
+  const double inf = __builtin_inf();
+  if (here(waves) > 1) {
+    Patience wait{0, 0};
+    while ((int32_t)((uint32_t)uniform_i32((int)__hip_atomic_load(finished, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) - updates * (uint32_t)waves) < 0)
+      if (give_up(wait, l, a.wait_ticks)) break;
+    keep_order();
+  }
+  if (!here(x.idle)) {
+    double v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = lds_read<double>(x.at[u]);
+    double d = min_of(min_of(v[0], v[1]), min_of(v[2], v[3]));
+    uint32_t at = x.at[0];
+    for (int i = here(x.rounds); i > 0; --i) {
+      double w[4];
+      at += 4 * x.step;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = lds_read<double>(min(at + u * x.step, x.last));
+      d = min_of(d, min_of(min_of(w[0], w[1]), min_of(w[2], w[3])));
+    }
+    d = min_over_lanes(d, here(x.lanes));
+    const uint64_t lo = half_under(number, __double2loint(d)), hi = half_under(number, __double2hiint(d));
+    if ((lane & (x.lanes - 1)) == 0) {
+      if (here(x.shared)) {
+        uint64_t *slot = reinterpret_cast<uint64_t *>(reinterpret_cast<char *>(a.slots) + x.slot);
+        __hip_atomic_store(slot, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(slot + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      APC_LDS uint64_t *p = (APC_LDS uint64_t *)(uintptr_t)x.own;
+      __hip_atomic_store(p, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __hip_atomic_store(p + 1, hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __builtin_amdgcn_s_setprio(0);  // (who waits steps back)
+    double tot = x.unary;
+    const int degree = here(x.degree);
+    if (degree <= 2 && here(x.far) == 0) {
+      add_near<2>(l, number, a.wait_ticks, x.ref, degree, tot);
+    } else if (degree <= 4 && here(x.far) == 0) {
+      add_near<4>(l, number, a.wait_ticks, x.ref, degree, tot);
+    } else {
+      Four now{{x.ref[0], x.ref[1], x.ref[2], x.ref[3]}, min(degree, 4), x.far, {}};
+      now.fetch_far(a.slots);  // (on their way while the LDS is read)
+      for (int t = 4;; t += 4) {
+        Four next;
+        if (t < degree) {
+          int place[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) place[u] = l.inc[x.inc + min(t + u, degree - 1)];
+          next.n = min(degree - t, 4);
+          next.far = 0;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const bool is_far = (uniform_i32(place[u]) & 0x40000000) != 0;
+            next.far |= is_far && u < next.n ? 1 << u : 0;
+            next.ref[u] = ((uint32_t)(place[u] & 0x3FFFFFFF) + x.label) * 32u + (x.own & 16u) + (is_far ? 0u : address_in_lds(l.places));
+          }
+          next.fetch_far(a.slots);
+        }
+        now.add(l, a.slots, number, a.wait_ticks, tot);
+        if (t >= degree) break;
+        now = next;
+      }
+    }
+    __builtin_amdgcn_s_setprio(3);
+    const bool finite = tot < inf;  // (then every minimum of the class is finite)
+    const double share = div_by(tot, (double)degree, x.inverse);  // (the division's quotient)
+    x.unary = 0.0;  // (or +inf, where the row's elements are)
+    x.finite = finite;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) lds_write(x.at[u], finite ? (v[u] - d) + share : inf);  // (a label that can never be taken: +inf)
+    at = x.at[0];
+    for (int i = here(x.rounds); i > 0; --i) {
+      double w[4];
+      uint32_t to[4];
+      at += 4 * x.step;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) to[u] = min(at + u * x.step, x.last);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = lds_read<double>(to[u]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) lds_write(to[u], finite ? (w[u] - d) + share : inf);
+    }
+    // the other set of places
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x.ref[u] ^= 16u;
+    x.own ^= 16u;
+    x.slot ^= 16u;
+  }
+  keep_order();
+  if (here(waves) > 1 && lane == 0) __hip_atomic_fetch_add(finished, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+__device__ __forceinline__ void team_side(TeamSide &x, const TeamLds &l, const ResidentArgs &a, const int4 *rows, const int32_t *labels, int first, int n, int tid,
+                                          int threads) {
+  const int shift = n * 16 <= threads ? 4 : n * 8 <= threads ? 3 : n * 4 <= threads ? 2 : n * 2 <= threads ? 1 : 0;
+  x.lanes = 1 << shift;
+  x.idle = uniform_i32((tid & ~63) >> shift >= n);
+  const int q = first + min(tid >> shift, n - 1), sub = tid & (x.lanes - 1);
+  const int4 r = rows[2 * q], ref = rows[2 * q + 1];
+  const uint32_t places = address_in_lds(l.places);
+  const uint32_t m = address_in_lds(l.m) + 8u * (uint32_t)(r.x & 0xFFFF);
+  const int count = uniform_i32((int)((uint32_t)r.x >> 16)), stride = uniform_i32(r.y & 0xFFFF) * 8;
+  x.last = m + (uint32_t)((count - 1) * stride);
+  x.step = (uint32_t)(x.lanes * stride);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) x.at[u] = min(m + (uint32_t)((sub + u * x.lanes) * stride), x.last);
+  x.rounds = (count + 4 * x.lanes - 1) / (4 * x.lanes) - 1;
+  x.own = (lds_address)(places + 32u * (uint32_t)q);
+  x.shared = uniform_i32(r.z) >= 0;
+  x.slot = (uint32_t)max(r.z, 0) * 32u;
+  x.label = (int)((uint32_t)r.y >> 16);
+  x.inc = uniform_i32(r.w & 0xFFFF);
+  x.degree = uniform_i32((int)((uint32_t)r.w >> 16));
+  x.far = 0;
+  const int refs[4] = {ref.x, ref.y, ref.z, ref.w};
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const bool far = (uniform_i32(refs[u]) & 0x40000000) != 0;
+    x.far |= far ? 1 << u : 0;
+    x.ref[u] = u >= x.degree ? x.own : (uint32_t)(refs[u] & 0x3FFFFFFF) * 32u + (far ? 0u : places);
+  }
+  x.inverse = x.degree > 0 ? 1.0 / (double)x.degree : 0.0;
+  const int32_t label = labels[q];
+  x.unary = a.unary[label & 0x7FFFFFFF];
+  x.finite = true;
+}
+
+template <int T>
+__device__ __forceinline__ void team_sweeps(const ResidentArgs &a, unsigned char *s_bytes) {
+  const int tid = threadIdx.x;
+  // Workgroups go to the XCDs in turn; those of one XCD take consecutive parts of the plan, which share most classes (a number
+  // is there after 0.4 us within an XCD, 0.5 - 0.65 between two).
+  const unsigned xcd = blockIdx.x % 8u, share = gridDim.x / 8u, rest = gridDim.x % 8u;
+  const int32_t *plan = a.plan + a.plan_begin[xcd * share + min(xcd, rest) + blockIdx.x / 8u];
+  const int64_t first = plan[0];
+  const int n_el = plan[1], n_rows = plan[2], n_inc = plan[3];
+  // the layout of LDS (apc_sweep_plan_host counts the same bytes)
+  TeamLds l;
+  l.places = reinterpret_cast<uint64_t *>(s_bytes);
+  l.m = reinterpret_cast<double *>(l.places + 4 * n_rows);
+  l.inc = reinterpret_cast<int *>(l.m + n_el);
+  l.finished = reinterpret_cast<uint32_t *>(l.inc + n_inc);
+  l.abort = reinterpret_cast<int *>(l.finished + APC_SWEEP_MAX_WAVES);
+  l.looks = a.wait_ticks == 0 ? 0 : 15;
+  const int4 *rows = reinterpret_cast<const int4 *>(plan + 8);
+  const int32_t *labels = reinterpret_cast<const int32_t *>(rows + 2 * n_rows);
+  const int32_t *incs = labels + n_rows;
+  const int32_t *wave = incs + n_inc + 4 * uniform_i32(tid >> 6);
+  const int first_row = uniform_i32(wave[0]), n_first = uniform_i32(wave[1]) & 0xFFFF, n_second = (int)((uint32_t)uniform_i32(wave[1]) >> 16);
+  const uint32_t team = (uint32_t)uniform_i32(wave[2]);
+  const int waves = (int)(team >> 16), of_team = 64 * (int)((team >> 8) & 0xFF) + (tid & 63);
+  TeamSide x, y;
+  if (waves > 0) {
+    team_side(x, l, a, rows, labels, first_row, n_first, of_team, 64 * waves);
+    team_side(y, l, a, rows, labels, first_row + n_first, n_second, of_team, 64 * waves);
+  }
+  for (int i = tid; i < 4 * n_rows; i += T) l.places[i] = 0;
+  for (int i = tid; i < n_el; i += T) l.m[i] = a.theta[first + i];
+  for (int i = tid; i < n_inc; i += T) l.inc[i] = incs[i];
+  if (tid < APC_SWEEP_MAX_WAVES) l.finished[tid] = 0;
+  if (tid == 0) *l.abort = 0;
+  __syncthreads();
+  if (waves > 0) {
+    uint32_t *const finished = l.finished + (team & 0xFF);
+    uint32_t updates = 0;
+    __builtin_amdgcn_s_setprio(3);
+    for (int sweep = 0; sweep < a.n_sweeps; ++sweep, updates += 2) {
+      team_update(l, a, x, (uint32_t)sweep + 1, waves, finished, updates, tid & 63);
+      team_update(l, a, y, (uint32_t)sweep + 1, waves, finished, updates + 1, tid & 63);
+    }
+    __builtin_amdgcn_s_setprio(0);
+  }
+  __syncthreads();
+  if (*l.abort) {
+    if (tid == 0) __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
+  for (int i = tid; i < n_el; i += T) a.theta_out[first + i] = l.m[i];
+  if (waves > 0 && a.n_sweeps > 0) {
+    const auto store = [&](const TeamSide &s) {
+      if (s.idle || ((tid & 63) & (s.lanes - 1)) != 0) return;
+      const int32_t label = labels[(s.own - address_in_lds(l.places)) / 32u];
+      if (label < 0) a.unary_out[label & 0x7FFFFFFF] = s.finite ? 0.0 : __builtin_inf();
+    };
+    store(x);
+    store(y);
+  }
+}
+
 template <int T>
 __global__ __launch_bounds__(T) void diffusion_resident_kernel(ResidentArgs a) {
-  extern __shared__ __align__(16) unsigned char s_bytes[];
+  extern __shared__ __align__(32) unsigned char s_bytes[];
   const int tid = threadIdx.x;
+  const bool teams = a.plan[a.plan_begin[0] + 5] == APC_SWEEP_TEAMS;
+  if (teams ? T == 256 : T == 512) {  // (uniform; no plan of apc_sweep_plan_host)
+    if (tid == 0) __hip_atomic_store(a.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
+  if constexpr (T != 256) {
+    if (teams) {
+      team_sweeps<T>(a, s_bytes);
+      return;
+    }
+  }
   const int32_t *plan = a.plan + a.plan_begin[blockIdx.x];
   const int64_t first = plan[0];
   const int n_el = plan[1], n_rows = plan[2], n_inc = plan[3], n_steps = plan[4];
@@ -4237,7 +4595,8 @@ int apc_diffusion_sweeps_resident(int32_t n_sweeps, int64_t n_workgroups, const 
     return fail(-1, "apc_diffusion_sweeps_resident: %lld workgroups, 1 .. %d can be resident", (long long)n_workgroups, APC_SWEEP_MAX_WORKGROUPS);
   if (lds_bytes < 1 || lds_bytes > APC_SWEEP_LDS_BYTES)
     return fail(-1, "apc_diffusion_sweeps_resident: %lld bytes of LDS, at most %d", (long long)lds_bytes, APC_SWEEP_LDS_BYTES);
-  if (threads != 256 && threads != 1024) return fail(-1, "apc_diffusion_sweeps_resident: workgroups of 256 or 1024 threads (%d)", threads);
+  if (threads != 256 && threads != 512 && threads != 1024)
+    return fail(-1, "apc_diffusion_sweeps_resident: workgroups of 256, 512 or 1024 threads (%d)", threads);
   if (!plan || !plan_begin || !theta || !unary || !theta_out || !unary_out || !status || (n_slots > 0 && !slots))
     return fail(-1, "apc_diffusion_sweeps_resident: NULL array");
   if (theta == theta_out || unary == unary_out) return fail(-1, "apc_diffusion_sweeps_resident: the outputs are arrays of their own");
@@ -4247,11 +4606,14 @@ int apc_diffusion_sweeps_resident(int32_t n_sweeps, int64_t n_workgroups, const 
   hipLaunchKernelGGL(resident_sweeps_begin_kernel, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, s, slots, words, unary, unary_out, n_labels, status);
   // at least half a compute unit's LDS plus a little: one workgroup per compute unit
   const size_t lds = (size_t)std::max<int64_t>((lds_bytes + 15) / 16 * 16, 84 * 1024);
-  const void *kernel = threads == 256 ? reinterpret_cast<const void *>(diffusion_resident_kernel<256>) : reinterpret_cast<const void *>(diffusion_resident_kernel<1024>);
+  const void *kernel = threads == 256   ? reinterpret_cast<const void *>(diffusion_resident_kernel<256>)
+                       : threads == 512 ? reinterpret_cast<const void *>(diffusion_resident_kernel<512>)
+                                        : reinterpret_cast<const void *>(diffusion_resident_kernel<1024>);
   hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return fail(-3, "apc_diffusion_sweeps_resident: %s", hipGetErrorString(e));
   const ResidentArgs a{plan, plan_begin, theta, unary, theta_out, unary_out, slots, n_slots, wait_ticks, status, n_sweeps};
   if (threads == 256) hipLaunchKernelGGL(diffusion_resident_kernel<256>, dim3((unsigned)n_workgroups), dim3(256), lds, s, a);
+  else if (threads == 512) hipLaunchKernelGGL(diffusion_resident_kernel<512>, dim3((unsigned)n_workgroups), dim3(512), lds, s, a);
   else hipLaunchKernelGGL(diffusion_resident_kernel<1024>, dim3((unsigned)n_workgroups), dim3(1024), lds, s, a);
   return check_launch("apc_diffusion_sweeps_resident");
 }

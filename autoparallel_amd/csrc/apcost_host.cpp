@@ -1086,14 +1086,53 @@ int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin, const int
   for (int64_t k = 0; k < n_edges; ++k)
     if (edge_begin[k + 1] == edge_begin[k]) return 0;  // (an empty matrix: left to the launches)
   if (n_edges == 0) return 0;  // (no plan: sizes[0] stays 0)
+  const int64_t total = edge_begin[n_edges];
+  std::vector<int32_t> owner(n_edges);
+  int64_t lds = 0, n_wg = 0, threads = 0;
+  auto deep = [&](int64_t c) { return inc_begin[c + 1] - inc_begin[c] > 4; };
+  // By teams: a matrix has wavefronts of its own, as many as leave one `per_wave` elements and a lane a row; the workgroups
+  // take them in order.
+  struct Team {
+    int64_t first_wave, waves;
+  };
+  std::vector<Team> teams(n_edges);
+  auto team_bytes = [&](int64_t el, int64_t r, int64_t in) { return 32 * r + 8 * el + 4 * (in + APC_SWEEP_MAX_WAVES + 1); };
+  auto by_teams = [&](int64_t per_wave, int64_t most_waves) {
+    std::vector<int64_t> seen(n_classes, -1);  // the last workgroup that met the class
+    int64_t elements = 0, rows = 0, incs = 0, waves = 0, words = 0;
+    n_wg = lds = 0;
+    for (int64_t k = 0; k < n_edges; ++k) {
+      const int64_t size = edge_begin[k + 1] - edge_begin[k], ni = g.labels(edge_i[k]), nj = g.labels(edge_j[k]);
+      int64_t w = 1;
+      while (w < most_waves && (std::max(ni, nj) > 64 * w || size > per_wave * w)) w *= 2;
+      if (std::max(ni, nj) > 64 * w || (w < APC_SWEEP_MAX_WAVES && size > 2 * per_wave * w)) return false;
+      for (int attempt = 0;; ++attempt) {
+        int64_t in = incs;
+        for (int64_t c : {edge_i[k], edge_j[k]})
+          if (seen[c] != n_wg && deep(c)) in += inc_begin[c + 1] - inc_begin[c];
+        if (waves + w <= most_waves && team_bytes(elements + size, rows + ni + nj, in) <= APC_SWEEP_LDS_BYTES && elements + size <= 0x10000 && in <= 0xFFFF) {
+          teams[k] = {waves, w};
+          elements += size, rows += ni + nj, incs = in, waves += w;
+          seen[edge_i[k]] = seen[edge_j[k]] = n_wg;
+          lds = std::max(lds, team_bytes(elements, rows, incs));
+          owner[k] = (int32_t)n_wg;
+          break;
+        }
+        if (attempt == 1) return false;
+        words += 8 + 9 * rows + incs + 4 * APC_SWEEP_MAX_WAVES + 3;
+        if (++n_wg >= max_workgroups) return false;
+        elements = rows = incs = waves = 0;
+      }
+    }
+    words += 8 + 9 * rows + incs + 4 * APC_SWEEP_MAX_WAVES + 3;
+    ++n_wg;
+    return words <= capacity_words;
+  };
   // Edges in order, workgroup by workgroup, until its share of the elements, its threads (one per row of a step)
   // or its memory is full.  (Neighbouring edges of a planning program share classes: kept together, most
   // exchanges stay inside a workgroup.)  256 threads, one wavefront per SIMD, unless that takes too many workgroups.
-  const int64_t total = edge_begin[n_edges];
   int64_t share = std::max<int64_t>(APC_SWEEP_MIN_ELEMENTS, (total + APC_SWEEP_AIM_WORKGROUPS - 1) / APC_SWEEP_AIM_WORKGROUPS);
-  std::vector<int32_t> owner(n_edges);
   auto bytes = [&](int64_t el, int64_t r, int64_t in) { return 8 * (el + 1) + (32 + 8 + 8) * r + 8 * 64 + 4 * in + 4 * (n_colors + 1) + 16; };
-  int64_t lds = 0, n_wg = 0;
   auto assign = [&](int64_t threads) {
     std::vector<int64_t> seen(n_classes, -1);  // the last workgroup that met the class
     std::vector<int64_t> step_rows(n_colors, 0);
@@ -1123,12 +1162,26 @@ int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin, const int
     }
     return ++n_wg <= max_workgroups;
   };
-  // (the matrices do not fill the shares exactly: larger ones until the workgroups are few enough)
-  int64_t threads = 0;
-  for (int attempt = 0;; ++attempt, share += share / 4) {
-    threads = share > APC_SWEEP_WIDE_ELEMENTS ? 1024 : 256;
-    if (assign(threads) || assign(threads = 1024)) break;
-    if (attempt == 12) return 0;
+  // One workgroup that exchanges nothing, else teams (four wavefronts a SIMD where two make too many workgroups, and then more elements a
+  // wavefront), else runs.  (Figures at the kernels.  Eight wavefronts a workgroup against sixteen, us a sweep: 358 matrices of at
+  // most 24 labels 3.5 / 4.4, 794 of 40 9.3 / 11.0; 512 elements a wavefront against 1 024: 1 428 matrices of at most 64 labels 8.1 /
+  // 8.5, 358 of 124 6.7 / 7.4.)
+  bool of_teams = false;
+  if (total > APC_SWEEP_MIN_ELEMENTS || !assign(threads = 256) || n_wg > 1) {
+    constexpr struct {
+      int64_t waves, per_wave;
+    } kForms[] = {{APC_SWEEP_MAX_WAVES / 2, 512}, {APC_SWEEP_MAX_WAVES, 512}, {APC_SWEEP_MAX_WAVES, 1024}, {APC_SWEEP_MAX_WAVES, 2048}, {APC_SWEEP_MAX_WAVES, 4096}};
+    for (const auto &form : kForms)
+      if (!of_teams && by_teams(form.per_wave, form.waves)) {
+        of_teams = true;
+        threads = 64 * form.waves;
+      }
+    // (the matrices do not fill the shares exactly: larger ones until the workgroups are few enough)
+    for (int attempt = 0; !of_teams; ++attempt, share += share / 4) {
+      threads = share > APC_SWEEP_WIDE_ELEMENTS ? 1024 : 256;
+      if (assign(threads) || assign(threads = 1024)) break;
+      if (attempt == 12) return 0;
+    }
   }
   // classes whose matrices lie in several workgroups exchange their minima through memory: a slot per (incidence, label)
   std::vector<int64_t> slot(inc_begin[n_classes], -1);
@@ -1142,7 +1195,7 @@ int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin, const int
       n_slots += g.labels(c);
     }
   }
-  if (n_slots > 0x3FFFFFFF || total > INT32_MAX) return 0;
+  if (n_slots > (of_teams ? 0x3FFFFFF : 0x3FFFFFFF) || total > INT32_MAX) return 0;
   std::vector<int64_t> inc_of(2 * n_edges);  // (edge, side) -> incidence
   for (int64_t t = 0; t < inc_begin[n_classes]; ++t) inc_of[2 * (int64_t)inc_edge[t] + inc_side[t]] = t;
   int64_t at = 0;
@@ -1157,7 +1210,9 @@ int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin, const int
     };
     std::vector<Side> sides;
     for (int64_t k = first; k < last; ++k) sides.push_back({k, 0, edge_i[k]}), sides.push_back({k, 1, edge_j[k]});
-    std::stable_sort(sides.begin(), sides.end(), [&](const Side &x, const Side &y) { return color[x.c] < color[y.c]; });
+    std::stable_sort(sides.begin(), sides.end(), [&](const Side &x, const Side &y) {
+      return of_teams && x.k != y.k ? x.k < y.k : color[x.c] < color[y.c];
+    });
     int64_t n_rows = 0, n_inc = 0, n_el = 0;
     std::vector<int64_t> classes;
     std::vector<int64_t> steps;  // first rows of the colours that have any
@@ -1169,7 +1224,7 @@ int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin, const int
       }
       row_of[2 * x.k + x.side] = n_rows;
       n_rows += g.labels(x.c);
-      if (met[x.c] != w) {
+      if (met[x.c] != w && (!of_teams || deep(x.c))) {
         met[x.c] = w;
         classes.push_back(x.c);
         inc_at[x.c] = n_inc;
@@ -1182,7 +1237,7 @@ int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin, const int
       el_of[k - first] = n_el;
       n_el += edge_begin[k + 1] - edge_begin[k];
     }
-    const int64_t words = (8 + 9 * n_rows + n_inc + (int64_t)steps.size() + 3) / 4 * 4;
+    const int64_t words = (8 + 9 * n_rows + n_inc + (of_teams ? 4 * APC_SWEEP_MAX_WAVES : (int64_t)steps.size()) + 3) / 4 * 4;
     if (at + words > capacity_words) return fail(-1, "apc_sweep_plan_host: the plan does not fit %lld words", (long long)capacity_words);
     plan_begin[w] = at;
     int32_t *p = plan + at;
@@ -1191,7 +1246,8 @@ int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin, const int
     p[1] = (int32_t)n_el;
     p[2] = (int32_t)n_rows;
     p[3] = (int32_t)n_inc;
-    p[4] = (int32_t)steps.size() - 1;
+    p[4] = of_teams ? 0 : (int32_t)steps.size() - 1;
+    p[5] = of_teams ? APC_SWEEP_TEAMS : 0;
     int32_t *q = p + 8, *label = p + 8 + 8 * n_rows;
     // where the minima of incidence t at label 0 are: a row here, or a slot
     auto place = [&](int64_t t) {
@@ -1212,7 +1268,19 @@ int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin, const int
     q = label;
     for (int64_t c : classes)
       for (int64_t t = inc_begin[c]; t < inc_begin[c + 1]; ++t) *q++ = (int32_t)place(t);
-    for (int64_t r : steps) *q++ = (int32_t)r;
+    if (of_teams) {
+      for (size_t i = 0; i < sides.size(); i += 2) {  // (the two sides of an edge stand together)
+        const int64_t k = sides[i].k;
+        for (int64_t of_team = 0; of_team < teams[k].waves; ++of_team) {
+          int32_t *wave = q + 4 * (teams[k].first_wave + of_team);
+          wave[0] = (int32_t)row_of[2 * k + sides[i].side];
+          wave[1] = (int32_t)(uint32_t)(g.labels(sides[i].c) | g.labels(sides[i + 1].c) << 16);
+          wave[2] = (int32_t)((k - first) | of_team << 8 | teams[k].waves << 16);
+        }
+      }
+    } else {
+      for (int64_t r : steps) *q++ = (int32_t)r;
+    }
     at += words;
     first = last;
   }

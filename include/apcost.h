@@ -454,7 +454,7 @@ int apc_diffusion_sweeps(int32_t n_sweeps, int32_t n_colors, const int64_t *colo
  * sweeps instead of one launch per colour.  Out of place: theta / unary are read, theta_out / unary_out
  * written.  apc_sweep_plan_host (HOST pointers) assigns the matrices to workgroups: plan_host holds at most
  * capacity_words = 9 * (sum over edges of the label counts of both ends) + sum over edges of the degrees of both
- * ends + max_workgroups * (n_colors + 16) words, plan_begin_host max_workgroups + 1 rows; sizes_host receives
+ * ends + max_workgroups * (n_colors + 16) words (64 more for each workgroup allow every plan its faster form), plan_begin_host max_workgroups + 1 rows; sizes_host receives
  * {workgroups, words, slots, bytes of LDS, threads per workgroup}, workgroups 0 when the problem does not fit (a matrix larger than a workgroup's share of LDS, too many workgroups or
  * colours).  slots: 4 * n_slots words of device memory, cleared by the call.
  * The workgroups wait for each other's minima, so all of them have to be resident: at most
@@ -463,6 +463,8 @@ int apc_diffusion_sweeps(int32_t n_sweeps, int32_t n_colors, const int64_t *colo
  * inputs.  *status = 0: the outputs are complete. */
 #define APC_SWEEP_MAX_WORKGROUPS 224
 #define APC_SWEEP_LDS_BYTES (150 * 1024)
+#define APC_SWEEP_MAX_WAVES 16        /* wavefronts of a workgroup */
+#define APC_SWEEP_TEAMS 2             /* the form of a plan by teams (word 5 of a workgroup; 0: runs of matrices) */
 #define APC_SWEEP_MIN_ELEMENTS 256    /* a workgroup's share of the matrix elements: at least this many, */
 #define APC_SWEEP_AIM_WORKGROUPS 200  /* or what spreads the problem over this many workgroups; */
 #define APC_SWEEP_WIDE_ELEMENTS 1536  /* above this many, workgroups of 1024 threads instead of 256 */

@@ -171,3 +171,78 @@ def test_a_plan_holds_every_matrix_once_and_places_every_minimum():
     degree = np.diff(g.inc_begin)
     assert (elements == 1).all() and np.array_equal(stored, np.repeat(degree > 0, np.diff(g.label_begin)))
     assert sorted(written) == list(range(n_slots)) and all(labels == {written[s]} for s, labels in read.items())
+
+
+def _star(centre, first_leaf, n):
+    """``n`` matrices between class ``centre`` and classes ``first_leaf`` .., stored either way round."""
+    return [(centre, first_leaf + i) if i % 2 else (first_leaf + i, centre) for i in range(n)]
+
+
+# (sizes, pairs, threads of a workgroup, whether the plan is by teams)
+TEAMS = {
+    "one wavefront a matrix, rows of 1 to 64 elements": (
+        [17, 15, 64, 63, 1, 5, 33, 16, 4, 3, 2, 31], [(i, i - 1) for i in range(1, 12)], 512, True),
+    "teams of two, four and eight wavefronts": ([64, 65, 90, 60, 20, 129, 9, 65, 3], [(i, i - 1) for i in range(1, 9)], 512, True),
+    "teams of sixteen wavefronts": ([600, 3, 70, 120, 9], [(i, i - 1) for i in range(1, 5)], 1024, True),
+    "classes of 4, 5, 8, 9 and 13 matrices over several workgroups": (
+        [6 + i % 9 for i in range(60)],
+        _star(0, 5, 4) + _star(1, 9, 5) + _star(2, 14, 8) + _star(3, 22, 9) + _star(4, 31, 13) + [(i, i - 5) for i in range(31, 60)], 512, True),
+    "one wavefront more than half the workgroups' hold": ([2, 3] * 897, [(i, i - 1) for i in range(1, 1794)], 1024, True),
+    "more matrices than wavefronts": ([1, 2] * 1800, [(i, i - 1) for i in range(1, 3600)], 256, False),
+    "few elements in one workgroup": ([3] * 20, [(i, i - 1) for i in range(1, 20)], 256, False),
+}
+
+
+@pytest.mark.parametrize("name", TEAMS)
+def test_a_plan_by_teams_gives_every_row_its_wavefronts(name):
+    """On the CPU: every matrix in one team, the side of the lower colour first, a lane for every row; all rows of a side agree on
+    what the kernel takes to be uniform; the words end inside the plan and the bytes inside the LDS asked for."""
+    from autoparallel_amd.device_tables import DeviceCostTables
+
+    sizes, pairs, threads_wanted, by_teams = TEAMS[name]
+    g = _problem(1, sizes, pairs)
+    words, begin, n_slots, lds, threads = DeviceCostTables._sweep_plan(g)
+    assert threads == threads_wanted and (words[begin[:-1] + 5] == (2 if by_teams else 0)).all()
+    color = np.empty(g.n_classes, int)
+    for c in range(len(g.color_begin) - 1):
+        color[g.color_nodes[g.color_begin[c]:g.color_begin[c + 1]]] = c
+    held = np.zeros(len(g.theta), int)
+    for b, e in zip(begin[:-1], begin[1:]) if by_teams else ():
+        p = words[b:e].astype(np.int64) & 0xFFFFFFFF
+        first, n_el, n_rows, n_inc = p[:4].tolist()
+        rows, labels = p[8:8 + 8 * n_rows].reshape(-1, 8), p[8 + 8 * n_rows:8 + 9 * n_rows] & 0x7FFFFFFF
+        wave = p[8 + 9 * n_rows + n_inc:][:64].reshape(16, 4)
+        assert 32 * n_rows + 8 * n_el + 4 * (n_inc + 17) <= lds <= 150 * 1024 and not wave[threads // 64:].any()
+        classes = np.searchsorted(g.label_begin, labels, side="right") - 1
+        teams, covered = {}, np.zeros(n_rows, int)
+        for w in wave.tolist():
+            if w[2] >> 16:
+                teams.setdefault(w[2] & 0xFF, []).append((w[2] >> 8 & 0xFF, w[2] >> 16, w[0], w[1] & 0xFFFF, w[1] >> 16))
+        for t in teams.values():
+            (waves, at, n, m), = {x[1:] for x in t}
+            assert sorted(x[0] for x in t) == list(range(waves)) and 1 <= n <= 64 * waves and 1 <= m <= 64 * waves
+            covered[at:at + n + m] += 1
+            side = rows[at:at + n], rows[at + n:at + n + m]
+            assert color[classes[at]] < color[classes[at + n]] and len(set(classes[at:at + n])) == len(set(classes[at + n:at + n + m])) == 1
+            for s, other in ((side[0], m), (side[1], n)):
+                assert (s[:, 0] >> 16 == other).all() and len({(*r[[1, 3]] & [0xFFFF, -1], r[2] == 0xFFFFFFFF, *r[4:] >> 30 & 1) for r in s}) == 1
+                elements = (s[:, :1] & 0xFFFF) + np.arange(other) * (s[:, 1:2] & 0xFFFF)
+                assert len(np.unique(elements)) == n * m and elements.max() < n_el
+                np.add.at(held, first + elements.ravel(), 1)
+        assert (covered == 1).all()
+    assert (held == (2 if by_teams else 0)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", TEAMS)
+def test_sweeps_by_teams_equal_the_oracle(gpu_device, name):
+    sizes, pairs, _, _ = TEAMS[name]
+    g = _problem(len(name), sizes, pairs)
+    dev = _device()
+    theta, unary = g.theta, g.unary
+    want = (g.theta, g.unary)
+    for n in (1, 2, 5):
+        theta, unary = dev.diffusion_sweeps(g, theta, unary, n)
+        want = _sweep(g, *want, n)
+        assert dev._diffusion_graph["plan"] is not None  # (no wait expired)
+        assert np.array_equal(theta, want[0]) and np.array_equal(unary, want[1])
