@@ -147,6 +147,7 @@ def cluster_regions(graph: torch.fx.Graph, strats: dict) -> dict:
     from torch._dynamo.graph_region_tracker import (InputPickler, _populate_recursive_ancestor_map,
                                                     fully_expand_region_group)
     from torch._inductor.codecache import sha256_hash
+    from torch.distributed.tensor._op_schema import OpStrategy
 
     rank = {node: i for i, node in enumerate(graph.nodes)}
     ancestors = _populate_recursive_ancestor_map(graph)
@@ -157,11 +158,26 @@ def cluster_regions(graph: torch.fx.Graph, strats: dict) -> dict:
             return a.meta.get("val")
         return a if isinstance(a, (torch.Tensor, int)) else None
 
+    # Nodes of one operator and metadata share their strategies' objects: each list is written out once.  Equal texts are one
+    # object, so that the bytes a key is pickled to, which tell an object met before from a new one, follow from its contents.
+    written: dict = {}
+    texts: dict = {}
+
+    def text_of(what, strategy):
+        key = (what, *map(id, strategy.strategies))
+        if key not in written:
+            text = what(strategy)
+            written[key] = texts.setdefault(text, text)
+        return written[key]
+
     def strategy_text(node):
         s = strats.get(node)
+        if type(s) is OpStrategy:
+            return text_of(str, s)
         if s is None and node.op == "output":  # (the reference keys the output node by its producers' strategies)
             s = [strats[x] for x in node.all_input_nodes]
-        return str(s)
+        text = str(s)
+        return texts.setdefault(text, text)
 
     same_key = defaultdict(list)
     group_of = {}
@@ -173,7 +189,7 @@ def cluster_regions(graph: torch.fx.Graph, strats: dict) -> dict:
         key = (node.meta.get("stack_trace"),
                (tuple(sorted(node.kwargs)), tuple(arg_value(a) for a in flat_args + flat_kwargs)),
                strategy_text(node),
-               tuple(_output_placements(strats[p]) for p in node.all_input_nodes))
+               tuple(text_of(_output_placements, strats[p]) for p in node.all_input_nodes))
         bucket = same_key[sha256_hash(pickler.dumps(key))]
         bucket.append(node)
         group_of[node] = bucket

@@ -100,6 +100,7 @@ def drop_uneven_shardings(strategy: OpStrategy, mesh) -> OpStrategy:
     """Keeps a strategy only if every Shard of every input and output spec divides its
     tensor dim evenly, mesh dim after mesh dim (propagation_rules.py:104-135)."""
     kept = []
+    sizes = tuple(mesh.shape)  # (worked out anew by every look at the mesh: a fifth of an enumeration when asked for every spec)
     for s in strategy.strategies:
         out = s.output_specs
         if isinstance(out, DTensorSpec):
@@ -113,7 +114,7 @@ def drop_uneven_shardings(strategy: OpStrategy, mesh) -> OpStrategy:
             if spec is None:
                 continue
             shape = list(spec.tensor_meta.shape)
-            for n, p in zip(mesh.shape, spec.placements):
+            for n, p in zip(sizes, spec.placements):
                 if p.is_shard():
                     if shape[p.dim] % n == 0:
                         shape[p.dim] //= n

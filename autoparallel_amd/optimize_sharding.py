@@ -1182,7 +1182,8 @@ class ShardingOptimizer:
         """Sum over parameters of (local size / global size) stays within [low, high] x #params."""
         from torch._functorch._aot_autograd.fx_utils import get_param_nodes
 
-        world_size = math.prod(self.mesh.shape)
+        sizes = tuple(self.mesh.shape)
+        world_size = math.prod(sizes)
         cols, vals = [], []
         considered = 0
         per_node = []
@@ -1197,7 +1198,7 @@ class ShardingOptimizer:
                 spec: DTensorSpec = self.strats[node].strategies[oi].input_specs[0]
                 shape = list(spec.tensor_meta.shape)
                 old = math.prod(shape)
-                for n, p in zip(self.mesh.shape, spec.placements):
+                for n, p in zip(sizes, spec.placements):
                     if p.is_shard():
                         shape[p.dim] = (shape[p.dim] + n - 1) // n
                 cols.append(b + oi * ns)
