@@ -2547,6 +2547,51 @@ __global__ __launch_bounds__(kBlock) void greedy_strategies_kernel(int64_t n_nod
   }
 }
 
+// Several arrays in one launch, kCopyUnit bytes of one a workgroup, in pieces of 16 bytes where both its ends allow it.  For what travels
+// between device and pinned host memory together: bound by the bus, and behind it by what every copy of the runtime costs, some
+// 10 us between two of them.  us until the stream has finished, the runtime's copies / this: five arrays of 4 KB 21 / 12, of 64 KB 50 / 18, of 1 MB 137 /
+// 106; 84 MB to the host in parts of 2 MB with an event each 2 150 / 1 810 (one copy of all: 1 550).  (4, 16, 32 and 64 KB a
+// workgroup: 1 770 / 1 810 to the host, 2 460 / 1 910 from it, larger ones as 16.)
+constexpr int kCopyUnit = 16384;
+struct CopyArrays {
+  const char *from[APC_COPY_MAX_ARRAYS];
+  char *to[APC_COPY_MAX_ARRAYS];
+  int64_t bytes[APC_COPY_MAX_ARRAYS];
+  int32_t first_block[APC_COPY_MAX_ARRAYS];
+  int32_t n;
+};
+template <typename V>
+__device__ __forceinline__ void copy_unit(const char *from, char *to, int n) {  // n bytes, at most kCopyUnit
+  constexpr int kAhead = 4, kRound = kAhead * kBlock;  // loads a thread issues before it waits for the first
+  const V *x = reinterpret_cast<const V *>(from);
+  V *y = reinterpret_cast<V *>(to);
+  const int whole = n / (int)sizeof(V), tid = threadIdx.x;
+  for (int base = 0; base < whole; base += kRound) {
+    V v[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (const int i = base + u * kBlock + tid; i < whole) v[u] = x[i];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+      if (const int i = base + u * kBlock + tid; i < whole) y[i] = v[u];
+  }
+  if (const int i = whole * (int)sizeof(V) + tid; i < n) to[i] = from[i];  // (fewer than 16)
+}
+__global__ __launch_bounds__(kBlock) void copy_arrays_kernel(CopyArrays a) {
+  const int lane = threadIdx.x & 63, b = (int)blockIdx.x;
+  // the last array that begins at this workgroup or before (none is empty)
+  const int k = uniform_i32(__popcll(__ballot(lane < a.n && a.first_block[min(lane, APC_COPY_MAX_ARRAYS - 1)] <= b))) - 1;
+  if (k < 0) return;
+  const int64_t at = (int64_t)(b - a.first_block[k]) * kCopyUnit;
+  const int n = (int)min((int64_t)kCopyUnit, a.bytes[k] - at);
+  const char *from = a.from[k] + at;
+  char *to = a.to[k] + at;
+  const uint32_t low = (uint32_t)(reinterpret_cast<uintptr_t>(from) | reinterpret_cast<uintptr_t>(to));
+  if ((low & 15) == 0) copy_unit<u32x4>(from, to, n);
+  else if ((low & 3) == 0) copy_unit<uint32_t>(from, to, n);
+  else copy_unit<uint8_t>(from, to, n);
+}
+
 // First matrix row of every edge: one workgroup walks the edges in blocks of four a thread, four blocks at a time, whose sums are scanned
 // across it behind one barrier.  Bound by the latency of the counts, which may be in host memory.  (us a call with its wait, a consecutive
 // run of edges a thread / these / the host's sum and its transfer: 8 300 edges 19 / 18 / 25, 100 000 135 / 54 / 97, 1 000 000 2 116 / 430 / 1 110.)
@@ -4451,6 +4496,28 @@ int apc_edge_rows(int64_t n_edges, const int32_t *edge_n_tgt, int64_t *edge_row_
   if (!edge_n_tgt || !edge_row_begin) return fail(-1, "apc_edge_rows: NULL array");
   hipLaunchKernelGGL(edge_rows_kernel, dim3(1), dim3(kScanThreads), 0, (hipStream_t)stream, n_edges, edge_n_tgt, edge_row_begin);
   return check_launch("apc_edge_rows");
+}
+
+int apc_copy_arrays(int64_t n, const void *const *from_host, void *const *to_host, const int64_t *bytes_host, void *stream) {
+  if (n < 0 || n > APC_COPY_MAX_ARRAYS) return fail(-1, "apc_copy_arrays: %lld arrays, at most %d", (long long)n, APC_COPY_MAX_ARRAYS);
+  if (n > 0 && (!from_host || !to_host || !bytes_host)) return fail(-1, "apc_copy_arrays: NULL array");
+  CopyArrays a{};
+  int64_t blocks = 0;
+  for (int64_t k = 0; k < n; ++k) {
+    if (bytes_host[k] < 0) return fail(-1, "apc_copy_arrays: array %lld has a negative size", (long long)k);
+    if (bytes_host[k] == 0) continue;
+    if (!from_host[k] || !to_host[k]) return fail(-1, "apc_copy_arrays: array %lld is NULL", (long long)k);
+    if (bytes_host[k] > (int64_t)INT32_MAX * kCopyUnit || (blocks + (bytes_host[k] + kCopyUnit - 1) / kCopyUnit) > INT32_MAX)
+      return fail(-1, "apc_copy_arrays: too many bytes for one launch");
+    a.from[a.n] = static_cast<const char *>(from_host[k]);
+    a.to[a.n] = static_cast<char *>(to_host[k]);
+    a.bytes[a.n] = bytes_host[k];
+    a.first_block[a.n++] = (int32_t)blocks;
+    blocks += (bytes_host[k] + kCopyUnit - 1) / kCopyUnit;
+  }
+  if (blocks == 0) return 0;
+  hipLaunchKernelGGL(copy_arrays_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, (hipStream_t)stream, a);
+  return check_launch("apc_copy_arrays");
 }
 
 int apc_check_tables(const apc_params *params, int32_t with_rows, int64_t n_tensors, const int32_t *tensor_rank, int64_t n_specs,

@@ -410,6 +410,11 @@ int apc_edge_classes(int64_t n_specs, const uint32_t *spec_codes, const int32_t 
  * sum of edge_n_tgt[0 .. e).  The counts may be in pinned host memory. */
 int apc_edge_rows(int64_t n_edges, const int32_t *edge_n_tgt, int64_t *edge_row_begin, void *stream);
 
+/* Arrays copied in one launch: bytes_host[k] bytes from from_host[k] to to_host[k] (HOST tables of n addresses and sizes, read before the
+ * call returns), any of the arrays in pinned host memory.  No two of them overlap. */
+#define APC_COPY_MAX_ARRAYS 32
+int apc_copy_arrays(int64_t n, const void *const *from_host, void *const *to_host, const int64_t *bytes_host, void *stream);
+
 /* The ILP objective vector, summed on the device so that only one number per variable (not
  * three arrays per entry) has to leave it.
  * Replaces the accumulation at optimize_sharding.py:650-655 (opt_target[va] += cost over

@@ -214,3 +214,47 @@ def test_malformed_tables_raise_runtime_error_through_the_operator(mutate, messa
     else:
         with pytest.raises(RuntimeError, match=message):
             call()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [(1,), (16_384,), (0, 15, 16, 17), (16_383, 16_385, 1), (100_003, 3, 0, 64 * 1024), (5,) * 32])
+@pytest.mark.parametrize("offset", [0, 1, 4, 8])
+def test_copy_arrays_moves_every_byte_and_no_other(gpu_device, sizes, offset):
+    """apc_copy_arrays to pinned memory, on the device and back: workgroups that end inside an array, pieces of 16, 4 and 1 bytes."""
+    import ctypes
+
+    lib = _native.lib()
+    gap = 48  # (a multiple of 16: every array has the offset's alignment)
+    begins = np.cumsum([0] + [(n + 15) // 16 * 16 + gap for n in sizes]) + offset
+    total = int(begins[-1]) + 64
+    want = torch.from_numpy(np.random.default_rng(len(sizes)).integers(0, 255, total, dtype=np.uint8))
+    source, buffers = want.to(gpu_device), [torch.full((total,), 255, dtype=torch.uint8, pin_memory=True),
+                                            torch.full((total,), 255, dtype=torch.uint8, device=gpu_device)]
+    stream = torch.cuda.current_stream(gpu_device).cuda_stream
+
+    def copy(to, src):
+        n = len(sizes)
+        address = lambda t: (ctypes.c_void_p * n)(*(t.data_ptr() + int(b) for b in begins[:-1]))  # noqa: E731
+        _native.check(lib.apc_copy_arrays(ctypes.c_int64(n), address(src), address(to), (ctypes.c_int64 * n)(*sizes), ctypes.c_void_p(stream)),
+                      "apc_copy_arrays")
+
+    copy(buffers[0], source)
+    copy(buffers[1], buffers[0])
+    torch.cuda.synchronize()
+    moved = np.zeros(total, bool)
+    for b, n in zip(begins, sizes):
+        moved[b:b + n] = True
+    for buffer in buffers:
+        got = buffer.cpu().numpy()
+        assert np.array_equal(got[moved], want.numpy()[moved]) and (got[~moved] == 255).all()
+
+
+def test_copy_arrays_refuses_what_a_launch_cannot_hold():
+    import ctypes
+
+    lib = _native.lib()
+    one = (ctypes.c_void_p * 33)(*range(16, 16 + 33))
+    for n, sizes in ((33, [1] * 33), (-1, [1]), (1, [-1]), (1, [1 << 50])):
+        assert lib.apc_copy_arrays(ctypes.c_int64(n), one, one, (ctypes.c_int64 * 33)(*sizes), None) != 0
+    assert lib.apc_copy_arrays(ctypes.c_int64(1), None, one, (ctypes.c_int64 * 1)(1), None) != 0
+    assert lib.apc_copy_arrays(ctypes.c_int64(2), one, one, (ctypes.c_int64 * 2)(0, 0), None) == 0
