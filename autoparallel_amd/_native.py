@@ -111,6 +111,7 @@ EXPORTS = (
     "apc_refine_labels_host",
     "apc_prune_masks_host",
     "apc_build_tables_packed",
+    "apc_build_tables_packed_small",
     "apc_keep_next_launch",
     "apc_run_kept",
     "apc_calibrate_launch",

@@ -2069,12 +2069,12 @@ __device__ __forceinline__ FlatConstants<M> flat_constants(const apc_params &p) 
 // not branched on: the ring term of the one collective the dim can need (none: + 0.0, which
 // leaves a non-negative sum unchanged), 0, 1 or 2 read+write reshuffles ((double)copies x rw:
 // 0.0, rw, 2.0 x rw).  FIRST = 1 (2-D meshes): dim 1 before dim 0 (:146-151).  CONT: the tensor
-// is contiguous (no lane ever adds the non-contiguity term).  gb = bytes / num_shards / 1024^3.
+// is contiguous (no lane ever adds the non-contiguity term); else `contiguous`: whether the lane's is.  gb = bytes / num_shards / 1024^3.
 template <int M, int FIRST, bool CONT>
 __device__ __forceinline__ double entry_cost_flat(uint32_t srcp, uint32_t tgtp, double gb, const apc_params &p,
-                                                  const FlatConstants<M> &k) {
+                                                  const FlatConstants<M> &k, bool contiguous = false) {
   double cost = 0.0;
-  bool banned = false, cont = CONT;
+  bool banned = false, cont = CONT || contiguous;
   bool tgt_partial = false;
 #pragma unroll
   for (int s = 0; s < M; ++s) {
@@ -2123,9 +2123,10 @@ struct Pow2Constants {
 };
 
 template <int M, int FIRST, bool CONT>
-__device__ __forceinline__ double entry_cost_pow2(uint32_t srcp, uint32_t tgtp, int j, double a2a_scale, const Pow2Constants<M> &k) {
+__device__ __forceinline__ double entry_cost_pow2(uint32_t srcp, uint32_t tgtp, int j, double a2a_scale, const Pow2Constants<M> &k,
+                                                  bool contiguous = false) {
   double cost = 0.0;
-  bool banned = false, cont = CONT, tgt_partial = false;
+  bool banned = false, cont = CONT || contiguous, tgt_partial = false;
 #pragma unroll
   for (int s = 0; s < M; ++s) {
     const int i = (M == 2 && FIRST == 1) ? 1 - s : s;
@@ -2187,10 +2188,10 @@ struct PackedArgs {
   int32_t exponents, lg_total, lg[APC_MAX_MESH];
 };
 
-template <int M, bool POW2>
+template <int M, bool POW2, bool ALONE>  // ALONE: a wavefront takes the tile, else those of the workgroup
 __device__ __forceinline__ void packed_tile(const apc_packed_tile *T, double *cost_out, const PackedArgs &a) {
   const apc_params &p = a.p;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = ALONE ? 0 : tid >> 6, waves = ALONE ? 1 : blockDim.x >> 6;
   // ---- the one round of loads: nothing here depends on another load ---------------------------
   const i32x16 h = uniform_load(reinterpret_cast<const i32x16 *>(T));
   const int64_t dim_size = T->tensor_shape[lane & (APC_MAX_RANK - 1)], dim_stride = T->tensor_stride[lane & (APC_MAX_RANK - 1)];
@@ -2347,6 +2348,255 @@ __device__ __forceinline__ void packed_tile(const apc_packed_tile *T, double *co
   }
 }
 
+// ------------------------------------------------------------------------------------------
+// The same pass over small tiles: kLanes (16 or 32) lanes take a tile, a wavefront four or two.  A tile costs a wavefront some 900
+// instructions, eleven arrays to fetch and what the dispatcher does for it whether it has four entries or 256: from a few thousand tiles on
+// that, and not latency, is the launch.  Everything that is wave-uniform above is a lane's own here: the record's words and the copies' offsets by
+// DPP broadcasts within 16 lanes, each of which fetches them; a lane's row and column by quotients, and whole rows go round by round, though one round
+// (1.5 us: a chain of bpermutes and fp64, few wavefronts to hide it) is what the host takes few lanes for (CostTables.packed_lanes).
+// us a pass before (the faster of a workgroup a tile and of staged tiles) / now: 4 292 tiles of at most 16 entries on (64,) 6.5 / 4.2, 5 770 on (12, 6)
+// 9.1 / 5.5, 2 908 on (3, 2, 2, 2) 10.2 / 5.8; with 32 lanes 4 644 of at most 25 on (16, 8, 4) 7.4 / 6.4, 4 693 on (3, 2, 2, 2) 15.1 / 9.5.
+// ------------------------------------------------------------------------------------------
+static_assert(APC_PACKED_MAX_DUPS == 16 && APC_MAX_RANK <= 16, "16 lanes hold a tile's dims, identical edges and the first words of its record");
+
+// The value of lane N of the lane's row of 16 (DPP row_newbcast:N).
+template <int N>
+__device__ __forceinline__ int of_lane16(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, 0x150 + N, 0xF, 0xF, true);
+}
+template <int N>
+__device__ __forceinline__ int64_t of_lane16(int64_t x) {
+  return (int64_t)((uint64_t)(uint32_t)of_lane16<N>((int)((uint64_t)x >> 32)) << 32 | (uint32_t)of_lane16<N>((int)(uint32_t)x));
+}
+// The largest over the four tiles of a value that their 16 lanes share.
+__device__ __forceinline__ int most_of_tiles(int x) {
+  return max(max(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 16)),
+             max(__builtin_amdgcn_readlane(x, 32), __builtin_amdgcn_readlane(x, 48)));
+}
+
+// tensor_info_of_lanes, every 16 lanes of their own tensor.
+__device__ __forceinline__ void tensor_info_of_lanes16(int rank, int itemsize, int64_t x, int64_t y, int lane, double &bytes, bool &contiguous) {
+  const int dim = lane & 15;
+  const bool live = dim < min(rank, APC_MAX_RANK);
+  const double size = live ? (double)x : 1.0;
+  double product = size;
+  product *= from_lane_behind<1>(product, 1.0);
+  product *= from_lane_behind<2>(product, 1.0);
+  product *= from_lane_behind<4>(product, 1.0);
+  const double expected = from_lane_behind<1>(product, 1.0);
+  const bool differs = size != 1.0 && (double)y != expected;
+  const int shift = lane & 48;
+  contiguous = ((__ballot(differs) >> shift) & 0xFFFF) == 0;
+  const double total = __hiloint2double(of_lane16<0>(__double2hiint(product)), of_lane16<0>(__double2loint(product))) * (double)itemsize;
+  bytes = total;
+  const uint64_t odd = __ballot(!(size >= 1.0) || !(product < 0x1p53) || !(total < 0x1p53));
+  if (odd != 0) {  // (uniform)
+    int64_t nbytes = itemsize, one = 1, most = 1;
+    bool dims_contiguous = true;
+#pragma unroll 1
+    for (int i = APC_MAX_RANK - 1; i >= 0; --i) {
+      const int64_t xi = from_lane_i64(x, shift + i), yi = from_lane_i64(y, shift + i);  // (every lane takes part)
+      if (i >= rank) continue;
+      nbytes *= xi;
+      if (xi == 1) continue;
+      if (yi != one && yi != most) dims_contiguous = false;
+      most *= xi > 1 ? xi : 1;
+      one *= xi;
+    }
+    if (((odd >> shift) & 0xFFFF) != 0) {
+      bytes = (double)nbytes;
+      contiguous = dims_contiguous;
+    }
+  }
+}
+
+__device__ __forceinline__ void store_at(double *to, double value) {  // written through, as above
+  __asm__ volatile("global_store_dwordx2 %0, %1, off sc0 sc1" ::"v"(to), "v"(value) : "memory");
+}
+// x / y for 0 <= x <= 32, 1 <= y <= 32: x + 0.5 is nowhere nearer to a multiple of y than half of one, the reciprocal as good as exact
+__device__ __forceinline__ int small_quotient(int x, float inverse) { return (int)(((float)x + 0.5f) * inverse); }
+
+template <int D>
+__device__ __forceinline__ void store_copies16(int64_t entry0, double *cost_out, int64_t local, int dup_count, int most_dups, bool active, double total) {
+  if constexpr (D < APC_PACKED_MAX_DUPS) {
+    if (D >= most_dups) return;  // (uniform)
+    double *const to = cost_out + (of_lane16<D>(entry0) + local);
+    if (active && D < dup_count) store_at(to, total);
+    store_copies16<D + 1>(entry0, cost_out, local, dup_count, most_dups, active, total);
+  }
+}
+
+// `first`: the wavefront's first tile.
+template <int M, bool POW2, int kLanes>
+__device__ __forceinline__ void packed_small_tiles(const apc_packed_tile *tiles, int first, int n_tiles, double *cost_out, const PackedArgs &a) {
+  const apc_params &p = a.p;
+  const int lane = threadIdx.x & 63, sub = lane & (kLanes - 1), first_lane = lane & (64 - kLanes);
+  const int tile = first + lane / kLanes;
+  // ---- the one round of loads -------------------------------------------------------------------
+  const char *const T = reinterpret_cast<const char *>(tiles + min(tile, n_tiles - 1));
+  const char *const T4 = T + sub * 4, *const T8 = T + sub * 8, *const of_16 = T + (lane & 15) * 8, *const dims = T + (sub & (APC_MAX_RANK - 1)) * 8;
+#define APC_OF(TYPE_, BASE_, FIELD_) (*reinterpret_cast<const TYPE_ *>((BASE_) + offsetof(apc_packed_tile, FIELD_)))
+  const int h = *reinterpret_cast<const int32_t *>(T + (lane & 15) * 4);
+  const int64_t dim_size = APC_OF(int64_t, dims, tensor_shape), dim_stride = APC_OF(int64_t, dims, tensor_stride);
+  TileCopies copies;
+  copies.entry0 = APC_OF(int64_t, of_16, dup_entry_begin);
+  copies.row0 = APC_OF(int64_t, of_16, dup_row_begin);
+  copies.row_out = 0;
+  const uint32_t col_code = APC_OF(uint32_t, T4, col_codes), row_code = APC_OF(uint32_t, T4, row_codes);
+  const int col_tensor = APC_OF(int32_t, T4, col_tensor), row_tensor = APC_OF(int32_t, T4, row_tensor);
+  const int64_t row_flops = APC_OF(int64_t, T8, row_flops), row_rw = APC_OF(int64_t, T8, row_rw_bytes);
+  const int row_meta = APC_OF(int32_t, T4, row_meta);
+#undef APC_OF
+  const double gf_of_lane = a.p.gpu_flops[lane & (APC_MAX_DTYPES - 1)], inv_gf_of_lane = a.p.inv_gpu_flops[lane & (APC_MAX_DTYPES - 1)];
+  fetch_arguments_now(a.row_min_out, a.row_arg_out, p.hbm_bw, p.inv_hbm_bw, p.rw_eff, p.inv_rw_eff, p.launch_floor, p.compute_eff,
+                      p.inv_compute_eff, a.inv_rescale, p.rescale, p.a2a_scale, p.base_latency);
+  int rows = of_lane16<0>(h);
+  const int cols = of_lane16<1>(h), flags = of_lane16<2>(h), dup_count = of_lane16<3>(h), t0 = of_lane16<4>(h);
+  if (tile >= n_tiles || (unsigned)rows > (unsigned)kLanes || (unsigned)(cols - 1) >= (unsigned)kLanes || (unsigned)dup_count > (unsigned)APC_PACKED_MAX_DUPS)
+    rows = 0;  // none, or no small tile
+  const int64_t entry_begin = (int64_t)((uint64_t)(uint32_t)of_lane16<9>(h) << 32 | (uint32_t)of_lane16<8>(h));
+  const int64_t row_begin = (int64_t)((uint64_t)(uint32_t)of_lane16<11>(h) << 32 | (uint32_t)of_lane16<10>(h));
+  // ---- the tensor's bytes, the rows' compute costs ------------------------------------------------
+  double fbytes;
+  bool contiguous;
+  tensor_info_of_lanes16(of_lane16<5>(h), of_lane16<6>(h), dim_size, dim_stride, lane, fbytes, contiguous);
+  const int dt = (int)(int8_t)(row_meta & 0xFF);
+  const bool known_dtype = dt >= 0 && dt < APC_MAX_DTYPES;
+  const double gf = from_lane(gf_of_lane, dt & (APC_MAX_DTYPES - 1)), inv_gf = from_lane(inv_gf_of_lane, dt & (APC_MAX_DTYPES - 1));
+  const double cpa = compute_cost_through_reciprocals(p, ((row_meta >> 8) & 0xFF) != 0, row_rw, row_flops, known_dtype ? gf : 0.0,
+                                                      known_dtype ? inv_gf : 0.0) /
+                     (double)(row_meta >> 16);  // (lanes past the tile's rows: never read)
+  settle(copies);
+  FlatConstants<M> k;
+  Pow2Constants<M> k2;
+  if constexpr (!POW2) k = flat_constants<M>(p);
+  if constexpr (POW2) {
+    k2.R = div_by(div_by(fbytes, p.hbm_bw, p.inv_hbm_bw) * 1e6, p.rw_eff, p.inv_rw_eff);
+    k2.rw_shift = 1 - a.lg_total;
+    k2.floor = p.launch_floor;
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+      const double hops1 = (double)(p.mesh_size[i] - 1), hops2 = (double)(2 * (p.mesh_size[i] - 1));
+      k2.B[i] = div_by(fbytes * hops1, p.bw[i], p.inv_bw[i]) * 1e6;
+      k2.lat1[i] = p.base_latency + hops1 * p.lat[i];
+      k2.lat2[i] = p.base_latency + hops2 * p.lat[i];
+      k2.lg[i] = a.lg[i];
+      k2.shift[i] = -a.lg_total - 30 - a.lg[i];
+    }
+  }
+  // ---- whole rows, `cols` lanes a row ---------------------------------------------------------------
+  const float inv_cols = __builtin_amdgcn_rcpf((float)cols);
+  const int rows_per_pass = rows > 0 ? small_quotient(kLanes, inv_cols) : 1;
+  const int r_local = small_quotient(sub, inv_cols), c = sub - r_local * cols;
+  const bool in_pass = r_local < rows_per_pass;
+  // (the stores of the row minima: lane -> (row of the pass, copy))
+  const float inv_rows = __builtin_amdgcn_rcpf((float)rows_per_pass);
+  const int copies_per_store = small_quotient(kLanes, inv_rows);
+  const int copy_slot = small_quotient(sub, inv_rows), q = sub - copy_slot * rows_per_pass;
+  const int q_first_lane = first_lane + q * cols;
+  const bool rescale = (flags & APC_EDGE_GRAD_RESCALE) != 0, no_producer = (flags & APC_EDGE_NO_PRODUCER) != 0;
+  const bool entry_by_entry = (flags & APC_PACKED_MIXED) != 0 || no_producer || t0 < 0;
+  const bool all_contiguous = __ballot(rows > 0 && !contiguous) == 0;
+  const int most_dups = most_of_tiles(rows > 0 ? dup_count : 0), most_cols = most_of_tiles(rows > 0 ? cols : 1);
+  for (int row0 = 0; __ballot(row0 < rows) != 0; row0 += rows_per_pass) {
+    const int r = row0 + r_local;
+    const bool active = in_pass && r < rows;
+    const uint32_t src = (uint32_t)from_lane((int)col_code, first_lane + c), tgt = (uint32_t)from_lane((int)row_code, first_lane + (r & (kLanes - 1)));
+    const double row_cpa = from_lane(cpa, first_lane + (r & (kLanes - 1)));
+    const int64_t local = entry_begin + (r * cols + c);
+    const bool flip = M == 2 && src == 0x4040u && ((tgt >> 6) & 3u) == 2u && ((tgt >> 14) & 3u) == 2u;
+    const bool some_flip = M == 2 && __ballot(flip && active) != 0;  // (Partial, Partial) -> all Shard walks dim 1 first (:146-151)
+    double comm;
+    if constexpr (POW2) {
+      int j = a.lg_total;  // bytes / num_shards = bytes x 2^(j - L)
+#pragma unroll
+      for (int i = 0; i < M; ++i) j -= ((src >> (8 * i + 6)) & 3u) == 2u ? k2.lg[i] : 0;
+      comm = all_contiguous ? entry_cost_pow2<M, 0, true>(src, tgt, j, p.a2a_scale, k2) : entry_cost_pow2<M, 0, false>(src, tgt, j, p.a2a_scale, k2, contiguous);
+      if (some_flip) {
+        const double other = entry_cost_pow2<M, 1, false>(src, tgt, j, p.a2a_scale, k2, contiguous);
+        comm = flip ? other : comm;
+      }
+    } else {
+      double shards = 1.0;  // exact: a product of mesh sizes (torch _dtensor_spec.py:555-561)
+#pragma unroll
+      for (int i = 0; i < M; ++i) shards *= ((src >> (8 * i + 6)) & 3u) == 2u ? (double)p.mesh_size[i] : 1.0;
+      const double gb = fbytes / shards * 0x1p-30;  // / 1024 / 1024 / 1024 (:66-68)
+      comm = all_contiguous ? entry_cost_flat<M, 0, true>(src, tgt, gb, p, k) : entry_cost_flat<M, 0, false>(src, tgt, gb, p, k, contiguous);
+      if (some_flip) {
+        const double other = entry_cost_flat<M, 1, false>(src, tgt, gb, p, k, contiguous);
+        comm = flip ? other : comm;
+      }
+    }
+    int trans = src != tgt ? p.transition_scale : 0;  // optimize_sharding.py:345-351
+    // :358-359; the quotient through the reciprocal is the division's (div_by), +inf stays +inf
+    if (rescale) comm = comm < __builtin_inf() ? div_by(comm, p.rescale, a.inv_rescale) : comm;
+    if (__ballot(active && entry_by_entry) != 0) {  // pass-through edges, and tiles whose specs are not all DTensorSpecs on one tensor
+      const int sten = from_lane(col_tensor, first_lane + c), tten = from_lane(row_tensor, first_lane + (r & (kLanes - 1)));
+      const int64_t pt_begin = (int64_t)((uint64_t)(uint32_t)of_lane16<13>(h) << 32 | (uint32_t)of_lane16<12>(h));  // (every lane takes part)
+      if (active && entry_by_entry) {
+        trans = 0;
+        if (no_producer || sten < 0 || tten < 0) {
+          comm = a.pt_values[pt_begin + (r * cols + c)];
+        } else {
+          trans = src != tgt ? p.transition_scale : 0;
+          int64_t shards = 1;
+#pragma unroll
+          for (int i = 0; i < M; ++i)
+            if (kind_of((src >> (8 * i)) & 0xFF) == 2) shards *= p.mesh_size[i];
+          int64_t sten_bytes;
+          bool sten_contiguous;
+          tensor_bytes_and_contiguity(a.rank[sten], a.itemsize[sten], a.shape + (int64_t)sten * APC_MAX_RANK,
+                                      a.stride + (int64_t)sten * APC_MAX_RANK, sten_bytes, sten_contiguous);
+          const double gb = (double)sten_bytes / (double)shards / 1024 / 1024 / 1024;
+          comm = entry_cost<M>(src, tgt, gb, sten_contiguous, p);
+        }
+        if (rescale) comm = comm / p.rescale;
+      }
+    }
+    const double total = comm + row_cpa + (double)trans;  // optimize_sharding.py:368-372
+    // ---- the entry, to the tile's edge and to every identical edge ------------------------------------
+    if (active) store_at(cost_out + local, total);
+    store_copies16<0>(copies.entry0, cost_out, local - entry_begin, dup_count, most_dups, active, total);
+    // ---- the rows' minima (row_min_in_wave, within 16 lanes) -------------------------------------------
+    double m = active ? total : __builtin_inf();
+    int mc = c;
+#define APC_ROW_MIN_STEP(N_)                                        \
+  if (N_ < most_cols) {                                             \
+    const double om = from_lane_ahead<N_>(m);                       \
+    const int oc = from_lane_ahead<N_>(mc);                         \
+    if ((sub & 15) + N_ < 16 && c + N_ < cols && om < m) {                 \
+      m = om;                                                       \
+      mc = oc;                                                      \
+    }                                                               \
+  }
+    APC_ROW_MIN_STEP(1)
+    APC_ROW_MIN_STEP(2)
+    APC_ROW_MIN_STEP(4)
+    APC_ROW_MIN_STEP(8)
+#undef APC_ROW_MIN_STEP
+    if constexpr (kLanes == 32) {
+      const double pm = from_lane(m, first_lane + 16);
+      const int pc = from_lane(mc, first_lane + 16);
+      if (sub < 16 && c + 16 - sub < cols && pm < m) {
+        m = pm;
+        mc = pc;
+      }
+    }
+    const double m_q = from_lane(m, q_first_lane);
+    const int mc_q = from_lane(mc, q_first_lane);
+    const bool row_live = row0 + q < rows && copy_slot < copies_per_store;
+    for (int copy0 = 0; __ballot(row_live && copy0 <= dup_count) != 0; copy0 += copies_per_store) {
+      const int copy = copy0 + copy_slot;
+      const int64_t first_row = from_lane_i64(copies.row0, first_lane + ((copy - 1) & 15));  // (every lane takes part)
+      if (row_live && copy <= dup_count) {
+        const int64_t out = (copy == 0 ? row_begin : first_row) + row0 + q;
+        a.row_min_out[out] = m_q;
+        a.row_arg_out[out] = mc_q;
+      }
+    }
+  }
+}
+
 struct PackedBlock {
   PackedArgs a;
   apc_params p;
@@ -2355,14 +2605,24 @@ struct PackedBlock {
   int64_t tensor_blocks;
 };
 
-template <int M, bool POW2, bool KEPT>
+template <int M, bool POW2, bool KEPT, int LANES>  // LANES a tile
 __global__ __launch_bounds__(kBlock) void build_tables_packed_kernel(APC_LAUNCH_PARAMS(PackedBlock, KEPT)) {
   const PackedBlock &k = launch_block<KEPT>(kept);
   const int64_t b = blockIdx.x;
   if (b < tile_blocks) {
-    const int tile_id = tile_of_block((int)b, n_tiles, xcd_shift);
-    if (tile_id >= n_tiles) return;
-    packed_tile<M, POW2>(static_cast<const apc_packed_tile *>(work) + tile_id, cost_out, k.a);
+    const apc_packed_tile *const tiles = static_cast<const apc_packed_tile *>(work);
+    if constexpr (LANES == kBlock) {
+      const int tile_id = tile_of_block((int)b, n_tiles, xcd_shift);
+      if (tile_id >= n_tiles) return;
+      packed_tile<M, POW2, false>(tiles + tile_id, cost_out, k.a);
+    } else {
+      constexpr int per_block = kBlock / LANES;
+      const int n_groups = (n_tiles + per_block - 1) / per_block, group = tile_of_block((int)b, n_groups, xcd_shift);
+      const int first = group * per_block + uniform_i32((int)threadIdx.x >> 6) * (64 / LANES);
+      if (group >= n_groups || first >= n_tiles) return;
+      if constexpr (LANES == 64) packed_tile<M, POW2, true>(tiles + first, cost_out, k.a);
+      else packed_small_tiles<M, POW2, LANES>(tiles, first, n_tiles, cost_out, k.a);
+    }
     return;
   }
   const int64_t tb = b - tile_blocks;
@@ -4770,7 +5030,7 @@ static int build_tables_packed_impl(const apc_params *params, int64_t n_tensors,
                             int64_t n_strategies, const int64_t *flops, const int64_t *rw_bytes, const int8_t *dtype,
                             const uint8_t *zero_cost, const int32_t *num_args, double *compute, double *per_arg,
                             int32_t *error_flag, const double *pt_values, int64_t n_tiles, const apc_packed_tile *packed,
-                            int64_t n_entries, double *cost_out, double *row_min, int32_t *row_argmin,
+                            int64_t n_entries, double *cost_out, double *row_min, int32_t *row_argmin, int lanes,
                                     const LaunchTo &to) {
   if (int rc = check_params(params)) return rc;
   if (n_tensors < 0 || n_strategies < 0 || n_entries < 0) return fail(-1, "apc_build_tables_packed: negative count");
@@ -4783,7 +5043,10 @@ static int build_tables_packed_impl(const apc_params *params, int64_t n_tensors,
     return fail(-1, "apc_build_tables_packed: NULL tile records or outputs");
   if ((reinterpret_cast<uintptr_t>(packed) & 63) != 0) return fail(-1, "apc_build_tables_packed: packed tiles must be 64-byte aligned");
   const int xs = xcd_shift();
-  const int64_t tile_blocks = ((n_tiles + (1 << xs) - 1) >> xs) << xs;
+  if (lanes != 16 && lanes != 32 && lanes != 64 && lanes != kBlock)
+    return fail(-1, "apc_build_tables_packed: 16, 32, 64 or %d lanes a tile (got %d)", kBlock, lanes);
+  const int64_t groups = blocks_for(n_tiles, kBlock / lanes);
+  const int64_t tile_blocks = ((groups + (1 << xs) - 1) >> xs) << xs;
   const int64_t tb = blocks_for(n_tensors, kBlock), cb = blocks_for(n_strategies, kBlock);
   const int64_t blocks = tile_blocks + tb + cb;
   if (blocks == 0) return 0;
@@ -4796,10 +5059,12 @@ static int build_tables_packed_impl(const apc_params *params, int64_t n_tensors,
   const ComputeCostArgs ca{n_strategies, flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag};
   const PackedBlock block{a, *params, ta, ca, tb};
   using K = TableKernel<PackedBlock>;
-#define APC_LAUNCH_PACKED(M_)                                                                                             \
-  return launch_table_kernel("apc_build_tables_packed", to,                                                             \
-                             lay.exponents ? K{build_tables_packed_kernel<M_, true, false>, build_tables_packed_kernel<M_, true, true>}     \
-                                           : K{build_tables_packed_kernel<M_, false, false>, build_tables_packed_kernel<M_, false, true>}, \
+#define APC_PACKED_FORM(M_, POW2_, LANES_) \
+  K { build_tables_packed_kernel<M_, POW2_, false, LANES_>, build_tables_packed_kernel<M_, POW2_, true, LANES_> }
+#define APC_PACKED_FORMS(M_, POW2_) \
+  (lanes == 16 ? APC_PACKED_FORM(M_, POW2_, 16) : lanes == 32 ? APC_PACKED_FORM(M_, POW2_, 32) : lanes == 64 ? APC_PACKED_FORM(M_, POW2_, 64) : APC_PACKED_FORM(M_, POW2_, kBlock))
+#define APC_LAUNCH_PACKED(M_)                                                                                                         \
+  return launch_table_kernel("apc_build_tables_packed", to, lay.exponents ? APC_PACKED_FORMS(M_, true) : APC_PACKED_FORMS(M_, false), \
                              (unsigned)blocks, kBlock, 0, packed, (int)n_tiles, xs, tile_blocks, cost_out, block)
   switch (params->mesh_ndim) {
     case 1: APC_LAUNCH_PACKED(1);
@@ -4808,6 +5073,8 @@ static int build_tables_packed_impl(const apc_params *params, int64_t n_tensors,
     default: APC_LAUNCH_PACKED(4);
   }
 #undef APC_LAUNCH_PACKED
+#undef APC_PACKED_FORMS
+#undef APC_PACKED_FORM
 }
 
 extern "C" {
@@ -4820,7 +5087,18 @@ int apc_build_tables_packed(const apc_params *params, int64_t n_tensors, const i
                             int64_t n_entries, double *cost_out, double *row_min, int32_t *row_argmin, void *stream) {
   return build_tables_packed_impl(params, n_tensors, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous, n_strategies,
                                   flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag, pt_values, n_tiles, packed,
-                                  n_entries, cost_out, row_min, row_argmin, launch_to(stream));
+                                  n_entries, cost_out, row_min, row_argmin, kBlock, launch_to(stream));
+}
+
+int apc_build_tables_packed_small(const apc_params *params, int64_t n_tensors, const int32_t *rank, const int32_t *itemsize,
+                            const int64_t *shape, const int64_t *stride, int64_t *tensor_bytes, uint8_t *tensor_contiguous,
+                            int64_t n_strategies, const int64_t *flops, const int64_t *rw_bytes, const int8_t *dtype,
+                            const uint8_t *zero_cost, const int32_t *num_args, double *compute, double *per_arg,
+                            int32_t *error_flag, const double *pt_values, int64_t n_tiles, const apc_packed_tile *packed,
+                            int64_t n_entries, double *cost_out, double *row_min, int32_t *row_argmin, int32_t lanes_per_tile, void *stream) {
+  return build_tables_packed_impl(params, n_tensors, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous, n_strategies,
+                                  flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag, pt_values, n_tiles, packed,
+                                  n_entries, cost_out, row_min, row_argmin, lanes_per_tile, launch_to(stream));
 }
 
 }  // extern "C"

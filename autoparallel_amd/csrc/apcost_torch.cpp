@@ -935,7 +935,7 @@ c10::intrusive_ptr<BoundLaunch> bind_cost_tables_packed(const Tensor &params, co
                                                         const Tensor &num_args, const Tensor &compute, const Tensor &per_arg,
                                                         const Tensor &error_flag, const Tensor &pt_values, const Tensor &packed,
                                                         int64_t n_entries, int64_t n_rows, const Tensor &cost,
-                                                        const Tensor &row_min, const Tensor &row_argmin) {
+                                                        const Tensor &row_min, const Tensor &row_argmin, int64_t lanes) {
   auto b = c10::make_intrusive<BoundLaunch>();
   const apc_params p = params_of(params);
   const TensorTable t = tensor_table(rank, itemsize, shape, stride);
@@ -967,9 +967,12 @@ c10::intrusive_ptr<BoundLaunch> bind_cost_tables_packed(const Tensor &params, co
   b->recordable = true;
   b->device = rank.device();
   b->launch = [=](void *s) {
-    return apc_build_tables_packed(&p, t.n, t.rank, t.itemsize, t.shape, t.stride, bytes, contiguous, st.n, st.flops, st.rw_bytes,
-                                   st.dtype, st.zero_cost, st.num_args, cc, cpa, err, pt, n_tiles, tiles, n_entries, cost_out, mins,
-                                   args, s);
+#define APCOST_PACKED_ARGS                                                                                                              \
+  &p, t.n, t.rank, t.itemsize, t.shape, t.stride, bytes, contiguous, st.n, st.flops, st.rw_bytes, st.dtype, st.zero_cost, st.num_args, cc, cpa, \
+      err, pt, n_tiles, tiles, n_entries, cost_out, mins, args
+    if (lanes != 0) return apc_build_tables_packed_small(APCOST_PACKED_ARGS, (int32_t)lanes, s);
+    return apc_build_tables_packed(APCOST_PACKED_ARGS, s);
+#undef APCOST_PACKED_ARGS
   };
   return b;
 }
@@ -1377,7 +1380,7 @@ TORCH_LIBRARY(apcost, m) {
         &bind_cost_tables);
   m.def("bind_cost_tables_packed(Tensor params, " APCOST_TENSOR_TABLE ", Tensor tensor_bytes, Tensor tensor_contiguous, "
         APCOST_STRATEGY_TABLE ", Tensor compute_cost, Tensor compute_cost_per_arg, Tensor error_flag, Tensor pt_values, "
-        "Tensor packed, int n_entries, int n_rows, Tensor cost, Tensor row_min, Tensor row_argmin) "
+        "Tensor packed, int n_entries, int n_rows, Tensor cost, Tensor row_min, Tensor row_argmin, int lanes_per_tile=0) "
         "-> __torch__.torch.classes.apcost.BoundLaunch",
         &bind_cost_tables_packed);
 }

@@ -440,7 +440,8 @@ class DeviceCostTables:
     # Fewer tiles are packed by the host: 93 take it 56 us with their transfer and the device 80, 437 128 / 80.
     PACK_ON_DEVICE_MIN_TILES = 200
 
-    # (tile records, whether in launch order, the packed ones on the device), and whether those are of the tables as they are now
+    # (tile records, whether in launch order, the packed ones on the device, lanes that take one), and whether those are of the tables as
+    # they are now
     _packed_cache, _packed_current = None, True
 
     def _packed_tiles(self, repeated):
@@ -451,10 +452,11 @@ class DeviceCostTables:
         if cached is not None and cached[0] is tb.tile_records and (cached[1] or not repeated) and (
                 self._packed_current or torch.cuda.is_current_stream_capturing()):
             return cached[2]
+        lanes = tb.packed_lanes()
         dev, packed = self._pack_on_device(repeated) if tb.n_tiles >= self.PACK_ON_DEVICE_MIN_TILES else (None, False)
         if not packed:  # (the host packs them, or says which it cannot)
             dev = _to_device(tb.pack_tiles(tb.launch_records() if repeated else None), self.device)
-        self._packed_cache, self._packed_current = (tb.tile_records, repeated, dev), True
+        self._packed_cache, self._packed_current = (tb.tile_records, repeated, dev, lanes), True
         return dev
 
     def _pack_on_device(self, repeated):
@@ -497,16 +499,17 @@ class DeviceCostTables:
     def _pack_again(self):
         """The packed tiles anew where a table they are made of was uploaded: a pass that is prepared next, also while the stream
         captures, finds them.  (Launches bound earlier keep theirs.)"""
-        records, repeated, _ = self._packed_cache
+        records, repeated, *_ = self._packed_cache
         self._packed_cache = None
         if records is not self.tables.tile_records:
             return
+        lanes = self.tables.packed_lanes()
         try:
             dev, packed = self._pack_on_device(repeated)
         except ValueError:  # (host tables of different lengths: one of several that are being replaced)
             return
         if packed:
-            self._packed_cache, self._packed_current = (records, repeated, dev), True
+            self._packed_cache, self._packed_current = (records, repeated, dev, lanes), True
 
     def _tile_records(self, repeated):
         """The device copy of the tile records, in launch order for a pass that is repeated: of the tiling that is on the
@@ -537,7 +540,7 @@ class DeviceCostTables:
         flop / byte counts this pass reads).  ``packed``: the one launch runs over packed tiles
         (``apc_build_tables_packed``: the assembled cost and the row minima, no spec table);
         ``None`` takes them when the pass is of that kind, ``packed_pass_pays`` and staged tiles
-        (``CostTables.staging_pays``) are not faster still.  Packed tiles hold the host's tables as they are at the first
+        (``CostTables.staging_pays``, ``small_packing_pays``) are not faster still.  Packed tiles hold the host's tables as they are at the first
         preparation after a tiling or an upload; where staged tiles are faster for the repeated pass of a small table, they are taken if the tables on the device, which
         they read, are the same.  ``repeated=False``: the pass will run once, and the arguments
         of its launches are not laid out in device memory first (``apc_kept_launch``: one copy, for 0.75 us less a launch over packed
@@ -568,7 +571,9 @@ class DeviceCostTables:
         packed_kind = bool(one_launch) and row_min_in_tiles and outputs == ("cost",) and not spec_table
         if packed is None:
             packed = packed_kind and self.packed_pass_pays()
-            if packed and (self._edge_rows is not None or not capturing):
+            small = packed and tb.small_packing_pays() and (not capturing or (
+                self._packed_cache is not None and self._packed_cache[0] is tb.tile_records))
+            if packed and not small and (self._edge_rows is not None or not capturing):
                 of_tiles = tb.computed_entries(), tb.n_tiles
                 packed = not (tb.staging_pays(*of_tiles, repeated=False) or (
                     not runs_once and tb.staging_pays(*of_tiles) and self._staged_is_as_packed(capturing)))
@@ -612,10 +617,11 @@ class DeviceCostTables:
         erb, rmin, rarg = rows if rows is not None else (None, None, None)
         dup_rows = d["dup_row_begin"] if rows is not None else None
         if packed:
+            tiles = self._packed_tiles(repeated)
             step = {"build_tables_packed": bind(ops.bind_cost_tables_packed(
                 self.p, *self._tensor_table(), self.tensor_bytes, self.tensor_contiguous, *self._strategy_table(),
-                self.compute_cost, self.compute_cost_per_arg, err, d["pt_values"], self._packed_tiles(repeated), tb.n_entries, tb.n_rows,
-                self.cost, self.row_min, self.row_argmin))}
+                self.compute_cost, self.compute_cost_per_arg, err, d["pt_values"], tiles, tb.n_entries, tb.n_rows,
+                self.cost, self.row_min, self.row_argmin, self._packed_cache[3]))}
         elif one_launch:
             step = {"build_tables": bind(ops.bind_cost_tables(
                 *input_tables, d["pt_values"], self._tile_records(repeated), d["dup_entry_begin"], tb.n_entries, self.comm,

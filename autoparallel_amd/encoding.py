@@ -113,6 +113,19 @@ AUTO_SMALL_TABLE_ENTRIES = 4_000_000
 #   25.0 / 25.7, 149 k of 94 11.3 / 11.6, 81 k of 17 15.7 / 25.2.
 STAGED_MIN_COMPUTED, STAGED_MAX_COPIES, STAGED_MANY_EDGES, STAGED_MIN_PER_EDGE_OF_STATES = 40_000, 6, 2048, 30
 STAGED_MAX_STORED_PER_EDGE = 304
+# Packed tiles of few entries.  A workgroup of four wavefronts a tile (256 lanes) leaves lanes idle where the rows of every tile are
+# evaluated at once by fewer: then 64, and from more than PACKED_MANY_TILES on, where at most PACKED_MAX_SMALL_COPIES values are stored for one
+# computed, 32 or 16.  us, 256 / 64 / 32 / 16 lanes: tiles of at most 16 entries, 436 on (64,) 3.3 / 3.4 / 3.7 / 3.6, 1 928 4.7 / 3.7 / 3.8 / 3.8,
+# 2 906 6.2 / 4.2 / 4.2 / 3.7, 3 488 in two layers on (6,) 7.1 / 5.2 / 4.7 / 4.0, 3 158 of nine copies 7.5 / 5.9 / - / 6.3, 926 of sixteen 5.7 / 5.2 / 6.0 / 6.0; of at
+# most 25, 1 446 on (16, 8, 4) 5.1 / 4.4 / 4.4, 4 644 10.8 / 8.0 / 6.4, 4 693 on (3, 2, 2, 2) 15.1 / 11.4 / 9.5, 2 596 of twenty copies on (3, 8) 8.1 / 7.0 / 7.4; of
+# at most 64, 944 of sixteen copies on (32, 8) 5.9 / 5.3, 4 297 on (8, 8, 8) 10.0 / 7.8, 5 571 on (3, 2, 2, 2) 17.2 / 12.8.  Where a wavefront
+# goes over its tile twice it loses (944 tiles of at most 81 entries on (32, 8) 6.1 / 6.9, 4 297 of 100 9.3 / 8.0 with 7.3 staged), but on
+# meshes whose states are staged one by one and that leave no other choice (2 910 of at most 100 on (3, 2, 2, 2) 11.9 / 10.1, 3 720 of 81 on (6, 4, 2)
+# 12.2 / 11.1).
+# They beat staged tiles (same cases: 5.4 / 3.7 for 2 906 tiles of 16 entries, 7.3 / 6.4 for 4 644 of 25, 7.4 / 6.0 for 2 188 of 64 and ten copies, 12.7 / 9.7
+# for 5 571 of 64 on (6, 4, 2)) except, with 64 lanes, PACKED_MANY_TILES_OF_64 and more without copies on power-of-two meshes of
+# three dims or four (staged / packed: 2 910 6.2 / 6.1 on (2, 4, 2, 2), 5.9 / 5.4 on (16, 8, 4); then 4 297 7.3 / 7.8 on (8, 8, 8), 7.5 / 9.3 on (2, 4, 2, 2)).
+PACKED_MANY_TILES, PACKED_MAX_SMALL_COPIES, PACKED_MANY_TILES_OF_64 = 2048, 4, 3072
 STAGED_MIN_COMPUTED_OF_COPIES, STAGED_MIN_COMPUTED_PER_TILE = 150_000, {1: 100, 2: 100, 3: 100, 4: 180}
 # Its tiles are cut until there are this many: enough workgroups for the chip, few enough stagings.  But no smaller than what
 # a STAGED_SMALLEST_SHARE-th of the entries to compute is (its power of two), at least 512: a launch is as long as its largest tile, and larger
@@ -542,12 +555,45 @@ class CostTables:
         if tiled_edges is None:
             tiled_edges = (self.tiling or {}).get("tiled_edges", 0)
         M = len(self.mesh_sizes)
-        states = M >= 3 and any(m & (m - 1) for m in self.mesh_sizes)  # (staged one by one)
+        states = self._states_one_by_one()
         if repeated and (not states or (M == 3 and computed >= STAGED_MIN_PER_EDGE_OF_STATES * (tiled_edges or n_tiles))):
             stored = M >= 3 or self.n_entries <= STAGED_MAX_STORED_PER_EDGE * tiled_edges
             if (tiled_edges > STAGED_MANY_EDGES and stored) or (computed >= STAGED_MIN_COMPUTED and self.n_entries <= STAGED_MAX_COPIES * computed):
                 return True
         return computed >= STAGED_MIN_COMPUTED_OF_COPIES and computed >= n_tiles * STAGED_MIN_COMPUTED_PER_TILE[M]
+
+    def packed_lanes(self, records: Optional[np.ndarray] = None) -> int:
+        """Lanes a packed tile is evaluated by (above: PACKED_MANY_TILES), for the tiling's records or the ``records`` given."""
+        counts = (self.tile_records if records is None else records)["counts"]
+        rows, cols = counts & 0xFFFF, np.maximum(counts >> 16, 1)
+        n, stored = len(counts), self.n_entries
+
+        def passes(lanes):  # of the tile that takes most
+            per_pass = lanes // cols
+            return int((-(-rows // np.maximum(per_pass, 1))).max()) if per_pass.all() else n + APC_TILE_MAX_ROWS
+
+        if n == 0:
+            return 256
+        most = passes(64)
+        if most > 1:
+            return 64 if most == 2 and n > PACKED_MANY_TILES and self._states_one_by_one() else 256
+        if n > PACKED_MANY_TILES and stored <= PACKED_MAX_SMALL_COPIES * int((rows.astype(np.int64) * cols).sum()):
+            for lanes in (16, 32):
+                if passes(lanes) == 1:
+                    return lanes
+        return 64
+
+    def small_packing_pays(self) -> bool:
+        """Whether packed tiles, a few lanes each, beat staged ones (above: PACKED_MANY_TILES)."""
+        lanes = self.packed_lanes()
+        if lanes < 64 or self._states_one_by_one():
+            return lanes < 256
+        return lanes == 64 and (len(self.mesh_sizes) < 3 or self.n_tiles < PACKED_MANY_TILES_OF_64 or
+                                2 * self.n_entries >= 3 * self.computed_entries())
+
+    def _states_one_by_one(self) -> bool:
+        """Whether a staged tile works out the running-bytes states of a mesh of three dims or four one by one."""
+        return len(self.mesh_sizes) >= 3 and any(m & (m - 1) for m in self.mesh_sizes)
 
     def largest_tiles_first_pays(self) -> bool:
         """Whether a launch takes the tiles by size instead of edge by edge (above: ORDERED_MAX_ENTRIES)."""

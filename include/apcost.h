@@ -625,11 +625,21 @@ int apc_build_tables_packed(const apc_params *params, int64_t n_tensors, const i
                             const int32_t *num_args, double *compute_cost, double *compute_cost_per_arg,
                             int32_t *error_flag, const double *pt_values, int64_t n_tiles, const apc_packed_tile *packed,
                             int64_t n_entries, double *cost_out, double *row_min, int32_t *row_argmin, void *stream);
+/* The same by fewer lanes a tile than a workgroup's 256: 64, or, where no tile has more rows or columns than that (a larger one's
+ * entries are not written), 32 or 16. */
+int apc_build_tables_packed_small(const apc_params *params, int64_t n_tensors, const int32_t *tensor_rank,
+                            const int32_t *tensor_itemsize, const int64_t *tensor_shape, const int64_t *tensor_stride,
+                            int64_t *tensor_bytes, uint8_t *tensor_contiguous, int64_t n_strategies, const int64_t *flops,
+                            const int64_t *rw_bytes, const int8_t *dtype_code, const uint8_t *zero_cost,
+                            const int32_t *num_args, double *compute_cost, double *compute_cost_per_arg,
+                            int32_t *error_flag, const double *pt_values, int64_t n_tiles, const apc_packed_tile *packed,
+                            int64_t n_entries, double *cost_out, double *row_min, int32_t *row_argmin, int32_t lanes_per_tile,
+                            void *stream);
 
 /* A launch that is kept for repeating (a plan's pass).  A launch passes its arguments by value in a segment that the
  * host has just written, which every compute unit reads past the caches; a kept launch has them in device memory.
  *   apc_keep_next_launch(&k);              the next apc_input_tables, apc_redistribute_tables[_row_min],
- *   apc_build_tables...(args, NULL);       apc_build_tables[_row_min] or apc_build_tables_packed of this thread checks
+ *   apc_build_tables...(args, NULL);       apc_build_tables[_row_min] or apc_build_tables_packed[_small] of this thread checks
  *                                          its arguments and is recorded in k instead of being enqueued; k.kernel stays
  *                                          NULL when it fails or has nothing to launch
  *   copy k.block (k.block_bytes) to device memory, 64-byte aligned

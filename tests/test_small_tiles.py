@@ -1,0 +1,89 @@
+"""Packed tiles by few lanes each: 16, 32 or 64 instead of a workgroup (``CostTables.packed_lanes``)."""
+
+import numpy as np
+import pytest
+import torch
+
+from autoparallel_amd import CostModelParams
+from autoparallel_amd.device_tables import DeviceCostTables
+from autoparallel_amd.encoding import PACKED_MANY_TILES
+from autoparallel_amd.synthetic import stress_dag
+from oracle import c_oracle
+from oracle import cost_oracle as po
+
+MESHES = [(64,), (6,), (32, 8), (12, 6), (8, 8, 8), (6, 4, 2), (2, 4, 2, 2), (3, 2, 2, 2)]
+
+
+def _tables(mesh, nodes, lo, hi, seed=3):
+    odd = int(np.lcm.reduce([m // (m & -m) for m in mesh]))
+    tb = stress_dag(seed=seed, n_nodes=nodes, mesh_sizes=tuple(1 << (m - 1).bit_length() for m in mesh), min_strategies=lo, max_strategies=hi)
+    tb.mesh_sizes = mesh
+    live = np.arange(tb.tensor_shape.shape[1])[None, :] < tb.tensor_rank[:, None]
+    tb.tensor_shape[live] *= odd
+    # a third of the tensors with the strides of another layout, some with an empty dim
+    tb.tensor_stride[::3] = tb.tensor_stride[::3, ::-1]
+    tb.tensor_shape[5::11, 0] = 0
+    tb.build_tiles(None, dedupe=True)
+    return tb
+
+
+@pytest.mark.parametrize("mesh", [(64,), (3, 2, 2, 2)])
+def test_lanes_are_those_that_take_a_tile_at_once(mesh):
+    few, many = (_tables(mesh, n, 1, 4) for n in (100, 3000))
+    assert few.packed_lanes() == 64 and many.n_tiles > PACKED_MANY_TILES and many.packed_lanes() == 16
+    assert _tables(mesh, 3000, 5, 5).packed_lanes() == 32  # 5 x 5: three rows of 16 lanes, six of 32
+    assert _tables(mesh, 300, 1, 8).packed_lanes() == 64  # 8 x 8
+    assert _tables(mesh, 300, 1, 11).packed_lanes() == 256  # 11 x 11: three rounds of five rows
+    many.tile_records = many.tile_records[:0]
+    assert many.packed_lanes() == 256
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mesh", MESHES)
+@pytest.mark.parametrize("nodes,lo,hi", [(37, 1, 4), (90, 2, 5), (61, 1, 8), (150, 1, 16)])
+def test_every_number_of_lanes_has_the_oracles_bits(gpu_device, monkeypatch, mesh, nodes, lo, hi):
+    """Tiles of one round of lanes and of several, numbers of tiles that leave the last wavefront partly empty, copies, pass-through
+    entries, layouts and empty dims: the oracle's costs, row minima, compute costs and tensor bytes."""
+    tb = _tables(mesh, nodes, lo, hi)
+    want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh, rescale=2.2))["cost"]
+    lowest, where = c_oracle.segmented_min(want, tb.row_ptr())
+    kept = None
+    for lanes in (256, 64, 32, 16):
+        monkeypatch.setattr(tb, "packed_lanes", lambda: lanes)
+        d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
+        step = d.prepare_step(fused_inputs=True, one_launch=True, row_min_in_tiles=True, outputs=("cost",), spec_table=False, packed=True)
+        for t in (d.cost, d.row_min, d.row_argmin):
+            t.fill_(-1)
+        for launch in step.values():
+            launch()
+        torch.cuda.synchronize()
+        for got, expected in ((d.cost, want), (d.row_min, lowest), (d.row_argmin, where)):
+            assert np.array_equal(got.cpu().numpy(), expected), lanes
+        rest = [t.cpu().numpy() for t in (d.compute_cost, d.compute_cost_per_arg, d.tensor_bytes, d.tensor_contiguous)]
+        kept = kept or rest
+        assert all(np.array_equal(a, b) for a, b in zip(rest, kept))
+
+
+@pytest.mark.gpu
+def test_small_tiles_under_capture(gpu_device):
+    """A table that goes over few lanes a tile: a captured pass finds the tiles of an earlier preparation, or, where that was over staged
+    tiles, goes over those."""
+    mesh = (64,)
+    tb = _tables(mesh, 2200, 1, 4)
+    assert tb.small_packing_pays() and tb.staging_pays(tb.computed_entries(), tb.n_tiles)
+    want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh, rescale=2.2))["cost"]
+    for before in (None, False):
+        d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
+        assert d.row_min_in_tiles_pays()
+        d.planner_pass(packed=before)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            step = d.planner_pass()
+            for launch in step.values():
+                launch()
+        assert list(step) == ["build_tables" if before is False else "build_tables_packed"]
+        for _ in range(3):
+            d.cost.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(d.cost.cpu().numpy(), want)
