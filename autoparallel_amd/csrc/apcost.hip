@@ -2758,9 +2758,13 @@ __global__ __launch_bounds__(kBlock) void strategy_bounds_kernel(int64_t n_strat
 }
 
 // The bounds, the smallest of every node and the first strategy that has it: G consecutive lanes to a node, its
-// strategies and their order those of segmented_min_kernel, so that the result is its result, NaN included.  (One launch instead of two,
-// and a node's edges are looked up by a lane once for its strategies.)
-template <int G>
+// strategies and their order those of segmented_min_kernel, so that the result is its result, NaN included.
+// Bound by a chain of loads: a node's ranges, its edges, their first rows, the minima.  A lane has four edges and eight of its
+// strategies in flight and goes through the chain once for them all; pair of strategies by pair and edge by edge that was a dozen round
+// trips one behind the other.  us by rocprofv3, before / now: 8 320 nodes of some 12 strategies 13.3 / 7.4, 3 000 of 34 30.7 / 10.1,
+// 2 500 of 30 27.9 / 10.0, 24 000 of 12 14.9 / 9.1, 2 000 of 15 17.3 / 7.6, 8 000 of 3 4.3 / 4.5.
+// (Workgroups of one wavefront: more compute units take part.)
+template <int G, int kPairs>  // kPairs: of a lane's strategies, in flight
 __global__ __launch_bounds__(kBlock) void greedy_strategies_kernel(int64_t n_nodes, const int64_t *__restrict__ node_strat_begin,
                                                                    const int64_t *__restrict__ node_edge_begin,
                                                                    const int32_t *__restrict__ edges_by_node,
@@ -2768,7 +2772,7 @@ __global__ __launch_bounds__(kBlock) void greedy_strategies_kernel(int64_t n_nod
                                                                    const double *__restrict__ row_min, double *__restrict__ bound,
                                                                    double *__restrict__ node_min, int32_t *__restrict__ node_argmin) {
   const int sub = threadIdx.x & (G - 1);
-  const int64_t n = (int64_t)blockIdx.x * (kBlock / G) + (threadIdx.x / G);
+  const int64_t n = (int64_t)blockIdx.x * (blockDim.x / G) + (threadIdx.x / G);
   const bool live = n < n_nodes;
   const int64_t lo = live ? node_strat_begin[n] : 0, hi = live ? node_strat_begin[n + 1] : 0;
   const int64_t e0 = live ? node_edge_begin[n] : 0, e1 = live ? node_edge_begin[n + 1] : 0;
@@ -2781,16 +2785,34 @@ __global__ __launch_bounds__(kBlock) void greedy_strategies_kernel(int64_t n_nod
       arg = j;
     }
   };
-  for (int64_t j = lo + 2 * sub; j < hi; j += 2 * G) {
-    const bool second = j + 1 < hi;
-    double x = 0.0, y = 0.0;
-    for (int64_t e = e0; e < e1; ++e) {
-      const double *row = row_min + edge_row_begin[edges_by_node[e]] + (j - lo);
-      x += row[0];
-      if (second) y += row[1];
+  constexpr int kEdges = 4;
+  for (int64_t j = lo + 2 * sub; j < hi; j += 2 * G * kPairs) {
+    double sum[2 * kPairs] = {};
+    for (int64_t e = e0; e < e1; e += kEdges) {
+      const double *row[kEdges];
+      double v[kEdges][2 * kPairs] = {};
+      int32_t edge[kEdges];
+#pragma unroll
+      for (int u = 0; u < kEdges; ++u)
+        if (e + u < e1) edge[u] = edges_by_node[e + u];
+#pragma unroll
+      for (int u = 0; u < kEdges; ++u)
+        if (e + u < e1) row[u] = row_min + edge_row_begin[edge[u]] - lo;
+#pragma unroll
+      for (int u = 0; u < kEdges; ++u)
+        if (e + u < e1) {
+#pragma unroll
+          for (int k = 0; k < 2 * kPairs; ++k)
+            if (const int64_t at = j + (k / 2) * 2 * G + (k & 1); at < hi) v[u][k] = row[u][at];
+        }
+#pragma unroll
+      for (int u = 0; u < kEdges; ++u)
+#pragma unroll
+        for (int k = 0; k < 2 * kPairs; ++k) sum[k] = e + u < e1 ? sum[k] + v[u][k] : sum[k];
     }
-    take(x, j);
-    if (second) take(y, j + 1);
+#pragma unroll
+    for (int k = 0; k < 2 * kPairs; ++k)
+      if (const int64_t at = j + (k / 2) * 2 * G + (k & 1); at < hi) take(sum[k], at);
   }
 #pragma unroll
   for (int off = G / 2; off > 0; off >>= 1) {
@@ -4729,10 +4751,11 @@ int apc_greedy_strategies(int64_t n_nodes, int64_t n_strategies, const int64_t *
   if (!node_strat_begin || !node_edge_begin || !node_min || !node_argmin || (n_strategies > 0 && !bound))
     return fail(-1, "apc_greedy_strategies: NULL array");
   if (n_nodes > (int64_t)INT32_MAX * 4) return fail(-1, "n_nodes %lld too large", (long long)n_nodes);
-  const int g = segment_lanes(n_strategies, n_nodes);
+  const int g = segment_lanes(n_strategies, n_nodes), threads = n_nodes <= INT32_MAX ? 64 : kBlock;
+  const bool few = n_strategies <= 2 * g * n_nodes;  // a lane has a pair
 #define APC_GREEDY(G_)                                                                                                       \
   case G_:                                                                                                                   \
-    hipLaunchKernelGGL((greedy_strategies_kernel<G_>), dim3(blocks_for(n_nodes, kBlock / G_)), dim3(kBlock), 0,               \
+    hipLaunchKernelGGL((few ? greedy_strategies_kernel<G_, 1> : greedy_strategies_kernel<G_, 4>), dim3(blocks_for(n_nodes, threads / G_)), dim3(threads), 0, \
                        (hipStream_t)stream, n_nodes, node_strat_begin, node_edge_begin, edges_by_node, edge_row_begin,        \
                        row_min, bound, node_min, node_argmin);                                                               \
     break

@@ -60,6 +60,32 @@ def test_greedy_strategies_are_the_two_launches(gpu_device, group, most, monkeyp
     assert torch.equal(node_arg, want_arg)
 
 
+@pytest.mark.parametrize("group", [None, 1, 8])
+@pytest.mark.parametrize("most,edges", [(2, 9), (4, 5), (9, 13), (70, 6)])
+def test_greedy_strategies_of_nodes_of_many_edges(gpu_device, group, most, edges, monkeypatch):
+    """Sums over more edges than a lane has in flight, in their order: magnitudes of which another order has other bits."""
+    if group:
+        monkeypatch.setenv("APC_SEGMIN_GROUP", str(group))
+    rng = np.random.default_rng(most + edges)
+    n_nodes = 97
+    n_strat, n_edges_of = rng.integers(0, most + 1, n_nodes), rng.integers(0, edges + 1, n_nodes)
+    begin, edge_begin = (np.concatenate([[0], np.cumsum(a)]).astype(np.int64) for a in (n_strat, n_edges_of))
+    owner = np.repeat(np.arange(n_nodes), n_edges_of)
+    row_begin = (np.cumsum(n_strat[owner]) - n_strat[owner]).astype(np.int64)
+    row_min = 10.0 ** rng.uniform(-9, 9, int(n_strat[owner].sum()))
+    row_min[rng.random(len(row_min)) < 0.05] = np.nan
+    on = [torch.from_numpy(a).to(gpu_device) for a in (begin, edge_begin, np.arange(len(owner), dtype=np.int32), row_begin, row_min)]
+    want = np.zeros(int(begin[-1]))
+    for n in range(n_nodes):
+        for e in range(edge_begin[n], edge_begin[n + 1]):
+            want[begin[n]:begin[n + 1]] += row_min[row_begin[e]:row_begin[e] + n_strat[n]]
+    ops = _native.torch_ops()
+    bound, node_min, node_arg = ops.greedy_strategies(*on, int(begin[-1]))
+    assert np.array_equal(bound.cpu().numpy(), want, equal_nan=True)
+    for got, ref in zip((node_min, node_arg), ops.segmented_min(bound, on[0])):
+        assert np.array_equal(got.cpu().numpy(), ref.cpu().numpy(), equal_nan=got.is_floating_point())
+
+
 def test_an_unsupported_dtype_is_refused(gpu_device):
     tb = stress_dag(seed=5, n_nodes=200, mesh_sizes=(4, 2))
     params = CostModelParams.from_mesh((4, 2))
