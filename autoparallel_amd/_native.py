@@ -86,6 +86,7 @@ EXPORTS = (
     "apc_strategy_bounds",
     "apc_greedy_strategies",
     "apc_edge_rows",
+    "apc_report_inputs",
     "apc_copy_arrays",
     "apc_check_tables",
     "apc_edge_classes",

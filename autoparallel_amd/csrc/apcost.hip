@@ -2878,7 +2878,7 @@ __global__ __launch_bounds__(kBlock) void copy_arrays_kernel(CopyArrays a) {
 // across it behind one barrier.  Bound by the latency of the counts, which may be in host memory.  (us a call with its wait, a consecutive
 // run of edges a thread / these / the host's sum and its transfer: 8 300 edges 19 / 18 / 25, 100 000 135 / 54 / 97, 1 000 000 2 116 / 430 / 1 110.)
 constexpr int kScanThreads = 1024, kScanEdges = 4, kScanBlocks = 4;
-__global__ __launch_bounds__(kScanThreads) void edge_rows_kernel(int64_t n_edges, const int32_t *__restrict__ n_tgt, int64_t *__restrict__ begin) {
+__device__ __forceinline__ void edge_rows_of_workgroup(int64_t n_edges, const int32_t *__restrict__ n_tgt, int64_t *__restrict__ begin) {
   constexpr int kWaves = kScanThreads / 64;
   constexpr int64_t kBlockEdges = kScanThreads * kScanEdges;
   __shared__ int64_t s_wave[2][kScanBlocks][kWaves];
@@ -2935,6 +2935,29 @@ __global__ __launch_bounds__(kScanThreads) void edge_rows_kernel(int64_t n_edges
       }
     }
   }
+}
+__global__ __launch_bounds__(kScanThreads) void edge_rows_kernel(int64_t n_edges, const int32_t *__restrict__ n_tgt, int64_t *__restrict__ begin) {
+  edge_rows_of_workgroup(n_edges, n_tgt, begin);
+}
+
+// What the tiles of a report read, in one launch: the first rows of the edges by the first workgroup, the tensor table and the compute
+// costs by the others, which are done before it is.  The flag of an unsupported dtype may be in host memory.  (As two launches, with a fill of the
+// flag in front and a copy of it behind, a report of 1.5 M entries on (64, 4) takes 278 us and 250 this way, the faster greedy strategies above
+// included; 5.8 M on (16, 8, 4) 265 / 235, 530 k on (3, 2, 2, 2) 249 / 222.)
+struct ReportInputsArgs {
+  apc_params p;
+  TensorTableArgs t;
+  ComputeCostArgs c;
+  int64_t n_edges;
+  const int32_t *n_tgt;
+  int64_t *row_begin;
+  int64_t row_blocks, tensor_blocks;
+};
+__global__ __launch_bounds__(kScanThreads) void report_inputs_kernel(ReportInputsArgs a) {
+  const int64_t b = (int64_t)blockIdx.x - a.row_blocks;
+  if (b < 0) edge_rows_of_workgroup(a.n_edges, a.n_tgt, a.row_begin);
+  else if (b < a.tensor_blocks) tensor_tables_block<kScanThreads>(b, a.t);
+  else compute_costs_block<kScanThreads>(b - a.tensor_blocks, a.p, a.c);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -4779,6 +4802,26 @@ int apc_edge_rows(int64_t n_edges, const int32_t *edge_n_tgt, int64_t *edge_row_
   if (!edge_n_tgt || !edge_row_begin) return fail(-1, "apc_edge_rows: NULL array");
   hipLaunchKernelGGL(edge_rows_kernel, dim3(1), dim3(kScanThreads), 0, (hipStream_t)stream, n_edges, edge_n_tgt, edge_row_begin);
   return check_launch("apc_edge_rows");
+}
+
+int apc_report_inputs(const apc_params *params, int64_t n_tensors, const int32_t *rank, const int32_t *itemsize, const int64_t *shape,
+                      const int64_t *stride, int64_t *tensor_bytes, uint8_t *tensor_contiguous, int64_t n_strategies, const int64_t *flops,
+                      const int64_t *rw_bytes, const int8_t *dtype, const uint8_t *zero_cost, const int32_t *num_args, double *compute,
+                      double *per_arg, int32_t *error_flag, int64_t n_edges, const int32_t *edge_n_tgt, int64_t *edge_row_begin, void *stream) {
+  if (int rc = check_params(params)) return rc;
+  if (n_tensors < 0 || n_strategies < 0 || n_edges < 0) return fail(-1, "apc_report_inputs: negative count");
+  if (n_tensors > 0 && (!rank || !itemsize || !shape || !stride || !tensor_bytes || !tensor_contiguous))
+    return fail(-1, "apc_report_inputs: NULL tensor array");
+  if (n_strategies > 0 && (!flops || !rw_bytes || !dtype || !zero_cost || !num_args)) return fail(-1, "apc_report_inputs: NULL strategy array");
+  if (n_edges > 0 && (!edge_n_tgt || !edge_row_begin)) return fail(-1, "apc_report_inputs: NULL edge array");
+  const int64_t rb = n_edges > 0 ? 1 : 0, tb = blocks_for(n_tensors, kScanThreads), cb = blocks_for(n_strategies, kScanThreads);
+  if (rb + tb + cb == 0) return 0;
+  if (rb + tb + cb > INT32_MAX) return fail(-1, "apc_report_inputs: too many rows for one launch");
+  const ReportInputsArgs a{*params, {n_tensors, rank, itemsize, shape, stride, tensor_bytes, tensor_contiguous},
+                           {n_strategies, flops, rw_bytes, dtype, zero_cost, num_args, compute, per_arg, error_flag},
+                           n_edges, edge_n_tgt, edge_row_begin, rb, tb};
+  hipLaunchKernelGGL(report_inputs_kernel, dim3((unsigned)(rb + tb + cb)), dim3(kScanThreads), 0, (hipStream_t)stream, a);
+  return check_launch("apc_report_inputs");
 }
 
 int apc_copy_arrays(int64_t n, const void *const *from_host, void *const *to_host, const int64_t *bytes_host, void *stream) {

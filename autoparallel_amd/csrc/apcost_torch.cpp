@@ -815,10 +815,10 @@ Tensor edge_classes(const Tensor &spec_codes, const Tensor &spec_tensor, const T
   return out;
 }
 
-// The tables of a report: tensor and compute-cost tables in one launch, then every per-entry array and, where edge_n_tgt is given
+// The tables of a report: tensor and compute-cost tables and the first rows of the edges in one launch, then every per-entry array and, where edge_n_tgt is given
 // (on the host or on the device), the row minima.  -> ([tensor_bytes, tensor_contiguous, compute, per_arg, comm, transition, cost, row_min, row_argmin], whether a
-// strategy with flops has an unsupported dtype).  Waits for the first launch's flag only, which a copy behind that launch brings
-// while the second one runs.
+// strategy with flops has an unsupported dtype).  Waits for the first launch only, which writes its flag to host memory, while the second one
+// runs.
 std::tuple<std::vector<Tensor>, bool> report_tables(
     const Tensor &params, const Tensor &rank, const Tensor &itemsize, const Tensor &shape, const Tensor &stride,
     const Tensor &spec_codes, const Tensor &spec_tensor, const Tensor &flops, const Tensor &rw_bytes, const Tensor &dtype,
@@ -834,30 +834,34 @@ std::tuple<std::vector<Tensor>, bool> report_tables(
   OptTensor row_begin, dup_rows, row_min, row_argmin;
   Tensor counts;  // (pinned; the flag's event stands behind the launch that reads them too, and the flag goes first)
   Staging flag((int64_t)sizeof(int32_t), stream, 2);  // (with an event)
-  if (edge_n_tgt.has_value() && edge_n_tgt->is_cpu()) {  // (read where they are, while the launch behind is prepared: a copy first is 10 us more)
-    TORCH_CHECK(edge_n_tgt->scalar_type() == at::kInt && edge_n_tgt->is_contiguous(), "apcost: edge_n_tgt must be a contiguous int32 tensor");
+  const int32_t *n_tgt = nullptr;
+  if (edge_n_tgt.has_value()) {
     const int64_t n = edge_n_tgt->numel();
-    counts = at::empty({n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
     row_begin = empty_like_device(rank, {n}, at::kLong);
-    const int32_t *n_tgt = edge_n_tgt->data_ptr<int32_t>();
-    int32_t *to = counts.data_ptr<int32_t>();
-    int64_t sum = 0;
-    for (int64_t e = 0; e < n; ++e) sum += to[e] = n_tgt[e];
-    TORCH_CHECK(sum == n_rows, "apcost: edge_n_tgt has ", sum, " rows, n_rows says ", n_rows);
-    check_rc(apc_edge_rows(n, to, static_cast<int64_t *>(row_begin->data_ptr()), stream), "apc_edge_rows");
-  } else if (edge_n_tgt.has_value()) {
-    row_begin = edge_rows(*edge_n_tgt);
+    if (edge_n_tgt->is_cpu()) {  // (read where they are: a copy first is 10 us more)
+      TORCH_CHECK(edge_n_tgt->scalar_type() == at::kInt && edge_n_tgt->is_contiguous(), "apcost: edge_n_tgt must be a contiguous int32 tensor");
+      counts = at::empty({n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+      const int32_t *from = edge_n_tgt->data_ptr<int32_t>();
+      int32_t *to = counts.data_ptr<int32_t>();
+      int64_t sum = 0;
+      for (int64_t e = 0; e < n; ++e) sum += to[e] = from[e];
+      TORCH_CHECK(sum == n_rows, "apcost: edge_n_tgt has ", sum, " rows, n_rows says ", n_rows);
+      n_tgt = to;
+    } else {
+      n_tgt = dev<int32_t>(*edge_n_tgt, at::kInt, "edge_n_tgt");
+      same_device(rank, *edge_n_tgt, "edge_n_tgt");
+    }
   }
   Tensor bytes = empty_like_device(rank, {t.n}, at::kLong), contiguous = empty_like_device(rank, {t.n}, at::kByte);
   Tensor compute = empty_like_device(rank, {st.n}, at::kDouble), per_arg = empty_like_device(rank, {st.n}, at::kDouble);
-  Tensor error = at::zeros({1}, rank.options().dtype(at::kInt));
-  check_rc(apc_input_tables(&p, t.n, t.rank, t.itemsize, t.shape, t.stride, dev<int64_t>(bytes, at::kLong, "tensor_bytes"),
-                            dev<uint8_t>(contiguous, at::kByte, "tensor_contiguous"), 0, nullptr, nullptr, nullptr, nullptr, nullptr, 2,
-                            nullptr, nullptr, st.n, st.flops, st.rw_bytes, st.dtype, st.zero_cost, st.num_args,
-                            dev<double>(compute, at::kDouble, "compute"), dev<double>(per_arg, at::kDouble, "per_arg"),
-                            error.data_ptr<int32_t>(), stream),
-           "apc_input_tables");
-  check_hip(hipMemcpyAsync(flag.slot(0), error.data_ptr(), sizeof(int32_t), hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
+  int32_t *const error = reinterpret_cast<int32_t *>(flag.slot(0));  // (pinned: the launch writes it where it is read)
+  *error = 0;
+  check_rc(apc_report_inputs(&p, t.n, t.rank, t.itemsize, t.shape, t.stride, dev<int64_t>(bytes, at::kLong, "tensor_bytes"),
+                             dev<uint8_t>(contiguous, at::kByte, "tensor_contiguous"), st.n, st.flops, st.rw_bytes, st.dtype, st.zero_cost,
+                             st.num_args, dev<double>(compute, at::kDouble, "compute"), dev<double>(per_arg, at::kDouble, "per_arg"), error,
+                             row_begin.has_value() ? row_begin->numel() : 0, n_tgt,
+                             row_begin.has_value() && row_begin->numel() > 0 ? static_cast<int64_t *>(row_begin->data_ptr()) : nullptr, stream),
+           "apc_report_inputs");
   check_hip(hipEventRecord(flag.events[0], stream), "hipEventRecord");
   Tensor comm = empty_like_device(rank, {n_entries}, at::kDouble), transition = empty_like_device(rank, {n_entries}, at::kByte),
          cost = empty_like_device(rank, {n_entries}, at::kDouble);
@@ -873,9 +877,7 @@ std::tuple<std::vector<Tensor>, bool> report_tables(
                            transition, cost, row_begin, dup_rows, row_min, row_argmin)
       ->run();
   check_hip(hipEventSynchronize(flag.events[0]), "hipEventSynchronize");
-  int32_t unsupported;
-  std::memcpy(&unsupported, flag.slot(0), sizeof(unsupported));
-  return {out, unsupported != 0};
+  return {out, *static_cast<const volatile int32_t *>(error) != 0};
 }
 
 // apc_input_tables: tensor table, compute costs and (with spec_outputs) the spec table in one launch.

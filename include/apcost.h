@@ -410,6 +410,14 @@ int apc_edge_classes(int64_t n_specs, const uint32_t *spec_codes, const int32_t 
  * sum of edge_n_tgt[0 .. e).  The counts may be in pinned host memory. */
 int apc_edge_rows(int64_t n_edges, const int32_t *edge_n_tgt, int64_t *edge_row_begin, void *stream);
 
+/* apc_input_tables without the spec table, and apc_edge_rows, in one launch.  error_flag, which the caller clears, and the counts may be in pinned
+ * host memory. */
+int apc_report_inputs(const apc_params *params, int64_t n_tensors, const int32_t *tensor_rank, const int32_t *tensor_itemsize,
+                      const int64_t *tensor_shape, const int64_t *tensor_stride, int64_t *tensor_bytes, uint8_t *tensor_contiguous,
+                      int64_t n_strategies, const int64_t *flops, const int64_t *rw_bytes, const int8_t *dtype_code,
+                      const uint8_t *zero_cost, const int32_t *num_args, double *compute_cost, double *compute_cost_per_arg,
+                      int32_t *error_flag, int64_t n_edges, const int32_t *edge_n_tgt, int64_t *edge_row_begin, void *stream);
+
 /* Arrays copied in one launch: bytes_host[k] bytes from from_host[k] to to_host[k] (HOST tables of n addresses and sizes, read before the
  * call returns), any of the arrays in pinned host memory.  No two of them overlap. */
 #define APC_COPY_MAX_ARRAYS 32

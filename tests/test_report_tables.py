@@ -86,6 +86,27 @@ def test_greedy_strategies_of_nodes_of_many_edges(gpu_device, group, most, edges
         assert np.array_equal(got.cpu().numpy(), ref.cpu().numpy(), equal_nan=got.is_floating_point())
 
 
+@pytest.mark.parametrize("n_nodes", [2, 60, 1100])
+@pytest.mark.parametrize("row_min", [False, True])
+def test_inputs_of_a_report_are_those_of_the_single_launches(gpu_device, n_nodes, row_min, monkeypatch):
+    """Tensors and strategies below and beyond a workgroup, with and without the edges' first rows; the flag of the last strategy alone."""
+    tb = stress_dag(seed=8, n_nodes=n_nodes, mesh_sizes=(4, 2))
+    tb.build_tiles(None, dedupe=True)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh((4, 2)), device=gpu_device)
+    monkeypatch.setattr(d, "row_min_in_tiles_pays", lambda: row_min)
+    d.build_all()
+    got = [d.tensor_bytes, d.tensor_contiguous, d.compute_cost, d.compute_cost_per_arg]
+    for a, b in zip(got, (*d.run_tensor_tables(), *d.run_compute_costs())):
+        assert torch.equal(a, b)
+    if row_min:
+        for a, b in zip((d.row_min, d.row_argmin), d.segmented_min(d.cost, tb.row_ptr())):
+            assert torch.equal(a, b)
+    tb.strat_flops[-1], tb.strat_dtype[-1], tb.strat_zero_cost[-1] = 1, 7, 0
+    d.refresh("strat_flops", "strat_dtype", "strat_zero_cost")
+    with pytest.raises(ValueError, match="dtype not supported"):
+        d.build_all()
+
+
 def test_an_unsupported_dtype_is_refused(gpu_device):
     tb = stress_dag(seed=5, n_nodes=200, mesh_sizes=(4, 2))
     params = CostModelParams.from_mesh((4, 2))
