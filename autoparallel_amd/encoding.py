@@ -119,8 +119,8 @@ STAGED_MAX_STORED_PER_EDGE = 304
 # 2 906 6.2 / 4.2 / 4.2 / 3.7, 3 488 in two layers on (6,) 7.1 / 5.2 / 4.7 / 4.0, 3 158 of nine copies 7.5 / 5.9 / - / 6.3, 926 of sixteen 5.7 / 5.2 / 6.0 / 6.0; of at
 # most 25, 1 446 on (16, 8, 4) 5.1 / 4.4 / 4.4, 4 644 10.8 / 8.0 / 6.4, 4 693 on (3, 2, 2, 2) 15.1 / 11.4 / 9.5, 2 596 of twenty copies on (3, 8) 8.1 / 7.0 / 7.4; of
 # at most 64, 944 of sixteen copies on (32, 8) 5.9 / 5.3, 4 297 on (8, 8, 8) 10.0 / 7.8, 5 571 on (3, 2, 2, 2) 17.2 / 12.8.  Where a wavefront
-# goes over its tile twice it loses (944 tiles of at most 81 entries on (32, 8) 6.1 / 6.9, 4 297 of 100 9.3 / 8.0 with 7.3 staged), but on
-# meshes whose states are staged one by one and that leave no other choice (2 910 of at most 100 on (3, 2, 2, 2) 11.9 / 10.1, 3 720 of 81 on (6, 4, 2)
+# goes over its tile twice it loses (944 tiles of at most 81 entries on (32, 8) 6.1 / 6.9, 4 297 of 100 9.3 / 8.0 with 7.3 staged), except on
+# meshes whose states are staged one by one, for tables that go over packed tiles anyway (2 910 of at most 100 on (3, 2, 2, 2) 11.9 / 10.1, 3 720 of 81 on (6, 4, 2)
 # 12.2 / 11.1).
 # They beat staged tiles (same cases: 5.4 / 3.7 for 2 906 tiles of 16 entries, 7.3 / 6.4 for 4 644 of 25, 7.4 / 6.0 for 2 188 of 64 and ten copies, 12.7 / 9.7
 # for 5 571 of 64 on (6, 4, 2)) except, with 64 lanes, PACKED_MANY_TILES_OF_64 and more without copies on power-of-two meshes of
@@ -564,32 +564,36 @@ class CostTables:
 
     def packed_lanes(self, records: Optional[np.ndarray] = None) -> int:
         """Lanes a packed tile is evaluated by (above: PACKED_MANY_TILES), for the tiling's records or the ``records`` given."""
+        return self._packed_lanes_and_rounds(records)[0]
+
+    def _packed_lanes_and_rounds(self, records: Optional[np.ndarray] = None) -> tuple:
+        """-> (``packed_lanes``, rounds in which a wavefront takes the tile that needs most)"""
         counts = (self.tile_records if records is None else records)["counts"]
         rows, cols = counts & 0xFFFF, np.maximum(counts >> 16, 1)
         n, stored = len(counts), self.n_entries
 
-        def passes(lanes):  # of the tile that takes most
-            per_pass = lanes // cols
-            return int((-(-rows // np.maximum(per_pass, 1))).max()) if per_pass.all() else n + APC_TILE_MAX_ROWS
+        def rounds(lanes):
+            per_round = lanes // cols
+            return int((-(-rows // np.maximum(per_round, 1))).max()) if per_round.all() else n + APC_TILE_MAX_ROWS
 
         if n == 0:
-            return 256
-        most = passes(64)
+            return 256, 0
+        most = rounds(64)
         if most > 1:
-            return 64 if most == 2 and n > PACKED_MANY_TILES and self._states_one_by_one() else 256
+            return 64 if most == 2 and n > PACKED_MANY_TILES and self._states_one_by_one() else 256, most
         if n > PACKED_MANY_TILES and stored <= PACKED_MAX_SMALL_COPIES * int((rows.astype(np.int64) * cols).sum()):
             for lanes in (16, 32):
-                if passes(lanes) == 1:
-                    return lanes
-        return 64
+                if rounds(lanes) == 1:
+                    return lanes, 1
+        return 64, most
 
     def small_packing_pays(self) -> bool:
-        """Whether packed tiles, a few lanes each, beat staged ones (above: PACKED_MANY_TILES)."""
-        lanes = self.packed_lanes()
-        if lanes < 64 or self._states_one_by_one():
-            return lanes < 256
-        return lanes == 64 and (len(self.mesh_sizes) < 3 or self.n_tiles < PACKED_MANY_TILES_OF_64 or
-                                2 * self.n_entries >= 3 * self.computed_entries())
+        """Whether packed tiles, a few lanes each and in one round, beat staged ones (above: PACKED_MANY_TILES)."""
+        lanes, rounds = self._packed_lanes_and_rounds()
+        if lanes == 256 or rounds != 1:
+            return False
+        return lanes < 64 or self._states_one_by_one() or len(self.mesh_sizes) < 3 or self.n_tiles < PACKED_MANY_TILES_OF_64 or \
+            2 * self.n_entries >= 3 * self.computed_entries()
 
     def _states_one_by_one(self) -> bool:
         """Whether a staged tile works out the running-bytes states of a mesh of three dims or four one by one."""

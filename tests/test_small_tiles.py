@@ -34,6 +34,10 @@ def test_lanes_are_those_that_take_a_tile_at_once(mesh):
     assert _tables(mesh, 3000, 5, 5).packed_lanes() == 32  # 5 x 5: three rows of 16 lanes, six of 32
     assert _tables(mesh, 300, 1, 8).packed_lanes() == 64  # 8 x 8
     assert _tables(mesh, 300, 1, 11).packed_lanes() == 256  # 11 x 11: three rounds of five rows
+    # 10 x 10: two rounds of six rows, by a wavefront on meshes of many states; no reason to leave staged tiles
+    twice = _tables(mesh, 2500, 1, 10)
+    assert twice.packed_lanes() == (64 if len(mesh) > 1 else 256) and not twice.small_packing_pays()
+    assert few.small_packing_pays() and many.small_packing_pays()
     many.tile_records = many.tile_records[:0]
     assert many.packed_lanes() == 256
 
