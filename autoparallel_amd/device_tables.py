@@ -126,6 +126,7 @@ class DeviceCostTables:
             self._edge_rows = None
         if not set(_PACKED).isdisjoint(names):
             self._host_on_device = None
+            self._drop_stand_ins()
             if self._packed_cache is not None:
                 self._pack_again()
 
@@ -267,6 +268,7 @@ class DeviceCostTables:
         for key, t in zip(("strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost"), out):
             self.d[key] = t
         self._packed_current, self._host_on_device = False, None  # (the host's strategy table is about to change)
+        self._drop_stand_ins()
         return out
 
     # ---- per-strategy compute cost ---------------------------------------------------------
@@ -478,23 +480,58 @@ class DeviceCostTables:
 
     _host_on_device = None  # (tile records, whether a preparation over them found the host's tables on the device), since the last upload
 
-    def _staged_is_as_packed(self, capturing) -> bool:
+    def _staged_is_as_packed(self, capturing, sent) -> bool:
         """Whether a pass over staged tiles, which read the tables on the device, has the results of one over packed ones, which are
-        the host's: whether no table was changed on the host and not uploaded.  Found once per tiling, as those are made (0.1 to 0.4 ms); while
-        the stream captures, as an earlier preparation found it, or left it without packed tiles."""
+        the host's: whether no table was changed on the host and not uploaded.  Found once per tiling, as those are made (0.1 to 0.4 ms);
+        ``sent``, a list, then receives the copies of the host's tables (``_packed_of``) and of the edges' first rows.  While the stream captures, as
+        an earlier preparation found it, or left it without packed tiles."""
         tb, known = self.tables, self._host_on_device
         if known is not None and known[0] is tb.tile_records:
             return known[1]
         if capturing:
             return self._packed_cache is None or self._packed_cache[0] is not tb.tile_records
-        sent, there = self._upload(*self._packed_of(False)), [self.d[k] for k in _PACKED]
+        *tables, edge_rows = self._upload(*self._packed_of(False), tb.edge_row_begin())
+        sent[:] = tables, edge_rows
+        there = [self.d[k] for k in _PACKED]
 
         def joined(arrays):
             return torch.cat([a.reshape(-1).view(torch.uint8) for a in arrays])
 
-        same = all(a.dtype == b.dtype and a.shape == b.shape for a, b in zip(sent, there)) and torch.equal(joined(sent), joined(there))
+        same = all(a.dtype == b.dtype and a.shape == b.shape for a, b in zip(tables, there)) and torch.equal(joined(tables), joined(there))
         self._host_on_device = tb.tile_records, same
         return same
+
+    # Whether the packed tiles are there in place of staged ones only.  What a pass over staged tiles would have left behind, the edges' first
+    # rows, is there then too, and where a table changes they go: the next preparation makes others with its look at the
+    # host's tables, and while a stream captures staged tiles take the pass.  (Made again with every upload, as those that a pass has
+    # no choice but to go over, they cost it 0.1 to 0.4 ms for the 1 to 3 us that they save a pass.)
+    _packed_stands_in = False
+
+    def _packed_for_staged(self, capturing, sent) -> bool:
+        """Whether packed tiles, a few lanes each, take a pass that staged ones could take; ``sent``: of ``_staged_is_as_packed``."""
+        tb, cached = self.tables, self._packed_cache
+        there = cached is not None and cached[0] is tb.tile_records
+        if there and self._packed_stands_in:
+            return True
+        if capturing and not (there and self._packed_current):
+            return False
+        lanes = tb.small_packing_lanes()
+        if not lanes or capturing:
+            return bool(lanes)
+        tables, self._edge_rows = sent or (None, self._edge_rows)
+        if self._edge_rows is None:
+            self._edge_rows = _to_device(tb.edge_row_begin(), self.device)
+        if not there:
+            self._packed_stands_in = True
+            if tables and tb.n_tiles >= self.PACK_ON_DEVICE_MIN_TILES and not tb.largest_tiles_first_pays():
+                dev, packed = self.ops.pack_tiles(*tables)
+                if packed:
+                    self._packed_cache, self._packed_current = (tb.tile_records, True, dev, lanes), True
+        return True
+
+    def _drop_stand_ins(self):
+        if self._packed_stands_in:
+            self._packed_cache, self._packed_stands_in = None, False
 
     def _pack_again(self):
         """The packed tiles anew where a table they are made of was uploaded: a pass that is prepared next, also while the stream
@@ -540,7 +577,7 @@ class DeviceCostTables:
         flop / byte counts this pass reads).  ``packed``: the one launch runs over packed tiles
         (``apc_build_tables_packed``: the assembled cost and the row minima, no spec table);
         ``None`` takes them when the pass is of that kind, ``packed_pass_pays`` and staged tiles
-        (``CostTables.staging_pays``, ``small_packing_pays``) are not faster still.  Packed tiles hold the host's tables as they are at the first
+        (``CostTables.staging_pays``, ``small_packing_lanes``) are not faster still.  Packed tiles hold the host's tables as they are at the first
         preparation after a tiling or an upload; where staged tiles are faster for the repeated pass of a small table, they are taken if the tables on the device, which
         they read, are the same.  ``repeated=False``: the pass will run once, and the arguments
         of its launches are not laid out in device memory first (``apc_kept_launch``: one copy, for 0.75 us less a launch over packed
@@ -548,7 +585,8 @@ class DeviceCostTables:
         into launch order (``CostTables.launch_records``: 10 ns a tile on the host).  Those copies, one a launch
         and one of the tiles, are waited for.  So are the uploads of row indices and packed tiles; while the current stream
         captures, a pass is prepared as with ``repeated=False`` and takes the edges' first rows, or the packed tiles, of an earlier preparation
-        (a table that staged tiles are faster for goes over packed ones where only those are there)."""
+        (a table that staged tiles are faster for goes over packed ones where only those are there, and one that packed tiles are faster for over
+        staged ones where a table or the tiling was uploaded since)."""
         tb = self.tables
         capturing, runs_once = torch.cuda.is_current_stream_capturing(), not repeated
         repeated = bool(repeated) and not capturing
@@ -569,14 +607,15 @@ class DeviceCostTables:
         if one_launch is None:
             one_launch = bool(fused_inputs) and total <= self.one_launch_limit(row_min_in_tiles)
         packed_kind = bool(one_launch) and row_min_in_tiles and outputs == ("cost",) and not spec_table
+        stands_in = False
         if packed is None:
             packed = packed_kind and self.packed_pass_pays()
-            small = packed and tb.small_packing_pays() and (not capturing or (
-                self._packed_cache is not None and self._packed_cache[0] is tb.tile_records))
-            if packed and not small and (self._edge_rows is not None or not capturing):
-                of_tiles = tb.computed_entries(), tb.n_tiles
+            if packed and (self._edge_rows is not None or not capturing):
+                of_tiles, sent = (tb.computed_entries(), tb.n_tiles), []
                 packed = not (tb.staging_pays(*of_tiles, repeated=False) or (
-                    not runs_once and tb.staging_pays(*of_tiles) and self._staged_is_as_packed(capturing)))
+                    not runs_once and tb.staging_pays(*of_tiles) and self._staged_is_as_packed(capturing, sent)))
+                stands_in = not packed and self._packed_for_staged(capturing, sent)
+                packed = packed or stands_in
         elif packed and not (packed_kind and self.tables.packable()):
             raise ValueError("a pass over packed tiles is one launch that writes the assembled cost and the row minima, "
                              "without the spec table, over tiles of whole rows")
@@ -617,6 +656,8 @@ class DeviceCostTables:
         erb, rmin, rarg = rows if rows is not None else (None, None, None)
         dup_rows = d["dup_row_begin"] if rows is not None else None
         if packed:
+            if not stands_in and not capturing:
+                self._packed_stands_in = False
             tiles = self._packed_tiles(repeated)
             step = {"build_tables_packed": bind(ops.bind_cost_tables_packed(
                 self.p, *self._tensor_table(), self.tensor_bytes, self.tensor_contiguous, *self._strategy_table(),

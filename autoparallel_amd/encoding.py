@@ -589,11 +589,16 @@ class CostTables:
 
     def small_packing_pays(self) -> bool:
         """Whether packed tiles, a few lanes each and in one round, beat staged ones (above: PACKED_MANY_TILES)."""
+        return self.small_packing_lanes() > 0
+
+    def small_packing_lanes(self) -> int:
+        """``packed_lanes`` where ``small_packing_pays``, else 0."""
         lanes, rounds = self._packed_lanes_and_rounds()
         if lanes == 256 or rounds != 1:
-            return False
-        return lanes < 64 or self._states_one_by_one() or len(self.mesh_sizes) < 3 or self.n_tiles < PACKED_MANY_TILES_OF_64 or \
+            return 0
+        pays = lanes < 64 or self._states_one_by_one() or len(self.mesh_sizes) < 3 or self.n_tiles < PACKED_MANY_TILES_OF_64 or \
             2 * self.n_entries >= 3 * self.computed_entries()
+        return lanes if pays else 0
 
     def _states_one_by_one(self) -> bool:
         """Whether a staged tile works out the running-bytes states of a mesh of three dims or four one by one."""

@@ -7,6 +7,7 @@ import torch
 from autoparallel_amd import CostModelParams
 from autoparallel_amd.device_tables import DeviceCostTables
 from autoparallel_amd.encoding import PACKED_MANY_TILES
+from autoparallel_amd.graphs.cost_inputs import StrategyRecipes
 from autoparallel_amd.synthetic import stress_dag
 from oracle import c_oracle
 from oracle import cost_oracle as po
@@ -91,3 +92,62 @@ def test_small_tiles_under_capture(gpu_device):
             graph.replay()
             torch.cuda.synchronize()
             assert np.array_equal(d.cost.cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change", ["tiling", "tables", "tables of two lengths", "strategy inputs", "changed on the host", "prepared for one run"])
+def test_a_capture_after_a_change_of_small_tiles(gpu_device, change):
+    """A table that goes over few lanes a tile though it could be staged, one of whose tables or whose tiling is another before a pass is
+    captured, with no preparation between the two: it has the costs of the tables as they are then."""
+    mesh = (64,)
+    tb = _tables(mesh, 2200, 1, 4)
+    assert tb.small_packing_pays() and tb.staging_pays(tb.computed_entries(), tb.n_tiles)
+    op = po.make_params(mesh, rescale=2.2)
+    before = c_oracle.build_tables(tb.as_dict(), op)["cost"]
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=gpu_device)
+    if change == "changed on the host":  # (not uploaded: the pass is of the host's tables, and staged tiles are no way out)
+        tb.strat_rw_bytes *= 2
+    d.planner_pass()
+    repeated = change != "prepared for one run"
+    if not repeated:
+        d.planner_pass(repeated=False)
+    packed = d._packed_cache
+    assert packed is not None and (change == "changed on the host") == (d._edge_rows is None)
+    if change == "tiling":
+        tb.build_tiles(None, dedupe=True, max_copies=2)
+        d.refresh("tile_records", "dup_entry_begin", "dup_row_begin")
+    elif change == "strategy inputs":  # (the device counts, and the host's table receives the result)
+        recipes = StrategyRecipes(tb.n_nodes)
+        recipes.node_kind[:] = 1
+        recipes.node_row_begin[:] = np.arange(tb.n_nodes + 1)
+        recipes.byte_rows = np.zeros(tb.n_nodes, np.int32)
+        for name, t in zip(("strat_flops", "strat_rw_bytes", "strat_dtype", "strat_zero_cost"), d.run_strategy_inputs(recipes)):
+            getattr(tb, name)[:] = t.cpu().numpy()
+    else:
+        tb.strat_flops[:] = 0
+        if change == "tables of two lengths":
+            kept, tb.strat_flops = tb.strat_flops, np.append(tb.strat_flops, 0)
+            d.refresh("strat_flops")
+            tb.strat_flops = kept
+        d.refresh("strat_flops")
+    # what a pass has no choice but to go over is made again at once, and nothing where staged tiles are one
+    assert (d._packed_cache is not None) == (change in ("changed on the host", "prepared for one run"))
+    want = c_oracle.build_tables(tb.as_dict(), op)["cost"]
+    assert change == "tiling" or not np.array_equal(want, before)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step = d.planner_pass(repeated=repeated)
+        for launch in step.values():
+            launch()
+    assert list(step) == ["build_tables" if d._packed_cache is None else "build_tables_packed"]
+    for _ in range(3):
+        d.cost.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(d.cost.cpu().numpy(), want)
+    step = d.planner_pass()  # the next preparation is over packed tiles again
+    assert list(step) == ["build_tables_packed"]
+    for launch in step.values():
+        launch()
+    torch.cuda.synchronize()
+    assert np.array_equal(d.cost.cpu().numpy(), want)
