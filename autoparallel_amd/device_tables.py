@@ -862,7 +862,7 @@ class DeviceCostTables:
         labels, degree = np.diff(graph.label_begin), np.diff(graph.inc_begin)
         ends = np.concatenate([graph.edge_i, graph.edge_j])
         n_colors = len(graph.color_begin) - 1
-        capacity = (n_colors + 64) * most + int((9 * labels + degree)[ends].sum()) + 3 * graph.n_edges
+        capacity = (n_colors + 80) * most + int((9 * labels + degree)[ends].sum())
         plan, begin, sizes = np.empty(capacity, np.int32), np.empty(most + 1, np.int64), np.empty(5, np.int64)
         index = index_arrays(graph)
         color_begin, color_nodes = np.ascontiguousarray(graph.color_begin, np.int64), np.ascontiguousarray(graph.color_nodes, np.int32)

@@ -233,6 +233,15 @@ def test_a_plan_by_teams_gives_every_row_its_wavefronts(name):
     assert (held == (2 if by_teams else 0)).all()
 
 
+@pytest.mark.parametrize("n_matrices", [1, 215, 218, 224])
+def test_the_plan_buffer_holds_teams_up_to_the_most_workgroups(n_matrices):
+    """On the CPU: one matrix a workgroup, up to as many workgroups as can be resident."""
+    from autoparallel_amd.device_tables import DeviceCostTables
+
+    words, begin, *_ = DeviceCostTables._sweep_plan(_problem(1, [130] * (n_matrices + 1), [(i, i - 1) for i in range(1, n_matrices + 1)]))
+    assert len(begin) - 1 == n_matrices and set(words[begin[:-1] + 5].tolist()) == {2}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", TEAMS)
 def test_sweeps_by_teams_equal_the_oracle(gpu_device, name):
