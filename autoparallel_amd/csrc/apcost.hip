@@ -2426,9 +2426,11 @@ __device__ __forceinline__ void store_copies16(int64_t entry0, double *cost_out,
   }
 }
 
-// `first`: the wavefront's first tile.
+// `first`: the wavefront's first tile.  A tile of more rows or columns than lanes is left out and says so.
+constexpr int kTooFewLanes = 2;  // in the error flag
 template <int M, bool POW2, int kLanes>
-__device__ __forceinline__ void packed_small_tiles(const apc_packed_tile *tiles, int first, int n_tiles, double *cost_out, const PackedArgs &a) {
+__device__ __forceinline__ void packed_small_tiles(const apc_packed_tile *tiles, int first, int n_tiles, double *cost_out, const PackedArgs &a,
+                                                   int32_t *const &error_flag) {
   const apc_params &p = a.p;
   const int lane = threadIdx.x & 63, sub = lane & (kLanes - 1), first_lane = lane & (64 - kLanes);
   const int tile = first + lane / kLanes;
@@ -2452,8 +2454,12 @@ __device__ __forceinline__ void packed_small_tiles(const apc_packed_tile *tiles,
                       p.inv_compute_eff, a.inv_rescale, p.rescale, p.a2a_scale, p.base_latency);
   int rows = of_lane16<0>(h);
   const int cols = of_lane16<1>(h), flags = of_lane16<2>(h), dup_count = of_lane16<3>(h), t0 = of_lane16<4>(h);
-  if (tile >= n_tiles || (unsigned)rows > (unsigned)kLanes || (unsigned)(cols - 1) >= (unsigned)kLanes || (unsigned)dup_count > (unsigned)APC_PACKED_MAX_DUPS)
-    rows = 0;  // none, or no small tile
+  const bool refused = (unsigned)rows > (unsigned)kLanes || (unsigned)(cols - 1) >= (unsigned)kLanes || (unsigned)dup_count > (unsigned)APC_PACKED_MAX_DUPS;
+  if (__ballot(refused && tile < n_tiles) != 0) {  // (uniform: the flag's address is fetched here)
+    int32_t *const flag = error_flag;
+    if (refused && tile < n_tiles && flag) *flag = kTooFewLanes;
+  }
+  if (tile >= n_tiles || refused) rows = 0;
   const int64_t entry_begin = (int64_t)((uint64_t)(uint32_t)of_lane16<9>(h) << 32 | (uint32_t)of_lane16<8>(h));
   const int64_t row_begin = (int64_t)((uint64_t)(uint32_t)of_lane16<11>(h) << 32 | (uint32_t)of_lane16<10>(h));
   // ---- the tensor's bytes, the rows' compute costs ------------------------------------------------
@@ -2621,7 +2627,7 @@ __global__ __launch_bounds__(kBlock) void build_tables_packed_kernel(APC_LAUNCH_
       const int first = group * per_block + uniform_i32((int)threadIdx.x >> 6) * (64 / LANES);
       if (group >= n_groups || first >= n_tiles) return;
       if constexpr (LANES == 64) packed_tile<M, POW2, true>(tiles + first, cost_out, k.a);
-      else packed_small_tiles<M, POW2, LANES>(tiles, first, n_tiles, cost_out, k.a);
+      else packed_small_tiles<M, POW2, LANES>(tiles, first, n_tiles, cost_out, k.a, k.c.error_flag);
     }
     return;
   }
@@ -5099,6 +5105,8 @@ static int build_tables_packed_impl(const apc_params *params, int64_t n_tensors,
                             int64_t n_entries, double *cost_out, double *row_min, int32_t *row_argmin, int lanes,
                                     const LaunchTo &to) {
   if (int rc = check_params(params)) return rc;
+  if (lanes != 16 && lanes != 32 && lanes != 64 && lanes != kBlock)
+    return fail(-1, "apc_build_tables_packed: 16, 32, 64 or %d lanes a tile (got %d)", kBlock, lanes);
   if (n_tensors < 0 || n_strategies < 0 || n_entries < 0) return fail(-1, "apc_build_tables_packed: negative count");
   if (n_tiles < 0 || n_tiles > (1 << 30)) return fail(-1, "n_tiles %lld out of range", (long long)n_tiles);
   if (n_tensors > 0 && (!rank || !itemsize || !shape || !stride || !tensor_bytes || !tensor_contiguous))
@@ -5109,8 +5117,6 @@ static int build_tables_packed_impl(const apc_params *params, int64_t n_tensors,
     return fail(-1, "apc_build_tables_packed: NULL tile records or outputs");
   if ((reinterpret_cast<uintptr_t>(packed) & 63) != 0) return fail(-1, "apc_build_tables_packed: packed tiles must be 64-byte aligned");
   const int xs = xcd_shift();
-  if (lanes != 16 && lanes != 32 && lanes != 64 && lanes != kBlock)
-    return fail(-1, "apc_build_tables_packed: 16, 32, 64 or %d lanes a tile (got %d)", kBlock, lanes);
   const int64_t groups = blocks_for(n_tiles, kBlock / lanes);
   const int64_t tile_blocks = ((groups + (1 << xs) - 1) >> xs) << xs;
   const int64_t tb = blocks_for(n_tensors, kBlock), cb = blocks_for(n_strategies, kBlock);

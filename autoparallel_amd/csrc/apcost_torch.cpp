@@ -938,6 +938,7 @@ c10::intrusive_ptr<BoundLaunch> bind_cost_tables_packed(const Tensor &params, co
                                                         const Tensor &error_flag, const Tensor &pt_values, const Tensor &packed,
                                                         int64_t n_entries, int64_t n_rows, const Tensor &cost,
                                                         const Tensor &row_min, const Tensor &row_argmin, int64_t lanes) {
+  TORCH_CHECK(lanes == 0 || lanes == 16 || lanes == 32 || lanes == 64 || lanes == 256, "apcost: 16, 32, 64 or 256 lanes a tile (got ", lanes, ")");
   auto b = c10::make_intrusive<BoundLaunch>();
   const apc_params p = params_of(params);
   const TensorTable t = tensor_table(rank, itemsize, shape, stride);

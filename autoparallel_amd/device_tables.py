@@ -721,6 +721,8 @@ class DeviceCostTables:
             self._check_flag(int(err.item()))
 
     def _check_flag(self, flag: int):
+        if flag == 2:
+            raise RuntimeError("packed tiles were taken by fewer lanes than some tile has rows or columns")
         if flag != 0:
             # compute_estimation.py:198-201
             raise ValueError(f"a strategy with non-zero flops uses a dtype not supported on {self.params.device_name}")

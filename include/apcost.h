@@ -633,8 +633,8 @@ int apc_build_tables_packed(const apc_params *params, int64_t n_tensors, const i
                             const int32_t *num_args, double *compute_cost, double *compute_cost_per_arg,
                             int32_t *error_flag, const double *pt_values, int64_t n_tiles, const apc_packed_tile *packed,
                             int64_t n_entries, double *cost_out, double *row_min, int32_t *row_argmin, void *stream);
-/* The same by fewer lanes a tile than a workgroup's 256: 64, or, where no tile has more rows or columns than that (a larger one's
- * entries are not written), 32 or 16. */
+/* The same by lanes_per_tile lanes: 256, a workgroup, as above; 64; or, where no tile has more rows or columns than that, 32 or 16.
+ * The entries of a larger tile are then not written, and *error_flag is set to 2. */
 int apc_build_tables_packed_small(const apc_params *params, int64_t n_tensors, const int32_t *tensor_rank,
                             const int32_t *tensor_itemsize, const int64_t *tensor_shape, const int64_t *tensor_stride,
                             int64_t *tensor_bytes, uint8_t *tensor_contiguous, int64_t n_strategies, const int64_t *flops,

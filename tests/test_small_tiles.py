@@ -1,10 +1,12 @@
 """Packed tiles by few lanes each: 16, 32 or 64 instead of a workgroup (``CostTables.packed_lanes``)."""
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from autoparallel_amd import CostModelParams
+from autoparallel_amd import CostModelParams, _native
 from autoparallel_amd.device_tables import DeviceCostTables
 from autoparallel_amd.encoding import PACKED_MANY_TILES
 from autoparallel_amd.graphs.cost_inputs import StrategyRecipes
@@ -67,6 +69,58 @@ def test_every_number_of_lanes_has_the_oracles_bits(gpu_device, monkeypatch, mes
         rest = [t.cpu().numpy() for t in (d.compute_cost, d.compute_cost_per_arg, d.tensor_bytes, d.tensor_contiguous)]
         kept = kept or rest
         assert all(np.array_equal(a, b) for a, b in zip(rest, kept))
+
+
+def _packed_pass(tb, mesh, device, monkeypatch, lanes):
+    monkeypatch.setattr(tb, "packed_lanes", lambda: lanes)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh(mesh, rescale=2.2), device=device)
+    step = d.prepare_step(fused_inputs=True, one_launch=True, row_min_in_tiles=True, outputs=("cost",), spec_table=False, packed=True)
+    for t in (d.cost, d.row_min, d.row_argmin):
+        t.fill_(-1)
+    for launch in step.values():
+        launch()
+    torch.cuda.synchronize()
+    return d
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lanes", [16, 32])
+def test_a_tile_larger_than_its_lanes_is_reported(gpu_device, monkeypatch, lanes):
+    """The entries of the others are the oracle's, those of the larger ones are left alone, and the error flag says so."""
+    mesh = (12, 6)
+    tb = _tables(mesh, 60, 1, lanes + 8)
+    tb.build_tiles(lanes, dedupe=False)
+    want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh, rescale=2.2))["cost"]
+    large = np.zeros(tb.n_entries, bool)
+    counts = tb.tile_records["counts"]
+    for e, row, n in zip(tb.tile_edge, tb.tile_row_begin, counts):
+        cols, first = n >> 16, tb.edge_entry_begin[e] + row * (n >> 16)
+        large[first:first + (n & 0xFFFF) * cols] = max(n & 0xFFFF, cols) > lanes
+    assert large.any() and not large.all()
+    d = _packed_pass(tb, mesh, gpu_device, monkeypatch, lanes)
+    got = d.cost.cpu().numpy()
+    assert np.array_equal(got[~large], want[~large]) and (got[large] == -1).all()
+    with pytest.raises(RuntimeError, match="fewer lanes"):
+        d._check_flag(int(d._step_error_flag.item()))
+    d = _packed_pass(tb, mesh, gpu_device, monkeypatch, 64)
+    d._check_flag(int(d._step_error_flag.item()))
+    assert np.array_equal(d.cost.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("lanes,through_the_operator", [(0, False), (8, False), (128, False), (-16, False), (8, True), ((1 << 32) + 16, True)])
+def test_other_numbers_of_lanes_are_refused(lanes, through_the_operator):
+    """On the CPU; 2^32 + 16 is not 16."""
+    params = CostModelParams.from_mesh((4,)).to_c()
+    if through_the_operator:
+        t = torch.empty(0)
+        with pytest.raises(RuntimeError, match="lanes a tile"):
+            _native.torch_ops().bind_cost_tables_packed(_native.params_tensor(params), *[t] * 16, 0, 0, *[t] * 3, lanes)
+        return
+    null, none = ctypes.c_void_p(None), ctypes.c_int64(0)
+    call = lambda n: _native.lib().apc_build_tables_packed_small(  # noqa: E731
+        ctypes.byref(params), none, *[null] * 6, none, *[null] * 9, none, null, none, *[null] * 3, ctypes.c_int32(n), null)
+    assert call(lanes) != 0 and b"lanes a tile" in _native.lib().apc_last_error()
+    assert [call(n) for n in (16, 32, 64, 256)] == [0] * 4
 
 
 @pytest.mark.gpu
