@@ -3848,6 +3848,7 @@ struct TeamLds {
   uint32_t *finished;
   int *inc, *abort;
   uint32_t looks;  // the clock is read at every (looks + 1)th: it takes longer than the LDS
+  mutable int sweeps;  // of this wavefront: no more where it has given up
 };
 
 __device__ __forceinline__ void keep_order() { __asm__ volatile("" ::: "memory"); }
@@ -3880,8 +3881,10 @@ __device__ __forceinline__ int here(int v) {
 }
 __device__ __forceinline__ uint64_t half_under(uint32_t number, int half) { return (uint64_t)number << 32 | (uint32_t)half; }
 
-// A wait that lasts too long is given up: the workgroup's results are then not used, and what follows goes on with whatever it finds,
-// without waiting.
+// A wait that lasts too long is given up: the workgroup's results are then not used.  The wavefront ends its sweep with whatever it finds and
+// leaves; those that wait for it find the flag at their next look at the clock and do the same, and other workgroups, whose waits began
+// when this one's did, give up themselves.  (1 000 000 sweeps given up at their first wait, ms when wavefronts went on to the last sweep / now: 149
+// matrices in 20 workgroups 2 850 / 0.02, a class with 70 matrices 16 300 / 0.05; a sweep that nothing is given up in takes as long as before.)
 struct Patience {
   uint64_t began;
   uint32_t tries;
@@ -3892,6 +3895,7 @@ __device__ __forceinline__ bool give_up(Patience &w, const TeamLds &l, uint64_t 
   if (w.tries == l.looks + 1) w.began = now;
   if (uniform_i32(__hip_atomic_load(l.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) == 0 && now - w.began < wait_ticks) return false;
   __hip_atomic_store(l.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  l.sweeps = 0;
   return true;
 }
 
@@ -4119,6 +4123,7 @@ __device__ __forceinline__ void team_sweeps(const ResidentArgs &a, unsigned char
   l.finished = reinterpret_cast<uint32_t *>(l.inc + n_inc);
   l.abort = reinterpret_cast<int *>(l.finished + APC_SWEEP_MAX_WAVES);
   l.looks = a.wait_ticks == 0 ? 0 : 15;
+  l.sweeps = a.n_sweeps;
   const int4 *rows = reinterpret_cast<const int4 *>(plan + 8);
   const int32_t *labels = reinterpret_cast<const int32_t *>(rows + 2 * n_rows);
   const int32_t *incs = labels + n_rows;
@@ -4141,7 +4146,7 @@ __device__ __forceinline__ void team_sweeps(const ResidentArgs &a, unsigned char
     uint32_t *const finished = l.finished + (team & 0xFF);
     uint32_t updates = 0;
     __builtin_amdgcn_s_setprio(3);
-    for (int sweep = 0; sweep < a.n_sweeps; ++sweep, updates += 2) {
+    for (int sweep = 0; sweep < l.sweeps; ++sweep, updates += 2) {
       team_update(l, a, x, (uint32_t)sweep + 1, waves, finished, updates, tid & 63);
       team_update(l, a, y, (uint32_t)sweep + 1, waves, finished, updates + 1, tid & 63);
     }

@@ -71,6 +71,28 @@ def test_an_expired_wait_leaves_the_sweeps_to_the_launches(gpu_device):
     assert np.array_equal(theta, want[0]) and np.array_equal(unary, want[1])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["a chain over many workgroups", "a class with 70 matrices (more than the kept reciprocals)"])
+def test_an_expired_wait_ends_the_kernel_whatever_the_sweeps(gpu_device, name):
+    """By teams: a million sweeps whose first unmet wait is given up.  An update takes 0.2 us and more, so that all of them would
+    be 400 ms; those of a sweep after the wait are some microseconds."""
+    import torch
+
+    g = _problem(4, *CASES[name])
+    dev = _device()
+    plan = dev._sweep_plan(g)
+    assert (plan[0][plan[1][:-1] + 5] == 2).all() and len(plan[1]) > 3
+    arrays = dev._upload(*plan[:2], g.theta, g.unary)
+    run = lambda n: dev.ops.diffusion_sweeps_resident(  # noqa: E731
+        n, *arrays[:2], *plan[2:], int(g.label_begin[-1]), int(g.edge_begin[-1]), *arrays[2:], 0)
+    run(1)
+    begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    begin.record()
+    *_, status = run(1_000_000)
+    end.record()
+    assert int(status.item()) == 1 and begin.elapsed_time(end) < 40
+
+
 def test_an_expired_wait_is_paid_once_per_problem():
     """On the CPU, with operators that only keep count: after a wait that expired, the chunks that follow take the launches
     at once; another problem has a plan again."""
