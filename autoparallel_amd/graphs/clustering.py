@@ -158,16 +158,14 @@ def cluster_regions(graph: torch.fx.Graph, strats: dict) -> dict:
             return a.meta.get("val")
         return a if isinstance(a, (torch.Tensor, int)) else None
 
-    # Nodes of one operator and metadata share their strategies' objects: each list is written out once.  Equal texts are one
-    # object, so that the bytes a key is pickled to, which tell an object met before from a new one, follow from its contents.
+    # Nodes of one operator and metadata share their strategies' objects: each list is written out once.  (The pickler has no memo: a
+    # key's bytes follow from its contents, whichever of its texts are one object.)
     written: dict = {}
-    texts: dict = {}
 
     def text_of(what, strategy):
         key = (what, *map(id, strategy.strategies))
         if key not in written:
-            text = what(strategy)
-            written[key] = texts.setdefault(text, text)
+            written[key] = what(strategy)
         return written[key]
 
     def strategy_text(node):
@@ -176,8 +174,7 @@ def cluster_regions(graph: torch.fx.Graph, strats: dict) -> dict:
             return text_of(str, s)
         if s is None and node.op == "output":  # (the reference keys the output node by its producers' strategies)
             s = [strats[x] for x in node.all_input_nodes]
-        text = str(s)
-        return texts.setdefault(text, text)
+        return str(s)
 
     same_key = defaultdict(list)
     group_of = {}

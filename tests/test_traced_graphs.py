@@ -180,6 +180,28 @@ def test_tiny_moe_regions_and_plan(fake_pg):
             assert str(plan[node]) == str(opt.strats[node].strategies[0])
 
 
+def test_links_follow_from_the_texts_of_strategies_not_from_their_objects(fake_pg):
+    """Nodes that share their strategies' objects against nodes with objects of their own: the same keys, the same links."""
+    import copy
+
+    from torch._dynamo.graph_region_tracker import InputPickler
+    from torch.distributed.tensor._op_schema import OpStrategy
+
+    from autoparallel_amd.graphs.clustering import cluster_regions
+
+    with _planner(OraclePlanner, TINY_MOE, (8, 4), 16, 64, repeated_subgraphs=True) as autop:
+        opt = autop.sharding_optimizer
+        graph, strats = autop.gm.graph, opt.strats
+        own = {n: OpStrategy([copy.copy(x) for x in s.strategies]) if type(s) is OpStrategy else s for n, s in strats.items()}
+        objects = [{id(x) for s in of.values() if type(s) is OpStrategy for x in s.strategies} for of in (strats, own)]
+        assert len(objects[0]) < len(objects[1])
+        links = cluster_regions(graph, strats)
+        assert links and cluster_regions(graph, own) == links
+    text = "S(0)" * 50
+    equal = text, (text + "x")[:-1]
+    assert equal[0] is not equal[1] and InputPickler().dumps((text, text)) == InputPickler().dumps(equal)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("case", list(CASES))
 def test_device_tables_match_oracle_on_benchmark_configurations(gpu_device, fake_pg, case):
