@@ -187,11 +187,12 @@ struct Staging {
 int64_t padded(int64_t n) { return (n + 255) / 256 * 256; }
 
 // Copies between the device and pinned memory that travel together: one launch (apc_copy_arrays) instead of a copy of the runtime's each,
-// 10 us apart.  One alone is faster as such a copy up to about kAlone (300 KB to the device 20 / 25 us).  us a call, by copies / by launches, of
-// `download`: five arrays of up to 10 KB 26 / 17, 292 + 23 KB and a flag 42 / 28, 8.1 MB with them 275 / 255, two of 1.1 MB and two of 136 KB 158 / 140; of
-// `upload`: 8.6 MB in six places 307 / 258, 8 MB and 0.1 246 / 235; 84 MB to the host 2 330 either way, by what the threads do.
+// 10 us apart.  us a call, by copies / by launches, of `download`: five arrays of up to 10 KB 26 / 17, 292 + 23 KB and a flag 42 / 28, 8 MB and
+// 0.05 275 / 255; of `upload`: 8.6 MB in six places 307 / 258, 8 MB and two of 1.2 336 / 288.  One alone is the runtime's in a transfer of at most
+// kAlone (to the device 1.2 MB 49 / 57, 2 MB 75 / 83, 4 MB 120 - 144 / 150, 8 MB 235 / 235; to the host 67 / 74, 105 / 111, 165 / 178, 257 / 257); beyond,
+// where chunk follows chunk, a launch (16 MB 430 / 418, 38 MB 945 / 895, 84 MB 1 945 / 1 856; 450 / 425, 1 157 / 1 170, 2 330 / 2 283).
 struct Copies {
-  static constexpr int64_t kAlone = 1 << 20;
+  static constexpr int64_t kAlone = 2 * kStagingChunk;
   std::vector<const void *> from;
   std::vector<void *> to;
   std::vector<int64_t> bytes;
@@ -201,8 +202,8 @@ struct Copies {
     to.push_back(t);
     bytes.push_back(n);
   }
-  void enqueue(hipMemcpyKind kind, hipStream_t stream) const {
-    if (from.size() == 1 && bytes[0] < kAlone) {
+  void enqueue(hipMemcpyKind kind, hipStream_t stream, int64_t of_transfer) const {
+    if (from.size() == 1 && of_transfer <= kAlone) {
       check_hip(hipMemcpyAsync(to[0], from[0], bytes[0], kind, stream), "hipMemcpyAsync");
       return;
     }
@@ -280,7 +281,7 @@ std::vector<Tensor> upload(const std::vector<Tensor> &arrays, at::Device device)
       const int64_t b = std::max(begin, runs[i].begin), e = std::min(end, runs[i].end);
       copies.add(runs[i].to + (b - runs[i].begin), to + (b - begin), e - b);
     }
-    copies.enqueue(hipMemcpyHostToDevice, stream);
+    copies.enqueue(hipMemcpyHostToDevice, stream, total);
     if (n_slots > 1) check_hip(hipEventRecord(staging.events[slot], stream), "hipEventRecord");
   }
   check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize");
@@ -351,7 +352,7 @@ std::vector<Tensor> download(const std::vector<Tensor> &arrays) {
   auto enqueue = [&](size_t c) {
     Copies copies;
     for (const Piece &p : chunks[c]) copies.add(slot(c) + p.at, static_cast<const char *>(arrays[p.k].data_ptr()) + p.from, p.n);
-    copies.enqueue(hipMemcpyDeviceToHost, stream);
+    copies.enqueue(hipMemcpyDeviceToHost, stream, total);
     if (n_slots > 1) check_hip(hipEventRecord(staging.events[c % n_slots], stream), "hipEventRecord");
   };
   const size_t n_chunks = chunks.size();

@@ -258,3 +258,16 @@ def test_copy_arrays_refuses_what_a_launch_cannot_hold():
         assert lib.apc_copy_arrays(ctypes.c_int64(n), one, one, (ctypes.c_int64 * 33)(*sizes), None) != 0
     assert lib.apc_copy_arrays(ctypes.c_int64(1), None, one, (ctypes.c_int64 * 1)(1), None) != 0
     assert lib.apc_copy_arrays(ctypes.c_int64(2), one, one, (ctypes.c_int64 * 2)(0, 0), None) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [(1,), (1_200_003,), (3 << 20, 5), (17_000_001,), (17_000_001, 7, 1_200_000), (40_000_003,), (300,) * 40])
+def test_transfers_bring_every_byte_there_and_back(gpu_device, sizes):
+    """One array and several, in one chunk of the staging, in several and in more than it holds."""
+    rng = np.random.default_rng(len(sizes))
+    arrays = [torch.from_numpy(rng.integers(0, 255, n, dtype=np.uint8)) for n in sizes]
+    ops = _native.torch_ops()
+    there = ops.upload(arrays, gpu_device)
+    back = ops.download(there)
+    for a, d, b in zip(arrays, there, back):
+        assert torch.equal(a, b) and torch.equal(a, d.cpu())
