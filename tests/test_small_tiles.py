@@ -13,6 +13,7 @@ from autoparallel_amd.graphs.cost_inputs import StrategyRecipes
 from autoparallel_amd.synthetic import stress_dag
 from oracle import c_oracle
 from oracle import cost_oracle as po
+from test_abi_and_encoding import twin_graph
 
 MESHES = [(64,), (6,), (32, 8), (12, 6), (8, 8, 8), (6, 4, 2), (2, 4, 2, 2), (3, 2, 2, 2)]
 
@@ -51,7 +52,9 @@ def test_lanes_are_those_that_take_a_tile_at_once(mesh):
 def test_every_number_of_lanes_has_the_oracles_bits(gpu_device, monkeypatch, mesh, nodes, lo, hi):
     """Tiles of one round of lanes and of several, numbers of tiles that leave the last wavefront partly empty, copies, pass-through
     entries, layouts and empty dims: the oracle's costs, row minima, compute costs and tensor bytes."""
-    tb = _tables(mesh, nodes, lo, hi)
+    tb = _with_copies(_tables(mesh, nodes, lo, hi))
+    tb.build_tiles(None, dedupe=True)
+    assert len(np.unique(tb.tile_records["dup_count"])) > 3
     want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh, rescale=2.2))["cost"]
     lowest, where = c_oracle.segmented_min(want, tb.row_ptr())
     kept = None
@@ -81,6 +84,36 @@ def _packed_pass(tb, mesh, device, monkeypatch, lanes):
         launch()
     torch.cuda.synchronize()
     return d
+
+
+def _with_copies(tb, seed=1):
+    """Eight copies of every node and edge, of which some have another strategy table: from none to seven identical edges to a tile."""
+    for _ in range(3):
+        tb = twin_graph(tb)
+    nodes = np.random.default_rng(seed).random(tb.n_nodes) < np.linspace(0, 0.6, tb.n_nodes)
+    changed = np.repeat(nodes, np.diff(tb.node_strat_begin))
+    tb.strat_rw_bytes[changed] += 1 + np.arange(tb.n_strategies)[changed] // 3
+    return tb
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mesh", [(64,), (12, 6), (8, 8, 8), (3, 2, 2, 2)])
+@pytest.mark.parametrize("most", [16, 32])
+def test_copies_and_sides_up_to_the_lanes(gpu_device, monkeypatch, mesh, most):
+    """Single rows of up to as many columns as lanes (over both halves of 32), single columns and tiles between, next to each other in a
+    wavefront with different numbers of copies."""
+    tb = _with_copies(_tables(mesh, 40, 1, most, seed=most))
+    tb.build_tiles(most, dedupe=True)
+    rows, cols, copies = tb.tile_row_count, tb.tile_col_count, tb.tile_records["dup_count"]
+    assert rows.max() == cols.max() == most and (rows == 1).any() and (cols == 1).any() and len(np.unique(copies)) >= 6
+    want = c_oracle.build_tables(tb.as_dict(), po.make_params(mesh, rescale=2.2))["cost"]
+    lowest, where = c_oracle.segmented_min(want, tb.row_ptr())
+    wide = where[np.isfinite(lowest) & (np.diff(tb.row_ptr()) > 16)]
+    assert most == 16 or ((wide >= 16).any() and (wide < 16).any())
+    for lanes in (256, 64, 32, 16)[:4 if most == 16 else 3]:
+        d = _packed_pass(tb, mesh, gpu_device, monkeypatch, lanes)
+        for got, expected in ((d.cost, want), (d.row_min, lowest), (d.row_argmin, where)):
+            assert np.array_equal(got.cpu().numpy(), expected), lanes
 
 
 @pytest.mark.gpu
