@@ -188,11 +188,10 @@ int64_t padded(int64_t n) { return (n + 255) / 256 * 256; }
 
 // Copies between the device and pinned memory that travel together: one launch (apc_copy_arrays) instead of a copy of the runtime's each,
 // 10 us apart.  us a call, by copies / by launches, of `download`: five arrays of up to 10 KB 26 / 17, 292 + 23 KB and a flag 42 / 28, 8 MB and
-// 0.05 275 / 255; of `upload`: 8.6 MB in six places 307 / 258, 8 MB and two of 1.2 336 / 288.  One alone is the runtime's in a transfer of at most
-// kAlone (to the device 1.2 MB 49 / 57, 2 MB 75 / 83, 4 MB 120 - 144 / 150, 8 MB 235 / 235; to the host 67 / 74, 105 / 111, 165 / 178, 257 / 257); beyond,
-// where chunk follows chunk, a launch (16 MB 430 / 418, 38 MB 945 / 895, 84 MB 1 945 / 1 856; 450 / 425, 1 157 / 1 170, 2 330 / 2 283).
+// 0.05 275 / 255; of `upload`: 8.6 MB in six places 307 / 258, 8 MB and two of 1.2 336 / 288.  One alone is the runtime's in a transfer of one
+// chunk (to the device 1.2 MB 49 / 57, 2 MB 75 / 83, 4 MB 120 - 144 / 150; to the host 67 / 74, 105 / 111, 165 / 178); where chunk follows chunk, a
+// launch (8 MB 235 / 235, 16 MB 430 / 418, 38 MB 945 / 895, 84 MB 1 945 / 1 856; 257 / 257, 450 / 425, 1 157 / 1 170, 2 330 / 2 283).
 struct Copies {
-  static constexpr int64_t kAlone = 2 * kStagingChunk;
   std::vector<const void *> from;
   std::vector<void *> to;
   std::vector<int64_t> bytes;
@@ -203,7 +202,7 @@ struct Copies {
     bytes.push_back(n);
   }
   void enqueue(hipMemcpyKind kind, hipStream_t stream, int64_t of_transfer) const {
-    if (from.size() == 1 && of_transfer <= kAlone) {
+    if (from.size() == 1 && of_transfer <= kStagingChunk) {
       check_hip(hipMemcpyAsync(to[0], from[0], bytes[0], kind, stream), "hipMemcpyAsync");
       return;
     }
