@@ -1166,21 +1166,30 @@ int apc_sweep_plan_host(int64_t n_classes, const int64_t *label_begin, const int
   // wavefront), else runs.  (Figures at the kernels.  Eight wavefronts a workgroup against sixteen, us a sweep: 358 matrices of at
   // most 24 labels 3.5 / 4.4, 794 of 40 9.3 / 11.0; 512 elements a wavefront against 1 024: 1 428 matrices of at most 64 labels 8.1 /
   // 8.5, 358 of 124 6.7 / 7.4.)
+  //   With two colours a sweep of the runs is two steps, and small matrices are little work between them.  us a sweep, runs / teams, of at most
+  //   so many labels with so many elements a matrix: 300 of 3 (4) 2.4 / 2.9, 200 of 5 (8) 3.0 / 3.4, 40 of 5 (9) 2.8 / 3.5; then 500 of 6 (13) 3.7 / 3.3, 60
+  //   of 7 (14) 2.9 / 2.4, 300 of 8 (20) 2.9 / 2.7, though 80 of 6 (13) 3.1 / 3.7 and 30 of 7 (13) 3.2 / 4.1.  With sixteen wavefronts a workgroup 1 900 of 4 (6)
+  //   3.6 / 5.2, 2 600 of 10 (30) 4.4 / 6.7, 1 900 of 12 (42) 4.3 / 4.9; then 2 600 of 14 (56) 4.1 / 3.3, 1 900 of 16 (72) 4.6 / 3.5.  With three colours and more a
+  //   step more a sweep decides for the teams (315 of 3 (2) 3.7 / 2.8, 659 of 5 (5) 4.7 / 3.7), short of 64 matrices of 5 labels 3.2 / 3.8.
   bool of_teams = false;
   if (total > APC_SWEEP_MIN_ELEMENTS || !assign(threads = 256) || n_wg > 1) {
     constexpr struct {
-      int64_t waves, per_wave;
-    } kForms[] = {{APC_SWEEP_MAX_WAVES / 2, 512}, {APC_SWEEP_MAX_WAVES, 512}, {APC_SWEEP_MAX_WAVES, 1024}, {APC_SWEEP_MAX_WAVES, 2048}, {APC_SWEEP_MAX_WAVES, 4096}};
-    for (const auto &form : kForms)
-      if (!of_teams && by_teams(form.per_wave, form.waves)) {
-        of_teams = true;
-        threads = 64 * form.waves;
-      }
+      int64_t waves, per_wave, elements_of_two_colours;
+    } kForms[] = {{APC_SWEEP_MAX_WAVES / 2, 512, 10}, {APC_SWEEP_MAX_WAVES, 512, 48}, {APC_SWEEP_MAX_WAVES, 1024, 48}, {APC_SWEEP_MAX_WAVES, 2048, 48}, {APC_SWEEP_MAX_WAVES, 4096, 48}};
+    auto teams_hold = [&](bool small_too) {
+      for (const auto &form : kForms)
+        if ((small_too || n_colors > 2 || total >= form.elements_of_two_colours * n_edges) && by_teams(form.per_wave, form.waves)) {
+          threads = 64 * form.waves;
+          return true;
+        }
+      return false;
+    };
+    of_teams = teams_hold(false);
     // (the matrices do not fill the shares exactly: larger ones until the workgroups are few enough)
     for (int attempt = 0; !of_teams; ++attempt, share += share / 4) {
       threads = share > APC_SWEEP_WIDE_ELEMENTS ? 1024 : 256;
       if (assign(threads) || assign(threads = 1024)) break;
-      if (attempt == 12) return 0;
+      if (attempt == 12 && !(of_teams = teams_hold(true))) return 0;
     }
   }
   // classes whose matrices lie in several workgroups exchange their minima through memory: a slot per (incidence, label)

@@ -209,7 +209,12 @@ TEAMS = {
     "classes of 4, 5, 8, 9 and 13 matrices over several workgroups": (
         [6 + i % 9 for i in range(60)],
         _star(0, 5, 4) + _star(1, 9, 5) + _star(2, 14, 8) + _star(3, 22, 9) + _star(4, 31, 13) + [(i, i - 5) for i in range(31, 60)], 512, True),
-    "one wavefront more than half the workgroups' hold": ([2, 3] * 897, [(i, i - 1) for i in range(1, 1794)], 1024, True),
+    # (two colours: teams of sixteen wavefronts a workgroup from 48 elements a matrix on, of eight from 10)
+    "one wavefront more than half the workgroups' hold": ([7, 8] * 897, [(i, i - 1) for i in range(1, 1794)], 1024, True),
+    "as many with few elements": ([6, 7] * 897, [(i, i - 1) for i in range(1, 1794)], 256, False),
+    "as many with few elements and three colours": ([2, 3] * 897, [(i, i - 1) for i in range(1, 1794)] + [(2, 0)], 1024, True),
+    "ten elements a matrix": ([2, 5] * 40, [(i, i - 1) for i in range(1, 80)], 512, True),
+    "nine elements a matrix": ([3] * 80, [(i, i - 1) for i in range(1, 80)], 256, False),
     "more matrices than wavefronts": ([1, 2] * 1800, [(i, i - 1) for i in range(1, 3600)], 256, False),
     "few elements in one workgroup": ([3] * 20, [(i, i - 1) for i in range(1, 20)], 256, False),
 }
