@@ -2354,6 +2354,8 @@ __device__ __forceinline__ void packed_tile(const apc_packed_tile *T, double *co
 // that, and not latency, is the launch.  Everything that is wave-uniform above is a lane's own here: the record's words and the copies' offsets by
 // DPP broadcasts within 16 lanes, each of which fetches them; a lane's row and column by quotients, and whole rows go round by round, though one round
 // (1.5 us: a chain of bpermutes and fp64, few wavefronts to hide it) is what the host takes few lanes for (CostTables.packed_lanes).
+// What a launch's constants cost: the compiler keeps 54 to 116 scalar registers in vector lanes (pow2 meshes; 62 to 180 on others), where the form
+// with 256 lanes has 7 to 43 (11 to 81).  Four numbers of lanes are 64 forms of the kernel instead of 16.
 // us a pass before (the faster of a workgroup a tile and of staged tiles) / now: 4 292 tiles of at most 16 entries on (64,) 6.5 / 4.2, 5 770 on (12, 6)
 // 9.1 / 5.5, 2 908 on (3, 2, 2, 2) 10.2 / 5.8; with 32 lanes 4 644 of at most 25 on (16, 8, 4) 7.4 / 6.4, 4 693 on (3, 2, 2, 2) 15.1 / 9.5.
 // ------------------------------------------------------------------------------------------
@@ -2947,9 +2949,9 @@ __global__ __launch_bounds__(kScanThreads) void edge_rows_kernel(int64_t n_edges
 }
 
 // What the tiles of a report read, in one launch: the first rows of the edges by the first workgroup, the tensor table and the compute
-// costs by the others, which are done before it is.  The flag of an unsupported dtype may be in host memory.  (As two launches, with a fill of the
-// flag in front and a copy of it behind, a report of 1.5 M entries on (64, 4) takes 278 us and 250 this way, the faster greedy strategies above
-// included; 5.8 M on (16, 8, 4) 265 / 235, 530 k on (3, 2, 2, 2) 249 / 222.)
+// costs by the others, which are done before it is.  The flag of an unsupported dtype may be in host memory.  (us a report, as two launches with a
+// fill of the flag in front and a copy of it behind / this way, in turn: 1.5 M entries on (64, 4) 276 / 241, 5.8 M on (16, 8, 4) 257 / 228, 530 k on
+// (3, 2, 2, 2) 237 / 215; the faster greedy strategies above show by 0 to 6 us in the same calls.)
 struct ReportInputsArgs {
   apc_params p;
   TensorTableArgs t;
@@ -3834,7 +3836,9 @@ __device__ __forceinline__ bool resident_step(const ResidentLds &l, const Reside
 // through memory 0.4 - 0.65 us more; a sweep is as long as the longest cycle of classes, three updates and more around a class
 // with many.  us a sweep, before (runs) and now: 358 matrices of at most 24 labels 5.5 -> 3.5, of at most 124 8.5 -> 6.7, 794 of 40
 // in five colours 14.7 -> 9.4, 1 098 of 12 6.0 -> 3.9, 1 428 of 64 12.0 -> 7.8.  Runs stay where one workgroup holds them all, which
-// exchanges nothing (27 matrices of at most 3 labels 2.7 against 3.3, 38 of 6 2.3 against 2.6), and where the matrices are too many.
+// exchanges nothing (27 matrices of at most 3 labels 2.7 against 3.3, 38 of 6 2.3 against 2.6), and where the matrices are too many, or small and
+// of two colours (apc_sweep_plan_host).  Chains without hubs, which are two steps a sweep, gain least: 358 of at most 24 labels 3.2 / 3.2, 794 of 40
+// 4.5 / 4.2, 1 428 of 64 13.8 / 6.8.
 // Tried: any wavefront waiting per lane instead of uniformly, with the plan's rows read from LDS for every step (16 % slower than the
 // barriers); waiting wavefronts at the priority of the others (13 % slower); sleeping between two looks (no difference).
 // ------------------------------------------------------------------------------------------

@@ -122,6 +122,8 @@ STAGED_MAX_STORED_PER_EDGE = 304
 # goes over its tile twice it loses (944 tiles of at most 81 entries on (32, 8) 6.1 / 6.9, 4 297 of 100 9.3 / 8.0 with 7.3 staged), except on
 # meshes whose states are staged one by one, for tables that go over packed tiles anyway (2 910 of at most 100 on (3, 2, 2, 2) 11.9 / 10.1, 3 720 of 81 on (6, 4, 2)
 # 12.2 / 11.1).
+# (A launch of 256 lanes a tile runs at one of two speeds from process to process, one of 64 at one in between or as fast: 436 tiles on (64,) 3.3 or 4.2 /
+# 3.3 or 3.75, 126 of eleven copies on (6, 4, 2) 4.5 or 5.0 / 4.7.)
 # They beat staged tiles (same cases: 5.4 / 3.7 for 2 906 tiles of 16 entries, 7.3 / 6.4 for 4 644 of 25, 7.4 / 6.0 for 2 188 of 64 and ten copies, 12.7 / 9.7
 # for 5 571 of 64 on (6, 4, 2)) except, with 64 lanes, PACKED_MANY_TILES_OF_64 and more without copies on power-of-two meshes of
 # three dims or four (staged / packed: 2 910 6.2 / 6.1 on (2, 4, 2, 2), 5.9 / 5.4 on (16, 8, 4); then 4 297 7.3 / 7.8 on (8, 8, 8), 7.5 / 9.3 on (2, 4, 2, 2)).
