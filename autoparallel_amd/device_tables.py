@@ -185,11 +185,14 @@ class DeviceCostTables:
             self.tables.validate(self.params)
             self._refresh(names)
             return
-        before = dict(self.d), self._tiles, self._ordered_tiles, self._edge_rows, self._packed_cache, self._packed_current
+        kept = "_tiles", "_ordered_tiles", "_edge_rows", "_packed_cache", "_packed_current", "_packed_stands_in"
+        before = dict(self.d), [getattr(self, k) for k in kept]
         try:
             self.tables._validate(self.params, lambda: self._refresh_and_check(names, "tables", rows or self.send_rows()))
         except BaseException:
-            self.d, self._tiles, self._ordered_tiles, self._edge_rows, self._packed_cache, self._packed_current = before
+            self.d, values = before
+            for k, v in zip(kept, values):
+                setattr(self, k, v)
             raise
 
     # ---- helpers -------------------------------------------------------------------------

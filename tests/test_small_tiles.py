@@ -238,3 +238,20 @@ def test_a_capture_after_a_change_of_small_tiles(gpu_device, change):
         launch()
     torch.cuda.synchronize()
     assert np.array_equal(d.cost.cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+def test_a_tiling_that_is_refused_leaves_the_small_tiles_as_they_were(gpu_device, monkeypatch):
+    monkeypatch.setattr(DeviceCostTables, "CHECK_ON_DEVICE_MIN_ROWS", 0)
+    tb = _tables((64,), 2200, 1, 4)
+    d = DeviceCostTables(tb, CostModelParams.from_mesh((64,), rescale=2.2), device=gpu_device)
+    d.planner_pass()
+    packed = d._packed_cache
+    assert packed is not None and d._packed_stands_in
+    tb.tile_records["row_begin"][3] += 10**6
+    with pytest.raises(RuntimeError):
+        d.refresh_tiling("tile_records", "dup_entry_begin", "dup_row_begin")
+    tb.tile_records["row_begin"][3] -= 10**6
+    assert d._packed_cache is packed and d._packed_stands_in
+    d.refresh("strat_flops")
+    assert d._packed_cache is None
